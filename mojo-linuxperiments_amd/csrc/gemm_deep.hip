@@ -1,0 +1,381 @@
+// W8A8 contraction for everything between one token and the sizes that fill the chip with 256-wide tiles:
+//   acc[m,n] = sum_k qx[m,k] * qw[n,k],   y = ((float)acc * sx[m]) * sw[n]
+//
+// One workgroup of eight waves per tile, the tile chosen from sixteen (16 x 16 to 128 x 128) so that every compute unit
+// has one, and one load stream per workgroup: stages of 128 to 512 bytes of K go straight to LDS through a ring of D
+// buffers, D - 1 stages in flight, one barrier a stage.  The barrier of stage s says that stage s + 1 has landed and
+// that everybody holds its fragments of stage s in registers; behind it a wave requests the fragments of stage s + 1,
+// the loads of stage s + D into the buffer just freed, and multiplies stage s.  Small tiles leave most of the eight
+// waves without rows of their own, so the waves split K inside a stage (WK slices of 64 bytes) and meet once, through
+// LDS, at the tile's end; every wave finishes an equal share of the matrix-instruction tiles.
+//
+// What bounds it.  The load path of a compute unit: at 128 x 128, K = 14336, one to 256 workgroups alike, a stage takes
+// 850 - 900 clocks of which the matrix instructions need 512 and, with the loads taken out, 705 (550 without the
+// fragment reads as well); no wait for memory is left in the stage.  32 direct-to-LDS loads of 1 KB at 28 clocks each are
+// those 900.  Measured and equal or slower: loads through registers and ds_write, 16 waves, the loads spread between the
+// matrix instructions, another K phase per workgroup, rows of 256 bytes.  So the tile decides: rows loaded per result.
+//
+// Measured (us a call, us before): 16 x 4096 -> 14336 12.3 (14.3), 32 x 4096 -> 4096 5.4 (7.2), 64 x 4096 -> 14336 15.3
+// (27.2), 200 x 4096 -> 14336 24.3 (34.3), 256 x 14336 -> 4096 34.5 (97), 512 x 4096 -> 4096 14.2 (28.3).
+//
+// LDS layout, swizzle and shape of the loads are those of gemm_tiled.hip: 1 KB blocks of 8 rows x 128 bytes, chunk position
+// XORed with sigma(row, block parity), free of bank conflicts for the fragment reads.  Operand A is the weights.
+//
+#include <algorithm>
+
+#include "common.h"
+
+namespace mi {
+namespace deep {
+
+typedef __attribute__((address_space(3))) void *lptr_t;
+
+template <int N>
+__device__ __forceinline__ void wait_vm()
+{
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// direct-to-LDS load of 16 bytes per lane: global address = sbase + voff, LDS address = ldsaddr + 16 * lane
+__device__ __forceinline__ void dma16(const int8_t *sbase, unsigned voff, unsigned ldsaddr)
+{
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(voff), "s"(sbase), "s"(ldsaddr)
+                 : "memory", "m0");
+}
+__device__ __forceinline__ int ror8(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, false); }
+
+template <int TM_, int TN_, int WM_, int WN_, int WK_, int D_>
+struct Cfg {
+    static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, WK = WK_, D = D_;
+    static constexpr int NW = WM * WN * WK, TPB = 64 * NW;
+    static constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
+    static constexpr int SUB = WK / 2;                  // 128-byte K steps per stage
+    static constexpr int BX = BM / 8, BW = BN / 8;      // 1 KB blocks (8 rows x 128 B) per step
+    static constexpr int BLK = (BX + BW) * SUB;         // per stage
+    static constexpr int L = BLK / NW;                  // load instructions per wave and stage
+    static constexpr int STAGE = BLK * 1024;
+    static constexpr int NF = TM * TN;                  // matrix-instruction tiles of a wave
+    static constexpr int OWN = (NF + WK - 1) / WK;      // of which it finishes this many (the last waves fewer or none)
+    static constexpr int PART = WM * WN * NF * (WK - 1) * 1024;
+    static constexpr int LDS = D * STAGE > PART ? D * STAGE : PART;
+    static constexpr bool PAIR = OWN % 2 == 0 && TN % 2 == 0 && NF % OWN == 0;
+    static constexpr int PRE = D > 3 ? 3 : D;           // stages requested before the first is waited for
+    static_assert(WK % 2 == 0 && BLK % NW == 0 && LDS <= 160 * 1024, "");
+    static_assert((D - 1) * L < 60 && D >= 2 && D <= 7, "vmcnt counts to 63");
+};
+
+template <typename C, bool DEQ>
+__device__ __forceinline__ void tile(const int8_t *__restrict__ qx, const int8_t *__restrict__ qw, const float *__restrict__ sx,
+                                     const float *__restrict__ sw, void *__restrict__ out, const int M, const int N, const int K,
+                                     const int m0, const int n0, char *smem)
+{
+    constexpr int TM = C::TM, TN = C::TN, WK = C::WK, D = C::D, SUB = C::SUB, L = C::L, OWN = C::OWN;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nk = K >> 7, ns = (nk + SUB - 1) / SUB;
+
+    // load side: load i of wave w fills block b = w + NW * i of a stage; lane l = 8 * rho + c fetches chunk c ^ sigma of row rho
+    const int8_t *base[L];
+    unsigned roff[L];
+    int sub[L];
+    {
+        const int rho = lane >> 3, c = lane & 7;
+        const int8_t *const xt = qx + (int64_t)m0 * K, *const wt = qw + (int64_t)n0 * K;
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            const int b = wave + C::NW * i;
+            sub[i] = SUB == 1 ? 0 : b / (C::BX + C::BW);
+            const int rb = b - sub[i] * (C::BX + C::BW);
+            const bool isx = rb < C::BX;
+            const int blk = isx ? rb : rb - C::BX;
+            const int sigma = ((blk & 1) << 2) | (rho >> 1);
+            const int row = min(blk * 8 + rho, isx ? M - 1 - m0 : N - 1 - n0);   // rows past the edge repeat the last one
+            base[i] = isx ? xt : wt;
+            roff[i] = (unsigned)row * (unsigned)K + (unsigned)((c ^ sigma) << 4);
+        }
+    }
+    const unsigned lds0 = (unsigned)(uintptr_t)(lptr_t)smem + wave * 1024;
+    auto issue = [&](int s, unsigned buf) {
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            int k = s * SUB + sub[i];
+            if (SUB > 1 && k > nk - 1) k = nk - 1;   // a last stage that is not whole: its steps past K are not used
+            dma16(base[i], roff[i] + (unsigned)(k << 7), lds0 + buf + i * C::NW * 1024);
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < C::PRE; ++s)
+        if (s < ns) issue(s, s * C::STAGE);
+
+    // read side: wave (wm, wn, wk) multiplies K half wk % 2 of step wk / 2 of every stage
+    const int wk = wave % WK, wmn = wave / WK;
+    const int wm = wmn % C::WM, wn = wmn / C::WM;
+    const int r = lane & 15, g = lane >> 4;
+    const char *xa, *wa;
+    {
+        const int rho = r & 7, par = r >> 3, sigma = (par << 2) | (rho >> 1);
+        const int off = par * 1024 + ((8 * rho + ((4 * (wk & 1) + g) ^ sigma)) << 4);
+        const char *st = smem + (wk >> 1) * (C::BX + C::BW) * 1024 + off;
+        xa = st + wm * TM * 2048;
+        wa = st + C::BX * 1024 + wn * TN * 2048;
+    }
+    struct Frags {
+        v4i x[TM], w[TN];
+    };
+    auto fetch = [&](Frags &f, unsigned buf) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) f.x[i] = *reinterpret_cast<const v4i *>(xa + buf + i * 2048);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) f.w[j] = *reinterpret_cast<const v4i *>(wa + buf + j * 2048);
+    };
+
+    // tile f = i * TN + j of a wave is finished by the wave of K slice f / OWN; its scales are requested here
+    const int f0 = wk * OWN;
+    const int mw = m0 + wm * TM * 16, nw = n0 + wn * TN * 16;
+    const bool lo = r < 8;
+    float sxv[OWN];
+    float4 swv[OWN];
+    if constexpr (DEQ) {
+#pragma unroll
+        for (int o = 0; o < OWN; ++o) {
+            const int f = min(f0 + o, C::NF - 1), i = f / TN, j = f % TN;
+            if constexpr (C::PAIR) {   // of an even and an odd tile side by side, see the stores
+                const int m = mw + i * 16 + (o & 1) * 8 + (r & 7), n = nw + (j & ~1) * 16 + (lo ? 0 : 16) + 4 * g;
+                sxv[o] = sx[min(m, M - 1)];
+                if (!(o & 1)) swv[o] = *reinterpret_cast<const float4 *>(sw + min(n, N - 4));
+            } else {
+                const int m = mw + i * 16 + r, n = nw + j * 16 + 4 * g;
+                sxv[o] = sx[min(m, M - 1)];
+                swv[o] = *reinterpret_cast<const float4 *>(sw + min(n, N - 4));
+            }
+        }
+    }
+
+    v4i acc[C::NF];
+#pragma unroll
+    for (int f = 0; f < C::NF; ++f) acc[f] = (v4i){0, 0, 0, 0};
+
+    // at most the loads of the `behind` stages issued after it may be in flight: a stage has landed (this wave's share)
+    auto landed = [&](int behind) {   // wave-uniform
+        if (behind >= D - 1) wait_vm<(D - 1) * L>();
+        else if (D > 2 && behind == D - 2) wait_vm<(D > 2 ? D - 2 : 0) * L>();
+        else if (D > 3 && behind == D - 3) wait_vm<(D > 3 ? D - 3 : 0) * L>();
+        else if (D > 4 && behind == D - 4) wait_vm<(D > 4 ? D - 4 : 0) * L>();
+        else if (D > 5 && behind == D - 5) wait_vm<(D > 5 ? D - 5 : 0) * L>();
+        else wait_vm<0>();
+    };
+    landed(min(ns, C::PRE) - 1);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    Frags fa, fb;
+    fetch(fa, 0);
+#pragma unroll
+    for (int s = C::PRE; s < D; ++s)
+        if (s < ns) issue(s, s * C::STAGE);
+
+    unsigned cur = 0;
+    auto body = [&](auto STEADY, int s, Frags &now, Frags &next) {
+        constexpr bool steady = decltype(STEADY)::value;   // stage s + D exists
+        const unsigned nxt = cur + C::STAGE == D * C::STAGE ? 0 : cur + C::STAGE;
+        // this stage's fragments are in registers, the next stage has landed; behind the barrier both hold for all waves
+        __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0), as an instruction that the compiler's own counting sees
+        if constexpr (steady) wait_vm<(D - 2) * L>();
+        else if (s + 1 < ns) landed(ns - 2 - s);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (steady || s + 1 < ns) fetch(next, nxt);
+        if constexpr (steady) issue(s + D, cur);
+        if (steady || SUB == 1 || s * SUB + (wk >> 1) < nk) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                    acc[i * TN + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(now.w[j], now.x[i], acc[i * TN + j], 0, 0, 0);
+        }
+        cur = nxt;
+    };
+    int s = 0;
+    for (; s + 1 + D < ns; s += 2) {
+        body(std::true_type{}, s, fa, fb);
+        body(std::true_type{}, s + 1, fb, fa);
+    }
+    if (s + D < ns) {
+        body(std::true_type{}, s++, fa, fb);
+        fa = fb;
+    }
+    for (; s < ns; s += 2) {
+        body(std::false_type{}, s, fa, fb);
+        if (s + 1 < ns) body(std::false_type{}, s + 1, fb, fa);
+    }
+    __syncthreads();
+
+    // the K slices meet: every wave hands the tiles it does not finish to the wave that does, [wmn][tile][slice][lane]
+    char *const part = smem + wmn * C::NF * (WK - 1) * 1024 + lane * 16;
+#pragma unroll
+    for (int f = 0; f < C::NF; ++f) {
+        const int own = f / OWN;
+        if (own != wk) *reinterpret_cast<v4i *>(part + (f * (WK - 1) + (wk < own ? wk : wk - 1)) * 1024) = acc[f];
+    }
+    __syncthreads();
+    if (f0 >= C::NF) return;
+    v4i sum[OWN];
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) {
+#pragma unroll
+        for (int w = 0; w < WK; ++w)
+            if (w == wk) sum[o] = acc[w * OWN + o < C::NF ? w * OWN + o : 0];
+        const int f = min(f0 + o, C::NF - 1);
+#pragma unroll
+        for (int w = 0; w < WK - 1; ++w) sum[o] += *reinterpret_cast<const v4i *>(part + (f * (WK - 1) + w) * 1024);
+    }
+    // a lane holds channels 4 g .. + 3 of token r of a tile
+    auto put = [&](const v4i &v, float sxm, const float4 &s4, int m, int n) {
+        if (m >= M || n >= N) return;
+        const int64_t at = (int64_t)m * N + n;
+        if constexpr (DEQ) {
+            float4 o;
+            o.x = ((float)v[0] * sxm) * s4.x;
+            o.y = ((float)v[1] * sxm) * s4.y;
+            o.z = ((float)v[2] * sxm) * s4.z;
+            o.w = ((float)v[3] * sxm) * s4.w;
+            *reinterpret_cast<float4 *>(static_cast<float *>(out) + at) = o;
+        } else {
+            *reinterpret_cast<v4i *>(static_cast<int32_t *>(out) + at) = v;
+        }
+    };
+    if constexpr (C::PAIR) {
+        // two tiles side by side trade halves between lanes r and r ^ 8: one store writes 8 rows x 128 bytes
+#pragma unroll
+        for (int o = 0; o < OWN; o += 2) {
+            const int i = (f0 + o) / TN, j = (f0 + o) % TN;
+            v4i t0, t1;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                t0[e] = ror8(sum[o][e]);
+                t1[e] = ror8(sum[o + 1][e]);
+            }
+            const int m = mw + i * 16 + (r & 7), n = nw + j * 16 + (lo ? 0 : 16) + 4 * g;
+            put(lo ? sum[o] : t1, sxv[o], swv[o], m, n);
+            put(lo ? t0 : sum[o + 1], sxv[o + 1], swv[o], m + 8, n);
+        }
+    } else {
+#pragma unroll
+        for (int o = 0; o < OWN; ++o) {
+            if (f0 + o >= C::NF) break;
+            const int i = (f0 + o) / TN, j = (f0 + o) % TN;
+            put(sum[o], sxv[o], swv[o], mw + i * 16 + r, nw + j * 16 + 4 * g);
+        }
+    }
+}
+
+// grid (8, row tiles, column tiles per XCD): workgroup ids go round robin over the XCDs, so blockIdx.x is the XCD
+template <typename C, bool DEQ>
+__global__ __launch_bounds__(C::TPB) void k_w8a8_deep(const int8_t *__restrict__ qx, const int8_t *__restrict__ qw, int M, int N,
+                                                      int K, int tiles_n, const float *__restrict__ sx,
+                                                      const float *__restrict__ sw, void *__restrict__ out)
+{
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int x = blockIdx.x;
+    const int t = ((tiles_n * x) >> 3) + (int)blockIdx.z;
+    if (t >= (tiles_n * (x + 1)) >> 3) return;
+    tile<C, DEQ>(qx, qw, sx, sw, out, M, N, K, (int)blockIdx.y * C::BM, t * C::BN, smem);
+}
+
+template <typename C, bool DEQ>
+static int32_t launch(const int8_t *qx, const float *sx, const int8_t *qw, const float *sw, void *out, int M, int N, int K,
+                      hipStream_t s)
+{
+    // ragged M and N are the kernel's to clamp; it moves whole 128-byte K steps and stores whole 16-column groups
+    if (M <= 0 || N <= 0 || N % 16 || K < 128 || K % 128) return MI_EINVAL;
+    MI_LDS_OPT_IN((&k_w8a8_deep<C, DEQ>), C::LDS);
+    const int tiles_m = (M + C::BM - 1) / C::BM, tiles_n = (N + C::BN - 1) / C::BN;
+    if (tiles_m > 65535 || tiles_n > 8 * 65535) return MI_ERANGE;
+    const dim3 grid(8, (unsigned)tiles_m, (unsigned)((tiles_n + 7) / 8));
+    hipLaunchKernelGGL((k_w8a8_deep<C, DEQ>), grid, dim3(C::TPB), C::LDS, s, qx, qw, M, N, K, tiles_n, sx, sw, out);
+    return launch_status();
+}
+
+// ---- which tile ----------------------------------------------------------------------------------------------------
+// Time of a launch in microseconds, fitted to 250 shapes (M of 2 to 2048, N of 784 to 28672, K of 1024 to 14336, every
+// tile; graph of back-to-back launches, weights from HBM).  A unit moves (BM + BN) * 128 bytes per K step through its
+// load path at 1.68 ns a row (75 GB/s: the direct-to-LDS loads of eight waves take about 28 clocks a KB, which is more
+// than the matrix instructions of any of these tiles), shares it between the workgroups it holds, and pays 1.4 us plus
+// the tile's outputs per round of tiles.  The memory takes its share on top: bytes at 4.6 TB/s, joined as a 4-norm.
+// Picking by it costs 1.2 % on average over picking the fastest tile of every shape, 12 % at worst.
+struct Tile {
+    int bm, bn, sub, per_cu;
+};
+constexpr Tile TILES[] = {
+    {128, 128, 1, 1}, {128, 64, 1, 1}, {64, 128, 1, 1}, {64, 64, 2, 1}, {64, 32, 2, 1}, {32, 128, 2, 1}, {32, 64, 4, 1},
+    {32, 48, 2, 1},   {32, 32, 4, 1},  {32, 16, 4, 1},  {16, 112, 2, 1}, {16, 64, 4, 1}, {16, 48, 2, 1}, {16, 32, 4, 1},
+    {16, 16, 4, 1},   {128, 64, 1, 2}};
+
+// core time (without the memory's share, which does not depend on the tile) of the best tile
+static float pick(int M, int N, int K, int cus, int *which)
+{
+    const int nk = K >> 7;
+    float best = 0.0f;
+    int at = -1;
+    for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
+        const Tile &t = TILES[i];
+        if (t.bn == 112 && M > 16) continue;   // its weights would be fetched once per row tile
+        const unsigned tiles = (unsigned)((M + t.bm - 1) / t.bm) * (unsigned)((N + t.bn - 1) / t.bn);
+        const unsigned slots = (unsigned)(cus * t.per_cu), full = tiles / slots, rem = tiles - full * slots;
+        const float steps = (float)((nk + t.sub - 1) / t.sub * t.sub) * (float)(t.bm + t.bn) * 0.00168f;
+        const float area = (float)(t.bm * t.bn) * 2.08e-4f;
+        float c = (float)full * (1.36f + (float)t.per_cu * (area + steps));
+        if (rem) c += (full ? 1.14f : 1.0f) * (1.36f + (rem > (unsigned)cus ? 2.0f : 1.0f) * (area + steps));
+        if (at < 0 || c < best) {
+            best = c;
+            at = i;
+        }
+    }
+    *which = at;
+    return best;
+}
+
+}  // namespace deep
+
+// Microseconds that launch_deep would take (see above); *which is the tile to pass on.
+float deep_estimate(int M, int N, int K, int cus, int *which)
+{
+    const float core = deep::pick(M, N, K, cus, which);
+    const float mem = 0.218e-6f * ((float)N * (float)K + (float)M * (float)K + 4.0f * (float)M * (float)N);
+    const float c2 = core * core, m2 = mem * mem;
+    return 0.75f + sqrtf(sqrtf(c2 * c2 + m2 * m2));
+}
+
+template <bool DEQ>
+int32_t launch_deep(int which, const int8_t *qx, const float *sx, const int8_t *qw, const float *sw, int32_t *acc, float *y,
+                    int64_t M64, int64_t N64, int64_t K64, hipStream_t s)
+{
+    using namespace deep;
+    const int M = (int)M64, N = (int)N64, K = (int)K64;
+    void *out = DEQ ? (void *)y : (void *)acc;
+    switch (which) {   // in the order of TILES
+    case 0: return launch<Cfg<4, 4, 2, 2, 2, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 1: return launch<Cfg<4, 2, 2, 2, 2, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 2: return launch<Cfg<2, 4, 2, 2, 2, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 3: return launch<Cfg<2, 4, 2, 1, 4, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 4: return launch<Cfg<2, 2, 2, 1, 4, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 5: return launch<Cfg<2, 4, 1, 2, 4, 4>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 6: return launch<Cfg<2, 4, 1, 1, 8, 3>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 7: return launch<Cfg<2, 3, 1, 1, 4, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 8: return launch<Cfg<2, 2, 1, 1, 8, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 9: return launch<Cfg<2, 1, 1, 1, 8, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 10: return launch<Cfg<1, 7, 1, 1, 4, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 11: return launch<Cfg<1, 4, 1, 1, 8, 4>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 12: return launch<Cfg<1, 3, 1, 1, 4, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 13: return launch<Cfg<1, 2, 1, 1, 8, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 14: return launch<Cfg<1, 1, 1, 1, 8, 7>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 15: return launch<Cfg<4, 2, 2, 2, 2, 3>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    default: return MI_EINVAL;
+    }
+}
+template int32_t launch_deep<true>(int, const int8_t *, const float *, const int8_t *, const float *, int32_t *, float *,
+                                   int64_t, int64_t, int64_t, hipStream_t);
+template int32_t launch_deep<false>(int, const int8_t *, const float *, const int8_t *, const float *, int32_t *, float *,
+                                    int64_t, int64_t, int64_t, hipStream_t);
+
+}  // namespace mi

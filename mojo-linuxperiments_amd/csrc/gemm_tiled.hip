@@ -1,4 +1,4 @@
-// W8A8 contraction for prefill (M > 64): LDS-tiled v_mfma_i32_16x16x64_i8.
+// W8A8 contraction for prefill (sizes that fill the chip with its tiles): LDS-tiled v_mfma_i32_16x16x64_i8.
 //   acc[m,n] = sum_k qx[m,k] * qw[n,k],   y = ((float)acc * sx[m]) * sw[n]
 //
 // Tiling.  A workgroup of four waves (2 x 2) owns a (32*TM) x (32*TN) output
@@ -117,12 +117,11 @@ __device__ __forceinline__ void store4(float *y, int32_t *acc_out, int64_t idx, 
     }
 }
 
-// LDS budget: two activation buffers and, where 160 KB allow it, three weight buffers (a small tile keeps
-// two so that two workgroups share a compute unit)
+// LDS budget: two activation buffers and, where 160 KB allow it, three weight buffers
 template <int TM, int TN>
 struct TiledCfg {
     static constexpr int NBX = 4 * TM, NBW = 4 * TN;
-    static constexpr int NWB = (TM * TN <= 16) ? 2 : ((2 * NBX + 3 * NBW <= 160) ? 3 : 2);
+    static constexpr int NWB = (2 * NBX + 3 * NBW <= 160) ? 3 : 2;
     static constexpr int LDS = (2 * NBX + NWB * NBW) * 1024;
 };
 
@@ -420,37 +419,49 @@ template <bool DEQ>
 int32_t launch_pair(int tm, int tn, const int8_t *, const float *, const int8_t *, const float *, int32_t *, float *, int,
                     int, int, hipStream_t);
 
+// the tile with the least (rounds of tiles over the chip) x (work a compute unit does per round)
+constexpr TileShape SHAPES[] = {{8, 8}, {8, 7}, {8, 6}, {4, 8}};
+static int pick_shape(int M, int N, int cus, int64_t *rounds_out)
+{
+    int pick = 0;
+    double best = 0;
+    for (int i = 0; i < 4; ++i) {
+        const int bm = 32 * SHAPES[i].tm, bn = 32 * SHAPES[i].tn;
+        const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        const int64_t rounds = (tiles + cus - 1) / cus;
+        // smaller wave tiles read more LDS bytes per MFMA
+        const double eff = SHAPES[i].tm * SHAPES[i].tn >= 48 ? 1.0 : 1.08;
+        const double cost = (double)rounds * bm * bn * eff;
+        if (i == 0 || cost < best) { best = cost; pick = i; *rounds_out = rounds; }
+    }
+    return pick;
+}
+
+// Microseconds that launch_tiled takes: a constant and a time per K step and round of each tile, least squares over 150
+// shapes (within 13 %; 28 % where 128 x 256 tiles cover a fraction of the chip, which no choice depends on).
+float tiled_estimate(int M, int N, int K, int cus)
+{
+    int64_t rounds = 1;
+    const int p = pick_shape(M, N, cus, &rounds);
+    constexpr float c0[4] = {2.0f, 6.0f, 1.0f, 6.0f}, c1[4] = {1.85f, 1.67f, 1.53f, 0.80f};
+    return c0[p] + c1[p] * (float)rounds * (float)(K >> 7);
+}
+
 template <bool DEQ>
 int32_t launch_tiled(const int8_t *qx, const float *sx, const int8_t *qw, const float *sw, int32_t *acc, float *y,
                      int64_t M64, int64_t N64, int64_t K64, hipStream_t s)
 {
     const int M = (int)M64, N = (int)N64, K = (int)K64;
-    const int cus = compute_units();
-    // pick the tile with the least (rounds of tiles over the chip) x (work a compute unit does per round)
-    const TileShape shapes[] = {{8, 8}, {8, 7}, {8, 6}, {4, 8}, {4, 4}};
-    int pick = 0;
-    double best = 0;
-    for (int i = 0; i < 5; ++i) {
-        const int bm = 32 * shapes[i].tm, bn = 32 * shapes[i].tn;
-        const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-        const int per_cu = (shapes[i].tm * shapes[i].tn <= 16) ? 2 : 1;  // small tiles fit twice in LDS
-        const int64_t slots = (int64_t)cus * per_cu;
-        const int64_t rounds = (tiles + slots - 1) / slots;
-        // co-resident tiles share the compute unit's MFMA and LDS; smaller wave tiles read more LDS bytes per MFMA
-        const int area = shapes[i].tm * shapes[i].tn;
-        const double eff = area >= 48 ? 1.0 : (area >= 32 ? 1.08 : 1.5);
-        const double cost = (double)rounds * per_cu * bm * bn * eff;
-        if (i == 0 || cost < best) { best = cost; pick = i; }
-    }
+    int64_t rounds;
+    const int pick = pick_shape(M, N, compute_units(), &rounds);
     // one tile per compute unit of a shape that divides evenly: two waves per SIMD on the same wave tile
-    if ((pick == 2 || pick == 3) && M % (32 * shapes[pick].tm) == 0 && N % (32 * shapes[pick].tn) == 0)
-        return launch_pair<DEQ>(shapes[pick].tm, shapes[pick].tn, qx, sx, qw, sw, acc, y, M, N, K, s);
+    if ((pick == 2 || pick == 3) && M % (32 * SHAPES[pick].tm) == 0 && N % (32 * SHAPES[pick].tn) == 0)
+        return launch_pair<DEQ>(SHAPES[pick].tm, SHAPES[pick].tn, qx, sx, qw, sw, acc, y, M, N, K, s);
     switch (pick) {
     case 0: return launch_shape<8, 8, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, s);
     case 1: return launch_shape<8, 7, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, s);
     case 2: return launch_shape<8, 6, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, s);
-    case 3: return launch_shape<4, 8, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, s);
-    default: return launch_shape<4, 4, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, s);
+    default: return launch_shape<4, 8, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, s);
     }
 }
 

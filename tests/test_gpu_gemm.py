@@ -71,6 +71,30 @@ def test_paired_wave_kernel_bit_exact(mi, dev, orc, M, N, K):
     assert np.array_equal(y, orc.dequant(want, sx, sw))
 
 
+@pytest.mark.parametrize("M,N,K", [
+    # every tile of the small-tile kernel on a chip of 256 units, in its order (128 x 128 to 16 x 16, then 128 x 64 two a
+    # unit): fewer stages than its ring holds, a last stage that K fills in part, ragged rows and columns
+    (67, 16464, 128), (714, 4304, 384), (164, 7648, 256), (773, 1664, 512), (63, 16592, 128), (41, 16880, 512),
+    (35, 8368, 128), (75, 5552, 1152), (57, 6448, 128), (361, 1200, 384), (17, 17040, 128), (194, 4384, 1920),
+    (18, 12560, 128), (92, 5056, 768), (59, 4784, 640), (650, 528, 128), (22, 6224, 384), (736, 336, 896),
+    (17, 2448, 384), (714, 112, 1408), (2, 16400, 128), (14, 18640, 1408), (3, 13552, 128), (140, 1776, 384),
+    (3, 10864, 128), (32, 4272, 640), (2, 4272, 384), (15, 5024, 384), (2, 16, 128), (49, 16, 640),
+    (773, 4672, 384), (665, 5440, 384),
+])
+def test_small_tile_kernel_bit_exact(mi, dev, orc, M, N, K):
+    qx, qw = rand_codes(M + N + K, (M, K)), rand_codes(K + 11, (N, K))
+    want = orc.gemm_i8_i32(qx, qw)
+    assert np.array_equal(gpu_gemm_i32(mi, dev, qx, qw), want)
+    g = np.random.default_rng(M)
+    sx, sw = g.uniform(0.01, 1, M).astype(np.float32), g.uniform(0.001, 0.1, N).astype(np.float32)
+    mark = dev.mark()
+    dy = dev.empty((M, N), np.float32)
+    mi.gemm_dequant(dev.upload(qx), dev.upload(sx), dev.upload(qw), dev.upload(sw), dy)
+    y = dev.download(dy)
+    dev.reset_to(mark)
+    assert np.array_equal(y, orc.dequant(want, sx, sw))
+
+
 def test_random_skinny_shapes_bit_exact(mi, dev, orc):
     """Seeded random shapes over every skinny path (1 to 64 tokens, K of 1 to 39 stages, N any multiple of 16 or a
     multiple of 2048, which takes the evenly dealt ring kernels): exact against the oracle."""
