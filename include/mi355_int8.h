@@ -177,8 +177,8 @@ MI_API int32_t mi_fwht_f32(const float *x, float *out, int64_t M, int64_t K,
 
 /* ---- a4 / a5: W8A8 contraction, acc[m,n] = sum_k qx[m,k] * qw[n,k]
  * qx int8 [M,K], qw int8 [N,K] (both K-contiguous), acc int32 [M,N].
- * M <= 64 streams the weights once through a skinny MFMA kernel (decode
- * GEMV); larger M uses the LDS-tiled v_mfma_i32_16x16x64_i8 kernel (prefill).
+ * One token streams the weights through a GEMV; more rows run on v_mfma_i32_16x16x64_i8 in tiles of 16 x 16 to
+ * 256 x 256 by a cost estimate of the shape.
  * K % 128 == 0, N % 16 == 0.  Exact integer arithmetic. */
 MI_API int32_t mi_w8a8_gemm_i32(const int8_t *qx, const int8_t *qw, int32_t *acc,
                                 int64_t M, int64_t N, int64_t K, void *stream);
@@ -188,8 +188,9 @@ MI_API int32_t mi_w8a8_gemm_dequant_f32(const int8_t *qx, const float *sx,
                                         int64_t M, int64_t N, int64_t K, void *stream);
 /* a4 for several contractions at once: ONE launch whose workgroups (one per compute unit) walk a list of 256 x 256
  * output tiles drawn from every problem of the batch, so that no problem's tile count has to divide by the number
- * of compute units, and no launch gap or first memory round trip lies between the problems.  No upstream
- * counterpart.  A batch is made once for a list of shapes
+ * of compute units, and no launch gap or first memory round trip lies between the problems.  Where such a list would be
+ * badly balanced (few tiles, or a few of much longer K) some or all problems run in smaller tiles instead, in a launch
+ * of their own in front of it: which is decided when the batch is made.  No upstream counterpart.  A batch is made once for a list of shapes
  * (mnk int64 [n][3] = M, N, K per problem; n <= 8; M >= 256, N >= 256, N % 16 == 0, K % 128 == 0, K >= 384, 127 * 127 * K < 2^31): the tile lists
  * are computed on the host and copied (synchronously) into `plan`, device memory of the caller of at least
  * mi_gemm_batch_plan_bytes(mnk, n) bytes that must stay untouched while the batch lives.  A run takes the operands

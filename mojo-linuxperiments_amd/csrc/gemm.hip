@@ -3,6 +3,7 @@
 #include <atomic>
 
 #include "common.h"
+#include "gemm_deep.h"
 
 namespace mi {
 template <bool DEQ>
@@ -12,10 +13,6 @@ template <bool DEQ>
 int32_t launch_tiled(const int8_t *, const float *, const int8_t *, const float *, int32_t *, float *, int64_t,
                      int64_t, int64_t, hipStream_t);
 
-template <bool DEQ>
-int32_t launch_deep(int, const int8_t *, const float *, const int8_t *, const float *, int32_t *, float *, int64_t,
-                    int64_t, int64_t, hipStream_t);
-float deep_estimate(int M, int N, int K, int cus, int *which);
 float tiled_estimate(int M, int N, int K, int cus);
 
 int32_t launch_linear_fused(const float *, const int8_t *, const float *, float *, int8_t *, float *, int64_t, int64_t,

@@ -22,8 +22,11 @@
 // XORed with sigma(row, block parity), free of bank conflicts for the fragment reads.  Operand A is the weights.
 //
 #include <algorithm>
+#include <utility>
+#include <vector>
 
 #include "common.h"
+#include "gemm_deep.h"
 
 namespace mi {
 namespace deep {
@@ -282,6 +285,43 @@ __global__ __launch_bounds__(C::TPB) void k_w8a8_deep(const int8_t *__restrict__
     tile<C, DEQ>(qx, qw, sx, sw, out, M, N, K, (int)blockIdx.y * C::BM, t * C::BN, smem);
 }
 
+// several contractions in one launch, workgroups of the first problem first
+struct Batch {
+    DeepProblem p[DEEP_MAX];
+    int n;
+};
+template <typename C, bool DEQ>
+__global__ __launch_bounds__(C::TPB) void k_w8a8_deep_batch(const Batch b)
+{
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    int pi = 0;
+#pragma unroll
+    for (int k = 1; k < DEEP_MAX; ++k)
+        if (k < b.n && (int)blockIdx.x >= b.p[k].first) pi = k;
+    const DeepProblem &P = b.p[pi];
+    const int id = (int)blockIdx.x - P.first, x = id & 7, li = id >> 3;   // P.first % 8 == 0: x is the XCD
+    const int tiles_m = (P.M + C::BM - 1) / C::BM, tiles_n = (P.N + C::BN - 1) / C::BN;
+    const int t = ((tiles_n * x) >> 3) + li / tiles_m;
+    if (t >= (tiles_n * (x + 1)) >> 3) return;
+    tile<C, DEQ>(P.qx, P.qw, P.sx, P.sw, P.out, P.M, P.N, P.K, li % tiles_m * C::BM, t * C::BN, smem);
+}
+
+template <typename C, bool DEQ>
+static int32_t launch_batch(Batch &b, hipStream_t s)
+{
+    int64_t grid = 0;
+    for (int i = 0; i < b.n; ++i) {
+        DeepProblem &p = b.p[i];
+        if (p.M <= 0 || p.N <= 0 || p.N % 16 || p.K < 128 || p.K % 128) return MI_EINVAL;
+        p.first = (int)grid;
+        grid += (int64_t)((p.M + C::BM - 1) / C::BM) * (((p.N + C::BN - 1) / C::BN + 7) / 8) * 8;
+        if (grid > 0x7fffffff / C::TPB) return MI_ERANGE;
+    }
+    MI_LDS_OPT_IN((&k_w8a8_deep_batch<C, DEQ>), C::LDS);
+    hipLaunchKernelGGL((k_w8a8_deep_batch<C, DEQ>), dim3((unsigned)grid), dim3(C::TPB), C::LDS, s, b);
+    return launch_status();
+}
+
 template <typename C, bool DEQ>
 static int32_t launch(const int8_t *qx, const float *sx, const int8_t *qw, const float *sw, void *out, int M, int N, int K,
                       hipStream_t s)
@@ -377,5 +417,70 @@ template int32_t launch_deep<true>(int, const int8_t *, const float *, const int
                                    int64_t, int64_t, int64_t, hipStream_t);
 template int32_t launch_deep<false>(int, const int8_t *, const float *, const int8_t *, const float *, int32_t *, float *,
                                     int64_t, int64_t, int64_t, hipStream_t);
+
+// ---- several contractions of at least 256 rows in one launch (a part of a batch, see gemm_list.hip)
+// Time of a workgroup on a tile, as above; the tiles go to the units as these come free, longest K first.  A launch of
+// several rounds takes 1.25 times the sum of its tiles (measured 147 us where the sum says 115 and 83 where it says 66).
+float deep_batch_estimate(const int64_t *mnk, const int *idx, int n, int cus, int *which)
+{
+    using namespace deep;
+    constexpr int TRY[] = {0, 1, 3};
+    float best = -1.0f;
+    double mem = 0.0;
+    for (int i = 0; i < n; ++i) {
+        const int64_t M = mnk[3 * idx[i]], N = mnk[3 * idx[i] + 1], K = mnk[3 * idx[i] + 2];
+        mem += 0.218e-6 * ((double)N * K + (double)M * K + 4.0 * M * N);
+    }
+    std::vector<std::pair<float, int64_t>> free;   // when units are free, and how many
+    for (int t : TRY) {
+        const Tile &T = TILES[t];
+        free.assign(1, {0.0f, cus});
+        float end = 0.0f;
+        int64_t count = 0;
+        for (int i = 0; i < n; ++i) {
+            const int64_t M = mnk[3 * idx[i]], N = mnk[3 * idx[i] + 1], nk = mnk[3 * idx[i] + 2] >> 7;
+            int64_t tiles = ((M + T.bm - 1) / T.bm) * ((N + T.bn - 1) / T.bn);
+            const float cost = 1.36f + (float)(T.bm * T.bn) * 2.08e-4f + (float)((nk + T.sub - 1) / T.sub * T.sub) * (float)(T.bm + T.bn) * 0.00168f;
+            count += tiles;
+            while (tiles > 0) {   // as many tiles as units are free first, all at once
+                const size_t at = (size_t)(std::min_element(free.begin(), free.end()) - free.begin());
+                const int64_t k = std::min(tiles, free[at].second);
+                const float done = free[at].first + cost;
+                tiles -= k;
+                if (k == free[at].second) free[at].first = done;
+                else {
+                    free[at].second -= k;
+                    free.push_back({done, k});
+                }
+                end = std::max(end, done);
+            }
+        }
+        if (count > cus) end *= 1.25f;
+        if (best < 0.0f || end < best) {
+            best = end;
+            *which = t;
+        }
+    }
+    const float m = (float)mem, c2 = best * best, m2 = m * m;
+    return 0.75f + sqrtf(sqrtf(c2 * c2 + m2 * m2));
+}
+
+template <bool DEQ>
+int32_t launch_deep_batch(int which, const DeepProblem *p, int n, hipStream_t s)
+{
+    using namespace deep;
+    if (n < 1 || n > DEEP_MAX) return MI_EINVAL;
+    Batch b = {};
+    for (int i = 0; i < n; ++i) b.p[i] = p[i];
+    b.n = n;
+    switch (which) {
+    case 0: return launch_batch<Cfg<4, 4, 2, 2, 2, 5>, DEQ>(b, s);
+    case 1: return launch_batch<Cfg<4, 2, 2, 2, 2, 6>, DEQ>(b, s);
+    case 3: return launch_batch<Cfg<2, 4, 2, 1, 4, 5>, DEQ>(b, s);
+    default: return MI_EINVAL;
+    }
+}
+template int32_t launch_deep_batch<true>(int, const DeepProblem *, int, hipStream_t);
+template int32_t launch_deep_batch<false>(int, const DeepProblem *, int, hipStream_t);
 
 }  // namespace mi

@@ -50,6 +50,7 @@
 #include <vector>
 
 #include "common.h"
+#include "gemm_deep.h"
 #include "gemm_pair_ops.h"
 
 #ifndef MI_STORE_MOD
@@ -613,6 +614,76 @@ static int64_t build_lists(const int64_t *mnk, int n, int cus, std::vector<v4i> 
 
 using LC = Cfg;
 
+// ---- how a batch is run: the problems of `tiled` by the list kernel, the others by the small-tile kernel in a second
+// launch.  A list of few tiles is badly balanced, above all where their K differ: 509 tokens through the four prefill
+// projections are 304 tiles of which 32 are 3.5 times as long as the others, and the launch lasts as long as one
+// of those and its start (166 us where the mean workgroup is busy for 80).  The small tiles move twice the bytes per result,
+// but hundreds of them level out.  Estimates: a list's longest sum of tile costs at 1.36 us a unit (measured from 2048
+// rows through the four projections, 252 units in 340 us, down to one tile a workgroup) and deep_batch_estimate.
+// Measured, weights from HBM, us before -> after: the four projections with 256 rows 150 -> 82, with 384 rows 159 -> 121,
+// with 509 rows 159 -> 134 (gate and up tiled, qkv and down in small tiles); 2048 -> 3072, 2048, 11008 and
+// 11008 -> 2048 with 512 rows 102 -> 45.
+struct Split {
+    int n_tiled = 0, n_deep = 0;
+    int tiled[MAX_PROBLEMS], deep[MAX_PROBLEMS];
+    int which = 0;   // tile of the second launch
+};
+
+// the longest workgroup of a list, in tile costs: blocks of equal K dealt longest first to the least loaded XCD
+static int64_t list_load(const int64_t *mnk, const int *idx, int n, int cus)
+{
+    const int nx = (cus % 8 == 0) ? 8 : 1, slots = cus / nx;
+    int64_t load[8] = {};
+    for (int i = 0; i < n;) {
+        const int64_t K = mnk[3 * idx[i] + 2];
+        int64_t tiles = 0;
+        for (; i < n && mnk[3 * idx[i] + 2] == K; ++i)
+            tiles += ((mnk[3 * idx[i]] + LC::BM - 1) / LC::BM) * ((mnk[3 * idx[i] + 1] + LC::BN - 1) / LC::BN);
+        for (; tiles > 0; tiles -= slots) *std::min_element(load, load + nx) += tile_cost(K);
+    }
+    return *std::max_element(load, load + nx);
+}
+
+static Split split_batch(const int64_t *mnk, int n, int cus)
+{
+    int order[MAX_PROBLEMS];
+    for (int p = 0; p < n; ++p) order[p] = p;
+    std::stable_sort(order, order + n, [&](int a, int b) { return mnk[3 * a + 2] > mnk[3 * b + 2]; });
+    Split best;
+    best.n_tiled = n;
+    for (int i = 0; i < n; ++i) best.tiled[i] = order[i];
+    double sum = 0.0, tiles = 0.0;
+    for (int p = 0; p < n; ++p) {
+        const double t = (double)((mnk[3 * p] + LC::BM - 1) / LC::BM) * (double)((mnk[3 * p + 1] + LC::BN - 1) / LC::BN);
+        tiles += t;
+        sum += t * tile_cost(mnk[3 * p + 2]);
+    }
+    const int64_t load = list_load(mnk, best.tiled, n, cus);
+    // nothing to level out (the small tiles cost 1.65 times as much), or so many tiles that a list is level
+    if ((double)load * cus < 1.2 * sum || tiles > 8.0 * cus) return best;
+    // the estimates are good to a tenth: what they promise has to be more
+    float t_best = 0.9f * (3.0f + 1.36f * (float)load);
+    for (int mask = 1; mask < (1 << n); ++mask) {   // the problems of the second launch
+        Split s;
+        for (int i = 0; i < n; ++i) {
+            if (mask >> i & 1) s.deep[s.n_deep++] = order[i];
+            else s.tiled[s.n_tiled++] = order[i];
+        }
+        // of equal problems only a leading run goes over: one order of them is enough
+        bool skip = false;
+        for (int i = 1; i < n; ++i)
+            if ((mask >> i & 1) && !(mask >> (i - 1) & 1) && !memcmp(mnk + 3 * order[i], mnk + 3 * order[i - 1], 3 * sizeof(int64_t))) skip = true;
+        if (skip) continue;
+        float t = deep_batch_estimate(mnk, s.deep, s.n_deep, cus, &s.which);
+        if (s.n_tiled) t += 5.0f + 1.36f * (float)list_load(mnk, s.tiled, s.n_tiled, cus);
+        if (t < t_best) {
+            t_best = t;
+            best = s;
+        }
+    }
+    return best;
+}
+
 static int32_t check_shapes(const int64_t *mnk, int32_t n)
 {
     if (!mnk || n < 1 || n > MAX_PROBLEMS) return MI_EINVAL;
@@ -635,7 +706,8 @@ struct mi_gemm_batch {
     int32_t device;
     int32_t grid, per_wg;
     int64_t mnk[3 * list::MAX_PROBLEMS];
-    const v4i *lists;   // device memory of the caller
+    list::Split split;
+    const v4i *lists;   // device memory of the caller; entries count problems in the order of split.tiled
 };
 
 extern "C" int64_t mi_gemm_batch_plan_bytes(const int64_t *mnk, int32_t n)
@@ -672,18 +744,31 @@ extern "C" int32_t mi_gemm_batch_create(const int64_t *mnk, int32_t n, void *pla
     std::vector<v4i> lists;
     int per_wg = 0;
     const int cus = compute_units();
-    const int64_t bytes = list::build_lists<list::LC::BM, list::LC::BN>(mnk, n, cus, &lists, &per_wg);
-    if (bytes < 0) return (int32_t)bytes;
-    if (plan_bytes < bytes) return MI_ENOSPC;
+    const int64_t whole = list::build_lists<list::LC::BM, list::LC::BN>(mnk, n, cus, &lists, &per_wg);
+    if (whole < 0) return (int32_t)whole;
+    if (plan_bytes < whole) return MI_ENOSPC;
+    list::Split split = list::split_batch(mnk, n, cus);
+    int64_t bytes = whole;
+    if (split.n_deep) {
+        int64_t sub[3 * list::MAX_PROBLEMS];
+        for (int i = 0; i < split.n_tiled; ++i)
+            for (int k = 0; k < 3; ++k) sub[3 * i + k] = mnk[3 * split.tiled[i] + k];
+        bytes = 0;
+        if (split.n_tiled) bytes = list::build_lists<list::LC::BM, list::LC::BN>(sub, split.n_tiled, cus, &lists, &per_wg);
+        if (bytes < 0 || bytes > plan_bytes) return MI_ENOSPC;
+    } else {
+        for (int i = 0; i < n; ++i) split.tiled[i] = i;
+    }
     int dev = 0;
     MI_HIP(hipGetDevice(&dev));
-    MI_HIP(hipMemcpy(plan, lists.data(), (size_t)bytes, hipMemcpyHostToDevice));   // returns when the list is in place
+    if (bytes) MI_HIP(hipMemcpy(plan, lists.data(), (size_t)bytes, hipMemcpyHostToDevice));   // returns when the list is in place
     mi_gemm_batch *b = new (std::nothrow) mi_gemm_batch();
     if (!b) return MI_ENOMEM;
     b->n = n;
     b->device = dev;
     b->grid = cus;
     b->per_wg = per_wg;
+    b->split = split;
     for (int i = 0; i < 3 * n; ++i) b->mnk[i] = mnk[i];
     b->lists = static_cast<const v4i *>(plan);
     *out = b;
@@ -701,12 +786,28 @@ template <bool DEQ>
 static int32_t batch_run(mi_gemm_batch *b, const mi_gemm_problem *p, void *stream)
 {
     if (!b || !p) return MI_EINVAL;
-    list::Batch bt = {};
     for (int i = 0; i < b->n; ++i) {
         const mi_gemm_problem &g = p[i];
         if (g.M != b->mnk[3 * i] || g.N != b->mnk[3 * i + 1] || g.K != b->mnk[3 * i + 2]) return MI_EINVAL;
         if (!g.qx || !g.qw || !g.out || !aligned16(g.qx) || !aligned16(g.qw) || !aligned16(g.out)) return MI_EINVAL;
         if (DEQ && (!g.sx || !g.sw || !aligned4(g.sx) || !aligned4(g.sw))) return MI_EINVAL;
+    }
+    int dev = -1;
+    MI_HIP(hipGetDevice(&dev));
+    if (dev != b->device) return MI_EINVAL;   // the list lives in that device's memory
+    const list::Split &sp = b->split;
+    if (sp.n_deep) {
+        DeepProblem d[list::MAX_PROBLEMS];
+        for (int i = 0; i < sp.n_deep; ++i) {
+            const mi_gemm_problem &g = p[sp.deep[i]];
+            d[i] = {g.qx, g.qw, g.sx, g.sw, g.out, (int)g.M, (int)g.N, (int)g.K, 0};
+        }
+        const int32_t rc = launch_deep_batch<DEQ>(sp.which, d, sp.n_deep, as_stream(stream));
+        if (rc || !sp.n_tiled) return rc;
+    }
+    list::Batch bt = {};
+    for (int i = 0; i < sp.n_tiled; ++i) {
+        const mi_gemm_problem &g = p[sp.tiled[i]];
         list::Problem &d = bt.p[i];
         d.qx = g.qx;
         d.qw = g.qw;
@@ -717,9 +818,6 @@ static int32_t batch_run(mi_gemm_batch *b, const mi_gemm_problem *p, void *strea
         d.N = (int)g.N;
         d.K = (int)g.K;
     }
-    int dev = -1;
-    MI_HIP(hipGetDevice(&dev));
-    if (dev != b->device) return MI_EINVAL;   // the list lives in that device's memory
     MI_LDS_OPT_IN((&list::k_w8a8_list<DEQ>), list::LC::LDS);
     hipLaunchKernelGGL((list::k_w8a8_list<DEQ>), dim3((unsigned)b->grid), dim3(512), list::LC::LDS,
                        as_stream(stream), bt, b->lists, b->per_wg);

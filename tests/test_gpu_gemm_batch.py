@@ -58,6 +58,32 @@ def test_batch_accumulators_bit_exact(mi, dev, orc, shapes):
     dev.reset_to(mark)
 
 
+# batches whose list would be badly balanced: a long K in small tiles beside two round ones in a list (two launches), and
+# batches that the small tiles take whole, in one launch of 64 x 64, 128 x 64 and 128 x 128 tiles
+@pytest.mark.parametrize("shapes", [
+    [(509, 14336, 2048), (509, 2048, 7168), (509, 14336, 2048), (509, 3072, 2048)],
+    [(300, 2048, 896), (256, 1040, 2176)],
+    [(300, 3072, 2048), (300, 2048, 2048)],
+    [(512, 3072, 2048), (512, 2048, 2048), (512, 2048, 5504)],
+])
+def test_batch_with_small_tiles(mi, dev, orc, shapes):
+    mark = dev.mark()
+    batch = mi.GemmBatch(dev, shapes)
+    ops, host = make_ops(dev, shapes, 900 + len(shapes), np.float32)
+    acc = [dev.empty((M, N), np.int32) for M, N, K in shapes]
+    for b in acc + [o[4] for o in ops]:   # poison: every element must be written
+        mi.check(mi.lib.mi_fill_u32(b.ptr, 0x7F7F7F7F, b.nbytes // 4, None))
+    batch.run_i32([(qx, None, qw, None, a) for (qx, _, qw, _, _), a in zip(ops, acc)])
+    batch.run_f32(ops)
+    dev.sync()
+    for o, a, (qx, sx, qw, sw) in zip(ops, acc, host):
+        want = orc.gemm_i8_i32(qx, qw)
+        assert np.array_equal(dev.download(a), want)
+        assert np.array_equal(dev.download(o[4]), orc.dequant(want, sx, sw))
+    batch.destroy()
+    dev.reset_to(mark)
+
+
 @pytest.mark.parametrize("shapes", [
     [(256, 256, 384)],
     [(300, 272, 512)],
