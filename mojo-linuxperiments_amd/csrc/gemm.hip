@@ -57,7 +57,7 @@ int32_t gemm_dispatch(const int8_t *qx, const float *sx, const int8_t *qw, const
     if (M <= 64 || deep < tiled_estimate((int)M, (int)N, (int)K, cus)) {
         const int32_t rc = y ? launch_deep<true>(which, qx, sx, qw, sw, nullptr, y, M, N, K, s)
                              : launch_deep<false>(which, qx, nullptr, qw, nullptr, acc, nullptr, M, N, K, s);
-        if (rc != MI_ERANGE) return rc;   // more tiles than a three-dimensional grid holds
+        if (rc != MI_ERANGE) return rc;   // more tiles than it counts
     }
     return y ? launch_tiled<true>(qx, sx, qw, sw, nullptr, y, M, N, K, s)
              : launch_tiled<false>(qx, nullptr, qw, nullptr, acc, nullptr, M, N, K, s);

@@ -10,7 +10,9 @@ struct DeepProblem {
     const float *sx, *sw;
     void *out;
     int M, N, K;
-    int first;   // first workgroup, filled in by the launch
+    // filled in by the launch: first workgroup, tiles, row tiles and what divides by their number
+    int first, tiles, tiles_m;
+    unsigned magic;
 };
 
 // microseconds that the launch would take; *which is the tile to pass on

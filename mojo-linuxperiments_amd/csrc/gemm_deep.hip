@@ -1,11 +1,13 @@
 // W8A8 contraction for everything between one token and the sizes that fill the chip with 256-wide tiles:
 //   acc[m,n] = sum_k qx[m,k] * qw[n,k],   y = ((float)acc * sx[m]) * sw[n]
 //
-// One workgroup of eight waves per tile, the tile chosen from sixteen (16 x 16 to 128 x 128) so that every compute unit
-// has one, and one load stream per workgroup: stages of 128 to 512 bytes of K go straight to LDS through a ring of D
-// buffers, D - 1 stages in flight, one barrier a stage.  The barrier of stage s says that stage s + 1 has landed and
+// One workgroup of four or eight waves per tile, the tile chosen from ten (16 x 16 to 128 x 128) so that every compute
+// unit has one, and one load stream per workgroup: stages of 128 to 512 bytes of K go straight to LDS through a ring of D
+// buffers, D - 1 stages in flight, one barrier a stage.  All but the largest tiles take at most half of a unit's LDS:
+// where there are tiles enough two workgroups share a unit and hide each other's first loads and last stores (16 rows,
+// 4096 -> 28672 inside a decode step: 24.3 instead of 27.2 us).  The barrier of stage s says that stage s + 1 has landed and
 // that everybody holds its fragments of stage s in registers; behind it a wave requests the fragments of stage s + 1,
-// the loads of stage s + D into the buffer just freed, and multiplies stage s.  Small tiles leave most of the eight
+// the loads of stage s + D into the buffer just freed, and multiplies stage s.  Small tiles leave most
 // waves without rows of their own, so the waves split K inside a stage (WK slices of 64 bytes) and meet once, through
 // LDS, at the tile's end; every wave finishes an equal share of the matrix-instruction tiles.
 //
@@ -15,8 +17,9 @@
 // those 900.  Measured and equal or slower: loads through registers and ds_write, 16 waves, the loads spread between the
 // matrix instructions, another K phase per workgroup, rows of 256 bytes.  So the tile decides: rows loaded per result.
 //
-// Measured (us a call, us before): 16 x 4096 -> 14336 12.3 (14.3), 32 x 4096 -> 4096 5.4 (7.2), 64 x 4096 -> 14336 15.3
-// (27.2), 200 x 4096 -> 14336 24.3 (34.3), 256 x 14336 -> 4096 34.5 (97), 512 x 4096 -> 4096 14.2 (28.3).
+// Measured (us a call, and with the LDS-tiled and ring kernels before): 16 x 4096 -> 14336 12.0 (14.3), 32 x 4096 -> 4096
+// 5.2 (7.2), 64 x 4096 -> 14336 15.1 (27.2), 200 x 4096 -> 14336 24.3 (34.3), 256 x 14336 -> 4096 34.5 (97),
+// 512 x 4096 -> 4096 14.3 (28.3).
 //
 // LDS layout, swizzle and shape of the loads are those of gemm_tiled.hip: 1 KB blocks of 8 rows x 128 bytes, chunk position
 // XORed with sigma(row, block parity), free of bank conflicts for the fragment reads.  Operand A is the weights.
@@ -272,17 +275,39 @@ __device__ __forceinline__ void tile(const int8_t *__restrict__ qx, const int8_t
     }
 }
 
-// grid (8, row tiles, column tiles per XCD): workgroup ids go round robin over the XCDs, so blockIdx.x is the XCD
+// Tile of workgroup `id` of a problem (ids go round robin over the XCDs): an XCD takes an eighth of the tiles, column by
+// column, so that the row tiles of a weight column meet in its L2 and no XCD has a tile more than another.
+// magic = ceil(2^32 / tiles_m) divides exactly: tiles * tiles_m < 2^32.
+__device__ __forceinline__ bool tile_of(int id, int tiles, int tiles_m, unsigned magic, int *tm, int *tn)
+{
+    const unsigned x = (unsigned)id & 7, t = (((unsigned)tiles * x) >> 3) + ((unsigned)id >> 3);
+    *tn = tiles_m == 1 ? (int)t : (int)__umulhi(t, magic);
+    *tm = (int)t - *tn * tiles_m;
+    return t < ((unsigned)tiles * (x + 1)) >> 3;
+}
+
 template <typename C, bool DEQ>
 __global__ __launch_bounds__(C::TPB) void k_w8a8_deep(const int8_t *__restrict__ qx, const int8_t *__restrict__ qw, int M, int N,
-                                                      int K, int tiles_n, const float *__restrict__ sx,
-                                                      const float *__restrict__ sw, void *__restrict__ out)
+                                                      int K, int tiles, int tiles_m, unsigned magic,
+                                                      const float *__restrict__ sx, const float *__restrict__ sw,
+                                                      void *__restrict__ out)
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int x = blockIdx.x;
-    const int t = ((tiles_n * x) >> 3) + (int)blockIdx.z;
-    if (t >= (tiles_n * (x + 1)) >> 3) return;
-    tile<C, DEQ>(qx, qw, sx, sw, out, M, N, K, (int)blockIdx.y * C::BM, t * C::BN, smem);
+    int tm, tn;
+    if (!tile_of((int)blockIdx.x, tiles, tiles_m, magic, &tm, &tn)) return;
+    tile<C, DEQ>(qx, qw, sx, sw, out, M, N, K, tm * C::BM, tn * C::BN, smem);
+}
+
+// false: more tiles than the kernel's arithmetic covers
+template <typename C>
+static bool tile_grid(int M, int N, int *tiles, int *tiles_m, unsigned *magic)
+{
+    const int64_t tm = ((int64_t)M + C::BM - 1) / C::BM, all = tm * (((int64_t)N + C::BN - 1) / C::BN);
+    if (all > (1 << 24) || all * tm >= (1ll << 32)) return false;
+    *tiles = (int)all;
+    *tiles_m = (int)tm;
+    *magic = (unsigned)(((1ull << 32) + (unsigned long long)tm - 1) / (unsigned long long)tm);
+    return true;
 }
 
 // several contractions in one launch, workgroups of the first problem first
@@ -299,11 +324,9 @@ __global__ __launch_bounds__(C::TPB) void k_w8a8_deep_batch(const Batch b)
     for (int k = 1; k < DEEP_MAX; ++k)
         if (k < b.n && (int)blockIdx.x >= b.p[k].first) pi = k;
     const DeepProblem &P = b.p[pi];
-    const int id = (int)blockIdx.x - P.first, x = id & 7, li = id >> 3;   // P.first % 8 == 0: x is the XCD
-    const int tiles_m = (P.M + C::BM - 1) / C::BM, tiles_n = (P.N + C::BN - 1) / C::BN;
-    const int t = ((tiles_n * x) >> 3) + li / tiles_m;
-    if (t >= (tiles_n * (x + 1)) >> 3) return;
-    tile<C, DEQ>(P.qx, P.qw, P.sx, P.sw, P.out, P.M, P.N, P.K, li % tiles_m * C::BM, t * C::BN, smem);
+    int tm, tn;   // (P.first % 8 == 0)
+    if (!tile_of((int)blockIdx.x - P.first, P.tiles, P.tiles_m, P.magic, &tm, &tn)) return;
+    tile<C, DEQ>(P.qx, P.qw, P.sx, P.sw, P.out, P.M, P.N, P.K, tm * C::BM, tn * C::BN, smem);
 }
 
 template <typename C, bool DEQ>
@@ -313,8 +336,9 @@ static int32_t launch_batch(Batch &b, hipStream_t s)
     for (int i = 0; i < b.n; ++i) {
         DeepProblem &p = b.p[i];
         if (p.M <= 0 || p.N <= 0 || p.N % 16 || p.K < 128 || p.K % 128) return MI_EINVAL;
+        if (!tile_grid<C>(p.M, p.N, &p.tiles, &p.tiles_m, &p.magic)) return MI_ERANGE;
         p.first = (int)grid;
-        grid += (int64_t)((p.M + C::BM - 1) / C::BM) * (((p.N + C::BN - 1) / C::BN + 7) / 8) * 8;
+        grid += (p.tiles + 7) / 8 * 8;
         if (grid > 0x7fffffff / C::TPB) return MI_ERANGE;
     }
     MI_LDS_OPT_IN((&k_w8a8_deep_batch<C, DEQ>), C::LDS);
@@ -329,43 +353,47 @@ static int32_t launch(const int8_t *qx, const float *sx, const int8_t *qw, const
     // ragged M and N are the kernel's to clamp; it moves whole 128-byte K steps and stores whole 16-column groups
     if (M <= 0 || N <= 0 || N % 16 || K < 128 || K % 128) return MI_EINVAL;
     MI_LDS_OPT_IN((&k_w8a8_deep<C, DEQ>), C::LDS);
-    const int tiles_m = (M + C::BM - 1) / C::BM, tiles_n = (N + C::BN - 1) / C::BN;
-    if (tiles_m > 65535 || tiles_n > 8 * 65535) return MI_ERANGE;
-    const dim3 grid(8, (unsigned)tiles_m, (unsigned)((tiles_n + 7) / 8));
-    hipLaunchKernelGGL((k_w8a8_deep<C, DEQ>), grid, dim3(C::TPB), C::LDS, s, qx, qw, M, N, K, tiles_n, sx, sw, out);
+    int tiles, tiles_m;
+    unsigned magic;
+    if (!tile_grid<C>(M, N, &tiles, &tiles_m, &magic)) return MI_ERANGE;
+    hipLaunchKernelGGL((k_w8a8_deep<C, DEQ>), dim3((unsigned)(tiles + 7) / 8 * 8), dim3(C::TPB), C::LDS, s, qx, qw, M, N, K,
+                       tiles, tiles_m, magic, sx, sw, out);
     return launch_status();
 }
 
 // ---- which tile ----------------------------------------------------------------------------------------------------
-// Time of a launch in microseconds, fitted to 250 shapes (M of 2 to 2048, N of 784 to 28672, K of 1024 to 14336, every
-// tile; graph of back-to-back launches, weights from HBM).  A unit moves (BM + BN) * 128 bytes per K step through its
-// load path at 1.68 ns a row (75 GB/s: the direct-to-LDS loads of eight waves take about 28 clocks a KB, which is more
-// than the matrix instructions of any of these tiles), shares it between the workgroups it holds, and pays 1.4 us plus
-// the tile's outputs per round of tiles.  The memory takes its share on top: bytes at 4.6 TB/s, joined as a 4-norm.
-// Picking by it costs 1.2 % on average over picking the fastest tile of every shape, 12 % at worst.
+// Time of a launch in microseconds, fitted to 250 shapes (M of 2 to 1024, N of 784 to 28672, K of 1024 to 14336) times
+// every tile, each measured behind the quantizer that feeds it and with weights from HBM.  A unit moves (BM + BN) * 128
+// bytes per K step through its load path at 1.69 ns a row (76 GB/s: the direct-to-LDS loads of a workgroup take about
+// 28 clocks a KB, which is more than the matrix instructions of any of these tiles), 1.82 instead of 2 times as long
+// for two workgroups side by side, and pays 0.7 us plus the tile's outputs per round of tiles.  The memory's share,
+// bytes at 5 TB/s, is joined as a 4-norm: it does not depend on the tile.  Picking by it costs 0.5 % on average over
+// picking the fastest tile of every shape, 15 % at worst.
 struct Tile {
     int bm, bn, sub, per_cu;
 };
-constexpr Tile TILES[] = {
-    {128, 128, 1, 1}, {128, 64, 1, 1}, {64, 128, 1, 1}, {64, 64, 2, 1}, {64, 32, 2, 1}, {32, 128, 2, 1}, {32, 64, 4, 1},
-    {32, 48, 2, 1},   {32, 32, 4, 1},  {32, 16, 4, 1},  {16, 112, 2, 1}, {16, 64, 4, 1}, {16, 48, 2, 1}, {16, 32, 4, 1},
-    {16, 16, 4, 1},   {128, 64, 1, 2}};
+constexpr Tile TILES[] = {{128, 128, 1, 1}, {128, 64, 1, 1}, {64, 64, 1, 2}, {64, 32, 1, 2}, {32, 48, 2, 1},
+                          {32, 32, 2, 2},   {32, 16, 2, 2},  {16, 48, 2, 2}, {16, 32, 2, 2}, {16, 16, 4, 2}};
+constexpr float PER_LAUNCH = 1.72f, PER_ROUND = 0.68f, PER_OUTPUT = 2.34e-4f, PER_ROW_STEP = 0.00169f, BESIDE = 0.82f,
+                LAST_ROUND = 1.04f, PER_MB = 0.202f;
 
-// core time (without the memory's share, which does not depend on the tile) of the best tile
+static float alone(const Tile &t, int64_t nk)   // a tile on a unit of its own, without PER_ROUND
+{
+    return (float)(t.bm * t.bn) * PER_OUTPUT + (float)((nk + t.sub - 1) / t.sub * t.sub) * (float)(t.bm + t.bn) * PER_ROW_STEP;
+}
+
+// core time (without the memory's share) of the best tile
 static float pick(int M, int N, int K, int cus, int *which)
 {
-    const int nk = K >> 7;
     float best = 0.0f;
     int at = -1;
     for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
         const Tile &t = TILES[i];
-        if (t.bn == 112 && M > 16) continue;   // its weights would be fetched once per row tile
-        const unsigned tiles = (unsigned)((M + t.bm - 1) / t.bm) * (unsigned)((N + t.bn - 1) / t.bn);
-        const unsigned slots = (unsigned)(cus * t.per_cu), full = tiles / slots, rem = tiles - full * slots;
-        const float steps = (float)((nk + t.sub - 1) / t.sub * t.sub) * (float)(t.bm + t.bn) * 0.00168f;
-        const float area = (float)(t.bm * t.bn) * 2.08e-4f;
-        float c = (float)full * (1.36f + (float)t.per_cu * (area + steps));
-        if (rem) c += (full ? 1.14f : 1.0f) * (1.36f + (rem > (unsigned)cus ? 2.0f : 1.0f) * (area + steps));
+        const uint64_t tiles = (uint64_t)(((unsigned)M + t.bm - 1) / t.bm) * (((unsigned)N + t.bn - 1) / t.bn);
+        const uint64_t slots = (uint64_t)(cus * t.per_cu), full = tiles / slots, rem = tiles - full * slots;
+        const float one = alone(t, K >> 7), two = (1.0f + BESIDE) * one;
+        float c = (float)full * (PER_ROUND + (t.per_cu == 2 ? two : one));
+        if (rem) c += (full ? LAST_ROUND : 1.0f) * (PER_ROUND + (rem > (uint64_t)cus ? two : one));
         if (at < 0 || c < best) {
             best = c;
             at = i;
@@ -375,15 +403,19 @@ static float pick(int M, int N, int K, int cus, int *which)
     return best;
 }
 
+static float with_memory(float core, double bytes)
+{
+    const float mem = PER_MB * 1e-6f * (float)bytes, c2 = core * core, m2 = mem * mem;
+    return PER_LAUNCH + sqrtf(sqrtf(c2 * c2 + m2 * m2));
+}
+
 }  // namespace deep
 
 // Microseconds that launch_deep would take (see above); *which is the tile to pass on.
 float deep_estimate(int M, int N, int K, int cus, int *which)
 {
     const float core = deep::pick(M, N, K, cus, which);
-    const float mem = 0.218e-6f * ((float)N * (float)K + (float)M * (float)K + 4.0f * (float)M * (float)N);
-    const float c2 = core * core, m2 = mem * mem;
-    return 0.75f + sqrtf(sqrtf(c2 * c2 + m2 * m2));
+    return deep::with_memory(core, (double)N * K + (double)M * K + 4.0 * M * N);
 }
 
 template <bool DEQ>
@@ -396,20 +428,14 @@ int32_t launch_deep(int which, const int8_t *qx, const float *sx, const int8_t *
     switch (which) {   // in the order of TILES
     case 0: return launch<Cfg<4, 4, 2, 2, 2, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
     case 1: return launch<Cfg<4, 2, 2, 2, 2, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 2: return launch<Cfg<2, 4, 2, 2, 2, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 3: return launch<Cfg<2, 4, 2, 1, 4, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 4: return launch<Cfg<2, 2, 2, 1, 4, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 5: return launch<Cfg<2, 4, 1, 2, 4, 4>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 6: return launch<Cfg<2, 4, 1, 1, 8, 3>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 7: return launch<Cfg<2, 3, 1, 1, 4, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 8: return launch<Cfg<2, 2, 1, 1, 8, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 9: return launch<Cfg<2, 1, 1, 1, 8, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 10: return launch<Cfg<1, 7, 1, 1, 4, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 11: return launch<Cfg<1, 4, 1, 1, 8, 4>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 12: return launch<Cfg<1, 3, 1, 1, 4, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 13: return launch<Cfg<1, 2, 1, 1, 8, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 14: return launch<Cfg<1, 1, 1, 1, 8, 7>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
-    case 15: return launch<Cfg<4, 2, 2, 2, 2, 3>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 2: return launch<Cfg<2, 2, 2, 2, 2, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 3: return launch<Cfg<2, 2, 2, 1, 2, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 4: return launch<Cfg<2, 3, 1, 1, 4, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 5: return launch<Cfg<2, 2, 1, 1, 4, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 6: return launch<Cfg<2, 1, 1, 1, 4, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 7: return launch<Cfg<1, 3, 1, 1, 4, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 8: return launch<Cfg<1, 2, 1, 1, 4, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 9: return launch<Cfg<1, 1, 1, 1, 8, 4>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
     default: return MI_EINVAL;
     }
 }
@@ -419,30 +445,31 @@ template int32_t launch_deep<false>(int, const int8_t *, const float *, const in
                                     int64_t, int64_t, int64_t, hipStream_t);
 
 // ---- several contractions of at least 256 rows in one launch (a part of a batch, see gemm_list.hip)
-// Time of a workgroup on a tile, as above; the tiles go to the units as these come free, longest K first.  A launch of
-// several rounds takes 1.25 times the sum of its tiles (measured 147 us where the sum says 115 and 83 where it says 66).
+// Times as above; the tiles go to the units as these come free, longest K first.  A launch of several rounds takes 1.25
+// times the sum of its tiles (measured 147 us where the sum says 115 and 83 where it says 66).
 float deep_batch_estimate(const int64_t *mnk, const int *idx, int n, int cus, int *which)
 {
     using namespace deep;
-    constexpr int TRY[] = {0, 1, 3};
+    constexpr int TRY = 3;   // 128 x 128, 128 x 64, 64 x 64
     float best = -1.0f;
-    double mem = 0.0;
+    double bytes = 0.0;
     for (int i = 0; i < n; ++i) {
-        const int64_t M = mnk[3 * idx[i]], N = mnk[3 * idx[i] + 1], K = mnk[3 * idx[i] + 2];
-        mem += 0.218e-6 * ((double)N * K + (double)M * K + 4.0 * M * N);
+        const double M = (double)mnk[3 * idx[i]], N = (double)mnk[3 * idx[i] + 1], K = (double)mnk[3 * idx[i] + 2];
+        bytes += N * K + M * K + 4.0 * M * N;
     }
-    std::vector<std::pair<float, int64_t>> free;   // when units are free, and how many
-    for (int t : TRY) {
+    std::vector<std::pair<float, int64_t>> free;   // when slots are free, and how many
+    for (int t = 0; t < TRY; ++t) {
         const Tile &T = TILES[t];
-        free.assign(1, {0.0f, cus});
+        const int64_t slots = (int64_t)cus * T.per_cu;
+        free.assign(1, {0.0f, slots});
         float end = 0.0f;
         int64_t count = 0;
         for (int i = 0; i < n; ++i) {
             const int64_t M = mnk[3 * idx[i]], N = mnk[3 * idx[i] + 1], nk = mnk[3 * idx[i] + 2] >> 7;
             int64_t tiles = ((M + T.bm - 1) / T.bm) * ((N + T.bn - 1) / T.bn);
-            const float cost = 1.36f + (float)(T.bm * T.bn) * 2.08e-4f + (float)((nk + T.sub - 1) / T.sub * T.sub) * (float)(T.bm + T.bn) * 0.00168f;
             count += tiles;
-            while (tiles > 0) {   // as many tiles as units are free first, all at once
+            const float cost = PER_ROUND + (T.per_cu == 2 ? 1.0f + BESIDE : 1.0f) * alone(T, nk);
+            while (tiles > 0) {   // as many tiles as slots are free first, all at once
                 const size_t at = (size_t)(std::min_element(free.begin(), free.end()) - free.begin());
                 const int64_t k = std::min(tiles, free[at].second);
                 const float done = free[at].first + cost;
@@ -455,14 +482,13 @@ float deep_batch_estimate(const int64_t *mnk, const int *idx, int n, int cus, in
                 end = std::max(end, done);
             }
         }
-        if (count > cus) end *= 1.25f;
+        if (count > slots) end *= 1.25f;
         if (best < 0.0f || end < best) {
             best = end;
             *which = t;
         }
     }
-    const float m = (float)mem, c2 = best * best, m2 = m * m;
-    return 0.75f + sqrtf(sqrtf(c2 * c2 + m2 * m2));
+    return with_memory(best, bytes);
 }
 
 template <bool DEQ>
@@ -476,7 +502,7 @@ int32_t launch_deep_batch(int which, const DeepProblem *p, int n, hipStream_t s)
     switch (which) {
     case 0: return launch_batch<Cfg<4, 4, 2, 2, 2, 5>, DEQ>(b, s);
     case 1: return launch_batch<Cfg<4, 2, 2, 2, 2, 6>, DEQ>(b, s);
-    case 3: return launch_batch<Cfg<2, 4, 2, 1, 4, 5>, DEQ>(b, s);
+    case 2: return launch_batch<Cfg<2, 2, 2, 2, 2, 5>, DEQ>(b, s);
     default: return MI_EINVAL;
     }
 }

@@ -800,7 +800,7 @@ static int32_t batch_run(mi_gemm_batch *b, const mi_gemm_problem *p, void *strea
         DeepProblem d[list::MAX_PROBLEMS];
         for (int i = 0; i < sp.n_deep; ++i) {
             const mi_gemm_problem &g = p[sp.deep[i]];
-            d[i] = {g.qx, g.qw, g.sx, g.sw, g.out, (int)g.M, (int)g.N, (int)g.K, 0};
+            d[i] = {g.qx, g.qw, g.sx, g.sw, g.out, (int)g.M, (int)g.N, (int)g.K, 0, 0, 0, 0};
         }
         const int32_t rc = launch_deep_batch<DEQ>(sp.which, d, sp.n_deep, as_stream(stream));
         if (rc || !sp.n_tiled) return rc;

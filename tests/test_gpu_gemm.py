@@ -72,14 +72,12 @@ def test_paired_wave_kernel_bit_exact(mi, dev, orc, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [
-    # every tile of the small-tile kernel on a chip of 256 units, in its order (128 x 128 to 16 x 16, then 128 x 64 two a
-    # unit): fewer stages than its ring holds, a last stage that K fills in part, ragged rows and columns
-    (67, 16464, 128), (714, 4304, 384), (164, 7648, 256), (773, 1664, 512), (63, 16592, 128), (41, 16880, 512),
-    (35, 8368, 128), (75, 5552, 1152), (57, 6448, 128), (361, 1200, 384), (17, 17040, 128), (194, 4384, 1920),
-    (18, 12560, 128), (92, 5056, 768), (59, 4784, 640), (650, 528, 128), (22, 6224, 384), (736, 336, 896),
-    (17, 2448, 384), (714, 112, 1408), (2, 16400, 128), (14, 18640, 1408), (3, 13552, 128), (140, 1776, 384),
-    (3, 10864, 128), (32, 4272, 640), (2, 4272, 384), (15, 5024, 384), (2, 16, 128), (49, 16, 640),
-    (773, 4672, 384), (665, 5440, 384),
+    # every tile of the small-tile kernel on a chip of 256 units, in its order (128 x 128 to 16 x 16): fewer stages than
+    # its ring holds, a last stage that K fills in part, ragged rows and columns
+    (72, 25936, 128), (692, 4752, 256), (66, 10480, 384), (809, 1360, 1024), (17, 26240, 128), (373, 4560, 128),
+    (570, 992, 384), (35, 6240, 128), (258, 1568, 640), (578, 848, 128), (18, 8272, 128), (97, 2640, 384), (792, 448, 1024),
+    (18, 6320, 128), (387, 544, 256), (499, 448, 128), (18, 2176, 128), (845, 80, 1664), (2, 8224, 128), (270, 624, 128),
+    (61, 2080, 896), (2, 4112, 128), (7, 5872, 1536), (2, 16, 128), (9, 16, 384), (11, 2848, 512),
 ])
 def test_small_tile_kernel_bit_exact(mi, dev, orc, M, N, K):
     qx, qw = rand_codes(M + N + K, (M, K)), rand_codes(K + 11, (N, K))
