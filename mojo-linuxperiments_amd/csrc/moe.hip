@@ -60,6 +60,9 @@ __device__ __forceinline__ void fold(float (&p)[NP], int lane)
 // two waves share a SIMD where EW = 16 leaves one alone with its memory round trips (cfg4: 17.2 -> 13.8 us; four
 // experts a wave, or loads two rounds ahead in three register sets, measured the same 13.8).  The first butterfly
 // round (offset 32) is then the plain one; lanes l and l ^ 32 end with the same pair.
+// EW = 1: few tokens.  Sixteen tokens are 16 workgroups at EW = 8, each a chain of H / 256 memory round trips; one
+// expert a wave makes them 128 whose loads go out at once (H = 2048, E = 128: 16 tokens 11.8 -> 6.4 us, 128 tokens
+// 11.4 -> 10.7; at 512 the activations would be read 128 times).
 template <int CQ, int EW>
 __global__ __launch_bounds__(256) void k_moe_logits(const float *__restrict__ x, const float *__restrict__ wr,
                                                     float *__restrict__ logits, int T, int H, int E,
@@ -147,6 +150,46 @@ __global__ __launch_bounds__(256) void k_moe_logits(const float *__restrict__ x,
     #pragma unroll
             for (int tt = 0; tt < 4; ++tt) xv[tt] = xn[tt];
         }
+    } else if constexpr (EW == 1) {
+        // few tokens: one expert a wave and JB rounds' loads requested at a time, the next JB behind them, so that rows of
+        // up to 2048 floats are in flight as a whole before the first FMA
+        constexpr int JB = 4;
+        float4 xa[2][JB][4], wa[2][JB];
+        auto request = [&](int set, int j0) {
+#pragma unroll
+            for (int u = 0; u < JB; ++u) {
+                const int j = min(j0 + u, nj - 1);
+                wa[set][u] = *reinterpret_cast<const float4 *>(wp + 256 * j);
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) xa[set][u][tt] = *reinterpret_cast<const float4 *>(xr[tt] + 256 * j);
+            }
+        };
+        auto add = [&](int set, int j0) {
+#pragma unroll
+            for (int u = 0; u < JB; ++u) {
+                if (j0 + u >= nj) break;   // (uniform)
+                const float4 w = wa[set][u];
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) {
+                    const float4 v = xa[set][u][tt];
+                    float a = p[tt];
+                    a = __builtin_fmaf(v.x, w.x, a);
+                    a = __builtin_fmaf(v.y, w.y, a);
+                    a = __builtin_fmaf(v.z, w.z, a);
+                    a = __builtin_fmaf(v.w, w.w, a);
+                    p[tt] = a;
+                }
+            }
+        };
+        if (t0 < T) {   // whole wave
+            request(0, 0);
+            for (int j = 0; j < nj; j += 2 * JB) {
+                request(1, j + JB);
+                add(0, j);
+                if (j + 2 * JB < nj) request(0, j + 2 * JB);
+                add(1, j + JB);
+            }
+        }
     } else {
         // one group of eight experts: the next round's weights and token rows are requested before this round's
         // 128 FMAs
@@ -188,6 +231,13 @@ __global__ __launch_bounds__(256) void k_moe_logits(const float *__restrict__ x,
         // lane l now holds pair l: token l/16, expert e0 + l%16
         const int t = t0 + (lane >> 4);
         if (t < T) logits[(int64_t)t * E + e0 + (lane & 15)] = p[0];
+    } else if constexpr (EW == 1) {
+        fold<32, 2>(p, lane);
+        fold<16, 1>(p, lane);
+#pragma unroll
+        for (int off = 8; off >= 1; off >>= 1) p[0] = p[0] + shfl_xor_f(p[0], off);
+        const int t = t0 + (lane >> 4);   // the 16 lanes of a group hold the same token's sum
+        if ((lane & 15) == 0 && t < T) logits[(int64_t)t * E + e0] = p[0];
     } else {
         static_assert(EW == 8, "experts per wave");
 #pragma unroll
@@ -967,13 +1017,18 @@ static bool route_can_quantize(int64_t H) { return H % 128 == 0 && H <= 2048; }
 static int32_t launch_route(const float *x, const float *wr, int32_t *idx, float *w, int64_t T, int64_t H, int64_t E,
                             int32_t topk, float *logits, int8_t *qx, float *sx, void *stream)
 {
-    // eight experts a wave (twice the workgroups) while sixteen would leave at most two workgroups to a compute unit
-    const bool narrow = (int64_t)((T + 15) / 16) * (E / 16) <= 2 * (int64_t)compute_units();
-    const dim3 grid((unsigned)((T + 15) / 16), (unsigned)(E / (narrow ? 8 : 16)));
+    // eight experts a wave (twice the workgroups) while sixteen would leave at most two workgroups to a compute unit,
+    // one while eight would leave half of the units without any
+    const int64_t groups = (T + 15) / 16;
+    const int ew = groups * (E / 8) <= compute_units() / 2 ? 1 : groups * (E / 16) <= 2 * (int64_t)compute_units() ? 8 : 16;
+    const dim3 grid((unsigned)groups, (unsigned)(E / ew));
     const int cq = qx ? (int)((H / 8 + 63) / 64) : 0;
 #define MI_LOGITS(CQ_)                                                                                                  \
     do {                                                                                                                \
-        if (narrow)                                                                                                     \
+        if (ew == 1)                                                                                                    \
+            hipLaunchKernelGGL((k_moe_logits<CQ_, 1>), grid, dim3(256), 0, as_stream(stream), x, wr, logits, (int)T,    \
+                               (int)H, (int)E, qx, sx);                                                                 \
+        else if (ew == 8)                                                                                               \
             hipLaunchKernelGGL((k_moe_logits<CQ_, 8>), grid, dim3(256), 0, as_stream(stream), x, wr, logits, (int)T,    \
                                (int)H, (int)E, qx, sx);                                                                 \
         else                                                                                                            \

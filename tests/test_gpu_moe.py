@@ -231,3 +231,29 @@ def test_argument_errors(mi, dev):
     args = (b.ptr,) * 10
     assert lib.mi_moe_ffn(*args, 8, 256, 256, 16, 2, b.ptr, 64, None) == mi.ENOSPC
     dev.reset_to(mark)
+
+
+@pytest.mark.parametrize("T,H,I,E,topk", [
+    (1, 256, 256, 16, 1),       # one round of the logits, one token
+    (15, 1280, 512, 64, 4),     # a last batch of rounds that is not whole
+    (16, 2048, 768, 128, 8), (17, 2048, 768, 128, 8),
+    (33, 2304, 256, 256, 8),    # rows that the logits kernel does not quantize
+    (128, 512, 256, 128, 8), (129, 512, 256, 128, 8),   # the last token count of one expert a wave, and the first beyond
+])
+def test_layer_of_few_tokens_equals_route_and_ffn(mi, dev, orc, T, H, I, E, topk):
+    """The layer's own router launches against the separate calls: the same picks as the oracle, then the same bits."""
+    x, wr = workload.activations(61, T, H), workload.weights(62, E, H)
+    experts = make_experts(orc, 63, E, H, I)
+    mark = dev.mark()
+    a = run_ffn(mi, dev, x, None, None, experts, layer_wr=(wr, topk))
+    idx, w = gpu_route(mi, dev, x, wr, topk)
+    b = run_ffn(mi, dev, x, idx, w, experts)
+    dev.reset_to(mark)
+    idxo, wo = orc.moe_route(x, wr, topk)
+    assert np.array_equal(a["idx"], idxo) and np.array_equal(idx, idxo)
+    assert np.max(np.abs(a["w"] - wo)) <= 2e-6
+    permo, sego = orc.moe_dispatch(idxo, E)
+    assert np.array_equal(a["perm"], permo) and np.array_equal(a["seg"], sego)
+    assert np.array_equal(a["w"], w)
+    for name in ("qx", "sx", "h", "hq", "hs", "out", "y"):
+        assert np.array_equal(a[name], b[name]), name
