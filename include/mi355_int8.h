@@ -342,6 +342,16 @@ MI_API int32_t mi_gqa_decode_attn_tiled_linear_f32(const float *q, const int8_t 
                                                    int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t T_cap,
                                                    const int32_t *seq_len, int64_t T_max, int64_t N,
                                                    void *workspace, int64_t workspace_bytes, void *stream);
+/* ... and with the rotary embedding and the append in front of it: mi_rope_kv_append_tiled_f32_i8 followed by
+ * mi_gqa_decode_attn_tiled_linear_f32 on q_out, bit for bit, the append done by the attention kernel.  A sequence whose
+ * pos lies outside [0, T_cap) appends nothing and attends with the rows that q_out holds.  q_out 16-byte aligned. */
+MI_API int32_t mi_rope_append_attn_tiled_linear_f32(const float *qkv, int64_t row_stride, const float *rope_cos,
+                                                    const float *rope_sin, float *q_out, int8_t *kt, float *ks,
+                                                    int8_t *vt, float *vs, const int32_t *pos, float *o_rot,
+                                                    const int8_t *qw, const float *sw, float *y,
+                                                    int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t T_cap,
+                                                    const int32_t *seq_len, int64_t T_max, int64_t N,
+                                                    void *workspace, int64_t workspace_bytes, void *stream);
 /* Row-major codes [rows, src_stride tokens, 128] (rows = B*Hkv) -> the tiled layouts, first T tokens of every row
  * (the rest of the last 64-token block touched is zero-filled); either pair (kq, kt) / (vq, vt) may be NULL.  For
  * caches that were quantized in one go (prefill) with mi_fwht_quant_f32_i8. */

@@ -67,7 +67,45 @@ struct Params {
     int8_t *dbg_qq;
     float *dbg_sq;
     int32_t *dbg_dots;
+    // APPEND kernels: fused QKV rows [Hq | Hkv | Hkv] x 128 in place of q, the rotary tables, and the position that
+    // each sequence's new token takes in the cache; q receives the rotated query rows
+    const float *qkv;
+    int64_t qkv_stride;
+    const float *cs, *sn;
+    const int32_t *pos;
 };
+
+// Rotary embedding of the eight elements 4 j .. and 64 + 4 j .. of a head (the arithmetic of k_rope_kv_append, layer_ops.hip)
+__device__ __forceinline__ void rope8(float (&v)[8], const float4 &c4, const float4 &s4)
+{
+    const float c[4] = {c4.x, c4.y, c4.z, c4.w}, s[4] = {s4.x, s4.y, s4.z, s4.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float a = v[e], bb = v[e + 4];
+        v[e] = a * c[e] - bb * s[e];
+        v[e + 4] = bb * c[e] + a * s[e];
+    }
+}
+
+// Codes 4 j .. (c0) and 64 + 4 j .. (c1) of a head of token tp to their place; blk0: first token of its 64-token block
+__device__ __forceinline__ void store_token(bool is_v, int j, int tp, int64_t blk0, uint32_t c0, uint32_t c1, int8_t *kq,
+                                            int8_t *vt)
+{
+    if (!is_v) {
+        // codes 4j .. 4j+3: chunk j/4, bytes 4*(j%4) .. of token tp % 16 in tile tp / 16; codes 64 + 4j ..: chunk 4 + j/4
+        int8_t *q = kq + (blk0 + (tp & 48)) * D + (j >> 2) * 256 + (tp & 15) * 16 + 4 * (j & 3);
+        *reinterpret_cast<uint32_t *>(q) = c0;
+        *reinterpret_cast<uint32_t *>(q + 1024) = c1;
+    } else {
+        // code d of token tp: block tp / 64, piece d / 16, token chunk (tp % 64) / 16, row d % 16, byte tp % 16
+        int8_t *blk = vt + blk0 * D + (j >> 2) * 1024 + ((tp & 63) >> 4) * 256 + 4 * (j & 3) * 16 + (tp & 15);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            blk[e * 16] = (int8_t)(c0 >> (8 * e));
+            blk[4096 + e * 16] = (int8_t)(c1 >> (8 * e));
+        }
+    }
+}
 
 template <int MASK>
 __device__ __forceinline__ float fmax_xor(float v)
@@ -78,7 +116,14 @@ __device__ __forceinline__ float fmax_xor(float v)
 // NW: waves per workgroup; NT: blocks per wave; RING: 1 KB loads a wave keeps in flight (8 or 16).
 // DIRECT: the workgroup covers the whole sequence (one split): it normalizes and writes the output rows itself and
 // no partial result leaves the chip.
-template <int NW, int NT, int RING, bool DIRECT>
+// APPEND: the decode step's rotary embedding and cache append happen here instead of in a launch of their own (dense
+// layout).  Every wave rotates its own copy of the query rows; the one wave in the grid whose block holds the new token
+// (the last split's first wave if no block does) quantizes the key and value heads, stores them, and only then requests
+// its blocks: nobody else reads that token.  The new scales meet the loaded ones in LDS.  A launch of its own takes 4 to 5
+// us of latency for a few KB; here it is one more memory round trip in a few workgroups.  Decode steps, us with two
+// launches -> one: 16 sequences of 4096 tokens, four layers 402 -> 392; one of 1531, four layers 300 -> 287; 16 of 1024
+// with experts, two layers 286 -> 280.
+template <int NW, int NT, int RING, bool DIRECT, bool APPEND>
 __global__ __launch_bounds__(64 * NW) void k_gqa_tiled_split(Params p)
 {
     constexpr int SPAN = NW * NT * 64;                    // tokens a workgroup can cover
@@ -107,7 +152,57 @@ __global__ __launch_bounds__(64 * NW) void k_gqa_tiled_split(Params p)
     if (p.seq_len) T = min(max(__builtin_amdgcn_readfirstlane(p.seq_len[b]), 0), p.T);
     const int blk_lo = split * p.blocks_per_split;
     const int t_lo = blk_lo * 64;
+    int tp = -1;              // the new token's position, if it has one in the cache
+    bool owner = false;       // this wave appends it
+    float new_ks = 0.0f, new_vs = 0.0f;
+    if constexpr (APPEND) {
+        tp = __builtin_amdgcn_readfirstlane(p.pos[b]);
+        if (tp < 0 || tp >= p.Tstride) tp = -1;
+        const int at = (tp >> 6) - blk_lo;
+        const bool last = split == (int)gridDim.x - 1;
+        if (tp >= 0 && at >= 0 && (at < p.blocks_per_split || last)) owner = wave == (at < p.blocks_per_split ? at % NW : 0);
+        if (owner) {
+            const int j = lane & 15;
+            const bool is_v = (lane >> 4) & 1;   // lanes 0 - 15: the key head, 16 - 31: the value head (and both again)
+            const float *src = p.qkv + b * p.qkv_stride + (int64_t)(p.Hq + (is_v ? p.Hkv : 0) + kvh) * D + 4 * j;
+            const float4 lo = *reinterpret_cast<const float4 *>(src), hi = *reinterpret_cast<const float4 *>(src + D / 2);
+            float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            if (!is_v)
+                rope8(v, *reinterpret_cast<const float4 *>(p.cs + (int64_t)tp * (D / 2) + 4 * j),
+                      *reinterpret_cast<const float4 *>(p.sn + (int64_t)tp * (D / 2) + 4 * j));
+            fwht_chunk<D>(v, j);
+            float a = abs8(v);
+            a = fmax_xor<1>(a); a = fmax_xor<2>(a); a = fmax_xor<4>(a); a = fmax_xor<8>(a);
+            const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
+            const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
+            const int64_t blk0 = (int64_t)bkv * p.Tstride + (tp & ~63);
+            if (lane < 32) {
+                store_token(is_v, j, tp, blk0, quant4(v[0], v[1], v[2], v[3], inv), quant4(v[4], v[5], v[6], v[7], inv),
+                            const_cast<int8_t *>(p.kq), const_cast<int8_t *>(p.vt));
+                if (j == 0) const_cast<float *>(is_v ? p.vs : p.ks)[blk0 + (tp & 63)] = sc;
+            }
+            new_ks = __shfl(sc, 0, 64);
+            new_vs = __shfl(sc, 16, 64);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // stored before the wave's blocks are requested
+        }
+    }
     if (t_lo >= T) {
+        if constexpr (APPEND) {
+            if (split == 0 && tp >= 0) {   // nothing to attend to; the query rows are rotated all the same
+                const int hr = tid >> 4, j = tid & 15;
+                if (hr < G) {
+                    const int64_t row = (int64_t)(kvh * G + hr) * D + 4 * j;
+                    const float *src = p.qkv + b * p.qkv_stride + row;
+                    const float4 lo = *reinterpret_cast<const float4 *>(src), hi = *reinterpret_cast<const float4 *>(src + D / 2);
+                    float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                    rope8(v, *reinterpret_cast<const float4 *>(p.cs + (int64_t)tp * (D / 2) + 4 * j),
+                          *reinterpret_cast<const float4 *>(p.sn + (int64_t)tp * (D / 2) + 4 * j));
+                    float *dst = const_cast<float *>(p.q) + (int64_t)b * p.Hq * D + row;
+                    *reinterpret_cast<float4 *>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+                    *reinterpret_cast<float4 *>(dst + D / 2) = make_float4(v[4], v[5], v[6], v[7]);
+                }
+            }
+        }
         if constexpr (DIRECT) {
             // a sequence of length 0: a row of zeros
             for (int o = tid; o < G * D; o += 64 * NW) p.o[((int64_t)b * p.Hq + kvh * G) * D + o] = 0.0f;
@@ -146,6 +241,14 @@ __global__ __launch_bounds__(64 * NW) void k_gqa_tiled_split(Params p)
     const int hr = lane >> 4, jj = lane & 15;
     const int head = kvh * G + min(hr, G - 1);
     const float *qr = p.q + ((int64_t)b * p.Hq + head) * D;
+    float4 rc4 = make_float4(1.f, 1.f, 1.f, 1.f), rs4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (APPEND) {
+        if (tp >= 0) {   // (a sequence without a new token attends with what q holds)
+            qr = p.qkv + b * p.qkv_stride + (int64_t)head * D;
+            rc4 = *reinterpret_cast<const float4 *>(p.cs + (int64_t)tp * (D / 2) + 4 * jj);
+            rs4 = *reinterpret_cast<const float4 *>(p.sn + (int64_t)tp * (D / 2) + 4 * jj);
+        }
+    }
     const float4 qlo = *reinterpret_cast<const float4 *>(qr + 4 * jj);
     const float4 qhi = *reinterpret_cast<const float4 *>(qr + 64 + 4 * jj);
 
@@ -191,9 +294,10 @@ __global__ __launch_bounds__(64 * NW) void k_gqa_tiled_split(Params p)
         const float v[4] = {vs4.x, vs4.y, vs4.z, vs4.w};
         float vm = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) vm = fmaxf(vm, (t_lo + sidx + e < t_end) ? v[e] : 0.0f);
+        for (int e = 0; e < 4; ++e) vm = fmaxf(vm, (t_lo + sidx + e < t_end && (!APPEND || t_lo + sidx + e != tp)) ? v[e] : 0.0f);
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) vm = fmaxf(vm, __shfl_xor(vm, off, 64));
+        if (APPEND && owner && tp < t_end) vm = fmaxf(vm, new_vs);
         if (sidx < SPAN) {
             *reinterpret_cast<float4 *>(s_ks + sidx) = ks4;
             *reinterpret_cast<float4 *>(s_vs + sidx) = vs4;
@@ -203,6 +307,16 @@ __global__ __launch_bounds__(64 * NW) void k_gqa_tiled_split(Params p)
     // ---- query heads of this group: every wave rotates and quantizes them for itself
     {
         float v[8] = {qlo.x, qlo.y, qlo.z, qlo.w, qhi.x, qhi.y, qhi.z, qhi.w};
+        if constexpr (APPEND) {
+            if (tp >= 0) {
+                rope8(v, rc4, rs4);
+                if (split == 0 && wave == 0 && hr < G) {
+                    float *dst = const_cast<float *>(p.q) + ((int64_t)b * p.Hq + head) * D + 4 * jj;
+                    *reinterpret_cast<float4 *>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+                    *reinterpret_cast<float4 *>(dst + D / 2) = make_float4(v[4], v[5], v[6], v[7]);
+                }
+            }
+        }
         fwht_chunk<D>(v, jj);
         float a = abs8(v);
         a = fmax_xor<1>(a); a = fmax_xor<2>(a); a = fmax_xor<4>(a); a = fmax_xor<8>(a);
@@ -221,6 +335,10 @@ __global__ __launch_bounds__(64 * NW) void k_gqa_tiled_split(Params p)
     }
     // LDS only: the ring's loads stay in flight across this barrier
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (APPEND && owner && tp < t_end && lane == 0) {   // scales of the wave's own block: no one else reads them
+        s_ks[tp - t_lo] = new_ks;
+        s_vs[tp - t_lo] = new_vs;
+    }
     float vmax = s_vmax[0];
 #pragma unroll
     for (int w = 1; w < NW; ++w) vmax = fmaxf(vmax, s_vmax[w]);
@@ -496,13 +614,7 @@ __global__ __launch_bounds__(256) void k_kv_append_vt(const float *__restrict__ 
         if (live && !is_v) {
             const float4 c4 = *reinterpret_cast<const float4 *>(cs + (int64_t)tp * (D / 2) + 4 * j);
             const float4 s4 = *reinterpret_cast<const float4 *>(sn + (int64_t)tp * (D / 2) + 4 * j);
-            const float c[4] = {c4.x, c4.y, c4.z, c4.w}, s[4] = {s4.x, s4.y, s4.z, s4.w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float a = v[e], bb = v[e + 4];
-                v[e] = a * c[e] - bb * s[e];
-                v[e + 4] = bb * c[e] + a * s[e];
-            }
+            rope8(v, c4, s4);
             if (is_q) {
                 float *dst = q_out + ((int64_t)b * Hq + hd) * D + 4 * j;
                 *reinterpret_cast<float4 *>(dst) = make_float4(v[0], v[1], v[2], v[3]);
@@ -522,21 +634,7 @@ __global__ __launch_bounds__(256) void k_kv_append_vt(const float *__restrict__ 
                                          : ((int64_t)b * Hkv + h) * T_cap + (tp & ~63);
         const uint32_t c0 = quant4(v[0], v[1], v[2], v[3], inv), c1 = quant4(v[4], v[5], v[6], v[7], inv);
         if (j == 0) (is_v ? vs : ks)[blk0 + (tp & 63)] = sc;
-        if (!is_v) {
-            // codes 4j .. 4j+3: chunk j/4, bytes 4*(j%4) .. of token tp % 16 in tile tp / 16; codes 64 + 4j ..: chunk 4 + j/4
-            int8_t *q = kq + (blk0 + (tp & 48)) * D + (j >> 2) * 256 + (tp & 15) * 16 + 4 * (j & 3);
-            *reinterpret_cast<uint32_t *>(q) = c0;
-            *reinterpret_cast<uint32_t *>(q + 1024) = c1;
-        } else {
-            // code d of token tp: block tp / 64, piece d / 16, token chunk (tp % 64) / 16, row d % 16, byte tp % 16
-            int8_t *blk = vt + blk0 * D + (j >> 2) * 1024 + ((tp & 63) >> 4) * 256 +
-                          4 * (j & 3) * 16 + (tp & 15);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                blk[e * 16] = (int8_t)(c0 >> (8 * e));
-                blk[4096 + e * 16] = (int8_t)(c1 >> (8 * e));
-            }
-        }
+        store_token(is_v, j, tp, blk0, c0, c1, kq, vt);
     }
 }
 
@@ -583,6 +681,14 @@ using namespace mi;
 
 static int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
+// the decode step's rotary embedding and append, done by the attention kernel itself
+struct StepIn {
+    const float *qkv;
+    int64_t stride;
+    const float *cs, *sn;
+    const int32_t *pos;
+};
+
 struct ScoreGate {
     int8_t *qq;
     float *sq;
@@ -593,7 +699,7 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
                       int8_t *oq, float *oscale, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t T_cap,
                       const int32_t *seq_len, int64_t T_max, int32_t out_rotated, void *workspace,
                       int64_t workspace_bytes, hipStream_t s, const int32_t *block_table = nullptr,
-                      int64_t max_pages = 0, const ScoreGate *dbg = nullptr)
+                      int64_t max_pages = 0, const ScoreGate *dbg = nullptr, const StepIn *step = nullptr)
 {
     if (block_table) {   // paged: the capacity of a sequence is its share of the table
         if (max_pages <= 0 || max_pages > (1 << 18) || !seq_len || !aligned4(block_table)) return MI_EINVAL;
@@ -610,7 +716,7 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
     const avt::Plan plan = avt::pick(B, Hkv, T_max);
     // one workgroup sees the whole sequence: it writes the output rows (the gate takes the split form: it wants no o)
     const bool direct = plan.splits == 1 && !oq && !dbg;
-    avt::Params p;
+    avt::Params p = {};
     p.q = q; p.kq = kq; p.ks = ks; p.vt = vt; p.vs = vs;
     p.Hq = (int)Hq; p.Hkv = (int)Hkv; p.G = (int)(Hq / Hkv); p.T = (int)T_max;
     p.Tstride = (int)T_cap;
@@ -624,12 +730,17 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
     p.part_o = static_cast<float *>(workspace);
     p.part_ml = reinterpret_cast<float *>(static_cast<char *>(workspace) +
                                           align_up(B * Hkv * plan.splits * 4 * avt::D * 4, 256));
+    if (step) {
+        p.qkv = step->qkv; p.qkv_stride = step->stride; p.cs = step->cs; p.sn = step->sn; p.pos = step->pos;
+    }
     p.blocks_per_split = plan.per;
     const dim3 grid((unsigned)plan.splits, (unsigned)(B * Hkv));
     const int nt = (plan.per + 3) / 4;
-#define MI_TILED(NT_, DIR_) hipLaunchKernelGGL((avt::k_gqa_tiled_split<4, NT_, 8, DIR_>), grid, dim3(256), 0, s, p)
-    if (direct) { if (nt <= 1) MI_TILED(1, true); else if (nt <= 2) MI_TILED(2, true); else MI_TILED(4, true); }
-    else { if (nt <= 1) MI_TILED(1, false); else if (nt <= 2) MI_TILED(2, false); else MI_TILED(4, false); }
+#define MI_TILED(NT_, DIR_, APP_) hipLaunchKernelGGL((avt::k_gqa_tiled_split<4, NT_, 8, DIR_, APP_>), grid, dim3(256), 0, s, p)
+#define MI_TILED_NT(DIR_, APP_) do { if (nt <= 1) MI_TILED(1, DIR_, APP_); else if (nt <= 2) MI_TILED(2, DIR_, APP_); else MI_TILED(4, DIR_, APP_); } while (0)
+    if (step) { if (direct) MI_TILED_NT(true, true); else MI_TILED_NT(false, true); }
+    else { if (direct) MI_TILED_NT(true, false); else MI_TILED_NT(false, false); }
+#undef MI_TILED_NT
 #undef MI_TILED
     if (direct || dbg) return launch_status();
     int32_t rc = launch_status();
@@ -686,12 +797,10 @@ extern "C" int64_t mi_gqa_decode_attn_linear_workspace_bytes(int64_t B, int64_t 
     return a + align_up(B * Hq * D * 4, 256) + align_up(B * Hq * D, 256) + align_up(B * 4, 256);
 }
 
-extern "C" int32_t mi_gqa_decode_attn_tiled_linear_f32(const float *q, const int8_t *kq, const float *ks,
-                                                       const int8_t *vt, const float *vs, float *o_rot,
-                                                       const int8_t *qw, const float *sw, float *y, int64_t B,
-                                                       int64_t Hq, int64_t Hkv, int64_t D, int64_t T_cap,
-                                                       const int32_t *seq_len, int64_t T_max, int64_t N,
-                                                       void *workspace, int64_t workspace_bytes, void *stream)
+static int32_t attn_linear(const float *q, const int8_t *kq, const float *ks, const int8_t *vt, const float *vs, float *o_rot,
+                           const int8_t *qw, const float *sw, float *y, int64_t B, int64_t Hq, int64_t Hkv, int64_t D,
+                           int64_t T_cap, const int32_t *seq_len, int64_t T_max, int64_t N, void *workspace,
+                           int64_t workspace_bytes, void *stream, const StepIn *step)
 {
     if (!qw || !sw || !y || !workspace || N <= 0 || N % 16) return MI_EINVAL;
     if (!aligned16(qw) || !aligned16(sw) || !aligned16(y) || !aligned16(workspace) || (o_rot && !aligned16(o_rot)))
@@ -714,14 +823,25 @@ extern "C" int32_t mi_gqa_decode_attn_tiled_linear_f32(const float *q, const int
         // (the same row quantizer on the same values: identical codes, scale and y).
         float *orow = o_rot ? o_rot : row;
         int32_t rc = run_tiled(q, kq, ks, vt, vs, orow, nullptr, nullptr, B, Hq, Hkv, D, T_cap, seq_len, T_max, 1, attn_ws,
-                               attn_bytes, s);
+                               attn_bytes, s, nullptr, 0, nullptr, step);
         if (rc) return rc;
         return launch_linear_fused(orow, qw, sw, y, oq, oscale, 1, N, K, s, false);
     }
     int32_t rc = run_tiled(q, kq, ks, vt, vs, o_rot, oq, oscale, B, Hq, Hkv, D, T_cap, seq_len, T_max, 1, attn_ws,
-                           attn_bytes, s);
+                           attn_bytes, s, nullptr, 0, nullptr, step);
     if (rc) return rc;
     return mi_w8a8_gemm_dequant_f32(oq, oscale, qw, sw, y, B, N, K, stream);
+}
+
+extern "C" int32_t mi_gqa_decode_attn_tiled_linear_f32(const float *q, const int8_t *kq, const float *ks,
+                                                       const int8_t *vt, const float *vs, float *o_rot,
+                                                       const int8_t *qw, const float *sw, float *y, int64_t B,
+                                                       int64_t Hq, int64_t Hkv, int64_t D, int64_t T_cap,
+                                                       const int32_t *seq_len, int64_t T_max, int64_t N,
+                                                       void *workspace, int64_t workspace_bytes, void *stream)
+{
+    return attn_linear(q, kq, ks, vt, vs, o_rot, qw, sw, y, B, Hq, Hkv, D, T_cap, seq_len, T_max, N, workspace,
+                       workspace_bytes, stream, nullptr);
 }
 
 extern "C" int32_t mi_kv_tiled_from_rows_i8(const int8_t *kq, const int8_t *vq, int8_t *kt, int8_t *vt, int64_t rows,
@@ -777,6 +897,23 @@ extern "C" int32_t mi_rope_kv_append_tiled_f32_i8(const float *qkv, int64_t row_
                        qkv, (const float *)nullptr, row_stride, rope_cos, rope_sin, q_out, kq, ks, vt, vs, pos, (int)B,
                        (int)Hq, (int)Hkv, (int)T_cap, (const int32_t *)nullptr, 0);
     return launch_status();
+}
+
+extern "C" int32_t mi_rope_append_attn_tiled_linear_f32(const float *qkv, int64_t row_stride, const float *rope_cos,
+                                                        const float *rope_sin, float *q_out, int8_t *kq, float *ks,
+                                                        int8_t *vt, float *vs, const int32_t *pos, float *o_rot,
+                                                        const int8_t *qw, const float *sw, float *y, int64_t B,
+                                                        int64_t Hq, int64_t Hkv, int64_t D, int64_t T_cap,
+                                                        const int32_t *seq_len, int64_t T_max, int64_t N,
+                                                        void *workspace, int64_t workspace_bytes, void *stream)
+{
+    int32_t rc = check_append(qkv, q_out, kq, ks, vt, vs, pos, B, Hkv, D, T_cap);
+    if (rc) return rc;
+    if (!rope_cos || !rope_sin || !aligned16(rope_cos) || !aligned16(rope_sin) || Hq <= 0) return MI_EINVAL;
+    if (row_stride < (Hq + 2 * Hkv) * D || row_stride % 4) return MI_EINVAL;
+    const StepIn step = {qkv, row_stride, rope_cos, rope_sin, pos};
+    return attn_linear(q_out, kq, ks, vt, vs, o_rot, qw, sw, y, B, Hq, Hkv, D, T_cap, seq_len, T_max, N, workspace,
+                       workspace_bytes, stream, &step);
 }
 
 // ---- the paged form of the tiled cache: pools of 64-token pages, one page = one 8 KB key block (four 16-token tiles)

@@ -303,6 +303,17 @@ struct KvCache {
         return mi_gqa_decode_attn_tiled_linear_f32(q, kq, ks, vq, vs, o_rot, qw, sw, y, B, Hq, Hkv, D, T_cap, seq_len, t_max,
                                                    N, workspace, workspace_bytes, stream);
     }
+    // the decode step's rotary embedding and append in front of it, as one call: fused QKV rows [Hq | Hkv | Hkv] x 128, q
+    // receives the rotated query rows
+    int32_t append_attend_project(const float *qkv, int64_t row_stride, const float *rope_cos, const float *rope_sin, float *q,
+                                  const int32_t *pos, float *o_rot, const int8_t *qw, const float *sw, float *y, int64_t N,
+                                  const int32_t *seq_len, int64_t t_max, void *stream) const
+    {
+        if (!tiled) return MI_EINVAL;
+        return mi_rope_append_attn_tiled_linear_f32(qkv, row_stride, rope_cos, rope_sin, q, kq, ks, vq, vs, pos, o_rot, qw, sw,
+                                                    y, B, Hq, Hkv, D, T_cap, seq_len, t_max, N, workspace, workspace_bytes,
+                                                    stream);
+    }
     // a cache quantized in one go (prefill): row-major codes [B*Hkv, T, 128] (rows src_stride tokens apart) into this
     // cache's layout, first T tokens of every row; the scales are the caller's to copy into ks / vs
     int32_t load_rows(const int8_t *kq_rows, const int8_t *vq_rows, int64_t T, int64_t src_stride, void *stream) const
@@ -403,7 +414,8 @@ struct MoeFfn {
     }
 };
 
-// One decoder layer of a decode step (one new token per sequence), chained on one stream, ten launches (eight for a single sequence):
+// One decoder layer of a decode step (one new token per sequence), chained on one stream, nine launches (seven for a
+// single sequence; a row-major cache takes one more, for the append):
 // (residual +) RMSNorm + quantize -> QKV GEMV -> rotary + cache append -> attention over the cache (split, merge +
 // quantize: the output projection takes the rows in the rotated basis of V) -> O GEMV -> residual + RMSNorm +
 // quantize -> gate|up GEMV -> SwiGLU + quantize -> down GEMV (-> residual).
@@ -482,10 +494,13 @@ struct DecoderLayer {
         int32_t rc = mi_rmsnorm_linear_f32(x, residual, g1, eps, residual ? h0 : nullptr, xn, qkv.qw, qkv.sw, qkv_out, B,
                                            qkv.N, H, 128, qkv.workspace, qkv.workspace_bytes, stream);
         const float *xin = residual ? h0 : x;
-        if (rc == MI_OK) rc = cache.rope_append(qkv_out, (Hq + 2 * Hkv) * 128, rope_cos, rope_sin, q, pos, stream);
+        const int64_t row = (Hq + 2 * Hkv) * 128;
         if (cache.tiled) {
-            if (rc == MI_OK) rc = cache.attend_project(q, att, o.qw, o.sw, ao, H, seq_len, t_max, stream);
+            if (rc == MI_OK)
+                rc = cache.append_attend_project(qkv_out, row, rope_cos, rope_sin, q, pos, att, o.qw, o.sw, ao, H, seq_len, t_max,
+                                                 stream);
         } else {
+            if (rc == MI_OK) rc = cache.rope_append(qkv_out, row, rope_cos, rope_sin, q, pos, stream);
             if (rc == MI_OK) rc = cache.attend_quant(q, att, ca, sa, seq_len, t_max, stream);
             if (rc == MI_OK) rc = mi_w8a8_gemm_dequant_f32(ca, sa, o.qw, o.sw, ao, B, H, Hq * 128, stream);
         }

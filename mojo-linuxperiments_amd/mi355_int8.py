@@ -117,6 +117,8 @@ SIGNATURES = {
     "mi_gqa_decode_attn_linear_workspace_bytes": (i64, [i64, i64, i64, i64, i64]),
     "mi_gqa_decode_attn_tiled_linear_f32": (i32, [vp, vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, vp, i64, i64,
                                                   vp, i64, vp]),
+    "mi_rope_append_attn_tiled_linear_f32": (i32, [vp, i64, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64,
+                                                   i64, i64, vp, i64, i64, vp, i64, vp]),
     "mi_gqa_decode_attn_tiled_quant_i8": (i32, [vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, vp, i64, vp, i64,
                                              vp]),
     "mi_kv_tiled_from_rows_i8": (i32, [vp, vp, vp, vp, i64, i64, i64, i64, vp]),
@@ -486,9 +488,9 @@ def kv_tiled_to_rows(kt, vt):
 
 class DecoderLayer:
     """One decoder layer of a decode step, chained from the C-ABI entry points on one stream:
-    (residual +) RMSNorm + quantize -> QKV GEMV -> rotary + KV-cache append -> attention over the cache (split,
-    merge + quantize) -> O GEMV -> residual + RMSNorm + quantize -> gate|up GEMV -> SwiGLU + quantize -> down GEMV
-    (-> residual).  Ten launches.  Test and bench plumbing over the same calls the C++ host struct of the same name makes
+    (residual +) RMSNorm + quantize -> QKV GEMV -> rotary + KV-cache append (tiled: in the attention kernel) ->
+    attention over the cache (split, merge + quantize) -> O GEMV -> residual + RMSNorm + quantize -> gate|up GEMV -> SwiGLU + quantize -> down GEMV
+    (-> residual).  Nine launches with a tiled cache.  Test and bench plumbing over the same calls the C++ host struct of the same name makes
     (host/mi355_host.hpp).  trace=True also writes the fp32 rows the fused kernels normally keep in registers
     (xn, att, hn, act) so that a test can gate every stage."""
 
@@ -562,18 +564,20 @@ class DecoderLayer:
                                         self.wqkv[1].ptr, self.qkv.ptr, B, self.NQKV, H, self.block, self.lin_ws.ptr,
                                         self.lin_ws.nbytes, s), "mi_rmsnorm_linear_f32")
         xin = self.h0 if residual is not None else x
-        append = lib.mi_rope_kv_append_tiled_f32_i8 if self.tiled else lib.mi_rope_kv_append_f32_i8
-        check(append(self.qkv.ptr, self.NQKV, self.cos.ptr, self.sin.ptr, self.q.ptr, self.kq.ptr, self.ks.ptr,
-                     self.vq.ptr, self.vs.ptr, pos.ptr, B, Hq, Hkv, D, self.T_cap, s), "mi_rope_kv_append")
         # attention output stays in the rotated basis of V and is quantized by the merge itself: the O weights were
         # rotated with block 128 = head_dim along K, so their GEMV takes these codes as they are
         if self.tiled:
-            # attention and the O projection as one call (for one token the projection's GEMV quantizes the merged row)
-            check(lib.mi_gqa_decode_attn_tiled_linear_f32(self.q.ptr, self.kq.ptr, self.ks.ptr, self.vq.ptr, self.vs.ptr,
-                                                          p(self.att), self.wo[0].ptr, self.wo[1].ptr, self.ao.ptr, B, Hq,
-                                                          Hkv, D, self.T_cap, seq_len.ptr, t_max, H, self.att_ws.ptr,
-                                                          self.att_ws.nbytes, s), "mi_gqa_decode_attn_tiled_linear_f32")
+            # rotary embedding, append, attention and the O projection as one call (for one token the projection's GEMV
+            # quantizes the merged row)
+            check(lib.mi_rope_append_attn_tiled_linear_f32(self.qkv.ptr, self.NQKV, self.cos.ptr, self.sin.ptr, self.q.ptr,
+                                                           self.kq.ptr, self.ks.ptr, self.vq.ptr, self.vs.ptr, pos.ptr,
+                                                           p(self.att), self.wo[0].ptr, self.wo[1].ptr, self.ao.ptr, B,
+                                                           Hq, Hkv, D, self.T_cap, seq_len.ptr, t_max, H, self.att_ws.ptr,
+                                                           self.att_ws.nbytes, s), "mi_rope_append_attn_tiled_linear_f32")
         else:
+            check(lib.mi_rope_kv_append_f32_i8(self.qkv.ptr, self.NQKV, self.cos.ptr, self.sin.ptr, self.q.ptr, self.kq.ptr,
+                                               self.ks.ptr, self.vq.ptr, self.vs.ptr, pos.ptr, B, Hq, Hkv, D, self.T_cap, s),
+                  "mi_rope_kv_append_f32_i8")
             check(lib.mi_gqa_decode_attn_cache_quant_i8(self.q.ptr, self.kq.ptr, self.ks.ptr, self.vq.ptr, self.vs.ptr,
                                                         p(self.att), self.ca.ptr, self.sa.ptr, B, Hq, Hkv, D, self.T_cap,
                                                         seq_len.ptr, t_max, self.att_ws.ptr, self.att_ws.nbytes, s),

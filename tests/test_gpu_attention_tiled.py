@@ -444,3 +444,54 @@ def test_vt_weights_with_v_scales_over_six_decades(mi, dev, orc):
     assert err <= T * 127 * 2.0 ** -29 * float(vs.max())
     assert err <= 1e-2 * size, (err, size)
     dev.reset_to(mark)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,T_cap,T_max", [
+    (1, 8, 2, 64, 64),           # one block: the kernel that writes the output rows itself or a single split
+    (1, 32, 8, 640, 500),        # one sequence: short spans, the GEMV behind it
+    (6, 4, 4, 384, 321),         # one head a group; T_max inside a block
+    (9, 16, 4, 2112, 2100),      # full spans of 16 blocks
+    (40, 32, 8, 192, 130),       # one split a row
+])
+def test_append_inside_the_attention_equals_the_two_calls(mi, dev, B, Hq, Hkv, T_cap, T_max):
+    """mi_rope_append_attn_tiled_linear_f32 = mi_rope_kv_append_tiled_f32_i8 + mi_gqa_decode_attn_tiled_linear_f32, bit for
+    bit: rotated queries, the whole cache and the projection, for positions at block and span edges, inside the sequence,
+    past its end, past T_max, and outside the cache, and for empty sequences."""
+    mark = dev.mark()
+    lib, g, D = mi.lib, np.random.default_rng(B * 7919 + T_cap), 128
+    heads, N = Hq + 2 * Hkv, 128
+    stride = heads * D + 4
+    qkv = g.standard_normal((B, stride)).astype(np.float32)
+    angle = np.arange(T_cap)[:, None] * (10000.0 ** (-np.arange(D // 2) * (2.0 / D)))[None]
+    cos, sin = dev.upload(np.cos(angle).astype(np.float32)), dev.upload(np.sin(angle).astype(np.float32))
+    kq0, vq0 = (g.integers(-127, 128, (B, Hkv, T_cap, D)).astype(np.int8) for _ in range(2))
+    ks0, vs0 = (((g.random((B, Hkv, T_cap)) + 0.5) * 0.03).astype(np.float32) for _ in range(2))
+    qw, sw = dev.upload(g.integers(-127, 128, (N, Hq * D)).astype(np.int8)), dev.upload(g.random(N, dtype=np.float32))
+    dqkv = dev.upload(qkv)
+    q0 = g.standard_normal((B, Hq, D)).astype(np.float32)
+    ws_bytes = lib.mi_gqa_decode_attn_linear_workspace_bytes(B, Hq, Hkv, D, T_max)
+    ws = dev.empty(ws_bytes, np.uint8)
+    full = [(T_max - 1, T_max), (0, 1), (63, 64), (0, T_max), (T_max // 2, T_max), (T_cap - 1, T_max), (T_max - 1, T_max // 2 + 1),
+            (-1, T_max), (T_cap, T_max), (T_max - 1, 0), (min(64, T_max - 1), min(65, T_max))]
+    for first in range(0, len(full), min(B, len(full))):
+        cases = [full[(first + b) % len(full)] for b in range(B)]
+        pos, lens = (dev.upload(np.array(c, np.int32)) for c in zip(*cases))
+        got = []
+        for fused in (False, True):
+            q, y = dev.upload(q0), dev.empty((B, N), np.float32)
+            orot = dev.empty((B, Hq, D), np.float32)
+            cache = [dev.upload(a) for a in (kq0, ks0, vq0, vs0)]
+            c = [b.ptr for b in cache]
+            row = (dqkv.ptr, stride, cos.ptr, sin.ptr, q.ptr)
+            tail = (orot.ptr, qw.ptr, sw.ptr, y.ptr, B, Hq, Hkv, D, T_cap, lens.ptr, T_max, N, ws.ptr, ws_bytes, None)
+            if fused:
+                mi.check(lib.mi_rope_append_attn_tiled_linear_f32(*row, *c, pos.ptr, *tail))
+            else:
+                mi.check(lib.mi_rope_kv_append_tiled_f32_i8(*row, *c, pos.ptr, B, Hq, Hkv, D, T_cap, None))
+                mi.check(lib.mi_gqa_decode_attn_tiled_linear_f32(q.ptr, *c, *tail))
+            got.append([dev.download(b) for b in [q, orot, y] + cache])
+        for name, a, b in zip(("q", "o_rot", "y", "kq", "ks", "vq", "vs"), *got):
+            assert np.array_equal(a, b), (name, cases)
+    assert lib.mi_rope_append_attn_tiled_linear_f32(*row, *c, None, *tail) == mi.EINVAL
+    assert lib.mi_rope_append_attn_tiled_linear_f32(dqkv.ptr, heads * D - 4, *row[2:], *c, pos.ptr, *tail) == mi.EINVAL
+    dev.reset_to(mark)
