@@ -53,6 +53,7 @@ struct Params {
     float *part_ml;   // [B*Hkv, splits, 2, 4]   (max in log2 units, sum)
     int Hq, Hkv, G, T;
     int Tstride;              // tokens between consecutive (batch, kv head) rows of the cache, a multiple of 64
+    int splits;               // workgroups per row (gridDim.x would be one more cache line of arguments)
     const int32_t *seq_len;   // per-sequence token counts [B] (device), or null: every sequence holds T tokens
     int blocks_per_split;     // 64-token blocks per workgroup, <= NW * NT
     float score_scale;        // log2(e) / sqrt(D)
@@ -146,7 +147,7 @@ __global__ __launch_bounds__(64 * NW) void k_gqa_tiled_split(Params p)
     const int split = blockIdx.x, bkv = blockIdx.y;
     const int b = bkv / p.Hkv, kvh = bkv % p.Hkv;
     const int G = p.G;
-    const int64_t pbase = (int64_t)bkv * gridDim.x + split;
+    const int64_t pbase = (int64_t)bkv * p.splits + split;
 
     int T = p.T;
     if (p.seq_len) T = min(max(__builtin_amdgcn_readfirstlane(p.seq_len[b]), 0), p.T);
@@ -159,7 +160,7 @@ __global__ __launch_bounds__(64 * NW) void k_gqa_tiled_split(Params p)
         tp = __builtin_amdgcn_readfirstlane(p.pos[b]);
         if (tp < 0 || tp >= p.Tstride) tp = -1;
         const int at = (tp >> 6) - blk_lo;
-        const bool last = split == (int)gridDim.x - 1;
+        const bool last = split == p.splits - 1;
         if (tp >= 0 && at >= 0 && (at < p.blocks_per_split || last)) owner = wave == (at < p.blocks_per_split ? at % NW : 0);
         if (owner) {
             const int j = lane & 15;
@@ -720,6 +721,7 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
     p.q = q; p.kq = kq; p.ks = ks; p.vt = vt; p.vs = vs;
     p.Hq = (int)Hq; p.Hkv = (int)Hkv; p.G = (int)(Hq / Hkv); p.T = (int)T_max;
     p.Tstride = (int)T_cap;
+    p.splits = plan.splits;
     p.seq_len = seq_len;
     p.score_scale = 1.4426950408889634f * 0.08838834764831845f;  // log2(e) / sqrt(128)
     p.o = o; p.out_rotated = out_rotated;

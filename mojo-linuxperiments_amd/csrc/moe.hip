@@ -698,7 +698,7 @@ __device__ __forceinline__ void moe_expert_rx_body(const int8_t *__restrict__ ac
                                                          const int8_t *__restrict__ w0, const float *__restrict__ sc0,
                                                          const int8_t *__restrict__ w1, const float *__restrict__ sc1,
                                                          float *__restrict__ out, int Kdim, int Nrows, int Hout,
-                                                         int topk, int nch, int e, int bx)
+                                                         int topk, int nch, int e, int c0)
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -707,11 +707,12 @@ __device__ __forceinline__ void moe_expert_rx_body(const int8_t *__restrict__ ac
     if (count <= 0) return;
     // gate/up: the 4 waves split K (2048 bytes = 16 steps).  down: K is short (768 bytes = 6 steps), so each
     // wave takes its own 32 rows over the whole of K and nothing has to be added across waves
-    // A workgroup walks `nch` consecutive row chunks (16 rows for gate/up, 128 for down) as ONE stream: the
+    // A workgroup walks `nch` consecutive row chunks from chunk c0 on (16 rows for gate/up, 128 for down; all of them
+    // inside the expert: the loads are not checked per row beyond the first chunk) as ONE stream: the
     // loads of the next chunk are already in flight while the partial sums of this one are added and stored,
     // and the segment / permutation lookups are paid once per workgroup.
     constexpr int CHUNK_ROWS = DOWN ? 128 : 16;
-    const int n0 = DOWN ? bx * nch * 128 + wave * 32 : bx * nch * 16;
+    const int n0 = DOWN ? c0 * 128 + wave * 32 : c0 * 16;
     constexpr int RX_RING = rx_ring(DOWN), RX_RING_BYTES = rx_ring_bytes(DOWN);
     char *ring = smem + wave * (RX_RING * RX_STAGE);
     int *s_red = reinterpret_cast<int *>(smem + RX_RING_BYTES);    // [NGRP][MTT][4][64] sums over the four K slices (gate/up)
@@ -731,10 +732,10 @@ __device__ __forceinline__ void moe_expert_rx_body(const int8_t *__restrict__ ac
         float v = 0.0f;
         if (o < nch * SCW) {
             if constexpr (DOWN) {
-                const int n = (bx * nch + ch) * 128 + nl;
+                const int n = (c0 + ch) * 128 + nl;
                 if (n < Nrows) v = sc0[(int64_t)e * Nrows + n];
             } else {
-                const int n = (bx * nch + ch) * 16 + (nl & 15);
+                const int n = (c0 + ch) * 16 + (nl & 15);
                 if (n < Nrows) v = (nl < 16 ? sc0 : sc1)[(int64_t)e * Nrows + n];
             }
         }
@@ -884,7 +885,7 @@ __device__ __forceinline__ void moe_expert_rx_body(const int8_t *__restrict__ ac
         } else {
             // every wave owns its 32 rows over the whole of K: results leave straight from the accumulators, four
             // consecutive channels of one token per lane; out[pair] in pair order
-            const int nbase = (bx * nch + ch) * 128;
+            const int nbase = (c0 + ch) * 128;
 #pragma unroll
             for (int a = 0; a < NGRP; ++a) {
                 const int nl = wave * 32 + a * 16 + 4 * g_;
@@ -938,15 +939,17 @@ __global__ __launch_bounds__(256) void k_moe_expert_rx(const int8_t *__restrict_
             y = y_split + j / wpe2; bx = j - (j / wpe2) * wpe2;
         }
     }
+    const int c0 = bx * nchl;
+    nchl = min(nchl, chunks - c0);   // the last workgroup of an expert whose chunks nchl does not divide
     const int e = order[y];
     // tokens per pass follow the size of the expert's segment: every extra pass streams the weights again
     const int count = seg_off[e + 1] - seg_off[e];
     if (count <= 16)
-        moe_expert_rx_body<DOWN, NSMAX, 1>(act, act_scale, perm, seg_off, w0, sc0, w1, sc1, out, Kdim, Nrows, Hout, topk, nchl, e, bx);
+        moe_expert_rx_body<DOWN, NSMAX, 1>(act, act_scale, perm, seg_off, w0, sc0, w1, sc1, out, Kdim, Nrows, Hout, topk, nchl, e, c0);
     else if (count <= 32 || NSMAX > 6)
-        moe_expert_rx_body<DOWN, NSMAX, 2>(act, act_scale, perm, seg_off, w0, sc0, w1, sc1, out, Kdim, Nrows, Hout, topk, nchl, e, bx);
+        moe_expert_rx_body<DOWN, NSMAX, 2>(act, act_scale, perm, seg_off, w0, sc0, w1, sc1, out, Kdim, Nrows, Hout, topk, nchl, e, c0);
     else
-        moe_expert_rx_body<DOWN, NSMAX, 3>(act, act_scale, perm, seg_off, w0, sc0, w1, sc1, out, Kdim, Nrows, Hout, topk, nchl, e, bx);
+        moe_expert_rx_body<DOWN, NSMAX, 3>(act, act_scale, perm, seg_off, w0, sc0, w1, sc1, out, Kdim, Nrows, Hout, topk, nchl, e, c0);
 }
 
 // y[t, n] = sum over slots in order of w[t, slot] * out[t*topk + slot, n].  A slot whose expert index lies outside

@@ -239,6 +239,7 @@ def test_argument_errors(mi, dev):
     (16, 2048, 768, 128, 8), (17, 2048, 768, 128, 8),
     (33, 2304, 256, 256, 8),    # rows that the logits kernel does not quantize
     (128, 512, 256, 128, 8), (129, 512, 256, 128, 8),   # the last token count of one expert a wave, and the first beyond
+    (160, 1024, 768, 112, 8),   # 48 row chunks in runs of five: an expert's last workgroup has fewer
 ])
 def test_layer_of_few_tokens_equals_route_and_ffn(mi, dev, orc, T, H, I, E, topk):
     """The layer's own router launches against the separate calls: the same picks as the oracle, then the same bits."""
