@@ -325,24 +325,26 @@ __device__ __forceinline__ float readlane_f(float v, int l)
 
 // one wave per token: k rounds of (wave-wide max, lowest index among the lanes that hold it); lane l holds
 // experts l, l+64, l+128, l+192.  Ties go to the lower expert index; picks come out by descending logit.
-__global__ __launch_bounds__(256) void k_moe_topk(const float *__restrict__ logits, int32_t *__restrict__ idx,
-                                                  float *__restrict__ w, int T, int E, int topk)
+// Lane s < topk returns pick s and leaves its weight in weight.  U: the slots of 64 experts that there are.
+// The loop is one serial chain, so a slot less is a link less: the layer with four slots always and the picks' values in
+// an array of registers, before -> after: 1 token 37.9 -> 37.3 us, 16 tokens 110.1 -> 109.4, 16 of 64 experts 58.4 -> 57.6.
+template <int U>
+__device__ __forceinline__ int topk_row(const float *__restrict__ logits, int t, int E, int topk, int lane, float &weight)
 {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int t = blockIdx.x * 4 + wave;
-    if (t >= T) return;   // whole wave
-    float mine[4];
+    float mine[U];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < U; ++u) {
         const int i = lane + 64 * u;
         mine[u] = i < E ? logits[(int64_t)t * E + i] : -INFINITY;
     }
-    float top[MAX_TOPK];
-    int pick_lane = 0;       // lane s keeps pick s
+    float first = 0.0f, mine_top = 0.0f;   // of pick 0; of pick "lane"
+    int pick_lane = 0;                     // lane s keeps pick s
     for (int s = 0; s < topk; ++s) {
         // wave-wide maximum: four DPP steps leave every 16-lane row with its own maximum, four scalar reads join the
         // rows (a chain of cross-lane permutes costs five times as many cycles, and this loop is all latency)
-        float v = fmaxf(fmaxf(mine[0], mine[1]), fmaxf(mine[2], mine[3]));
+        float v = -INFINITY;               // also what a row of nothing but NaN gives
+#pragma unroll
+        for (int u = 0; u < U; ++u) v = fmaxf(v, mine[u]);
         v = fmaxf(v, dpp_f<0xB1>(v));    // quad_perm [1,0,3,2]
         v = fmaxf(v, dpp_f<0x4E>(v));    // quad_perm [2,3,0,1]
         v = fmaxf(v, dpp_f<0x124>(v));   // row_ror:4
@@ -351,7 +353,7 @@ __global__ __launch_bounds__(256) void k_moe_topk(const float *__restrict__ logi
         // lowest expert index holding v: experts of slot u are 64u .. 64u+63, so the first non-empty ballot wins
         int win = -1;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < U; ++u) {
             const unsigned long long bal = __ballot(mine[u] == v);
             if (win < 0 && bal) {
                 const int wl = __ffsll((long long)bal) - 1;
@@ -359,24 +361,38 @@ __global__ __launch_bounds__(256) void k_moe_topk(const float *__restrict__ logi
                 if (lane == wl) mine[u] = -INFINITY;   // taken
             }
         }
-        if (lane == s) pick_lane = win;
-#pragma unroll
-        for (int q = 0; q < MAX_TOPK; ++q)
-            if (q == s) top[q] = v;
+        if (win < 0 && U < 4) win = 64 * U;   // a row of nothing but NaN: an expert that is not there, which the dispatch skips
+        if (s == 0) first = v;
+        if (lane == s) pick_lane = win, mine_top = v;
     }
     // lane s evaluates e_s = expf(l_s - l_0) once; the sum runs over the picks in pick order, as the oracle's does
-    float mine_top = top[0];
-#pragma unroll
-    for (int q = 1; q < MAX_TOPK; ++q)
-        if (q == lane) mine_top = top[q];
-    const float e = lane < topk ? expf(mine_top - top[0]) : 0.0f;
+    const float e = lane < topk ? expf(mine_top - first) : 0.0f;
     float sum = 0.0f;
 #pragma unroll
     for (int q = 0; q < MAX_TOPK; ++q)
         if (q < topk) sum = sum + readlane_f(e, q);
+    weight = e / sum;
+    return pick_lane;
+}
+
+__device__ __forceinline__ int topk_row(const float *__restrict__ logits, int t, int E, int topk, int lane, float &weight)
+{
+    return E <= 64    ? topk_row<1>(logits, t, E, topk, lane, weight)
+           : E <= 128 ? topk_row<2>(logits, t, E, topk, lane, weight)
+                      : topk_row<4>(logits, t, E, topk, lane, weight);
+}
+
+__global__ __launch_bounds__(256) void k_moe_topk(const float *__restrict__ logits, int32_t *__restrict__ idx,
+                                                  float *__restrict__ w, int T, int E, int topk)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int t = blockIdx.x * 4 + wave;
+    if (t >= T) return;   // whole wave
+    float weight;
+    const int pick = topk_row(logits, t, E, topk, lane, weight);
     if (lane < topk) {
-        idx[(int64_t)t * topk + lane] = pick_lane;
-        w[(int64_t)t * topk + lane] = e / sum;
+        idx[(int64_t)t * topk + lane] = pick;
+        w[(int64_t)t * topk + lane] = weight;
     }
 }
 
