@@ -402,11 +402,10 @@ __global__ __launch_bounds__(256) void k_moe_topk(const float *__restrict__ logi
 // its expert is the number of set bits below t in row e.
 // order (optional): expert ids by descending segment size, so that the grouped GEMMs can start their longest
 // workgroups first.
-__global__ __launch_bounds__(1024) void k_moe_dispatch(const int32_t *__restrict__ idx, int32_t *__restrict__ perm,
-                                                       int32_t *__restrict__ seg_off, int32_t *__restrict__ order,
-                                                       int T, int E, int topk)
+__device__ __forceinline__ void dispatch_pairs(uint32_t *s_dyn, const int32_t *idx, int32_t *__restrict__ perm,
+                                               int32_t *__restrict__ seg_off, int32_t *__restrict__ order, int T, int E,
+                                               int topk)
 {
-    extern __shared__ uint32_t s_dyn[];
     const int W = (T + 31) >> 5;
     uint32_t *bm = s_dyn;                 // [E][W]
     uint32_t *pre = s_dyn + E * W;        // [E][W] exclusive popcount prefix
@@ -508,6 +507,41 @@ __global__ __launch_bounds__(1024) void k_moe_dispatch(const int32_t *__restrict
             perm[pos] = pr;
         }
     }
+}
+
+__global__ __launch_bounds__(1024) void k_moe_dispatch(const int32_t *__restrict__ idx, int32_t *__restrict__ perm,
+                                                       int32_t *__restrict__ seg_off, int32_t *__restrict__ order,
+                                                       int T, int E, int topk)
+{
+    extern __shared__ uint32_t s_dyn[];
+    dispatch_pairs(s_dyn, idx, perm, seg_off, order, T, E, topk);
+}
+
+// Top-k and dispatch of few tokens in one launch: a wave a token, the picks go to the dispatch
+// through LDS.  Both kernels are all latency (a launch of 4 to 5 us for a few hundred bytes), so one of the two is saved;
+// the layer's time, two launches -> one: 1 token of 128 experts 37.3 -> 36.4 us, 4 tokens 47.7 -> 46.8, 16 tokens 109.5 -> 109.1,
+// 16 of 64 experts 57.6 -> 57.0.  Beyond a token a wave the one workgroup's rounds cost more than the launch: 32 tokens
+// 123.9 -> 126.0 us, 64 tokens 138.2 -> 146.6.
+constexpr int64_t ROUTE_DISPATCH_MAX_T = 16;
+__global__ __launch_bounds__(1024) void k_moe_topk_dispatch(const float *__restrict__ logits, int32_t *__restrict__ idx,
+                                                            float *__restrict__ w, int32_t *__restrict__ perm,
+                                                            int32_t *__restrict__ seg_off, int32_t *__restrict__ order,
+                                                            int T, int E, int topk)
+{
+    __shared__ int32_t s_idx[ROUTE_DISPATCH_MAX_T * MAX_TOPK];
+    extern __shared__ uint32_t s_dyn[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (const int t = wave; t < T) {   // one token a wave
+        float weight;
+        const int pick = topk_row(logits, t, E, topk, lane, weight);
+        if (lane < topk) {
+            s_idx[t * topk + lane] = pick;
+            idx[t * topk + lane] = pick;
+            w[t * topk + lane] = weight;
+        }
+    }
+    __syncthreads();
+    dispatch_pairs(s_dyn, s_idx, perm, seg_off, order, T, E, topk);
 }
 
 // ------------------------------------------------------- a11 grouped GEMMs
@@ -1032,9 +1066,10 @@ static int32_t check_shapes(int64_t T, int64_t H, int64_t I, int64_t E, int32_t 
 // can the router's first kernel also produce the FFN's activation codes? (block 128, a wave per row)
 static bool route_can_quantize(int64_t H) { return H % 128 == 0 && H <= 2048; }
 
-// logits + top-k; qx / sx non-null (and route_can_quantize(H)): the logits kernel also rotates and quantizes x
+// logits + top-k; qx / sx non-null (and route_can_quantize(H)): the logits kernel also rotates and quantizes x;
+// perm / seg non-null (and T <= ROUTE_DISPATCH_MAX_T): the top-k kernel also dispatches
 static int32_t launch_route(const float *x, const float *wr, int32_t *idx, float *w, int64_t T, int64_t H, int64_t E,
-                            int32_t topk, float *logits, int8_t *qx, float *sx, void *stream)
+                            int32_t topk, float *logits, int8_t *qx, float *sx, int32_t *perm, int32_t *seg, void *stream)
 {
     // eight experts a wave (twice the workgroups) while sixteen would leave at most two workgroups to a compute unit,
     // one while eight would leave half of the units without any
@@ -1064,6 +1099,12 @@ static int32_t launch_route(const float *x, const float *wr, int32_t *idx, float
 #undef MI_LOGITS
     int32_t rc = launch_status();
     if (rc) return rc;
+    if (perm) {
+        const size_t words = (size_t)(2 * E * ((T + 31) / 32) + E + 1);
+        hipLaunchKernelGGL(k_moe_topk_dispatch, dim3(1), dim3(1024), words * 4, as_stream(stream), logits, idx, w, perm, seg,
+                           seg + E + 1, (int)T, (int)E, (int)topk);
+        return launch_status();
+    }
     hipLaunchKernelGGL(k_moe_topk, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, as_stream(stream), logits, idx, w, (int)T,
                        (int)E, (int)topk);
     return launch_status();
@@ -1090,7 +1131,8 @@ extern "C" int32_t mi_moe_route(const float *x, const float *wr, int32_t *idx, f
     if (!workspace || !aligned16(workspace)) return MI_EINVAL;
     if (workspace_bytes < mi_moe_route_workspace_bytes(T, E)) return MI_ENOSPC;
     if (T == 0) return MI_OK;
-    return moe::launch_route(x, wr, idx, w, T, H, E, topk, static_cast<float *>(workspace), nullptr, nullptr, stream);
+    return moe::launch_route(x, wr, idx, w, T, H, E, topk, static_cast<float *>(workspace), nullptr, nullptr, nullptr,
+                             nullptr, stream);
 }
 
 static int32_t launch_dispatch(const int32_t *idx, int32_t *perm, int32_t *seg_off, int32_t *order, int64_t T,
@@ -1134,10 +1176,11 @@ extern "C" int64_t mi_moe_ffn_workspace_offset(int32_t which, int64_t T, int64_t
 }
 
 // codes_ready: the activation codes and scales already sit in the workspace (written by the router's first kernel)
+// dispatched: so do the dispatch's outputs
 static int32_t run_ffn(const float *x, const int32_t *idx, const float *w, const int8_t *wg, const float *sg,
                        const int8_t *wu, const float *su, const int8_t *wd, const float *sd, float *y, int64_t T,
                        int64_t H, int64_t I, int64_t E, int32_t topk, void *workspace, int64_t workspace_bytes,
-                       void *stream, bool codes_ready)
+                       void *stream, bool codes_ready, bool dispatched)
 {
     int32_t rc = moe::check_shapes(T, H, I, E, topk);
     if (rc) return rc;
@@ -1160,8 +1203,10 @@ static int32_t run_ffn(const float *x, const int32_t *idx, const float *w, const
     const int64_t P = T * topk;
 
     int32_t *order = seg + E + 1;
-    rc = launch_dispatch(idx, perm, seg, order, T, E, topk, stream);
-    if (rc) return rc;
+    if (!dispatched) {
+        rc = launch_dispatch(idx, perm, seg, order, T, E, topk, stream);
+        if (rc) return rc;
+    }
     if (!codes_ready) {
         rc = mi_fwht_quant_f32_i8(x, qx, sx, T, H, 128, stream);
         if (rc) return rc;
@@ -1243,7 +1288,7 @@ extern "C" int32_t mi_moe_ffn(const float *x, const int32_t *idx, const float *w
                               int64_t T, int64_t H, int64_t I, int64_t E, int32_t topk, void *workspace,
                               int64_t workspace_bytes, void *stream)
 {
-    return run_ffn(x, idx, w, wg, sg, wu, su, wd, sd, y, T, H, I, E, topk, workspace, workspace_bytes, stream, false);
+    return run_ffn(x, idx, w, wg, sg, wu, su, wd, sd, y, T, H, I, E, topk, workspace, workspace_bytes, stream, false, false);
 }
 
 extern "C" int32_t mi_moe_layer(const float *x, const float *wr, const int8_t *wg, const float *sg, const int8_t *wu,
@@ -1262,10 +1307,12 @@ extern "C" int32_t mi_moe_layer(const float *x, const float *wr, const int8_t *w
     float *w = reinterpret_cast<float *>(ws + L.off[9]);
     // the checks of mi_moe_route, which this call stands in for
     if (!x || !wr || H % 256 || E % 16 || E > 256 || !aligned16(x) || !aligned16(wr)) return MI_EINVAL;
-    const bool fuse = moe::route_can_quantize(H);
+    const bool fuse = moe::route_can_quantize(H), few = T <= moe::ROUTE_DISPATCH_MAX_T;
     rc = moe::launch_route(x, wr, idx, w, T, H, E, topk, reinterpret_cast<float *>(ws + L.off[10]),
                            fuse ? reinterpret_cast<int8_t *>(ws + L.off[0]) : nullptr,
-                           fuse ? reinterpret_cast<float *>(ws + L.off[1]) : nullptr, stream);
+                           fuse ? reinterpret_cast<float *>(ws + L.off[1]) : nullptr,
+                           few ? reinterpret_cast<int32_t *>(ws + L.off[2]) : nullptr,
+                           few ? reinterpret_cast<int32_t *>(ws + L.off[3]) : nullptr, stream);
     if (rc) return rc;
-    return run_ffn(x, idx, w, wg, sg, wu, su, wd, sd, y, T, H, I, E, topk, workspace, workspace_bytes, stream, fuse);
+    return run_ffn(x, idx, w, wg, sg, wu, su, wd, sd, y, T, H, I, E, topk, workspace, workspace_bytes, stream, fuse, few);
 }

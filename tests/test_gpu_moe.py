@@ -236,7 +236,7 @@ def test_argument_errors(mi, dev):
 @pytest.mark.parametrize("T,H,I,E,topk", [
     (1, 256, 256, 16, 1),       # one round of the logits, one token
     (15, 1280, 512, 64, 4),     # a last batch of rounds that is not whole
-    (16, 2048, 768, 128, 8), (17, 2048, 768, 128, 8),
+    (16, 2048, 768, 128, 8), (17, 2048, 768, 128, 8),   # the last token count of one launch for top-k and dispatch, the first of two
     (33, 2304, 256, 256, 8),    # rows that the logits kernel does not quantize
     (128, 512, 256, 128, 8), (129, 512, 256, 128, 8),   # the last token count of one expert a wave, and the first beyond
     (160, 1024, 768, 112, 8),   # 48 row chunks in runs of five: an expert's last workgroup has fewer
