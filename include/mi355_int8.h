@@ -207,12 +207,19 @@ typedef struct mi_gemm_problem {
 } mi_gemm_problem;
 typedef struct mi_gemm_batch mi_gemm_batch;
 MI_API int64_t mi_gemm_batch_plan_bytes(const int64_t *mnk, int32_t n);
-/* The tile lists a batch would hold on a device of `compute_units` units, written to host memory (int32
+/* The tile lists over all n problems on a device of `compute_units` units, written to host memory (int32
  * [compute_units][per_wg][4] = problem or -1 for the end of a workgroup's list, first row, first column, cost in K
- * stages; workgroup w runs on XCD w % 8): for tests and for callers that want to look at the balance.  Returns the
- * bytes written.  Makes no device call. */
+ * stages; workgroup w runs on XCD w % 8): for tests and for callers that want to look at the balance.  A batch holds
+ * these lists where none of its problems runs in small tiles, otherwise those over the problems that are left.  Returns
+ * the bytes written.  Makes no device call. */
 MI_API int64_t mi_gemm_batch_plan_host(const int64_t *mnk, int32_t n, int32_t compute_units, int32_t *lists_out,
                                        int64_t capacity_bytes, int32_t *per_wg_out);
+/* How a batch of these shapes runs on such a device: small_out int32 [n] = 1 for a problem that runs in small tiles,
+ * 0 for one that the lists hold; tile_out int32 [2] = rows and columns of the small tiles (0, 0: there are none).
+ * Returns the bytes of the lists that mi_gemm_batch_create stores in `plan`, 0 where no problem is left for them, never
+ * more than the lists over all n problems take.  Makes no device call. */
+MI_API int64_t mi_gemm_batch_split_host(const int64_t *mnk, int32_t n, int32_t compute_units, int32_t *small_out,
+                                        int32_t *tile_out);
 MI_API int32_t mi_gemm_batch_create(const int64_t *mnk, int32_t n, void *plan, int64_t plan_bytes, mi_gemm_batch **out);
 MI_API int32_t mi_gemm_batch_destroy(mi_gemm_batch *b);
 MI_API int32_t mi_gemm_batch_run_f32(mi_gemm_batch *b, const mi_gemm_problem *problems, void *stream);

@@ -418,6 +418,12 @@ float deep_estimate(int M, int N, int K, int cus, int *which)
     return deep::with_memory(core, (double)N * K + (double)M * K + 4.0 * M * N);
 }
 
+void deep_tile(int which, int32_t *rows, int32_t *cols)
+{
+    *rows = deep::TILES[which].bm;
+    *cols = deep::TILES[which].bn;
+}
+
 template <bool DEQ>
 int32_t launch_deep(int which, const int8_t *qx, const float *sx, const int8_t *qw, const float *sw, int32_t *acc, float *y,
                     int64_t M64, int64_t N64, int64_t K64, hipStream_t s)

@@ -629,19 +629,27 @@ struct Split {
     int which = 0;   // tile of the second launch
 };
 
-// the longest workgroup of a list, in tile costs: blocks of equal K dealt longest first to the least loaded XCD
-static int64_t list_load(const int64_t *mnk, const int *idx, int n, int cus)
+// the longest workgroup of a list, in tile costs and in tiles: blocks of equal K dealt longest first to the least loaded
+// XCD, as build_lists deals them
+struct Load {
+    int64_t cost, tiles;
+};
+static Load list_load(const int64_t *mnk, const int *idx, int n, int cus)
 {
     const int nx = (cus % 8 == 0) ? 8 : 1, slots = cus / nx;
-    int64_t load[8] = {};
+    int64_t load[8] = {}, blocks[8] = {};
     for (int i = 0; i < n;) {
         const int64_t K = mnk[3 * idx[i] + 2];
         int64_t tiles = 0;
         for (; i < n && mnk[3 * idx[i] + 2] == K; ++i)
             tiles += ((mnk[3 * idx[i]] + LC::BM - 1) / LC::BM) * ((mnk[3 * idx[i] + 1] + LC::BN - 1) / LC::BN);
-        for (; tiles > 0; tiles -= slots) *std::min_element(load, load + nx) += tile_cost(K);
+        for (; tiles > 0; tiles -= slots) {
+            const int x = (int)(std::min_element(load, load + nx) - load);
+            load[x] += tile_cost(K);
+            ++blocks[x];
+        }
     }
-    return *std::max_element(load, load + nx);
+    return {*std::max_element(load, load + nx), *std::max_element(blocks, blocks + nx)};
 }
 
 static Split split_batch(const int64_t *mnk, int n, int cus)
@@ -658,11 +666,11 @@ static Split split_batch(const int64_t *mnk, int n, int cus)
         tiles += t;
         sum += t * tile_cost(mnk[3 * p + 2]);
     }
-    const int64_t load = list_load(mnk, best.tiled, n, cus);
+    const Load whole = list_load(mnk, best.tiled, n, cus);
     // nothing to level out (the small tiles cost 1.65 times as much), or so many tiles that a list is level
-    if ((double)load * cus < 1.2 * sum || tiles > 8.0 * cus) return best;
+    if ((double)whole.cost * cus < 1.2 * sum || tiles > 8.0 * cus) return best;
     // the estimates are good to a tenth: what they promise has to be more
-    float t_best = 0.9f * (3.0f + 1.36f * (float)load);
+    float t_best = 0.9f * (3.0f + 1.36f * (float)whole.cost);
     for (int mask = 1; mask < (1 << n); ++mask) {   // the problems of the second launch
         Split s;
         for (int i = 0; i < n; ++i) {
@@ -674,14 +682,36 @@ static Split split_batch(const int64_t *mnk, int n, int cus)
         for (int i = 1; i < n; ++i)
             if ((mask >> i & 1) && !(mask >> (i - 1) & 1) && !memcmp(mnk + 3 * order[i], mnk + 3 * order[i - 1], 3 * sizeof(int64_t))) skip = true;
         if (skip) continue;
+        const Load part = list_load(mnk, s.tiled, s.n_tiled, cus);
+        // without the long tiles the short ones can be dealt to fewer XCDs, more of them to a workgroup than in the whole
+        // list: such a list would not fit the memory that the whole one is given
+        if (part.tiles > whole.tiles) continue;
         float t = deep_batch_estimate(mnk, s.deep, s.n_deep, cus, &s.which);
-        if (s.n_tiled) t += 5.0f + 1.36f * (float)list_load(mnk, s.tiled, s.n_tiled, cus);
+        if (s.n_tiled) t += 5.0f + 1.36f * (float)part.cost;
         if (t < t_best) {
             t_best = t;
             best = s;
         }
     }
     return best;
+}
+
+// What a batch holds: its split and the list of split.tiled (entries count problems in that order).  Returns the list's
+// bytes, at most those of the list over all problems, which mi_gemm_batch_plan_bytes promises; 0: no problem is left for it.
+static int64_t plan_batch(const int64_t *mnk, int n, int cus, Split *split, std::vector<v4i> *lists, int *per_wg)
+{
+    const int64_t whole = build_lists<LC::BM, LC::BN>(mnk, n, cus, lists, per_wg);
+    if (whole < 0) return whole;
+    *split = split_batch(mnk, n, cus);
+    if (!split->n_deep) {
+        for (int i = 0; i < n; ++i) split->tiled[i] = i;
+        return whole;
+    }
+    if (!split->n_tiled) return 0;
+    int64_t sub[3 * MAX_PROBLEMS];
+    for (int i = 0; i < split->n_tiled; ++i)
+        for (int k = 0; k < 3; ++k) sub[3 * i + k] = mnk[3 * split->tiled[i] + k];
+    return build_lists<LC::BM, LC::BN>(sub, split->n_tiled, cus, lists, per_wg);
 }
 
 static int32_t check_shapes(const int64_t *mnk, int32_t n)
@@ -733,6 +763,24 @@ extern "C" int64_t mi_gemm_batch_plan_host(const int64_t *mnk, int32_t n, int32_
     return bytes;
 }
 
+extern "C" int64_t mi_gemm_batch_split_host(const int64_t *mnk, int32_t n, int32_t compute_units_, int32_t *small_out,
+                                            int32_t *tile_out)
+{
+    int32_t rc = list::check_shapes(mnk, n);
+    if (rc) return rc;
+    if (compute_units_ < 1 || compute_units_ > 4096 || !small_out || !tile_out) return MI_EINVAL;
+    list::Split split;
+    std::vector<v4i> lists;
+    int per_wg = 0;
+    const int64_t bytes = list::plan_batch(mnk, n, compute_units_, &split, &lists, &per_wg);
+    if (bytes < 0) return bytes;
+    for (int i = 0; i < n; ++i) small_out[i] = 0;
+    for (int i = 0; i < split.n_deep; ++i) small_out[split.deep[i]] = 1;
+    tile_out[0] = tile_out[1] = 0;
+    if (split.n_deep) deep_tile(split.which, &tile_out[0], &tile_out[1]);
+    return bytes;
+}
+
 extern "C" int32_t mi_gemm_batch_create(const int64_t *mnk, int32_t n, void *plan, int64_t plan_bytes,
                                         mi_gemm_batch **out)
 {
@@ -744,21 +792,12 @@ extern "C" int32_t mi_gemm_batch_create(const int64_t *mnk, int32_t n, void *pla
     std::vector<v4i> lists;
     int per_wg = 0;
     const int cus = compute_units();
-    const int64_t whole = list::build_lists<list::LC::BM, list::LC::BN>(mnk, n, cus, &lists, &per_wg);
-    if (whole < 0) return (int32_t)whole;
-    if (plan_bytes < whole) return MI_ENOSPC;
-    list::Split split = list::split_batch(mnk, n, cus);
-    int64_t bytes = whole;
-    if (split.n_deep) {
-        int64_t sub[3 * list::MAX_PROBLEMS];
-        for (int i = 0; i < split.n_tiled; ++i)
-            for (int k = 0; k < 3; ++k) sub[3 * i + k] = mnk[3 * split.tiled[i] + k];
-        bytes = 0;
-        if (split.n_tiled) bytes = list::build_lists<list::LC::BM, list::LC::BN>(sub, split.n_tiled, cus, &lists, &per_wg);
-        if (bytes < 0 || bytes > plan_bytes) return MI_ENOSPC;
-    } else {
-        for (int i = 0; i < n; ++i) split.tiled[i] = i;
-    }
+    const int64_t room = list::build_lists<list::LC::BM, list::LC::BN>(mnk, n, cus, nullptr, nullptr);
+    if (room < 0) return (int32_t)room;
+    if (plan_bytes < room) return MI_ENOSPC;
+    list::Split split;
+    const int64_t bytes = list::plan_batch(mnk, n, cus, &split, &lists, &per_wg);
+    if (bytes < 0) return (int32_t)bytes;
     int dev = 0;
     MI_HIP(hipGetDevice(&dev));
     if (bytes) MI_HIP(hipMemcpy(plan, lists.data(), (size_t)bytes, hipMemcpyHostToDevice));   // returns when the list is in place

@@ -88,6 +88,7 @@ SIGNATURES = {
     "mi_dequant_i32_f32": (i32, [vp, vp, vp, vp, i64, i64, vp]),
     "mi_gemm_batch_plan_bytes": (i64, [vp, i32]),
     "mi_gemm_batch_plan_host": (i64, [vp, i32, i32, vp, i64, C.POINTER(i32)]),
+    "mi_gemm_batch_split_host": (i64, [vp, i32, i32, vp, vp]),
     "mi_gemm_batch_create": (i32, [vp, i32, vp, i64, C.POINTER(vp)]),
     "mi_gemm_batch_destroy": (i32, [vp]),
     "mi_gemm_batch_run_f32": (i32, [vp, vp, vp]),

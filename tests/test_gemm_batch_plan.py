@@ -49,6 +49,42 @@ def test_every_output_is_covered_once_or_with_equal_tiles(mi, shapes, cus):
         assert int(c.sum()) == tiles * BM * BN
 
 
+def split(mi, shapes, cus=256):
+    """(bytes of the stored lists, which problems run in small tiles, the small tile)"""
+    n = len(shapes)
+    mnk = (C.c_int64 * (3 * n))(*[v for s in shapes for v in s])
+    small, tile = np.zeros(n, np.int32), np.zeros(2, np.int32)
+    nbytes = mi.lib.mi_gemm_batch_split_host(mnk, n, cus, small.ctypes.data, tile.ctypes.data)
+    assert nbytes >= 0, nbytes
+    return nbytes, small.tolist(), tuple(tile)
+
+
+def test_stored_lists_fit_the_memory_that_the_caller_was_told_to_bring(mi):
+    """Where some problems run in small tiles the lists over the others are dealt anew; they are never longer than the
+    lists over all problems, whose size mi_gemm_batch_plan_bytes returns."""
+    rng = np.random.default_rng(23)
+    kinds = set()
+    batches = [
+        [(1869, 1680, 7168), (1869, 272, 512), (1869, 6848, 5504), (1869, 5792, 640)],
+        [(1204, 11008, 7424), (1204, 1360, 1920), (1204, 704, 14464), (1204, 624, 3328)] + [(1204, 704, 640)] * 3 +
+        [(1204, 1248, 1408)],
+        [(1536, 3072, 1024), (1536, 8816, 5504), (1536, 1024, 11008)],
+        [(700, 14336, 4096), (700, 4096, 28672), (700, 14336, 11008)],
+        CFG3,
+    ]
+    for _ in range(400):
+        M = int(rng.integers(256, 2049))
+        batches.append([(M, 16 * int(rng.integers(16, 900)), 128 * int(rng.integers(3, 113)))
+                        for _ in range(int(rng.integers(1, 9)))])
+    for shapes in batches:
+        nbytes, small, tile = split(mi, shapes)
+        assert nbytes <= plan(mi, shapes).nbytes, shapes
+        assert (nbytes == 0) == all(small) and any(small) == (tile != (0, 0)), shapes
+        kinds.add("all" if all(small) else "some" if any(small) else "none")
+    assert kinds == {"all", "some", "none"}
+    assert split(mi, CFG3) == (plan(mi, CFG3).nbytes, [0] * 4, (0, 0))
+
+
 def test_addresses_formed_from_a_tile_stay_inside(mi):
     """Replays the kernel's address arithmetic for the first and last tile rows/columns of a problem: global byte
     offsets of the direct-to-LDS loads (wave w of eight fills blocks w + 8q: row (w + 8q) * 8 + rho of the tile,
