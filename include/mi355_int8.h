@@ -351,7 +351,8 @@ MI_API int32_t mi_gqa_decode_attn_tiled_linear_f32(const float *q, const int8_t 
                                                    void *workspace, int64_t workspace_bytes, void *stream);
 /* ... and with the rotary embedding and the append in front of it: mi_rope_kv_append_tiled_f32_i8 followed by
  * mi_gqa_decode_attn_tiled_linear_f32 on q_out, bit for bit, the append done by the attention kernel.  A sequence whose
- * pos lies outside [0, T_cap) appends nothing and attends with the rows that q_out holds.  q_out 16-byte aligned. */
+ * pos lies outside [0, T_cap) appends nothing and attends with the rows that q_out holds.  q_out 16-byte aligned.  Where
+ * q_out or o_rot overlaps qkv, or o_rot q_out, the two calls are made as they are. */
 MI_API int32_t mi_rope_append_attn_tiled_linear_f32(const float *qkv, int64_t row_stride, const float *rope_cos,
                                                     const float *rope_sin, float *q_out, int8_t *kt, float *ks,
                                                     int8_t *vt, float *vs, const int32_t *pos, float *o_rot,

@@ -913,6 +913,17 @@ extern "C" int32_t mi_rope_append_attn_tiled_linear_f32(const float *qkv, int64_
     if (rc) return rc;
     if (!rope_cos || !rope_sin || !aligned16(rope_cos) || !aligned16(rope_sin) || Hq <= 0) return MI_EINVAL;
     if (row_stride < (Hq + 2 * Hkv) * D || row_stride % 4) return MI_EINVAL;
+    // The attention kernel stores rows of q_out (and, with one split, of o_rot) while other workgroups still read qkv, and
+    // both in no order among each other: a caller whose buffers overlap gets the two launches.
+    const int64_t out_bytes = B * Hq * D * 4, qkv_bytes = ((B - 1) * row_stride + (Hq + 2 * Hkv) * D) * 4;
+    if (overlaps(q_out, out_bytes, qkv, qkv_bytes) || overlaps(o_rot, out_bytes, qkv, qkv_bytes) ||
+        overlaps(o_rot, out_bytes, q_out, out_bytes)) {
+        rc = mi_rope_kv_append_tiled_f32_i8(qkv, row_stride, rope_cos, rope_sin, q_out, kq, ks, vt, vs, pos, B, Hq, Hkv, D,
+                                            T_cap, stream);
+        if (rc) return rc;
+        return attn_linear(q_out, kq, ks, vt, vs, o_rot, qw, sw, y, B, Hq, Hkv, D, T_cap, seq_len, T_max, N, workspace,
+                           workspace_bytes, stream, nullptr);
+    }
     const StepIn step = {qkv, row_stride, rope_cos, rope_sin, pos};
     return attn_linear(q_out, kq, ks, vt, vs, o_rot, qw, sw, y, B, Hq, Hkv, D, T_cap, seq_len, T_max, N, workspace,
                        workspace_bytes, stream, &step);

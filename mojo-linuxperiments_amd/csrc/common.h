@@ -36,6 +36,13 @@ inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s);
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline bool aligned4(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0; }
+// do the byte ranges [a, a + an) and [b, b + bn) share a byte (null = no range)
+inline bool overlaps(const void *a, int64_t an, const void *b, int64_t bn)
+{
+    if (!a || !b) return false;
+    const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+    return pa < pb + (uintptr_t)bn && pb < pa + (uintptr_t)an;
+}
 
 int32_t compute_units();   // of the current device, cached
 int32_t lds_limit();       // largest LDS allocation of one workgroup on the current device, cached

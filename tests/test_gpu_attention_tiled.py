@@ -495,3 +495,42 @@ def test_append_inside_the_attention_equals_the_two_calls(mi, dev, B, Hq, Hkv, T
     assert lib.mi_rope_append_attn_tiled_linear_f32(*row, *c, None, *tail) == mi.EINVAL
     assert lib.mi_rope_append_attn_tiled_linear_f32(dqkv.ptr, heads * D - 4, *row[2:], *c, pos.ptr, *tail) == mi.EINVAL
     dev.reset_to(mark)
+
+
+@pytest.mark.parametrize("T", [40, 3000])   # one split, which writes the output rows itself, and many
+@pytest.mark.parametrize("q_at,o_at", [("qkv", None), ("qkv", "qkv"), (None, "qkv"), ("both", "both")])
+def test_append_inside_the_attention_with_overlapping_buffers(mi, dev, T, q_at, o_at):
+    """q_out or o_rot over the query heads of the one sequence's fused QKV row, or one buffer for both: still what the two
+    calls give."""
+    mark = dev.mark()
+    lib, g, D = mi.lib, np.random.default_rng(T), 128
+    Hq, Hkv, T_cap, N = 8, 2, 3072, 128
+    heads = Hq + 2 * Hkv
+    qkv0 = g.standard_normal((1, heads * D)).astype(np.float32)
+    angle = np.arange(T_cap)[:, None] * (10000.0 ** (-np.arange(D // 2) * (2.0 / D)))[None]
+    cos, sin = dev.upload(np.cos(angle).astype(np.float32)), dev.upload(np.sin(angle).astype(np.float32))
+    cache0 = [g.integers(-127, 128, (1, Hkv, T_cap, D)).astype(np.int8), (g.random((1, Hkv, T_cap)) * 0.03).astype(np.float32)] * 2
+    qw, sw = dev.upload(g.integers(-127, 128, (N, Hq * D)).astype(np.int8)), dev.upload(g.random(N, dtype=np.float32))
+    pos, lens = dev.upload(np.array([T - 1], np.int32)), dev.upload(np.array([T], np.int32))
+    ws_bytes = lib.mi_gqa_decode_attn_linear_workspace_bytes(1, Hq, Hkv, D, T)
+    ws = dev.empty(ws_bytes, np.uint8)
+    got = []
+    for fused in (False, True):
+        qkv, both = dev.upload(qkv0), dev.empty((Hq, D), np.float32)
+        q, o = dev.empty((Hq, D), np.float32).ptr, dev.empty((Hq, D), np.float32).ptr
+        q = {None: q, "qkv": qkv.ptr, "both": both.ptr}[q_at]
+        o = {None: o, "qkv": qkv.ptr, "both": both.ptr}[o_at]
+        y, cache = dev.empty((1, N), np.float32), [dev.upload(a) for a in cache0]
+        c = [b.ptr for b in cache]
+        row = (qkv.ptr, heads * D, cos.ptr, sin.ptr, q)
+        tail = (o, qw.ptr, sw.ptr, y.ptr, 1, Hq, Hkv, D, T_cap, lens.ptr, T, N, ws.ptr, ws_bytes, None)
+        if fused:
+            mi.check(lib.mi_rope_append_attn_tiled_linear_f32(*row, *c, pos.ptr, *tail))
+        else:
+            mi.check(lib.mi_rope_kv_append_tiled_f32_i8(*row, *c, pos.ptr, 1, Hq, Hkv, D, T_cap, None))
+            mi.check(lib.mi_gqa_decode_attn_tiled_linear_f32(q, *c, *tail))
+        got.append([dev.download(mi.DevBuf(p, (Hq, D), np.float32)) for p in (q, o)] +
+                   [dev.download(b) for b in [qkv, y] + cache])
+    for name, a, b in zip(("q", "o_rot", "qkv", "y", "kq", "ks", "vq", "vs"), *got):
+        assert np.array_equal(a, b), name
+    dev.reset_to(mark)
