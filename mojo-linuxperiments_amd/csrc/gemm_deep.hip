@@ -35,6 +35,7 @@ namespace mi {
 namespace deep {
 
 typedef __attribute__((address_space(3))) void *lptr_t;
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));   // four scales: a batch asks only 4 bytes of alignment of them
 
 template <int N>
 __device__ __forceinline__ void wait_vm()
@@ -141,7 +142,7 @@ __device__ __forceinline__ void tile(const int8_t *__restrict__ qx, const int8_t
     const int mw = m0 + wm * TM * 16, nw = n0 + wn * TN * 16;
     const bool lo = r < 8;
     float sxv[OWN];
-    float4 swv[OWN];
+    f4u swv[OWN];
     if constexpr (DEQ) {
 #pragma unroll
         for (int o = 0; o < OWN; ++o) {
@@ -149,11 +150,11 @@ __device__ __forceinline__ void tile(const int8_t *__restrict__ qx, const int8_t
             if constexpr (C::PAIR) {   // of an even and an odd tile side by side, see the stores
                 const int m = mw + i * 16 + (o & 1) * 8 + (r & 7), n = nw + (j & ~1) * 16 + (lo ? 0 : 16) + 4 * g;
                 sxv[o] = sx[min(m, M - 1)];
-                if (!(o & 1)) swv[o] = *reinterpret_cast<const float4 *>(sw + min(n, N - 4));
+                if (!(o & 1)) swv[o] = *reinterpret_cast<const f4u *>(sw + min(n, N - 4));
             } else {
                 const int m = mw + i * 16 + r, n = nw + j * 16 + 4 * g;
                 sxv[o] = sx[min(m, M - 1)];
-                swv[o] = *reinterpret_cast<const float4 *>(sw + min(n, N - 4));
+                swv[o] = *reinterpret_cast<const f4u *>(sw + min(n, N - 4));
             }
         }
     }
@@ -236,7 +237,7 @@ __device__ __forceinline__ void tile(const int8_t *__restrict__ qx, const int8_t
         for (int w = 0; w < WK - 1; ++w) sum[o] += *reinterpret_cast<const v4i *>(part + (f * (WK - 1) + w) * 1024);
     }
     // a lane holds channels 4 g .. + 3 of token r of a tile
-    auto put = [&](const v4i &v, float sxm, const float4 &s4, int m, int n) {
+    auto put = [&](const v4i &v, float sxm, const f4u &s4, int m, int n) {
         if (m >= M || n >= N) return;
         const int64_t at = (int64_t)m * N + n;
         if constexpr (DEQ) {

@@ -85,6 +85,27 @@ def test_batch_with_small_tiles(mi, dev, orc, shapes):
 
 
 @pytest.mark.parametrize("shapes", [
+    [(300, 2048, 896), (256, 1040, 2176)],     # in small tiles
+    [(2048, 6144, 384)],                       # in the list
+])
+def test_batch_scales_need_four_bytes_of_alignment(mi, dev, orc, shapes):
+    mark = dev.mark()
+    batch = mi.GemmBatch(dev, shapes)
+    ops, host = make_ops(dev, shapes, 31, np.float32)
+    moved = []
+    for (qx, _, qw, _, y), (_, sx, _, sw) in zip(ops, host):
+        dsx, dsw = (dev.upload(np.concatenate([np.zeros(k, np.float32), v])).offset(4 * k, v.shape, np.float32)
+                    for k, v in ((3, sx), (1, sw)))
+        moved.append((qx, dsx, qw, dsw, y))
+    batch.run_f32(moved)
+    dev.sync()
+    for o, (qx, sx, qw, sw) in zip(moved, host):
+        assert np.array_equal(dev.download(o[4]), orc.dequant(orc.gemm_i8_i32(qx, qw), sx, sw))
+    batch.destroy()
+    dev.reset_to(mark)
+
+
+@pytest.mark.parametrize("shapes", [
     [(256, 256, 384)],
     [(300, 272, 512)],
     [(2048, 6144, 384), (520, 4096, 1024)],
