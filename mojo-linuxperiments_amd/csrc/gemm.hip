@@ -1,4 +1,4 @@
-// C ABI of the W8A8 contraction: argument checks and the choice between the GEMV for one token, the deep-pipelined
+// C ABI of the W8A8 contraction: argument checks and the choice between the GEMV for very few tokens, the deep-pipelined
 // small-tile kernel and the LDS-tiled kernel for sizes that fill the chip.
 #include <atomic>
 
@@ -8,11 +8,12 @@
 namespace mi {
 template <bool DEQ>
 int32_t launch_gemv(const int8_t *, const float *, const int8_t *, const float *, int32_t *, float *, int64_t, int64_t,
-                    hipStream_t);
+                    int64_t, hipStream_t);
 template <bool DEQ>
 int32_t launch_tiled(const int8_t *, const float *, const int8_t *, const float *, int32_t *, float *, int64_t,
                      int64_t, int64_t, hipStream_t);
 
+bool gemv_takes(int M, int N, int K, int cus);
 float tiled_estimate(int M, int N, int K, int cus);
 
 int32_t launch_linear_fused(const float *, const int8_t *, const float *, float *, int8_t *, float *, int64_t, int64_t,
@@ -44,14 +45,11 @@ int32_t gemm_dispatch(const int8_t *qx, const float *sx, const int8_t *qw, const
                       int64_t M, int64_t N, int64_t K, hipStream_t s)
 {
     if (M == 0) return MI_OK;
-    // one token: the GEMV that keeps its activation codes in registers, where K splits for it
-    if (M == 1) {
-        const int32_t rc = y ? launch_gemv<true>(qx, sx, qw, sw, nullptr, y, N, K, s)
-                             : launch_gemv<false>(qx, nullptr, qw, nullptr, acc, nullptr, N, K, s);
-        if (rc != MI_ERANGE) return rc;
-    }
-    // by the two kernels' own estimates; at most 64 rows never fill the large tiles
     const int cus = compute_units();
+    if (gemv_takes((int)M, (int)N, (int)K, cus))
+        return y ? launch_gemv<true>(qx, sx, qw, sw, nullptr, y, M, N, K, s)
+                 : launch_gemv<false>(qx, nullptr, qw, nullptr, acc, nullptr, M, N, K, s);
+    // by the two kernels' own estimates; at most 64 rows never fill the large tiles
     int which = 0;
     const float deep = deep_estimate((int)M, (int)N, (int)K, cus, &which);
     if (M <= 64 || deep < tiled_estimate((int)M, (int)N, (int)K, cus)) {

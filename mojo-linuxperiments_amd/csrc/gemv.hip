@@ -1,13 +1,13 @@
-// W8A8 contraction for one token (decode GEMV):
-//   acc[n] = sum_k qx[k] * qw[n,k],   y = ((float)acc * sx) * sw[n]
+// W8A8 contraction for one token, and for two to four where they have few rows of a long K (decode GEMV):
+//   acc[m,n] = sum_k qx[m,k] * qw[n,k],   y = ((float)acc * sx[m]) * sw[n]
 // The weights [N,K] are read from HBM exactly once; everything else is small.
-// Bound: HBM.  Algorithmic bytes per call = N*K (weights) + K (codes) + 4*N (output) + 4*(N+1) (scales).
+// Bound: HBM.  Algorithmic bytes per call = N*K (weights) + M*K (codes) + 4*M*N (output) + 4*(N+M) (scales).
 //
 //  k_gemv_reg: a lane always works on the same byte offsets of a weight row, so its share of the activation codes
 //  lives in registers for the whole kernel: no LDS and no barrier in the streaming part, 16 x 1 KB weight loads in
 //  flight per wave, v_dot4_i32_i8, one transposed butterfly per wave.
 //  k_gemv_fused is the same kernel with the rotate + quantize prologue (and optionally the RMSNorm) inside, for
-//  K <= 4096.
+//  one token and K <= 4096.
 #include <algorithm>
 #include "common.h"
 #include "fwht_core.h"
@@ -42,16 +42,16 @@ constexpr int pow2_ceil(int v) { int p = 1; while (p < v) p <<= 1; return p; }
 
 // K = 1024 * CW * QW up to a ragged last chunk: lane l always works on the same byte offsets of a row (16*l + 1024*c
 // for the wave's CW chunks).  A wave issues all the loads of its R rows at once (R*CW <= 16 x 1 KB in flight per wave),
-// runs v_dot4_i32_i8 on them and reduces its R per-lane sums with one transposed butterfly.  QW waves that split a row
-// add their totals in LDS.
-template <int CW, bool DEQ>
+// runs v_dot4_i32_i8 on them and reduces its R * MB per-lane sums with one transposed butterfly.  QW waves that split a row
+// add their totals in LDS.  MB: tokens, M of which are there.
+template <int MB, int CW, bool DEQ>
 __global__ __launch_bounds__(256) void k_gemv_reg(const int8_t *__restrict__ qx, const int8_t *__restrict__ qw,
                                                   const float *__restrict__ sx, const float *__restrict__ sw,
-                                                  int32_t *__restrict__ acc_out, float *__restrict__ y, int N, int K,
-                                                  int QW)
+                                                  int32_t *__restrict__ acc_out, float *__restrict__ y, int M, int N,
+                                                  int K, int QW)
 {
     constexpr int R = (16 / CW) < 1 ? 1 : (16 / CW);   // rows per wave
-    constexpr int V = pow2_ceil(R);
+    constexpr int V = pow2_ceil(R * MB);
     __shared__ int s_red[4][V];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int q = wave % QW;                  // which CW-chunk slice of the row
@@ -68,27 +68,31 @@ __global__ __launch_bounds__(256) void k_gemv_reg(const int8_t *__restrict__ qx,
             w[r][c] = (row0 + r < N && off < K) ? *reinterpret_cast<const v4i *>(qw + (int64_t)(row0 + r) * K + off)
                                                 : (v4i){0, 0, 0, 0};
         }
-    v4i xr[CW];
+    v4i xr[MB][CW];
 #pragma unroll
-    for (int c = 0; c < CW; ++c) {
-        const int off = kbase + c * 1024;
-        xr[c] = off < K ? *reinterpret_cast<const v4i *>(qx + off) : (v4i){0, 0, 0, 0};
-    }
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int c = 0; c < CW; ++c) {
+            const int off = kbase + c * 1024, ms = MB == 1 || m < M ? m : M - 1;
+            xr[m][c] = off < K ? *reinterpret_cast<const v4i *>(qx + (int64_t)ms * K + off) : (v4i){0, 0, 0, 0};
+        }
     int p[V];
 #pragma unroll
     for (int i = 0; i < V; ++i) p[i] = 0;
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-        int a = 0;
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int c = 0; c < CW; ++c) {
-            a = __builtin_amdgcn_sdot4(w[r][c][0], xr[c][0], a, false);
-            a = __builtin_amdgcn_sdot4(w[r][c][1], xr[c][1], a, false);
-            a = __builtin_amdgcn_sdot4(w[r][c][2], xr[c][2], a, false);
-            a = __builtin_amdgcn_sdot4(w[r][c][3], xr[c][3], a, false);
+        for (int m = 0; m < MB; ++m) {
+            int a = 0;
+#pragma unroll
+            for (int c = 0; c < CW; ++c) {
+                a = __builtin_amdgcn_sdot4(w[r][c][0], xr[m][c][0], a, false);
+                a = __builtin_amdgcn_sdot4(w[r][c][1], xr[m][c][1], a, false);
+                a = __builtin_amdgcn_sdot4(w[r][c][2], xr[m][c][2], a, false);
+                a = __builtin_amdgcn_sdot4(w[r][c][3], xr[m][c][3], a, false);
+            }
+            p[r * MB + m] = a;
         }
-        p[r] = a;
-    }
     fold_sum<V, 32>(p, lane);
     // lane l holds value v = l >> SH; the first lane of each group of 64/V lanes speaks for it
     constexpr int SH = 6 - __builtin_ctz(V);
@@ -102,11 +106,11 @@ __global__ __launch_bounds__(256) void k_gemv_reg(const int8_t *__restrict__ qx,
             for (int o = 1; o < QW; ++o) total += s_red[wave + o][v];
         }
     }
-    if (q == 0 && speaker && v < R) {
-        const int n = row0 + v;
-        if (n < N) {
-            if constexpr (DEQ) y[n] = ((float)total * sx[0]) * sw[n];
-            else acc_out[n] = total;
+    if (q == 0 && speaker && v < R * MB) {
+        const int m = v % MB, n = row0 + v / MB;
+        if (n < N && m < M) {
+            if constexpr (DEQ) y[(int64_t)m * N + n] = ((float)total * sx[m]) * sw[n];
+            else acc_out[(int64_t)m * N + n] = total;
         }
     }
 }
@@ -395,43 +399,73 @@ int32_t launch_norm_linear_fused(const float *x, const float *res, const float *
     return MI_EINVAL;
 }
 
-template <int CW, bool DEQ>
+template <int MB, int CW, bool DEQ>
 static int32_t launch_reg(const int8_t *qx, const float *sx, const int8_t *qw, const float *sw, int32_t *acc,
-                          float *y, int N, int K, int QW, hipStream_t s)
+                          float *y, int M, int N, int K, int QW, hipStream_t s)
 {
     constexpr int R = (16 / CW) < 1 ? 1 : (16 / CW);
     const int rows_per_wg = (4 / QW) * R;
     const unsigned grid = (unsigned)((N + rows_per_wg - 1) / rows_per_wg);
-    hipLaunchKernelGGL((k_gemv_reg<CW, DEQ>), dim3(grid), dim3(256), 0, s, qx, qw, sx, sw, acc, y, N, K, QW);
+    hipLaunchKernelGGL((k_gemv_reg<MB, CW, DEQ>), dim3(grid), dim3(256), 0, s, qx, qw, sx, sw, acc, y, M, N, K, QW);
     return launch_status();
 }
 
-// MI_ERANGE: a K that the kernel does not split (the caller takes the small-tile kernel)
+// K = 1024 * CW * QW (last chunk may be ragged) with CW <= 7 chunks per wave and QW in {1, 2, 4} waves per row; 0: no such QW
+static int gemv_split(int K)
+{
+    const int nchunk = (K + 1023) >> 10;
+    for (int QW = 1; QW <= 4; QW <<= 1)
+        if (nchunk % QW == 0 && nchunk / QW <= 7) return QW;
+    return 0;
+}
+
+// Whether the GEMV takes M tokens, by measurement against the small-tile kernel (weights from HBM, us GEMV : small tiles).
+// One token: wherever K splits (4096 -> 14336 12.4, 14336 -> 4096 12.4); of the others K = 11008 -> 4096 takes 12.5 in
+// small tiles.  Two to four: the small tiles read the codes once per 16 rows instead of once per one to three rows and win
+// (2 tokens, 4096 -> 4096 6.0 : 5.8), but up to 8 rows a unit they leave half of the units idle behind a long
+// chain of stages: 2 tokens, 5632 -> 512 3.6 : 4.3, 7168 -> 1024 4.1 : 4.7, 5632 -> 2048 4.9 : 5.4, 8064 -> 2048 6.1 : 7.1,
+// and 4 tokens, 7168 -> 512 4.4 : 4.6, 8064 -> 2048 6.7 : 6.9.  The lines lie where the two met in a scan of K from 2048 to 8064
+// in steps of 384 and N from 16 to 4096.
+bool gemv_takes(int M, int N, int K, int cus)
+{
+    if (M == 1) return gemv_split(K) != 0;
+    if (M > 4 || K >= 8192) return false;
+    return M == 2 ? (N <= 4 * cus && K > 4096) || (N <= 8 * cus && K > 5376)
+                  : (N <= 3 * cus && K > 5376) || (N <= 8 * cus && K > 7168);
+}
+
+template <int MB, int CW0, bool DEQ>
+static int32_t launch_tokens(const int8_t *qx, const float *sx, const int8_t *qw, const float *sw, int32_t *acc, float *y,
+                             int M, int N, int K, hipStream_t s)
+{
+    const int QW = gemv_split(K);
+    switch (((K + 1023) >> 10) / QW) {
+    case 1: if constexpr (CW0 <= 1) return launch_reg<MB, 1, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s); break;
+    case 2: if constexpr (CW0 <= 2) return launch_reg<MB, 2, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s); break;
+    case 3: if constexpr (CW0 <= 3) return launch_reg<MB, 3, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s); break;
+    case 4: return launch_reg<MB, 4, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
+    case 5: return launch_reg<MB, 5, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
+    case 6: return launch_reg<MB, 6, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
+    case 7: return launch_reg<MB, 7, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
+    }
+    return MI_EINVAL;
+}
+
+// for what gemv_takes
 template <bool DEQ>
 int32_t launch_gemv(const int8_t *qx, const float *sx, const int8_t *qw, const float *sw, int32_t *acc, float *y,
-                    int64_t N64, int64_t K64, hipStream_t s)
+                    int64_t M64, int64_t N64, int64_t K64, hipStream_t s)
 {
-    const int N = (int)N64, K = (int)K64;
-    // K = 1024 * CW * QW (last chunk may be ragged) with CW <= 7 chunks per wave and QW in {1, 2, 4} waves per row
-    const int nchunk = (K + 1023) >> 10;
-    for (int QW = 1; QW <= 4; QW <<= 1) {
-        if (nchunk % QW || nchunk / QW > 7) continue;
-        switch (nchunk / QW) {
-        case 1: return launch_reg<1, DEQ>(qx, sx, qw, sw, acc, y, N, K, QW, s);
-        case 2: return launch_reg<2, DEQ>(qx, sx, qw, sw, acc, y, N, K, QW, s);
-        case 3: return launch_reg<3, DEQ>(qx, sx, qw, sw, acc, y, N, K, QW, s);
-        case 4: return launch_reg<4, DEQ>(qx, sx, qw, sw, acc, y, N, K, QW, s);
-        case 5: return launch_reg<5, DEQ>(qx, sx, qw, sw, acc, y, N, K, QW, s);
-        case 6: return launch_reg<6, DEQ>(qx, sx, qw, sw, acc, y, N, K, QW, s);
-        default: return launch_reg<7, DEQ>(qx, sx, qw, sw, acc, y, N, K, QW, s);
-        }
-    }
-    return MI_ERANGE;
+    const int M = (int)M64, N = (int)N64, K = (int)K64;
+    if (M < 1 || M > 4 || !gemv_split(K)) return MI_EINVAL;
+    if (M == 1) return launch_tokens<1, 1, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, s);
+    if (M == 2) return launch_tokens<2, 4, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, s);   // five to eight chunks
+    return launch_tokens<4, 4, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, s);
 }
 
 template int32_t launch_gemv<true>(const int8_t *, const float *, const int8_t *, const float *, int32_t *, float *,
-                                   int64_t, int64_t, hipStream_t);
+                                   int64_t, int64_t, int64_t, hipStream_t);
 template int32_t launch_gemv<false>(const int8_t *, const float *, const int8_t *, const float *, int32_t *, float *,
-                                    int64_t, int64_t, hipStream_t);
+                                    int64_t, int64_t, int64_t, hipStream_t);
 
 }  // namespace mi

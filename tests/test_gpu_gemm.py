@@ -93,6 +93,26 @@ def test_small_tile_kernel_bit_exact(mi, dev, orc, M, N, K):
     assert np.array_equal(y, orc.dequant(want, sx, sw))
 
 
+@pytest.mark.parametrize("M,N,K", [
+    # two to four tokens in the GEMV: its smallest and largest N and K on a chip of 256 units, five to eight chunks of K, a
+    # last chunk that is not whole, rows past N in the last workgroup, three tokens in the kernel for four
+    (2, 16, 4224), (2, 1024, 4992), (2, 1024, 5120), (2, 2048, 5504), (2, 1040, 6144), (2, 528, 7168), (2, 2048, 8064),
+    (3, 16, 5504), (3, 768, 6016), (3, 1040, 7296), (4, 768, 5504), (4, 272, 6656), (4, 2048, 7296), (4, 1296, 8064),
+])
+def test_gemv_of_few_tokens_bit_exact(mi, dev, orc, M, N, K):
+    qx, qw = rand_codes(M + N + K, (M, K)), rand_codes(K + 13, (N, K))
+    want = orc.gemm_i8_i32(qx, qw)
+    assert np.array_equal(gpu_gemm_i32(mi, dev, qx, qw), want)
+    g = np.random.default_rng(N)
+    sx, sw = g.uniform(0.01, 1, M).astype(np.float32), g.uniform(0.001, 0.1, N).astype(np.float32)
+    mark = dev.mark()
+    dy = dev.empty((M, N), np.float32)
+    mi.gemm_dequant(dev.upload(qx), dev.upload(sx), dev.upload(qw), dev.upload(sw), dy)
+    y = dev.download(dy)
+    dev.reset_to(mark)
+    assert np.array_equal(y, orc.dequant(want, sx, sw))
+
+
 def test_random_skinny_shapes_bit_exact(mi, dev, orc):
     """Seeded random shapes over every skinny path (1 to 64 tokens, K of 1 to 39 stages, N any multiple of 16 or a
     multiple of 2048, which takes the evenly dealt ring kernels): exact against the oracle."""
