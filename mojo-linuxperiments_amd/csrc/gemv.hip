@@ -43,19 +43,19 @@ constexpr int pow2_ceil(int v) { int p = 1; while (p < v) p <<= 1; return p; }
 // K = 1024 * CW * QW up to a ragged last chunk: lane l always works on the same byte offsets of a row (16*l + 1024*c
 // for the wave's CW chunks).  A wave issues all the loads of its R rows at once (R*CW <= 16 x 1 KB in flight per wave),
 // runs v_dot4_i32_i8 on them and reduces its R * MB per-lane sums with one transposed butterfly.  QW waves that split a row
-// add their totals in LDS.  MB: tokens, M of which are there.
-template <int MB, int CW, bool DEQ>
-__global__ __launch_bounds__(256) void k_gemv_reg(const int8_t *__restrict__ qx, const int8_t *__restrict__ qw,
+// add their totals in LDS.  MB: tokens, M of which are there.  WG: waves of the workgroup, a multiple of QW.
+template <int MB, int CW, int WG, bool DEQ>
+__global__ __launch_bounds__(64 * WG) void k_gemv_reg(const int8_t *__restrict__ qx, const int8_t *__restrict__ qw,
                                                   const float *__restrict__ sx, const float *__restrict__ sw,
                                                   int32_t *__restrict__ acc_out, float *__restrict__ y, int M, int N,
                                                   int K, int QW)
 {
     constexpr int R = (16 / CW) < 1 ? 1 : (16 / CW);   // rows per wave
     constexpr int V = pow2_ceil(R * MB);
-    __shared__ int s_red[4][V];
+    __shared__ int s_red[WG][V];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int q = wave % QW;                  // which CW-chunk slice of the row
-    const int rows_per_wg = (4 / QW) * R;
+    const int rows_per_wg = (WG / QW) * R;
     const int row0 = blockIdx.x * rows_per_wg + (wave / QW) * R;
     const int kbase = q * CW * 1024 + lane * 16;
 
@@ -399,54 +399,61 @@ int32_t launch_norm_linear_fused(const float *x, const float *res, const float *
     return MI_EINVAL;
 }
 
-template <int MB, int CW, bool DEQ>
+template <int MB, int CW, int WG, bool DEQ>
 static int32_t launch_reg(const int8_t *qx, const float *sx, const int8_t *qw, const float *sw, int32_t *acc,
                           float *y, int M, int N, int K, int QW, hipStream_t s)
 {
     constexpr int R = (16 / CW) < 1 ? 1 : (16 / CW);
-    const int rows_per_wg = (4 / QW) * R;
+    const int rows_per_wg = (WG / QW) * R;
     const unsigned grid = (unsigned)((N + rows_per_wg - 1) / rows_per_wg);
-    hipLaunchKernelGGL((k_gemv_reg<MB, CW, DEQ>), dim3(grid), dim3(256), 0, s, qx, qw, sx, sw, acc, y, M, N, K, QW);
+    hipLaunchKernelGGL((k_gemv_reg<MB, CW, WG, DEQ>), dim3(grid), dim3(64 * WG), 0, s, qx, qw, sx, sw, acc, y, M, N, K, QW);
     return launch_status();
 }
 
-// K = 1024 * CW * QW (last chunk may be ragged) with CW <= 7 chunks per wave and QW in {1, 2, 4} waves per row; 0: no such QW
+// Waves that share a row: the fewest whose shares of K = 1024 * chunks are equal and at most 7 chunks, else the fewest
+// whose shares are at most 7 chunks (the last wave's is shorter); 0: more than 16.
 static int gemv_split(int K)
 {
     const int nchunk = (K + 1023) >> 10;
     for (int QW = 1; QW <= 4; QW <<= 1)
         if (nchunk % QW == 0 && nchunk / QW <= 7) return QW;
+    for (int QW = 2; QW <= 16; QW <<= 1)
+        if (nchunk <= 7 * QW) return QW;
     return 0;
 }
 
 // Whether the GEMV takes M tokens, by measurement against the small-tile kernel (weights from HBM, us GEMV : small tiles).
-// One token: wherever K splits (4096 -> 14336 12.4, 14336 -> 4096 12.4); of the others K = 11008 -> 4096 takes 12.5 in
-// small tiles.  Two to four: the small tiles read the codes once per 16 rows instead of once per one to three rows and win
-// (2 tokens, 4096 -> 4096 6.0 : 5.8), but up to 8 rows a unit they leave half of the units idle behind a long
-// chain of stages: 2 tokens, 5632 -> 512 3.6 : 4.3, 7168 -> 1024 4.1 : 4.7, 5632 -> 2048 4.9 : 5.4, 8064 -> 2048 6.1 : 7.1,
-// and 4 tokens, 7168 -> 512 4.4 : 4.6, 8064 -> 2048 6.7 : 6.9.  The lines lie where the two met in a scan of K from 2048 to 8064
-// in steps of 384 and N from 16 to 4096.
+// One token: wherever K splits (11264 -> 1024 4.9 : 7.9, 15360 -> 256 4.2 : 9.2, 27648 -> 28672 123.5 : 133), but for shares so
+// uneven that the waves move more than a tenth less than they could (9, 17 or 33 chunks): there from 12 to 40 rows a unit are
+// faster in small tiles (8320 -> 8192 14.0 : 13.3, 33792 -> 4096 22.9 : 21.9), fewer and more are not (8320 -> 2048 6.5 : 7.5,
+// 17408 -> 14336 43.1 : 44.4).
+// Two to four: the small tiles read the codes once per 16 rows instead of once per one to three rows and win (2 tokens,
+// 2048 -> 1024 2.8 : 2.5), but up to 8 rows a unit they leave half of the units idle behind a long chain of stages:
+// 2 tokens, 5632 -> 512 3.6 : 4.3, 7168 -> 1024 4.1 : 4.7, 8064 -> 2048 6.1 : 7.1, and 4 tokens, 7168 -> 512 4.4 : 4.6,
+// 8064 -> 2048 6.7 : 6.9.  The lines lie where the two met in a scan of K from 2048 to 7808 in steps of 384 and N from 16 to
+// 3072, for each number of tokens.
 bool gemv_takes(int M, int N, int K, int cus)
 {
-    if (M == 1) return gemv_split(K) != 0;
+    const int QW = gemv_split(K), nchunk = (K + 1023) >> 10;
+    if (!QW) return false;
+    if (M == 1) return 10 * QW * ((nchunk + QW - 1) / QW) <= 11 * nchunk || N <= 12 * cus || N > 40 * cus;
     if (M > 4 || K >= 8192) return false;
-    return M == 2 ? (N <= 4 * cus && K > 4096) || (N <= 8 * cus && K > 5376)
-                  : (N <= 3 * cus && K > 5376) || (N <= 8 * cus && K > 7168);
+    return M == 2 ? (N <= 5 * cus && K > 3072) || (N <= 8 * cus && K > 4096) || (N <= 12 * cus && K > 7168)
+                  : (N <= 6 * cus && K > 5120) || (N <= 8 * cus && K > 5760);
 }
 
-template <int MB, int CW0, bool DEQ>
+template <int MB, int CW0, int WG, bool DEQ>
 static int32_t launch_tokens(const int8_t *qx, const float *sx, const int8_t *qw, const float *sw, int32_t *acc, float *y,
-                             int M, int N, int K, hipStream_t s)
+                             int M, int N, int K, int QW, hipStream_t s)
 {
-    const int QW = gemv_split(K);
-    switch (((K + 1023) >> 10) / QW) {
-    case 1: if constexpr (CW0 <= 1) return launch_reg<MB, 1, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s); break;
-    case 2: if constexpr (CW0 <= 2) return launch_reg<MB, 2, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s); break;
-    case 3: if constexpr (CW0 <= 3) return launch_reg<MB, 3, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s); break;
-    case 4: return launch_reg<MB, 4, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
-    case 5: return launch_reg<MB, 5, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
-    case 6: return launch_reg<MB, 6, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
-    case 7: return launch_reg<MB, 7, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
+    switch ((((K + 1023) >> 10) + QW - 1) / QW) {
+    case 1: if constexpr (CW0 <= 1) return launch_reg<MB, 1, WG, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s); break;
+    case 2: if constexpr (CW0 <= 2) return launch_reg<MB, 2, WG, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s); break;
+    case 3: if constexpr (CW0 <= 3) return launch_reg<MB, 3, WG, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s); break;
+    case 4: return launch_reg<MB, 4, WG, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
+    case 5: return launch_reg<MB, 5, WG, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
+    case 6: return launch_reg<MB, 6, WG, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
+    case 7: return launch_reg<MB, 7, WG, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
     }
     return MI_EINVAL;
 }
@@ -457,10 +464,13 @@ int32_t launch_gemv(const int8_t *qx, const float *sx, const int8_t *qw, const f
                     int64_t M64, int64_t N64, int64_t K64, hipStream_t s)
 {
     const int M = (int)M64, N = (int)N64, K = (int)K64;
-    if (M < 1 || M > 4 || !gemv_split(K)) return MI_EINVAL;
-    if (M == 1) return launch_tokens<1, 1, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, s);
-    if (M == 2) return launch_tokens<2, 4, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, s);   // five to eight chunks
-    return launch_tokens<4, 4, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, s);
+    const int QW = gemv_split(K);
+    if (M < 1 || M > 4 || !QW || (M > 1 && QW > 2)) return MI_EINVAL;
+    if (QW == 16) return launch_tokens<1, 4, 16, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);   // 57 to 112 chunks
+    if (QW == 8) return launch_tokens<1, 4, 8, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);     // 29 to 56
+    if (M == 1) return launch_tokens<1, 1, 4, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
+    if (M == 2) return launch_tokens<2, 4, 4, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);      // four to eight
+    return launch_tokens<4, 4, 4, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, QW, s);
 }
 
 template int32_t launch_gemv<true>(const int8_t *, const float *, const int8_t *, const float *, int32_t *, float *,

@@ -94,10 +94,17 @@ def test_small_tile_kernel_bit_exact(mi, dev, orc, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [
-    # two to four tokens in the GEMV: its smallest and largest N and K on a chip of 256 units, five to eight chunks of K, a
+    # two to four tokens in the GEMV: its smallest and largest N and K on a chip of 256 units, four to eight chunks of K, a
     # last chunk that is not whole, rows past N in the last workgroup, three tokens in the kernel for four
+    (2, 16, 3200), (2, 1280, 3968), (2, 3072, 7296), (3, 16, 5248), (4, 1536, 5376), (4, 2048, 5888),
     (2, 16, 4224), (2, 1024, 4992), (2, 1024, 5120), (2, 2048, 5504), (2, 1040, 6144), (2, 528, 7168), (2, 2048, 8064),
     (3, 16, 5504), (3, 768, 6016), (3, 1040, 7296), (4, 768, 5504), (4, 272, 6656), (4, 2048, 7296), (4, 1296, 8064),
+    # one token whose waves have unequal shares of K: two, four, eight and sixteen waves a row at their fewest and most chunks,
+    # a last wave with one chunk less and with one chunk in all, rows past N in the last workgroup; the first K beyond, and
+    # sizes on both sides of the small tiles' share
+    (1, 16, 8320), (1, 272, 11264), (1, 1040, 13312), (1, 96, 15360), (1, 48, 20608), (1, 64, 26752), (1, 32, 28672),
+    (1, 112, 28800), (1, 48, 57344), (1, 32, 57472), (1, 80, 66560), (1, 16, 114688), (1, 16, 114816), (1, 3072, 8320),
+    (1, 3088, 8320), (1, 10240, 8448), (1, 10256, 8448),
 ])
 def test_gemv_of_few_tokens_bit_exact(mi, dev, orc, M, N, K):
     qx, qw = rand_codes(M + N + K, (M, K)), rand_codes(K + 13, (N, K))
