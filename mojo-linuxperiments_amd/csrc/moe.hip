@@ -1072,10 +1072,20 @@ static int32_t launch_route(const float *x, const float *wr, int32_t *idx, float
                             int32_t topk, float *logits, int8_t *qx, float *sx, int32_t *perm, int32_t *seg, void *stream)
 {
     // eight experts a wave (twice the workgroups) while sixteen would leave at most two workgroups to a compute unit,
-    // one while eight would leave half of the units without any
+    // one while eight would leave half of the units without any.  One a wave requests eight rounds of 256 floats at a time,
+    // also where the row ends before: fewer token groups where that is most of them.  Router alone, us eight -> one, groups x E:
+    // H = 256, 256 5.9 -> 5.3, 384 5.9 -> 6.3; H = 1024, 512 7.8 -> 6.9, 1024 7.8 -> 9.2; H = 1536, 768 9.0 -> 7.7, 1024 9.0 -> 9.4;
+    // H = 3072, 1024 12.4 -> 14.0; a layer at 1024, H = 2048 67.4 -> 64.2, H = 4096 109 -> 102.
     const int64_t groups = (T + 15) / 16;
-    const int ew = groups * (E / 8) <= compute_units() / 2 ? 1 : groups * (E / 16) <= 2 * (int64_t)compute_units() ? 8 : 16;
-    const dim3 grid((unsigned)groups, (unsigned)(E / ew));
+    const int cus = compute_units(), nj = (int)(H / 256);
+    const int64_t few = nj == 1 ? cus / 8 : std::max(cus / 4, cus / 2 * nj / ((nj + 7) / 8 * 8));
+    const int ew = groups * (E / 8) <= few ? 1 : groups * (E / 16) <= 2 * (int64_t)cus ? 8 : 16;
+    // one expert a wave: a multiple of 8 in x keeps the E workgroups of a token group on one XCD, which then reads the group's
+    // rows once.  It pays where the activations are more than an XCD's 4 MB of L2: router alone, 16 experts, us without -> with,
+    // H = 4096, 269 tokens 11.1 -> 9.4, 1005 tokens 47.0 -> 15.6; below, the XCDs that get a group less cost more than it gives
+    // (H = 2048, 64 experts, 141 tokens 7.8 -> 9.5).
+    const int64_t gx = ew == 1 && T * H > (1 << 20) ? (groups + 7) / 8 * 8 : groups;
+    const dim3 grid((unsigned)gx, (unsigned)(E / ew));
     const int cq = qx ? (int)((H / 8 + 63) / 64) : 0;
 #define MI_LOGITS(CQ_)                                                                                                  \
     do {                                                                                                                \

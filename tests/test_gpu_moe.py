@@ -29,7 +29,12 @@ def gpu_route(mi, dev, x, wr, topk):
 
 
 @pytest.mark.parametrize("T,H,E,topk", [(512, 2048, 128, 8), (7, 256, 16, 2), (33, 512, 64, 8), (5, 1024, 256, 4),
-                                        (1, 2048, 128, 1)])
+                                        (1, 2048, 128, 1),
+                                        # the last and the first token count of one expert a wave for rows of one, two, six and
+                                        # twelve rounds, and more activations than an XCD's L2 holds (groups dealt by eights)
+                                        (32, 256, 128, 2), (33, 256, 128, 2), (128, 512, 64, 4), (129, 512, 64, 4),
+                                        (384, 1536, 32, 2), (385, 1536, 32, 2), (768, 3072, 16, 2), (769, 3072, 16, 2),
+                                        (256, 4096, 16, 2), (257, 4096, 16, 2), (1009, 4096, 16, 4)])
 def test_router_indices_exact_weights_close(mi, dev, orc, T, H, E, topk):
     x = workload.activations(41, T, H)
     wr = workload.weights(42, E, H)
@@ -238,7 +243,9 @@ def test_argument_errors(mi, dev):
     (15, 1280, 512, 64, 4),     # a last batch of rounds that is not whole
     (16, 2048, 768, 128, 8), (17, 2048, 768, 128, 8),   # the last token count of one launch for top-k and dispatch, the first of two
     (33, 2304, 256, 256, 8),    # rows that the logits kernel does not quantize
-    (128, 512, 256, 128, 8), (129, 512, 256, 128, 8),   # the last token count of one expert a wave, and the first beyond
+    (64, 512, 256, 128, 8), (65, 512, 256, 128, 8),     # the last token count of one expert a wave, and the first beyond
+    (128, 512, 256, 128, 8), (129, 512, 256, 128, 8),   # eight experts a wave
+    (520, 2048, 256, 16, 2),    # token groups dealt by eights, the last three without tokens, and quantized rows
     (160, 1024, 768, 112, 8),   # 48 row chunks in runs of five: an expert's last workgroup has fewer
 ])
 def test_layer_of_few_tokens_equals_route_and_ffn(mi, dev, orc, T, H, I, E, topk):
