@@ -186,6 +186,10 @@ MI_API int32_t mi_w8a8_gemm_i32(const int8_t *qx, const int8_t *qw, int32_t *acc
 MI_API int32_t mi_w8a8_gemm_dequant_f32(const int8_t *qx, const float *sx,
                                         const int8_t *qw, const float *sw, float *y,
                                         int64_t M, int64_t N, int64_t K, void *stream);
+/* Which kernel these two calls run for a shape on a device of `compute_units` units: 0 the GEMV, 1 the small-tile kernel,
+ * 2 the LDS-tiled kernel, 3 its form with two waves per SIMD; tile_out int32 [2] = rows and columns of its tiles (0, 0 for
+ * the GEMV).  MI_EINVAL / MI_ERANGE for what they refuse and for M = 0.  Makes no device call. */
+MI_API int32_t mi_w8a8_gemm_route_host(int64_t M, int64_t N, int64_t K, int32_t compute_units, int32_t *tile_out);
 /* a4 for several contractions at once: ONE launch whose workgroups (one per compute unit) walk a list of 256 x 256
  * output tiles drawn from every problem of the batch, so that no problem's tile count has to divide by the number
  * of compute units, and no launch gap or first memory round trip lies between the problems.  Where such a list would be

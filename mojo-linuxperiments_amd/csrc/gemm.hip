@@ -15,6 +15,7 @@ int32_t launch_tiled(const int8_t *, const float *, const int8_t *, const float 
 
 bool gemv_takes(int M, int N, int K, int cus);
 float tiled_estimate(int M, int N, int K, int cus);
+bool tiled_tile(int M, int N, int cus, int32_t *rows, int32_t *cols);
 
 int32_t launch_linear_fused(const float *, const int8_t *, const float *, float *, int8_t *, float *, int64_t, int64_t,
                             int64_t, hipStream_t, bool);
@@ -31,34 +32,49 @@ __global__ void k_dequant(const int32_t *__restrict__ acc, const float *__restri
     }
 }
 
-static int32_t check_gemm(const void *qx, const void *qw, const void *out, int64_t M, int64_t N, int64_t K)
+static int32_t check_sizes(int64_t M, int64_t N, int64_t K)
 {
-    if (!qx || !qw || !out || M < 0 || N <= 0 || K <= 0) return MI_EINVAL;
+    if (M < 0 || N <= 0 || K <= 0) return MI_EINVAL;
     if (K % 128 || N % 16) return MI_EINVAL;
     if (M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return MI_ERANGE;
     if ((int64_t)127 * 127 * K > 0x7fffffffLL) return MI_ERANGE;  // int32 accumulator bound
+    return MI_OK;
+}
+
+static int32_t check_gemm(const void *qx, const void *qw, const void *out, int64_t M, int64_t N, int64_t K)
+{
+    if (!qx || !qw || !out) return MI_EINVAL;
+    const int32_t rc = check_sizes(M, N, K);
+    if (rc) return rc;
     if (!aligned16(qx) || !aligned16(qw) || !aligned16(out)) return MI_EINVAL;
     return MI_OK;
+}
+
+// Which kernel: 0 the GEMV, 1 the small-tile kernel (`which` is its tile), 2 the LDS-tiled kernels
+static int gemm_route(int M, int N, int K, int cus, int *which)
+{
+    if (gemv_takes(M, N, K, cus)) return 0;
+    // by the two kernels' own estimates; at most 64 rows never fill the large tiles
+    const float deep = deep_estimate(M, N, K, cus, which);
+    return (M <= 64 || deep < tiled_estimate(M, N, K, cus)) && deep_fits(*which, M, N) ? 1 : 2;
 }
 
 int32_t gemm_dispatch(const int8_t *qx, const float *sx, const int8_t *qw, const float *sw, int32_t *acc, float *y,
                       int64_t M, int64_t N, int64_t K, hipStream_t s)
 {
     if (M == 0) return MI_OK;
-    const int cus = compute_units();
-    if (gemv_takes((int)M, (int)N, (int)K, cus))
+    int which = 0;
+    switch (gemm_route((int)M, (int)N, (int)K, compute_units(), &which)) {
+    case 0:
         return y ? launch_gemv<true>(qx, sx, qw, sw, nullptr, y, M, N, K, s)
                  : launch_gemv<false>(qx, nullptr, qw, nullptr, acc, nullptr, M, N, K, s);
-    // by the two kernels' own estimates; at most 64 rows never fill the large tiles
-    int which = 0;
-    const float deep = deep_estimate((int)M, (int)N, (int)K, cus, &which);
-    if (M <= 64 || deep < tiled_estimate((int)M, (int)N, (int)K, cus)) {
-        const int32_t rc = y ? launch_deep<true>(which, qx, sx, qw, sw, nullptr, y, M, N, K, s)
-                             : launch_deep<false>(which, qx, nullptr, qw, nullptr, acc, nullptr, M, N, K, s);
-        if (rc != MI_ERANGE) return rc;   // more tiles than it counts
+    case 1:
+        return y ? launch_deep<true>(which, qx, sx, qw, sw, nullptr, y, M, N, K, s)
+                 : launch_deep<false>(which, qx, nullptr, qw, nullptr, acc, nullptr, M, N, K, s);
+    default:
+        return y ? launch_tiled<true>(qx, sx, qw, sw, nullptr, y, M, N, K, s)
+                 : launch_tiled<false>(qx, nullptr, qw, nullptr, acc, nullptr, M, N, K, s);
     }
-    return y ? launch_tiled<true>(qx, sx, qw, sw, nullptr, y, M, N, K, s)
-             : launch_tiled<false>(qx, nullptr, qw, nullptr, acc, nullptr, M, N, K, s);
 }
 }  // namespace mi
 
@@ -79,6 +95,19 @@ extern "C" int32_t mi_w8a8_gemm_dequant_f32(const int8_t *qx, const float *sx, c
     if (rc) return rc;
     if (!sx || !sw || !aligned4(sx) || !aligned16(sw)) return MI_EINVAL;
     return gemm_dispatch(qx, sx, qw, sw, nullptr, y, M, N, K, as_stream(stream));
+}
+
+extern "C" int32_t mi_w8a8_gemm_route_host(int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_out)
+{
+    const int32_t rc = check_sizes(M, N, K);
+    if (rc) return rc;
+    if (M == 0 || cus < 1 || cus > 4096 || !tile_out) return MI_EINVAL;
+    int which = 0;
+    const int kind = gemm_route((int)M, (int)N, (int)K, cus, &which);
+    tile_out[0] = tile_out[1] = 0;
+    if (kind == 1) deep_tile(which, &tile_out[0], &tile_out[1]);
+    if (kind == 2) return tiled_tile((int)M, (int)N, cus, &tile_out[0], &tile_out[1]) ? 3 : 2;
+    return kind;
 }
 
 extern "C" int32_t mi_dequant_i32_f32(const int32_t *acc, const float *sx, const float *sw, float *y, int64_t M,

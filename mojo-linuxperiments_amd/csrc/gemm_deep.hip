@@ -300,10 +300,9 @@ __global__ __launch_bounds__(C::TPB) void k_w8a8_deep(const int8_t *__restrict__
 }
 
 // false: more tiles than the kernel's arithmetic covers
-template <typename C>
-static bool tile_grid(int M, int N, int *tiles, int *tiles_m, unsigned *magic)
+static bool tile_grid(int bm, int bn, int M, int N, int *tiles, int *tiles_m, unsigned *magic)
 {
-    const int64_t tm = ((int64_t)M + C::BM - 1) / C::BM, all = tm * (((int64_t)N + C::BN - 1) / C::BN);
+    const int64_t tm = ((int64_t)M + bm - 1) / bm, all = tm * (((int64_t)N + bn - 1) / bn);
     if (all > (1 << 24) || all * tm >= (1ll << 32)) return false;
     *tiles = (int)all;
     *tiles_m = (int)tm;
@@ -337,7 +336,7 @@ static int32_t launch_batch(Batch &b, hipStream_t s)
     for (int i = 0; i < b.n; ++i) {
         DeepProblem &p = b.p[i];
         if (p.M <= 0 || p.N <= 0 || p.N % 16 || p.K < 128 || p.K % 128) return MI_EINVAL;
-        if (!tile_grid<C>(p.M, p.N, &p.tiles, &p.tiles_m, &p.magic)) return MI_ERANGE;
+        if (!tile_grid(C::BM, C::BN, p.M, p.N, &p.tiles, &p.tiles_m, &p.magic)) return MI_ERANGE;
         p.first = (int)grid;
         grid += (p.tiles + 7) / 8 * 8;
         if (grid > 0x7fffffff / C::TPB) return MI_ERANGE;
@@ -356,7 +355,7 @@ static int32_t launch(const int8_t *qx, const float *sx, const int8_t *qw, const
     MI_LDS_OPT_IN((&k_w8a8_deep<C, DEQ>), C::LDS);
     int tiles, tiles_m;
     unsigned magic;
-    if (!tile_grid<C>(M, N, &tiles, &tiles_m, &magic)) return MI_ERANGE;
+    if (!tile_grid(C::BM, C::BN, M, N, &tiles, &tiles_m, &magic)) return MI_ERANGE;
     hipLaunchKernelGGL((k_w8a8_deep<C, DEQ>), dim3((unsigned)(tiles + 7) / 8 * 8), dim3(C::TPB), C::LDS, s, qx, qw, M, N, K,
                        tiles, tiles_m, magic, sx, sw, out);
     return launch_status();
@@ -423,6 +422,13 @@ void deep_tile(int which, int32_t *rows, int32_t *cols)
 {
     *rows = deep::TILES[which].bm;
     *cols = deep::TILES[which].bn;
+}
+
+bool deep_fits(int which, int M, int N)
+{
+    int tiles, tiles_m;
+    unsigned magic;
+    return deep::tile_grid(deep::TILES[which].bm, deep::TILES[which].bn, M, N, &tiles, &tiles_m, &magic);
 }
 
 template <bool DEQ>

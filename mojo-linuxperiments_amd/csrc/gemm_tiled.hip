@@ -447,6 +447,22 @@ float tiled_estimate(int M, int N, int K, int cus)
     return c0[p] + c1[p] * (float)rounds * (float)(K >> 7);
 }
 
+// one tile per compute unit of a shape that divides evenly: two waves per SIMD on the same wave tile
+static bool paired(int pick, int M, int N)
+{
+    return (pick == 2 || pick == 3) && M % (32 * SHAPES[pick].tm) == 0 && N % (32 * SHAPES[pick].tn) == 0;
+}
+
+// the tile that launch_tiled takes, and whether gemm_pair.hip computes it
+bool tiled_tile(int M, int N, int cus, int32_t *rows, int32_t *cols)
+{
+    int64_t rounds;
+    const int pick = pick_shape(M, N, cus, &rounds);
+    *rows = 32 * SHAPES[pick].tm;
+    *cols = 32 * SHAPES[pick].tn;
+    return paired(pick, M, N);
+}
+
 template <bool DEQ>
 int32_t launch_tiled(const int8_t *qx, const float *sx, const int8_t *qw, const float *sw, int32_t *acc, float *y,
                      int64_t M64, int64_t N64, int64_t K64, hipStream_t s)
@@ -454,8 +470,7 @@ int32_t launch_tiled(const int8_t *qx, const float *sx, const int8_t *qw, const 
     const int M = (int)M64, N = (int)N64, K = (int)K64;
     int64_t rounds;
     const int pick = pick_shape(M, N, compute_units(), &rounds);
-    // one tile per compute unit of a shape that divides evenly: two waves per SIMD on the same wave tile
-    if ((pick == 2 || pick == 3) && M % (32 * SHAPES[pick].tm) == 0 && N % (32 * SHAPES[pick].tn) == 0)
+    if (paired(pick, M, N))
         return launch_pair<DEQ>(SHAPES[pick].tm, SHAPES[pick].tn, qx, sx, qw, sw, acc, y, M, N, K, s);
     switch (pick) {
     case 0: return launch_shape<8, 8, DEQ>(qx, sx, qw, sw, acc, y, M, N, K, s);

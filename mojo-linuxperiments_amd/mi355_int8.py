@@ -85,6 +85,7 @@ SIGNATURES = {
     "mi_fwht_f32": (i32, [vp, vp, i64, i64, i32, vp]),
     "mi_w8a8_gemm_i32": (i32, [vp, vp, vp, i64, i64, i64, vp]),
     "mi_w8a8_gemm_dequant_f32": (i32, [vp, vp, vp, vp, vp, i64, i64, i64, vp]),
+    "mi_w8a8_gemm_route_host": (i32, [i64, i64, i64, i32, vp]),
     "mi_dequant_i32_f32": (i32, [vp, vp, vp, vp, i64, i64, vp]),
     "mi_gemm_batch_plan_bytes": (i64, [vp, i32]),
     "mi_gemm_batch_plan_host": (i64, [vp, i32, i32, vp, i64, C.POINTER(i32)]),

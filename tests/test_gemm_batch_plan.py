@@ -24,6 +24,7 @@ def plan(mi, shapes, cus=256):
 
 @pytest.mark.parametrize("shapes,cus", [
     (CFG3, 256), ([(300, 272, 512)], 256), ([(256, 256, 384)], 256), ([(2048, 6144, 384)] * 8, 256),
+    ([(1066, 7264, 384)], 256), ([(735, 4512, 640), (1191, 2464, 512), (780, 3264, 384)], 256),   # ragged lists that a batch holds
     ([(1000, 1008, 384), (4096, 272, 512)], 64), (CFG3, 304), ([(777, 4096, 1024)], 7),
 ])
 def test_every_output_is_covered_once_or_with_equal_tiles(mi, shapes, cus):
@@ -85,6 +86,30 @@ def test_stored_lists_fit_the_memory_that_the_caller_was_told_to_bring(mi):
     assert split(mi, CFG3) == (plan(mi, CFG3).nbytes, [0] * 4, (0, 0))
 
 
+def test_route_of_a_single_contraction(mi):
+    """0: GEMV, 1: small tiles, 2: LDS-tiled, 3: its paired form, with the tile; what the calls refuse is refused."""
+    tile = np.zeros(2, np.int32)
+
+    def r(M, N, K, cus=256):
+        return mi.lib.mi_w8a8_gemm_route_host(M, N, K, cus, tile.ctypes.data), tuple(tile.tolist())
+
+    assert r(1, 4096, 4096) == (0, (0, 0)) and r(2, 1024, 7168) == (0, (0, 0))
+    assert r(16, 4096, 4096)[0] == 1 and r(1, 16, 114816)[0] == 1
+    assert r(2048, 6144, 4096) == (3, (256, 192)) and r(2000, 6144, 4096) == (2, (256, 192))
+    assert r(4096, 4096, 256) == (2, (256, 256)) and r(509, 14336, 4096) == (2, (128, 256))
+    rng = np.random.default_rng(3)
+    for _ in range(2000):
+        M, N, K = int(rng.integers(1, 3000)), 16 * int(rng.integers(1, 2000)), 128 * int(rng.integers(1, 128))
+        kind, (bm, bn) = r(M, N, K)
+        assert kind in (0, 1, 2, 3) and (kind == 0) == (bm == 0) and (kind != 0 or M <= 4) and (kind < 2 or M > 64)
+        assert kind != 3 or (M % bm == 0 and N % bn == 0)
+    # more rows of tiles than the small-tile kernel counts
+    assert r(1 << 30, 16, 128)[0] == 2
+    for bad in [(0, 16, 128), (-1, 16, 128), (1, 8, 128), (1, 16, 64), (1, 0, 128), (1, 16, 128, 0)]:
+        assert r(*bad)[0] == mi.EINVAL, bad
+    assert r(1, 16, 1 << 18)[0] == mi.ERANGE and r(1 << 31, 16, 128)[0] == mi.ERANGE
+
+
 def test_addresses_formed_from_a_tile_stay_inside(mi):
     """Replays the kernel's address arithmetic for the first and last tile rows/columns of a problem: global byte
     offsets of the direct-to-LDS loads (wave w of eight fills blocks w + 8q: row (w + 8q) * 8 + rho of the tile,
@@ -94,7 +119,8 @@ def test_addresses_formed_from_a_tile_stay_inside(mi):
     XSTAGE, WSTAGE = NBX * 1024, NBW * 1024
     XAREA, STAGES = 2 * XSTAGE, 2 * XSTAGE + 3 * WSTAGE
     assert STAGES == 160 * 1024
-    for M, N, K in [(2048, 14336, 4096), (300, 272, 512), (256, 256, 384), (2048, 4096, 14336)]:
+    for M, N, K in [(2048, 14336, 4096), (300, 272, 512), (256, 256, 384), (2048, 4096, 14336), (1066, 7264, 384),
+                    (1667, 4784, 3200)]:
         lists = plan(mi, [(M, N, K)])
         tiles = lists[lists[:, :, 0] >= 0]
         for _, m0, n0, _ in tiles[[0, -1]]:

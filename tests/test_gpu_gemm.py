@@ -1,4 +1,4 @@
-"""GPU parity: W8A8 contraction (skinny GEMV and LDS-tiled MFMA GEMM), the
+"""GPU parity: W8A8 contraction (GEMV, small-tile and LDS-tiled matrix kernels), the
 dequant epilogue and the whole rotated linear.  Gates: int32 accumulators and
 int8 codes bit-exact; dequantized fp32 within rel-L2 1e-3 (in fact equal)."""
 import numpy as np
@@ -26,9 +26,8 @@ def gpu_gemm_i32(mi, dev, qx, qw):
 @pytest.mark.parametrize("M,N,K", [
     (1, 64, 128), (1, 6144, 4096), (4, 4096, 14336), (16, 256, 4096), (13, 48, 1024),
     (17, 64, 768), (32, 4096, 4096), (33, 128, 2048), (48, 160, 256), (64, 512, 1408),
-    (2, 96, 9216), (3, 80, 11264),    # K that the register-resident GEMV cannot split: the LDS-staged one
-    # 5 to 16 tokens with N = 8 * 256 * P rows: the ring kernel with the rows dealt to the compute units in 8-row
-    # blocks, P = 3, 5, 7 as two workgroups of unequal size per unit, P = 10, 12, 14 as two equal ones
+    (2, 96, 9216), (3, 80, 11264),    # a long K for few rows, in small tiles
+    # 5 to 16 tokens with thousands of rows: one to many tiles per compute unit
     (16, 6144, 4096), (5, 6144, 1024), (16, 10240, 1024), (9, 14336, 2048), (16, 14336, 4096),
     (16, 20480, 1024), (12, 24576, 1024), (16, 28672, 4096), (7, 28672, 1024),
 ])
@@ -66,6 +65,35 @@ def test_paired_wave_kernel_bit_exact(mi, dev, orc, M, N, K):
     mi.check(mi.lib.mi_w8a8_gemm_dequant_f32(dev.upload(qx).ptr, dev.upload(sx).ptr, dev.upload(qw).ptr,
                                              dev.upload(sw).ptr, dy.ptr, M, N, K, None))
     dev.sync()
+    y = dev.download(dy)
+    dev.reset_to(mark)
+    assert np.array_equal(y, orc.dequant(want, sx, sw))
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    # the LDS-tiled kernel on a chip of 256 units, each of its tiles with rows, columns or both ragged, K of 1 to 8 stages
+    # (its prologue and last stages branch up to 5), one tile of a single row or of 16 columns at the edge
+    (130, 16400, 128, (128, 256)), (132, 16416, 256, (128, 256)), (131, 16640, 384, (128, 256)), (129, 16464, 512, (128, 256)),
+    (130, 16432, 640, (128, 256)), (128, 24656, 128, (128, 256)), (129, 16544, 768, (128, 256)),
+    (259, 21920, 128, (256, 192)), (512, 17056, 128, (256, 192)), (263, 21840, 256, (256, 192)), (260, 22464, 384, (256, 192)),
+    (261, 22064, 512, (256, 192)), (265, 21840, 640, (256, 192)), (257, 21856, 768, (256, 192)),
+    (257, 24672, 128, (256, 224)), (260, 24976, 256, (256, 224)), (264, 24864, 384, (256, 224)), (262, 24784, 512, (256, 224)),
+    (257, 24656, 640, (256, 224)), (1024, 25088, 1024, (256, 224)),
+    (259, 28832, 128, (256, 256)), (258, 28896, 256, (256, 256)), (257, 29488, 384, (256, 256)), (259, 28896, 512, (256, 256)),
+    (257, 28928, 640, (256, 256)), (257, 28752, 768, (256, 256)), (1792, 8496, 512, (256, 256)),
+])
+def test_lds_tiled_kernel_ragged_bit_exact(mi, dev, orc, M, N, K, tile):
+    """The shapes are chosen for the kernel that they reach: a change of the choice has to bring others."""
+    got = np.zeros(2, np.int32)
+    assert mi.lib.mi_w8a8_gemm_route_host(M, N, K, 256, got.ctypes.data) == 2 and tuple(got) == tile
+    qx, qw = rand_codes(M + N + K, (M, K)), rand_codes(K + 17, (N, K))
+    want = orc.gemm_i8_i32(qx, qw)
+    assert np.array_equal(gpu_gemm_i32(mi, dev, qx, qw), want)
+    g = np.random.default_rng(N)
+    sx, sw = g.uniform(0.01, 1, M).astype(np.float32), g.uniform(0.001, 0.1, N).astype(np.float32)
+    mark = dev.mark()
+    dy = dev.empty((M, N), np.float32)
+    mi.gemm_dequant(dev.upload(qx), dev.upload(sx), dev.upload(qw), dev.upload(sw), dy)
     y = dev.download(dy)
     dev.reset_to(mark)
     assert np.array_equal(y, orc.dequant(want, sx, sw))
@@ -121,8 +149,8 @@ def test_gemv_of_few_tokens_bit_exact(mi, dev, orc, M, N, K):
 
 
 def test_random_skinny_shapes_bit_exact(mi, dev, orc):
-    """Seeded random shapes over every skinny path (1 to 64 tokens, K of 1 to 39 stages, N any multiple of 16 or a
-    multiple of 2048, which takes the evenly dealt ring kernels): exact against the oracle."""
+    """Seeded random shapes of few tokens (1 to 64, K of 1 to 39 stages, N any multiple of 16 or a multiple of 2048): the GEMV
+    and the small tiles, exact against the oracle."""
     rng = np.random.default_rng(7)
     for _ in range(60):
         M, K = int(rng.integers(1, 65)), int(rng.integers(1, 40)) * 128
