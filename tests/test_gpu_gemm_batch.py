@@ -1,5 +1,5 @@
-"""GPU parity: several W8A8 contractions in one launch (mi_gemm_batch_*), the kernel whose workgroups walk a list of
-256 x 256 tiles.  Gates: int32 accumulators bit-exact against the oracle; the dequantized form equal to the
+"""GPU parity: several W8A8 contractions at once (mi_gemm_batch_*), in the kernel whose workgroups walk a list of
+256 x 256 tiles, in small tiles, or some in either.  Gates: int32 accumulators bit-exact against the oracle; the dequantized form equal to the
 oracle's fp32 operations; both equal, bit for bit, to the single-problem entry points."""
 import numpy as np
 import pytest
@@ -26,10 +26,10 @@ def make_ops(dev, shapes, seed, dtype):
 
 
 # K of 3 to 7 stages (short tiles: the stores of the tile before them are still in flight when they end) and of 24, 25
-# and 32; shapes that are no multiple of the tile exercise the tiles that are moved inwards (rows: 300 = 256 + 44,
-# columns: 272 = 256 + 16, 1168 = 4 * 256 + 144); several tiles per workgroup exercise the load
-# stream across tile boundaries, the scales that change registers' contents between tiles and the clearing of the
-# accumulators; mixed K in one batch exercises a cursor that changes its stride between tiles.
+# and 32.  The batches of fewer than about 200 tiles run in small tiles; in the others, which the list kernel walks, several
+# tiles per workgroup exercise the load stream across tile boundaries, the scales that change registers' contents between
+# tiles and the clearing of the accumulators, mixed K a cursor that changes its stride between tiles, and 264 rows or 1168
+# columns the tiles that are moved inwards (more of those in test_batch_by_route).
 @pytest.mark.parametrize("shapes", [
     [(256, 256, 384)],
     [(256, 256, 512)],
@@ -59,7 +59,7 @@ def test_batch_accumulators_bit_exact(mi, dev, orc, shapes):
 
 
 # batches whose list would be badly balanced: a long K in small tiles beside two round ones in a list (two launches), and
-# batches that the small tiles take whole, in one launch of 64 x 64, 128 x 64 and 128 x 128 tiles
+# batches that the small tiles take whole, in one launch of 128 x 64 or 128 x 128 tiles
 @pytest.mark.parametrize("shapes", [
     [(509, 14336, 2048), (509, 2048, 7168), (509, 14336, 2048), (509, 3072, 2048)],
     [(300, 2048, 896), (256, 1040, 2176)],
@@ -180,7 +180,9 @@ def test_batch_rejects_what_it_cannot_run(mi, dev):
 
 def test_random_batches_equal_the_single_problem_kernels(mi, dev):
     """Seeded random batches (1 to 4 problems, ragged M and N, 3 to 19 K stages, mixed K in one batch): every
-    dequantized output equals, bit for bit, what the single-problem entry point writes for the same operands."""
+    dequantized output equals, bit for bit, what the single-problem entry point writes for the same operands.  Batches as
+    small as these run in small tiles, as the single problems do; test_random_batches_by_route_equal_the_oracle has the
+    others, and the oracle."""
     rng = np.random.default_rng(20251125)
     for _ in range(12):
         shapes = [(int(rng.integers(256, 1200)), max(256, int(rng.integers(16, 90)) * 16), int(rng.integers(3, 20)) * 128)
@@ -204,3 +206,75 @@ def test_random_batches_equal_the_single_problem_kernels(mi, dev):
             assert np.array_equal(dev.download(o[4]), dev.download(r)), (shapes, s)
         batch.destroy()
         dev.reset_to(mark)
+
+
+def route(mi, shapes, cus=256):
+    """(which problems run in small tiles, the small tile)"""
+    import ctypes as C
+    mnk = (C.c_int64 * (3 * len(shapes)))(*[v for s in shapes for v in s])
+    small, tile = np.zeros(len(shapes), np.int32), np.zeros(2, np.int32)
+    assert mi.lib.mi_gemm_batch_split_host(mnk, len(shapes), cus, small.ctypes.data, tile.ctypes.data) >= 0
+    return small.tolist(), tuple(tile.tolist())
+
+
+def check_batch(mi, dev, orc, shapes, seed):
+    mark = dev.mark()
+    batch = mi.GemmBatch(dev, shapes)
+    ops, host = make_ops(dev, shapes, seed, np.float32)
+    acc = [dev.empty((M, N), np.int32) for M, N, K in shapes]
+    for b in acc + [o[4] for o in ops]:   # poison: every element must be written
+        mi.check(mi.lib.mi_fill_u32(b.ptr, 0x7F7F7F7F, b.nbytes // 4, None))
+    batch.run_i32([(qx, None, qw, None, a) for (qx, _, qw, _, _), a in zip(ops, acc)])
+    batch.run_f32(ops)
+    dev.sync()
+    for s, o, a, (qx, sx, qw, sw) in zip(shapes, ops, acc, host):
+        want = orc.gemm_i8_i32(qx, qw)
+        assert np.array_equal(dev.download(a), want), (shapes, s)
+        assert np.array_equal(dev.download(o[4]), orc.dequant(want, sx, sw)), (shapes, s)
+    batch.destroy()
+    dev.reset_to(mark)
+
+
+@pytest.mark.parametrize("shapes,small,tile", [
+    # the list kernel: ragged rows, columns and both (tiles moved inwards by up to 255), K of 3, 4, 5, 7 and 25 stages, mixed
+    # lengths in one list, a problem of two tiles beside one of hundreds
+    ([(1066, 7264, 384)], [0], (0, 0)),
+    ([(1430, 5536, 384)], [0], (0, 0)),
+    ([(1667, 4784, 3200)], [0], (0, 0)),
+    ([(533, 272, 896), (1029, 7616, 384)], [0, 0], (0, 0)),
+    ([(1824, 2736, 384), (555, 6096, 384)], [0, 0], (0, 0)),
+    ([(1124, 3792, 512), (537, 5984, 384), (1812, 608, 384)], [0, 0, 0], (0, 0)),
+    ([(735, 4512, 640), (1191, 2464, 512), (780, 3264, 384)], [0, 0, 0], (0, 0)),
+    # small tiles: each of the three, one problem and several
+    ([(291, 5536, 384)], [1], (64, 64)),
+    ([(1021, 688, 512), (667, 1888, 384)], [1, 1], (64, 64)),
+    ([(300, 6128, 512), (692, 4432, 384), (792, 320, 768)], [1, 1, 1], (64, 64)),
+    ([(262, 272, 384)], [1], (128, 64)),
+    ([(860, 320, 1792), (302, 432, 2176), (536, 1536, 1408)], [1, 1, 1], (128, 64)),
+    ([(276, 6688, 384)], [1], (128, 128)),
+    ([(260, 288, 1024), (339, 6272, 512), (763, 496, 1152)], [1, 1, 1], (128, 128)),
+    # some in either, each small tile
+    ([(418, 4576, 384), (1137, 5856, 768), (947, 5296, 512)], [1, 0, 0], (64, 64)),
+    ([(1048, 2368, 384), (564, 2752, 640), (1810, 1472, 384), (1663, 3584, 512)], [0, 1, 0, 0], (128, 64)),
+    ([(875, 4272, 512), (1322, 7088, 384)], [1, 0], (128, 128)),
+])
+def test_batch_by_route(mi, dev, orc, shapes, small, tile):
+    """Ragged batches, each chosen for the launches that it takes on 256 units: a change of the rule has to bring others."""
+    assert route(mi, shapes) == (small, tile)
+    check_batch(mi, dev, orc, shapes, 501 + shapes[0][0])
+
+
+def test_random_batches_by_route_equal_the_oracle(mi, dev, orc):
+    """Seeded random ragged batches until there are three of each kind: all in the list, all in small tiles, some in either."""
+    rng = np.random.default_rng(20251203)
+    seen = {"list": 0, "small": 0, "both": 0}
+    while min(seen.values()) < 3:
+        shapes = [(int(rng.integers(256, 2200)), int(rng.integers(17, 500)) * 16, int(rng.integers(3, 16)) * 128)
+                  for _ in range(int(rng.integers(1, 6)))]
+        if sum(M * N * K for M, N, K in shapes) > 1.2e10:
+            continue
+        small, _ = route(mi, shapes)
+        kind = "small" if all(small) else "both" if any(small) else "list"
+        if seen[kind] < 3:
+            seen[kind] += 1
+            check_batch(mi, dev, orc, shapes, 700 + sum(seen.values()))
