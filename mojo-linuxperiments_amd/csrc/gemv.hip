@@ -117,7 +117,7 @@ __global__ __launch_bounds__(64 * WG) void k_gemv_reg(const int8_t *__restrict__
 
 // k_gemv_fused: k_gemv_reg with the rotate + quantize prologue inside.  The row's own loads go out first and the
 // first group's weight loads right behind them; while the weights are in flight the workgroup rotates and quantizes
-// the M activation rows (the same per-chunk code as the stand-alone quantizer, so the codes and scales are
+// the activation row (the same per-chunk code as the stand-alone quantizer, so the codes and scales are
 // bit-identical), parks the codes in LDS and every lane picks up its share.  One launch per linear instead of two.
 // ROT = false: the row arrives in the rotated basis and is only quantized.
 // NORM: the row is first normalized, v = ((x (+ res)) * r) * g with r = 1 / sqrt(mean((x + res)^2) + eps), the
@@ -129,32 +129,29 @@ struct FusedNorm {
     float eps;
 };
 
-template <int MB, int CW, int CQ, bool NORM, bool ROT>
+template <int CW, int CQ, bool NORM, bool ROT>
 __global__ __launch_bounds__(256) void k_gemv_fused(const float *__restrict__ x, const int8_t *__restrict__ qw,
                                                     const float *__restrict__ sw, float *__restrict__ y,
-                                                    int8_t *__restrict__ qx_out, float *__restrict__ sx_out, int M,
-                                                    int N, int K, int QW, FusedNorm nm)
+                                                    int8_t *__restrict__ qx_out, float *__restrict__ sx_out, int N,
+                                                    int K, FusedNorm nm)
 {
     constexpr int BLOCK = 128, LPB = BLOCK / 8;
     constexpr int R = (16 / CW) < 1 ? 1 : (16 / CW);   // rows per wave
-    constexpr int V = pow2_ceil(R * MB);
+    constexpr int V = pow2_ceil(R);
     extern __shared__ __attribute__((aligned(16))) char s_dyn[];
-    int8_t *s_x = reinterpret_cast<int8_t *>(s_dyn);                       // [MB][K] codes
-    float *s_scale = reinterpret_cast<float *>(s_dyn + (size_t)MB * K);    // [MB]
-    float *s_max = s_scale + MB;                                           // [4] row maxima, then [4 * CQ] sums of squares
-    int *s_red = reinterpret_cast<int *>(s_max + 4 + 4 * CQ);              // [4][V]
+    int8_t *s_x = reinterpret_cast<int8_t *>(s_dyn);            // [K] codes
+    float *s_max = reinterpret_cast<float *>(s_dyn + K);        // [4] row maxima, then [4 * CQ] sums of squares
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int q = wave % QW;                  // which CW-chunk slice of the row
-    const int rows_per_wg = (4 / QW) * R;
+    constexpr int rows_per_wg = 4 * R;
     // the workgroup owns a run of consecutive groups of rows_per_wg weight rows (the groups dealt out evenly over
     // the grid): one prologue serves them all
     const int ngroups = (N + rows_per_wg - 1) / rows_per_wg;
     const int g0 = (int)((int64_t)ngroups * blockIdx.x / gridDim.x);
     const int g1 = (int)((int64_t)ngroups * (blockIdx.x + 1) / gridDim.x);
-    const int kbase = q * CW * 1024 + lane * 16;
+    const int kbase = lane * 16;
 
     auto load_w = [&](v4i (&w)[R][CW], int g) {
-        const int row0 = g * rows_per_wg + (wave / QW) * R;
+        const int row0 = g * rows_per_wg + wave * R;
 #pragma unroll
         for (int r = 0; r < R; ++r)
 #pragma unroll
@@ -170,131 +167,119 @@ __global__ __launch_bounds__(256) void k_gemv_fused(const float *__restrict__ x,
     // flight while the prologue computes).
     v4i w[R][CW];
 
-    // rotate + quantize, one row at a time: thread t owns chunks t, t + 256, ... of the row
+    // rotate + quantize: thread t owns chunks t, t + 256, ... of the row
     const int j = tid % LPB;
     const int nchunk = K / 8;
-    for (int m = 0; m < MB && m < M; ++m) {
-        const float *xr = x + (int64_t)m * K;
-        float v[CQ][8];
-        int base[CQ];
+    float v[CQ][8];
+    int base[CQ];
 #pragma unroll
-        for (int i = 0; i < CQ; ++i) {
-            const int c = tid + i * 256;
-            base[i] = (c / LPB) * BLOCK + 4 * j;
-            if (c < nchunk) {
-                const float4 lo = *reinterpret_cast<const float4 *>(xr + base[i]);
-                const float4 hi = *reinterpret_cast<const float4 *>(xr + base[i] + BLOCK / 2);
-                v[i][0] = lo.x; v[i][1] = lo.y; v[i][2] = lo.z; v[i][3] = lo.w;
-                v[i][4] = hi.x; v[i][5] = hi.y; v[i][6] = hi.z; v[i][7] = hi.w;
-            } else {
+    for (int i = 0; i < CQ; ++i) {
+        const int c = tid + i * 256;
+        base[i] = (c / LPB) * BLOCK + 4 * j;
+        if (c < nchunk) {
+            const float4 lo = *reinterpret_cast<const float4 *>(x + base[i]);
+            const float4 hi = *reinterpret_cast<const float4 *>(x + base[i] + BLOCK / 2);
+            v[i][0] = lo.x; v[i][1] = lo.y; v[i][2] = lo.z; v[i][3] = lo.w;
+            v[i][4] = hi.x; v[i][5] = hi.y; v[i][6] = hi.z; v[i][7] = hi.w;
+        } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[i][e] = 0.0f;
-            }
+            for (int e = 0; e < 8; ++e) v[i][e] = 0.0f;
         }
-        const bool keeper = blockIdx.x == 0;   // one workgroup also leaves the codes and scales in the caller's workspace
-        if constexpr (!NORM) {
-            if (m == 0) load_w(w, g0);
-        }
-        if constexpr (NORM) {
-            float4 gl[CQ], gh[CQ], rl_[CQ], rh_[CQ];
-            float ss[CQ];   // per chunk, then per group of 64 chunks (group wave + 4 * i): the order of fwht_core.h
-#pragma unroll
-            for (int i = 0; i < CQ; ++i) {
-                if (tid + i * 256 < nchunk) {
-                    gl[i] = *reinterpret_cast<const float4 *>(nm.g + base[i]);
-                    gh[i] = *reinterpret_cast<const float4 *>(nm.g + base[i] + BLOCK / 2);
-                    if (nm.res) {
-                        const float *rr = nm.res + (int64_t)m * K + base[i];
-                        rl_[i] = *reinterpret_cast<const float4 *>(rr);
-                        rh_[i] = *reinterpret_cast<const float4 *>(rr + BLOCK / 2);
-                    }
-                }
-            }
-            if (m == 0) load_w(w, g0);
-#pragma unroll
-            for (int i = 0; i < CQ; ++i) {
-                ss[i] = 0.0f;
-                if (tid + i * 256 < nchunk) {
-                    if (nm.res) {
-                        const float4 rl = rl_[i], rh = rh_[i];
-                        v[i][0] = v[i][0] + rl.x; v[i][1] = v[i][1] + rl.y; v[i][2] = v[i][2] + rl.z; v[i][3] = v[i][3] + rl.w;
-                        v[i][4] = v[i][4] + rh.x; v[i][5] = v[i][5] + rh.y; v[i][6] = v[i][6] + rh.z; v[i][7] = v[i][7] + rh.w;
-                        if (keeper) {
-                            float *ho = nm.h_out + (int64_t)m * K + base[i];
-                            *reinterpret_cast<float4 *>(ho) = make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
-                            *reinterpret_cast<float4 *>(ho + BLOCK / 2) = make_float4(v[i][4], v[i][5], v[i][6], v[i][7]);
-                        }
-                    }
-                    ss[i] = chunk_sumsq(v[i]);
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < CQ; ++i) ss[i] = group_sum(ss[i]);
-            __syncthreads();   // the previous row's sums have been read
-            if (lane == 0) {
-#pragma unroll
-                for (int i = 0; i < CQ; ++i) s_max[4 + wave + 4 * i] = ss[i];
-            }
-            __syncthreads();
-            const float total = tree_sum<4 * CQ>(s_max + 4);
-            const float r = 1.0f / sqrtf(total / (float)K + nm.eps);
-#pragma unroll
-            for (int i = 0; i < CQ; ++i) {
-                if (tid + i * 256 < nchunk) {
-                    v[i][0] = (v[i][0] * r) * gl[i].x; v[i][1] = (v[i][1] * r) * gl[i].y;
-                    v[i][2] = (v[i][2] * r) * gl[i].z; v[i][3] = (v[i][3] * r) * gl[i].w;
-                    v[i][4] = (v[i][4] * r) * gh[i].x; v[i][5] = (v[i][5] * r) * gh[i].y;
-                    v[i][6] = (v[i][6] * r) * gh[i].z; v[i][7] = (v[i][7] * r) * gh[i].w;
-                    if (keeper && nm.xn_out) {
-                        float *xo = nm.xn_out + (int64_t)m * K + base[i];
-                        *reinterpret_cast<float4 *>(xo) = make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
-                        *reinterpret_cast<float4 *>(xo + BLOCK / 2) = make_float4(v[i][4], v[i][5], v[i][6], v[i][7]);
-                    }
-                }
-            }
-        }
-        float amax = 0.0f;
-#pragma unroll
-        for (int i = 0; i < CQ; ++i) {
-            if constexpr (ROT) fwht_chunk<BLOCK>(v[i], j);   // !ROT: the row arrives in the rotated basis
-            amax = fmaxf(amax, abs8(v[i]));
-        }
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-        __syncthreads();   // the previous row's maxima have been read
-        if (lane == 0) s_max[wave] = amax;
-        __syncthreads();
-        const float a = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
-        const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
-        const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
-        if (tid == 0) s_scale[m] = sc;
-        int8_t *qrow = s_x + (size_t)m * K;
-        if (keeper && tid == 0) sx_out[m] = sc;
+    }
+    const bool keeper = blockIdx.x == 0;   // one workgroup also leaves the codes and scales in the caller's workspace
+    if constexpr (!NORM) load_w(w, g0);
+    if constexpr (NORM) {
+        float4 gl[CQ], gh[CQ], rl_[CQ], rh_[CQ];
+        float ss[CQ];   // per chunk, then per group of 64 chunks (group wave + 4 * i): the order of fwht_core.h
 #pragma unroll
         for (int i = 0; i < CQ; ++i) {
             if (tid + i * 256 < nchunk) {
-                const uint32_t c0 = quant4(v[i][0], v[i][1], v[i][2], v[i][3], inv);
-                const uint32_t c1 = quant4(v[i][4], v[i][5], v[i][6], v[i][7], inv);
-                *reinterpret_cast<uint32_t *>(qrow + base[i]) = c0;
-                *reinterpret_cast<uint32_t *>(qrow + base[i] + BLOCK / 2) = c1;
-                if (keeper) {
-                    *reinterpret_cast<uint32_t *>(qx_out + (int64_t)m * K + base[i]) = c0;
-                    *reinterpret_cast<uint32_t *>(qx_out + (int64_t)m * K + base[i] + BLOCK / 2) = c1;
+                gl[i] = *reinterpret_cast<const float4 *>(nm.g + base[i]);
+                gh[i] = *reinterpret_cast<const float4 *>(nm.g + base[i] + BLOCK / 2);
+                if (nm.res) {
+                    const float *rr = nm.res + base[i];
+                    rl_[i] = *reinterpret_cast<const float4 *>(rr);
+                    rh_[i] = *reinterpret_cast<const float4 *>(rr + BLOCK / 2);
                 }
+            }
+        }
+        load_w(w, g0);
+#pragma unroll
+        for (int i = 0; i < CQ; ++i) {
+            ss[i] = 0.0f;
+            if (tid + i * 256 < nchunk) {
+                if (nm.res) {
+                    const float4 rl = rl_[i], rh = rh_[i];
+                    v[i][0] = v[i][0] + rl.x; v[i][1] = v[i][1] + rl.y; v[i][2] = v[i][2] + rl.z; v[i][3] = v[i][3] + rl.w;
+                    v[i][4] = v[i][4] + rh.x; v[i][5] = v[i][5] + rh.y; v[i][6] = v[i][6] + rh.z; v[i][7] = v[i][7] + rh.w;
+                    if (keeper) {
+                        float *ho = nm.h_out + base[i];
+                        *reinterpret_cast<float4 *>(ho) = make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
+                        *reinterpret_cast<float4 *>(ho + BLOCK / 2) = make_float4(v[i][4], v[i][5], v[i][6], v[i][7]);
+                    }
+                }
+                ss[i] = chunk_sumsq(v[i]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < CQ; ++i) ss[i] = group_sum(ss[i]);
+        if (lane == 0) {
+#pragma unroll
+            for (int i = 0; i < CQ; ++i) s_max[4 + wave + 4 * i] = ss[i];
+        }
+        __syncthreads();
+        const float total = tree_sum<4 * CQ>(s_max + 4);
+        const float r = 1.0f / sqrtf(total / (float)K + nm.eps);
+#pragma unroll
+        for (int i = 0; i < CQ; ++i) {
+            if (tid + i * 256 < nchunk) {
+                v[i][0] = (v[i][0] * r) * gl[i].x; v[i][1] = (v[i][1] * r) * gl[i].y;
+                v[i][2] = (v[i][2] * r) * gl[i].z; v[i][3] = (v[i][3] * r) * gl[i].w;
+                v[i][4] = (v[i][4] * r) * gh[i].x; v[i][5] = (v[i][5] * r) * gh[i].y;
+                v[i][6] = (v[i][6] * r) * gh[i].z; v[i][7] = (v[i][7] * r) * gh[i].w;
+                if (keeper && nm.xn_out) {
+                    float *xo = nm.xn_out + base[i];
+                    *reinterpret_cast<float4 *>(xo) = make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
+                    *reinterpret_cast<float4 *>(xo + BLOCK / 2) = make_float4(v[i][4], v[i][5], v[i][6], v[i][7]);
+                }
+            }
+        }
+    }
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < CQ; ++i) {
+        if constexpr (ROT) fwht_chunk<BLOCK>(v[i], j);   // !ROT: the row arrives in the rotated basis
+        amax = fmaxf(amax, abs8(v[i]));
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+    if (lane == 0) s_max[wave] = amax;
+    __syncthreads();
+    const float a = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
+    const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
+    const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
+    if (keeper && tid == 0) *sx_out = sc;
+#pragma unroll
+    for (int i = 0; i < CQ; ++i) {
+        if (tid + i * 256 < nchunk) {
+            const uint32_t c0 = quant4(v[i][0], v[i][1], v[i][2], v[i][3], inv);
+            const uint32_t c1 = quant4(v[i][4], v[i][5], v[i][6], v[i][7], inv);
+            *reinterpret_cast<uint32_t *>(s_x + base[i]) = c0;
+            *reinterpret_cast<uint32_t *>(s_x + base[i] + BLOCK / 2) = c1;
+            if (keeper) {
+                *reinterpret_cast<uint32_t *>(qx_out + base[i]) = c0;
+                *reinterpret_cast<uint32_t *>(qx_out + base[i] + BLOCK / 2) = c1;
             }
         }
     }
     __syncthreads();
 
-    v4i xr[MB][CW];
+    v4i xr[CW];
 #pragma unroll
-    for (int m = 0; m < MB; ++m)
-#pragma unroll
-        for (int c = 0; c < CW; ++c) {
-            const int off = kbase + c * 1024;
-            const int ms = m < M ? m : M - 1;
-            xr[m][c] = off < K ? *reinterpret_cast<const v4i *>(s_x + (size_t)ms * K + off) : (v4i){0, 0, 0, 0};
-        }
+    for (int c = 0; c < CW; ++c) {
+        const int off = kbase + c * 1024;
+        xr[c] = off < K ? *reinterpret_cast<const v4i *>(s_x + off) : (v4i){0, 0, 0, 0};
+    }
     constexpr int SH = 6 - __builtin_ctz(V);
     const int vi = lane >> SH;
     const bool speaker = (lane & ((1 << SH) - 1)) == 0;
@@ -308,33 +293,20 @@ __global__ __launch_bounds__(256) void k_gemv_fused(const float *__restrict__ x,
 #pragma unroll
         for (int i = 0; i < V; ++i) p[i] = 0;
 #pragma unroll
-        for (int r = 0; r < R; ++r)
+        for (int r = 0; r < R; ++r) {
+            int a = 0;
 #pragma unroll
-            for (int m = 0; m < MB; ++m) {
-                int a = 0;
-#pragma unroll
-                for (int c = 0; c < CW; ++c) {
-                    a = __builtin_amdgcn_sdot4(w[r][c][0], xr[m][c][0], a, false);
-                    a = __builtin_amdgcn_sdot4(w[r][c][1], xr[m][c][1], a, false);
-                    a = __builtin_amdgcn_sdot4(w[r][c][2], xr[m][c][2], a, false);
-                    a = __builtin_amdgcn_sdot4(w[r][c][3], xr[m][c][3], a, false);
-                }
-                p[r * MB + m] = a;
+            for (int c = 0; c < CW; ++c) {
+                a = __builtin_amdgcn_sdot4(w[r][c][0], xr[c][0], a, false);
+                a = __builtin_amdgcn_sdot4(w[r][c][1], xr[c][1], a, false);
+                a = __builtin_amdgcn_sdot4(w[r][c][2], xr[c][2], a, false);
+                a = __builtin_amdgcn_sdot4(w[r][c][3], xr[c][3], a, false);
             }
+            p[r] = a;
+        }
         fold_sum<V, 32>(p, lane);
-        int total = p[0];
-        if (QW > 1) {
-            if (speaker) s_red[wave * V + vi] = total;
-            __syncthreads();
-            if (q == 0 && speaker) {
-                for (int o = 1; o < QW; ++o) total += s_red[(wave + o) * V + vi];
-            }
-            __syncthreads();   // s_red is free for the next group
-        }
-        if (q == 0 && speaker && vi < R * MB) {
-            const int r = vi / MB, m = vi % MB, n = g * rows_per_wg + (wave / QW) * R + r;
-            if (n < N && m < M) y[(int64_t)m * N + n] = ((float)total * s_scale[m]) * sw[n];
-        }
+        const int n = g * rows_per_wg + wave * R + vi;
+        if (speaker && vi < R && n < N) y[n] = ((float)p[0] * sc) * sw[n];
         if (more) {
 #pragma unroll
             for (int r = 0; r < R; ++r)
@@ -344,22 +316,19 @@ __global__ __launch_bounds__(256) void k_gemv_fused(const float *__restrict__ x,
     }
 }
 
-template <int MB, int CW, int CQ, bool NORM, bool ROT = true>
-static int32_t launch_fused(const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx, int M,
-                            int N, int K, int QW, const FusedNorm &nm, hipStream_t s)
+template <int CW, int CQ, bool NORM, bool ROT = true>
+static int32_t launch_fused(const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx, int N, int K,
+                            const FusedNorm &nm, hipStream_t s)
 {
     constexpr int R = (16 / CW) < 1 ? 1 : (16 / CW);
-    constexpr int V = pow2_ceil(R * MB);
-    const size_t lds = (size_t)MB * K + (MB + 4 + 4 * CQ) * sizeof(float) + 4 * V * sizeof(int);
-    MI_LDS_OPT_IN((&k_gemv_fused<MB, CW, CQ, NORM, ROT>), 96 * 1024);
+    const size_t lds = (size_t)K + (4 + 4 * CQ) * sizeof(float);   // at most 4,144 bytes
     // Every workgroup reads the whole activation row (with the norm: the residual and the gain too, 48 KB at
     // K = 4096) before its first dot product.  Beyond two workgroups per compute unit a workgroup therefore takes
     // several groups of rows in turn, the next group's weights on their way while it works on the current one.
-    const int rows_per_wg = (4 / QW) * R;
+    constexpr int rows_per_wg = 4 * R;
     const int ngroups = (N + rows_per_wg - 1) / rows_per_wg;
     const unsigned grid = (unsigned)std::min(ngroups, 2 * compute_units());   // three per unit measured the same
-    hipLaunchKernelGGL((k_gemv_fused<MB, CW, CQ, NORM, ROT>), dim3(grid), dim3(256), lds, s, x, qw, sw, y, qx, sx, M, N,
-                       K, QW, nm);
+    hipLaunchKernelGGL((k_gemv_fused<CW, CQ, NORM, ROT>), dim3(grid), dim3(256), lds, s, x, qw, sw, y, qx, sx, N, K, nm);
     return launch_status();
 }
 
@@ -371,16 +340,16 @@ static int32_t launch_fused(const float *x, const int8_t *qw, const float *sw, f
 int32_t launch_linear_fused(const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx,
                             int64_t M64, int64_t N64, int64_t K64, hipStream_t s, bool rotate)
 {
-    const int M = (int)M64, N = (int)N64, K = (int)K64;
-    if (M != 1 || K % 1024) return MI_EINVAL;
+    const int N = (int)N64, K = (int)K64;
+    if (M64 != 1 || K % 1024) return MI_EINVAL;
     const int nchunk = K >> 10;
     const FusedNorm none = {nullptr, nullptr, nullptr, nullptr, 0.0f};
     if (rotate) {
-        if (nchunk == 4) return launch_fused<1, 4, 2, false>(x, qw, sw, y, qx, sx, M, N, K, 1, none, s);   // K = 4096
-        if (nchunk == 2) return launch_fused<1, 2, 1, false>(x, qw, sw, y, qx, sx, M, N, K, 1, none, s);   // K = 2048
+        if (nchunk == 4) return launch_fused<4, 2, false>(x, qw, sw, y, qx, sx, N, K, none, s);   // K = 4096
+        if (nchunk == 2) return launch_fused<2, 1, false>(x, qw, sw, y, qx, sx, N, K, none, s);   // K = 2048
     } else {
-        if (nchunk == 4) return launch_fused<1, 4, 2, false, false>(x, qw, sw, y, qx, sx, M, N, K, 1, none, s);
-        if (nchunk == 2) return launch_fused<1, 2, 1, false, false>(x, qw, sw, y, qx, sx, M, N, K, 1, none, s);
+        if (nchunk == 4) return launch_fused<4, 2, false, false>(x, qw, sw, y, qx, sx, N, K, none, s);
+        if (nchunk == 2) return launch_fused<2, 1, false, false>(x, qw, sw, y, qx, sx, N, K, none, s);
     }
     return MI_EINVAL;
 }
@@ -390,12 +359,12 @@ int32_t launch_norm_linear_fused(const float *x, const float *res, const float *
                                  float *xn_out, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx,
                                  int64_t M64, int64_t N64, int64_t K64, hipStream_t s)
 {
-    const int M = (int)M64, N = (int)N64, K = (int)K64;
-    if (M != 1 || K % 1024) return MI_EINVAL;
+    const int N = (int)N64, K = (int)K64;
+    if (M64 != 1 || K % 1024) return MI_EINVAL;
     const int nchunk = K >> 10;
     const FusedNorm nm = {res, g, h_out, xn_out, eps};
-    if (nchunk == 4) return launch_fused<1, 4, 2, true>(x, qw, sw, y, qx, sx, M, N, K, 1, nm, s);
-    if (nchunk == 2) return launch_fused<1, 2, 1, true>(x, qw, sw, y, qx, sx, M, N, K, 1, nm, s);
+    if (nchunk == 4) return launch_fused<4, 2, true>(x, qw, sw, y, qx, sx, N, K, nm, s);
+    if (nchunk == 2) return launch_fused<2, 1, true>(x, qw, sw, y, qx, sx, N, K, nm, s);
     return MI_EINVAL;
 }
 
