@@ -177,8 +177,8 @@ MI_API int32_t mi_fwht_f32(const float *x, float *out, int64_t M, int64_t K,
 
 /* ---- a4 / a5: W8A8 contraction, acc[m,n] = sum_k qx[m,k] * qw[n,k]
  * qx int8 [M,K], qw int8 [N,K] (both K-contiguous), acc int32 [M,N].
- * One token streams the weights through a GEMV; more rows run on v_mfma_i32_16x16x64_i8 in tiles of 16 x 16 to
- * 256 x 256 by a cost estimate of the shape.
+ * One token, and two to four with few rows of a long K, stream the weights through a GEMV; more run on
+ * v_mfma_i32_16x16x64_i8 in tiles of 16 x 16 to 256 x 256 by a cost estimate of the shape.
  * K % 128 == 0, N % 16 == 0.  Exact integer arithmetic. */
 MI_API int32_t mi_w8a8_gemm_i32(const int8_t *qx, const int8_t *qw, int32_t *acc,
                                 int64_t M, int64_t N, int64_t K, void *stream);

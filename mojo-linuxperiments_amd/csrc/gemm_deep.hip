@@ -1,10 +1,10 @@
-// W8A8 contraction for everything between one token and the sizes that fill the chip with 256-wide tiles:
+// W8A8 contraction for everything between the GEMV's few tokens and the sizes that fill the chip with 256-wide tiles:
 //   acc[m,n] = sum_k qx[m,k] * qw[n,k],   y = ((float)acc * sx[m]) * sw[n]
 //
 // One workgroup of four or eight waves per tile, the tile chosen from ten (16 x 16 to 128 x 128) so that every compute
 // unit has one, and one load stream per workgroup: stages of 128 to 512 bytes of K go straight to LDS through a ring of D
-// buffers, D - 1 stages in flight, one barrier a stage.  All but the largest tiles take at most half of a unit's LDS:
-// where there are tiles enough two workgroups share a unit and hide each other's first loads and last stores (16 rows,
+// buffers, D - 1 stages in flight, one barrier a stage.  All tiles but 128 x 128, 128 x 64 and 32 x 48 take at most half
+// of a unit's LDS: where there are tiles enough two workgroups share a unit and hide each other's first loads and last stores (16 rows,
 // 4096 -> 28672 inside a decode step: 24.3 instead of 27.2 us).  The barrier of stage s says that stage s + 1 has landed and
 // that everybody holds its fragments of stage s in registers; behind it a wave requests the fragments of stage s + 1,
 // the loads of stage s + D into the buffer just freed, and multiplies stage s.  Small tiles leave most
@@ -17,9 +17,9 @@
 // those 900.  Measured and equal or slower: loads through registers and ds_write, 16 waves, the loads spread between the
 // matrix instructions, another K phase per workgroup, rows of 256 bytes.  So the tile decides: rows loaded per result.
 //
-// Measured (us a call, and with the LDS-tiled and ring kernels before): 16 x 4096 -> 14336 12.0 (14.3), 32 x 4096 -> 4096
-// 5.2 (7.2), 64 x 4096 -> 14336 15.1 (27.2), 200 x 4096 -> 14336 24.3 (34.3), 256 x 14336 -> 4096 34.5 (97),
-// 512 x 4096 -> 4096 14.3 (28.3).
+// Measured (us a call in a graph of them, weights from HBM, and with the LDS-tiled and ring kernels before):
+// 16 x 4096 -> 14336 12.0 (13.7), 32 x 4096 -> 4096 7.2 (9.0), 64 x 4096 -> 14336 15.1 (25.4), 200 x 4096 -> 14336
+// 24.2 (34.5), 256 x 14336 -> 4096 31.9 (91.3), 512 x 4096 -> 4096 17.7 (32.4).
 //
 // LDS layout, swizzle and shape of the loads are those of gemm_tiled.hip: 1 KB blocks of 8 rows x 128 bytes, chunk position
 // XORed with sigma(row, block parity), free of bank conflicts for the fragment reads.  Operand A is the weights.
@@ -411,11 +411,28 @@ static float with_memory(float core, double bytes)
 
 }  // namespace deep
 
-// Microseconds that launch_deep would take (see above); *which is the tile to pass on.
+// Microseconds that launch_deep would take, to be compared with the LDS-tiled kernel's; *which is the tile to pass on.  The fit
+// above tells tiles apart but not kernels: it is 6 % low on average and 17 % beyond six rounds.  For the tiles that meet the
+// other kernel: a constant, a time per round and per K step of a round, which grows with the share of the chip that has a
+// tile, and the output; least squares over 2043 of 2600 drawn shapes (M of 65 to 4096, N of 256 to 28672, K of 128 to 14336,
+// weights from HBM; standard deviation 6 to 8 %).  Raised by 4 %: near a tie the LDS-tiled kernel is taken, whose own
+// estimate is the better one.
 float deep_estimate(int M, int N, int K, int cus, int *which)
 {
-    const float core = deep::pick(M, N, K, cus, which);
-    return deep::with_memory(core, (double)N * K + (double)M * K + 4.0 * M * N);
+    using namespace deep;
+    constexpr float c0[3] = {3.52f, 2.90f, 3.20f}, per_round[3] = {3.09f, 1.25f, 0.31f}, per_step[3] = {0.317f, 0.262f, 0.185f},
+                    with_fill[3] = {0.845f, 0.134f, 0.153f}, per_out_mb[3] = {0.067f, 0.242f, 0.200f};
+    const float core = pick(M, N, K, cus, which);
+    const int w = *which;
+    if (w > 2) return 1.06f * with_memory(core, (double)N * K + (double)M * K + 4.0 * M * N);
+    const Tile &t = TILES[w];
+    const uint64_t tiles = (uint64_t)(((unsigned)M + t.bm - 1) / t.bm) * (((unsigned)N + t.bn - 1) / t.bn);
+    const uint64_t slots = (uint64_t)(cus * t.per_cu), full = tiles / slots, rem = tiles - full * slots;
+    const float two = 1.0f + BESIDE;   // rounds of one tile a unit
+    const float rounds = (float)full * (t.per_cu == 2 ? two : 1.0f) + (rem > (uint64_t)cus ? two : rem ? 1.0f : 0.0f);
+    const float fill = (float)tiles / (float)(slots * (full + (rem != 0)));
+    const float step = per_step[w] * (1.0f + with_fill[w] * fill * fill);
+    return 1.04f * (c0[w] + rounds * (per_round[w] + step * (float)(K >> 7)) + per_out_mb[w] * 4e-6f * (float)M * (float)N);
 }
 
 void deep_tile(int which, int32_t *rows, int32_t *cols)
@@ -459,7 +476,8 @@ template int32_t launch_deep<false>(int, const int8_t *, const float *, const in
 
 // ---- several contractions of at least 256 rows in one launch (a part of a batch, see gemm_list.hip)
 // Times as above; the tiles go to the units as these come free, longest K first.  A launch of several rounds takes 1.25
-// times the sum of its tiles (measured 147 us where the sum says 115 and 83 where it says 66).
+// times the sum of its tiles (measured 147 us where the sum says 115 and 83 where it says 66; what the choice that rests on
+// it gives over 124 drawn batches stands in gemm_list.hip).
 float deep_batch_estimate(const int64_t *mnk, const int *idx, int n, int cus, int *which)
 {
     using namespace deep;

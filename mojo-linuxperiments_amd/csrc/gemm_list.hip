@@ -620,9 +620,10 @@ using LC = Cfg;
 // of those and its start (166 us where the mean workgroup is busy for 80).  The small tiles move twice the bytes per result,
 // but hundreds of them level out.  Estimates: a list's longest sum of tile costs at 1.36 us a unit (measured from 2048
 // rows through the four projections, 252 units in 340 us, down to one tile a workgroup) and deep_batch_estimate.
-// Measured, weights from HBM, us before -> after: the four projections with 256 rows 150 -> 82, with 384 rows 159 -> 121,
-// with 509 rows 159 -> 134 (gate and up tiled, qkv and down in small tiles); 2048 -> 3072, 2048, 11008 and
-// 11008 -> 2048 with 512 rows 102 -> 45.
+// Measured, weights from HBM, us before -> after: the four projections with 256 rows 150 -> 84, with 384 rows 157 -> 122,
+// with 509 rows 160 -> 131 (gate and up tiled, qkv and down in small tiles); 2048 -> 3072, 2048, 11008 and
+// 11008 -> 2048 with 512 rows 109 -> 59.  Of 124 drawn batches (256 to 2048 rows, one to five problems) 97 go over in whole or
+// in part and take 0.26 to 1.00 of the list's time, 0.55 in the mean.
 struct Split {
     int n_tiled = 0, n_deep = 0;
     int tiled[MAX_PROBLEMS], deep[MAX_PROBLEMS];
@@ -667,7 +668,9 @@ static Split split_batch(const int64_t *mnk, int n, int cus)
         sum += t * tile_cost(mnk[3 * p + 2]);
     }
     const Load whole = list_load(mnk, best.tiled, n, cus);
-    // nothing to level out (the small tiles cost 1.65 times as much), or so many tiles that a list is level
+    // nothing to level out (the small tiles cost 1.65 times as much), or so many tiles that a list is level.  Without these
+    // two limits and the 0.9 below 106 of 1200 drawn batches run otherwise, half of them faster and half slower: 0.81 to 1.16
+    // times as long, 0.99 in the mean, the same in sum.
     if ((double)whole.cost * cus < 1.2 * sum || tiles > 8.0 * cus) return best;
     // the estimates are good to a tenth: what they promise has to be more
     float t_best = 0.9f * (3.0f + 1.36f * (float)whole.cost);

@@ -437,20 +437,30 @@ static int pick_shape(int M, int N, int cus, int64_t *rounds_out)
     return pick;
 }
 
-// Microseconds that launch_tiled takes: a constant and a time per K step and round of each tile, least squares over 150
-// shapes (within 13 %; 28 % where 128 x 256 tiles cover a fraction of the chip, which no choice depends on).
-float tiled_estimate(int M, int N, int K, int cus)
-{
-    int64_t rounds = 1;
-    const int p = pick_shape(M, N, cus, &rounds);
-    constexpr float c0[4] = {2.0f, 6.0f, 1.0f, 6.0f}, c1[4] = {1.85f, 1.67f, 1.53f, 0.80f};
-    return c0[p] + c1[p] * (float)rounds * (float)(K >> 7);
-}
-
 // one tile per compute unit of a shape that divides evenly: two waves per SIMD on the same wave tile
 static bool paired(int pick, int M, int N)
 {
     return (pick == 2 || pick == 3) && M % (32 * SHAPES[pick].tm) == 0 && N % (32 * SHAPES[pick].tn) == 0;
+}
+
+// Microseconds that launch_tiled takes: a constant, a time per round and per K step of a round of each tile (the paired forms
+// of the last two behind them), which grows with the share of the chip that has a tile, and the output; least squares over the
+// shapes of deep_estimate (standard deviation 3 to 5 %).  The choice by the two estimates costs 0.15 % on average over the
+// faster kernel of each of the 2600 shapes, and 13 of them take more than 3 % longer than here (one 23 %).  With a constant and
+// a time per K step alone 71 had, the largest sizes most (2741 x 10240 -> 13008 319 -> 482 us, 764 x 9856 -> 16064 110 -> 156).
+float tiled_estimate(int M, int N, int K, int cus)
+{
+    int64_t rounds = 1;
+    int p = pick_shape(M, N, cus, &rounds);
+    const int bm = 32 * SHAPES[p].tm, bn = 32 * SHAPES[p].tn;
+    const float fill = (float)((int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn)) / (float)(rounds * cus);
+    if (paired(p, M, N)) p += 2;
+    constexpr float c0[6] = {4.42f, 3.80f, 4.36f, 2.82f, 4.25f, 4.21f}, per_round[6] = {21.4f, 8.03f, 6.71f, 4.62f, 7.82f, 3.23f},
+                    per_step[6] = {0.980f, 0.886f, 0.928f, 0.727f, 0.767f, 0.641f},
+                    with_fill[6] = {0.590f, 0.649f, 0.360f, 0.325f, 0.668f, 0.593f},
+                    per_out_mb[6] = {0.003f, 0.053f, 0.059f, 0.144f, 0.032f, 0.129f};
+    const float step = per_step[p] * (1.0f + with_fill[p] * fill * fill);
+    return c0[p] + (float)rounds * (per_round[p] + step * (float)(K >> 7)) + per_out_mb[p] * 4e-6f * (float)M * (float)N;
 }
 
 // the tile that launch_tiled takes, and whether gemm_pair.hip computes it

@@ -39,7 +39,7 @@ def test_skinny_accumulators_bit_exact(mi, dev, orc, M, N, K):
 @pytest.mark.parametrize("M,N,K", [
     (65, 256, 128), (128, 128, 256), (256, 256, 1024), (200, 192, 512), (257, 272, 384),
     (512, 448, 768), (300, 1000 // 16 * 16, 640), (2048, 224 * 3, 512), (1024, 6144, 256),
-    (4096, 4096, 256),                # the 256 x 256 tile
+    (4096, 4096, 256),
 ])
 def test_tiled_accumulators_bit_exact(mi, dev, orc, M, N, K):
     qx, qw = rand_codes(M + 3 * N, (M, K)), rand_codes(K + 5, (N, K))
@@ -71,16 +71,18 @@ def test_paired_wave_kernel_bit_exact(mi, dev, orc, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K,tile", [
-    # the LDS-tiled kernel on a chip of 256 units, each of its tiles with rows, columns or both ragged, K of 1 to 8 stages
-    # (its prologue and last stages branch up to 5), one tile of a single row or of 16 columns at the edge
-    (130, 16400, 128, (128, 256)), (132, 16416, 256, (128, 256)), (131, 16640, 384, (128, 256)), (129, 16464, 512, (128, 256)),
-    (130, 16432, 640, (128, 256)), (128, 24656, 128, (128, 256)), (129, 16544, 768, (128, 256)),
-    (259, 21920, 128, (256, 192)), (512, 17056, 128, (256, 192)), (263, 21840, 256, (256, 192)), (260, 22464, 384, (256, 192)),
-    (261, 22064, 512, (256, 192)), (265, 21840, 640, (256, 192)), (257, 21856, 768, (256, 192)),
-    (257, 24672, 128, (256, 224)), (260, 24976, 256, (256, 224)), (264, 24864, 384, (256, 224)), (262, 24784, 512, (256, 224)),
-    (257, 24656, 640, (256, 224)), (1024, 25088, 1024, (256, 224)),
-    (259, 28832, 128, (256, 256)), (258, 28896, 256, (256, 256)), (257, 29488, 384, (256, 256)), (259, 28896, 512, (256, 256)),
-    (257, 28928, 640, (256, 256)), (257, 28752, 768, (256, 256)), (1792, 8496, 512, (256, 256)),
+    # the LDS-tiled kernel on a chip of 256 units, each of its tiles with rows, columns or both ragged, as few stages of K as it is
+    # chosen for (its prologue and last stages branch up to 5)
+    (193, 24800, 128, (128, 256)), (3200, 1968, 128, (128, 256)), (386, 12256, 256, (128, 256)),
+    (193, 20784, 384, (128, 256)), (195, 20592, 512, (128, 256)), (194, 21248, 512, (128, 256)),
+    (142, 27616, 640, (128, 256)), (129, 27520, 768, (128, 256)), (449, 16528, 128, (256, 192)),
+    (3072, 2704, 128, (256, 192)), (324, 21984, 256, (256, 192)), (392, 16992, 384, (256, 192)),
+    (387, 16496, 512, (256, 192)), (285, 24000, 512, (256, 192)), (269, 23088, 640, (256, 192)),
+    (258, 23152, 768, (256, 192)), (321, 24768, 128, (256, 224)), (768, 16448, 128, (256, 224)),
+    (322, 24752, 256, (256, 224)), (289, 26368, 384, (256, 224)), (266, 26416, 512, (256, 224)),
+    (269, 26208, 512, (256, 224)), (258, 26400, 640, (256, 224)), (257, 26336, 768, (256, 224)),
+    (3070, 16320, 640, (256, 256)), (636, 19632, 896, (256, 256)), (1280, 12848, 768, (256, 256)),
+    (407, 31744, 896, (256, 256)),
 ])
 def test_lds_tiled_kernel_ragged_bit_exact(mi, dev, orc, M, N, K, tile):
     """The shapes are chosen for the kernel that they reach: a change of the choice has to bring others."""
