@@ -549,7 +549,7 @@ static inline int tile_cost(int64_t K) { return (int)(K / 128) + 10; }
 // measured 355 / 344 / 339 us (resident) and 366 / 364 / 369 us (from HBM).
 template <int BM, int BN>
 static int64_t build_lists(const int64_t *mnk, int n, int cus, std::vector<v4i> *lists, int *per_wg_out)
-{
+try {
     const int nx = (cus % 8 == 0) ? 8 : 1, slots = cus / nx;
     constexpr int ROWS = 4;
     std::vector<int> order((size_t)n);
@@ -610,6 +610,8 @@ static int64_t build_lists(const int64_t *mnk, int n, int cus, std::vector<v4i> 
             }
     }
     return (int64_t)cus * per_wg * (int64_t)sizeof(v4i);
+} catch (const std::bad_alloc &) {   // its callers are C entries
+    return MI_ENOMEM;
 }
 
 using LC = Cfg;
@@ -702,7 +704,7 @@ static Split split_batch(const int64_t *mnk, int n, int cus)
 // What a batch holds: its split and the list of split.tiled (entries count problems in that order).  Returns the list's
 // bytes, at most those of the list over all problems, which mi_gemm_batch_plan_bytes promises; 0: no problem is left for it.
 static int64_t plan_batch(const int64_t *mnk, int n, int cus, Split *split, std::vector<v4i> *lists, int *per_wg)
-{
+try {
     const int64_t whole = build_lists<LC::BM, LC::BN>(mnk, n, cus, lists, per_wg);
     if (whole < 0) return whole;
     *split = split_batch(mnk, n, cus);
@@ -715,6 +717,8 @@ static int64_t plan_batch(const int64_t *mnk, int n, int cus, Split *split, std:
     for (int i = 0; i < split->n_tiled; ++i)
         for (int k = 0; k < 3; ++k) sub[3 * i + k] = mnk[3 * split->tiled[i] + k];
     return build_lists<LC::BM, LC::BN>(sub, split->n_tiled, cus, lists, per_wg);
+} catch (const std::bad_alloc &) {
+    return MI_ENOMEM;
 }
 
 static int32_t check_shapes(const int64_t *mnk, int32_t n)

@@ -2,6 +2,8 @@
 is covered by a tile that lies inside its matrix, every address the kernel forms from a tile stays inside the
 operands and inside the kernel's LDS areas, and the list is balanced."""
 import ctypes as C
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -84,6 +86,25 @@ def test_stored_lists_fit_the_memory_that_the_caller_was_told_to_bring(mi):
         kinds.add("all" if all(small) else "some" if any(small) else "none")
     assert kinds == {"all", "some", "none"}
     assert split(mi, CFG3) == (plan(mi, CFG3).nbytes, [0] * 4, (0, 0))
+
+
+def test_planner_without_memory_returns_an_error(mi):
+    """The planner's lists for a million tiles do not fit a process whose address space may not grow: MI_ENOMEM, no exception
+    through the C interface."""
+    code = """
+import ctypes as C, resource, sys
+lib = C.CDLL(sys.argv[1])
+lib.mi_gemm_batch_plan_host.restype = lib.mi_gemm_batch_split_host.restype = C.c_int64
+i64 = C.c_int64
+mnk, pw, out = (i64 * 3)(262144, 262144, 384), C.c_int32(), (C.c_int32 * 4)()
+vm = int(open('/proc/self/statm').read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (vm + (4 << 20), resource.RLIM_INFINITY))
+a = lib.mi_gemm_batch_plan_host(mnk, 1, 256, out, i64(16), C.byref(pw))
+b = lib.mi_gemm_batch_split_host(mnk, 1, 256, out, out)
+print(a, b)
+"""
+    r = subprocess.run([sys.executable, "-c", code, mi.LIB_PATH], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout.split() == [str(mi.ENOMEM)] * 2, (r.returncode, r.stdout, r.stderr[-500:])
 
 
 def test_route_of_a_single_contraction(mi):
