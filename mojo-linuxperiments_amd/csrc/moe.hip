@@ -10,10 +10,10 @@
 //              y[token] = sum_slot w[token,slot] * out[pair]    (fixed order, no atomics)
 //
 // The expert GEMMs are weight-streaming bound (each expert sees ~32 rows): a
-// workgroup owns 16 gate + 16 up rows (or 32 down rows) of one expert, streams
-// them from HBM once through wave-private LDS rings, and walks the expert's
-// tokens 32 at a time with the gathered activation codes as MFMA B fragments.
-// Waves split K; partial accumulators meet in LDS.
+// workgroup takes row chunks of 16 gate + 16 up rows (or 128 down rows), streams
+// them from HBM once through wave-private LDS rings, and holds the expert's
+// tokens, up to 64 at a time, in registers as MFMA B fragments.  The chunks of all
+// experts that have tokens are dealt evenly to two workgroups a compute unit.
 //
 // Bound: HBM on the int8 expert weights, E * 3 * H * I bytes per layer call.
 #include "common.h"
@@ -400,11 +400,8 @@ __global__ __launch_bounds__(256) void k_moe_topk(const float *__restrict__ logi
 // One workgroup.  bm[e][t/32] bit t%32 = "token t picked expert e" (a token
 // picks an expert at most once), so the stable rank of pair (t, slot) inside
 // its expert is the number of set bits below t in row e.
-// order (optional): expert ids by descending segment size, so that the grouped GEMMs can start their longest
-// workgroups first.
 __device__ __forceinline__ void dispatch_pairs(uint32_t *s_dyn, const int32_t *idx, int32_t *__restrict__ perm,
-                                               int32_t *__restrict__ seg_off, int32_t *__restrict__ order, int T, int E,
-                                               int topk)
+                                               int32_t *__restrict__ seg_off, int T, int E, int topk)
 {
     const int W = (T + 31) >> 5;
     uint32_t *bm = s_dyn;                 // [E][W]
@@ -470,24 +467,6 @@ __device__ __forceinline__ void dispatch_pairs(uint32_t *s_dyn, const int32_t *i
     }
     __syncthreads();
     for (int e = tid; e <= E; e += nt) seg_off[e] = seg[e];
-    if (order) {
-        // rank of expert e among the counts (descending, ties by index): 8 lanes share an expert
-        for (int e0 = 0; e0 < E; e0 += nt / 8) {
-            const int e = e0 + (tid >> 3), part = tid & 7;
-            int rank = 0;
-            if (e < E) {
-                const int c = seg[e + 1] - seg[e];
-                for (int o = part; o < E; o += 8) {
-                    const int co = seg[o + 1] - seg[o];
-                    rank += (co > c || (co == c && o < e)) ? 1 : 0;
-                }
-            }
-            rank += __shfl_xor(rank, 1, 64);
-            rank += __shfl_xor(rank, 2, 64);
-            rank += __shfl_xor(rank, 4, 64);
-            if (e < E && part == 0) order[rank] = e;
-        }
-    }
     if (keep) {
 #pragma unroll
         for (int i = 0; i < KEEP; ++i) {
@@ -510,11 +489,10 @@ __device__ __forceinline__ void dispatch_pairs(uint32_t *s_dyn, const int32_t *i
 }
 
 __global__ __launch_bounds__(1024) void k_moe_dispatch(const int32_t *__restrict__ idx, int32_t *__restrict__ perm,
-                                                       int32_t *__restrict__ seg_off, int32_t *__restrict__ order,
-                                                       int T, int E, int topk)
+                                                       int32_t *__restrict__ seg_off, int T, int E, int topk)
 {
     extern __shared__ uint32_t s_dyn[];
-    dispatch_pairs(s_dyn, idx, perm, seg_off, order, T, E, topk);
+    dispatch_pairs(s_dyn, idx, perm, seg_off, T, E, topk);
 }
 
 // Top-k and dispatch of few tokens in one launch: a wave a token, the picks go to the dispatch
@@ -525,8 +503,7 @@ __global__ __launch_bounds__(1024) void k_moe_dispatch(const int32_t *__restrict
 constexpr int64_t ROUTE_DISPATCH_MAX_T = 16;
 __global__ __launch_bounds__(1024) void k_moe_topk_dispatch(const float *__restrict__ logits, int32_t *__restrict__ idx,
                                                             float *__restrict__ w, int32_t *__restrict__ perm,
-                                                            int32_t *__restrict__ seg_off, int32_t *__restrict__ order,
-                                                            int T, int E, int topk)
+                                                            int32_t *__restrict__ seg_off, int T, int E, int topk)
 {
     __shared__ int32_t s_idx[ROUTE_DISPATCH_MAX_T * MAX_TOPK];
     extern __shared__ uint32_t s_dyn[];
@@ -541,7 +518,7 @@ __global__ __launch_bounds__(1024) void k_moe_topk_dispatch(const float *__restr
         }
     }
     __syncthreads();
-    dispatch_pairs(s_dyn, s_idx, perm, seg_off, order, T, E, topk);
+    dispatch_pairs(s_dyn, s_idx, perm, seg_off, T, E, topk);
 }
 
 // ------------------------------------------------------- a11 grouped GEMMs
@@ -558,6 +535,16 @@ template <int N>
 __device__ __forceinline__ void wait_vm()
 {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// direct-to-LDS load of 16 bytes per lane: global address = sbase + voff, LDS address = ldsaddr + 16 * lane.  As an asm
+// statement: in front of an LDS atomic the compiler waits for every such load in flight that it knows of.
+__device__ __forceinline__ void dma16(const int8_t *sbase, unsigned voff, unsigned ldsaddr)
+{
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(voff), "s"(sbase), "s"(ldsaddr)
+                 : "memory", "m0");
 }
 
 constexpr int MT = 2;             // 16-token fragments per pass
@@ -729,153 +716,129 @@ __global__ __launch_bounds__(256) void k_moe_expert_gemm(const int8_t *__restric
 // The same contraction with the activation fragments held in registers (possible when a wave's K slice is at
 // most NSMAX steps of 128 bytes): only weights travel through the ring, twice as many of them are in flight
 // for the same LDS, and a workgroup walks several row chunks against one set of activation registers.
-// stages in flight per wave.  The down projection's workgroups are short (two chunks of 768-byte rows) and pay
-// their set-up (segment -> permutation -> activation rows, two dependent round trips) for little streaming: a ring
-// of two stages lets three of them share a compute unit instead of two (measured 61.5 -> 56 us); gate/up streams
-// six chunks of 2048-byte rows per workgroup and is better off with four stages in flight.
-constexpr int rx_ring(bool down) { return down ? 2 : 4; }
+constexpr int RX_RING = 4;   // stages in flight per wave (down with two, 2 or 3 workgroups a unit: 1.5 to 3 % slower a layer)
 constexpr int RX_STAGE = 2 * NGRP * 1024;
-constexpr int rx_ring_bytes(bool down) { return 4 * rx_ring(down) * RX_STAGE; }
-constexpr int RX_MT = 3;   // most 16-token fragments per pass
+constexpr int RX_RING_BYTES = 4 * RX_RING * RX_STAGE;
+constexpr int RX_MT = 4;   // most 16-token fragments per pass
 constexpr int RX_RED_BYTES = NGRP * RX_MT * 4 * 64 * 4;
-constexpr int rx_lds(bool down) { return rx_ring_bytes(down) + RX_RED_BYTES + 16 * RX_MT * 8 + 8 * 128 * 4; }   // + metadata + scales of <= 8 chunks
+constexpr int RX_LDS = RX_RING_BYTES + RX_RED_BYTES + 16 * RX_MT * 8 + 8 * 128 * 4;   // + metadata + scales of a run of chunks
 
+// Most tokens of a pass over an expert's weights: what the registers hold.  (512 tokens, H = 2048, 12 of 128 experts with more
+// than 48: 180 us for the layer's FFN with passes of 48, 176 with 64.)
+constexpr int rx_most(int nsmax) { return nsmax > 6 ? 32 : nsmax > 4 ? 48 : 64; }
+
+// One pass: at most 16 * MTT of an expert's pairs (from pos0 on, n of them) against nch row chunks from chunk c0 on.
+// first: the workgroup's first pass over these chunks, which brings their weight scales.
 template <bool DOWN, int NSMAX, int MTT>
-__device__ __forceinline__ void moe_expert_rx_body(const int8_t *__restrict__ act,
-                                                         const float *__restrict__ act_scale,
-                                                         const int32_t *__restrict__ perm,
-                                                         const int32_t *__restrict__ seg_off,
-                                                         const int8_t *__restrict__ w0, const float *__restrict__ sc0,
-                                                         const int8_t *__restrict__ w1, const float *__restrict__ sc1,
-                                                         float *__restrict__ out, int Kdim, int Nrows, int Hout,
-                                                         int topk, int nch, int e, int c0)
+__device__ __forceinline__ void rx_pass(char *smem, const int8_t *__restrict__ act, const float *__restrict__ act_scale,
+                                        const int32_t *__restrict__ perm, const int8_t *__restrict__ w0,
+                                        const float *__restrict__ sc0, const int8_t *__restrict__ w1,
+                                        const float *__restrict__ sc1, float *__restrict__ out, int Kdim, int Nrows, int topk,
+                                        int e, int c0, int nch, int pos0, int n, bool first)
 {
-    extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int seg0 = seg_off[e], count = seg_off[e + 1] - seg0;
-    if (count <= 0) return;
     // gate/up: the 4 waves split K (2048 bytes = 16 steps).  down: K is short (768 bytes = 6 steps), so each
-    // wave takes its own 32 rows over the whole of K and nothing has to be added across waves
-    // A workgroup walks `nch` consecutive row chunks from chunk c0 on (16 rows for gate/up, 128 for down; all of them
-    // inside the expert: the loads are not checked per row beyond the first chunk) as ONE stream: the
-    // loads of the next chunk are already in flight while the partial sums of this one are added and stored,
-    // and the segment / permutation lookups are paid once per workgroup.
-    constexpr int CHUNK_ROWS = DOWN ? 128 : 16;
-    const int n0 = DOWN ? c0 * 128 + wave * 32 : c0 * 16;
-    constexpr int RX_RING = rx_ring(DOWN), RX_RING_BYTES = rx_ring_bytes(DOWN);
-    char *ring = smem + wave * (RX_RING * RX_STAGE);
+    // wave takes its own 32 rows over the whole of K and nothing has to be added across waves.
+    // The row chunks (16 gate and 16 up rows, or 128 down rows) are ONE stream: the loads of the next chunk are already
+    // in flight while the partial sums of this one are added and stored.
+    constexpr int CHUNK_ROWS = DOWN ? 128 : 16, SCW = DOWN ? 128 : 32;
+    constexpr int RING = RX_RING;
+    char *ring = smem + wave * (RING * RX_STAGE);
     int *s_red = reinterpret_cast<int *>(smem + RX_RING_BYTES);    // [NGRP][MTT][4][64] sums over the four K slices (gate/up)
-    // per-pass token metadata and per-chunk weight scales sit in LDS so that the epilogue of a chunk issues no
-    // dependent global loads (each would cost a memory round trip per chunk)
-    int *s_dst = reinterpret_cast<int *>(smem + RX_RING_BYTES + RX_RED_BYTES);                  // [16*MTT] output row
-    float *s_tsc = reinterpret_cast<float *>(s_dst + 16 * MTT);                                  // [16*MTT] token scale
-    float *s_wsc = s_tsc + 16 * MTT;                                                             // [nch][SCW]
-    constexpr int SCW = DOWN ? 128 : 32;
-    // weight scales of every chunk: requested here, parked in LDS only after the weight stream and the
-    // activation loads have been issued, so that the whole set-up costs one memory round trip
-    float wsv[4];   // nch * SCW <= 8 * 128 = 4 values per thread
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int o = tid + u * 256;
-        const int ch = o / SCW, nl = o - ch * SCW;
-        float v = 0.0f;
-        if (o < nch * SCW) {
-            if constexpr (DOWN) {
-                const int n = (c0 + ch) * 128 + nl;
-                if (n < Nrows) v = sc0[(int64_t)e * Nrows + n];
-            } else {
-                const int n = (c0 + ch) * 16 + (nl & 15);
-                if (n < Nrows) v = (nl < 16 ? sc0 : sc1)[(int64_t)e * Nrows + n];
-            }
-        }
-        wsv[u] = v;
-    }
-    if constexpr (!DOWN) {
-        for (int o = tid; o < NGRP * MTT * 256; o += 256) s_red[o] = 0;
-    }
+    // token metadata and the chunks' weight scales sit in LDS so that the epilogue of a chunk issues no dependent global
+    // loads (each would cost a memory round trip per chunk)
+    int *s_dst = reinterpret_cast<int *>(smem + RX_RING_BYTES + RX_RED_BYTES);            // [48] output row
+    float *s_tsc = reinterpret_cast<float *>(s_dst + 16 * RX_MT);                                // [48] token scale
+    float *s_wsc = s_tsc + 16 * RX_MT;                                                           // [nch][SCW]
 
-    // load side: lane l = 8*rho + c fetches chunk c ^ sigma(rho, block parity) of row rho of the block
+    __syncthreads();   // the previous pass has finished with the token metadata and the scales, and every ring is idle
+
+    // load side: lane l = 8*rho + c8 fetches chunk c8 ^ sigma(rho, block parity) of row rho of a block of 8 rows
     const int rho = lane >> 3, c8 = lane & 7;
-    const int8_t *wsrc[2 * NGRP];
-#pragma unroll
-    for (int b = 0; b < 2 * NGRP; ++b) {
-        const int sigma = ((b & 1) << 2) | (rho >> 1);
-        const int grp = b >> 1;
-        int rowi = n0 + (DOWN ? grp * 16 : 0) + (b & 1) * 8 + rho;
-        if (rowi > Nrows - 1) rowi = Nrows - 1;
-        const int8_t *base = (DOWN || grp == 0) ? w0 : w1;
-        wsrc[b] = base + ((int64_t)e * Nrows + rowi) * Kdim + ((c8 ^ sigma) << 4);
-    }
     const int steps = Kdim >> 7;
-    const int s0 = DOWN ? 0 : steps * wave / 4, s1 = DOWN ? steps : steps * (wave + 1) / 4;
-
-    // read side: fragment (16-row group, K half kk): lane (r = l%16, g = l/16) reads row r, chunk 4*kk + g
-    const int r = lane & 15, g_ = lane >> 4;
-    int roff[2];
-    {
-        const int rr = r & 7, bpar = r >> 3;
-        const int sigma = (bpar << 2) | (rr >> 1);
-        roff[0] = bpar * 1024 + ((8 * rr + ((0 + g_) ^ sigma)) << 4);
-        roff[1] = bpar * 1024 + ((8 * rr + ((4 + g_) ^ sigma)) << 4);
+    const int s0 = DOWN ? 0 : steps * wave / 4;
+    const int nsw = (DOWN ? steps : steps * (wave + 1) / 4) - s0;   // K steps of this wave per chunk (<= NSMAX)
+    const unsigned woff0 = (unsigned)rho * (unsigned)Kdim + ((c8 ^ (rho >> 1)) << 4);   // an even block; an odd one is below it
+    const unsigned woff1 = (unsigned)(8 + rho) * (unsigned)Kdim + ((c8 ^ (4 | rho >> 1)) << 4);
+    // the (chunk, step) stages of this wave are one stream; past its end the last stage is fetched again (uniform vmcnt
+    // arithmetic)
+    const int64_t row0 = (int64_t)e * Nrows + c0 * CHUNK_ROWS;
+    const int8_t *p0 = w0 + (row0 + (DOWN ? wave * 32 : 0)) * Kdim + s0 * 128;
+    const int8_t *p1 = DOWN ? p0 : w1 + row0 * Kdim + s0 * 128;
+    const unsigned second = DOWN ? 16u * (unsigned)Kdim : 0;   // of the down rows: from the first 16 to the next
+    int step_left = nsw, chunk_left = nch;
+    const unsigned ring_at = (unsigned)(uintptr_t)(lptr_t)ring;
+    auto issue = [&](int slot) {
+        const unsigned at = ring_at + slot * RX_STAGE;
+        dma16(p0, woff0, at);
+        dma16(p0, woff1, at + 1024);
+        dma16(DOWN ? p0 : p1, woff0 + second, at + 2048);
+        dma16(DOWN ? p0 : p1, woff1 + second, at + 3072);
+        int by = 128;
+        if (--step_left == 0) {
+            step_left = nsw;
+            by = CHUNK_ROWS * Kdim - (nsw - 1) * 128;
+            if (--chunk_left <= 0) by = 0, step_left = 1;
+        }
+        p0 += by;
+        if (!DOWN) p1 += by;
+    };
+    // weight scales (nch * SCW <= 1024) and the pair whose metadata this thread brings: requested here, parked below
+    float wsc_now[4];
+    if (first) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int o = min(tid + u * 256, nch * SCW - 1);
+            if constexpr (DOWN) wsc_now[u] = sc0[row0 + o];
+            else wsc_now[u] = ((o & 16) ? sc1 : sc0)[row0 + (o >> 5) * 16 + (o & 15)];
+        }
     }
+    const int pos = pos0 + min(tid, n - 1), pair = perm[pos];
+    // the weight stream starts first: its addresses do not depend on the tokens, whose lookups cost two dependent memory
+    // round trips
+    if (nsw > 0) {
+#pragma unroll
+        for (int d = 0; d < RING; ++d) issue(d);
+    }
+    // Activation rows as MFMA fragments held in registers for every chunk: lane (token r, 16-byte chunk g_ (+4)).  Rows past
+    // the segment repeat its last row and are never stored.
+    const int r = lane & 15, g_ = lane >> 4;
+    v4i xr[MTT][NSMAX][2];
+    int last_step = steps - 1 - s0;
+    asm volatile("" : "+v"(last_step));   // (scalar registers are what this kernel has fewest of)
+#pragma unroll
+    for (int b = 0; b < MTT; ++b) {
+        const int at = pos0 + min(b * 16 + r, n - 1);
+        const int8_t *xp = act + (DOWN ? (int64_t)at : (int64_t)(perm[at] / topk)) * Kdim + g_ * 16 + s0 * 128;
+#pragma unroll
+        for (int i = 0; i < NSMAX; ++i) {
+            const unsigned st = (unsigned)min(i, last_step) * 128;
+            xr[b][i][0] = *reinterpret_cast<const v4i *>(xp + st);
+            xr[b][i][1] = *reinterpret_cast<const v4i *>(xp + st + 64);
+        }
+    }
+    if (tid < 16 * MTT) {
+        s_dst[tid] = DOWN ? pair : pos;
+        s_tsc[tid] = act_scale[DOWN ? pos : pair / topk];
+    }
+    if (first) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s_wsc[min(tid + u * 256, nch * SCW - 1)] = wsc_now[u];
+    }
+    __syncthreads();   // token metadata, weight scales and the zeroed sums are visible to every wave
 
-    for (int base = 0; base < count; base += 16 * MTT) {
-        const int nsw = s1 - s0;            // K steps of this wave per chunk (<= NSMAX)
-        const int total_f = nch * nsw;      // flattened (chunk, step) stages of this wave
-        auto issue = [&](int slot, int f) {
-            const int fc = f < total_f ? f : total_f - 1;   // past the end: re-fetch the last stage (uniform vmcnt arithmetic)
-            const int ch = fc / nsw, st = s0 + (fc - ch * nsw);
-            char *sb = ring + slot * RX_STAGE;
-            const int64_t woff = (int64_t)ch * CHUNK_ROWS * Kdim + (int64_t)st * 128;
-#pragma unroll
-            for (int b = 0; b < 2 * NGRP; ++b)
-                __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[b] + woff), (lptr_t)(sb + b * 1024), 16, 0, 0);
-        };
-        // Activation rows of this pass, as MFMA fragments held in registers for every row chunk the workgroup
-        // walks: lane (token r, 16-byte chunk g_ (+4)).  Rows past the segment repeat its last row and are never
-        // stored.
-        v4i xr[MTT][NSMAX][2];
-        __syncthreads();   // the previous pass has finished with the token metadata and every ring is idle
-        int m_dst = 0, m_pr = 0;
-        if (tid < 16 * MTT && base + tid < count) {
-            const int pos = seg0 + base + tid;
-            m_pr = perm[pos];
-            m_dst = DOWN ? m_pr : pos;
-        }
-        {
-            // the weight stream starts first: its addresses do not depend on the tokens, whose lookups cost two
-            // dependent memory round trips
-            if (nsw > 0) {
-#pragma unroll
-                for (int d = 0; d < RX_RING; ++d) issue(d, d);
-            }
-#pragma unroll
-            for (int b = 0; b < MTT; ++b) {
-                const int pos = seg0 + min(base + b * 16 + r, count - 1);
-                const int8_t *xp = act + (DOWN ? (int64_t)pos : (int64_t)(perm[pos] / topk)) * Kdim + g_ * 16;
-#pragma unroll
-                for (int i = 0; i < NSMAX; ++i) {
-                    const int st = min(s0 + i, steps - 1);
-                    xr[b][i][0] = *reinterpret_cast<const v4i *>(xp + (int64_t)st * 128);
-                    xr[b][i][1] = *reinterpret_cast<const v4i *>(xp + (int64_t)st * 128 + 64);
-                }
-            }
-        }
-
-        if (tid < 16 * MTT && base + tid < count) {
-            s_dst[tid] = m_dst;
-            s_tsc[tid] = act_scale[DOWN ? seg0 + base + tid : m_pr / topk];
-        }
-        if (base == 0) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (tid + u * 256 < nch * SCW) s_wsc[tid + u * 256] = wsv[u];
-        }
-        __syncthreads();   // token metadata, weight scales and the zeroed sums are visible to every wave
-        int slot = 0, f = 0;
-        for (int ch = 0; ch < nch; ++ch) {
-        const int nc0 = n0 + ch * CHUNK_ROWS;
+    // read side: fragment (16-row group, K half kk): lane (row r = l%16, g_ = l/16) reads row r, chunk 4*kk + g_
+    const char *frag0, *frag1;
+    {
+        const int rr = r & 7, par = r >> 3, sigma = (par << 2) | (rr >> 1);
+        frag0 = ring + par * 1024 + ((8 * rr + (g_ ^ sigma)) << 4);
+        frag1 = ring + par * 1024 + ((8 * rr + ((4 + g_) ^ sigma)) << 4);
+    }
+    int slot = 0;
+    for (int ch = 0; ch < nch; ++ch) {
+        int left = n, steps_here = nsw;   // opaque, or the compiler keeps every comparison with them in scalar registers
+        asm volatile("" : "+s"(left), "+s"(steps_here));
         v4i acc[NGRP][MTT];
 #pragma unroll
         for (int a = 0; a < NGRP; ++a)
@@ -883,26 +846,25 @@ __device__ __forceinline__ void moe_expert_rx_body(const int8_t *__restrict__ ac
             for (int b = 0; b < MTT; ++b) acc[a][b] = (v4i){0, 0, 0, 0};
 #pragma unroll
         for (int i = 0; i < NSMAX; ++i) {
-            if (i < nsw) {
-                wait_vm<(RX_RING - 1) * 2 * NGRP>();   // the oldest stage in flight has landed
-                const char *sb = ring + slot * RX_STAGE;
-                v4i wf[NGRP][2];
+            asm volatile("" : "+s"(steps_here));
+            if (i >= steps_here) continue;
+            wait_vm<(RING - 1) * 2 * NGRP>();   // the oldest stage in flight has landed
+            v4i wf[NGRP][2];
 #pragma unroll
-                for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-                    for (int a = 0; a < NGRP; ++a) wf[a][kk] = *reinterpret_cast<const v4i *>(sb + a * 2048 + roff[kk]);
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // fragments are in registers: the slot may be refilled
-                issue(slot, f + RX_RING);
-#pragma unroll
-                for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-                    for (int a = 0; a < NGRP; ++a)
-#pragma unroll
-                        for (int b = 0; b < MTT; ++b)
-                            acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[a][kk], xr[b][i][kk], acc[a][b], 0, 0, 0);
-                slot = slot + 1 == RX_RING ? 0 : slot + 1;
-                ++f;
+            for (int a = 0; a < NGRP; ++a) {
+                wf[a][0] = *reinterpret_cast<const v4i *>(frag0 + slot * RX_STAGE + a * 2048);
+                wf[a][1] = *reinterpret_cast<const v4i *>(frag1 + slot * RX_STAGE + a * 2048);
             }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // fragments are in registers: the slot may be refilled
+            issue(slot);
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+                for (int a = 0; a < NGRP; ++a)
+#pragma unroll
+                    for (int b = 0; b < MTT; ++b)
+                        acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[a][kk], xr[b][i][kk], acc[a][b], 0, 0, 0);
+            slot = slot + 1 == RING ? 0 : slot + 1;
         }
         const float *wsc = s_wsc + ch * SCW;
         // accumulator layout: lane l, register q  <->  weight row 4*(l/16)+q, token l%16
@@ -918,24 +880,23 @@ __device__ __forceinline__ void moe_expert_rx_body(const int8_t *__restrict__ ac
             __syncthreads();
             // 16*MTT tokens x 16 channels, channel fastest; h = silu(g) * u in sorted-pair order
 #pragma unroll
-            for (int o = tid; o < 16 * MTT * 16; o += 256) {
-                const int nl = o & 15, row = o >> 4;
-                const int bq = (((row >> 4) * 4) + (nl & 3)) * 64 + (nl >> 2) * 16 + (row & 15);
+            for (int b = 0; b < MTT; ++b) {
+                const int nl = tid & 15, row = b * 16 + (tid >> 4);
+                const int bq = (b * 4 + (nl & 3)) * 64 + (nl >> 2) * 16 + (row & 15);
                 const int gi = s_red[bq], ui = s_red[MTT * 256 + bq];
                 s_red[bq] = 0;
                 s_red[MTT * 256 + bq] = 0;
-                if (base + row < count && nc0 + nl < Nrows) {
+                if (row < left) {
                     const float sxt = s_tsc[row];
                     const float gv = ((float)gi * sxt) * wsc[nl];
                     const float uv = ((float)ui * sxt) * wsc[16 + nl];
-                    out[(int64_t)s_dst[row] * Nrows + nc0 + nl] = (gv / (1.0f + expf(-gv))) * uv;
+                    out[(int64_t)s_dst[row] * Nrows + (c0 + ch) * 16 + nl] = (gv / (1.0f + expf(-gv))) * uv;
                 }
             }
             __syncthreads();   // the zeroes are in place before the next chunk's sums arrive
         } else {
             // every wave owns its 32 rows over the whole of K: results leave straight from the accumulators, four
             // consecutive channels of one token per lane; out[pair] in pair order
-            const int nbase = (c0 + ch) * 128;
 #pragma unroll
             for (int a = 0; a < NGRP; ++a) {
                 const int nl = wave * 32 + a * 16 + 4 * g_;
@@ -943,63 +904,115 @@ __device__ __forceinline__ void moe_expert_rx_body(const int8_t *__restrict__ ac
 #pragma unroll
                 for (int b = 0; b < MTT; ++b) {
                     const int row = b * 16 + r;
-                    if (base + row < count && nbase + nl < Nrows) {
+                    if (row < left) {
                         const float ts = s_tsc[row];
                         float4 o;
                         o.x = ((float)acc[a][b][0] * ts) * ws.x;
                         o.y = ((float)acc[a][b][1] * ts) * ws.y;
                         o.z = ((float)acc[a][b][2] * ts) * ws.z;
                         o.w = ((float)acc[a][b][3] * ts) * ws.w;
-                        *reinterpret_cast<float4 *>(out + (int64_t)s_dst[row] * Hout + nbase + nl) = o;
+                        *reinterpret_cast<float4 *>(out + (int64_t)s_dst[row] * Nrows + (c0 + ch) * 128 + nl) = o;
                     }
                 }
             }
         }
-        }   // chunks
-        wait_vm<0>();   // trailing re-fetches must not write LDS after the workgroup has gone
     }
+    wait_vm<0>();   // trailing re-fetches must not write LDS behind this pass
 }
 
-// Grid: one dimension.  The first y_split experts of the size order are cut into workgroups of `nch` row chunks,
-// the rest (the smallest segments, which run last: the launcher takes the last eighth) into workgroups of nch / 2
-// chunks: the work that is left when the kernel runs dry then comes in pieces half as long, and the tail of the
-// kernel with them (cfg4: 210 -> 205 us for the layer; halving a quarter or more of the experts gives it back).
-template <bool DOWN, int NSMAX>
-__global__ __launch_bounds__(256) void k_moe_expert_rx(const int8_t *__restrict__ act,
-                                                       const float *__restrict__ act_scale,
-                                                       const int32_t *__restrict__ perm,
-                                                       const int32_t *__restrict__ seg_off,
-                                                       const int8_t *__restrict__ w0, const float *__restrict__ sc0,
-                                                       const int8_t *__restrict__ w1, const float *__restrict__ sc1,
-                                                       float *__restrict__ out, int Kdim, int Nrows, int Hout,
-                                                       int topk, int nch, const int32_t *__restrict__ order,
-                                                       int chunks, int y_split)
+// Inclusive sum over the lanes up to this one, on the vector pipe alone (a shuffle would cost an LDS round trip a step).
+__device__ __forceinline__ int wave_scan(int v)
 {
-    // workgroups are handed out in grid order: the experts with the most tokens go first
-    const int wpe = (chunks + nch - 1) / nch;
-    int y, bx, nchl;
-    {
-        const int i = blockIdx.x;
-        if (i < y_split * wpe) {
-            y = i / wpe; bx = i - y * wpe; nchl = nch;
-        } else {
-            nchl = nch > 1 ? nch / 2 : 1;
-            const int wpe2 = (chunks + nchl - 1) / nchl;
-            const int j = i - y_split * wpe;
-            y = y_split + j / wpe2; bx = j - (j / wpe2) * wpe2;
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);    // row_shr:1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
+// The row chunks of all experts that have tokens, one behind the other in expert order and once per pass over them, are dealt
+// evenly to two workgroups a compute unit (what LDS and registers hold): workgroup i of G takes the chunks that begin in the
+// i-th of G equal shares, a run that may end one expert and begin the next.  Before, runs of a fixed length in an order by size
+// filled the units twice and a bit, with half of the experts idle at 16 tokens, and every run paid its set-up.
+// Bound by HBM.  Both expert kernels at H = 2048, I = 768, 128 experts, top-8, us before -> after: 16 tokens 90 -> 75,
+// 512 tokens at 32 an expert 147 -> 137 (604 MB at 4.4 TB/s; 115 without the results' 46 MB of stores, 110 without the matrix
+// instructions as well).  Measured without gain: non-temporal stores and loads, whole 128-byte lines per store, exact counts of
+// the stores in the waits, costs that grow with an expert's tokens, rings of two stages, three workgroups a unit.
+// by_chunk: at most a chunk a workgroup, all of the same cost, with the compute units' own order as the balance.
+template <bool DOWN, int NSMAX>
+__global__ __launch_bounds__(256, 2) void k_moe_expert_rx(const int8_t *__restrict__ act,
+                                                          const float *__restrict__ act_scale,
+                                                          const int32_t *__restrict__ perm,
+                                                          const int32_t *__restrict__ seg_off,
+                                                          const int8_t *__restrict__ w0, const float *__restrict__ sc0,
+                                                          const int8_t *__restrict__ w1, const float *__restrict__ sc1,
+                                                          float *__restrict__ out, int Kdim, int Nrows, int topk, int chunks,
+                                                          int E, int by_chunk)
+{
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    constexpr int PASS = rx_most(NSMAX);
+    if constexpr (!DOWN) {
+        int *s_red = reinterpret_cast<int *>(smem + RX_RING_BYTES);
+        for (int o = tid; o < RX_RED_BYTES / 4; o += 256) s_red[o] = 0;
+    }
+    // cost of a row chunk: the passes over it (all sums fit in 31 bits: at most (65535 + 2^24 / 32) passes of 2048 chunks)
+    const int per_pass = by_chunk ? INT32_MAX - (1 << 24) : PASS;
+    auto cost = [&](int count) { return (int)((unsigned)(count + per_pass - 1) / (unsigned)per_pass); };
+    auto segment = [&](int e, int *first, int *count) {   // of expert e, which may lie past the last one
+        *first = seg_off[min(e, E)];
+        *count = seg_off[min(e + 1, E)] - *first;
+    };
+    int total = 0;
+    for (int b = 0; b < E; b += 64) {
+        int s, c;
+        segment(b + lane, &s, &c);
+        total += __builtin_amdgcn_readlane(wave_scan(cost(c)), 63);
+    }
+    total *= chunks;
+    const int share = total / gridDim.x, rest = total - share * gridDim.x, wg = blockIdx.x;
+    const int lo = wg * share + min(wg, rest), hi = lo + share + (wg < rest ? 1 : 0);
+    // the first expert that reaches past lo, and where it begins
+    int e = 0, at = 0, seg0 = 0, count = 0;
+    for (; e < E; e += 64) {
+        int s, n;
+        segment(e + lane, &s, &n);
+        const int c = cost(n), incl = wave_scan(c);
+        const unsigned long long past = __ballot((at + incl) * chunks > lo);
+        if (past) {
+            const int l = __ffsll((long long)past) - 1;
+            at += __builtin_amdgcn_readlane(incl - c, l);
+            seg0 = __builtin_amdgcn_readlane(s, l);
+            count = __builtin_amdgcn_readlane(n, l);
+            e += l;
+            break;
+        }
+        at += __builtin_amdgcn_readlane(incl, 63);
+    }
+    int skip = lo - at * chunks, left = hi - at * chunks;   // of the share, from where expert e begins
+    constexpr int MOST = DOWN ? 8 : 32;   // chunks whose weight scales LDS holds
+    for (; e < E && left > 0; segment(++e, &seg0, &count)) {
+        const int passes = cost(count);
+        const int last = passes ? min(chunks, (left + passes - 1) / passes) : 0;
+        int c0 = passes ? (skip + passes - 1) / passes : 0;
+        skip = 0;
+        left -= passes * chunks;
+        for (; c0 < last; c0 += MOST) {
+            const int nch = min(MOST, last - c0);
+            for (int base = 0; base < count; base += PASS) {
+                const int n = min(PASS, count - base);
+#define MI_RX_PASS(MT_) rx_pass<DOWN, NSMAX, MT_>(smem, act, act_scale, perm, w0, sc0, w1, sc1, out, Kdim, Nrows, topk, e, c0, \
+                                                  nch, seg0 + base, n, base == 0)
+                if (n <= 16) MI_RX_PASS(1);
+                else if (n <= 32 || PASS == 32) MI_RX_PASS(2);
+                else if (n <= 48 || PASS == 48) MI_RX_PASS(PASS == 32 ? 2 : 3);
+                else MI_RX_PASS(PASS / 16);
+#undef MI_RX_PASS
+            }
         }
     }
-    const int c0 = bx * nchl;
-    nchl = min(nchl, chunks - c0);   // the last workgroup of an expert whose chunks nchl does not divide
-    const int e = order[y];
-    // tokens per pass follow the size of the expert's segment: every extra pass streams the weights again
-    const int count = seg_off[e + 1] - seg_off[e];
-    if (count <= 16)
-        moe_expert_rx_body<DOWN, NSMAX, 1>(act, act_scale, perm, seg_off, w0, sc0, w1, sc1, out, Kdim, Nrows, Hout, topk, nchl, e, c0);
-    else if (count <= 32 || NSMAX > 6)
-        moe_expert_rx_body<DOWN, NSMAX, 2>(act, act_scale, perm, seg_off, w0, sc0, w1, sc1, out, Kdim, Nrows, Hout, topk, nchl, e, c0);
-    else
-        moe_expert_rx_body<DOWN, NSMAX, 3>(act, act_scale, perm, seg_off, w0, sc0, w1, sc1, out, Kdim, Nrows, Hout, topk, nchl, e, c0);
 }
 
 // y[t, n] = sum over slots in order of w[t, slot] * out[t*topk + slot, n].  A slot whose expert index lies outside
@@ -1046,7 +1059,7 @@ struct Layout {
 static Layout layout(int64_t T, int64_t H, int64_t I, int64_t E, int64_t topk)
 {
     const int64_t P = T * topk;
-    const int64_t sz[11] = {T * H, T * 4, P * 4, (2 * E + 1) * 4 /* seg_off, then experts by size */, P * I * 4, P * I, P * 4, P * H * 4, P * 4, P * 4, T * E * 4};
+    const int64_t sz[11] = {T * H, T * 4, P * 4, (2 * E + 1) * 4 /* seg_off */, P * I * 4, P * I, P * 4, P * H * 4, P * 4, P * 4, T * E * 4};
     Layout L;
     int64_t o = 0;
     for (int i = 0; i < 11; ++i) { L.off[i] = o; o += align_up(sz[i], 256); }
@@ -1112,7 +1125,7 @@ static int32_t launch_route(const float *x, const float *wr, int32_t *idx, float
     if (perm) {
         const size_t words = (size_t)(2 * E * ((T + 31) / 32) + E + 1);
         hipLaunchKernelGGL(k_moe_topk_dispatch, dim3(1), dim3(1024), words * 4, as_stream(stream), logits, idx, w, perm, seg,
-                           seg + E + 1, (int)T, (int)E, (int)topk);
+                           (int)T, (int)E, (int)topk);
         return launch_status();
     }
     hipLaunchKernelGGL(k_moe_topk, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, as_stream(stream), logits, idx, w, (int)T,
@@ -1145,8 +1158,8 @@ extern "C" int32_t mi_moe_route(const float *x, const float *wr, int32_t *idx, f
                              nullptr, stream);
 }
 
-static int32_t launch_dispatch(const int32_t *idx, int32_t *perm, int32_t *seg_off, int32_t *order, int64_t T,
-                               int64_t E, int32_t topk, void *stream)
+extern "C" int32_t mi_moe_dispatch(const int32_t *idx, int32_t *perm, int32_t *seg_off, int64_t T, int64_t E,
+                                   int32_t topk, void *stream)
 {
     if (!idx || !perm || !seg_off || T < 0 || E <= 0 || topk <= 0) return MI_EINVAL;
     if (T * topk > (1LL << 24) || E > 65535) return MI_ERANGE;
@@ -1154,14 +1167,8 @@ static int32_t launch_dispatch(const int32_t *idx, int32_t *perm, int32_t *seg_o
     if (words > moe::DISPATCH_MAX_WORDS) return MI_ERANGE;
     MI_LDS_OPT_IN((&moe::k_moe_dispatch), (int)(moe::DISPATCH_MAX_WORDS * 4));
     hipLaunchKernelGGL(moe::k_moe_dispatch, dim3(1), dim3(1024), (size_t)words * 4, as_stream(stream), idx, perm,
-                       seg_off, order, (int)T, (int)E, (int)topk);
+                       seg_off, (int)T, (int)E, (int)topk);
     return launch_status();
-}
-
-extern "C" int32_t mi_moe_dispatch(const int32_t *idx, int32_t *perm, int32_t *seg_off, int64_t T, int64_t E,
-                                   int32_t topk, void *stream)
-{
-    return launch_dispatch(idx, perm, seg_off, nullptr, T, E, topk, stream);
 }
 
 extern "C" int64_t mi_moe_ffn_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E, int32_t topk)
@@ -1212,9 +1219,8 @@ static int32_t run_ffn(const float *x, const int32_t *idx, const float *w, const
     hipStream_t s = as_stream(stream);
     const int64_t P = T * topk;
 
-    int32_t *order = seg + E + 1;
     if (!dispatched) {
-        rc = launch_dispatch(idx, perm, seg, order, T, E, topk, stream);
+        rc = mi_moe_dispatch(idx, perm, seg, T, E, topk, stream);
         if (rc) return rc;
     }
     if (!codes_ready) {
@@ -1223,24 +1229,19 @@ static int32_t run_ffn(const float *x, const int32_t *idx, const float *w, const
     }
     MI_LDS_OPT_IN((&moe::k_moe_expert_gemm<false>), moe::EXPERT_LDS);
     MI_LDS_OPT_IN((&moe::k_moe_expert_gemm<true>), moe::EXPERT_LDS);
-    // Row chunks per workgroup: with the activation fragments in registers a workgroup walks several chunks
-    // against them; about four workgroups per compute unit keep the stream dense.
     const int cus = compute_units();
-    auto pick_nch = [&](int64_t chunks) {
-        int64_t n = chunks * E / (4LL * cus);
-        return (int)(n < 1 ? 1 : (n > 8 ? 8 : n));
-    };
+    // Two workgroups a unit, or one per row chunk where these are fewer.  One per chunk beyond that loses where an expert needs a
+    // pass or two (a layer of 512 tokens, H = 2048, I = 768, 64 experts, top-8: 158 -> 201 us), three or four a unit by 1 to 15 %.
+    auto one_chunk = [&](int64_t chunks) { return (int)(chunks * std::min(E, P) <= 2 * cus); };
     const int steps_gu = (int)(H / 128), ns_gu = (steps_gu + 3) / 4;   // K steps per wave (the four waves split K)
     if (ns_gu <= 8) {
-        const int nch = pick_nch(I / 16);
-        const int chunks = (int)(I / 16), y_split = (int)(E - E / 8);
-        const int wpe = (chunks + nch - 1) / nch, nch2 = nch > 1 ? nch / 2 : 1, wpe2 = (chunks + nch2 - 1) / nch2;
-        const dim3 grid((unsigned)(y_split * wpe + (E - y_split) * wpe2));
+        const int chunks = (int)(I / 16), by_chunk = one_chunk(chunks);
+        const dim3 grid(by_chunk ? (unsigned)(chunks * std::min<int64_t>(E, P)) : 2u * cus);
 #define MI_RX_GU(NS)                                                                                            \
     do {                                                                                                        \
-        MI_LDS_OPT_IN((&moe::k_moe_expert_rx<false, NS>), moe::rx_lds(false));                                        \
-        hipLaunchKernelGGL((moe::k_moe_expert_rx<false, NS>), grid, dim3(256), moe::rx_lds(false), s, qx, sx, perm, seg, \
-                           wg, sg, wu, su, h, (int)H, (int)I, (int)I, (int)topk, nch, order, chunks, y_split);  \
+        MI_LDS_OPT_IN((&moe::k_moe_expert_rx<false, NS>), moe::RX_LDS);                                        \
+        hipLaunchKernelGGL((moe::k_moe_expert_rx<false, NS>), grid, dim3(256), moe::RX_LDS, s, qx, sx, perm, seg, \
+                           wg, sg, wu, su, h, (int)H, (int)I, (int)topk, chunks, (int)E, by_chunk);     \
     } while (0)
         if (ns_gu <= 2) MI_RX_GU(2);
         else if (ns_gu <= 4) MI_RX_GU(4);
@@ -1257,16 +1258,14 @@ static int32_t run_ffn(const float *x, const int32_t *idx, const float *w, const
     if (rc) return rc;
     const int steps_dn = (int)(I / 128);   // every wave walks the whole of K
     if (steps_dn <= 8) {
-        const int chunks = (int)((H + 127) / 128);
-        const int nch = pick_nch(chunks), y_split = (int)(E - E / 8);
-        const int wpe = (chunks + nch - 1) / nch, nch2 = nch > 1 ? nch / 2 : 1, wpe2 = (chunks + nch2 - 1) / nch2;
-        const dim3 grid((unsigned)(y_split * wpe + (E - y_split) * wpe2));
+        const int chunks = (int)(H / 128), by_chunk = one_chunk(chunks);
+        const dim3 grid(by_chunk ? (unsigned)(chunks * std::min<int64_t>(E, P)) : 2u * cus);
 #define MI_RX_DN(NS)                                                                                            \
     do {                                                                                                        \
-        MI_LDS_OPT_IN((&moe::k_moe_expert_rx<true, NS>), moe::rx_lds(true));                                        \
-        hipLaunchKernelGGL((moe::k_moe_expert_rx<true, NS>), grid, dim3(256), moe::rx_lds(true), s, hq, hs, perm, seg, wd, \
-                           sd, (const int8_t *)nullptr, (const float *)nullptr, out, (int)I, (int)H, (int)H,    \
-                           (int)topk, nch, order, chunks, y_split);                                             \
+        MI_LDS_OPT_IN((&moe::k_moe_expert_rx<true, NS>), moe::RX_LDS);                                        \
+        hipLaunchKernelGGL((moe::k_moe_expert_rx<true, NS>), grid, dim3(256), moe::RX_LDS, s, hq, hs, perm, seg, wd, \
+                           sd, (const int8_t *)nullptr, (const float *)nullptr, out, (int)I, (int)H,            \
+                           (int)topk, chunks, (int)E, by_chunk);                                                \
     } while (0)
         if (steps_dn <= 2) MI_RX_DN(2);
         else if (steps_dn <= 4) MI_RX_DN(4);

@@ -169,6 +169,28 @@ def test_ffn_skewed_routing_many_rows_per_expert(mi, dev, orc):
     dev.reset_to(mark)
 
 
+@pytest.mark.parametrize("H,I,E,counts", [
+    (256, 256, 80, (0, 1, 15, 16, 17, 32, 33, 48, 49, 64, 65)),   # both sides of every group of 16 tokens and of a second pass
+    (256, 768, 130, (0, 0, 0, 3, 64, 0, 0, 129)),                 # runs of idle experts, more than two waves of 64 of them
+    (4096, 1024, 16, (31, 32, 33, 65)),                           # passes of 32 tokens
+    (128, 256, 4, (0, 2, 0, 0)),                                  # fewer row chunks than compute units
+    (128, 4096, 96, (1,)),                                        # more row chunks a workgroup than LDS holds scales of
+])
+def test_ffn_segments_of_every_size(mi, dev, orc, H, I, E, counts):
+    """One pick a token, so that expert e gets counts[e % len] tokens: the dealing of the experts' row chunks to workgroups and
+    the passes over them."""
+    mark = dev.mark()
+    flat = np.repeat(np.arange(E), [counts[e % len(counts)] for e in range(E)]).astype(np.int32)
+    idx = np.random.default_rng(58).permutation(flat).reshape(-1, 1)
+    T = idx.shape[0]
+    x = workload.activations(58, T, H)
+    w = np.ones((T, 1), np.float32)
+    experts = make_experts(orc, 59, E, H, I)
+    r = run_ffn(mi, dev, x, idx, w, experts)
+    check_ffn_against_oracle(orc, x, idx, w, experts, r)
+    dev.reset_to(mark)
+
+
 def test_ffn_slot_with_an_expert_out_of_range_contributes_nothing(mi, dev, orc):
     """A caller-made idx with an index outside [0, E): that pair is never dispatched, its row of the workspace is
     never written, and the combine leaves it out: y equals the FFN over the remaining slots."""
