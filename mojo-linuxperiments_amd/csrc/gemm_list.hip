@@ -52,6 +52,7 @@
 #include "common.h"
 #include "gemm_deep.h"
 #include "gemm_pair_ops.h"
+#include "gemm_stream.h"
 
 #ifndef MI_STORE_MOD
 #define MI_STORE_MOD " nt"   // the results are not read again by this kernel: stores that do not displace the operands in L2 (measured: 385 -> 363 us for the four prefill projections as one batch)
@@ -547,9 +548,10 @@ static inline int tile_cost(int64_t K) { return (int)(K / 128) + 10; }
 // instead of 1,189 MB fetched per launch (operands 256 MB), 338 against 344 us with the weights resident in the
 // memory-side cache and 355 against 371 us with weights that come from HBM; patches of 1, 2 and 8 row tiles
 // measured 355 / 344 / 339 us (resident) and 366 / 364 / 369 us (from HBM).
+// Returns the entries of the longest workgroup's list, or an error.
 template <int BM, int BN>
-static int64_t build_lists(const int64_t *mnk, int n, int cus, std::vector<v4i> *lists, int *per_wg_out)
-try {
+static int64_t deal_tiles(const int64_t *mnk, int n, int cus, std::vector<std::vector<Tile>> *out)
+{
     const int nx = (cus % 8 == 0) ? 8 : 1, slots = cus / nx;
     constexpr int ROWS = 4;
     std::vector<int> order((size_t)n);
@@ -576,7 +578,8 @@ try {
                     blocks.back().push_back(tl);
                 }
     }
-    std::vector<std::vector<Tile>> q((size_t)cus);
+    std::vector<std::vector<Tile>> &q = *out;
+    q.assign((size_t)cus, {});
     std::vector<int64_t> load((size_t)nx, 0);
     std::vector<std::vector<const std::vector<Tile> *>> mine((size_t)nx);
     for (const auto &b : blocks) {
@@ -599,6 +602,15 @@ try {
     }
     size_t longest = 0;
     for (const auto &v : q) longest = std::max(longest, v.size());
+    return (int64_t)longest;
+}
+
+template <int BM, int BN>
+static int64_t build_lists(const int64_t *mnk, int n, int cus, std::vector<v4i> *lists, int *per_wg_out)
+try {
+    std::vector<std::vector<Tile>> q;
+    const int64_t longest = deal_tiles<BM, BN>(mnk, n, cus, &q);
+    if (longest < 0) return longest;
     const int per_wg = (int)longest + 1;
     if (per_wg_out) *per_wg_out = per_wg;
     if (lists) {
@@ -629,7 +641,8 @@ using LC = Cfg;
 struct Split {
     int n_tiled = 0, n_deep = 0;
     int tiled[MAX_PROBLEMS], deep[MAX_PROBLEMS];
-    int which = 0;   // tile of the second launch
+    int which = 0;         // tile of the second launch
+    bool stream = false;   // the list is of 256 x 128 tiles, for the kernel of gemm_stream.hip
 };
 
 // the longest workgroup of a list, in tile costs and in tiles: blocks of equal K dealt longest first to the least loaded
@@ -637,7 +650,7 @@ struct Split {
 struct Load {
     int64_t cost, tiles;
 };
-static Load list_load(const int64_t *mnk, const int *idx, int n, int cus)
+static Load list_load(const int64_t *mnk, const int *idx, int n, int cus, int bn = LC::BN)
 {
     const int nx = (cus % 8 == 0) ? 8 : 1, slots = cus / nx;
     int64_t load[8] = {}, blocks[8] = {};
@@ -645,7 +658,7 @@ static Load list_load(const int64_t *mnk, const int *idx, int n, int cus)
         const int64_t K = mnk[3 * idx[i] + 2];
         int64_t tiles = 0;
         for (; i < n && mnk[3 * idx[i] + 2] == K; ++i)
-            tiles += ((mnk[3 * idx[i]] + LC::BM - 1) / LC::BM) * ((mnk[3 * idx[i] + 1] + LC::BN - 1) / LC::BN);
+            tiles += ((mnk[3 * idx[i]] + LC::BM - 1) / LC::BM) * ((mnk[3 * idx[i] + 1] + bn - 1) / bn);
         for (; tiles > 0; tiles -= slots) {
             const int x = (int)(std::min_element(load, load + nx) - load);
             load[x] += tile_cost(K);
@@ -654,6 +667,18 @@ static Load list_load(const int64_t *mnk, const int *idx, int n, int cus)
     }
     return {*std::max_element(load, load + nx), *std::max_element(blocks, blocks + nx)};
 }
+
+// The list in 256 x 128 tiles (gemm_stream.hip): 0.84 us a unit of tile cost and 4 us beside that at best, 0.88 to 0.95 with
+// weights from HBM; taken as 1.0, for what the other estimates are good to (at 0.95 five problems with 419 rows went over and
+// took 159 instead of 146 us).  Half as large, its tiles level out where the others do not: the four projections with 509 rows
+// 142 -> 118 us, 8608 and 6144 columns of 503 rows, K = 8704, 97 -> 80, 6192 columns of 1241 rows, K = 6272, 66 -> 56.  With many
+// rounds the large tiles are 1.2 times as fast (2048 rows 355 against 419 us).  Of 120 drawn batches nine go over, 0.83 to 0.96 of
+// the time before.  From eight stages a tile on; shorter ones stay where they were (nine such batches: 0.76 to 0.92 of their time).
+constexpr int64_t STREAM_MIN_K = 1024;
+
+// bytes of the lists of workgroups with at most this many tiles
+static int64_t list_bytes(int cus, int64_t tiles) { return cus * (tiles + 1) * (int64_t)sizeof(v4i); }
+static int64_t stream_bytes(int cus, int64_t tiles) { return cus * (tiles + 1) * (int64_t)sizeof(v2i); }
 
 static Split split_batch(const int64_t *mnk, int n, int cus)
 {
@@ -676,7 +701,7 @@ static Split split_batch(const int64_t *mnk, int n, int cus)
     if ((double)whole.cost * cus < 1.2 * sum || tiles > 8.0 * cus) return best;
     // the estimates are good to a tenth: what they promise has to be more
     float t_best = 0.9f * (3.0f + 1.36f * (float)whole.cost);
-    for (int mask = 1; mask < (1 << n); ++mask) {   // the problems of the second launch
+    for (int mask = 0; mask < (1 << n); ++mask) {   // the problems of the second launch
         Split s;
         for (int i = 0; i < n; ++i) {
             if (mask >> i & 1) s.deep[s.n_deep++] = order[i];
@@ -691,11 +716,19 @@ static Split split_batch(const int64_t *mnk, int n, int cus)
         // without the long tiles the short ones can be dealt to fewer XCDs, more of them to a workgroup than in the whole
         // list: such a list would not fit the memory that the whole one is given
         if (part.tiles > whole.tiles) continue;
-        float t = deep_batch_estimate(mnk, s.deep, s.n_deep, cus, &s.which);
-        if (s.n_tiled) t += 5.0f + 1.36f * (float)part.cost;
-        if (t < t_best) {
-            t_best = t;
+        const float t = s.n_deep ? deep_batch_estimate(mnk, s.deep, s.n_deep, cus, &s.which) : 0.0f;
+        const float t_list = t + (s.n_tiled ? 5.0f + 1.36f * (float)part.cost : 0.0f);
+        if (s.n_deep && t_list < t_best) {
+            t_best = t_list;
             best = s;
+        }
+        if (!s.n_tiled || mnk[3 * s.tiled[s.n_tiled - 1] + 2] < STREAM_MIN_K) continue;   // (the last has the shortest K)
+        const Load narrow = list_load(mnk, s.tiled, s.n_tiled, cus, STREAM_BN);
+        const float t_stream = t + (s.n_deep ? 6.0f : 4.0f) + 1.0f * (float)narrow.cost;
+        if (t_stream < t_best && stream_bytes(cus, narrow.tiles) <= list_bytes(cus, whole.tiles)) {
+            t_best = t_stream;
+            best = s;
+            best.stream = true;
         }
     }
     return best;
@@ -708,7 +741,7 @@ try {
     const int64_t whole = build_lists<LC::BM, LC::BN>(mnk, n, cus, lists, per_wg);
     if (whole < 0) return whole;
     *split = split_batch(mnk, n, cus);
-    if (!split->n_deep) {
+    if (!split->n_deep && !split->stream) {
         for (int i = 0; i < n; ++i) split->tiled[i] = i;
         return whole;
     }
@@ -716,7 +749,20 @@ try {
     int64_t sub[3 * MAX_PROBLEMS];
     for (int i = 0; i < split->n_tiled; ++i)
         for (int k = 0; k < 3; ++k) sub[3 * i + k] = mnk[3 * split->tiled[i] + k];
-    return build_lists<LC::BM, LC::BN>(sub, split->n_tiled, cus, lists, per_wg);
+    if (!split->stream) return build_lists<LC::BM, LC::BN>(sub, split->n_tiled, cus, lists, per_wg);
+    std::vector<std::vector<Tile>> q;
+    const int64_t longest = deal_tiles<LC::BM, STREAM_BN>(sub, split->n_tiled, cus, &q);
+    if (longest < 0) return longest;
+    const int64_t bytes = stream_bytes(cus, longest);
+    *per_wg = (int)longest + 1;
+    lists->assign((size_t)(bytes + (int64_t)sizeof(v4i) - 1) / sizeof(v4i), (v4i){-1, -1, -1, -1});
+    v2i *const to = reinterpret_cast<v2i *>(lists->data());
+    for (int w = 0; w < cus; ++w)
+        for (size_t i = 0; i < q[(size_t)w].size(); ++i) {
+            const Tile &t = q[(size_t)w][i];
+            to[(size_t)w * *per_wg + i] = (v2i){t.m0, t.n0 | t.p};   // (columns come in sixteens)
+        }
+    return bytes;
 } catch (const std::bad_alloc &) {
     return MI_ENOMEM;
 }
@@ -850,6 +896,14 @@ static int32_t batch_run(mi_gemm_batch *b, const mi_gemm_problem *p, void *strea
         }
         const int32_t rc = launch_deep_batch<DEQ>(sp.which, d, sp.n_deep, as_stream(stream));
         if (rc || !sp.n_tiled) return rc;
+    }
+    if (sp.stream) {
+        StreamBatch sb = {};
+        for (int i = 0; i < sp.n_tiled; ++i) {
+            const mi_gemm_problem &g = p[sp.tiled[i]];
+            sb.p[i] = {g.qx, g.qw, g.sx, g.sw, g.out, (int)g.M, (int)g.N, (int)g.K, 0};
+        }
+        return launch_stream<DEQ>(sb, reinterpret_cast<const v2i *>(b->lists), b->grid, b->per_wg, as_stream(stream));
     }
     list::Batch bt = {};
     for (int i = 0; i < sp.n_tiled; ++i) {

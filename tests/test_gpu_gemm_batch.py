@@ -264,6 +264,27 @@ def test_batch_by_route(mi, dev, orc, shapes, small, tile):
     check_batch(mi, dev, orc, shapes, 501 + shapes[0][0])
 
 
+@pytest.mark.parametrize("shapes", [
+    [(783, 5008, 1664)],                                              # one tile a workgroup, moved inwards in rows and columns
+    [(797, 2800, 1536), (257, 5808, 1536), (257, 2208, 1152)],
+    [(595, 11088, 1024), (595, 8896, 1152)],                          # two: 8 and 9 stages, which end in either set of fragments
+    [(400, 1728, 4096), (400, 6928, 1664), (400, 12560, 1152), (400, 4464, 1664)],
+    [(400, 9008, 4096), (400, 5520, 1024), (400, 2000, 7168), (473, 12944, 1664)],   # up to three
+    [(405, 5664, 1152), (400, 4800, 1152), (400, 7648, 4096)],        # the longest in small tiles
+])
+def test_batch_in_narrow_tiles(mi, dev, orc, shapes):
+    """Batches whose list is of 256 x 128 tiles: its entries take half the bytes of the other list's."""
+    import ctypes as C
+    mnk = (C.c_int64 * (3 * len(shapes)))(*[v for s in shapes for v in s])
+    small, tile, per_wg = np.zeros(len(shapes), np.int32), np.zeros(2, np.int32), C.c_int32()
+    stored = mi.lib.mi_gemm_batch_split_host(mnk, len(shapes), 256, small.ctypes.data, tile.ctypes.data)
+    rest = [s for s, x in zip(shapes, small) if not x]
+    mnk = (C.c_int64 * (3 * len(rest)))(*[v for s in rest for v in s])
+    buf = np.empty(1 << 20, np.uint8)
+    assert 0 < stored != mi.lib.mi_gemm_batch_plan_host(mnk, len(rest), 256, buf.ctypes.data, buf.nbytes, C.byref(per_wg))
+    check_batch(mi, dev, orc, shapes, 601 + shapes[0][0])
+
+
 def test_random_batches_by_route_equal_the_oracle(mi, dev, orc):
     """Seeded random ragged batches until there are three of each kind: all in the list, all in small tiles, some in either."""
     rng = np.random.default_rng(20251203)
