@@ -509,6 +509,12 @@ MI_API int32_t mi_rmsnorm_linear_f32(const float *x, const float *residual, cons
                                      float *h_out, float *xn_out, const int8_t *qw, const float *sw, float *y,
                                      int64_t M, int64_t N, int64_t K, int32_t block,
                                      void *workspace, int64_t workspace_bytes, void *stream);
+/* SwiGLU + rotate + quantize + W8A8 contraction + dequant as one call: y = linear(swiglu(gate_up)), I the contraction length.
+ * q int8 [M,I], scale fp32 [M] and h_out (optional) as in mi_swiglu_quant_f32_i8, qw int8 [N,I], sw fp32 [N], y fp32 [M,N].
+ * For one token and I in {2048, 4096, 14336} (block 128) it is ONE kernel; any other shape, and outputs that overlap gate_up,
+ * run mi_swiglu_quant_f32_i8 and the contraction.  The same bits either way. */
+MI_API int32_t mi_swiglu_linear_f32(const float *gate_up, float *h_out, int8_t *q, float *scale, const int8_t *qw,
+                                    const float *sw, float *y, int64_t M, int64_t N, int64_t I, int32_t block, void *stream);
 /* out = a + b over n floats (n % 4 == 0): the residual add that closes the layer. */
 MI_API int32_t mi_add_f32(const float *a, const float *b, float *out, int64_t n, void *stream);
 

@@ -21,6 +21,8 @@ int32_t launch_linear_fused(const float *, const int8_t *, const float *, float 
                             int64_t, hipStream_t, bool);
 int32_t launch_norm_linear_fused(const float *, const float *, const float *, float, float *, float *, const int8_t *,
                                  const float *, float *, int8_t *, float *, int64_t, int64_t, int64_t, hipStream_t);
+int32_t launch_swiglu_linear_fused(const float *, float *, const int8_t *, const float *, float *, int8_t *, float *, int64_t,
+                                   int64_t, int64_t, hipStream_t);
 
 __global__ void k_dequant(const int32_t *__restrict__ acc, const float *__restrict__ sx,
                           const float *__restrict__ sw, float *__restrict__ y, int64_t M, int64_t N)
@@ -159,6 +161,25 @@ extern "C" int32_t mi_rmsnorm_linear_f32(const float *x, const float *residual, 
     return gemm_dispatch(qx, sx, qw, sw, nullptr, y, M, N, K, as_stream(stream));
 }
 
+extern "C" int32_t mi_swiglu_linear_f32(const float *gate_up, float *h_out, int8_t *q, float *scale, const int8_t *qw,
+                                        const float *sw, float *y, int64_t M, int64_t N, int64_t I, int32_t block, void *stream)
+{
+    int32_t rc = check_gemm(q, qw, y, M, N, I);
+    if (rc) return rc;
+    if (!gate_up || !scale || !sw || !aligned16(gate_up) || !aligned4(scale) || !aligned16(sw) || (h_out && !aligned16(h_out)))
+        return MI_EINVAL;
+    // (the one-kernel form reads gate_up in every workgroup while others write)
+    const int64_t row = 2 * I * 4;
+    if (M == 1 && block == 128 && !overlaps(gate_up, row, h_out, I * 4) && !overlaps(gate_up, row, q, I) &&
+        !overlaps(gate_up, row, scale, 4) && !overlaps(gate_up, row, y, N * 4)) {
+        rc = launch_swiglu_linear_fused(gate_up, h_out, qw, sw, y, q, scale, M, N, I, as_stream(stream));
+        if (rc != MI_EINVAL) return rc;
+    }
+    rc = mi_swiglu_quant_f32_i8(gate_up, h_out, q, scale, M, I, block, stream);
+    if (rc) return rc;
+    return gemm_dispatch(q, scale, qw, sw, nullptr, y, M, N, I, as_stream(stream));
+}
+
 // The linear once its activation codes (qx) and scales (sx) have a home: the caller's workspace or the static array.
 static int32_t linear_with(const float *x, const int8_t *qw, const float *sw, float *y, int64_t M, int64_t N,
                            int64_t K, int32_t block, int8_t *qx, float *sx, void *stream)
@@ -166,8 +187,9 @@ static int32_t linear_with(const float *x, const int8_t *qw, const float *sw, fl
     int32_t rc = check_gemm(qx, qw, y, M, N, K);
     if (rc) return rc;
     if (!x || !sw || !aligned16(sw)) return MI_EINVAL;
-    if (M == 1 && block == 128 && aligned16(x)) {
-        // decode: one kernel that quantizes its own activations (MI_EINVAL = shape not covered)
+    if (M == 1 && block == 128 && aligned16(x) && !overlaps(x, K * 4, y, N * 4) && !overlaps(x, K * 4, qx, K)) {
+        // decode: one kernel that quantizes its own activations (MI_EINVAL = shape not covered); every workgroup reads the
+        // whole of x while others write
         rc = launch_linear_fused(x, qw, sw, y, qx, sx, M, N, K, as_stream(stream), true);
         if (rc != MI_EINVAL) return rc;
     }

@@ -6,8 +6,8 @@
 //  k_gemv_reg: a lane always works on the same byte offsets of a weight row, so its share of the activation codes
 //  lives in registers for the whole kernel: no LDS and no barrier in the streaming part, 16 x 1 KB weight loads in
 //  flight per wave, v_dot4_i32_i8, one transposed butterfly per wave.
-//  k_gemv_fused is the same kernel with the rotate + quantize prologue (and optionally the RMSNorm) inside, for
-//  one token and K <= 4096.
+//  k_gemv_row makes the codes of its one token itself (rotate + quantize, with RMSNorm or SwiGLU in front), for K of
+//  2048, 4096 and 14336.
 #include <algorithm>
 #include "common.h"
 #include "fwht_core.h"
@@ -115,153 +115,161 @@ __global__ __launch_bounds__(64 * WG) void k_gemv_reg(const int8_t *__restrict__
     }
 }
 
-// k_gemv_fused: k_gemv_reg with the rotate + quantize prologue inside.  The row's own loads go out first and the
-// first group's weight loads right behind them; while the weights are in flight the workgroup rotates and quantizes
-// the activation row (the same per-chunk code as the stand-alone quantizer, so the codes and scales are
-// bit-identical), parks the codes in LDS and every lane picks up its share.  One launch per linear instead of two.
-// ROT = false: the row arrives in the rotated basis and is only quantized.
-// NORM: the row is first normalized, v = ((x (+ res)) * r) * g with r = 1 / sqrt(mean((x + res)^2) + eps), the
-// arithmetic of the stand-alone RMSNorm + quantize kernel; workgroup 0 also leaves the residual sum (h_out) and, on
-// request, the normalized row (xn_out) for the caller.
-struct FusedNorm {
+// k_gemv_row: the GEMV of one token with what makes its codes inside, one launch instead of two.  One workgroup of eight
+// waves per compute unit (more where the rows are many); the rows of the weights are dealt evenly to the waves of the chip, and
+// a wave keeps two groups of R rows in flight: the row's own loads go out first (loads return in the order they were issued),
+// the first two groups right behind them (where the rows are few that is all the weights there are), and while they are on
+// their way the workgroup makes the codes, with the same arithmetic as the stand-alone kernels, so that codes and scales are the
+// same bits, parks them in LDS, and every lane picks up its share.  Every load is unconditional: behind a branch the compiler
+// no longer counts them and waits for the weights before it touches the row.
+// Bound: HBM, beside about 3 us from launch to first byte.  us, in workgroups of four waves that took 16 rows at a time and
+// (K = 14336) two launches -> here: 6144 x 4096 9.4 -> 7.9, with the norm 10.7 -> 9.1; 4096 x 4096 7.2 -> 5.7; 4096 x 14336
+// 19.6 -> 16.2, with SwiGLU 20.4 -> 17.8; 4096 x 2048 5.4 -> 4.1; 28672 x 4096 with the norm 25.3 -> 25.2.
+//   ROT: rotate + quantize; PLAIN: the row arrives in the rotated basis and is only quantized;
+//   NORM: v = ((x (+ res)) * r) * g with r = 1 / sqrt(mean((x + res)^2) + eps), then rotate + quantize; workgroup 0 also leaves
+//   the residual sum (h_out) and, on request, the normalized row (xn_out);
+//   SWIGLU: v = silu(gate) * up of a row [gate | up], then rotate + quantize; workgroup 0 leaves v in xn_out on request.
+// Workgroup 0 leaves codes and scale for the caller.
+enum RowOp { ROT, PLAIN, NORM, SWIGLU };
+struct RowArgs {
     const float *res, *g;
     float *h_out, *xn_out;
     float eps;
 };
 
-template <int CW, int CQ, bool NORM, bool ROT>
-__global__ __launch_bounds__(256) void k_gemv_fused(const float *__restrict__ x, const int8_t *__restrict__ qw,
-                                                    const float *__restrict__ sw, float *__restrict__ y,
-                                                    int8_t *__restrict__ qx_out, float *__restrict__ sx_out, int N,
-                                                    int K, FusedNorm nm)
+template <int CW, int CQ, int R, RowOp OP>
+__global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x, const int8_t *__restrict__ qw,
+                                                     const float *__restrict__ sw, float *__restrict__ y,
+                                                     int8_t *__restrict__ qx_out, float *__restrict__ sx_out, int N, int K,
+                                                     RowArgs ra)
 {
-    constexpr int BLOCK = 128, LPB = BLOCK / 8;
-    constexpr int R = (16 / CW) < 1 ? 1 : (16 / CW);   // rows per wave
+    constexpr int BLOCK = 128, LPB = BLOCK / 8, WG = 8;
     constexpr int V = pow2_ceil(R);
-    extern __shared__ __attribute__((aligned(16))) char s_dyn[];
-    int8_t *s_x = reinterpret_cast<int8_t *>(s_dyn);            // [K] codes
-    float *s_max = reinterpret_cast<float *>(s_dyn + K);        // [4] row maxima, then [4 * CQ] sums of squares
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    constexpr int rows_per_wg = 4 * R;
-    // the workgroup owns a run of consecutive groups of rows_per_wg weight rows (the groups dealt out evenly over
-    // the grid): one prologue serves them all
-    const int ngroups = (N + rows_per_wg - 1) / rows_per_wg;
-    const int g0 = (int)((int64_t)ngroups * blockIdx.x / gridDim.x);
-    const int g1 = (int)((int64_t)ngroups * (blockIdx.x + 1) / gridDim.x);
+    __shared__ __attribute__((aligned(16))) int8_t s_x[CW * 1024];   // codes
+    __shared__ float s_max[WG], s_sum[WG * CQ];                      // row maxima, sums of squares
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int waves = gridDim.x * WG, id = blockIdx.x * WG + wave;
+    const int row0 = (int)((int64_t)N * id / waves), row1 = (int)((int64_t)N * (id + 1) / waves);
     const int kbase = lane * 16;
-
-    auto load_w = [&](v4i (&w)[R][CW], int g) {
-        const int row0 = g * rows_per_wg + wave * R;
+    // (no branch around a load: the compiler would wait for all of them where it cannot count them.  Past the wave's rows the
+    // last one is fetched again)
+    auto load_w = [&](v4i (&w)[R][CW], int row) {
 #pragma unroll
-        for (int r = 0; r < R; ++r)
+        for (int r = 0; r < R; ++r) {
+            const int8_t *const p = qw + (int64_t)min(row + r, max(row1 - 1, 0)) * K + kbase;
 #pragma unroll
-            for (int c = 0; c < CW; ++c) {
-                const int off = kbase + c * 1024;
-                w[r][c] = (row0 + r < N && off < K) ? *reinterpret_cast<const v4i *>(qw + (int64_t)(row0 + r) * K + off)
-                                                    : (v4i){0, 0, 0, 0};
-            }
+            for (int c = 0; c < CW; ++c) w[r][c] = *reinterpret_cast<const v4i *>(p + c * 1024);
+        }
     };
-    // Loads return in the order they were issued: the first row's own loads (activations, residual, gain) go out
-    // BEFORE the first group's weights, so that the prologue's arithmetic runs while the weights are on their way
-    // (issued behind them, the row would arrive only after 64 KB of weights per workgroup, and nothing would be in
-    // flight while the prologue computes).
-    v4i w[R][CW];
 
-    // rotate + quantize: thread t owns chunks t, t + 256, ... of the row
-    const int j = tid % LPB;
-    const int nchunk = K / 8;
+    // thread t owns chunks t, t + 512, ... of the row, in the layout of fwht_core.h
+    const int j = tid % LPB, nchunk = K / 8;
+    const bool keeper = blockIdx.x == 0;
     float v[CQ][8];
     int base[CQ];
+    float4 gl[CQ], gh[CQ], rl[CQ], rh[CQ];
 #pragma unroll
     for (int i = 0; i < CQ; ++i) {
-        const int c = tid + i * 256;
+        const int c = tid + i * 512;
         base[i] = (c / LPB) * BLOCK + 4 * j;
         if (c < nchunk) {
             const float4 lo = *reinterpret_cast<const float4 *>(x + base[i]);
             const float4 hi = *reinterpret_cast<const float4 *>(x + base[i] + BLOCK / 2);
             v[i][0] = lo.x; v[i][1] = lo.y; v[i][2] = lo.z; v[i][3] = lo.w;
             v[i][4] = hi.x; v[i][5] = hi.y; v[i][6] = hi.z; v[i][7] = hi.w;
+            if constexpr (OP == NORM) {
+                gl[i] = *reinterpret_cast<const float4 *>(ra.g + base[i]);
+                gh[i] = *reinterpret_cast<const float4 *>(ra.g + base[i] + BLOCK / 2);
+                if (ra.res) {
+                    rl[i] = *reinterpret_cast<const float4 *>(ra.res + base[i]);
+                    rh[i] = *reinterpret_cast<const float4 *>(ra.res + base[i] + BLOCK / 2);
+                }
+            }
+            if constexpr (OP == SWIGLU) {
+                gl[i] = *reinterpret_cast<const float4 *>(x + K + base[i]);
+                gh[i] = *reinterpret_cast<const float4 *>(x + K + base[i] + BLOCK / 2);
+            }
         } else {
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[i][e] = 0.0f;
         }
     }
-    const bool keeper = blockIdx.x == 0;   // one workgroup also leaves the codes and scales in the caller's workspace
-    if constexpr (!NORM) load_w(w, g0);
-    if constexpr (NORM) {
-        float4 gl[CQ], gh[CQ], rl_[CQ], rh_[CQ];
-        float ss[CQ];   // per chunk, then per group of 64 chunks (group wave + 4 * i): the order of fwht_core.h
+    v4i wa[R][CW], wb[R][CW];
+    load_w(wa, row0);
+    load_w(wb, row0 + R);
+
+    auto leave = [&](float *to) {   // the row as it stands
 #pragma unroll
-        for (int i = 0; i < CQ; ++i) {
-            if (tid + i * 256 < nchunk) {
-                gl[i] = *reinterpret_cast<const float4 *>(nm.g + base[i]);
-                gh[i] = *reinterpret_cast<const float4 *>(nm.g + base[i] + BLOCK / 2);
-                if (nm.res) {
-                    const float *rr = nm.res + base[i];
-                    rl_[i] = *reinterpret_cast<const float4 *>(rr);
-                    rh_[i] = *reinterpret_cast<const float4 *>(rr + BLOCK / 2);
-                }
+        for (int i = 0; i < CQ; ++i)
+            if (tid + i * 512 < nchunk) {
+                *reinterpret_cast<float4 *>(to + base[i]) = make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
+                *reinterpret_cast<float4 *>(to + base[i] + BLOCK / 2) = make_float4(v[i][4], v[i][5], v[i][6], v[i][7]);
             }
-        }
-        load_w(w, g0);
+    };
+    if constexpr (OP == NORM) {
+        float ss[CQ];   // per chunk, then per group of 64 chunks (group wave + 8 i): the order of fwht_core.h
 #pragma unroll
         for (int i = 0; i < CQ; ++i) {
             ss[i] = 0.0f;
-            if (tid + i * 256 < nchunk) {
-                if (nm.res) {
-                    const float4 rl = rl_[i], rh = rh_[i];
-                    v[i][0] = v[i][0] + rl.x; v[i][1] = v[i][1] + rl.y; v[i][2] = v[i][2] + rl.z; v[i][3] = v[i][3] + rl.w;
-                    v[i][4] = v[i][4] + rh.x; v[i][5] = v[i][5] + rh.y; v[i][6] = v[i][6] + rh.z; v[i][7] = v[i][7] + rh.w;
-                    if (keeper) {
-                        float *ho = nm.h_out + base[i];
-                        *reinterpret_cast<float4 *>(ho) = make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
-                        *reinterpret_cast<float4 *>(ho + BLOCK / 2) = make_float4(v[i][4], v[i][5], v[i][6], v[i][7]);
-                    }
+            if (tid + i * 512 < nchunk) {
+                if (ra.res) {
+                    v[i][0] = v[i][0] + rl[i].x; v[i][1] = v[i][1] + rl[i].y; v[i][2] = v[i][2] + rl[i].z; v[i][3] = v[i][3] + rl[i].w;
+                    v[i][4] = v[i][4] + rh[i].x; v[i][5] = v[i][5] + rh[i].y; v[i][6] = v[i][6] + rh[i].z; v[i][7] = v[i][7] + rh[i].w;
                 }
                 ss[i] = chunk_sumsq(v[i]);
             }
         }
-#pragma unroll
-        for (int i = 0; i < CQ; ++i) ss[i] = group_sum(ss[i]);
-        if (lane == 0) {
-#pragma unroll
-            for (int i = 0; i < CQ; ++i) s_max[4 + wave + 4 * i] = ss[i];
-        }
-        __syncthreads();
-        const float total = tree_sum<4 * CQ>(s_max + 4);
-        const float r = 1.0f / sqrtf(total / (float)K + nm.eps);
+        if (ra.res && keeper) leave(ra.h_out);
 #pragma unroll
         for (int i = 0; i < CQ; ++i) {
-            if (tid + i * 256 < nchunk) {
+            ss[i] = group_sum(ss[i]);
+            if (lane == 0) s_sum[wave + WG * i] = ss[i];
+        }
+        __syncthreads();
+        const float total = tree_sum<WG * CQ>(s_sum);
+        const float r = 1.0f / sqrtf(total / (float)K + ra.eps);
+#pragma unroll
+        for (int i = 0; i < CQ; ++i)
+            if (tid + i * 512 < nchunk) {
                 v[i][0] = (v[i][0] * r) * gl[i].x; v[i][1] = (v[i][1] * r) * gl[i].y;
                 v[i][2] = (v[i][2] * r) * gl[i].z; v[i][3] = (v[i][3] * r) * gl[i].w;
                 v[i][4] = (v[i][4] * r) * gh[i].x; v[i][5] = (v[i][5] * r) * gh[i].y;
                 v[i][6] = (v[i][6] * r) * gh[i].z; v[i][7] = (v[i][7] * r) * gh[i].w;
-                if (keeper && nm.xn_out) {
-                    float *xo = nm.xn_out + base[i];
-                    *reinterpret_cast<float4 *>(xo) = make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
-                    *reinterpret_cast<float4 *>(xo + BLOCK / 2) = make_float4(v[i][4], v[i][5], v[i][6], v[i][7]);
-                }
+            }
+    }
+    if constexpr (OP == SWIGLU) {
+#pragma unroll
+        for (int i = 0; i < CQ; ++i) {
+            const float up[8] = {gl[i].x, gl[i].y, gl[i].z, gl[i].w, gh[i].x, gh[i].y, gh[i].z, gh[i].w};
+            if (tid + i * 512 < nchunk) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[i][e] = (v[i][e] / (1.0f + expf(-v[i][e]))) * up[e];
             }
         }
+    }
+    if constexpr (OP == NORM || OP == SWIGLU) {
+        if (keeper && ra.xn_out) leave(ra.xn_out);
     }
     float amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < CQ; ++i) {
-        if constexpr (ROT) fwht_chunk<BLOCK>(v[i], j);   // !ROT: the row arrives in the rotated basis
+        if constexpr (OP != PLAIN) fwht_chunk<BLOCK>(v[i], j);
         amax = fmaxf(amax, abs8(v[i]));
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
     if (lane == 0) s_max[wave] = amax;
     __syncthreads();
-    const float a = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
+    float a = s_max[0];
+#pragma unroll
+    for (int w = 1; w < WG; ++w) a = fmaxf(a, s_max[w]);
     const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
     const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
     if (keeper && tid == 0) *sx_out = sc;
 #pragma unroll
-    for (int i = 0; i < CQ; ++i) {
-        if (tid + i * 256 < nchunk) {
+    for (int i = 0; i < CQ; ++i)
+        if (tid + i * 512 < nchunk) {
             const uint32_t c0 = quant4(v[i][0], v[i][1], v[i][2], v[i][3], inv);
             const uint32_t c1 = quant4(v[i][4], v[i][5], v[i][6], v[i][7], inv);
             *reinterpret_cast<uint32_t *>(s_x + base[i]) = c0;
@@ -271,101 +279,97 @@ __global__ __launch_bounds__(256) void k_gemv_fused(const float *__restrict__ x,
                 *reinterpret_cast<uint32_t *>(qx_out + base[i] + BLOCK / 2) = c1;
             }
         }
-    }
     __syncthreads();
 
     v4i xr[CW];
 #pragma unroll
-    for (int c = 0; c < CW; ++c) {
-        const int off = kbase + c * 1024;
-        xr[c] = off < K ? *reinterpret_cast<const v4i *>(s_x + off) : (v4i){0, 0, 0, 0};
-    }
+    for (int c = 0; c < CW; ++c) xr[c] = *reinterpret_cast<const v4i *>(s_x + kbase + c * 1024);
     constexpr int SH = 6 - __builtin_ctz(V);
     const int vi = lane >> SH;
-    const bool speaker = (lane & ((1 << SH) - 1)) == 0;
-#pragma unroll 1
-    for (int g = g0; g < g1; ++g) {
-        // the next group's weight loads go out before this group's arithmetic
-        v4i wn[R][CW];
-        const bool more = g + 1 < g1;   // the same for every thread of the workgroup
-        if (more) load_w(wn, g + 1);
+    const bool speaker = (lane & ((1 << SH) - 1)) == 0 && vi < R;
+    auto rows = [&](v4i (&w)[R][CW], int row) {
         int p[V];
 #pragma unroll
         for (int i = 0; i < V; ++i) p[i] = 0;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            int a = 0;
+            int d = 0;
 #pragma unroll
-            for (int c = 0; c < CW; ++c) {
-                a = __builtin_amdgcn_sdot4(w[r][c][0], xr[c][0], a, false);
-                a = __builtin_amdgcn_sdot4(w[r][c][1], xr[c][1], a, false);
-                a = __builtin_amdgcn_sdot4(w[r][c][2], xr[c][2], a, false);
-                a = __builtin_amdgcn_sdot4(w[r][c][3], xr[c][3], a, false);
-            }
-            p[r] = a;
+            for (int c = 0; c < CW; ++c)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) d = __builtin_amdgcn_sdot4(w[r][c][q], xr[c][q], d, false);
+            p[r] = d;
         }
         fold_sum<V, 32>(p, lane);
-        const int n = g * rows_per_wg + wave * R + vi;
-        if (speaker && vi < R && n < N) y[n] = ((float)p[0] * sc) * sw[n];
-        if (more) {
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-#pragma unroll
-                for (int c = 0; c < CW; ++c) w[r][c] = wn[r][c];
-        }
+        if (speaker && row + vi < row1) y[row + vi] = ((float)p[0] * sc) * sw[row + vi];
+    };
+    int row = row0;
+#pragma unroll 1
+    for (; row + 2 * R < row1; row += 2 * R) {
+        rows(wa, row);
+        load_w(wa, row + 2 * R);
+        rows(wb, row + R);
+        load_w(wb, row + 3 * R);
     }
+    rows(wa, row);
+    if (row + R < row1) rows(wb, row + R);
 }
 
-template <int CW, int CQ, bool NORM, bool ROT = true>
-static int32_t launch_fused(const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx, int N, int K,
-                            const FusedNorm &nm, hipStream_t s)
+template <RowOp OP>
+static int32_t launch_row(const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx, int64_t N,
+                          int64_t K, const RowArgs &ra, hipStream_t s)
 {
-    constexpr int R = (16 / CW) < 1 ? 1 : (16 / CW);
-    const size_t lds = (size_t)K + (4 + 4 * CQ) * sizeof(float);   // at most 4,144 bytes
-    // Every workgroup reads the whole activation row (with the norm: the residual and the gain too, 48 KB at
-    // K = 4096) before its first dot product.  Beyond two workgroups per compute unit a workgroup therefore takes
-    // several groups of rows in turn, the next group's weights on their way while it works on the current one.
-    constexpr int rows_per_wg = 4 * R;
-    const int ngroups = (N + rows_per_wg - 1) / rows_per_wg;
-    const unsigned grid = (unsigned)std::min(ngroups, 2 * compute_units());   // three per unit measured the same
-    hipLaunchKernelGGL((k_gemv_fused<CW, CQ, NORM, ROT>), dim3(grid), dim3(256), lds, s, x, qw, sw, y, qx, sx, N, K, nm);
+    const int cus = compute_units(), per_wave = (int)((N + 8 * cus - 1) / (8 * cus));
+#define MI_ROW(CW_, CQ_, R_, WGS_)                                                                                              \
+    hipLaunchKernelGGL((k_gemv_row<CW_, CQ_, R_, OP>), dim3((unsigned)(WGS_) * cus), dim3(512), 0, s, x, qw, sw, y, qx, sx, (int)N, \
+                       (int)K, ra)
+    // Few rows: one workgroup a unit whose two groups cover them.  Many: two a unit with a row at a time (20000 x 4096 and the
+    // norm 18.0 us, one a unit with four rows at a time 19.9), three where the codes are quickly made (28672 x 4096 24.9 against
+    // 25.9 us; with the norm 25.9 against 25.2).  14336 floats a row: one a unit is what the registers hold, and with more than
+    // eight rows a wave the two launches are level (20000 rows 58.7 against 58.5 us, 28672 79.2 against 80.9).
+    if (K == 4096) {
+        if (per_wave <= 2) MI_ROW(4, 1, 1, 1);
+        else if (per_wave <= 4) MI_ROW(4, 1, 2, 1);
+        else if (per_wave <= 10 || OP == NORM) MI_ROW(4, 1, 1, 2);
+        else MI_ROW(4, 1, 1, 3);
+    } else if (K == 2048) {
+        if (per_wave <= 2) MI_ROW(2, 1, 1, 1);
+        else if (per_wave <= 4) MI_ROW(2, 1, 2, 1);
+        else if (per_wave <= 8) MI_ROW(2, 1, 4, 1);
+        else MI_ROW(2, 1, 1, 2);
+    } else {
+        if constexpr (OP == ROT || OP == SWIGLU) {
+            if (K != 14336 || per_wave > 8) return MI_EINVAL;
+            MI_ROW(14, 4, 1, 1);
+        } else {
+            return MI_EINVAL;
+        }
+    }
+#undef MI_ROW
     return launch_status();
 }
 
-// The fused decode linear is taken for one token and K <= 4096 only (MI_EINVAL tells the caller to take the
-// two-kernel path).  Measured: 9.3 against 10.6 us for 4096 -> 6144 at M = 1, but every workgroup repeats the
-// quantization, which at M = 4 or K = 14336 costs more than the launch it saves (15.6 against 11.7 us, 20.8
-// against 18.8 us).  rotate = false: x is already in the rotated basis (the attention output as the merge leaves
-// it) and is only quantized.
 int32_t launch_linear_fused(const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx,
-                            int64_t M64, int64_t N64, int64_t K64, hipStream_t s, bool rotate)
+                            int64_t M, int64_t N, int64_t K, hipStream_t s, bool rotate)
 {
-    const int N = (int)N64, K = (int)K64;
-    if (M64 != 1 || K % 1024) return MI_EINVAL;
-    const int nchunk = K >> 10;
-    const FusedNorm none = {nullptr, nullptr, nullptr, nullptr, 0.0f};
-    if (rotate) {
-        if (nchunk == 4) return launch_fused<4, 2, false>(x, qw, sw, y, qx, sx, N, K, none, s);   // K = 4096
-        if (nchunk == 2) return launch_fused<2, 1, false>(x, qw, sw, y, qx, sx, N, K, none, s);   // K = 2048
-    } else {
-        if (nchunk == 4) return launch_fused<4, 2, false, false>(x, qw, sw, y, qx, sx, N, K, none, s);
-        if (nchunk == 2) return launch_fused<2, 1, false, false>(x, qw, sw, y, qx, sx, N, K, none, s);
-    }
-    return MI_EINVAL;
+    if (M != 1) return MI_EINVAL;
+    const RowArgs none = {};
+    return rotate ? launch_row<ROT>(x, qw, sw, y, qx, sx, N, K, none, s) : launch_row<PLAIN>(x, qw, sw, y, qx, sx, N, K, none, s);
 }
 
-// The same with the (residual +) RMSNorm ahead of the quantizer: one launch for norm + quantize + GEMV of one token.
+// the same with the (residual +) RMSNorm, or SwiGLU of a row [gate | up], in front
 int32_t launch_norm_linear_fused(const float *x, const float *res, const float *g, float eps, float *h_out,
                                  float *xn_out, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx,
-                                 int64_t M64, int64_t N64, int64_t K64, hipStream_t s)
+                                 int64_t M, int64_t N, int64_t K, hipStream_t s)
 {
-    const int N = (int)N64, K = (int)K64;
-    if (M64 != 1 || K % 1024) return MI_EINVAL;
-    const int nchunk = K >> 10;
-    const FusedNorm nm = {res, g, h_out, xn_out, eps};
-    if (nchunk == 4) return launch_fused<4, 2, true>(x, qw, sw, y, qx, sx, N, K, nm, s);
-    if (nchunk == 2) return launch_fused<2, 1, true>(x, qw, sw, y, qx, sx, N, K, nm, s);
-    return MI_EINVAL;
+    if (M != 1) return MI_EINVAL;
+    return launch_row<NORM>(x, qw, sw, y, qx, sx, N, K, RowArgs{res, g, h_out, xn_out, eps}, s);
+}
+int32_t launch_swiglu_linear_fused(const float *gate_up, float *h_out, const int8_t *qw, const float *sw, float *y, int8_t *q,
+                                   float *scale, int64_t M, int64_t N, int64_t K, hipStream_t s)
+{
+    if (M != 1) return MI_EINVAL;
+    return launch_row<SWIGLU>(gate_up, qw, sw, y, q, scale, N, K, RowArgs{nullptr, nullptr, nullptr, h_out, 0.0f}, s);
 }
 
 template <int MB, int CW, int WG, bool DEQ>

@@ -414,7 +414,7 @@ struct MoeFfn {
     }
 };
 
-// One decoder layer of a decode step (one new token per sequence), chained on one stream, nine launches (seven for a
+// One decoder layer of a decode step (one new token per sequence), chained on one stream, nine launches (six for a
 // single sequence; a row-major cache takes one more, for the append):
 // (residual +) RMSNorm + quantize -> QKV GEMV -> rotary + cache append -> attention over the cache (split, merge +
 // quantize: the output projection takes the rows in the rotated basis of V) -> O GEMV -> residual + RMSNorm +
@@ -511,8 +511,7 @@ struct DecoderLayer {
             if (rc == MI_OK)
                 rc = mi_rmsnorm_linear_f32(ao, xin, g2, eps, h1, hn, gate_up.qw, gate_up.sw, gu, B, 2 * I, H, 128,
                                            gate_up.workspace, gate_up.workspace_bytes, stream);
-            if (rc == MI_OK) rc = mi_swiglu_quant_f32_i8(gu, act, ci, si, B, I, 128, stream);
-            if (rc == MI_OK) rc = mi_w8a8_gemm_dequant_f32(ci, si, down.qw, down.sw, dn, B, H, I, stream);
+            if (rc == MI_OK) rc = mi_swiglu_linear_f32(gu, act, ci, si, down.qw, down.sw, dn, B, H, I, 128, stream);
         }
         if (rc == MI_OK && out) rc = mi_add_f32(h1, dn, out, B * H, stream);
         return rc;

@@ -108,6 +108,7 @@ SIGNATURES = {
     "mi_rmsnorm_quant_f32_i8": (i32, [vp, vp, vp, C.c_float, vp, vp, vp, vp, i64, i64, i32, vp]),
     "mi_rmsnorm_linear_f32": (i32, [vp, vp, vp, C.c_float, vp, vp, vp, vp, vp, i64, i64, i64, i32, vp, i64, vp]),
     "mi_swiglu_quant_f32_i8": (i32, [vp, vp, vp, vp, i64, i64, i32, vp]),
+    "mi_swiglu_linear_f32": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i32, vp]),
     "mi_add_f32": (i32, [vp, vp, vp, i64, vp]),
     "mi_gqa_decode_attn_cache_quant_i8": (i32, [vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, vp, i64, vp,
                                                 i64, vp]),
@@ -589,9 +590,8 @@ class DecoderLayer:
             check(lib.mi_rmsnorm_linear_f32(self.ao.ptr, xin.ptr, self.g2.ptr, self.eps, self.h1.ptr, p(self.hn),
                                             self.wgu[0].ptr, self.wgu[1].ptr, self.gu.ptr, B, 2 * I, H, self.block,
                                             self.lin_ws.ptr, self.lin_ws.nbytes, s), "mi_rmsnorm_linear_f32")
-            check(lib.mi_swiglu_quant_f32_i8(self.gu.ptr, p(self.act), self.ci.ptr, self.si.ptr, B, I, self.block, s),
-                  "mi_swiglu_quant_f32_i8")
-            gemm_dequant(self.ci, self.si, self.wd[0], self.wd[1], self.dn, s)
+            check(lib.mi_swiglu_linear_f32(self.gu.ptr, p(self.act), self.ci.ptr, self.si.ptr, self.wd[0].ptr, self.wd[1].ptr,
+                                           self.dn.ptr, B, H, I, self.block, s), "mi_swiglu_linear_f32")
         else:
             m = self.moe
             check(lib.mi_rmsnorm_f32(self.ao.ptr, xin.ptr, self.g2.ptr, self.eps, self.h1.ptr, self.hn.ptr, B, H, s),

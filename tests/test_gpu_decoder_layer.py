@@ -304,6 +304,62 @@ def test_fused_swiglu_quant_equals_the_two_calls(mi, dev, orc, M, I, block):
     dev.reset_to(mark)
 
 
+@pytest.mark.parametrize("N,K", [(n, k) for k in (2048, 4096, 14336) for n in (16, 2048, 2064, 4112, 6144, 8208, 16400)] +
+                         [(28672, 4096), (28672, 14336)])
+def test_one_token_kernel_equals_the_separate_calls(mi, dev, N, K):
+    """The GEMV that makes its own codes, with fewer rows than waves, one to seven a wave and shares that differ by one: the
+    linear and SwiGLU + linear give the codes, the scale, the activated row and the results of the separate calls, bit for bit;
+    with an output on top of the input they are two launches, and the same."""
+    mark = dev.mark()
+    g = np.random.default_rng(N + K)
+    gu = dev.upload((2 * g.standard_normal((1, 2 * K))).astype(np.float32))
+    x = gu.offset(0, (1, K), np.float32)
+    qw, sw = dev.upload(g.integers(-127, 128, (N, K)).astype(np.int8)), dev.upload(g.uniform(0.001, 0.1, N).astype(np.float32))
+    h = [dev.empty((1, K), np.float32) for _ in range(2)]
+    q = [dev.empty((1, K), np.int8) for _ in range(2)]
+    sc = [dev.empty(1, np.float32) for _ in range(2)]
+    y = [dev.empty((1, N), np.float32) for _ in range(2)]
+    same = lambda a: np.array_equal(dev.download(a[0]), dev.download(a[1]))  # noqa: E731
+    ws = dev.empty(mi.lib.mi_w8a8_linear_workspace_bytes(1, N, K), np.uint8)
+    mi.linear(x, qw, sw, y[0], 128, ws)
+    mi.fwht_quant(x, q[1], sc[1], 128)
+    mi.gemm_dequant(q[1], sc[1], qw, sw, y[1])
+    assert same(y) and np.array_equal(dev.download(ws.offset(0, (1, K), np.int8)), dev.download(q[1]))
+    swiglu = lambda gu_, h_, y_: mi.check(mi.lib.mi_swiglu_linear_f32(  # noqa: E731
+        gu_.ptr, h_.ptr if h_ else None, q[0].ptr, sc[0].ptr, qw.ptr, sw.ptr, y_.ptr, 1, N, K, 128, None))
+    swiglu(gu, h[0], y[0])
+    mi.check(mi.lib.mi_swiglu_quant_f32_i8(gu.ptr, h[1].ptr, q[1].ptr, sc[1].ptr, 1, K, 128, None))
+    mi.gemm_dequant(q[1], sc[1], qw, sw, y[1])
+    assert same(y) and same(q) and same(sc) and same(h)
+    mi.check(mi.lib.mi_fill_u32(y[0].ptr, 0x7FC00000, N, None))
+    swiglu(gu, None, y[0])
+    assert same(y)
+    swiglu(gu, x, y[0])   # the activated row on top of the gate
+    h[0] = x
+    assert same(y) and same(q) and same(sc) and same(h)
+    dev.reset_to(mark)
+
+
+@pytest.mark.parametrize("M,N,I,block", [(3, 512, 14336, 128), (1, 512, 1024, 128), (1, 512, 2048, 256), (0, 512, 2048, 128)])
+def test_swiglu_linear_of_other_shapes(mi, dev, M, N, I, block):
+    mark = dev.mark()
+    g = np.random.default_rng(M + N + I)
+    gu = dev.upload(g.standard_normal((max(M, 1), 2 * I)).astype(np.float32))
+    qw, sw = dev.upload(g.integers(-127, 128, (N, I)).astype(np.int8)), dev.upload(g.uniform(0.001, 0.1, N).astype(np.float32))
+    q, sc = [dev.empty((max(M, 1), I), np.int8) for _ in range(2)], [dev.empty(max(M, 1), np.float32) for _ in range(2)]
+    y = [dev.empty((max(M, 1), N), np.float32) for _ in range(2)]
+    args = (gu.ptr, None, q[0].ptr, sc[0].ptr, qw.ptr, sw.ptr, y[0].ptr)
+    mi.check(mi.lib.mi_swiglu_linear_f32(*args, M, N, I, block, None))
+    if M:
+        mi.check(mi.lib.mi_swiglu_quant_f32_i8(gu.ptr, None, q[1].ptr, sc[1].ptr, M, I, block, None))
+        mi.gemm_dequant(q[1], sc[1], qw, sw, y[1])
+        assert all(np.array_equal(dev.download(a), dev.download(b)) for a, b in (q, sc, y))
+    for bad in ((-1, N, I, block), (M, N + 8, I, block), (M, N, I + 64, block), (1, N, I, 64)):
+        assert mi.lib.mi_swiglu_linear_f32(*args, *bad, None) == mi.EINVAL, bad
+    assert mi.lib.mi_swiglu_linear_f32(gu.ptr + 4, *args[1:], 1, N, I, block, None) == mi.EINVAL
+    dev.reset_to(mark)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 6144, 4096), (1, 28672, 4096), (1, 272, 2048), (1, 512, 1024), (3, 1024, 4096),
                                    (16, 512, 14336)])
 def test_rmsnorm_linear_one_call(mi, dev, orc, M, N, K):
