@@ -605,7 +605,7 @@ static SplitPlan pick_splits(int64_t B, int64_t Hkv, int64_t T)
 }
 
 // the largest split count pick_splits returns for any length in [1, T]
-static int max_splits(int64_t B, int64_t Hkv, int64_t T)
+int max_splits(int64_t B, int64_t Hkv, int64_t T)
 {
     const int ntiles = (int)((T + 15) / 16);
     int best = (ntiles + 4 * TILES_LONG - 1) / (4 * TILES_LONG);   // long spans: monotone in T
@@ -633,7 +633,9 @@ int32_t launch_merge(const float *part_o, const float *part_ml, float *o, int8_t
         switch (splits) {
         case 1: MI_MERGEQ(1); break;
         case 2: MI_MERGEQ(2); break;
+        case 3: MI_MERGEQ(3); break;
         case 4: MI_MERGEQ(4); break;
+        case 5: MI_MERGEQ(5); break;
         case 6: MI_MERGEQ(6); break;
         case 8: MI_MERGEQ(8); break;
         case 12: MI_MERGEQ(12); break;
@@ -658,7 +660,9 @@ int32_t launch_merge(const float *part_o, const float *part_ml, float *o, int8_t
     switch (splits) {
     case 1: MI_MERGE(1); break;
     case 2: MI_MERGE(2); break;
+    case 3: MI_MERGE(3); break;
     case 4: MI_MERGE(4); break;
+    case 5: MI_MERGE(5); break;
     case 6: MI_MERGE(6); break;
     case 8: MI_MERGE(8); break;
     case 12: MI_MERGE(12); break;

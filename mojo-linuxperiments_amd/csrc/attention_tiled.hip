@@ -28,10 +28,13 @@
 // The partial results have the layout the merge kernels of attention.hip take.
 //
 // Bound: HBM (the K and V codes, 2 * B * Hkv * T * 128 bytes, + 8 bytes of scales per token-head).
+#include <algorithm>
+
 #include "fwht_core.h"
 
 namespace mi {
 namespace attn {
+int max_splits(int64_t B, int64_t Hkv, int64_t T);   // the row-major layout's plan: the largest split count for any length up to T
 int32_t launch_merge(const float *part_o, const float *part_ml, float *o, int8_t *oq, float *oscale, int64_t B,
                      int64_t Hq, int64_t Hkv, int splits, int out_rotated, hipStream_t s);
 }
@@ -128,11 +131,11 @@ __device__ __forceinline__ float fmax_xor(float v)
 // us of latency for a few KB; here it is one more memory round trip in a few workgroups.  Decode steps, us with two
 // launches -> one: 16 sequences of 4096 tokens, four layers 402 -> 392; one of 1531, four layers 300 -> 287; 16 of 1024
 // with experts, two layers 286 -> 280.
-template <int NW, int NT, int RING, bool DIRECT, bool APPEND>
-__global__ __launch_bounds__(64 * NW) void k_gqa_tiled_split(std::conditional_t<APPEND, StepParams, Params> p)
+template <int NW, int NTM, int RING, bool DIRECT, bool APPEND>
+__global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_tiled_split(std::conditional_t<APPEND, StepParams, Params> p)
 {
-    constexpr int SPAN = NW * NT * 64;                    // tokens a workgroup can cover
-    constexpr int SC_BYTES = NW * NT * 4 * SROW * 4;      // scores [wave][block][head][SROW]
+    constexpr int SPAN = NW * NTM * 64;                   // tokens a workgroup can cover
+    constexpr int SC_BYTES = NW * NTM * 4 * SROW * 4;     // scores [wave][block][head][SROW]
     constexpr int SCALE_BYTES = 2 * SPAN * 4;             // ks, vs of the span
     constexpr int RED_BYTES = NW * 4 * D * 4;             // [wave][head][d] fp32, reuses the space above
     constexpr int UNION = (SC_BYTES + SCALE_BYTES > RED_BYTES) ? SC_BYTES + SCALE_BYTES : RED_BYTES;
@@ -260,6 +263,12 @@ __global__ __launch_bounds__(64 * NW) void k_gqa_tiled_split(std::conditional_t<
     const float4 qlo = *reinterpret_cast<const float4 *>(qr + 4 * jj);
     const float4 qhi = *reinterpret_cast<const float4 *>(qr + 64 + 4 * jj);
 
+    // The blocks that there are, NT to a wave: a span that ends with a short sequence is streamed as the shorter one that it is
+    // (16 sequences of 1024 to 4096 tokens 23.7 -> 22.3 us, 32 of 512 to 2048 25.9 -> 23.4).  The kernel that appends knows
+    // four and two blocks only, and no bound on its registers: with all four lengths under one its full spans took 0.3 us more
+    // (16 sequences of 4096 tokens, a step's attention and projection, 35.4 -> 35.7; so 35.4, of 1024 to 4096 31.3 -> 30.1).
+    auto stream = [&](auto BLOCKS) {
+    constexpr int NT = decltype(BLOCKS)::value;
     // block j of this wave: index blk_lo + NW*j + wave (the waves stream neighbouring blocks); blocks past the
     // end of the cache row fall back on its last block and are masked like any token past the end
     const int r16 = lane & 15, c4 = lane >> 4;
@@ -526,6 +535,14 @@ __global__ __launch_bounds__(64 * NW) void k_gqa_tiled_split(std::conditional_t<
             *reinterpret_cast<float4 *>(orow + 64 + 4 * jj) = make_float4(v[4], v[5], v[6], v[7]);
         }
     }
+    };
+    const int blocks = (t_end - t_lo + 63) >> 6;
+    constexpr int FEW = APPEND && NTM == 4 ? 2 : NTM - 1;
+    if (NTM == 1 || (APPEND && NTM < 4) || __builtin_expect(blocks > FEW * NW, 1)) stream(std::integral_constant<int, NTM>{});
+    else if (APPEND) stream(std::integral_constant<int, FEW < 1 ? 1 : FEW>{});
+    else if (NTM > 3 && blocks > 2 * NW) stream(std::integral_constant<int, APPEND || NTM < 3 ? 1 : 3>{});
+    else if (NTM > 2 && blocks > NW) stream(std::integral_constant<int, APPEND || NTM < 2 ? 1 : 2>{});
+    else stream(std::integral_constant<int, 1>{});
 }
 
 // Row-major codes [rows, src_stride tokens, 128] -> the two tiled layouts, one workgroup per (64-token block, row,
@@ -652,25 +669,41 @@ struct Plan {
     int splits, per;   // workgroups per cache row, 64-token blocks per workgroup
 };
 
-// Blocks per workgroup: 16 (four per wave) when that still gives every compute unit a workgroup, otherwise as few as
-// it takes to get there.
+int max_splits(int64_t B, int64_t Hkv, int64_t T);
+
+// How many spans a row is cut into, of equal length but for the last.  Where 16 blocks a workgroup (four a wave) do not give
+// every compute unit a workgroup: as many as it takes to get there.  Else the count whose busiest unit is done first, at four
+// blocks a wave or fewer: workgroups a unit times the blocks that a workgroup streams (a multiple of four) and C0 more for
+// its start and end; the merge counts as MERGE blocks of a unit, and a finer cut has to promise a tenth (for a twentieth, mixed
+// lengths lose what equal ones gain: 20 sequences of up to 3907 tokens 0.96 and 1.05 times the time).  us with spans of 16 blocks
+// -> here: 24 sequences of 3001 tokens 35.2 -> 31.3, of 750 to 3001 in pages 29.0 -> 24.7, 12 of 2500 21.4 -> 16.2, 25 of 600 to
+// 2400 25.0 -> 19.7, 32 of 318 9.5 -> 7.1; 16 of 4096 are two workgroups a unit either way, 28.7.
 static Plan pick(int64_t B, int64_t Hkv, int64_t T)
 {
+    constexpr int C0 = 2, MERGE = 5;
     const int blocks = (int)((T + 63) / 64);
     const int64_t rows = B * Hkv, cus = compute_units();
     Plan pl;
-    pl.per = 4 * NT_MAX;
-    pl.splits = (blocks + pl.per - 1) / pl.per;
-    if (rows * pl.splits < cus) {
-        int want = (int)((cus + rows - 1) / rows);
-        if (want > blocks) want = blocks;
-        pl.per = (blocks + want - 1) / want;
-        pl.splits = (blocks + pl.per - 1) / pl.per;
+    auto cut = [&](int s) { pl.per = (blocks + s - 1) / s, pl.splits = (blocks + pl.per - 1) / pl.per; };
+    const int fewest = (blocks + 4 * NT_MAX - 1) / (4 * NT_MAX);
+    if (rows * fewest < cus) {
+        cut((int)std::min<int64_t>((cus + rows - 1) / rows, blocks));
+        return pl;
     }
+    // (no more of them than the workspace was sized for before)
+    const int most = std::min(std::max(max_splits(B, Hkv, T), attn::max_splits(B, Hkv, T)), (blocks + 7) / 8);
+    int best = fewest;
+    int64_t best_cost = INT64_MAX;
+    for (int s = fewest; s <= std::max(fewest, most); ++s) {
+        cut(s);
+        const int64_t cost = (rows * pl.splits + cus - 1) / cus * ((pl.per + 3) / 4 * 4 + C0) + (pl.splits > 1 ? MERGE : 0);
+        if (best_cost == INT64_MAX || 10 * cost < 9 * best_cost) best = s, best_cost = cost;
+    }
+    cut(best);
     return pl;
 }
 
-// the largest split count pick() returns for any length in [1, T]
+// the largest split count of the plans above for any length in [1, T], and of the row-major layout's where that is larger
 int max_splits(int64_t B, int64_t Hkv, int64_t T)
 {
     const int blocks = (int)((T + 63) / 64);
@@ -746,7 +779,7 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
     const dim3 grid((unsigned)plan.splits, (unsigned)(B * Hkv));
     const int nt = (plan.per + 3) / 4;
 #define MI_TILED(NT_, DIR_, APP_) hipLaunchKernelGGL((avt::k_gqa_tiled_split<4, NT_, 8, DIR_, APP_>), grid, dim3(256), 0, s, p)   // (p as its base without APPEND)
-#define MI_TILED_NT(DIR_, APP_) do { if (nt <= 1) MI_TILED(1, DIR_, APP_); else if (nt <= 2) MI_TILED(2, DIR_, APP_); else MI_TILED(4, DIR_, APP_); } while (0)
+#define MI_TILED_NT(DIR_, APP_) do { if (nt <= 1) MI_TILED(1, DIR_, APP_); else if (nt <= 2) MI_TILED(2, DIR_, APP_); else if (nt <= 3) MI_TILED(3, DIR_, APP_); else MI_TILED(4, DIR_, APP_); } while (0)
     if (step) { if (direct) MI_TILED_NT(true, true); else MI_TILED_NT(false, true); }
     else { if (direct) MI_TILED_NT(true, false); else MI_TILED_NT(false, false); }
 #undef MI_TILED_NT

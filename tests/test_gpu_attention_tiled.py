@@ -128,6 +128,37 @@ def test_vt_ragged_lengths_and_zero_length(mi, dev, orc):
         assert np.max(np.abs(o[b] - oo[0])) <= 2e-5, b
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,T_cap,spread", [
+    (24, 16, 8, 3008, 750),    # four spans of 12 blocks, three to a wave
+    (12, 16, 8, 2560, 1),      # five of eight
+    (32, 16, 8, 320, 1),       # one of five: the kernel writes the output rows itself
+    (25, 8, 8, 2432, 600),
+    (64, 8, 4, 704, 1),        # one of eleven
+    (16, 8, 8, 4096, 1000),    # four of 16
+    (13, 8, 8, 4480, 64),
+])
+def test_vt_spans_of_every_length(mi, dev, orc, B, Hq, Hkv, T_cap, spread):
+    """Enough rows that the plan weighs how finely it cuts them; lengths spread over the capacity, so that spans end with
+    1, 2, ... blocks, in and on the edge of a block, and one sequence has none."""
+    mark = dev.mark()
+    lens = np.linspace(spread, T_cap - 1, B).astype(np.int32)
+    lens[1], lens[2], lens[3], lens[-1] = 0, 64 * (int(lens[2]) // 64 + 1), 64 * (T_cap // 128) + 1, T_cap
+    q, kq, ks, vq, vs, _, _ = make_cache(mi, dev, 18, B, Hq, Hkv, T_cap, T_cap)
+    dkq, dvt = convert(mi, dev, kq, vq, T_cap, T_cap)
+    ws = dev.empty(mi.lib.mi_gqa_decode_workspace_bytes(B, Hq, Hkv, 128, T_cap), np.uint8)
+    dq, dks, dvs, dl = dev.upload(q), dev.upload(ks), dev.upload(vs), dev.upload(lens)
+    do = dev.empty((B, Hq, 128), np.float32)
+    mi.check(mi.lib.mi_gqa_decode_attn_tiled(dq.ptr, dkq.ptr, dks.ptr, dvt.ptr, dvs.ptr, do.ptr, B, Hq, Hkv, 128, T_cap,
+                                          dl.ptr, T_cap, 0, ws.ptr, ws.nbytes, None))
+    o = dev.download(do)
+    dev.reset_to(mark)
+    assert np.all(o[1] == 0)
+    for b in [b for b in range(B) if lens[b]]:
+        n = int(lens[b])
+        oo = orc.gqa_decode(q[b:b + 1], kq[b:b + 1, :, :n], ks[b:b + 1, :, :n], vq[b:b + 1, :, :n], vs[b:b + 1, :, :n])
+        assert np.max(np.abs(o[b] - oo[0])) <= 2e-5, (b, n)
+
+
 def test_vt_peaked_and_flat_softmax(mi, dev, orc):
     """The fixed-point weights at their extremes: one token takes all the weight (its key is the query scaled up),
     and all tokens weigh the same (identical keys); V scales spread over three decades inside one span."""
@@ -495,6 +526,15 @@ def test_append_inside_the_attention_equals_the_two_calls(mi, dev, B, Hq, Hkv, T
     assert lib.mi_rope_append_attn_tiled_linear_f32(*row, *c, None, *tail) == mi.EINVAL
     assert lib.mi_rope_append_attn_tiled_linear_f32(dqkv.ptr, heads * D - 4, *row[2:], *c, pos.ptr, *tail) == mi.EINVAL
     dev.reset_to(mark)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,T_cap,T_max", [
+    (16, 8, 8, 4096, 4096),      # spans of 16 blocks, of which a short sequence has one or two a wave
+    (24, 16, 8, 3008, 3001),     # of 12
+    (12, 8, 8, 2560, 2500),      # of eight
+])
+def test_append_in_spans_of_every_length(mi, dev, B, Hq, Hkv, T_cap, T_max):
+    test_append_inside_the_attention_equals_the_two_calls(mi, dev, B, Hq, Hkv, T_cap, T_max)
 
 
 @pytest.mark.parametrize("T", [40, 3000])   # one split, which writes the output rows itself, and many
