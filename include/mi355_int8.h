@@ -214,8 +214,9 @@ MI_API int64_t mi_gemm_batch_plan_bytes(const int64_t *mnk, int32_t n);
 /* The tile lists over all n problems on a device of `compute_units` units, written to host memory (int32
  * [compute_units][per_wg][4] = problem or -1 for the end of a workgroup's list, first row, first column, cost in K
  * stages; workgroup w runs on XCD w % 8): for tests and for callers that want to look at the balance.  A batch holds
- * these lists where none of its problems runs in small tiles, otherwise those over the problems that are left.  Returns
- * the bytes written.  Makes no device call. */
+ * these lists where none of its problems runs in small tiles, otherwise those over the problems that are left, or, where
+ * its large tiles would leave compute units idle for long, lists of 256 x 128 tiles in no more bytes.  Returns the bytes
+ * written.  Makes no device call. */
 MI_API int64_t mi_gemm_batch_plan_host(const int64_t *mnk, int32_t n, int32_t compute_units, int32_t *lists_out,
                                        int64_t capacity_bytes, int32_t *per_wg_out);
 /* How a batch of these shapes runs on such a device: small_out int32 [n] = 1 for a problem that runs in small tiles,
