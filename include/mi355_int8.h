@@ -503,7 +503,8 @@ MI_API int32_t mi_swiglu_quant_f32_i8(const float *gate_up, float *h_out, int8_t
                                       int64_t M, int64_t I, int32_t block, void *stream);
 /* (residual +) RMSNorm + rotate + quantize + W8A8 contraction + dequant as one call: y = linear(rmsnorm(x (+ residual))).
  * For one token and K in {2048, 4096} (block 128) it is ONE kernel (the GEMV normalizes and quantizes the row
- * itself); any other shape runs mi_rmsnorm_quant_f32_i8 and the contraction.  workspace as for mi_w8a8_linear_f32
+ * itself); any other shape, and outputs or a workspace that overlap x, residual or g or each other, run
+ * mi_rmsnorm_quant_f32_i8 and the contraction.  workspace as for mi_w8a8_linear_f32
  * (it receives the codes and the scale); h_out (the residual sum, required with a residual) and xn_out (the
  * normalized row, optional) as in mi_rmsnorm_quant_f32_i8. */
 MI_API int32_t mi_rmsnorm_linear_f32(const float *x, const float *residual, const float *g, float eps,
@@ -512,8 +513,8 @@ MI_API int32_t mi_rmsnorm_linear_f32(const float *x, const float *residual, cons
                                      void *workspace, int64_t workspace_bytes, void *stream);
 /* SwiGLU + rotate + quantize + W8A8 contraction + dequant as one call: y = linear(swiglu(gate_up)), I the contraction length.
  * q int8 [M,I], scale fp32 [M] and h_out (optional) as in mi_swiglu_quant_f32_i8, qw int8 [N,I], sw fp32 [N], y fp32 [M,N].
- * For one token and I in {2048, 4096, 14336} (block 128) it is ONE kernel; any other shape, and outputs that overlap gate_up,
- * run mi_swiglu_quant_f32_i8 and the contraction.  The same bits either way. */
+ * For one token and I in {2048, 4096, 14336} (block 128) it is ONE kernel; any other shape, and outputs that overlap gate_up
+ * or each other, run mi_swiglu_quant_f32_i8 and the contraction.  The same bits either way. */
 MI_API int32_t mi_swiglu_linear_f32(const float *gate_up, float *h_out, int8_t *q, float *scale, const int8_t *qw,
                                     const float *sw, float *y, int64_t M, int64_t N, int64_t I, int32_t block, void *stream);
 /* out = a + b over n floats (n % 4 == 0): the residual add that closes the layer. */

@@ -862,12 +862,13 @@ static int32_t attn_linear(const float *q, const int8_t *kq, const float *ks, co
     float *oscale = reinterpret_cast<float *>(reinterpret_cast<char *>(oq) + align_up(B * K, 256));
     void *attn_ws = reinterpret_cast<char *>(oscale) + align_up(B * 4, 256);
     hipStream_t s = as_stream(stream);
-    if (B == 1 && (K == 2048 || K == 4096)) {
+    float *orow = o_rot ? o_rot : row;
+    if (B == 1 && (K == 2048 || K == 4096) && apart({{orow, K * 4}}, {{y, N * 4}, {oq, K}, {oscale, 4}})) {
         // One token: merging its Hq rows AND quantizing them in one workgroup makes that workgroup read every split's
         // partials (Hq x splits x 512 B, half a megabyte at 32 splits) through one compute unit.  Here the merge runs
         // over many workgroups and leaves the fp32 row; the projection's GEMV quantizes it in its own prologue
-        // (the same row quantizer on the same values: identical codes, scale and y).
-        float *orow = o_rot ? o_rot : row;
+        // (the same row quantizer on the same values: identical codes, scale and y).  Its workgroups read the row while
+        // others write: an output on top of the row takes the other route.
         int32_t rc = run_tiled(q, kq, ks, vt, vs, orow, nullptr, nullptr, B, Hq, Hkv, D, T_cap, seq_len, T_max, 1, attn_ws,
                                attn_bytes, s, nullptr, 0, nullptr, step);
         if (rc) return rc;

@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <initializer_list>
 #include <utility>
 
 #include "../../include/mi355_int8.h"
@@ -42,6 +43,22 @@ inline bool overlaps(const void *a, int64_t an, const void *b, int64_t bn)
     if (!a || !b) return false;
     const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
     return pa < pb + (uintptr_t)bn && pb < pa + (uintptr_t)an;
+}
+struct Span {
+    const void *at;
+    int64_t bytes;
+};
+// does none of the ranges that a kernel writes share a byte with one that it reads, or with another that it writes: what a
+// kernel needs whose workgroups all read the inputs while some already write
+inline bool apart(std::initializer_list<Span> reads, std::initializer_list<Span> writes)
+{
+    for (auto w = writes.begin(); w != writes.end(); ++w) {
+        for (const Span &r : reads)
+            if (overlaps(w->at, w->bytes, r.at, r.bytes)) return false;
+        for (auto v = writes.begin(); v != w; ++v)
+            if (overlaps(w->at, w->bytes, v->at, v->bytes)) return false;
+    }
+    return true;
 }
 
 int32_t compute_units();   // of the current device, cached

@@ -146,13 +146,9 @@ extern "C" int32_t mi_rmsnorm_linear_f32(const float *x, const float *residual, 
     if (!x || !g || !sw || !aligned16(sw) || !aligned16(x) || !aligned16(g) || !(eps >= 0.0f)) return MI_EINVAL;
     if (residual && (!h_out || !aligned16(residual) || !aligned16(h_out))) return MI_EINVAL;
     if (xn_out && !aligned16(xn_out)) return MI_EINVAL;
-    // The one-kernel form reads x and residual in every workgroup while one of them writes h_out / xn_out: a caller
-    // that updates its residual stream in place (h_out or xn_out overlapping x or residual) takes the two-kernel
-    // form, whose row operator reads each element before it writes it.
-    const int64_t row_bytes = M * K * 4;
-    const bool in_place = overlaps(h_out, row_bytes, x, row_bytes) || overlaps(h_out, row_bytes, residual, row_bytes) ||
-                          overlaps(xn_out, row_bytes, x, row_bytes) || overlaps(xn_out, row_bytes, residual, row_bytes);
-    if (M == 1 && block == 128 && !in_place) {
+    // one token: one kernel (MI_EINVAL = a shape that it does not cover, or buffers that share memory: a residual stream updated
+    // in place takes the two kernels, whose row operator reads each element before it writes it)
+    if (M == 1 && block == 128) {
         rc = launch_norm_linear_fused(x, residual, g, eps, h_out, xn_out, qw, sw, y, qx, sx, M, N, K, as_stream(stream));
         if (rc != MI_EINVAL) return rc;
     }
@@ -168,10 +164,7 @@ extern "C" int32_t mi_swiglu_linear_f32(const float *gate_up, float *h_out, int8
     if (rc) return rc;
     if (!gate_up || !scale || !sw || !aligned16(gate_up) || !aligned4(scale) || !aligned16(sw) || (h_out && !aligned16(h_out)))
         return MI_EINVAL;
-    // (the one-kernel form reads gate_up in every workgroup while others write)
-    const int64_t row = 2 * I * 4;
-    if (M == 1 && block == 128 && !overlaps(gate_up, row, h_out, I * 4) && !overlaps(gate_up, row, q, I) &&
-        !overlaps(gate_up, row, scale, 4) && !overlaps(gate_up, row, y, N * 4)) {
+    if (M == 1 && block == 128) {   // MI_EINVAL as above
         rc = launch_swiglu_linear_fused(gate_up, h_out, qw, sw, y, q, scale, M, N, I, as_stream(stream));
         if (rc != MI_EINVAL) return rc;
     }
@@ -187,9 +180,8 @@ static int32_t linear_with(const float *x, const int8_t *qw, const float *sw, fl
     int32_t rc = check_gemm(qx, qw, y, M, N, K);
     if (rc) return rc;
     if (!x || !sw || !aligned16(sw)) return MI_EINVAL;
-    if (M == 1 && block == 128 && aligned16(x) && !overlaps(x, K * 4, y, N * 4) && !overlaps(x, K * 4, qx, K)) {
-        // decode: one kernel that quantizes its own activations (MI_EINVAL = shape not covered); every workgroup reads the
-        // whole of x while others write
+    if (M == 1 && block == 128 && aligned16(x)) {
+        // decode: one kernel that quantizes its own activations (MI_EINVAL as above)
         rc = launch_linear_fused(x, qw, sw, y, qx, sx, M, N, K, as_stream(stream), true);
         if (rc != MI_EINVAL) return rc;
     }

@@ -319,6 +319,11 @@ template <RowOp OP>
 static int32_t launch_row(const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx, int64_t N,
                           int64_t K, const RowArgs &ra, hipStream_t s)
 {
+    // Every workgroup reads the whole row while others write, so buffers that share memory get the launches one behind the
+    // other.  (The weights are not looked at: results on top of them are no more defined in the contraction alone.)
+    if (!apart({{x, (OP == SWIGLU ? 2 : 1) * K * 4}, {ra.res, K * 4}, {ra.g, K * 4}},
+               {{y, N * 4}, {qx, K}, {sx, 4}, {ra.h_out, K * 4}, {ra.xn_out, K * 4}}))
+        return MI_EINVAL;
     const int cus = compute_units(), per_wave = (int)((N + 8 * cus - 1) / (8 * cus));
 #define MI_ROW(CW_, CQ_, R_, WGS_)                                                                                              \
     hipLaunchKernelGGL((k_gemv_row<CW_, CQ_, R_, OP>), dim3((unsigned)(WGS_) * cus), dim3(512), 0, s, x, qw, sw, y, qx, sx, (int)N, \

@@ -329,6 +329,29 @@ def test_vt_attention_with_projection_is_the_two_calls(mi, dev, orc, B, Hq, Hkv,
     assert np.array_equal(a, b) and np.array_equal(a, c)
 
 
+@pytest.mark.parametrize("Hq,Hkv,N", [(32, 8, 4096), (16, 4, 2048), (16, 4, 6144)])
+def test_projection_of_one_token_on_top_of_the_row_it_reads(mi, dev, Hq, Hkv, N):
+    """y over o_rot: the one-token projection reads the merged row in every workgroup while others already write y, so such a
+    call quantizes in the merge and contracts behind it, and y is what a buffer of its own gets."""
+    lib = mi.lib
+    mark = dev.mark()
+    D, K, T = 128, Hq * 128, 300
+    q, kq, _, vq, _, ks, vs = make_cache(mi, dev, 29, 1, Hq, Hkv, T, 320)
+    dkt, dvt = convert(mi, dev, kq, vq, T, 320)
+    w = workload.normal(6, (N, K), 3)
+    dqw, dsw = dev.empty((N, K), np.int8), dev.empty(N, np.float32)
+    mi.fwht_quant(dev.upload(w), dqw, dsw, 128)
+    args = tuple(dev.upload(a).ptr if isinstance(a, np.ndarray) else a.ptr for a in (q, dkt, ks, dvt, vs))
+    ws = dev.empty(lib.mi_gqa_decode_attn_linear_workspace_bytes(1, Hq, Hkv, D, T), np.uint8)
+    tail = (1, Hq, Hkv, D, 320, None, T, N, ws.ptr, ws.nbytes, None)
+    own, row = dev.empty(N, np.float32), dev.empty(max(N, K), np.float32)
+    mi.check(lib.mi_gqa_decode_attn_tiled_linear_f32(*args, row.ptr, dqw.ptr, dsw.ptr, own.ptr, *tail))
+    mi.check(lib.mi_gqa_decode_attn_tiled_linear_f32(*args, row.ptr, dqw.ptr, dsw.ptr, row.ptr, *tail))
+    a, b = dev.download(own), dev.download(row)[:N]
+    dev.reset_to(mark)
+    assert np.abs(a).max() > 0 and np.array_equal(a, b)
+
+
 # ---- the paged form of the tiled cache, and the gate on the tiled kernel's own integers
 
 def to_pages(dense, table, Hkv, per_page):

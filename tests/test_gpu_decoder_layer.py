@@ -340,6 +340,57 @@ def test_one_token_kernel_equals_the_separate_calls(mi, dev, N, K):
     dev.reset_to(mark)
 
 
+@pytest.mark.parametrize("K", [2048, 4096, 14336])
+@pytest.mark.parametrize("op", ["linear", "norm", "swiglu"])
+def test_one_token_results_on_top_of_what_they_are_made_from(mi, dev, op, K):
+    """Results, codes or scale of one token written over a row that the call reads (or results over a row that it leaves): every
+    workgroup of the one-kernel form reads the whole row while others already write, so such a call runs one launch behind the
+    other and gives what separate buffers give."""
+    mark = dev.mark()
+    N = K
+    al = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    g = np.random.default_rng(K)
+    rows = {"x": g.standard_normal(2 * K), "res": g.standard_normal(K), "g": 1 + 0.1 * g.standard_normal(K)}
+    rows = {k: v.astype(np.float32) for k, v in rows.items()}
+    qw, sw = dev.upload(g.integers(-127, 128, (N, K)).astype(np.int8)), dev.upload(g.uniform(0.001, 0.1, N).astype(np.float32))
+    need = mi.lib.mi_w8a8_linear_workspace_bytes(1, N, K)
+
+    def call(y_on=None, codes_on=None, scale_on=None):
+        """y, codes, scale; what is named lies on the first bytes of that row (the codes: the whole workspace)."""
+        at = dev.mark()
+        room = {k: dev.empty(need + 8 * K, np.uint8) for k in ("before", "x", "res", "g", "h", "y", "ws")}
+        for k, v in rows.items():
+            mi.check(mi.lib.mi_memcpy_h2d(room[k].ptr, v.ctypes.data, v.nbytes, None))
+        dev.sync()
+        x, res, gain, h = (room[k].ptr for k in ("x", "res", "g", "h"))
+        y = room[y_on or "y"].offset(0, (N,), np.float32)
+        ws = room[codes_on or "ws"].ptr
+        if scale_on:
+            ws = room[scale_on].ptr - al(K)   # (the end of the room in front of it, which is larger than what it holds)
+        codes, scale = mi.DevBuf(ws, (K,), np.int8), mi.DevBuf(ws + al(K), (1,), np.float32)
+        if op == "linear":
+            mi.check(mi.lib.mi_w8a8_linear_f32(x, qw.ptr, sw.ptr, y.ptr, 1, N, K, 128, ws, need, None))
+        elif op == "norm":
+            mi.check(mi.lib.mi_rmsnorm_linear_f32(x, res, gain, 1e-5, h, None, qw.ptr, sw.ptr, y.ptr, 1, N, K, 128, ws, need, None))
+        else:
+            mi.check(mi.lib.mi_swiglu_linear_f32(x, h, codes.ptr, scale.ptr, qw.ptr, sw.ptr, y.ptr, 1, N, K, 128, None))
+        got = dev.download(y), dev.download(codes), dev.download(scale)
+        dev.reset_to(at)
+        return got
+
+    want = call()
+    read = {"linear": ["x"], "norm": ["x", "res", "g"], "swiglu": ["x"]}[op]
+    left = [] if op == "linear" else ["h"]
+    for row in read + left:
+        got = call(y_on=row)
+        assert all(np.array_equal(a, b) for a, b in zip(got, want)), row
+    for row in read:
+        for where in ({"codes_on": row}, {"scale_on": row}):
+            got = call(**where)
+            assert all(np.array_equal(a, b) for a, b in zip(got, want)), where
+    dev.reset_to(mark)
+
+
 @pytest.mark.parametrize("M,N,I,block", [(3, 512, 14336, 128), (1, 512, 1024, 128), (1, 512, 2048, 256), (0, 512, 2048, 128)])
 def test_swiglu_linear_of_other_shapes(mi, dev, M, N, I, block):
     mark = dev.mark()
