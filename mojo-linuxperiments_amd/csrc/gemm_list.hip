@@ -673,8 +673,8 @@ static Load list_load(const int64_t *mnk, const int *idx, int n, int cus, int bn
 // took 159 instead of 146 us).  Half as large, its tiles level out where the others do not: the four projections with 509 rows
 // 142 -> 118 us, 8608 and 6144 columns of 503 rows, K = 8704, 97 -> 80, 6192 columns of 1241 rows, K = 6272, 66 -> 56.  With many
 // rounds the large tiles are 1.2 times as fast (2048 rows 355 against 419 us).  Of 120 drawn batches nine go over, 0.83 to 0.96 of
-// the time before.  From eight stages a tile on; shorter ones stay where they were (nine such batches: 0.76 to 0.92 of their time).
-constexpr int64_t STREAM_MIN_K = 1024;
+// the time before.  From STREAM_MIN_K on; batches with a shorter K stay where they were, also where this kernel would be faster
+// (nine such batches: 0.76 to 0.92 of their time).
 
 // bytes of the lists of workgroups with at most this many tiles
 static int64_t list_bytes(int cus, int64_t tiles) { return cus * (tiles + 1) * (int64_t)sizeof(v4i); }

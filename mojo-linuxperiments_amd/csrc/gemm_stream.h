@@ -8,6 +8,9 @@ typedef int v2i __attribute__((ext_vector_type(2)));
 
 constexpr int STREAM_MAX = 8;
 constexpr int STREAM_BN = 128;   // columns of a tile; it has 256 rows
+// The shortest K that a list may hold.  The kernel's two areas of scales need more stages of 128 bytes a tile than it has stage
+// buffers, three: four or more, K >= 512.  1024 is the line that the rule of gemm_list.hip was measured with.
+constexpr int64_t STREAM_MIN_K = 1024;
 struct StreamProblem {
     const int8_t *qx, *qw;
     const float *sx, *sw;

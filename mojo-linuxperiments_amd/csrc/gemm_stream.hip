@@ -18,8 +18,9 @@
 // fewer bytes per result and are 1.2 times as fast where there are enough of them; 128 x 128 tiles in this form were slower
 // than both (four projections with 509 rows 144 us, this kernel 115, 256 x 256 and small tiles in two launches 135).
 //
-// The scales of a tile come through LDS as well (a load of 64 for each wave with the tile's first stage, in two areas by turns:
-// a tile has at least as many stages as the ring has buffers).
+// The scales of a tile come through LDS as well (a load of 64 for each wave with the tile's first stage, in two areas by turns.
+// The loads run D stages ahead: with no more than D stages a tile they would enter the tile after the next, and write its
+// scales over those of the tile in work, before its end has read them.  So a tile has more stages than the ring has buffers).
 #include "common.h"
 #include "gemm_stream.h"
 
@@ -257,6 +258,7 @@ int32_t launch_stream(const StreamBatch &b, const v2i *lists, int grid, int per_
 {
     using C = stream::Cfg<4, 4, 4, 2, 3>;
     static_assert(C::BM == 256 && C::BN == STREAM_BN, "the tiles that the lists are made of");
+    static_assert(STREAM_MIN_K / 128 > C::D, "the scales of a tile are read before those of the tile after the next arrive");
     MI_LDS_OPT_IN((&stream::k_w8a8_stream<C, DEQ>), C::LDS);
     hipLaunchKernelGGL((stream::k_w8a8_stream<C, DEQ>), dim3((unsigned)grid), dim3(512), C::LDS, s, b, lists, per_wg);
     return launch_status();
