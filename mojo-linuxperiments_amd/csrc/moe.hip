@@ -716,12 +716,17 @@ __global__ __launch_bounds__(256) void k_moe_expert_gemm(const int8_t *__restric
 // The same contraction with the activation fragments held in registers (possible when a wave's K slice is at
 // most NSMAX steps of 128 bytes): only weights travel through the ring, twice as many of them are in flight
 // for the same LDS, and a workgroup walks several row chunks against one set of activation registers.
-constexpr int RX_RING = 4;   // stages in flight per wave (down with two, 2 or 3 workgroups a unit: 1.5 to 3 % slower a layer)
+// Stages in flight per wave.  The down kernel by itself, traced at 512 tokens and a router's own counts, takes 59.1 us with four,
+// 58.5 with three, 57.6 with two; the layer that it is part of 186.5, 187.0 and 188.4 (with two, 3 % less to 1 % more elsewhere).
+constexpr int RX_RING = 4;
 constexpr int RX_STAGE = 2 * NGRP * 1024;
 constexpr int RX_RING_BYTES = 4 * RX_RING * RX_STAGE;
 constexpr int RX_MT = 4;   // most 16-token fragments per pass
 constexpr int RX_RED_BYTES = NGRP * RX_MT * 4 * 64 * 4;
-constexpr int RX_LDS = RX_RING_BYTES + RX_RED_BYTES + 16 * RX_MT * 8 + 8 * 128 * 4;   // + metadata + scales of a run of chunks
+constexpr int RX_SCALES = 1024;   // weight scales of a run of chunks: four for each of 256 threads
+constexpr int rx_most_chunks(bool down) { return RX_SCALES / (down ? 128 : 32); }   // of a run
+constexpr int RX_LDS = RX_RING_BYTES + RX_RED_BYTES + 16 * RX_MT * 8 + RX_SCALES * 4;   // 8 bytes of metadata a token
+static_assert(2 * RX_LDS <= 160 * 1024, "two workgroups a unit");
 
 // Most tokens of a pass over an expert's weights: what the registers hold.  (512 tokens, H = 2048, 12 of 128 experts with more
 // than 48: 180 us for the layer's FFN with passes of 48, 176 with 64.)
@@ -748,8 +753,8 @@ __device__ __forceinline__ void rx_pass(char *smem, const int8_t *__restrict__ a
     int *s_red = reinterpret_cast<int *>(smem + RX_RING_BYTES);    // [NGRP][MTT][4][64] sums over the four K slices (gate/up)
     // token metadata and the chunks' weight scales sit in LDS so that the epilogue of a chunk issues no dependent global
     // loads (each would cost a memory round trip per chunk)
-    int *s_dst = reinterpret_cast<int *>(smem + RX_RING_BYTES + RX_RED_BYTES);            // [48] output row
-    float *s_tsc = reinterpret_cast<float *>(s_dst + 16 * RX_MT);                                // [48] token scale
+    int *s_dst = reinterpret_cast<int *>(smem + RX_RING_BYTES + RX_RED_BYTES);            // [16 RX_MT] output row
+    float *s_tsc = reinterpret_cast<float *>(s_dst + 16 * RX_MT);                                // [16 RX_MT] token scale
     float *s_wsc = s_tsc + 16 * RX_MT;                                                           // [nch][SCW]
 
     __syncthreads();   // the previous pass has finished with the token metadata and the scales, and every ring is idle
@@ -784,7 +789,7 @@ __device__ __forceinline__ void rx_pass(char *smem, const int8_t *__restrict__ a
         p0 += by;
         if (!DOWN) p1 += by;
     };
-    // weight scales (nch * SCW <= 1024) and the pair whose metadata this thread brings: requested here, parked below
+    // weight scales (nch * SCW <= RX_SCALES) and the pair whose metadata this thread brings: requested here, parked below
     float wsc_now[4];
     if (first) {
 #pragma unroll
@@ -938,7 +943,9 @@ __device__ __forceinline__ int wave_scan(int v)
 // filled the units twice and a bit, with half of the experts idle at 16 tokens, and every run paid its set-up.
 // Bound by HBM.  Both expert kernels at H = 2048, I = 768, 128 experts, top-8, us before -> after: 16 tokens 90 -> 75,
 // 512 tokens at 32 an expert 147 -> 137 (604 MB at 4.4 TB/s; 115 without the results' 46 MB of stores, 110 without the matrix
-// instructions as well).  Measured without gain: non-temporal stores and loads, whole 128-byte lines per store, exact counts of
+// instructions as well), 512 as a router sends them, up to 83 an expert, 156.1 -> 155.1 (gate/up 98.4 -> 96.0, down 57.7 -> 59.1:
+// its shares are four or five chunks, and longer where an expert has more tokens).  The layer with a router's own counts, over 38
+// shapes from 1 to 2048 tokens, 16 to 128 experts: 0.84 to 1.00 of the time before, 512 tokens 191.9 -> 186.5.  Measured without gain: non-temporal stores and loads, whole 128-byte lines per store, exact counts of
 // the stores in the waits, costs that grow with an expert's tokens, rings of two stages, three workgroups a unit.
 // by_chunk: at most a chunk a workgroup, all of the same cost, with the compute units' own order as the balance.
 template <bool DOWN, int NSMAX>
@@ -992,7 +999,7 @@ __global__ __launch_bounds__(256, 2) void k_moe_expert_rx(const int8_t *__restri
         at += __builtin_amdgcn_readlane(incl, 63);
     }
     int skip = lo - at * chunks, left = hi - at * chunks;   // of the share, from where expert e begins
-    constexpr int MOST = DOWN ? 8 : 32;   // chunks whose weight scales LDS holds
+    constexpr int MOST = rx_most_chunks(DOWN);   // chunks whose weight scales LDS holds
     for (; e < E && left > 0; segment(++e, &seg0, &count)) {
         const int passes = cost(count);
         const int last = passes ? min(chunks, (left + passes - 1) / passes) : 0;
@@ -1059,7 +1066,7 @@ struct Layout {
 static Layout layout(int64_t T, int64_t H, int64_t I, int64_t E, int64_t topk)
 {
     const int64_t P = T * topk;
-    const int64_t sz[11] = {T * H, T * 4, P * 4, (2 * E + 1) * 4 /* seg_off */, P * I * 4, P * I, P * 4, P * H * 4, P * 4, P * 4, T * E * 4};
+    const int64_t sz[11] = {T * H, T * 4, P * 4, (2 * E + 1) * 4 /* seg_off: E + 1; the rest keeps the offsets that callers know */, P * I * 4, P * I, P * 4, P * H * 4, P * 4, P * 4, T * E * 4};
     Layout L;
     int64_t o = 0;
     for (int i = 0; i < 11; ++i) { L.off[i] = o; o += align_up(sz[i], 256); }
