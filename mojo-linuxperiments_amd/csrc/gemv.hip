@@ -124,7 +124,9 @@ __global__ __launch_bounds__(64 * WG) void k_gemv_reg(const int8_t *__restrict__
 // no longer counts them and waits for the weights before it touches the row.
 // Bound: HBM, beside about 3 us from launch to first byte.  us, in workgroups of four waves that took 16 rows at a time and
 // (K = 14336) two launches -> here: 6144 x 4096 9.4 -> 7.9, with the norm 10.7 -> 9.1; 4096 x 4096 7.2 -> 5.7; 4096 x 14336
-// 19.6 -> 16.2, with SwiGLU 20.4 -> 17.8; 4096 x 2048 5.4 -> 4.1; 28672 x 4096 with the norm 25.3 -> 25.2.
+// 19.6 -> 16.2, with SwiGLU 20.4 -> 17.8; 4096 x 2048 5.4 -> 4.1; 28672 x 4096 with the norm 22.2 -> 20.9, 131072 rows of it 89.5 ->
+// 89.9.  With fewer rows than waves most of them own none and make the codes all the same: 512 x 4096 4.6 -> 3.8, 16 x 4096 4.2 ->
+// 3.3, with the norm 5.2 -> 4.2, where only the workgroups that had rows were started before.
 //   ROT: rotate + quantize; PLAIN: the row arrives in the rotated basis and is only quantized;
 //   NORM: v = ((x (+ res)) * r) * g with r = 1 / sqrt(mean((x + res)^2) + eps), then rotate + quantize; workgroup 0 also leaves
 //   the residual sum (h_out) and, on request, the normalized row (xn_out);
@@ -149,11 +151,18 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
     __shared__ float s_max[WG], s_sum[WG * CQ];                      // row maxima, sums of squares
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int waves = gridDim.x * WG, id = blockIdx.x * WG + wave;
-    const int row0 = (int)((int64_t)N * id / waves), row1 = (int)((int64_t)N * (id + 1) / waves);
+    const unsigned waves = gridDim.x * WG, id = blockIdx.x * WG + wave;
+    // Where two groups a wave do not cover the rows, they are dealt in rounds, a group to a wave, so that the chip reads one
+    // stretch of the weights at a time.  With a stretch of its own for every wave (as where two groups do) some 4096 streams run a
+    // fixed distance apart, and meet in the same channels where that is near a power of two.  us, stretches -> rounds: 131072 x 2048
+    // 58.9 -> 44.0, 65536 x 2048 24.6 -> 20.8, 98304 x 4096 79.8 -> 67.8, 131072 x 4096 with the norm 104.6 -> 89.9, 28672 x 4096
+    // 21.3 -> 20.7.
+    const bool rounds = N > 2 * R * waves;
+    const int next = rounds ? R * waves : R;   // from a group of rows to the wave's next
+    const int row0 = rounds ? R * id : (int)((unsigned)N * id / waves), row1 = rounds ? N : (int)((unsigned)N * (id + 1) / waves);
     const int kbase = lane * 16;
-    // (no branch around a load: the compiler would wait for all of them where it cannot count them.  Past the wave's rows the
-    // last one is fetched again)
+    // (no branch around a load: the compiler would wait for all of them where it cannot count them.  Past the wave's rows one
+    // of them is fetched again)
     auto load_w = [&](v4i (&w)[R][CW], int row) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -197,7 +206,7 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
     }
     v4i wa[R][CW], wb[R][CW];
     load_w(wa, row0);
-    load_w(wb, row0 + R);
+    load_w(wb, row0 + next);
 
     auto leave = [&](float *to) {   // the row as it stands
 #pragma unroll
@@ -305,14 +314,14 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
     };
     int row = row0;
 #pragma unroll 1
-    for (; row + 2 * R < row1; row += 2 * R) {
+    for (; row + 2 * next < row1; row += 2 * next) {
         rows(wa, row);
-        load_w(wa, row + 2 * R);
-        rows(wb, row + R);
-        load_w(wb, row + 3 * R);
+        load_w(wa, row + 2 * next);
+        rows(wb, row + next);
+        load_w(wb, row + 3 * next < row1 ? row + 3 * next : row + 2 * next);
     }
     rows(wa, row);
-    if (row + R < row1) rows(wb, row + R);
+    if (row + next < row1) rows(wb, row + next);
 }
 
 template <RowOp OP>
@@ -329,13 +338,13 @@ static int32_t launch_row(const float *x, const int8_t *qw, const float *sw, flo
     hipLaunchKernelGGL((k_gemv_row<CW_, CQ_, R_, OP>), dim3((unsigned)(WGS_) * cus), dim3(512), 0, s, x, qw, sw, y, qx, sx, (int)N, \
                        (int)K, ra)
     // Few rows: one workgroup a unit whose two groups cover them.  Many: two a unit with a row at a time (20000 x 4096 and the
-    // norm 18.0 us, one a unit with four rows at a time 19.9), three where the codes are quickly made (28672 x 4096 24.9 against
-    // 25.9 us; with the norm 25.9 against 25.2).  14336 floats a row: one a unit is what the registers hold, and with more than
+    // norm 18.0 us, one a unit with four rows at a time 19.9), three where the codes are quickly made or the rows many enough not
+    // to mind (28672 x 4096 24.9 against 25.9 us; with the norm 21.4 against 20.4, of 65536 rows 44.9 against 45.9).  14336 floats a row: one a unit is what the registers hold, and with more than
     // eight rows a wave the two launches are level (20000 rows 58.7 against 58.5 us, 28672 79.2 against 80.9).
     if (K == 4096) {
         if (per_wave <= 2) MI_ROW(4, 1, 1, 1);
         else if (per_wave <= 4) MI_ROW(4, 1, 2, 1);
-        else if (per_wave <= 10 || OP == NORM) MI_ROW(4, 1, 1, 2);
+        else if (per_wave <= (OP == NORM ? 20 : 10)) MI_ROW(4, 1, 1, 2);
         else MI_ROW(4, 1, 1, 3);
     } else if (K == 2048) {
         if (per_wave <= 2) MI_ROW(2, 1, 1, 1);

@@ -340,6 +340,51 @@ def test_one_token_kernel_equals_the_separate_calls(mi, dev, N, K):
     dev.reset_to(mark)
 
 
+def one_token_forms(mi, dev, N, K):
+    """The three calls of one token against the calls that they are made of, bit for bit: results, codes, scale and the rows that
+    they leave."""
+    mark = dev.mark()
+    lib = mi.lib
+    g = np.random.default_rng(3 * N + K)
+    x, res = (dev.upload((2 * g.standard_normal((1, n * K))).astype(np.float32)) for n in (2, 1))
+    gain = dev.upload((1 + 0.1 * g.standard_normal(K)).astype(np.float32))
+    qw = dev.upload(np.frombuffer(g.bytes(N * K), np.int8).reshape(N, K))
+    sw = dev.upload(g.uniform(0.001, 0.1, N).astype(np.float32))
+    need = lib.mi_w8a8_linear_workspace_bytes(1, N, K)
+    at = (K + 255) // 256 * 256
+    ws = [dev.empty(need, np.uint8) for _ in range(2)]
+    q, sc = ([b.offset(o, s, t) for b in ws] for o, s, t in ((0, (1, K), np.int8), (at, (1,), np.float32)))
+    h, xn = ([dev.empty((1, K), np.float32) for _ in range(2)] for _ in range(2))
+    y = [dev.empty((1, N), np.float32) for _ in range(2)]
+
+    def check(what, *pairs):
+        mi.gemm_dequant(q[1], sc[1], qw, sw, y[1])
+        for a, b in (y, q, sc) + pairs:
+            assert np.array_equal(dev.download(a), dev.download(b)), (what, N, K)
+        mi.check(lib.mi_fill_u32(y[0].ptr, 0x7FC00000, N, None))   # NaN: every result has to be written again
+
+    mi.linear(x.offset(0, (1, K), np.float32), qw, sw, y[0], 128, ws[0])
+    mi.fwht_quant(x.offset(0, (1, K), np.float32), q[1], sc[1], 128)
+    check("linear")
+    for r in (None, res.ptr):
+        rows = lambda i: (x.ptr, r, gain.ptr, 1e-5, h[i].ptr if r else None, xn[i].ptr)  # noqa: E731
+        mi.check(lib.mi_rmsnorm_linear_f32(*rows(0), qw.ptr, sw.ptr, y[0].ptr, 1, N, K, 128, ws[0].ptr, need, None))
+        mi.check(lib.mi_rmsnorm_quant_f32_i8(*rows(1), q[1].ptr, sc[1].ptr, 1, K, 128, None))
+        check("norm", xn, *([h] if r else []))
+    mi.check(lib.mi_swiglu_linear_f32(x.ptr, h[0].ptr, q[0].ptr, sc[0].ptr, qw.ptr, sw.ptr, y[0].ptr, 1, N, K, 128, None))
+    mi.check(lib.mi_swiglu_quant_f32_i8(x.ptr, h[1].ptr, q[1].ptr, sc[1].ptr, 1, K, 128, None))
+    check("swiglu", h)
+    dev.reset_to(mark)
+
+
+@pytest.mark.parametrize("N,K", [(n, 2048) for n in (16, 4112, 8208, 12304, 16400, 40976)] +
+                         [(n, 4096) for n in (16, 4112, 8208, 20496, 24592, 49168)] + [(4112, 14336), (16384, 14336)])
+def test_one_token_forms_equal_the_separate_calls(mi, dev, N, K):
+    """Every split of the rows: one group of one, two or four rows a wave, two, and rounds of one row with two and three
+    workgroups a unit, the last round not full."""
+    one_token_forms(mi, dev, N, K)
+
+
 @pytest.mark.parametrize("K", [2048, 4096, 14336])
 @pytest.mark.parametrize("op", ["linear", "norm", "swiglu"])
 def test_one_token_results_on_top_of_what_they_are_made_from(mi, dev, op, K):
