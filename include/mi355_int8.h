@@ -340,7 +340,7 @@ MI_API int32_t mi_gqa_decode_attn_tiled_quant_i8(const float *q, const int8_t *k
  * values in the rotated basis of V, quantized as one row) contracted with prepared projection weights qw int8
  * [N, Hq*D], sw fp32 [N] (rotated along K with block D), N % 16 == 0, Hq <= 64.  The values are those of
  * mi_gqa_decode_attn_tiled_quant_i8 followed by mi_w8a8_gemm_dequant_f32, bit for bit; what differs is the division
- * of the work for ONE token (B == 1, Hq*D in {2048, 4096}): the merge then runs over many workgroups and leaves the
+ * of the work for ONE token (B == 1, Hq*D >= 1024, N as in mi_rmsnorm_linear_f32): the merge then runs over many workgroups and leaves the
  * fp32 row, and the projection's GEMV quantizes that row in its own prologue (three launches, none of which reads
  * every split's partials through one compute unit).  o_rot (optional, fp32 [B,Hq,D]) receives the merged row.
  * Workspace: mi_gqa_decode_attn_linear_workspace_bytes(B, Hq, Hkv, D, T_max).  It starts with the merged rows
@@ -502,10 +502,10 @@ MI_API int32_t mi_rmsnorm_quant_f32_i8(const float *x, const float *residual, co
 MI_API int32_t mi_swiglu_quant_f32_i8(const float *gate_up, float *h_out, int8_t *q, float *scale,
                                       int64_t M, int64_t I, int32_t block, void *stream);
 /* (residual +) RMSNorm + rotate + quantize + W8A8 contraction + dequant as one call: y = linear(rmsnorm(x (+ residual))).
- * For one token and K in {2048, 4096} (block 128) it is ONE kernel (the GEMV normalizes and quantizes the row
- * itself); any other shape, and outputs or a workspace that overlap x, residual or g or each other, run
- * mi_rmsnorm_quant_f32_i8 and the contraction.  workspace as for mi_w8a8_linear_f32
- * (it receives the codes and the scale); h_out (the residual sum, required with a residual) and xn_out (the
+ * For one token (block 128) it is ONE kernel (the GEMV normalizes and quantizes the row itself) where that is the faster
+ * form: K up to 16384 with N up to 64 rows a compute unit, K from 1024 to 8192 with up to 160, and 2048, 3072 and 4096 with
+ * any N.  Any other shape, and outputs or a workspace that overlap x, residual or g or each other, run
+ * mi_rmsnorm_quant_f32_i8 and the contraction.  workspace as for mi_w8a8_linear_f32 (it receives the codes and the scale); h_out (the residual sum, required with a residual) and xn_out (the
  * normalized row, optional) as in mi_rmsnorm_quant_f32_i8. */
 MI_API int32_t mi_rmsnorm_linear_f32(const float *x, const float *residual, const float *g, float eps,
                                      float *h_out, float *xn_out, const int8_t *qw, const float *sw, float *y,
@@ -513,8 +513,8 @@ MI_API int32_t mi_rmsnorm_linear_f32(const float *x, const float *residual, cons
                                      void *workspace, int64_t workspace_bytes, void *stream);
 /* SwiGLU + rotate + quantize + W8A8 contraction + dequant as one call: y = linear(swiglu(gate_up)), I the contraction length.
  * q int8 [M,I], scale fp32 [M] and h_out (optional) as in mi_swiglu_quant_f32_i8, qw int8 [N,I], sw fp32 [N], y fp32 [M,N].
- * For one token and I in {2048, 4096, 14336} (block 128) it is ONE kernel; any other shape, and outputs that overlap gate_up
- * or each other, run mi_swiglu_quant_f32_i8 and the contraction.  The same bits either way. */
+ * One token (block 128) is ONE kernel for the I and N that mi_rmsnorm_linear_f32 names; any other shape, and outputs that
+ * overlap gate_up or each other, run mi_swiglu_quant_f32_i8 and the contraction.  The same bits either way. */
 MI_API int32_t mi_swiglu_linear_f32(const float *gate_up, float *h_out, int8_t *q, float *scale, const int8_t *qw,
                                     const float *sw, float *y, int64_t M, int64_t N, int64_t I, int32_t block, void *stream);
 /* out = a + b over n floats (n % 4 == 0): the residual add that closes the layer. */

@@ -830,6 +830,7 @@ extern "C" int32_t mi_gqa_decode_scores_tiled_i32(const float *q, const int8_t *
 }
 
 namespace mi {
+bool row_takes(int64_t N, int64_t K);
 int32_t launch_linear_fused(const float *, const int8_t *, const float *, float *, int8_t *, float *, int64_t, int64_t,
                             int64_t, hipStream_t, bool);
 }
@@ -863,12 +864,13 @@ static int32_t attn_linear(const float *q, const int8_t *kq, const float *ks, co
     void *attn_ws = reinterpret_cast<char *>(oscale) + align_up(B * 4, 256);
     hipStream_t s = as_stream(stream);
     float *orow = o_rot ? o_rot : row;
-    if (B == 1 && (K == 2048 || K == 4096) && apart({{orow, K * 4}}, {{y, N * 4}, {oq, K}, {oscale, 4}})) {
+    if (B == 1 && K >= 1024 && row_takes(N, K) && apart({{orow, K * 4}}, {{y, N * 4}, {oq, K}, {oscale, 4}})) {
         // One token: merging its Hq rows AND quantizing them in one workgroup makes that workgroup read every split's
         // partials (Hq x splits x 512 B, half a megabyte at 32 splits) through one compute unit.  Here the merge runs
         // over many workgroups and leaves the fp32 row; the projection's GEMV quantizes it in its own prologue
         // (the same row quantizer on the same values: identical codes, scale and y).  Its workgroups read the row while
-        // others write: an output on top of the row takes the other route.
+        // others write: an output on top of the row takes the other route.  So do rows of less than eight heads, whose merge has
+        // the fewest workgroups (four heads, 4000 tokens, 4096 outputs 24.2 us there, 25.1 here; eight heads 27.1 and 26.1).
         int32_t rc = run_tiled(q, kq, ks, vt, vs, orow, nullptr, nullptr, B, Hq, Hkv, D, T_cap, seq_len, T_max, 1, attn_ws,
                                attn_bytes, s, nullptr, 0, nullptr, step);
         if (rc) return rc;

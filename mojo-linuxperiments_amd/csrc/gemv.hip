@@ -6,8 +6,8 @@
 //  k_gemv_reg: a lane always works on the same byte offsets of a weight row, so its share of the activation codes
 //  lives in registers for the whole kernel: no LDS and no barrier in the streaming part, 16 x 1 KB weight loads in
 //  flight per wave, v_dot4_i32_i8, one transposed butterfly per wave.
-//  k_gemv_row makes the codes of its one token itself (rotate + quantize, with RMSNorm or SwiGLU in front), for K of
-//  2048, 4096 and 14336.
+//  k_gemv_row makes the codes of its one token itself (rotate + quantize, with RMSNorm or SwiGLU in front), for K up to
+//  16384.
 #include <algorithm>
 #include "common.h"
 #include "fwht_core.h"
@@ -139,14 +139,15 @@ struct RowArgs {
     float eps;
 };
 
-template <int CW, int CQ, int R, RowOp OP>
+// CW: 1024-byte chunks of a weight row, the last one shorter unless WHOLE.
+template <int CW, bool WHOLE, int R, RowOp OP>
 __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x, const int8_t *__restrict__ qw,
                                                      const float *__restrict__ sw, float *__restrict__ y,
                                                      int8_t *__restrict__ qx_out, float *__restrict__ sx_out, int N, int K,
                                                      RowArgs ra)
 {
     constexpr int BLOCK = 128, LPB = BLOCK / 8, WG = 8;
-    constexpr int V = pow2_ceil(R);
+    constexpr int V = pow2_ceil(R), CQ = (CW + 3) / 4;   // chunks of 8 floats a thread
     __shared__ __attribute__((aligned(16))) int8_t s_x[CW * 1024];   // codes
     __shared__ float s_max[WG], s_sum[WG * CQ];                      // row maxima, sums of squares
     const int tid = threadIdx.x, lane = tid & 63;
@@ -162,13 +163,14 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
     const int row0 = rounds ? R * id : (int)((unsigned)N * id / waves), row1 = rounds ? N : (int)((unsigned)N * (id + 1) / waves);
     const int kbase = lane * 16;
     // (no branch around a load: the compiler would wait for all of them where it cannot count them.  Past the wave's rows one
-    // of them is fetched again)
+    // of them is fetched again, past a row's end its last 16 bytes)
+    const int klast = WHOLE ? (CW - 1) * 1024 : min((CW - 1) * 1024, K - 16 - kbase);
     auto load_w = [&](v4i (&w)[R][CW], int row) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int8_t *const p = qw + (int64_t)min(row + r, max(row1 - 1, 0)) * K + kbase;
 #pragma unroll
-            for (int c = 0; c < CW; ++c) w[r][c] = *reinterpret_cast<const v4i *>(p + c * 1024);
+            for (int c = 0; c < CW; ++c) w[r][c] = *reinterpret_cast<const v4i *>(p + (c + 1 < CW ? c * 1024 : klast));
         }
     };
 
@@ -293,6 +295,7 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
     v4i xr[CW];
 #pragma unroll
     for (int c = 0; c < CW; ++c) xr[c] = *reinterpret_cast<const v4i *>(s_x + kbase + c * 1024);
+    if (!WHOLE && kbase + (CW - 1) * 1024 >= K) xr[CW - 1] = (v4i){0, 0, 0, 0};
     constexpr int SH = 6 - __builtin_ctz(V);
     const int vi = lane >> SH;
     const bool speaker = (lane & ((1 << SH) - 1)) == 0 && vi < R;
@@ -324,42 +327,69 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
     if (row + next < row1) rows(wb, row + next);
 }
 
+// The split of the rows by their number a wave, as far as registers go (two groups of R rows of CW chunks).  Few rows: one
+// workgroup a unit whose two groups cover them.  Many: two a unit with a row at a time (20000 x 4096 and the norm 18.0 us, one a
+// unit with four rows at a time 19.9), three where the codes are quickly made or the rows many enough not to mind (28672 x 4096 24.9
+// against 25.9 us; with the norm 21.4 against 20.4, of 65536 rows 44.9 against 45.9).  From five chunks on two a unit pay beyond six
+// rows a wave only (16384 x 5120 and the norm 18.2 -> 16.1, 6144 x 8192 12.9 -> 13.9), above eight chunks one is what the registers
+// hold.
+template <int CW, bool WHOLE, RowOp OP>
+static void start_row(int cus, int per_wave, const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx,
+                      int N, int K, const RowArgs &ra, hipStream_t s)
+{
+    auto go = [&](auto R, int wgs) {
+        hipLaunchKernelGGL((k_gemv_row<CW, WHOLE, decltype(R)::value, OP>), dim3((unsigned)(wgs * cus)), dim3(512), 0, s, x, qw, sw, y,
+                           qx, sx, N, K, ra);
+    };
+    using std::integral_constant;
+    if (per_wave <= 2) return go(integral_constant<int, 1>{}, 1);
+    if constexpr (CW <= 4) {
+        if (per_wave <= 4) return go(integral_constant<int, 2>{}, 1);
+        if constexpr (CW <= 2)
+            if (per_wave <= 8) return go(integral_constant<int, 4>{}, 1);
+        return go(integral_constant<int, 1>{}, CW == 4 && per_wave > (OP == NORM ? 20 : 10) ? 3 : 2);
+    }
+    go(integral_constant<int, 1>{}, CW <= 8 && per_wave > 6 ? 2 : 1);
+}
+
+// Where the one kernel is the faster form, against making the codes and contracting them one behind the other: linear, norm and
+// SwiGLU, 20 K from 128 to 16384, whole chunks and not, 16 to 131072 rows, weights from HBM.  Up to eight rows a wave 0.57 to 1.04
+// of their time (6144 x 5120 11.9 -> 8.7 us, 4096 x 12288 with the norm 17.1 -> 14.6; no gain for 16 rows of 16384).  Up to twenty 0.77 to 1.00 from K = 1024 to
+// 8192; shorter rows lose the time that a row costs beside its bytes (28672 x 640 8.3 -> 8.5), longer ones stream no better than in
+// the GEMV by itself (28672 x 14336 72.6 -> 74.0 with SwiGLU).  Beyond, 0.93 to 0.97 in two to four whole chunks (131072 x 2048 49.4
+// -> 44.0), up to 1.14 elsewhere.
+bool row_takes(int64_t N, int64_t K)
+{
+    const int64_t cus = compute_units();
+    return K % 128 == 0 && K <= 16384 &&
+           (N <= 64 * cus || (K >= 1024 && K <= 8192 && N <= 160 * cus) || (K >= 2048 && K <= 4096 && K % 1024 == 0));
+}
+
 template <RowOp OP>
 static int32_t launch_row(const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx, int64_t N,
                           int64_t K, const RowArgs &ra, hipStream_t s)
 {
     // Every workgroup reads the whole row while others write, so buffers that share memory get the launches one behind the
     // other.  (The weights are not looked at: results on top of them are no more defined in the contraction alone.)
-    if (!apart({{x, (OP == SWIGLU ? 2 : 1) * K * 4}, {ra.res, K * 4}, {ra.g, K * 4}},
-               {{y, N * 4}, {qx, K}, {sx, 4}, {ra.h_out, K * 4}, {ra.xn_out, K * 4}}))
+    if (!row_takes(N, K) || !apart({{x, (OP == SWIGLU ? 2 : 1) * K * 4}, {ra.res, K * 4}, {ra.g, K * 4}},
+                                   {{y, N * 4}, {qx, K}, {sx, 4}, {ra.h_out, K * 4}, {ra.xn_out, K * 4}}))
         return MI_EINVAL;
     const int cus = compute_units(), per_wave = (int)((N + 8 * cus - 1) / (8 * cus));
-#define MI_ROW(CW_, CQ_, R_, WGS_)                                                                                              \
-    hipLaunchKernelGGL((k_gemv_row<CW_, CQ_, R_, OP>), dim3((unsigned)(WGS_) * cus), dim3(512), 0, s, x, qw, sw, y, qx, sx, (int)N, \
-                       (int)K, ra)
-    // Few rows: one workgroup a unit whose two groups cover them.  Many: two a unit with a row at a time (20000 x 4096 and the
-    // norm 18.0 us, one a unit with four rows at a time 19.9), three where the codes are quickly made or the rows many enough not
-    // to mind (28672 x 4096 24.9 against 25.9 us; with the norm 21.4 against 20.4, of 65536 rows 44.9 against 45.9).  14336 floats a row: one a unit is what the registers hold, and with more than
-    // eight rows a wave the two launches are level (20000 rows 58.7 against 58.5 us, 28672 79.2 against 80.9).
-    if (K == 4096) {
-        if (per_wave <= 2) MI_ROW(4, 1, 1, 1);
-        else if (per_wave <= 4) MI_ROW(4, 1, 2, 1);
-        else if (per_wave <= (OP == NORM ? 20 : 10)) MI_ROW(4, 1, 1, 2);
-        else MI_ROW(4, 1, 1, 3);
-    } else if (K == 2048) {
-        if (per_wave <= 2) MI_ROW(2, 1, 1, 1);
-        else if (per_wave <= 4) MI_ROW(2, 1, 2, 1);
-        else if (per_wave <= 8) MI_ROW(2, 1, 4, 1);
-        else MI_ROW(2, 1, 1, 2);
-    } else {
-        if constexpr (OP == ROT || OP == SWIGLU) {
-            if (K != 14336 || per_wave > 8) return MI_EINVAL;
-            MI_ROW(14, 4, 1, 1);
-        } else {
-            return MI_EINVAL;
-        }
-    }
+    switch ((K + 1023) >> 10) {
+#define MI_ROW(CW_)                                                                                                          \
+    case CW_:                                                                                                                \
+        if (K % 1024) start_row<CW_, false, OP>(cus, per_wave, x, qw, sw, y, qx, sx, (int)N, (int)K, ra, s);                  \
+        else start_row<CW_, true, OP>(cus, per_wave, x, qw, sw, y, qx, sx, (int)N, (int)K, ra, s);                            \
+        break;
+        MI_ROW(1) MI_ROW(2) MI_ROW(3) MI_ROW(4) MI_ROW(5) MI_ROW(6) MI_ROW(7) MI_ROW(8)
+    default:
+        if constexpr (OP != PLAIN)   // (an attention row has at most 64 heads)
+            switch ((K + 1023) >> 10) {
+                MI_ROW(9) MI_ROW(10) MI_ROW(11) MI_ROW(12) MI_ROW(13) MI_ROW(14) MI_ROW(15) MI_ROW(16)
 #undef MI_ROW
+            }
+        else return MI_EINVAL;
+    }
     return launch_status();
 }
 

@@ -329,7 +329,36 @@ def test_vt_attention_with_projection_is_the_two_calls(mi, dev, orc, B, Hq, Hkv,
     assert np.array_equal(a, b) and np.array_equal(a, c)
 
 
-@pytest.mark.parametrize("Hq,Hkv,N", [(32, 8, 4096), (16, 4, 2048), (16, 4, 6144)])
+@pytest.mark.parametrize("Hq,Hkv,N", [(32, 8, 6000), (32, 8, 16400), (32, 8, 28672), (16, 4, 12304), (16, 4, 16400),
+                                       (4, 1, 2048), (8, 2, 4112), (9, 3, 16400), (20, 5, 8208), (24, 8, 41008), (40, 10, 6144),
+                                       (49, 49, 2048), (64, 16, 16400)])
+def test_projection_of_one_token_with_any_number_of_heads(mi, dev, Hq, Hkv, N):
+    """The codes made in the projection (or in the merge, with few heads) and every split of its rows: the attention that
+    quantizes and the contraction behind it, bit for bit."""
+    lib = mi.lib
+    mark = dev.mark()
+    D, K, T = 128, Hq * 128, 130
+    q, kq, _, vq, _, ks, vs = make_cache(mi, dev, 31, 1, Hq, Hkv, T, 192)
+    dkt, dvt = convert(mi, dev, kq, vq, T, 192)
+    g = np.random.default_rng(N + K)
+    dqw = dev.upload(np.frombuffer(g.bytes(N * K), np.int8).reshape(N, K))
+    dsw = dev.upload(g.uniform(0.001, 0.1, N).astype(np.float32))
+    args = tuple(dev.upload(a).ptr if isinstance(a, np.ndarray) else a.ptr for a in (q, dkt, ks, dvt, vs))
+    ws = dev.empty(lib.mi_gqa_decode_attn_linear_workspace_bytes(1, Hq, Hkv, D, T), np.uint8)
+    y = [dev.empty((1, N), np.float32) for _ in range(2)]
+    mi.check(lib.mi_fill_u32(y[0].ptr, 0x7FC00000, N, None))
+    mi.check(lib.mi_gqa_decode_attn_tiled_linear_f32(*args, None, dqw.ptr, dsw.ptr, y[0].ptr, 1, Hq, Hkv, D, 192, None, T, N,
+                                                     ws.ptr, ws.nbytes, None))
+    oq, osc = dev.empty((1, K), np.int8), dev.empty(1, np.float32)
+    mi.check(lib.mi_gqa_decode_attn_tiled_quant_i8(*args, None, oq.ptr, osc.ptr, 1, Hq, Hkv, D, 192, None, T, ws.ptr, ws.nbytes,
+                                                   None))
+    mi.gemm_dequant(oq, osc, dqw, dsw, y[1])
+    a, b = (dev.download(t) for t in y)
+    dev.reset_to(mark)
+    assert np.abs(a).max() > 0 and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("Hq,Hkv,N", [(32, 8, 4096), (16, 4, 2048), (16, 4, 6144), (24, 8, 3072)])
 def test_projection_of_one_token_on_top_of_the_row_it_reads(mi, dev, Hq, Hkv, N):
     """y over o_rot: the one-token projection reads the merged row in every workgroup while others already write y, so such a
     call quantizes in the merge and contracts behind it, and y is what a buffer of its own gets."""

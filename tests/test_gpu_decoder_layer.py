@@ -385,6 +385,19 @@ def test_one_token_forms_equal_the_separate_calls(mi, dev, N, K):
     one_token_forms(mi, dev, N, K)
 
 
+@pytest.mark.parametrize("N,K", [
+    (16, 128), (4112, 640), (8208, 1024), (16384, 896), (16400, 1024), (40976, 1024),          # one chunk, whole and not
+    (2064, 1920), (4112, 1152), (12304, 1536), (20016, 1920), (4112, 3072), (8208, 2560), (41008, 3072), (8208, 3968),
+    (24592, 3200),
+    (2064, 4992), (8208, 5120), (14352, 6272), (16400, 7168), (16, 7296), (20016, 8192),       # two chunks of codes a thread
+    (16, 8320), (4112, 9216), (10256, 10112), (4112, 11008), (2064, 12288),                    # three
+    (8208, 12416), (528, 13312), (16384, 13696), (4112, 15360), (16, 16256), (8208, 16384),    # four
+    (16400, 8320), (41008, 1920), (16400, 896),                                                # just past each limit
+])
+def test_one_token_forms_of_any_length(mi, dev, N, K):
+    one_token_forms(mi, dev, N, K)
+
+
 @pytest.mark.parametrize("K", [2048, 4096, 14336])
 @pytest.mark.parametrize("op", ["linear", "norm", "swiglu"])
 def test_one_token_results_on_top_of_what_they_are_made_from(mi, dev, op, K):
@@ -459,7 +472,7 @@ def test_swiglu_linear_of_other_shapes(mi, dev, M, N, I, block):
 @pytest.mark.parametrize("M,N,K", [(1, 6144, 4096), (1, 28672, 4096), (1, 272, 2048), (1, 512, 1024), (3, 1024, 4096),
                                    (16, 512, 14336)])
 def test_rmsnorm_linear_one_call(mi, dev, orc, M, N, K):
-    """One token and K in {2048, 4096}: a single kernel; other shapes: norm + quantize, then the contraction.  Either
+    """One token: a single kernel; other shapes: norm + quantize, then the contraction.  Either
     way the normalized row follows the RMSNorm oracle, the codes are the oracle quantizer's on that row and the
     output is the oracle's contraction of those codes, exactly."""
     mark = dev.mark()
