@@ -158,6 +158,7 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
     if constexpr (APPEND) splits = p.splits;
     else splits = gridDim.x;
     const int64_t pbase = (int64_t)bkv * splits + split;
+    const bool paged = !APPEND && p.block_table;   // (the step's cache is a dense one)
 
     int T = p.T;
     if (p.seq_len) T = min(max(__builtin_amdgcn_readfirstlane(p.seq_len[b]), 0), p.T);
@@ -230,17 +231,17 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
     const int t_end = min((blk_lo + p.blocks_per_split) * 64, T);   // first token this workgroup does not own
     const int nblk_row = p.Tstride >> 6;                            // blocks per cache row
 
-    // ---- loads, in the order they are needed: the span's scales, the query rows, then the ring
+    // ---- loads, in the order they are needed: the span's scales, the query rows, the pages of the wave's blocks, then the ring
+    const int last_blk = (T - 1) >> 6;   // the last block that holds a token of this sequence
     const int sidx = 4 * tid;   // one float4 of each scale array per thread
     float4 ks4 = make_float4(0.f, 0.f, 0.f, 0.f), vs4 = ks4;
-    const int last_blk = (T - 1) >> 6;   // the last block that holds a token of this sequence
     if (sidx < SPAN) {
-        if (p.block_table) {
+        if (paged) {
             // four consecutive tokens lie in one page; blocks past the sequence's last one (their table entries may
             // hold anything) fall back on it, and their tokens are masked like any token past the end
             const int tb = min((t_lo + sidx) >> 6, last_blk);
-            const int64_t page = p.block_table[(int64_t)b * p.max_pages + tb];
-            const int64_t at = (page * p.Hkv + kvh) * 64 + ((t_lo + sidx) & 63);
+            const int64_t of = p.block_table[(int64_t)b * p.max_pages + tb];
+            const int64_t at = (of * p.Hkv + kvh) * 64 + ((t_lo + sidx) & 63);
             ks4 = *reinterpret_cast<const float4 *>(p.ks + at);
             vs4 = *reinterpret_cast<const float4 *>(p.vs + at);
         } else {
@@ -262,11 +263,22 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
     }
     const float4 qlo = *reinterpret_cast<const float4 *>(qr + 4 * jj);
     const float4 qhi = *reinterpret_cast<const float4 *>(qr + 64 + 4 * jj);
+    // One look-up per block, all of them scalar and requested at once.  (Looked up where a block's address is formed, inside the
+    // branches below, they became vector loads that each waited for everything in front of them: 8 sequences of 2048 tokens 13.6
+    // instead of 13.1 us, 16 of 4096 30.6 instead of 29.6.  In front of the scales: 4 % slower with one block a wave.)
+    int page[NTM] = {};
+    if (paged) {
+        const auto *table = (const __attribute__((address_space(4))) int32_t *)(p.block_table + (int64_t)b * p.max_pages);
+#pragma unroll
+        for (int j = 0; j < NTM; ++j) page[j] = table[min(blk_lo + NW * j + wave, last_blk)];
+    }
 
     // The blocks that there are, NT to a wave: a span that ends with a short sequence is streamed as the shorter one that it is
     // (16 sequences of 1024 to 4096 tokens 23.7 -> 22.3 us, 32 of 512 to 2048 25.9 -> 23.4).  The kernel that appends knows
     // four and two blocks only, and no bound on its registers: with all four lengths under one its full spans took 0.3 us more
-    // (16 sequences of 4096 tokens, a step's attention and projection, 35.4 -> 35.7; so 35.4, of 1024 to 4096 31.3 -> 30.1).
+    // (16 sequences of 4096 tokens, a step's attention and projection, 35.4 -> 35.7; so 35.4, of 1024 to 4096 31.3 -> 30.1).  In
+    // pages a span is always streamed whole: its blocks past the end are the sequence's last one, out of a cache (16 sequences of
+    // 1024 to 4096 tokens 22.5 us, cut short 23.1).
     auto stream = [&](auto BLOCKS) {
     constexpr int NT = decltype(BLOCKS)::value;
     // block j of this wave: index blk_lo + NW*j + wave (the waves stream neighbouring blocks); blocks past the
@@ -278,10 +290,8 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
         int64_t off;
-        if (p.block_table) {   // one scalar table look-up per block
-            const int page = __builtin_amdgcn_readfirstlane(
-                p.block_table[(int64_t)b * p.max_pages + min(blk_lo + NW * j + wave, last_blk)]);
-            off = ((int64_t)page * p.Hkv + kvh) * 8192;
+        if (paged) {
+            off = ((int64_t)page[j] * p.Hkv + kvh) * 8192;
         } else {
             off = ((int64_t)bkv * nblk_row + min(blk_lo + NW * j + wave, nblk_row - 1)) * 8192;
         }
@@ -538,7 +548,7 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
     };
     const int blocks = (t_end - t_lo + 63) >> 6;
     constexpr int FEW = APPEND && NTM == 4 ? 2 : NTM - 1;
-    if (NTM == 1 || (APPEND && NTM < 4) || __builtin_expect(blocks > FEW * NW, 1)) stream(std::integral_constant<int, NTM>{});
+    if (NTM == 1 || (APPEND && NTM < 4) || paged || __builtin_expect(blocks > FEW * NW, 1)) stream(std::integral_constant<int, NTM>{});
     else if (APPEND) stream(std::integral_constant<int, FEW < 1 ? 1 : FEW>{});
     else if (NTM > 3 && blocks > 2 * NW) stream(std::integral_constant<int, APPEND || NTM < 3 ? 1 : 3>{});
     else if (NTM > 2 && blocks > NW) stream(std::integral_constant<int, APPEND || NTM < 2 ? 1 : 2>{});
