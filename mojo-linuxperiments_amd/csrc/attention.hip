@@ -619,6 +619,18 @@ int max_splits(int64_t B, int64_t Hkv, int64_t T)
     return best;
 }
 
+static bool merge_wide(int splits, int64_t rows) { return splits > 16 && splits <= 32 && rows <= 2 * compute_units(); }
+
+// How many dependent batches of loads the merge of `rows` rows makes: one for the split counts that are compiled in and in the
+// kernel for 17 to 32, one per eight splits otherwise.
+int merge_batches(int splits, int64_t rows, bool quant)
+{
+    switch (splits) {
+    case 1: case 2: case 3: case 4: case 5: case 6: case 8: case 12: case 16: return 1;
+    }
+    return !quant && merge_wide(splits, rows) ? 1 : (splits + 7) / 8;
+}
+
 // Merge of the splits' partial results [B*Hkv, splits, 4, 128] / [B*Hkv, splits, 2, 4].  oq: one workgroup per token
 // merges its Hq rows and quantizes them for the output projection (o then optionally receives the fp32 row in the
 // rotated basis); otherwise 16 rows per workgroup into o.
@@ -646,7 +658,7 @@ int32_t launch_merge(const float *part_o, const float *part_ml, float *o, int8_t
         return launch_status();
     }
     const int rows = (int)(B * Hq);
-    if (splits > 16 && splits <= 32 && rows <= 2 * compute_units()) {
+    if (merge_wide(splits, rows)) {
         hipLaunchKernelGGL(k_gqa_merge_wide, dim3((unsigned)((rows + 1) / 2)), dim3(64), 0, s, part_o, part_ml, o, rows,
                            (int)Hq, (int)Hkv, G, splits, out_rotated);
         return launch_status();

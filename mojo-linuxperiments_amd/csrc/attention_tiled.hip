@@ -35,6 +35,7 @@
 namespace mi {
 namespace attn {
 int max_splits(int64_t B, int64_t Hkv, int64_t T);   // the row-major layout's plan: the largest split count for any length up to T
+int merge_batches(int splits, int64_t rows, bool quant);
 int32_t launch_merge(const float *part_o, const float *part_ml, float *o, int8_t *oq, float *oscale, int64_t B,
                      int64_t Hq, int64_t Hkv, int splits, int out_rotated, hipStream_t s);
 }
@@ -687,14 +688,17 @@ int max_splits(int64_t B, int64_t Hkv, int64_t T);
 
 // How many spans a row is cut into, of equal length but for the last.  Where 16 blocks a workgroup (four a wave) do not give
 // every compute unit a workgroup: as many as it takes to get there.  Else the count whose busiest unit is done first, at four
-// blocks a wave or fewer: workgroups a unit times the blocks that a workgroup streams (a multiple of four) and C0 more for
-// its start and end; the merge counts as MERGE blocks of a unit, and a finer cut has to promise a tenth (for a twentieth, mixed
-// lengths lose what equal ones gain: 20 sequences of up to 3907 tokens 0.96 and 1.05 times the time).  us with spans of 16 blocks
-// -> here: 24 sequences of 3001 tokens 35.2 -> 31.3, of 750 to 3001 in pages 29.0 -> 24.7, 12 of 2500 21.4 -> 16.2, 25 of 600 to
-// 2400 25.0 -> 19.7, 32 of 318 9.5 -> 7.1; 16 of 4096 are two workgroups a unit either way, 28.7.
-static Plan pick(int64_t B, int64_t Hkv, int64_t T)
+// blocks a wave or fewer: workgroups a unit times the blocks that a workgroup streams and START more for its start and end; the
+// merge counts as MERGE blocks of a unit, a quarter more for every span and BATCH for every further batch of loads that it makes,
+// and a finer cut has to promise a tenth (for a twentieth, mixed lengths lose what equal ones gain: 20 sequences of up to 3907
+// tokens 0.96 and 1.05 times the time).  Fitted to timings of all cuts of 92 shapes, 500 to 60000 tokens, equal and mixed lengths,
+// rows and codes; with what it chooses there the kernels take 0.95 of the time of spans of 16 blocks throughout, 1.08 at worst.
+// us with spans of 16 blocks -> here: 24 sequences of 3001 tokens 35.2 -> 31.3, of 750 to 3001 in pages 29.0 -> 24.7, 12 of 2500
+// 21.4 -> 16.2, 25 of 600 to 2400 25.0 -> 19.7, 32 of 318 9.5 -> 7.1; 16 of 4096 are two workgroups a unit either way, 28.7.
+// Without BATCH three sequences of 32768 were cut into 64 spans instead of 32: 39.4 instead of 25.0, the merge alone 15 more.
+static Plan pick(int64_t B, int64_t Hq, int64_t Hkv, int64_t T, bool quant)
 {
-    constexpr int C0 = 2, MERGE = 5;
+    constexpr int START = 3, MERGE = 5, BATCH = 4;
     const int blocks = (int)((T + 63) / 64);
     const int64_t rows = B * Hkv, cus = compute_units();
     Plan pl;
@@ -704,16 +708,26 @@ static Plan pick(int64_t B, int64_t Hkv, int64_t T)
         cut((int)std::min<int64_t>((cus + rows - 1) / rows, blocks));
         return pl;
     }
+    // (a span takes whole rounds of its waves: one of 13 blocks is as long as one of 16, and loads blocks of the next.  31 sequences
+    // of 3199 tokens in pages 24.3 us in spans of 16, 16, 16 and 2 blocks, 26.0 in 13, 13, 13 and 11)
+    auto cut4 = [&](int s) { pl.per = ((blocks + s - 1) / s + 3) / 4 * 4, pl.splits = (blocks + pl.per - 1) / pl.per; };
+    auto cost = [&]() -> int64_t {   // in quarters
+        const int64_t stream = (rows * pl.splits + cus - 1) / cus * (pl.per + START);
+        const int merge = pl.splits > 1 ? MERGE + BATCH * (attn::merge_batches(pl.splits, B * Hq, quant) - 1) : 0;
+        return 4 * (stream + merge) + (pl.splits > 1 ? pl.splits : 0);
+    };
     // (no more of them than the workspace was sized for before)
     const int most = std::min(std::max(max_splits(B, Hkv, T), attn::max_splits(B, Hkv, T)), (blocks + 7) / 8);
+    cut4(fewest);
     int best = fewest;
-    int64_t best_cost = INT64_MAX;
-    for (int s = fewest; s <= std::max(fewest, most); ++s) {
-        cut(s);
-        const int64_t cost = (rows * pl.splits + cus - 1) / cus * ((pl.per + 3) / 4 * 4 + C0) + (pl.splits > 1 ? MERGE : 0);
-        if (best_cost == INT64_MAX || 10 * cost < 9 * best_cost) best = s, best_cost = cost;
+    const int64_t first = cost();
+    int64_t best_cost = first;
+    for (int s = fewest + 1; s <= most; ++s) {
+        cut4(s);
+        const int64_t c = cost();
+        if (10 * c < 9 * first && c < best_cost) best = s, best_cost = c;
     }
-    cut(best);
+    cut4(best);
     return pl;
 }
 
@@ -768,7 +782,7 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
         return MI_EINVAL;
     if (seq_len && !aligned4(seq_len)) return MI_EINVAL;
     if (workspace_bytes < mi_gqa_decode_workspace_bytes(B, Hq, Hkv, D, T_max)) return MI_ENOSPC;
-    const avt::Plan plan = avt::pick(B, Hkv, T_max);
+    const avt::Plan plan = avt::pick(B, Hq, Hkv, T_max, oq != nullptr);
     // one workgroup sees the whole sequence: it writes the output rows (the gate takes the split form: it wants no o)
     const bool direct = plan.splits == 1 && !oq && !dbg;
     avt::StepParams p = {};

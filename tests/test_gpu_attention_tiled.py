@@ -159,6 +159,15 @@ def test_vt_spans_of_every_length(mi, dev, orc, B, Hq, Hkv, T_cap, spread):
         assert np.max(np.abs(o[b] - oo[0])) <= 2e-5, (b, n)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,T_cap,spread", [
+    (4, 8, 8, 10240, 700),     # ten or more spans of one row: merges of one batch of loads and of several
+    (31, 4, 4, 3200, 100),     # three of 16 blocks and one of two
+    (30, 8, 8, 1856, 300),     # 16 and 13
+])
+def test_vt_spans_of_whole_rounds_of_blocks(mi, dev, orc, B, Hq, Hkv, T_cap, spread):
+    test_vt_spans_of_every_length(mi, dev, orc, B, Hq, Hkv, T_cap, spread)
+
+
 def test_vt_peaked_and_flat_softmax(mi, dev, orc):
     """The fixed-point weights at their extremes: one token takes all the weight (its key is the query scaled up),
     and all tokens weigh the same (identical keys); V scales spread over three decades inside one span."""
