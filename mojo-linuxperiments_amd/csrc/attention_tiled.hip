@@ -159,7 +159,7 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
     if constexpr (APPEND) splits = p.splits;
     else splits = gridDim.x;
     const int64_t pbase = (int64_t)bkv * splits + split;
-    const bool paged = !APPEND && p.block_table;   // (the step's cache is a dense one)
+    const bool paged = p.block_table;
 
     int T = p.T;
     if (p.seq_len) T = min(max(__builtin_amdgcn_readfirstlane(p.seq_len[b]), 0), p.T);
