@@ -30,27 +30,13 @@
 
 #include "common.h"
 #include "gemm_deep.h"
+#include "lds_ops.h"
 
 namespace mi {
 namespace deep {
 
-typedef __attribute__((address_space(3))) void *lptr_t;
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));   // four scales: a batch asks only 4 bytes of alignment of them
 
-template <int N>
-__device__ __forceinline__ void wait_vm()
-{
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-// direct-to-LDS load of 16 bytes per lane: global address = sbase + voff, LDS address = ldsaddr + 16 * lane
-__device__ __forceinline__ void dma16(const int8_t *sbase, unsigned voff, unsigned ldsaddr)
-{
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(sbase), "s"(ldsaddr)
-                 : "memory", "m0");
-}
-__device__ __forceinline__ int ror8(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, false); }
 
 template <int TM_, int TN_, int WM_, int WN_, int WK_, int D_>
 struct Cfg {

@@ -101,7 +101,7 @@ struct Cfg {
 __device__ __forceinline__ void dma16(const int8_t *sbase, unsigned voff, unsigned ldsaddr)
 {
     asm volatile("s_nop 4" ::: "memory");
-    pair::dma16(sbase, voff, ldsaddr);
+    mi::dma16(sbase, voff, ldsaddr);
 }
 #endif
 #ifdef MI_GEMM_TIMELINE

@@ -1,36 +1,12 @@
-// Instruction-level pieces shared by the eight-wave GEMM kernels (gemm_pair.hip, gemm_list.hip): explicit LDS
-// fragment reads, direct-to-LDS loads, and matrix instructions on hand-numbered accumulation registers.
+// Instruction-level pieces shared by the eight-wave GEMM kernels (gemm_pair.hip, gemm_list.hip): matrix
+// instructions on hand-numbered accumulation registers.
 #pragma once
 #include "common.h"
+#include "lds_ops.h"
 
 namespace mi {
 namespace pair {
 
-typedef __attribute__((address_space(3))) void *lptr_t;
-
-template <int N>
-__device__ __forceinline__ void wait_lgkm()
-{
-    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_vm()
-{
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-template <int OFF>
-__device__ __forceinline__ void ds_read128(v4i &dst, unsigned addr)
-{
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
-}
-// direct-to-LDS load of 16 bytes per lane: global address = sbase + voff, LDS address = ldsaddr + 16 * lane
-__device__ __forceinline__ void dma16(const int8_t *sbase, unsigned voff, unsigned ldsaddr)
-{
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(sbase), "s"(ldsaddr)
-                 : "memory", "m0");
-}
 // accumulator (j, i) lives in a[4*(j*TM+i) .. +3]
 template <int LO>
 __device__ __forceinline__ void mfma_acc(const v4i &a, const v4i &b)
@@ -114,7 +90,6 @@ __device__ __forceinline__ v4i acc_plus(const v4i &o)
     return r;
 }
 }  // namespace vacc
-__device__ __forceinline__ int ror8(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, false); }
 
 template <bool DEQ>
 __device__ __forceinline__ void store4(float *y, int32_t *acc_out, int64_t idx, const v4i &v, float sxm, const float4 &s4)

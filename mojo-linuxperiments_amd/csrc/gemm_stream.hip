@@ -23,33 +23,10 @@
 // scales over those of the tile in work, before its end has read them.  So a tile has more stages than the ring has buffers).
 #include "common.h"
 #include "gemm_stream.h"
+#include "lds_ops.h"
 
 namespace mi {
 namespace stream {
-
-typedef __attribute__((address_space(3))) void *lptr_t;
-
-template <int N>
-__device__ __forceinline__ void wait_vm()
-{
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-// direct-to-LDS loads of 16 and of 4 bytes per lane: global address = sbase + voff, LDS address = ldsaddr + 16 (4) * lane
-__device__ __forceinline__ void dma16(const int8_t *sbase, unsigned voff, unsigned ldsaddr)
-{
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(sbase), "s"(ldsaddr)
-                 : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(const float *sbase, unsigned voff, unsigned ldsaddr)
-{
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
-                 :
-                 : "v"(voff), "s"(sbase), "s"(ldsaddr)
-                 : "memory", "m0");
-}
-__device__ __forceinline__ int ror8(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, false); }
 
 template <int TM_, int TN_, int WM_, int WN_, int D_>
 struct Cfg {

@@ -58,33 +58,13 @@
 #include <utility>
 
 #include "common.h"
+#include "lds_ops.h"
 
 namespace mi {
-
-typedef const __attribute__((address_space(1))) void *gptr_t;
-typedef __attribute__((address_space(3))) void *lptr_t;
 
 __device__ __forceinline__ void mfma_i8(v4i &acc, const v4i &a, const v4i &b)
 {
     asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-}
-template <int N>
-__device__ __forceinline__ void wait_lgkm()
-{
-    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
-}
-template <int OFF>
-__device__ __forceinline__ void ds_read128(v4i &dst, unsigned addr)
-{
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
-}
-// direct-to-LDS load of 16 bytes per lane: global address = sbase + voff, LDS address = ldsaddr + 16 * lane
-__device__ __forceinline__ void dma16(const int8_t *sbase, unsigned voff, unsigned ldsaddr)
-{
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(sbase), "s"(ldsaddr)
-                 : "memory", "m0");
 }
 // how many second-half activation fragments are fetched during group g of the first half
 template <int TM, int TN>
@@ -95,7 +75,6 @@ constexpr int xb1_count(int g)
         if (i * TN / TM == g) ++c;
     return c;
 }
-__device__ __forceinline__ int ror8(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, false); }
 
 struct GemmGrid {
     int tiles_m, tiles_n;

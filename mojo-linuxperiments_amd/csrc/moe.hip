@@ -17,6 +17,7 @@
 //
 // Bound: HBM on the int8 expert weights, E * 3 * H * I bytes per layer call.
 #include "common.h"
+#include "lds_ops.h"
 #include "fwht_core.h"
 
 namespace mi {
@@ -529,24 +530,6 @@ __global__ __launch_bounds__(1024) void k_moe_topk_dispatch(const float *__restr
 // (weights and gathered activation rows alike; a load shaped like an MFMA fragment, 16 rows x 64 bytes, runs
 // at a third of the bandwidth), XOR-swizzled so that the v_mfma_i32_16x16x64_i8 fragment reads are conflict
 // free.  No barrier inside the stream; partial accumulators of the four waves meet in LDS.
-typedef const __attribute__((address_space(1))) void *gptr_t;
-typedef __attribute__((address_space(3))) void *lptr_t;
-template <int N>
-__device__ __forceinline__ void wait_vm()
-{
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// direct-to-LDS load of 16 bytes per lane: global address = sbase + voff, LDS address = ldsaddr + 16 * lane.  As an asm
-// statement: in front of an LDS atomic the compiler waits for every such load in flight that it knows of.
-__device__ __forceinline__ void dma16(const int8_t *sbase, unsigned voff, unsigned ldsaddr)
-{
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(sbase), "s"(ldsaddr)
-                 : "memory", "m0");
-}
-
 constexpr int MT = 2;             // 16-token fragments per pass
 constexpr int NGRP = 2;           // 16-row weight groups per workgroup
 constexpr int RING = 2;           // stages per wave
@@ -716,6 +699,7 @@ __global__ __launch_bounds__(256) void k_moe_expert_gemm(const int8_t *__restric
 // The same contraction with the activation fragments held in registers (possible when a wave's K slice is at
 // most NSMAX steps of 128 bytes): only weights travel through the ring, twice as many of them are in flight
 // for the same LDS, and a workgroup walks several row chunks against one set of activation registers.
+// Its direct-to-LDS loads are asm statements: in front of an LDS atomic the compiler waits for every one in flight that it knows of.
 // Stages in flight per wave.  The down kernel by itself, traced at 512 tokens and a router's own counts, takes 59.1 us with four,
 // 58.5 with three, 57.6 with two; the layer that it is part of 186.5, 187.0 and 188.4 (with two, 3 % less to 1 % more elsewhere).
 constexpr int RX_RING = 4;
