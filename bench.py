@@ -445,7 +445,8 @@ def main():
 def pmc_probe(mi, wl):
     """Three launches each of: the rotation-only kernel on fp32 [2048,14336] (reads and writes exactly
     117,440,512 B: the calibration for the FETCH_SIZE / WRITE_SIZE counters), the single-problem GEMMs on the cfg3
-    shapes and the batched GEMM over all four (k_w8a8_list), the decode GEMV (M=1, 4096->14336), decode attention (cfg2) and the MoE layer (cfg4)."""
+    shapes and the batched GEMM over all four (k_w8a8_list), the same for 509 rows (k_w8a8_stream), the decode GEMV (M=1,
+    4096->14336) and the linear with it (k_gemv_row), decode attention (cfg2) and the MoE layer (cfg4)."""
     lib = mi.lib
     dev = mi.Device(arena_bytes=8 << 30)
     M = wl.PREFILL_M
@@ -469,10 +470,20 @@ def pmc_probe(mi, wl):
         if name == "gate":
             for _ in range(3):
                 mi.check(lib.mi_w8a8_gemm_dequant_f32(qx.ptr, sx.ptr, qw.ptr, sw.ptr, y.ptr, 1, N, K, None))
+            ws = dev.empty(lib.mi_w8a8_linear_workspace_bytes(1, N, K), np.uint8)
+            for _ in range(3):
+                mi.check(lib.mi_w8a8_linear_f32(a.ptr, qw.ptr, sw.ptr, y.ptr, 1, N, K, 128, ws.ptr, ws.nbytes, None))
         dev.sync()
     batch = mi.GemmBatch(dev, [(M, N, K) for _, K, N in wl.PROJECTIONS])   # the four contractions as one launch
     for _ in range(3):
         batch.run_f32(bops)
+    dev.sync()
+    few = 509
+    batch = mi.GemmBatch(dev, [(few, N, K) for _, K, N in wl.PROJECTIONS])   # their first rows
+    rows = lambda b: b.offset(0, (few,) + b.shape[1:], b.dtype)  # noqa: E731
+    fops = [(rows(qx), rows(sx), qw, sw, rows(out)) for qx, sx, qw, sw, out in bops]
+    for _ in range(3):
+        batch.run_f32(fops)
     dev.sync()
     timer = Timer(mi, None)
     print(json.dumps({"probe": "done", "attention": decode_attention(mi, wl, dev, None, timer, reps=1, graph=False),

@@ -13,8 +13,9 @@
 // A tile that would cross the edge of its matrix is moved inwards, as in gemm_list.hip.
 //
 // What bounds it.  A stage takes 0.84 us on a full chip (2.55 POP/s), 0.71 without its loads, 0.63 with neither loads nor
-// fragment reads on an otherwise idle chip, for 0.43 of matrix instructions at 2.4 GHz: the loads' share of the issue slots and
-// the part's power limit.  A tile's end costs about ten stages when every unit stores its 128 KB at once.  256 x 256 tiles move
+// fragment reads on an otherwise idle chip (variants of the kernel that are not kept), for 0.43 of matrix instructions at 2.4 GHz:
+// the loads' share of the issue slots and the part's power limit.  A whole launch of the four projections with 509 rows keeps the
+// matrix pipe busy 43 % of its clocks at 2.06 GHz and fetches 252 MB for 215 MB of operands.  A tile's end costs about ten stages when every unit stores its 128 KB at once.  256 x 256 tiles move
 // fewer bytes per result and are 1.2 times as fast where there are enough of them; 128 x 128 tiles in this form were slower
 // than both (four projections with 509 rows 144 us, this kernel 115, 256 x 256 and small tiles in two launches 135).
 //

@@ -354,10 +354,10 @@ static void start_row(int cus, int per_wave, const float *x, const int8_t *qw, c
 
 // Where the one kernel is the faster form, against making the codes and contracting them one behind the other: linear, norm and
 // SwiGLU, 20 K from 128 to 16384, whole chunks and not, 16 to 131072 rows, weights from HBM.  Up to eight rows a wave 0.57 to 1.04
-// of their time (6144 x 5120 11.9 -> 8.7 us, 4096 x 12288 with the norm 17.1 -> 14.6; no gain for 16 rows of 16384).  Up to twenty 0.77 to 1.00 from K = 1024 to
-// 8192; shorter rows lose the time that a row costs beside its bytes (28672 x 640 8.3 -> 8.5), longer ones stream no better than in
-// the GEMV by itself (28672 x 14336 72.6 -> 74.0 with SwiGLU).  Beyond, 0.93 to 0.97 in two to four whole chunks (131072 x 2048 49.4
-// -> 44.0), up to 1.14 elsewhere.
+// of their time (6144 x 5120 11.9 -> 8.7 us, 4096 x 12288 with the norm 17.1 -> 14.6; no gain for 16 rows of 16384).  Up to twenty
+// 0.77 to 1.00 from K = 1024 to 8192; shorter rows lose the time that a row costs beside its bytes (28672 x 640 8.3 -> 8.5), longer
+// ones stream no better than in the GEMV by itself (28672 x 14336 72.6 -> 74.0 with SwiGLU).  Beyond, 0.93 to 0.97 in two to four
+// whole chunks (131072 x 2048 49.4 -> 44.0), up to 1.14 elsewhere.
 bool row_takes(int64_t N, int64_t K)
 {
     const int64_t cus = compute_units();

@@ -309,7 +309,7 @@ def test_fused_swiglu_quant_equals_the_two_calls(mi, dev, orc, M, I, block):
 def test_one_token_kernel_equals_the_separate_calls(mi, dev, N, K):
     """The GEMV that makes its own codes, with fewer rows than waves, one to seven a wave and shares that differ by one: the
     linear and SwiGLU + linear give the codes, the scale, the activated row and the results of the separate calls, bit for bit;
-    with an output on top of the input they are two launches, and the same."""
+    with an output on top of the input they are two launches, and the same (as are the most rows of the longest K)."""
     mark = dev.mark()
     g = np.random.default_rng(N + K)
     gu = dev.upload((2 * g.standard_normal((1, 2 * K))).astype(np.float32))
