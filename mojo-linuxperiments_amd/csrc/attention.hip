@@ -201,14 +201,8 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
     // ---- query heads of this group: every wave rotates and quantizes them for itself (no workgroup barrier)
     {
         float v[8] = {qlo.x, qlo.y, qlo.z, qlo.w, qhi.x, qhi.y, qhi.z, qhi.w};
-        fwht128(v, jj);
-        float a = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) a = fmaxf(a, fabsf(v[e]));
-        a = fmaxf(a, lane_xor<1>(a));
-        a = fmaxf(a, lane_xor<2>(a));
-        a = fmaxf(a, lane_xor<4>(a));
-        a = fmaxf(a, lane_xor<8>(a));
+        fwht_codes<D>(v, jj);
+        const float a = max_lanes<16>(abs8(v));
         const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
         const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
         const uint32_t c0 = quant4(v[0], v[1], v[2], v[3], inv), c1 = quant4(v[4], v[5], v[6], v[7], inv);
@@ -561,11 +555,9 @@ __global__ __launch_bounds__(1024) void k_gqa_merge_quant(const float *__restric
     const int kvh = h / G, hl = h % G;
     float v[8];
     merge_row<SP>(part_o, part_ml, splits_rt, (int64_t)b * Hkv + kvh, hl, j, v);
-    float a = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) a = fmaxf(a, fabsf(v[e]));
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) a = fmaxf(a, __shfl_xor(a, off, 64));
+    float a = max_lanes<16>(abs8(v));
+    a = fmaxf(a, __shfl_xor(a, 16, 64));   // (a last wave may hold fewer than four heads)
+    a = fmaxf(a, __shfl_xor(a, 32, 64));
     if (lane == 0) s_max[wave] = a;
     __syncthreads();
     const int nwave = (int)(blockDim.x >> 6);

@@ -116,12 +116,6 @@ __device__ __forceinline__ void store_token(bool is_v, int j, int tp, int64_t bl
     }
 }
 
-template <int MASK>
-__device__ __forceinline__ float fmax_xor(float v)
-{
-    return fmaxf(v, xor_lane<MASK>(v));
-}
-
 // NW: waves per workgroup; NT: blocks per wave; RING: 1 KB loads a wave keeps in flight (8 or 16).
 // DIRECT: the workgroup covers the whole sequence (one split): it normalizes and writes the output rows itself and
 // no partial result leaves the chip.
@@ -183,9 +177,8 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
             if (!is_v)
                 rope8(v, *reinterpret_cast<const float4 *>(p.cs + (int64_t)tp * (D / 2) + 4 * j),
                       *reinterpret_cast<const float4 *>(p.sn + (int64_t)tp * (D / 2) + 4 * j));
-            fwht_chunk<D>(v, j);
-            float a = abs8(v);
-            a = fmax_xor<1>(a); a = fmax_xor<2>(a); a = fmax_xor<4>(a); a = fmax_xor<8>(a);
+            fwht_codes<D>(v, j);
+            const float a = max_lanes<16>(abs8(v));
             const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
             const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
             const int64_t blk0 = (int64_t)bkv * p.Tstride + (tp & ~63);
@@ -323,8 +316,7 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
         float vm = 0.0f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) vm = fmaxf(vm, (t_lo + sidx + e < t_end && (!APPEND || t_lo + sidx + e != tp)) ? v[e] : 0.0f);
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) vm = fmaxf(vm, __shfl_xor(vm, off, 64));
+        vm = max_lanes<64>(vm);
         if (APPEND && owner && tp < t_end) vm = fmaxf(vm, new_vs);
         if (sidx < SPAN) {
             *reinterpret_cast<float4 *>(s_ks + sidx) = ks4;
@@ -345,9 +337,8 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
                 }
             }
         }
-        fwht_chunk<D>(v, jj);
-        float a = abs8(v);
-        a = fmax_xor<1>(a); a = fmax_xor<2>(a); a = fmax_xor<4>(a); a = fmax_xor<8>(a);
+        fwht_codes<D>(v, jj);
+        const float a = max_lanes<16>(abs8(v));
         const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
         const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
         const uint32_t c0 = quant4(v[0], v[1], v[2], v[3], inv), c1 = quant4(v[4], v[5], v[6], v[7], inv);
@@ -662,10 +653,8 @@ __global__ __launch_bounds__(256) void k_kv_append_vt(const float *__restrict__ 
             }
         }
     }
-    fwht_chunk<D>(v, j);   // every lane takes part in the cross-lane stages
-    float a = abs8(v);
-#pragma unroll
-    for (int m = LPB / 2; m >= 1; m >>= 1) a = fmaxf(a, __shfl_xor(a, m, 64));
+    fwht_codes<D>(v, j);   // every lane takes part in the cross-lane stages
+    const float a = max_lanes<LPB>(abs8(v));
     const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
     const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
     if (live && !is_q) {

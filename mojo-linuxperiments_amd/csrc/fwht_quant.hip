@@ -52,7 +52,8 @@ __device__ __forceinline__ void fwht_row_body(const float *x, int8_t *__restrict
     float amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < C; ++i) {
-        fwht_chunk<BLOCK>(v[i], j);
+        if constexpr (QUANT) fwht_codes<BLOCK>(v[i], j);
+        else fwht_chunk<BLOCK>(v[i], j);
         amax = fmaxf(amax, abs8(v[i]));
     }
 
@@ -68,8 +69,7 @@ __device__ __forceinline__ void fwht_row_body(const float *x, int8_t *__restrict
     } else {
         // row absmax: wave butterfly, then across waves through LDS
         __shared__ float s_max[16];
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+        amax = max_lanes<64>(amax);
         const int wave = t >> 6, nwave = (T + 63) >> 6;
         if ((t & 63) == 0) s_max[wave] = amax;
         __syncthreads();
@@ -167,7 +167,8 @@ __global__ __launch_bounds__(256) void k_fwht_wave(const float *x, int8_t *__res
     float amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < C; ++i) {
-        fwht_chunk<BLOCK>(v[i], j);
+        if constexpr (QUANT) fwht_codes<BLOCK>(v[i], j);
+        else fwht_chunk<BLOCK>(v[i], j);
         amax = fmaxf(amax, abs8(v[i]));
     }
     if constexpr (!QUANT) {
@@ -180,8 +181,7 @@ __global__ __launch_bounds__(256) void k_fwht_wave(const float *x, int8_t *__res
             }
         }
     } else {
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+        amax = max_lanes<64>(amax);
         const float sc = (amax == 0.0f) ? 1.0f : amax / 127.0f;
         const float inv = (amax == 0.0f) ? 0.0f : 127.0f / amax;
         if (lane == 0) scale[row] = sc;
@@ -219,7 +219,8 @@ __global__ __launch_bounds__(256) void k_fwht_small(const float *x, int8_t *__re
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = 0.0f;
     }
-    fwht_chunk<BLOCK>(v, j);
+    if constexpr (QUANT) fwht_codes<BLOCK>(v, j);
+    else fwht_chunk<BLOCK>(v, j);
     if constexpr (!QUANT) {
         if (live) {
             *reinterpret_cast<float4 *>(xrot + off) = make_float4(v[0], v[1], v[2], v[3]);
@@ -227,8 +228,7 @@ __global__ __launch_bounds__(256) void k_fwht_small(const float *x, int8_t *__re
         }
     } else {
         float a = abs8(v);
-#pragma unroll
-        for (int m = LPB / 2; m >= 1; m >>= 1) a = fmaxf(a, __shfl_xor(a, m, 64));
+        a = max_lanes<LPB>(a);
         const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
         const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
         if (live) {
@@ -267,10 +267,8 @@ __global__ __launch_bounds__(256) void k_kv_append(const float *__restrict__ k_n
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = 0.0f;
     }
-    fwht_chunk<BLOCK>(v, j);
-    float a = abs8(v);
-#pragma unroll
-    for (int m = LPB / 2; m >= 1; m >>= 1) a = fmaxf(a, __shfl_xor(a, m, 64));
+    fwht_codes<BLOCK>(v, j);
+    const float a = max_lanes<LPB>(abs8(v));
     const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
     const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
     if (live) {

@@ -25,16 +25,34 @@ __device__ __forceinline__ void fold_sum(int (&p)[V], int lane)
         int q[V / 2];
 #pragma unroll
         for (int i = 0; i < V / 2; ++i) {
-            const int keep = hi ? p[i + V / 2] : p[i];
-            const int send = hi ? p[i] : p[i + V / 2];
-            q[i] = keep + __shfl_xor(send, OFF, 64);
+            if constexpr (OFF == 32) {   // the exchange that the comment above describes is one instruction
+                const auto r = __builtin_amdgcn_permlane32_swap(p[i], p[i + V / 2], false, false);
+                q[i] = (int)r[0] + (int)r[1];
+            } else if constexpr (OFF == 16) {
+                const auto r = __builtin_amdgcn_permlane16_swap(p[i], p[i + V / 2], false, false);
+                q[i] = (int)r[0] + (int)r[1];
+            } else {
+                const int keep = hi ? p[i + V / 2] : p[i];
+                const int send = hi ? p[i] : p[i + V / 2];
+                q[i] = keep + xor_lane_i<OFF>(send);
+            }
         }
         fold_sum<V / 2, OFF / 2>(q, lane);
 #pragma unroll
         for (int i = 0; i < V / 2; ++i) p[i] = q[i];
     } else {
-#pragma unroll
-        for (int off = OFF; off >= 1; off >>= 1) p[0] += __shfl_xor(p[0], off, 64);
+        if constexpr (OFF >= 32) {
+            const auto r = __builtin_amdgcn_permlane32_swap(p[0], p[0], false, false);
+            p[0] = (int)r[0] + (int)r[1];
+        }
+        if constexpr (OFF >= 16) {
+            const auto r = __builtin_amdgcn_permlane16_swap(p[0], p[0], false, false);
+            p[0] = (int)r[0] + (int)r[1];
+        }
+        if constexpr (OFF >= 8) p[0] += xor_lane_i<8>(p[0]);
+        if constexpr (OFF >= 4) p[0] += xor_lane_i<4>(p[0]);
+        if constexpr (OFF >= 2) p[0] += xor_lane_i<2>(p[0]);
+        if constexpr (OFF >= 1) p[0] += xor_lane_i<1>(p[0]);
     }
 }
 
@@ -255,7 +273,7 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
             const float up[8] = {gl[i].x, gl[i].y, gl[i].z, gl[i].w, gh[i].x, gh[i].y, gh[i].z, gh[i].w};
             if (tid + i * 512 < nchunk) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[i][e] = (v[i][e] / (1.0f + expf(-v[i][e]))) * up[e];
+                for (int e = 0; e < 8; ++e) v[i][e] = silu(v[i][e]) * up[e];
             }
         }
     }
@@ -265,11 +283,10 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
     float amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < CQ; ++i) {
-        if constexpr (OP != PLAIN) fwht_chunk<BLOCK>(v[i], j);
+        if constexpr (OP != PLAIN) fwht_codes<BLOCK>(v[i], j);
         amax = fmaxf(amax, abs8(v[i]));
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+    amax = max_lanes<64>(amax);
     if (lane == 0) s_max[wave] = amax;
     __syncthreads();
     float a = s_max[0];

@@ -37,8 +37,7 @@ __global__ __launch_bounds__(256) void k_add_rmsnorm(const float *__restrict__ x
             v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         }
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) ss += __shfl_xor(ss, off, 64);
+    ss = group_sum(ss);
     if (lane == 0) s_part[wave] = ss;
     __syncthreads();
     const float total = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
@@ -102,10 +101,8 @@ __global__ __launch_bounds__(256) void k_rope_kv_append(const float *__restrict_
         }
     }
     // every lane takes part in the cross-lane stages; query heads simply do not store
-    fwht_chunk<D>(v, j);
-    float a = abs8(v);
-#pragma unroll
-    for (int m = LPB / 2; m >= 1; m >>= 1) a = fmaxf(a, __shfl_xor(a, m, 64));
+    fwht_codes<D>(v, j);
+    const float a = max_lanes<LPB>(abs8(v));
     const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
     const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
     if (live && !is_q) {
@@ -128,10 +125,10 @@ __global__ __launch_bounds__(256) void k_swiglu(const float *__restrict__ gu, fl
     const float4 g = *reinterpret_cast<const float4 *>(gu + m * 2 * I + n);
     const float4 u = *reinterpret_cast<const float4 *>(gu + m * 2 * I + I + n);
     float4 o;
-    o.x = (g.x / (1.0f + expf(-g.x))) * u.x;
-    o.y = (g.y / (1.0f + expf(-g.y))) * u.y;
-    o.z = (g.z / (1.0f + expf(-g.z))) * u.z;
-    o.w = (g.w / (1.0f + expf(-g.w))) * u.w;
+    o.x = silu(g.x) * u.x;
+    o.y = silu(g.y) * u.y;
+    o.z = silu(g.z) * u.z;
+    o.w = silu(g.w) * u.w;
     *reinterpret_cast<float4 *>(h + i) = o;
 }
 
@@ -184,7 +181,7 @@ __global__ __launch_bounds__(TPB) void k_row_op_quant(const float *__restrict__ 
                 const float gg[8] = {gl.x, gl.y, gl.z, gl.w, gh.x, gh.y, gh.z, gh.w};
                 const float uu[8] = {ul.x, ul.y, ul.z, ul.w, uh.x, uh.y, uh.z, uh.w};
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[i][e] = (gg[e] / (1.0f + expf(-gg[e]))) * uu[e];
+                for (int e = 0; e < 8; ++e) v[i][e] = silu(gg[e]) * uu[e];
             }
         } else {
 #pragma unroll
@@ -232,11 +229,10 @@ __global__ __launch_bounds__(TPB) void k_row_op_quant(const float *__restrict__ 
     float amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < C; ++i) {
-        fwht_chunk<BLOCK>(v[i], j);
+        fwht_codes<BLOCK>(v[i], j);
         amax = fmaxf(amax, abs8(v[i]));
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+    amax = max_lanes<64>(amax);
     if (lane == 0) s_max[wave] = amax;
     __syncthreads();
     float a = s_max[0];

@@ -257,11 +257,10 @@ __global__ __launch_bounds__(256) void k_moe_logits(const float *__restrict__ x,
             float amax = 0.0f;
 #pragma unroll
             for (int i = 0; i < CQ; ++i) {
-                fwht_chunk<128>(v[i], jq);
+                fwht_codes<128>(v[i], jq);
                 amax = fmaxf(amax, abs8(v[i]));
             }
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+            amax = max_lanes<64>(amax);
             const float sc = (amax == 0.0f) ? 1.0f : amax / 127.0f;
             const float inv = (amax == 0.0f) ? 0.0f : 127.0f / amax;
             if (lane == 0) sx[qrow] = sc;
@@ -294,11 +293,10 @@ __global__ __launch_bounds__(256) void k_moe_logits(const float *__restrict__ x,
             float amax = 0.0f;
 #pragma unroll
             for (int i = 0; i < CQ; ++i) {
-                fwht_chunk<128>(v[i], jq);
+                fwht_codes<128>(v[i], jq);
                 amax = fmaxf(amax, abs8(v[i]));
             }
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+            amax = max_lanes<64>(amax);
             const float sc = (amax == 0.0f) ? 1.0f : amax / 127.0f;
             const float inv = (amax == 0.0f) ? 0.0f : 127.0f / amax;
             if (lane == 0) sx[row] = sc;
@@ -677,7 +675,7 @@ __global__ __launch_bounds__(256) void k_moe_expert_gemm(const int8_t *__restric
                 const float sxt = act_scale[perm[pos] / topk];
                 const float gv = ((float)total(0, row, nl) * sxt) * sc0[(int64_t)e * Nrows + nc0 + nl];
                 const float uv = ((float)total(1, row, nl) * sxt) * sc1[(int64_t)e * Nrows + nc0 + nl];
-                out[(int64_t)pos * Nrows + nc0 + nl] = (gv / (1.0f + expf(-gv))) * uv;
+                out[(int64_t)pos * Nrows + nc0 + nl] = silu(gv) * uv;
             }
         } else {
             // 32 tokens x 128 channels (32 per wave); out[pair] in pair order, channel fastest
@@ -879,7 +877,7 @@ __device__ __forceinline__ void rx_pass(char *smem, const int8_t *__restrict__ a
                     const float sxt = s_tsc[row];
                     const float gv = ((float)gi * sxt) * wsc[nl];
                     const float uv = ((float)ui * sxt) * wsc[16 + nl];
-                    out[(int64_t)s_dst[row] * Nrows + (c0 + ch) * 16 + nl] = (gv / (1.0f + expf(-gv))) * uv;
+                    out[(int64_t)s_dst[row] * Nrows + (c0 + ch) * 16 + nl] = silu(gv) * uv;
                 }
             }
             __syncthreads();   // the zeroes are in place before the next chunk's sums arrive

@@ -93,6 +93,23 @@ def test_swiglu_matches_oracle(mi, dev, orc, M, I):
     assert np.max(np.abs(h - want)) <= 2e-6 * max(1.0, np.max(np.abs(want)))
 
 
+def test_swiglu_at_the_ends_of_the_range(mi, dev):
+    """Gates from where e^-g vanishes to where it overflows.  An ulp of the exponential, one each of the sum, the quotient and
+    the product: 3e-7; e^-g overflows in fp32 where the result is below 3e-37."""
+    big = np.array([0.0, 1e-30, 0.5, 20.0, 87.9, 88.7, 88.8, 89.5, 90.0, 103.9, 104.1, 1e4, 1e38, np.inf, np.nan, 1e-42], np.float32)
+    g = np.concatenate([big, -big])
+    mark = dev.mark()
+    gu, h = dev.upload(np.concatenate([g, np.full(32, 1.5, np.float32)])[None]), dev.empty((1, 32), np.float32)
+    mi.check(mi.lib.mi_swiglu_f32(gu.ptr, h.ptr, 1, 32, None))
+    got = dev.download(h)[0]
+    dev.reset_to(mark)
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = 1.5 * g.astype(np.float64) / (1.0 + np.exp(-g.astype(np.float64)))
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    f = np.isfinite(want)
+    assert np.all(np.abs(got[f] - want[f]) <= 3e-7 * np.abs(want[f]) + 5e-37)
+
+
 def test_add(mi, dev):
     mark = dev.mark()
     a, b = workload.normal(1, (3, 1024), 0), workload.normal(1, (3, 1024), 1)

@@ -129,6 +129,19 @@ def test_non_finite_rows_follow_the_oracle(mi, dev, orc, M, K, block):
     assert np.array_equal(q[0], orc.rotate_quant_rows(x[:1], block)[0][0])
 
 
+@pytest.mark.parametrize("M,K,block", [(9, 4096, 128), (9, 768, 256), (1030, 512, 256), (1030, 2048, 128), (9, 128, 128), (9, 256, 256)])
+def test_rows_of_every_magnitude(mi, dev, orc, M, K, block):
+    """From denormal rows (whose 127 / absmax overflows, so that the products are clamped) to rows near the largest float:
+    every operation of the rotation and of the codes is an IEEE one, so the bits are the oracle's."""
+    x = workload.activations(8, M, K)
+    for row, size in enumerate((1e-44, 1e-41, 1e-38, 3e-37, 1e-20, 1e20, 1e35)):
+        x[row] *= np.float32(size)
+    with np.errstate(over="ignore", invalid="ignore"):
+        q, s = run_quant(mi, dev, x, block)
+        qo, so = orc.rotate_quant_rows(x, block)
+    assert np.array_equal(s, so) and np.array_equal(q, qo)
+
+
 @pytest.mark.parametrize("M,K,block", [(7, 4096, 128), (3, 768, 256), (33, 128, 128), (1027, 512, 256)])
 def test_rotation_only_bit_exact_and_in_place(mi, dev, orc, M, K, block):
     x = workload.normal(3, (M, K))
