@@ -632,8 +632,8 @@ int32_t launch_merge(const float *part_o, const float *part_ml, float *o, int8_t
     const int G = (int)(Hq / Hkv);
     if (oq) {
 #define MI_MERGEQ(SP)                                                                                           \
-    hipLaunchKernelGGL(k_gqa_merge_quant<SP>, dim3((unsigned)B), dim3((unsigned)(Hq * 16)), 0, s, part_o, part_ml, \
-                       o, oq, oscale, (int)Hq, (int)Hkv, G, splits)
+    launch_kernel(k_gqa_merge_quant<SP>, dim3((unsigned)B), dim3((unsigned)(Hq * 16)), 0, s, part_o, part_ml, \
+                  o, oq, oscale, (int)Hq, (int)Hkv, G, splits)
         switch (splits) {
         case 1: MI_MERGEQ(1); break;
         case 2: MI_MERGEQ(2); break;
@@ -651,16 +651,16 @@ int32_t launch_merge(const float *part_o, const float *part_ml, float *o, int8_t
     }
     const int rows = (int)(B * Hq);
     if (merge_wide(splits, rows)) {
-        hipLaunchKernelGGL(k_gqa_merge_wide, dim3((unsigned)((rows + 1) / 2)), dim3(64), 0, s, part_o, part_ml, o, rows,
-                           (int)Hq, (int)Hkv, G, splits, out_rotated);
+        launch_kernel(k_gqa_merge_wide, dim3((unsigned)((rows + 1) / 2)), dim3(64), 0, s, part_o, part_ml, o, rows,
+                      (int)Hq, (int)Hkv, G, splits, out_rotated);
         return launch_status();
     }
     int rpw = 16;   // rows per workgroup: fewer while that still adds workgroups below half a chip's worth
     while (rpw > 1 && rows / rpw < compute_units() / 2) rpw >>= 1;
     const dim3 mgrid((unsigned)((rows + rpw - 1) / rpw)), mblock((unsigned)(16 * rpw));
 #define MI_MERGE(SP)                                                                                              \
-    hipLaunchKernelGGL(k_gqa_merge<SP>, mgrid, mblock, 0, s, part_o, part_ml, o, rows, (int)Hq, (int)Hkv, G, \
-                       splits, out_rotated)
+    launch_kernel(k_gqa_merge<SP>, mgrid, mblock, 0, s, part_o, part_ml, o, rows, (int)Hq, (int)Hkv, G, \
+                  splits, out_rotated)
     switch (splits) {
     case 1: MI_MERGE(1); break;
     case 2: MI_MERGE(2); break;
@@ -735,11 +735,11 @@ static int32_t run_attn(const float *q, const int8_t *kq, const float *ks, const
     p.score_scale = 1.4426950408889634f * 0.08838834764831845f;  // log2(e) / sqrt(128)
     const dim3 grid((unsigned)splits, (unsigned)(B * Hkv));
     if (plan.wave_tiles == attn::TILES_LONG) {
-        if (ddots) hipLaunchKernelGGL((attn::k_gqa_split<true, attn::TILES_LONG>), grid, dim3(256), 0, s, p);
-        else hipLaunchKernelGGL((attn::k_gqa_split<false, attn::TILES_LONG>), grid, dim3(256), 0, s, p);
+        if (ddots) launch_kernel((attn::k_gqa_split<true, attn::TILES_LONG>), grid, dim3(256), 0, s, p);
+        else launch_kernel((attn::k_gqa_split<false, attn::TILES_LONG>), grid, dim3(256), 0, s, p);
     } else {
-        if (ddots) hipLaunchKernelGGL((attn::k_gqa_split<true, attn::TILES_SHORT>), grid, dim3(256), 0, s, p);
-        else hipLaunchKernelGGL((attn::k_gqa_split<false, attn::TILES_SHORT>), grid, dim3(256), 0, s, p);
+        if (ddots) launch_kernel((attn::k_gqa_split<true, attn::TILES_SHORT>), grid, dim3(256), 0, s, p);
+        else launch_kernel((attn::k_gqa_split<false, attn::TILES_SHORT>), grid, dim3(256), 0, s, p);
     }
     rc = launch_status();
     if (rc) return rc;

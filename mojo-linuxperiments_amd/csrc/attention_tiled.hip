@@ -795,7 +795,7 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
     p.blocks_per_split = plan.per;
     const dim3 grid((unsigned)plan.splits, (unsigned)(B * Hkv));
     const int nt = (plan.per + 3) / 4;
-#define MI_TILED(NT_, DIR_, APP_) hipLaunchKernelGGL((avt::k_gqa_tiled_split<4, NT_, 8, DIR_, APP_>), grid, dim3(256), 0, s, p)   // (p as its base without APPEND)
+#define MI_TILED(NT_, DIR_, APP_) launch_kernel((avt::k_gqa_tiled_split<4, NT_, 8, DIR_, APP_>), grid, dim3(256), 0, s, p)   // (p as its base without APPEND)
 #define MI_TILED_NT(DIR_, APP_) do { if (nt <= 1) MI_TILED(1, DIR_, APP_); else if (nt <= 2) MI_TILED(2, DIR_, APP_); else if (nt <= 3) MI_TILED(3, DIR_, APP_); else MI_TILED(4, DIR_, APP_); } while (0)
     if (step) { if (direct) MI_TILED_NT(true, true); else MI_TILED_NT(false, true); }
     else { if (direct) MI_TILED_NT(true, false); else MI_TILED_NT(false, false); }
@@ -915,8 +915,8 @@ extern "C" int32_t mi_kv_tiled_from_rows_i8(const int8_t *kq, const int8_t *vq, 
     if (rows > 65535 || T_cap > (1LL << 24)) return MI_ERANGE;
     const unsigned blocks = (unsigned)((T + 63) / 64);
     const dim3 grid(blocks, (unsigned)rows, (kq && vq) ? 2 : 1);
-    hipLaunchKernelGGL(avt::k_tiled_from_rows, grid, dim3(256), 0, as_stream(stream), kq, vq, kt, vt, (int)T, src_stride,
-                       T_cap, (kq ? 0 : 1));
+    launch_kernel(avt::k_tiled_from_rows, grid, dim3(256), 0, as_stream(stream), kq, vq, kt, vt, (int)T, src_stride,
+                  T_cap, (kq ? 0 : 1));
     return launch_status();
 }
 
@@ -939,9 +939,9 @@ extern "C" int32_t mi_kv_append_tiled_f32_i8(const float *k_new, const float *v_
     if (rc) return rc;
     if (row_stride < Hkv * D || row_stride % 4) return MI_EINVAL;
     const dim3 grid((unsigned)((B * Hkv + 15) / 16), 2);
-    hipLaunchKernelGGL(avt::k_kv_append_vt<false>, grid, dim3(256), 0, as_stream(stream), k_new, v_new, row_stride,
-                       (const float *)nullptr, (const float *)nullptr, (float *)nullptr, kq, ks, vt, vs, pos, (int)B, 0,
-                       (int)Hkv, (int)T_cap, (const int32_t *)nullptr, 0);
+    launch_kernel(avt::k_kv_append_vt<false>, grid, dim3(256), 0, as_stream(stream), k_new, v_new, row_stride,
+                  (const float *)nullptr, (const float *)nullptr, (float *)nullptr, kq, ks, vt, vs, pos, (int)B, 0,
+                  (int)Hkv, (int)T_cap, (const int32_t *)nullptr, 0);
     return launch_status();
 }
 
@@ -955,9 +955,9 @@ extern "C" int32_t mi_rope_kv_append_tiled_f32_i8(const float *qkv, int64_t row_
     if (!rope_cos || !rope_sin || !aligned16(rope_cos) || !aligned16(rope_sin) || Hq <= 0) return MI_EINVAL;
     if (row_stride < (Hq + 2 * Hkv) * D || row_stride % 4) return MI_EINVAL;
     const int64_t heads = B * (Hq + 2 * Hkv);
-    hipLaunchKernelGGL(avt::k_kv_append_vt<true>, dim3((unsigned)((heads + 15) / 16)), dim3(256), 0, as_stream(stream),
-                       qkv, (const float *)nullptr, row_stride, rope_cos, rope_sin, q_out, kq, ks, vt, vs, pos, (int)B,
-                       (int)Hq, (int)Hkv, (int)T_cap, (const int32_t *)nullptr, 0);
+    launch_kernel(avt::k_kv_append_vt<true>, dim3((unsigned)((heads + 15) / 16)), dim3(256), 0, as_stream(stream),
+                  qkv, (const float *)nullptr, row_stride, rope_cos, rope_sin, q_out, kq, ks, vt, vs, pos, (int)B,
+                  (int)Hq, (int)Hkv, (int)T_cap, (const int32_t *)nullptr, 0);
     return launch_status();
 }
 
@@ -1027,9 +1027,9 @@ extern "C" int32_t mi_kv_append_tiled_paged_f32_i8(const float *k_new, const flo
     if (rc) return rc;
     if (row_stride < Hkv * D || row_stride % 4) return MI_EINVAL;
     const dim3 grid((unsigned)((B * Hkv + 15) / 16), 2);
-    hipLaunchKernelGGL(avt::k_kv_append_vt<false>, grid, dim3(256), 0, as_stream(stream), k_new, v_new, row_stride,
-                       (const float *)nullptr, (const float *)nullptr, (float *)nullptr, kt_pool, ks_pool, vt_pool,
-                       vs_pool, pos, (int)B, 0, (int)Hkv, (int)(max_pages * 64), block_table, (int)max_pages);
+    launch_kernel(avt::k_kv_append_vt<false>, grid, dim3(256), 0, as_stream(stream), k_new, v_new, row_stride,
+                  (const float *)nullptr, (const float *)nullptr, (float *)nullptr, kt_pool, ks_pool, vt_pool,
+                  vs_pool, pos, (int)B, 0, (int)Hkv, (int)(max_pages * 64), block_table, (int)max_pages);
     return launch_status();
 }
 
@@ -1046,8 +1046,8 @@ extern "C" int32_t mi_rope_kv_append_tiled_paged_f32_i8(const float *qkv, int64_
     if (!rope_cos || !rope_sin || !aligned16(rope_cos) || !aligned16(rope_sin) || Hq <= 0) return MI_EINVAL;
     if (row_stride < (Hq + 2 * Hkv) * D || row_stride % 4) return MI_EINVAL;
     const int64_t heads = B * (Hq + 2 * Hkv);
-    hipLaunchKernelGGL(avt::k_kv_append_vt<true>, dim3((unsigned)((heads + 15) / 16)), dim3(256), 0, as_stream(stream),
-                       qkv, (const float *)nullptr, row_stride, rope_cos, rope_sin, q_out, kt_pool, ks_pool, vt_pool,
-                       vs_pool, pos, (int)B, (int)Hq, (int)Hkv, (int)(max_pages * 64), block_table, (int)max_pages);
+    launch_kernel(avt::k_kv_append_vt<true>, dim3((unsigned)((heads + 15) / 16)), dim3(256), 0, as_stream(stream),
+                  qkv, (const float *)nullptr, row_stride, rope_cos, rope_sin, q_out, kt_pool, ks_pool, vt_pool,
+                  vs_pool, pos, (int)B, (int)Hq, (int)Hkv, (int)(max_pages * 64), block_table, (int)max_pages);
     return launch_status();
 }

@@ -292,7 +292,7 @@ static int32_t launch_rows(const float *x, int8_t *q, float *scale, float *xrot,
     if (K == BLOCK) {
         constexpr int ROWS = 256 / (BLOCK / 8);
         const int64_t grid = (M + ROWS - 1) / ROWS;
-        hipLaunchKernelGGL((k_fwht_small<BLOCK, QUANT>), dim3((unsigned)grid), dim3(256), 0, s, x, q, scale, xrot, M);
+        launch_kernel((k_fwht_small<BLOCK, QUANT>), dim3((unsigned)grid), dim3(256), 0, s, x, q, scale, xrot, M);
         return launch_status();
     }
     const int nchunk = (int)(K / 8);
@@ -301,7 +301,7 @@ static int32_t launch_rows(const float *x, int8_t *q, float *scale, float *xrot,
         const dim3 grid((unsigned)((M + 3) / 4));
         const int CW = (nchunk + 63) / 64;
 #define MI_WAVE_CASE(CC)                                                                                    \
-    hipLaunchKernelGGL((k_fwht_wave<BLOCK, CC, QUANT>), grid, dim3(256), 0, s, x, q, scale, xrot, (int)K, M)
+    launch_kernel((k_fwht_wave<BLOCK, CC, QUANT>), grid, dim3(256), 0, s, x, q, scale, xrot, (int)K, M)
         if (CW <= 1) MI_WAVE_CASE(1);
         else if (CW <= 2) MI_WAVE_CASE(2);
         else MI_WAVE_CASE(4);
@@ -312,7 +312,7 @@ static int32_t launch_rows(const float *x, int8_t *q, float *scale, float *xrot,
     const int C = (nchunk + T - 1) / T;
     const dim3 grid((unsigned)M), blk((unsigned)T);
 #define MI_ROWS_CASE(CC)                                                                                   \
-    hipLaunchKernelGGL((k_fwht_rows<BLOCK, CC, QUANT>), grid, blk, 0, s, x, q, scale, xrot, (int)K)
+    launch_kernel((k_fwht_rows<BLOCK, CC, QUANT>), grid, blk, 0, s, x, q, scale, xrot, (int)K)
     if (C <= 1) MI_ROWS_CASE(1);
     else if (C <= 2) MI_ROWS_CASE(2);
     else if (C <= 4) MI_ROWS_CASE(4);
@@ -382,7 +382,7 @@ extern "C" int32_t mi_fwht_quant_batch_f32_i8(const mi_quant_rows *sets, int32_t
     int cmax = 1;
     for (int i = 0; i < n; ++i) cmax = std::max(cmax, (b.s[i].K / 8 + 255) / 256);
 #define MI_QBATCH(BLOCK_, CMAX_) \
-    hipLaunchKernelGGL((k_fwht_rows_batch<BLOCK_, CMAX_>), dim3((unsigned)rows), dim3(256), 0, as_stream(stream), b)
+    launch_kernel((k_fwht_rows_batch<BLOCK_, CMAX_>), dim3((unsigned)rows), dim3(256), 0, as_stream(stream), b)
     if (block == 128) {
         if (cmax <= 2) MI_QBATCH(128, 2);
         else if (cmax <= 4) MI_QBATCH(128, 4);
@@ -410,8 +410,8 @@ extern "C" int32_t mi_kv_append_f32_i8(const float *k_new, const float *v_new, i
         !aligned4(pos))
         return MI_EINVAL;
     const dim3 grid((unsigned)((B * Hkv + 15) / 16), 2);
-    hipLaunchKernelGGL(k_kv_append, grid, dim3(256), 0, as_stream(stream), k_new, v_new, row_stride, kq, ks, vq, vs,
-                       pos, (int)B, (int)Hkv, (int)T_cap, (const int32_t *)nullptr, 0, 0);
+    launch_kernel(k_kv_append, grid, dim3(256), 0, as_stream(stream), k_new, v_new, row_stride, kq, ks, vq, vs,
+                  pos, (int)B, (int)Hkv, (int)T_cap, (const int32_t *)nullptr, 0, 0);
     return launch_status();
 }
 
@@ -432,9 +432,9 @@ extern "C" int32_t mi_kv_append_paged_f32_i8(const float *k_new, const float *v_
     while ((1LL << shift) < page_size) ++shift;
     const dim3 grid((unsigned)((B * Hkv + 15) / 16), 2);
     // positions are valid inside the sequence's table: [0, max_pages * page_size)
-    hipLaunchKernelGGL(k_kv_append, grid, dim3(256), 0, as_stream(stream), k_new, v_new, row_stride, kq_pool, ks_pool,
-                       vq_pool, vs_pool, pos, (int)B, (int)Hkv, (int)(max_pages * page_size), block_table,
-                       (int)max_pages, shift);
+    launch_kernel(k_kv_append, grid, dim3(256), 0, as_stream(stream), k_new, v_new, row_stride, kq_pool, ks_pool,
+                  vq_pool, vs_pool, pos, (int)B, (int)Hkv, (int)(max_pages * page_size), block_table,
+                  (int)max_pages, shift);
     return launch_status();
 }
 

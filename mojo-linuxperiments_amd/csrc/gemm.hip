@@ -119,7 +119,7 @@ extern "C" int32_t mi_dequant_i32_f32(const int32_t *acc, const float *sx, const
     if (M == 0) return MI_OK;
     int64_t blocks = (M * N + 255) / 256;
     if (blocks > 8192) blocks = 8192;
-    hipLaunchKernelGGL(k_dequant, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), acc, sx, sw, y, M, N);
+    launch_kernel(k_dequant, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), acc, sx, sw, y, M, N);
     return launch_status();
 }
 

@@ -328,7 +328,7 @@ static int32_t launch_batch(Batch &b, hipStream_t s)
         if (grid > 0x7fffffff / C::TPB) return MI_ERANGE;
     }
     MI_LDS_OPT_IN((&k_w8a8_deep_batch<C, DEQ>), C::LDS);
-    hipLaunchKernelGGL((k_w8a8_deep_batch<C, DEQ>), dim3((unsigned)grid), dim3(C::TPB), C::LDS, s, b);
+    launch_kernel((k_w8a8_deep_batch<C, DEQ>), dim3((unsigned)grid), dim3(C::TPB), C::LDS, s, b);
     return launch_status();
 }
 
@@ -342,8 +342,8 @@ static int32_t launch(const int8_t *qx, const float *sx, const int8_t *qw, const
     int tiles, tiles_m;
     unsigned magic;
     if (!tile_grid(C::BM, C::BN, M, N, &tiles, &tiles_m, &magic)) return MI_ERANGE;
-    hipLaunchKernelGGL((k_w8a8_deep<C, DEQ>), dim3((unsigned)(tiles + 7) / 8 * 8), dim3(C::TPB), C::LDS, s, qx, qw, M, N, K,
-                       tiles, tiles_m, magic, sx, sw, out);
+    launch_kernel((k_w8a8_deep<C, DEQ>), dim3((unsigned)(tiles + 7) / 8 * 8), dim3(C::TPB), C::LDS, s, qx, qw, M, N, K,
+                  tiles, tiles_m, magic, sx, sw, out);
     return launch_status();
 }
 

@@ -919,8 +919,8 @@ static int32_t batch_run(mi_gemm_batch *b, const mi_gemm_problem *p, void *strea
         d.K = (int)g.K;
     }
     MI_LDS_OPT_IN((&list::k_w8a8_list<DEQ>), list::LC::LDS);
-    hipLaunchKernelGGL((list::k_w8a8_list<DEQ>), dim3((unsigned)b->grid), dim3(512), list::LC::LDS,
-                       as_stream(stream), bt, b->lists, b->per_wg);
+    launch_kernel((list::k_w8a8_list<DEQ>), dim3((unsigned)b->grid), dim3(512), list::LC::LDS,
+                  as_stream(stream), bt, b->lists, b->per_wg);
     return launch_status();
 }
 

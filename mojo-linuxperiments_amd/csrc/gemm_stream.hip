@@ -238,7 +238,7 @@ int32_t launch_stream(const StreamBatch &b, const v2i *lists, int grid, int per_
     static_assert(C::BM == 256 && C::BN == STREAM_BN, "the tiles that the lists are made of");
     static_assert(STREAM_MIN_K / 128 > C::D, "the scales of a tile are read before those of the tile after the next arrive");
     MI_LDS_OPT_IN((&stream::k_w8a8_stream<C, DEQ>), C::LDS);
-    hipLaunchKernelGGL((stream::k_w8a8_stream<C, DEQ>), dim3((unsigned)grid), dim3(512), C::LDS, s, b, lists, per_wg);
+    launch_kernel((stream::k_w8a8_stream<C, DEQ>), dim3((unsigned)grid), dim3(512), C::LDS, s, b, lists, per_wg);
     return launch_status();
 }
 template int32_t launch_stream<true>(const StreamBatch &, const v2i *, int, int, hipStream_t);

@@ -389,7 +389,7 @@ static int32_t launch_shape(const int8_t *qx, const float *sx, const int8_t *qw,
         if (best < 0 || bytes < best) { best = bytes; gg.pm = pm; gg.pn = pn; }
     }
     const dim3 grid((unsigned)(gg.tiles_m * gg.tiles_n)), blk(256);
-    hipLaunchKernelGGL((k_w8a8_tiled<TM, TN, DEQ>), grid, blk, LDS, s, qx, qw, sx, sw, acc, y, M, N, K, gg);
+    launch_kernel((k_w8a8_tiled<TM, TN, DEQ>), grid, blk, LDS, s, qx, qw, sx, sw, acc, y, M, N, K, gg);
     return launch_status();
 }
 

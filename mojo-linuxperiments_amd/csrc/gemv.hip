@@ -355,8 +355,8 @@ static void start_row(int cus, int per_wave, const float *x, const int8_t *qw, c
                       int N, int K, const RowArgs &ra, hipStream_t s)
 {
     auto go = [&](auto R, int wgs) {
-        hipLaunchKernelGGL((k_gemv_row<CW, WHOLE, decltype(R)::value, OP>), dim3((unsigned)(wgs * cus)), dim3(512), 0, s, x, qw, sw, y,
-                           qx, sx, N, K, ra);
+        launch_kernel((k_gemv_row<CW, WHOLE, decltype(R)::value, OP>), dim3((unsigned)(wgs * cus)), dim3(512), 0, s, x, qw, sw, y,
+                      qx, sx, N, K, ra);
     };
     using std::integral_constant;
     if (per_wave <= 2) return go(integral_constant<int, 1>{}, 1);
@@ -440,7 +440,7 @@ static int32_t launch_reg(const int8_t *qx, const float *sx, const int8_t *qw, c
     constexpr int R = (16 / CW) < 1 ? 1 : (16 / CW);
     const int rows_per_wg = (WG / QW) * R;
     const unsigned grid = (unsigned)((N + rows_per_wg - 1) / rows_per_wg);
-    hipLaunchKernelGGL((k_gemv_reg<MB, CW, WG, DEQ>), dim3(grid), dim3(64 * WG), 0, s, qx, qw, sx, sw, acc, y, M, N, K, QW);
+    launch_kernel((k_gemv_reg<MB, CW, WG, DEQ>), dim3(grid), dim3(64 * WG), 0, s, qx, qw, sx, sw, acc, y, M, N, K, QW);
     return launch_status();
 }
 

@@ -259,8 +259,8 @@ static int32_t launch_row_op_quant(const float *x, const float *res, const float
     const int64_t nchunk = K / 8;
     const dim3 grid((unsigned)M);
 #define MI_ROWQ(CC, TT)                                                                                           \
-    hipLaunchKernelGGL((k_row_op_quant<BLOCK, CC, MODE, TT>), grid, dim3(TT), 0, s, x, res, g, eps, h_out, y_out, q, \
-                       scale, (int)K)
+    launch_kernel((k_row_op_quant<BLOCK, CC, MODE, TT>), grid, dim3(TT), 0, s, x, res, g, eps, h_out, y_out, q, \
+                  scale, (int)K)
     if (nchunk <= 256) MI_ROWQ(1, 256);
     else if (nchunk <= 512) MI_ROWQ(1, 512);
     else if (nchunk <= 1024) MI_ROWQ(1, 1024);
@@ -297,8 +297,8 @@ extern "C" int32_t mi_rmsnorm_f32(const float *x, const float *residual, const f
     const int C = (int)((H / 4 + 255) / 256);
     const dim3 grid((unsigned)M);
 #define MI_NORM(CC)                                                                                              \
-    hipLaunchKernelGGL(layer::k_add_rmsnorm<CC>, grid, dim3(256), 0, as_stream(stream), x, residual, g, eps, h_out, \
-                       y, (int)H)
+    launch_kernel(layer::k_add_rmsnorm<CC>, grid, dim3(256), 0, as_stream(stream), x, residual, g, eps, h_out, \
+                  y, (int)H)
     if (C <= 1) MI_NORM(1);
     else if (C <= 2) MI_NORM(2);
     else if (C <= 4) MI_NORM(4);
@@ -322,9 +322,9 @@ extern "C" int32_t mi_rope_kv_append_f32_i8(const float *qkv, int64_t row_stride
         !aligned4(ks) || !aligned4(vs) || !aligned4(pos))
         return MI_EINVAL;
     const int64_t rows = B * (Hq + 2 * Hkv);
-    hipLaunchKernelGGL(layer::k_rope_kv_append, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, as_stream(stream),
-                       qkv, row_stride, rope_cos, rope_sin, q_out, kq, ks, vq, vs, pos, (int)B, (int)Hq, (int)Hkv,
-                       (int)T_cap);
+    launch_kernel(layer::k_rope_kv_append, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, as_stream(stream),
+                  qkv, row_stride, rope_cos, rope_sin, q_out, kq, ks, vq, vs, pos, (int)B, (int)Hq, (int)Hkv,
+                  (int)T_cap);
     return launch_status();
 }
 
@@ -335,8 +335,8 @@ extern "C" int32_t mi_swiglu_f32(const float *gate_up, float *h, int64_t M, int6
     if (!aligned16(gate_up) || !aligned16(h)) return MI_EINVAL;
     if (M == 0) return MI_OK;
     const int64_t quads = M * I / 4;
-    hipLaunchKernelGGL(layer::k_swiglu, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, as_stream(stream),
-                       gate_up, h, M, (int)I);
+    launch_kernel(layer::k_swiglu, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, as_stream(stream),
+                  gate_up, h, M, (int)I);
     return launch_status();
 }
 
@@ -373,7 +373,7 @@ extern "C" int32_t mi_add_f32(const float *a, const float *b, float *out, int64_
     if (!a || !b || !out || n < 0 || n % 4) return MI_EINVAL;
     if (!aligned16(a) || !aligned16(b) || !aligned16(out)) return MI_EINVAL;
     if (n == 0) return MI_OK;
-    hipLaunchKernelGGL(layer::k_add, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, as_stream(stream), a, b,
-                       out, n);
+    launch_kernel(layer::k_add, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, as_stream(stream), a, b,
+                  out, n);
     return launch_status();
 }

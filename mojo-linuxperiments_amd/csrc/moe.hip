@@ -1092,14 +1092,14 @@ static int32_t launch_route(const float *x, const float *wr, int32_t *idx, float
 #define MI_LOGITS(CQ_)                                                                                                  \
     do {                                                                                                                \
         if (ew == 1)                                                                                                    \
-            hipLaunchKernelGGL((k_moe_logits<CQ_, 1>), grid, dim3(256), 0, as_stream(stream), x, wr, logits, (int)T,    \
-                               (int)H, (int)E, qx, sx);                                                                 \
+            launch_kernel((k_moe_logits<CQ_, 1>), grid, dim3(256), 0, as_stream(stream), x, wr, logits, (int)T,    \
+                          (int)H, (int)E, qx, sx);                                                                      \
         else if (ew == 8)                                                                                               \
-            hipLaunchKernelGGL((k_moe_logits<CQ_, 8>), grid, dim3(256), 0, as_stream(stream), x, wr, logits, (int)T,    \
-                               (int)H, (int)E, qx, sx);                                                                 \
+            launch_kernel((k_moe_logits<CQ_, 8>), grid, dim3(256), 0, as_stream(stream), x, wr, logits, (int)T,    \
+                          (int)H, (int)E, qx, sx);                                                                      \
         else                                                                                                            \
-            hipLaunchKernelGGL((k_moe_logits<CQ_, 16>), grid, dim3(256), 0, as_stream(stream), x, wr, logits, (int)T,   \
-                               (int)H, (int)E, qx, sx);                                                                 \
+            launch_kernel((k_moe_logits<CQ_, 16>), grid, dim3(256), 0, as_stream(stream), x, wr, logits, (int)T,   \
+                          (int)H, (int)E, qx, sx);                                                                      \
     } while (0)
     switch (cq) {
     case 0: MI_LOGITS(0); break;
@@ -1113,12 +1113,12 @@ static int32_t launch_route(const float *x, const float *wr, int32_t *idx, float
     if (rc) return rc;
     if (perm) {
         const size_t words = (size_t)(2 * E * ((T + 31) / 32) + E + 1);
-        hipLaunchKernelGGL(k_moe_topk_dispatch, dim3(1), dim3(1024), words * 4, as_stream(stream), logits, idx, w, perm, seg,
-                           (int)T, (int)E, (int)topk);
+        launch_kernel(k_moe_topk_dispatch, dim3(1), dim3(1024), words * 4, as_stream(stream), logits, idx, w, perm, seg,
+                      (int)T, (int)E, (int)topk);
         return launch_status();
     }
-    hipLaunchKernelGGL(k_moe_topk, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, as_stream(stream), logits, idx, w, (int)T,
-                       (int)E, (int)topk);
+    launch_kernel(k_moe_topk, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, as_stream(stream), logits, idx, w, (int)T,
+                  (int)E, (int)topk);
     return launch_status();
 }
 
@@ -1155,8 +1155,8 @@ extern "C" int32_t mi_moe_dispatch(const int32_t *idx, int32_t *perm, int32_t *s
     const int64_t words = 2 * E * ((T + 31) / 32) + E + 1;
     if (words > moe::DISPATCH_MAX_WORDS) return MI_ERANGE;
     MI_LDS_OPT_IN((&moe::k_moe_dispatch), (int)(moe::DISPATCH_MAX_WORDS * 4));
-    hipLaunchKernelGGL(moe::k_moe_dispatch, dim3(1), dim3(1024), (size_t)words * 4, as_stream(stream), idx, perm,
-                       seg_off, (int)T, (int)E, (int)topk);
+    launch_kernel(moe::k_moe_dispatch, dim3(1), dim3(1024), (size_t)words * 4, as_stream(stream), idx, perm,
+                  seg_off, (int)T, (int)E, (int)topk);
     return launch_status();
 }
 
@@ -1229,17 +1229,17 @@ static int32_t run_ffn(const float *x, const int32_t *idx, const float *w, const
 #define MI_RX_GU(NS)                                                                                            \
     do {                                                                                                        \
         MI_LDS_OPT_IN((&moe::k_moe_expert_rx<false, NS>), moe::RX_LDS);                                        \
-        hipLaunchKernelGGL((moe::k_moe_expert_rx<false, NS>), grid, dim3(256), moe::RX_LDS, s, qx, sx, perm, seg, \
-                           wg, sg, wu, su, h, (int)H, (int)I, (int)topk, chunks, (int)E, by_chunk);     \
+        launch_kernel((moe::k_moe_expert_rx<false, NS>), grid, dim3(256), moe::RX_LDS, s, qx, sx, perm, seg, \
+                      wg, sg, wu, su, h, (int)H, (int)I, (int)topk, chunks, (int)E, by_chunk);          \
     } while (0)
         if (ns_gu <= 2) MI_RX_GU(2);
         else if (ns_gu <= 4) MI_RX_GU(4);
         else MI_RX_GU(8);
 #undef MI_RX_GU
     } else {
-        hipLaunchKernelGGL(moe::k_moe_expert_gemm<false>, dim3((unsigned)(I / 16), (unsigned)E), dim3(256),
-                           moe::EXPERT_LDS, s, qx, sx, perm, seg, wg, sg, wu, su, h, (int)H, (int)I, (int)I, (int)topk,
-                           1);
+        launch_kernel(moe::k_moe_expert_gemm<false>, dim3((unsigned)(I / 16), (unsigned)E), dim3(256),
+                      moe::EXPERT_LDS, s, qx, sx, perm, seg, wg, sg, wu, su, h, (int)H, (int)I, (int)I, (int)topk,
+                      1);
     }
     rc = launch_status();
     if (rc) return rc;
@@ -1252,9 +1252,9 @@ static int32_t run_ffn(const float *x, const int32_t *idx, const float *w, const
 #define MI_RX_DN(NS)                                                                                            \
     do {                                                                                                        \
         MI_LDS_OPT_IN((&moe::k_moe_expert_rx<true, NS>), moe::RX_LDS);                                        \
-        hipLaunchKernelGGL((moe::k_moe_expert_rx<true, NS>), grid, dim3(256), moe::RX_LDS, s, hq, hs, perm, seg, wd, \
-                           sd, (const int8_t *)nullptr, (const float *)nullptr, out, (int)I, (int)H,            \
-                           (int)topk, chunks, (int)E, by_chunk);                                                \
+        launch_kernel((moe::k_moe_expert_rx<true, NS>), grid, dim3(256), moe::RX_LDS, s, hq, hs, perm, seg, wd, \
+                      sd, (const int8_t *)nullptr, (const float *)nullptr, out, (int)I, (int)H,                 \
+                      (int)topk, chunks, (int)E, by_chunk);                                                     \
     } while (0)
         if (steps_dn <= 2) MI_RX_DN(2);
         else if (steps_dn <= 4) MI_RX_DN(4);
@@ -1262,14 +1262,14 @@ static int32_t run_ffn(const float *x, const int32_t *idx, const float *w, const
         else MI_RX_DN(8);
 #undef MI_RX_DN
     } else {
-        hipLaunchKernelGGL(moe::k_moe_expert_gemm<true>, dim3((unsigned)((H + 127) / 128), (unsigned)E), dim3(256),
-                           moe::EXPERT_LDS, s, hq, hs, perm, seg, wd, sd, (const int8_t *)nullptr,
-                           (const float *)nullptr, out, (int)I, (int)H, (int)H, (int)topk, 1);
+        launch_kernel(moe::k_moe_expert_gemm<true>, dim3((unsigned)((H + 127) / 128), (unsigned)E), dim3(256),
+                      moe::EXPERT_LDS, s, hq, hs, perm, seg, wd, sd, (const int8_t *)nullptr,
+                      (const float *)nullptr, out, (int)I, (int)H, (int)H, (int)topk, 1);
     }
     rc = launch_status();
     if (rc) return rc;
     const dim3 cgrid((unsigned)((T * H / 4 + 255) / 256));
-#define MI_COMBINE(K_) hipLaunchKernelGGL(moe::k_moe_combine<K_>, cgrid, dim3(256), 0, s, out, w, idx, y, (int)T, (int)H, (int)topk, (int)E)
+#define MI_COMBINE(K_) launch_kernel(moe::k_moe_combine<K_>, cgrid, dim3(256), 0, s, out, w, idx, y, (int)T, (int)H, (int)topk, (int)E)
     switch (topk) {
     case 1: MI_COMBINE(1); break;
     case 2: MI_COMBINE(2); break;

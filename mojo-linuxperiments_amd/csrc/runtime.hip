@@ -14,6 +14,7 @@
 
 namespace mi {
 thread_local int32_t g_last_hip_error = 0;
+thread_local hipError_t g_launch_error = hipSuccess;
 
 int32_t compute_units()
 {
@@ -179,13 +180,17 @@ int32_t mi_arena_create(mi_ctx *ctx, int64_t size_bytes, int64_t alignment, mi_a
     // fresh mmap pages read as zero; give device memory the same property
     const int64_t words = size_bytes / 4;
     if (words > 0) {
-        hipLaunchKernelGGL(k_fill_u32, dim3(2048), dim3(256), 0, 0, (uint32_t *)p, 0u, words);
+        launch_kernel(k_fill_u32, dim3(2048), dim3(256), 0, 0, (uint32_t *)p, 0u, words);
     }
-    hipError_t e = hipDeviceSynchronize();
-    if (e != hipSuccess) {
+    int32_t rc = launch_status();
+    if (rc == MI_OK) {
+        const hipError_t e = hipDeviceSynchronize();
+        if (e != hipSuccess) rc = hip_fail(e);
+    }
+    if (rc != MI_OK) {
         (void)hipFree(p);
         delete a;
-        return hip_fail(e);
+        return rc;
     }
     a->ctx = ctx;
     a->base = (uint8_t *)p;
@@ -550,8 +555,8 @@ int32_t mi_fill_u32(void *dst, uint32_t value, int64_t count, void *stream)
     if (count == 0) return MI_OK;
     int64_t blocks = (count + 255) / 256;
     if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream),
-                       (uint32_t *)dst, value, count);
+    launch_kernel(k_fill_u32, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream),
+                  (uint32_t *)dst, value, count);
     return launch_status();
 }
 

@@ -9,6 +9,7 @@ upstream ones: make an arena, alloc, launch, wait, check
 There is no CPU fallback: if the shared library is missing, import fails.
 """
 import ctypes as C
+import math
 import os
 
 import numpy as np
@@ -181,7 +182,7 @@ class DevBuf:
 
     @property
     def nbytes(self):
-        return int(np.prod(self.shape, dtype=np.int64)) * self.dtype.itemsize
+        return math.prod(self.shape) * self.dtype.itemsize   # not np.prod: 2 us on the way to every launch
 
     def offset(self, nbytes, shape, dtype):
         return DevBuf(self.ptr + int(nbytes), shape, dtype)
