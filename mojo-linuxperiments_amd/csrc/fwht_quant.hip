@@ -254,30 +254,24 @@ __global__ __launch_bounds__(256) void k_kv_append(const float *__restrict__ k_n
     const int head = blockIdx.x * 16 + t / LPB;      // flat (b, h)
     const bool is_v = blockIdx.y != 0;
     const int b = min(head / Hkv, B - 1), h = head % Hkv;
+    const float *src = (is_v ? v_new : k_new) + (int64_t)b * row_stride + (int64_t)h * BLOCK + 4 * j;
+    // all latency: the head's row does not wait for the position, and the page is looked up while the row is on its way
+    const float4 lo = *reinterpret_cast<const float4 *>(src);
+    const float4 hi = *reinterpret_cast<const float4 *>(src + BLOCK / 2);
     const int tp = pos[b];
     const bool live = head < B * Hkv && tp >= 0 && tp < T_cap;
-    const float *src = (is_v ? v_new : k_new) + (int64_t)b * row_stride + (int64_t)h * BLOCK + 4 * j;
-    float v[8];
-    if (live) {
-        const float4 lo = *reinterpret_cast<const float4 *>(src);
-        const float4 hi = *reinterpret_cast<const float4 *>(src + BLOCK / 2);
-        v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w;
-        v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+    int64_t row = ((int64_t)b * Hkv + h) * T_cap + tp;
+    if (block_table && live) {
+        // paged pool [page][kv head][P tokens]: the page that holds token tp of sequence b
+        const int page = block_table[(int64_t)b * max_pages + (tp >> page_shift)];
+        row = (((int64_t)page * Hkv + h) << page_shift) + (tp & ((1 << page_shift) - 1));
     }
+    float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
     fwht_codes<BLOCK>(v, j);
     const float a = max_lanes<LPB>(abs8(v));
     const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
     const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
     if (live) {
-        int64_t row = ((int64_t)b * Hkv + h) * T_cap + tp;
-        if (block_table) {
-            // paged pool [page][kv head][P tokens]: the page that holds token tp of sequence b
-            const int page = block_table[(int64_t)b * max_pages + (tp >> page_shift)];
-            row = (((int64_t)page * Hkv + h) << page_shift) + (tp & ((1 << page_shift) - 1));
-        }
         int8_t *q = (is_v ? vq : kq) + row * BLOCK + 4 * j;
         if (j == 0) (is_v ? vs : ks)[row] = sc;
         *reinterpret_cast<uint32_t *>(q) = quant4(v[0], v[1], v[2], v[3], inv);

@@ -70,19 +70,12 @@ __global__ __launch_bounds__(256) void k_rope_kv_append(const float *__restrict_
     const int heads = Hq + 2 * Hkv;
     const int flat = blockIdx.x * 16 + t / LPB;
     const int b = min(flat / heads, B - 1), hd = flat % heads;
+    const float *src = qkv + (int64_t)b * row_stride + (int64_t)hd * D + 4 * j;
+    const float4 lo = *reinterpret_cast<const float4 *>(src);   // does not wait for the position
+    const float4 hi = *reinterpret_cast<const float4 *>(src + D / 2);
     const int tp = pos[b];
     const bool live = flat < B * heads && tp >= 0 && tp < T_cap;
-    const float *src = qkv + (int64_t)b * row_stride + (int64_t)hd * D + 4 * j;
-    float v[8];
-    if (live) {
-        const float4 lo = *reinterpret_cast<const float4 *>(src);
-        const float4 hi = *reinterpret_cast<const float4 *>(src + D / 2);
-        v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w;
-        v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = 0.0f;
-    }
+    float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
     const bool is_q = hd < Hq, is_v = hd >= Hq + Hkv;
     if (live && !is_v) {
         const float4 c4 = *reinterpret_cast<const float4 *>(cs + (int64_t)tp * (D / 2) + 4 * j);
