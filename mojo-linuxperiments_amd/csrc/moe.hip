@@ -736,10 +736,21 @@ static_assert(2 * RX_LDS <= 160 * 1024, "two workgroups a unit");
 // than 48: 180 us for the layer's FFN with passes of 48, 176 with 64.)
 constexpr int rx_most(int nsmax) { return nsmax > 6 ? 32 : nsmax > 4 ? 48 : 64; }
 
+// Where the down kernel makes the codes of its rows itself (OWN) and the quantizer's launch between the two expert kernels goes: with
+// so few tokens that every expert's are one pass, and few of them an expert, since every workgroup of an expert makes all of its
+// codes.  Layer, top-8, H = 2048, I = 768, 128 experts, us with the launch -> without: 1 token 31.4 -> 28.0, 4 50.6 -> 45.7,
+// 16 92.9 -> 88.0, 32 117.6 -> 116.3; 32 tokens of 64 experts, top-4, H = 1024, I = 512 40.2 -> 38.2; 16 of 16 experts, 8 rows an
+// expert, H = 1024, I = 256 28.0 -> 26.3.  Beyond: 128 of 128 experts 144.4 -> 144.6, 12 rows an expert (48 of 16 experts, top-4)
+// 43.4 -> 45.4, 64 of 16 experts, top-8, 30.3 -> 36.6, 512 of 128 174.8 -> 201.5.
+constexpr int OWN_PASS = 32;
+static bool own_codes(int64_t T, int64_t E, int topk) { return T <= OWN_PASS && T * topk <= 8 * E; }
+
 // One pass: at most 16 * MTT of an expert's pairs (from pos0 on, n of them) against nch row chunks from chunk c0 on.
 // first: the workgroup's first pass over these chunks, which brings their weight scales.
-template <bool DOWN, int NSMAX, int MTT>
-__device__ __forceinline__ void rx_pass(char *smem, const int8_t *__restrict__ act, const float *__restrict__ act_scale,
+// OWN (down, see own_codes): the pairs' codes are made here, from fp32 rows h; the workgroup with the expert's first
+// chunk leaves them in act and act_scale.
+template <bool DOWN, int NSMAX, int MTT, bool OWN>
+__device__ __forceinline__ void rx_pass(char *smem, const int8_t *act, const float *act_scale, const float *__restrict__ h,
                                         const int32_t *__restrict__ perm, const int8_t *__restrict__ w0,
                                         const float *__restrict__ sc0, const int8_t *__restrict__ w1,
                                         const float *__restrict__ sc1, float *__restrict__ out, int Kdim, int Nrows, int topk,
@@ -816,8 +827,75 @@ __device__ __forceinline__ void rx_pass(char *smem, const int8_t *__restrict__ a
     v4i xr[MTT][NSMAX][2];
     int last_step = steps - 1 - s0;
     asm volatile("" : "+v"(last_step));   // (scalar registers are what this kernel has fewest of)
+    if constexpr (OWN) {
+        // a wave a row, as the quantizer by itself; as many rows at a time as the sums' area holds, which this form does not use
+        static_assert(DOWN && NSMAX * 128 <= 1024, "rows of at most two chunks a lane");
+        constexpr int C = NSMAX * 128 > 512 ? 2 : 1;
+        int8_t *const s_code = reinterpret_cast<int8_t *>(smem + RX_RING_BYTES);
+        constexpr int AT_ONCE = RX_RED_BYTES / (NSMAX * 128) < 16 ? RX_RED_BYTES / (NSMAX * 128) : 16;
+        const int jq = lane & 31;
+        int kd = Kdim, writes = c0;
+        asm volatile("" : "+v"(kd), "+v"(writes));   // (as above)
+        static_for<MTT>([&](auto B) {
+            constexpr int b = decltype(B)::value;
+            const int end = min(n, 16 * b + 16);
+            for (int base = 16 * b; base < end; base += AT_ONCE) {
+                if (base) __syncthreads();   // the rows before have been read
+                for (int row = base + wave; row < min(end, base + AT_ONCE); row += 4) {
+                    const float *hr = h + (int64_t)(pos0 + row) * kd;
+                    float v[C][8];
+                    float amax = 0.0f;
 #pragma unroll
-    for (int b = 0; b < MTT; ++b) {
+                    for (int i = 0; i < C; ++i) {
+                        const int c = lane + 64 * i, of = (c >> 5) * 256 + 4 * jq;
+                        float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
+                        if ((C == 2 && i == 0) || c * 8 < kd) {   // (two chunks a lane: rows of more than 512)
+                            lo = *reinterpret_cast<const float4 *>(hr + of);
+                            hi = *reinterpret_cast<const float4 *>(hr + of + 128);
+                        }
+                        v[i][0] = lo.x; v[i][1] = lo.y; v[i][2] = lo.z; v[i][3] = lo.w;
+                        v[i][4] = hi.x; v[i][5] = hi.y; v[i][6] = hi.z; v[i][7] = hi.w;
+                    }
+#pragma unroll
+                    for (int i = 0; i < C; ++i) {
+                        fwht_codes<256>(v[i], jq);
+                        amax = fmaxf(amax, abs8(v[i]));
+                    }
+                    amax = max_lanes<64>(amax);
+                    const float sc = (amax == 0.0f) ? 1.0f : amax / 127.0f;
+                    const float inv = (amax == 0.0f) ? 0.0f : 127.0f / amax;
+                    if (lane == 0) s_tsc[row] = sc;
+                    if (lane == 0 && writes == 0) const_cast<float *>(act_scale)[pos0 + row] = sc;
+                    int8_t *const to = const_cast<int8_t *>(act) + (int64_t)(pos0 + row) * kd;
+#pragma unroll
+                    for (int i = 0; i < C; ++i) {
+                        const int c = lane + 64 * i, of = (c >> 5) * 256 + 4 * jq;
+                        if (!(C == 2 && i == 0) && c * 8 >= kd) continue;
+                        const uint32_t q0 = quant4(v[i][0], v[i][1], v[i][2], v[i][3], inv), q1 = quant4(v[i][4], v[i][5], v[i][6], v[i][7], inv);
+                        *reinterpret_cast<uint32_t *>(s_code + (row - base) * kd + of) = q0;
+                        *reinterpret_cast<uint32_t *>(s_code + (row - base) * kd + of + 128) = q1;
+                        if (writes == 0) {
+                            *reinterpret_cast<uint32_t *>(to + of) = q0;
+                            *reinterpret_cast<uint32_t *>(to + of + 128) = q1;
+                        }
+                    }
+                }
+                __syncthreads();
+                const int mine = min(16 * b + r, n - 1);
+                if (mine >= base && mine < base + AT_ONCE) {
+                    const int8_t *xp = s_code + (mine - base) * kd + g_ * 16;
+#pragma unroll
+                    for (int i = 0; i < NSMAX; ++i) {
+                        const int st = min(i, last_step) * 128;
+                        xr[b][i][0] = *reinterpret_cast<const v4i *>(xp + st);
+                        xr[b][i][1] = *reinterpret_cast<const v4i *>(xp + st + 64);
+                    }
+                }
+            }
+        });
+    }
+#pragma unroll
+    for (int b = 0; b < (OWN ? 0 : MTT); ++b) {
         const int at = pos0 + min(b * 16 + r, n - 1);
         const int8_t *xp = act + (DOWN ? (int64_t)at : (int64_t)(perm[at] / topk)) * Kdim + g_ * 16 + s0 * 128;
 #pragma unroll
@@ -829,7 +907,7 @@ __device__ __forceinline__ void rx_pass(char *smem, const int8_t *__restrict__ a
     }
     if (tid < 16 * MTT) {
         s_dst[tid] = DOWN ? pair : pos;
-        s_tsc[tid] = act_scale[DOWN ? pos : pair / topk];
+        if constexpr (!OWN) s_tsc[tid] = act_scale[DOWN ? pos : pair / topk];
     }
     if (first) {
 #pragma unroll
@@ -940,9 +1018,9 @@ __device__ __forceinline__ void rx_pass(char *smem, const int8_t *__restrict__ a
 // shapes from 1 to 2048 tokens, 16 to 128 experts: 0.84 to 1.00 of the time before, 512 tokens 191.9 -> 186.5.  Measured without gain: non-temporal stores and loads, whole 128-byte lines per store, exact counts of
 // the stores in the waits, costs that grow with an expert's tokens, rings of two stages, three workgroups a unit.
 // by_chunk: at most a chunk a workgroup, all of the same cost, with the compute units' own order as the balance.
-template <bool DOWN, int NSMAX>
-__global__ __launch_bounds__(256, 2) void k_moe_expert_rx(const int8_t *__restrict__ act,
-                                                          const float *__restrict__ act_scale,
+// OWN: see rx_pass.
+template <bool DOWN, int NSMAX, bool OWN>
+__global__ __launch_bounds__(256, 2) void k_moe_expert_rx(const int8_t *act, const float *act_scale, const float *__restrict__ h,
                                                           const int32_t *__restrict__ perm,
                                                           const int32_t *__restrict__ seg_off,
                                                           const int8_t *__restrict__ w0, const float *__restrict__ sc0,
@@ -952,7 +1030,8 @@ __global__ __launch_bounds__(256, 2) void k_moe_expert_rx(const int8_t *__restri
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
-    constexpr int PASS = rx_most(NSMAX);
+    constexpr int PASS = OWN ? OWN_PASS : rx_most(NSMAX);
+    if constexpr (OWN) asm volatile("" : "+v"(h), "+v"(act), "+v"(act_scale), "+v"(perm));   // (scalar registers are what this kernel has fewest of)
     if constexpr (!DOWN) {
         int *s_red = reinterpret_cast<int *>(smem + RX_RING_BYTES);
         for (int o = tid; o < RX_RED_BYTES / 4; o += 256) s_red[o] = 0;
@@ -1002,7 +1081,7 @@ __global__ __launch_bounds__(256, 2) void k_moe_expert_rx(const int8_t *__restri
             const int nch = min(MOST, last - c0);
             for (int base = 0; base < count; base += PASS) {
                 const int n = min(PASS, count - base);
-#define MI_RX_PASS(MT_) rx_pass<DOWN, NSMAX, MT_>(smem, act, act_scale, perm, w0, sc0, w1, sc1, out, Kdim, Nrows, topk, e, c0, \
+#define MI_RX_PASS(MT_) rx_pass<DOWN, NSMAX, MT_, OWN>(smem, act, act_scale, h, perm, w0, sc0, w1, sc1, out, Kdim, Nrows, topk, e, c0, \
                                                   nch, seg0 + base, n, base == 0)
                 if (n <= 16) MI_RX_PASS(1);
                 else if (n <= 32 || PASS == 32) MI_RX_PASS(2);
@@ -1238,9 +1317,9 @@ static int32_t run_ffn(const float *x, const int32_t *idx, const float *w, const
         const dim3 grid(by_chunk ? (unsigned)(chunks * std::min<int64_t>(E, P)) : 2u * cus);
 #define MI_RX_GU(NS)                                                                                            \
     do {                                                                                                        \
-        MI_LDS_OPT_IN((&moe::k_moe_expert_rx<false, NS>), moe::RX_LDS);                                        \
-        launch_kernel((moe::k_moe_expert_rx<false, NS>), grid, dim3(256), moe::RX_LDS, s, qx, sx, perm, seg, \
-                      wg, sg, wu, su, h, (int)H, (int)I, (int)topk, chunks, (int)E, by_chunk);          \
+        MI_LDS_OPT_IN((&moe::k_moe_expert_rx<false, NS, false>), moe::RX_LDS);                                 \
+        launch_kernel((moe::k_moe_expert_rx<false, NS, false>), grid, dim3(256), moe::RX_LDS, s, qx, sx,      \
+                      (const float *)nullptr, perm, seg, wg, sg, wu, su, h, (int)H, (int)I, (int)topk, chunks, (int)E, by_chunk);          \
     } while (0)
         if (ns_gu <= 2) MI_RX_GU(2);
         else if (ns_gu <= 4) MI_RX_GU(4);
@@ -1253,24 +1332,33 @@ static int32_t run_ffn(const float *x, const int32_t *idx, const float *w, const
     }
     rc = launch_status();
     if (rc) return rc;
-    rc = mi_fwht_quant_f32_i8(h, hq, hs, P, I, 256, stream);
-    if (rc) return rc;
     const int steps_dn = (int)(I / 128);   // every wave walks the whole of K
+    const bool own = steps_dn <= 8 && moe::own_codes(T, E, topk);
+    if (!own) {
+        rc = mi_fwht_quant_f32_i8(h, hq, hs, P, I, 256, stream);
+        if (rc) return rc;
+    }
     if (steps_dn <= 8) {
         const int chunks = (int)(H / 128), by_chunk = one_chunk(chunks);
         const dim3 grid(by_chunk ? (unsigned)(chunks * std::min<int64_t>(E, P)) : 2u * cus);
-#define MI_RX_DN(NS)                                                                                            \
+#define MI_RX_DN1(NS, OWN_)                                                                                     \
     do {                                                                                                        \
-        MI_LDS_OPT_IN((&moe::k_moe_expert_rx<true, NS>), moe::RX_LDS);                                        \
-        launch_kernel((moe::k_moe_expert_rx<true, NS>), grid, dim3(256), moe::RX_LDS, s, hq, hs, perm, seg, wd, \
+        MI_LDS_OPT_IN((&moe::k_moe_expert_rx<true, NS, OWN_>), moe::RX_LDS);                                    \
+        launch_kernel((moe::k_moe_expert_rx<true, NS, OWN_>), grid, dim3(256), moe::RX_LDS, s, hq, hs, h, perm, seg, wd, \
                       sd, (const int8_t *)nullptr, (const float *)nullptr, out, (int)I, (int)H,                 \
                       (int)topk, chunks, (int)E, by_chunk);                                                     \
+    } while (0)
+#define MI_RX_DN(NS)                 \
+    do {                             \
+        if (own) MI_RX_DN1(NS, true); \
+        else MI_RX_DN1(NS, false);   \
     } while (0)
         if (steps_dn <= 2) MI_RX_DN(2);
         else if (steps_dn <= 4) MI_RX_DN(4);
         else if (steps_dn <= 6) MI_RX_DN(6);
         else MI_RX_DN(8);
 #undef MI_RX_DN
+#undef MI_RX_DN1
     } else {
         launch_kernel(moe::k_moe_expert_gemm<true>, dim3((unsigned)((H + 127) / 128), (unsigned)E), dim3(256),
                       moe::EXPERT_LDS, s, hq, hs, perm, seg, wd, sd, (const int8_t *)nullptr,

@@ -287,3 +287,21 @@ def test_layer_of_few_tokens_equals_route_and_ffn(mi, dev, orc, T, H, I, E, topk
     assert np.array_equal(a["w"], w)
     for name in ("qx", "sx", "h", "hq", "hs", "out", "y"):
         assert np.array_equal(a[name], b[name]), name
+
+
+@pytest.mark.parametrize("T,I,E,topk", [
+    (1, 768, 16, 1), (8, 1024, 16, 8), (9, 1024, 16, 2), (10, 768, 16, 2), (11, 768, 16, 2), (16, 512, 16, 8),
+    (17, 256, 32, 4), (27, 768, 32, 4), (32, 768, 64, 2), (32, 1024, 128, 8),
+    (33, 768, 64, 2), (32, 768, 16, 8),     # the quantizer's own launch: a token more, more rows an expert
+])
+def test_codes_made_by_the_down_kernel(mi, dev, orc, T, I, E, topk):
+    """Every token picks expert 0, so that its rows fill the rounds of codes (8, 10 or 16 at a time) to their ends and past them."""
+    H = 512
+    rng = np.random.default_rng(T * I)
+    idx = np.stack([np.concatenate([[0], 1 + rng.permutation(E - 1)[:topk - 1]]) for _ in range(T)]).astype(np.int32)
+    w = rng.random((T, topk)).astype(np.float32)
+    x, experts = workload.activations(71, T, H), make_experts(orc, 73, E, H, I)
+    mark = dev.mark()
+    r = run_ffn(mi, dev, x, idx, w, experts)
+    dev.reset_to(mark)
+    check_ffn_against_oracle(orc, x, idx, w, experts, r)
