@@ -388,33 +388,40 @@ __global__ __launch_bounds__(256) void k_gqa_split(Params p)
 
 // Merge of the splits of one (b, h) row by the 16 lanes that own it (lane j: elements 4j..4j+3 and 64+4j..).
 // SP > 0: the split count is known at compile time and every load of the row goes out before the first use (one
-// memory round trip).  Returns the normalized row in the rotated basis of V.
+// memory round trip); SP < 0: the same for a count of at most -SP (the last split is read in place of those that are not there).
+// Returns the normalized row in the rotated basis of V.
 template <int SP, int BATCH = 8>
 __device__ __forceinline__ void merge_row(const float *__restrict__ part_o, const float *__restrict__ part_ml,
                                           int splits_rt, int64_t bkv, int hl, int j, float (&v)[8])
 {
+    constexpr int MOST = SP < 0 ? -SP : SP;
     const int splits = SP > 0 ? SP : splits_rt;
     const float *ml0 = part_ml + bkv * splits * 8;
     const float *po0 = part_o + (bkv * splits * 4 + hl) * attn::D;
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = 0.0f;
     float l = 0.0f;
-    if constexpr (SP > 0) {
-        float ms[SP], ls[SP];
-        float4 lo[SP], hi[SP];
+    if constexpr (MOST > 0) {
+        float ms[MOST], ls[MOST];
+        float4 lo[MOST], hi[MOST];
 #pragma unroll
-        for (int s = 0; s < SP; ++s) {
-            ms[s] = ml0[s * 8 + hl];
-            ls[s] = ml0[s * 8 + 4 + hl];
-            lo[s] = *reinterpret_cast<const float4 *>(po0 + s * 4 * attn::D + 4 * j);
-            hi[s] = *reinterpret_cast<const float4 *>(po0 + s * 4 * attn::D + 64 + 4 * j);
+        for (int i = 0; i < MOST; ++i) {
+            const int s = SP > 0 ? i : min(i, splits - 1);
+            ms[i] = ml0[s * 8 + hl];
+            ls[i] = ml0[s * 8 + 4 + hl];
+            lo[i] = *reinterpret_cast<const float4 *>(po0 + s * 4 * attn::D + 4 * j);
+            hi[i] = *reinterpret_cast<const float4 *>(po0 + s * 4 * attn::D + 64 + 4 * j);
         }
+        // all of them before the first use: the compiler otherwise saves registers and makes two round trips of it.  us of attention
+        // and merge, one sequence in spans of 256 tokens, 10 splits 10.4 -> 8.2, 14 10.5 -> 8.6, 16 8.9 -> 8.1.  (Not in workgroups
+        // of up to 1024 threads, which have 128 registers.)
+        if constexpr (BATCH == 16) __builtin_amdgcn_sched_barrier(0);
         float mx = ms[0];
 #pragma unroll
-        for (int s = 1; s < SP; ++s) mx = fmaxf(mx, ms[s]);
+        for (int s = 1; s < MOST; ++s) mx = fmaxf(mx, ms[s]);
 #pragma unroll
-        for (int s = 0; s < SP; ++s) {
-            const float w = (ms[s] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(ms[s] - mx);   // empty split
+        for (int s = 0; s < MOST; ++s) {
+            const float w = ((SP < 0 && s >= splits) || ms[s] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(ms[s] - mx);   // empty split
             l = __builtin_fmaf(ls[s], w, l);
             v[0] = __builtin_fmaf(lo[s].x, w, v[0]); v[1] = __builtin_fmaf(lo[s].y, w, v[1]);
             v[2] = __builtin_fmaf(lo[s].z, w, v[2]); v[3] = __builtin_fmaf(lo[s].w, w, v[3]);
@@ -613,13 +620,11 @@ int max_splits(int64_t B, int64_t Hkv, int64_t T)
 
 static bool merge_wide(int splits, int64_t rows) { return splits > 16 && splits <= 32 && rows <= 2 * compute_units(); }
 
-// How many dependent batches of loads the merge of `rows` rows makes: one for the split counts that are compiled in and in the
-// kernel for 17 to 32, one per eight splits otherwise.
+// How many dependent batches of loads the merge of `rows` rows makes: one up to 16 splits (8 where it quantizes) and in the kernel
+// for 17 to 32, one per eight splits otherwise.
 int merge_batches(int splits, int64_t rows, bool quant)
 {
-    switch (splits) {
-    case 1: case 2: case 3: case 4: case 5: case 6: case 8: case 12: case 16: return 1;
-    }
+    if (splits <= (quant ? 8 : 16) || splits == 12 || splits == 16) return 1;
     return !quant && merge_wide(splits, rows) ? 1 : (splits + 7) / 8;
 }
 
@@ -641,6 +646,7 @@ int32_t launch_merge(const float *part_o, const float *part_ml, float *o, int8_t
         case 4: MI_MERGEQ(4); break;
         case 5: MI_MERGEQ(5); break;
         case 6: MI_MERGEQ(6); break;
+        case 7: MI_MERGEQ(-8); break;
         case 8: MI_MERGEQ(8); break;
         case 12: MI_MERGEQ(12); break;
         case 16: MI_MERGEQ(16); break;
@@ -668,8 +674,11 @@ int32_t launch_merge(const float *part_o, const float *part_ml, float *o, int8_t
     case 4: MI_MERGE(4); break;
     case 5: MI_MERGE(5); break;
     case 6: MI_MERGE(6); break;
+    case 7: MI_MERGE(-8); break;
     case 8: MI_MERGE(8); break;
+    case 9: case 10: case 11: MI_MERGE(-12); break;
     case 12: MI_MERGE(12); break;
+    case 13: case 14: case 15: MI_MERGE(-16); break;
     case 16: MI_MERGE(16); break;
     default: MI_MERGE(0); break;
     }

@@ -672,7 +672,12 @@ struct Plan {
 int max_splits(int64_t B, int64_t Hkv, int64_t T);
 
 // How many spans a row is cut into, of equal length but for the last.  Where 16 blocks a workgroup (four a wave) do not give
-// every compute unit a workgroup: as many as it takes to get there.  Else the count whose busiest unit is done first, at four
+// every compute unit a workgroup: a block for each of a workgroup's waves, or two, three or four where these workgroups are more
+// than the units or, with codes, their spans more than the merge reads at once; and no cut at all up to eight blocks where the
+// workgroup then writes the output itself.  (Cut until every unit had a workgroup, a span was a block or two, most waves had
+// nothing to do and the merge was the longer half.  us of attention and merge before -> after, 8 heads: one sequence of 300 tokens
+// 7.2 -> 5.8, of 700 10.7 -> 7.0, of 1531 9.0 -> 7.5, of 4096 9.5 -> 8.1; 2 of 500 7.8 -> 6.3, 4 of 2500 11.2 -> 9.9; with codes,
+// one of 1531 14.3 -> 8.1, 4 of 1024 9.2 -> 8.0.)  Else the count whose busiest unit is done first, at four
 // blocks a wave or fewer: workgroups a unit times the blocks that a workgroup streams and START more for its start and end; the
 // merge counts as MERGE blocks of a unit, a quarter more for every span and BATCH for every further batch of loads that it makes,
 // and a finer cut has to promise a tenth (for a twentieth, mixed lengths lose what equal ones gain: 20 sequences of up to 3907
@@ -683,14 +688,22 @@ int max_splits(int64_t B, int64_t Hkv, int64_t T);
 // Without BATCH three sequences of 32768 were cut into 64 spans instead of 32: 39.4 instead of 25.0, the merge alone 15 more.
 static Plan pick(int64_t B, int64_t Hq, int64_t Hkv, int64_t T, bool quant)
 {
-    constexpr int START = 3, MERGE = 5, BATCH = 4;
+    constexpr int START = 3, MERGE = 5, BATCH = 4, DIRECT = 8;
     const int blocks = (int)((T + 63) / 64);
     const int64_t rows = B * Hkv, cus = compute_units();
     Plan pl;
     auto cut = [&](int s) { pl.per = (blocks + s - 1) / s, pl.splits = (blocks + pl.per - 1) / pl.per; };
     const int fewest = (blocks + 4 * NT_MAX - 1) / (4 * NT_MAX);
     if (rows * fewest < cus) {
-        cut((int)std::min<int64_t>((cus + rows - 1) / rows, blocks));
+        // (one sequence is cut alike with codes and without: the call with the projection makes its codes either way)
+        const bool codes = quant && B > 1;
+        if (!codes && blocks <= DIRECT) pl.per = blocks;
+        else {
+            const int64_t most = codes ? 8 : cus;
+            auto spans = [&] { return (int64_t)((blocks + pl.per - 1) / pl.per); };
+            for (pl.per = 4; pl.per < 4 * NT_MAX && (rows * spans() > cus || spans() > most); pl.per += 4) {}
+        }
+        pl.splits = (blocks + pl.per - 1) / pl.per;
         return pl;
     }
     // (a span takes whole rounds of its waves: one of 13 blocks is as long as one of 16, and loads blocks of the next.  31 sequences
