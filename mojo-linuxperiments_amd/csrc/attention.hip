@@ -19,8 +19,7 @@
 // l%4 = i supplies p(token, head i) * vs(token) as the A value and one V
 // element as the B value, so register i of the accumulator is head i.  Sixteen
 // such MFMAs (one per byte of the lane's 16) consume a load; int8 -> fp32 is
-// v_cvt_f32_ubyteN on (byte ^ 0x80) and the bias 128 * sum(p*vs) is removed
-// once at the end.  The fp32 matrix pipe does the 4-head FMA work that would
+// one v_cvt_f32_i32 that selects its byte.  The fp32 matrix pipe does the 4-head FMA work that would
 // otherwise cost 64 VALU FMAs per 16 bytes.
 //
 // Bound: HBM.  Algorithmic bytes = K and V codes (2*B*Hkv*T*D) + their scales
@@ -110,7 +109,7 @@ constexpr int RING = 8;           // loads a wave keeps in flight (1 KB each); t
 template <bool DUMP, bool RAGGED, bool PAGED, int WAVE_TILES>
 __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int8_t (&s_q)[4][4][D], float (&s_sq)[4][4],
                                                float (&s_red)[4][4][D], float (&s_sc)[4][WAVE_TILES][16][4],
-                                               float (&s_m)[4][4], float (&s_l)[4][4], float (&s_c)[4][4])
+                                               float (&s_m)[4][4], float (&s_l)[4][4])
 {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -283,28 +282,24 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
     v4f acc[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = (v4f){0.f, 0.f, 0.f, 0.f};
-    float lsum = 0.0f, csum = 0.0f;
+    float lsum = 0.0f;
 #pragma unroll
     for (int u = 0; u < 2 * WAVE_TILES; ++u) {
         const v4i vv = ring[(2 * WAVE_TILES + u) % RING];
         const float vscale = vsr[u % RING];
-        // int8 -> fp32 as (byte ^ 0x80) - 128: v_cvt_f32_ubyteN on the biased byte, the bias leaves at the end
+        // one conversion a code, which picks its byte and extends its sign.  (As biased bytes, v_cvt_f32_ubyte, with 128 times the
+        // weights taken off at the end, the sums lost two bits: error against 64-bit
+        // sums, 300 to 4096 tokens, 4.9e-7 to 8.5e-7 with it, 1.3e-7 to 1.9e-7 without; 16 sequences of 4096 tokens 29.8 and 29.2 us.)
         float f[16];
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const uint32_t x = (uint32_t)vv[w] ^ 0x80808080u;
-            f[4 * w + 0] = (float)(x & 0xffu);
-            f[4 * w + 1] = (float)((x >> 8) & 0xffu);
-            f[4 * w + 2] = (float)((x >> 16) & 0xffu);
-            f[4 * w + 3] = (float)(x >> 24);
-        }
+        for (int e = 0; e < 16; ++e) f[e] = (float)(int8_t)((uint32_t)vv[e >> 2] >> (8 * (e & 3)));
         if (u + RING < 2 * WAVE_TILES) load_v(u + RING);
         __builtin_amdgcn_sched_barrier(0);
         const float score = s_sc[wave][u >> 1][8 * (u & 1) + slot][hh];
         // a wave whose tokens are all masked has m_h = -inf: exp2(-inf - -inf) would be NaN
         const float pe = (score == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(score - m_h);
         const float a = pe * vscale;
-        if (counts) { lsum += pe; csum += a; }
+        if (counts) lsum += pe;
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[e] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, f[e], acc[e], 0, 0, 0);
     }
@@ -320,13 +315,12 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
     fold_slots<32, 16>(flat, lane);
     fold_slots<16, 8>(flat, lane);
     lsum += slot_xor<8>(lsum); lsum += slot_xor<16>(lsum); lsum += slot_xor<32>(lsum);
-    csum += slot_xor<8>(csum); csum += slot_xor<16>(csum); csum += slot_xor<32>(csum);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int fl = 8 * slot + j;   // = 4*e + head
         s_red[wave][fl & 3][16 * chunk + (fl >> 2)] = flat[j];
     }
-    if (lane < 4) { s_l[wave][lane] = lsum; s_c[wave][lane] = csum; }
+    if (lane < 4) s_l[wave][lane] = lsum;
     __syncthreads();
 
     // the four waves meet: rescale each wave's sums from its own maximum to the common one
@@ -338,7 +332,7 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
             const float f = (s_m[w][h] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(s_m[w][h] - m);
-            sum += (s_red[w][h][d] - 128.0f * s_c[w][h]) * f;
+            sum += s_red[w][h][d] * f;
         }
         p.part_o[(pbase * 4 + h) * D + d] = sum;
     }
@@ -359,7 +353,7 @@ __global__ __launch_bounds__(256) void k_gqa_split(Params p)
     __shared__ float s_sq[4][4];
     __shared__ float s_red[4][4][D];
     __shared__ __attribute__((aligned(16))) float s_sc[4][WAVE_TILES][16][4];
-    __shared__ float s_m[4][4], s_l[4][4], s_c[4][4];
+    __shared__ float s_m[4][4], s_l[4][4];
     const int tile_lo = blockIdx.x * p.tiles_per_split;
     int T = p.T;
     if (p.seq_len) {
@@ -378,12 +372,12 @@ __global__ __launch_bounds__(256) void k_gqa_split(Params p)
         }
     }
     if (p.block_table) {
-        gqa_split_body<false, true, true, WAVE_TILES>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l, s_c);
+        gqa_split_body<false, true, true, WAVE_TILES>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
         return;
     }
     const bool full = (tile_lo + 4 * WAVE_TILES) * 16 <= T;
-    if (full) gqa_split_body<DUMP, false, false, WAVE_TILES>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l, s_c);
-    else gqa_split_body<DUMP, true, false, WAVE_TILES>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l, s_c);
+    if (full) gqa_split_body<DUMP, false, false, WAVE_TILES>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
+    else gqa_split_body<DUMP, true, false, WAVE_TILES>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
 }
 
 // Merge of the splits of one (b, h) row by the 16 lanes that own it (lane j: elements 4j..4j+3 and 64+4j..).
@@ -586,30 +580,30 @@ struct SplitPlan {
     int splits, wave_tiles;
 };
 
+int max_splits(int64_t B, int64_t Hkv, int64_t T);
+
+// Spans of 256 tokens where they are at most two workgroups a unit (and no more than the merge reads at once and the workspace
+// holds), else of 704: a wave goes through all of its tiles, those past the end of its span as well, so a span that is not filled
+// costs what a full one does.  us, 8 heads, before -> here (a sequence of up to 256 tokens ran in a span of 704, and few rows were cut
+// into halves and quarters of 256): one sequence of 16 to 256 tokens 12.3 -> 8.9, of 1531 10.1 -> 9.6, 4 of 1500 13.8 -> 9.9, 32 of 256
+// 13.3 -> 10.1, 16 of 1000 14.6 -> 14.0; three workgroups a unit, 32 of 700, 16.9 in spans of 256 and 15.3 in one of 704.
 static SplitPlan pick_splits(int64_t B, int64_t Hkv, int64_t T)
 {
     const int ntiles = (int)((T + 15) / 16);
-    const int cus = compute_units();
-    SplitPlan pl;
-    pl.wave_tiles = TILES_LONG;
-    pl.splits = (ntiles + 4 * TILES_LONG - 1) / (4 * TILES_LONG);
-    if (B * Hkv * pl.splits < cus && ntiles > 4 * TILES_SHORT) {
-        // few rows: spans of 256 tokens, then halves of them while that still doubles the number of busy compute units
-        pl.wave_tiles = TILES_SHORT;
-        pl.splits = (ntiles + 4 * TILES_SHORT - 1) / (4 * TILES_SHORT);
-        while (B * Hkv * pl.splits < cus && (ntiles + pl.splits - 1) / pl.splits > 8 && pl.splits * 2 <= 16) pl.splits *= 2;
-    }
-    if (pl.splits > ntiles) pl.splits = ntiles;
-    return pl;
+    const int64_t rows = B * Hkv, cus = compute_units();
+    auto spans = [&](int tiles) { return (ntiles + 4 * tiles - 1) / (4 * tiles); };
+    const int few = spans(TILES_SHORT);
+    if (few == 1 || (rows * few <= 2 * cus && few <= 32 && few <= max_splits(B, Hkv, T))) return {few, TILES_SHORT};
+    return {spans(TILES_LONG), TILES_LONG};
 }
 
-// the largest split count pick_splits returns for any length in [1, T]
+// at least the largest split count pick_splits returns for any length in [1, T]: what workspaces are sized for
 int max_splits(int64_t B, int64_t Hkv, int64_t T)
 {
     const int ntiles = (int)((T + 15) / 16);
     int best = (ntiles + 4 * TILES_LONG - 1) / (4 * TILES_LONG);   // long spans: monotone in T
     if (B * Hkv < compute_units()) {
-        // short spans are possible for some length: ceil(n / 16) splits, doubled at most up to 16
+        // short spans are possible for some length: ceil(n / 16) splits (and room for 16, as there has always been)
         int s = (ntiles + 4 * TILES_SHORT - 1) / (4 * TILES_SHORT);
         if (s < 16) s = 16;
         if (s > ntiles) s = ntiles;

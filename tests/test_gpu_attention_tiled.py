@@ -635,3 +635,43 @@ def test_append_inside_the_attention_with_overlapping_buffers(mi, dev, T, q_at, 
     for name, a, b in zip(("q", "o_rot", "qkv", "y", "kq", "ks", "vq", "vs"), *got):
         assert np.array_equal(a, b), name
     dev.reset_to(mark)
+
+
+@pytest.mark.parametrize("B,Hkv,T", [
+    (1, 2, 65), (1, 2, 511), (1, 2, 512), (1, 2, 513), (3, 2, 512),       # one span of two to eight blocks, and the first cut
+    (1, 1, 1700), (1, 1, 2304), (1, 1, 2800), (1, 1, 3500), (1, 1, 4096),  # 7, 9, 11, 14 and 16 spans
+    (20, 8, 520), (20, 8, 1024), (33, 4, 900),                            # spans of 8 and 12 blocks, where 4 are too many workgroups
+])
+def test_few_rows_are_cut_into_whole_rounds(mi, dev, orc, B, Hkv, T):
+    """Both layouts at the ends of their spans and through every form of the merge, with codes and without."""
+    mark = dev.mark()
+    G, D, T_cap = 2, 128, (T + 63) // 64 * 64
+    Hq = G * Hkv
+    q, kq, ks, vq, vs, ks_c, vs_c = make_cache(mi, dev, 900 + T, B, Hq, Hkv, T, T_cap)
+    dkt, dvt = convert(mi, dev, kq, vq, T, T_cap)
+    lens = np.array([T - (i * T) // (2 * B) for i in range(B)], np.int32)
+    nbytes = mi.lib.mi_gqa_decode_workspace_bytes(B, Hq, Hkv, D, T)
+    guard = 4096
+    ws = dev.upload(np.full(nbytes + guard, 0x5A, np.uint8))
+    dq, dks, dvs, dl = dev.upload(q), dev.upload(ks_c), dev.upload(vs_c), dev.upload(lens)
+    kr, vr = np.zeros((B, Hkv, T_cap, D), np.int8), np.zeros((B, Hkv, T_cap, D), np.int8)
+    kr[:, :, :T], vr[:, :, :T] = kq, vq
+    dkr, dvr = dev.upload(kr), dev.upload(vr)
+    o1, o2, orot = (dev.empty((B, Hq, D), np.float32) for _ in range(3))
+    oq, osc = dev.empty((B, Hq * D), np.int8), dev.empty(B, np.float32)
+    mi.check(mi.lib.mi_gqa_decode_attn_tiled(dq.ptr, dkt.ptr, dks.ptr, dvt.ptr, dvs.ptr, o1.ptr, B, Hq, Hkv, D, T_cap, dl.ptr, T, 0,
+                                             ws.ptr, nbytes, None))
+    mi.check(mi.lib.mi_gqa_decode_attn_tiled_quant_i8(dq.ptr, dkt.ptr, dks.ptr, dvt.ptr, dvs.ptr, orot.ptr, oq.ptr, osc.ptr, B, Hq,
+                                                      Hkv, D, T_cap, dl.ptr, T, ws.ptr, nbytes, None))
+    mi.check(mi.lib.mi_gqa_decode_attn_cache(dq.ptr, dkr.ptr, dks.ptr, dvr.ptr, dvs.ptr, o2.ptr, B, Hq, Hkv, D, T_cap, dl.ptr, T, 0,
+                                             ws.ptr, nbytes, None))
+    a, b, c, codes, scales = (dev.download(x) for x in (o1, o2, orot, oq, osc))
+    assert np.all(dev.download(ws)[nbytes:] == 0x5A)     # nothing behind the workspace was written
+    dev.reset_to(mark)
+    for i in sorted({0, 1, B - 1} & set(range(B))):
+        n = int(lens[i])
+        args = (q[i:i + 1], kq[i:i + 1, :, :n], ks[i:i + 1, :, :n], vq[i:i + 1, :, :n], vs[i:i + 1, :, :n])
+        oo, oor = orc.gqa_decode(*args), orc.gqa_decode(*args, out_rotated=True)
+        assert max(np.max(np.abs(a[i] - oo[0])), np.max(np.abs(b[i] - oo[0])), np.max(np.abs(c[i] - oor[0]))) <= 2e-5, i
+        cq, cs = orc.quant_row(c[i].reshape(-1))
+        assert np.array_equal(codes[i], cq) and scales[i] == cs, i
