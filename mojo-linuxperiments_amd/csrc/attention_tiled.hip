@@ -692,7 +692,6 @@ static Plan pick(int64_t B, int64_t Hq, int64_t Hkv, int64_t T, bool quant)
     const int blocks = (int)((T + 63) / 64);
     const int64_t rows = B * Hkv, cus = compute_units();
     Plan pl;
-    auto cut = [&](int s) { pl.per = (blocks + s - 1) / s, pl.splits = (blocks + pl.per - 1) / pl.per; };
     const int fewest = (blocks + 4 * NT_MAX - 1) / (4 * NT_MAX);
     if (rows * fewest < cus) {
         // (one sequence is cut alike with codes and without: the call with the projection makes its codes either way)

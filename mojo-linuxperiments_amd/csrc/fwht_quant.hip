@@ -16,6 +16,8 @@
 // Every load is a float4 and the BLOCK/8 neighbouring lanes of a block read
 // 2*BLOCK contiguous bytes (whole 128-byte lines); the codes leave as one
 // dword per float4.  The kernel reads 4 B and writes 1 B per element: HBM-bound.
+#include <algorithm>
+
 #include "common.h"
 #include "fwht_core.h"
 
@@ -114,6 +116,10 @@ struct QuantBatch {
 // CMAX: the most 8-float chunks per thread any set of the batch needs.  The kernel's registers are those of its
 // widest row body whichever set a workgroup works on, so a batch of rows up to K = 14336 is not made to run at the
 // occupancy of the K = 32768 body (160 registers, three waves per SIMD).
+// Bound by HBM.  The longest rows go first, so that the launch does not end on them.  The three inputs of a layer's projections
+// (K = 4096, 4096, 14336), us in the callers' order -> here: 509 rows 12.7 -> 11.7, 1024 24.6 -> 22.2, 2048 43.7 -> 41.9; with the
+// contraction behind them 800 rows 206 -> 204, 1024 210 -> 208, 2048 391 -> 387.  (Read past the caches as well, 12.1, 20.3 and 37.0
+// by itself, and nothing with the contraction, which runs against the power limit.)
 template <int BLOCK, int CMAX>
 __global__ __launch_bounds__(256) void k_fwht_rows_batch(const QuantBatch b)
 {
@@ -348,6 +354,7 @@ extern "C" int32_t mi_fwht_quant_batch_f32_i8(const mi_quant_rows *sets, int32_t
     if (!sets || n < 1 || n > QUANT_BATCH_MAX) return MI_EINVAL;
     QuantBatch b = {};
     int64_t rows = 0;
+    int order[QUANT_BATCH_MAX];
     bool one_launch = true;
     for (int i = 0; i < n; ++i) {
         const mi_quant_rows &s = sets[i];
@@ -357,12 +364,8 @@ extern "C" int32_t mi_fwht_quant_batch_f32_i8(const mi_quant_rows *sets, int32_t
         // the batched kernel is the row-per-workgroup form at 256 threads; shorter rows (or a set without rows)
         // take the single launches, whose results are the same
         if (s.K < 2048 || s.M == 0) one_launch = false;
-        b.s[i].x = s.x;
-        b.s[i].q = s.q;
-        b.s[i].scale = s.scale;
-        b.s[i].K = (int)s.K;
-        b.s[i].first_row = (int)rows;
         rows += s.M;
+        order[i] = i;
     }
     if (rows > 0x7fffffffLL) return MI_ERANGE;
     if (!one_launch) {
@@ -372,9 +375,15 @@ extern "C" int32_t mi_fwht_quant_batch_f32_i8(const mi_quant_rows *sets, int32_t
         }
         return MI_OK;
     }
+    std::stable_sort(order, order + n, [&](int i, int j) { return sets[i].K > sets[j].K; });
     b.n = n;
-    int cmax = 1;
-    for (int i = 0; i < n; ++i) cmax = std::max(cmax, (b.s[i].K / 8 + 255) / 256);
+    int first = 0;
+    for (int i = 0; i < n; ++i) {
+        const mi_quant_rows &s = sets[order[i]];
+        b.s[i] = {s.x, s.q, s.scale, (int)s.K, first};
+        first += (int)s.M;
+    }
+    const int cmax = (b.s[0].K / 8 + 255) / 256;
 #define MI_QBATCH(BLOCK_, CMAX_) \
     launch_kernel((k_fwht_rows_batch<BLOCK_, CMAX_>), dim3((unsigned)rows), dim3(256), 0, as_stream(stream), b)
     if (block == 128) {
