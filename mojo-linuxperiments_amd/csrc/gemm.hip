@@ -146,9 +146,9 @@ extern "C" int32_t mi_rmsnorm_linear_f32(const float *x, const float *residual, 
     if (!x || !g || !sw || !aligned16(sw) || !aligned16(x) || !aligned16(g) || !(eps >= 0.0f)) return MI_EINVAL;
     if (residual && (!h_out || !aligned16(residual) || !aligned16(h_out))) return MI_EINVAL;
     if (xn_out && !aligned16(xn_out)) return MI_EINVAL;
-    // one token: one kernel (MI_EINVAL = a shape that it does not cover, or buffers that share memory: a residual stream updated
+    // one to four tokens: one kernel (MI_EINVAL = a shape that it does not cover, or buffers that share memory: a residual stream updated
     // in place takes the two kernels, whose row operator reads each element before it writes it)
-    if (M == 1 && block == 128) {
+    if (M >= 1 && M <= 4 && block == 128) {
         rc = launch_norm_linear_fused(x, residual, g, eps, h_out, xn_out, qw, sw, y, qx, sx, M, N, K, as_stream(stream));
         if (rc != MI_EINVAL) return rc;
     }
@@ -180,7 +180,7 @@ static int32_t linear_with(const float *x, const int8_t *qw, const float *sw, fl
     int32_t rc = check_gemm(qx, qw, y, M, N, K);
     if (rc) return rc;
     if (!x || !sw || !aligned16(sw)) return MI_EINVAL;
-    if (M == 1 && block == 128 && aligned16(x)) {
+    if (M >= 1 && M <= 4 && block == 128 && aligned16(x)) {
         // decode: one kernel that quantizes its own activations (MI_EINVAL as above)
         rc = launch_linear_fused(x, qw, sw, y, qx, sx, M, N, K, as_stream(stream), true);
         if (rc != MI_EINVAL) return rc;

@@ -6,8 +6,8 @@
 //  k_gemv_reg: a lane always works on the same byte offsets of a weight row, so its share of the activation codes
 //  lives in registers for the whole kernel: no LDS and no barrier in the streaming part, 16 x 1 KB weight loads in
 //  flight per wave, v_dot4_i32_i8, one transposed butterfly per wave.
-//  k_gemv_row makes the codes of its one token itself (rotate + quantize, with RMSNorm or SwiGLU in front), for K up to
-//  16384.
+//  k_gemv_row makes the codes of its one token, or its two to four, itself (rotate + quantize, with RMSNorm or SwiGLU in front),
+//  for K up to 16384 (4096).
 #include <algorithm>
 #include "common.h"
 #include "fwht_core.h"
@@ -157,17 +157,20 @@ struct RowArgs {
     float eps;
 };
 
-// CW: 1024-byte chunks of a weight row, the last one shorter unless WHOLE.
-template <int CW, bool WHOLE, int R, RowOp OP>
+// CW: 1024-byte chunks of a weight row, the last one shorter unless WHOLE.  MB: tokens, M of which are there (the last one is made
+// again for the others), each with a row of its own at K floats from the one before.
+template <int CW, bool WHOLE, int R, RowOp OP, int MB>
 __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x, const int8_t *__restrict__ qw,
                                                      const float *__restrict__ sw, float *__restrict__ y,
-                                                     int8_t *__restrict__ qx_out, float *__restrict__ sx_out, int N, int K,
+                                                     int8_t *__restrict__ qx_out, float *__restrict__ sx_out, int N, int K, int M,
                                                      RowArgs ra)
 {
+    static_assert(MB == 1 || MB == 2 || MB == 4, "");
+    static_assert(MB == 1 || OP == ROT || OP == NORM, "");
     constexpr int BLOCK = 128, LPB = BLOCK / 8, WG = 8;
-    constexpr int V = pow2_ceil(R), CQ = (CW + 3) / 4;   // chunks of 8 floats a thread
-    __shared__ __attribute__((aligned(16))) int8_t s_x[CW * 1024];   // codes
-    __shared__ float s_max[WG], s_sum[WG * CQ];                      // row maxima, sums of squares
+    constexpr int V = pow2_ceil(R * MB), CQ = (CW + 3) / 4;   // chunks of 8 floats a thread
+    __shared__ __attribute__((aligned(16))) int8_t s_x[MB][CW * 1024];   // codes
+    __shared__ float s_max[MB][WG], s_sum[MB][WG * CQ];                  // row maxima, sums of squares
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned waves = gridDim.x * WG, id = blockIdx.x * WG + wave;
@@ -195,25 +198,31 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
     // thread t owns chunks t, t + 512, ... of the row, in the layout of fwht_core.h
     const int j = tid % LPB, nchunk = K / 8;
     const bool keeper = blockIdx.x == 0;
-    float v[CQ][8];
+    float v[MB][CQ][8];
     int base[CQ];
-    float4 gl[CQ], gh[CQ], rl[CQ], rh[CQ];
+    float4 gl[CQ], gh[CQ], rl[MB][CQ], rh[MB][CQ];
 #pragma unroll
     for (int i = 0; i < CQ; ++i) {
         const int c = tid + i * 512;
         base[i] = (c / LPB) * BLOCK + 4 * j;
         if (c < nchunk) {
-            const float4 lo = *reinterpret_cast<const float4 *>(x + base[i]);
-            const float4 hi = *reinterpret_cast<const float4 *>(x + base[i] + BLOCK / 2);
-            v[i][0] = lo.x; v[i][1] = lo.y; v[i][2] = lo.z; v[i][3] = lo.w;
-            v[i][4] = hi.x; v[i][5] = hi.y; v[i][6] = hi.z; v[i][7] = hi.w;
+#pragma unroll
+            for (int m = 0; m < MB; ++m) {
+                const int64_t of = MB == 1 ? base[i] : (int64_t)min(m, M - 1) * K + base[i];
+                const float4 lo = *reinterpret_cast<const float4 *>(x + of);
+                const float4 hi = *reinterpret_cast<const float4 *>(x + of + BLOCK / 2);
+                v[m][i][0] = lo.x; v[m][i][1] = lo.y; v[m][i][2] = lo.z; v[m][i][3] = lo.w;
+                v[m][i][4] = hi.x; v[m][i][5] = hi.y; v[m][i][6] = hi.z; v[m][i][7] = hi.w;
+                if constexpr (OP == NORM) {
+                    if (ra.res) {
+                        rl[m][i] = *reinterpret_cast<const float4 *>(ra.res + of);
+                        rh[m][i] = *reinterpret_cast<const float4 *>(ra.res + of + BLOCK / 2);
+                    }
+                }
+            }
             if constexpr (OP == NORM) {
                 gl[i] = *reinterpret_cast<const float4 *>(ra.g + base[i]);
                 gh[i] = *reinterpret_cast<const float4 *>(ra.g + base[i] + BLOCK / 2);
-                if (ra.res) {
-                    rl[i] = *reinterpret_cast<const float4 *>(ra.res + base[i]);
-                    rh[i] = *reinterpret_cast<const float4 *>(ra.res + base[i] + BLOCK / 2);
-                }
             }
             if constexpr (OP == SWIGLU) {
                 gl[i] = *reinterpret_cast<const float4 *>(x + K + base[i]);
@@ -221,51 +230,66 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
             }
         } else {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[i][e] = 0.0f;
+            for (int m = 0; m < MB; ++m)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[m][i][e] = 0.0f;
         }
     }
     v4i wa[R][CW], wb[R][CW];
     load_w(wa, row0);
     load_w(wb, row0 + next);
 
-    auto leave = [&](float *to) {   // the row as it stands
+    auto leave = [&](float *to) {   // the rows as they stand
 #pragma unroll
-        for (int i = 0; i < CQ; ++i)
-            if (tid + i * 512 < nchunk) {
-                *reinterpret_cast<float4 *>(to + base[i]) = make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
-                *reinterpret_cast<float4 *>(to + base[i] + BLOCK / 2) = make_float4(v[i][4], v[i][5], v[i][6], v[i][7]);
-            }
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int i = 0; i < CQ; ++i)
+                if (tid + i * 512 < nchunk && (MB == 1 || m < M)) {
+                    float *const at = to + (int64_t)m * K + base[i];
+                    *reinterpret_cast<float4 *>(at) = make_float4(v[m][i][0], v[m][i][1], v[m][i][2], v[m][i][3]);
+                    *reinterpret_cast<float4 *>(at + BLOCK / 2) = make_float4(v[m][i][4], v[m][i][5], v[m][i][6], v[m][i][7]);
+                }
     };
     if constexpr (OP == NORM) {
-        float ss[CQ];   // per chunk, then per group of 64 chunks (group wave + 8 i): the order of fwht_core.h
+        float ss[MB][CQ];   // per chunk, then per group of 64 chunks (group wave + 8 i): the order of fwht_core.h
 #pragma unroll
-        for (int i = 0; i < CQ; ++i) {
-            ss[i] = 0.0f;
-            if (tid + i * 512 < nchunk) {
-                if (ra.res) {
-                    v[i][0] = v[i][0] + rl[i].x; v[i][1] = v[i][1] + rl[i].y; v[i][2] = v[i][2] + rl[i].z; v[i][3] = v[i][3] + rl[i].w;
-                    v[i][4] = v[i][4] + rh[i].x; v[i][5] = v[i][5] + rh[i].y; v[i][6] = v[i][6] + rh[i].z; v[i][7] = v[i][7] + rh[i].w;
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int i = 0; i < CQ; ++i) {
+                float (&w)[8] = v[m][i];
+                ss[m][i] = 0.0f;
+                if (tid + i * 512 < nchunk) {
+                    if (ra.res) {
+                        const float4 &lo = rl[m][i], &hi = rh[m][i];
+                        w[0] = w[0] + lo.x; w[1] = w[1] + lo.y; w[2] = w[2] + lo.z; w[3] = w[3] + lo.w;
+                        w[4] = w[4] + hi.x; w[5] = w[5] + hi.y; w[6] = w[6] + hi.z; w[7] = w[7] + hi.w;
+                    }
+                    ss[m][i] = chunk_sumsq(w);
                 }
-                ss[i] = chunk_sumsq(v[i]);
             }
-        }
         if (ra.res && keeper) leave(ra.h_out);
 #pragma unroll
-        for (int i = 0; i < CQ; ++i) {
-            ss[i] = group_sum(ss[i]);
-            if (lane == 0) s_sum[wave + WG * i] = ss[i];
-        }
-        __syncthreads();
-        const float total = tree_sum<WG * CQ>(s_sum);
-        const float r = 1.0f / sqrtf(total / (float)K + ra.eps);
+        for (int m = 0; m < MB; ++m)
 #pragma unroll
-        for (int i = 0; i < CQ; ++i)
-            if (tid + i * 512 < nchunk) {
-                v[i][0] = (v[i][0] * r) * gl[i].x; v[i][1] = (v[i][1] * r) * gl[i].y;
-                v[i][2] = (v[i][2] * r) * gl[i].z; v[i][3] = (v[i][3] * r) * gl[i].w;
-                v[i][4] = (v[i][4] * r) * gh[i].x; v[i][5] = (v[i][5] * r) * gh[i].y;
-                v[i][6] = (v[i][6] * r) * gh[i].z; v[i][7] = (v[i][7] * r) * gh[i].w;
+            for (int i = 0; i < CQ; ++i) {
+                ss[m][i] = group_sum(ss[m][i]);
+                if (lane == 0) s_sum[m][wave + WG * i] = ss[m][i];
             }
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+            const float total = tree_sum<WG * CQ>(s_sum[m]);
+            const float r = 1.0f / sqrtf(total / (float)K + ra.eps);
+#pragma unroll
+            for (int i = 0; i < CQ; ++i)
+                if (tid + i * 512 < nchunk) {
+                    float (&w)[8] = v[m][i];
+                    w[0] = (w[0] * r) * gl[i].x; w[1] = (w[1] * r) * gl[i].y;
+                    w[2] = (w[2] * r) * gl[i].z; w[3] = (w[3] * r) * gl[i].w;
+                    w[4] = (w[4] * r) * gh[i].x; w[5] = (w[5] * r) * gh[i].y;
+                    w[6] = (w[6] * r) * gh[i].z; w[7] = (w[7] * r) * gh[i].w;
+                }
+        }
     }
     if constexpr (OP == SWIGLU) {
 #pragma unroll
@@ -273,64 +297,85 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
             const float up[8] = {gl[i].x, gl[i].y, gl[i].z, gl[i].w, gh[i].x, gh[i].y, gh[i].z, gh[i].w};
             if (tid + i * 512 < nchunk) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[i][e] = silu(v[i][e]) * up[e];
+                for (int e = 0; e < 8; ++e) v[0][i][e] = silu(v[0][i][e]) * up[e];
             }
         }
     }
     if constexpr (OP == NORM || OP == SWIGLU) {
         if (keeper && ra.xn_out) leave(ra.xn_out);
     }
-    float amax = 0.0f;
 #pragma unroll
-    for (int i = 0; i < CQ; ++i) {
-        if constexpr (OP != PLAIN) fwht_codes<BLOCK>(v[i], j);
-        amax = fmaxf(amax, abs8(v[i]));
-    }
-    amax = max_lanes<64>(amax);
-    if (lane == 0) s_max[wave] = amax;
-    __syncthreads();
-    float a = s_max[0];
+    for (int m = 0; m < MB; ++m) {
+        float amax = 0.0f;
 #pragma unroll
-    for (int w = 1; w < WG; ++w) a = fmaxf(a, s_max[w]);
-    const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
-    const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
-    if (keeper && tid == 0) *sx_out = sc;
-#pragma unroll
-    for (int i = 0; i < CQ; ++i)
-        if (tid + i * 512 < nchunk) {
-            const uint32_t c0 = quant4(v[i][0], v[i][1], v[i][2], v[i][3], inv);
-            const uint32_t c1 = quant4(v[i][4], v[i][5], v[i][6], v[i][7], inv);
-            *reinterpret_cast<uint32_t *>(s_x + base[i]) = c0;
-            *reinterpret_cast<uint32_t *>(s_x + base[i] + BLOCK / 2) = c1;
-            if (keeper) {
-                *reinterpret_cast<uint32_t *>(qx_out + base[i]) = c0;
-                *reinterpret_cast<uint32_t *>(qx_out + base[i] + BLOCK / 2) = c1;
-            }
+        for (int i = 0; i < CQ; ++i) {
+            if constexpr (OP != PLAIN) fwht_codes<BLOCK>(v[m][i], j);
+            amax = fmaxf(amax, abs8(v[m][i]));
         }
+        amax = max_lanes<64>(amax);
+        if (lane == 0) s_max[m][wave] = amax;
+    }
+    __syncthreads();
+    float scs[MB];
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+        float a = s_max[m][0];
+#pragma unroll
+        for (int w = 1; w < WG; ++w) a = fmaxf(a, s_max[m][w]);
+        const float sc = (a == 0.0f) ? 1.0f : a / 127.0f;
+        const float inv = (a == 0.0f) ? 0.0f : 127.0f / a;
+        scs[m] = sc;
+        if (MB > 1 && m >= M) continue;
+        if (keeper && tid == 0) sx_out[m] = sc;
+#pragma unroll
+        for (int i = 0; i < CQ; ++i)
+            if (tid + i * 512 < nchunk) {
+                const uint32_t c0 = quant4(v[m][i][0], v[m][i][1], v[m][i][2], v[m][i][3], inv);
+                const uint32_t c1 = quant4(v[m][i][4], v[m][i][5], v[m][i][6], v[m][i][7], inv);
+                *reinterpret_cast<uint32_t *>(s_x[m] + base[i]) = c0;
+                *reinterpret_cast<uint32_t *>(s_x[m] + base[i] + BLOCK / 2) = c1;
+                if (keeper) {
+                    int8_t *const to = qx_out + (int64_t)m * K + base[i];
+                    *reinterpret_cast<uint32_t *>(to) = c0;
+                    *reinterpret_cast<uint32_t *>(to + BLOCK / 2) = c1;
+                }
+            }
+    }
     __syncthreads();
 
-    v4i xr[CW];
+    v4i xr[MB][CW];
 #pragma unroll
-    for (int c = 0; c < CW; ++c) xr[c] = *reinterpret_cast<const v4i *>(s_x + kbase + c * 1024);
-    if (!WHOLE && kbase + (CW - 1) * 1024 >= K) xr[CW - 1] = (v4i){0, 0, 0, 0};
+    for (int m = 0; m < MB; ++m) {
+        const int8_t *const from = s_x[MB == 1 ? 0 : min(m, M - 1)] + kbase;
+#pragma unroll
+        for (int c = 0; c < CW; ++c) xr[m][c] = *reinterpret_cast<const v4i *>(from + c * 1024);
+        if (!WHOLE && kbase + (CW - 1) * 1024 >= K) xr[m][CW - 1] = (v4i){0, 0, 0, 0};
+    }
+    // value r * MB + m of a group: row r of token m
     constexpr int SH = 6 - __builtin_ctz(V);
-    const int vi = lane >> SH;
-    const bool speaker = (lane & ((1 << SH) - 1)) == 0 && vi < R;
+    const int vi = lane >> SH, mi = vi % MB, ri = vi / MB;
+    const bool speaker = (lane & ((1 << SH) - 1)) == 0 && ri < R && (MB == 1 || mi < M);
+    float sc = scs[0];
+#pragma unroll
+    for (int m = 1; m < MB; ++m) sc = mi == m ? scs[m] : sc;
+    float *const yt = y + (int64_t)mi * N + ri;
     auto rows = [&](v4i (&w)[R][CW], int row) {
         int p[V];
 #pragma unroll
         for (int i = 0; i < V; ++i) p[i] = 0;
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            int d = 0;
+        for (int r = 0; r < R; ++r)
 #pragma unroll
-            for (int c = 0; c < CW; ++c)
+            for (int m = 0; m < MB; ++m) {
+                int d = 0;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) d = __builtin_amdgcn_sdot4(w[r][c][q], xr[c][q], d, false);
-            p[r] = d;
-        }
+                for (int c = 0; c < CW; ++c)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) d = __builtin_amdgcn_sdot4(w[r][c][q], xr[m][c][q], d, false);
+                p[r * MB + m] = d;
+            }
         fold_sum<V, 32>(p, lane);
-        if (speaker && row + vi < row1) y[row + vi] = ((float)p[0] * sc) * sw[row + vi];
+        if (speaker && row + ri < row1) yt[row] = ((float)p[0] * sc) * sw[row + ri];
     };
     int row = row0;
 #pragma unroll 1
@@ -350,21 +395,22 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
 // against 25.9 us; with the norm 21.4 against 20.4, of 65536 rows 44.9 against 45.9).  From five chunks on two a unit pay beyond six
 // rows a wave only (16384 x 5120 and the norm 18.2 -> 16.1, 6144 x 8192 12.9 -> 13.9), above eight chunks one is what the registers
 // hold.
-template <int CW, bool WHOLE, RowOp OP>
+template <int CW, bool WHOLE, RowOp OP, int MB>
 static void start_row(int cus, int per_wave, const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx,
-                      int N, int K, const RowArgs &ra, hipStream_t s)
+                      int N, int K, int M, const RowArgs &ra, hipStream_t s)
 {
     auto go = [&](auto R, int wgs) {
-        launch_kernel((k_gemv_row<CW, WHOLE, decltype(R)::value, OP>), dim3((unsigned)(wgs * cus)), dim3(512), 0, s, x, qw, sw, y,
-                      qx, sx, N, K, ra);
+        launch_kernel((k_gemv_row<CW, WHOLE, decltype(R)::value, OP, MB>), dim3((unsigned)(wgs * cus)), dim3(512), 0, s, x, qw, sw,
+                      y, qx, sx, N, K, M, ra);
     };
     using std::integral_constant;
+    if constexpr (MB == 4) return go(integral_constant<int, 1>{}, 2);   // (many rows, see rows_take)
     if (per_wave <= 2) return go(integral_constant<int, 1>{}, 1);
     if constexpr (CW <= 4) {
         if (per_wave <= 4) return go(integral_constant<int, 2>{}, 1);
         if constexpr (CW <= 2)
             if (per_wave <= 8) return go(integral_constant<int, 4>{}, 1);
-        return go(integral_constant<int, 1>{}, CW == 4 && per_wave > (OP == NORM ? 20 : 10) ? 3 : 2);
+        return go(integral_constant<int, 1>{}, MB == 1 && CW == 4 && per_wave > (OP == NORM ? 20 : 10) ? 3 : 2);
     }
     go(integral_constant<int, 1>{}, CW <= 8 && per_wave > 6 ? 2 : 1);
 }
@@ -395,8 +441,8 @@ static int32_t launch_row(const float *x, const int8_t *qw, const float *sw, flo
     switch ((K + 1023) >> 10) {
 #define MI_ROW(CW_)                                                                                                          \
     case CW_:                                                                                                                \
-        if (K % 1024) start_row<CW_, false, OP>(cus, per_wave, x, qw, sw, y, qx, sx, (int)N, (int)K, ra, s);                  \
-        else start_row<CW_, true, OP>(cus, per_wave, x, qw, sw, y, qx, sx, (int)N, (int)K, ra, s);                            \
+        if (K % 1024) start_row<CW_, false, OP, 1>(cus, per_wave, x, qw, sw, y, qx, sx, (int)N, (int)K, 1, ra, s);            \
+        else start_row<CW_, true, OP, 1>(cus, per_wave, x, qw, sw, y, qx, sx, (int)N, (int)K, 1, ra, s);                      \
         break;
         MI_ROW(1) MI_ROW(2) MI_ROW(3) MI_ROW(4) MI_ROW(5) MI_ROW(6) MI_ROW(7) MI_ROW(8)
     default:
@@ -410,11 +456,48 @@ static int32_t launch_row(const float *x, const int8_t *qw, const float *sw, flo
     return launch_status();
 }
 
+// The same for two tokens, and for three and four where the rows are many: every workgroup makes all the codes, which two launches
+// do once.  us of two launches -> one, weights from HBM, linear and with the norm, K = 512 to 4096, N = 16 to 40960: two tokens 0.69 to
+// 1.00 of the time and 0.75 to 1.02 (4096 x 4096 7.6 -> 5.7 and 8.5 -> 7.5, 28672 x 4096 25.3 -> 21.3 and 26.1 -> 21.9); three and four
+// from 80 rows a unit and K = 2048 on 0.83 to 1.00 and 0.87 to 1.01 (four, 28672 x 4096 25.7 -> 22.4 and 26.3 -> 23.6), fewer and
+// shorter rows 0.87 to 1.11 and up to 1.29.
+static bool rows_take(int64_t M, int64_t N, int64_t K)
+{
+    if (M < 2 || M > 4 || K > 4096 || !row_takes(N, K)) return false;
+    return M == 2 || (K >= 2048 && N > 80 * compute_units());
+}
+
+template <RowOp OP>
+static int32_t launch_rows_of(const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx, int64_t M,
+                              int64_t N, int64_t K, const RowArgs &ra, hipStream_t s)
+{
+    if (!rows_take(M, N, K) || !apart({{x, M * K * 4}, {ra.res, M * K * 4}, {ra.g, K * 4}},
+                                      {{y, M * N * 4}, {qx, M * K}, {sx, M * 4}, {ra.h_out, M * K * 4}, {ra.xn_out, M * K * 4}}))
+        return MI_EINVAL;
+    const int cus = compute_units(), per_wave = (int)((N + 8 * cus - 1) / (8 * cus));
+    switch ((K + 1023) >> 10) {
+#define MI_ROWS1(CW_, WHOLE_, MB_) start_row<CW_, WHOLE_, OP, MB_>(cus, per_wave, x, qw, sw, y, qx, sx, (int)N, (int)K, (int)M, ra, s)
+#define MI_ROWS(CW_)                                                          \
+    case CW_:                                                                 \
+        if (M == 2 && K % 1024) MI_ROWS1(CW_, false, 2);                      \
+        else if (M == 2) MI_ROWS1(CW_, true, 2);                              \
+        else if constexpr (CW_ == 1) return MI_EINVAL;                        \
+        else if (K % 1024) MI_ROWS1(CW_, false, 4);                           \
+        else MI_ROWS1(CW_, true, 4);                                          \
+        break;
+        MI_ROWS(1) MI_ROWS(2) MI_ROWS(3) MI_ROWS(4)
+#undef MI_ROWS
+#undef MI_ROWS1
+    default: return MI_EINVAL;
+    }
+    return launch_status();
+}
+
 int32_t launch_linear_fused(const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx,
                             int64_t M, int64_t N, int64_t K, hipStream_t s, bool rotate)
 {
-    if (M != 1) return MI_EINVAL;
     const RowArgs none = {};
+    if (M != 1) return rotate ? launch_rows_of<ROT>(x, qw, sw, y, qx, sx, M, N, K, none, s) : MI_EINVAL;
     return rotate ? launch_row<ROT>(x, qw, sw, y, qx, sx, N, K, none, s) : launch_row<PLAIN>(x, qw, sw, y, qx, sx, N, K, none, s);
 }
 
@@ -423,8 +506,8 @@ int32_t launch_norm_linear_fused(const float *x, const float *res, const float *
                                  float *xn_out, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx,
                                  int64_t M, int64_t N, int64_t K, hipStream_t s)
 {
-    if (M != 1) return MI_EINVAL;
-    return launch_row<NORM>(x, qw, sw, y, qx, sx, N, K, RowArgs{res, g, h_out, xn_out, eps}, s);
+    const RowArgs ra{res, g, h_out, xn_out, eps};
+    return M == 1 ? launch_row<NORM>(x, qw, sw, y, qx, sx, N, K, ra, s) : launch_rows_of<NORM>(x, qw, sw, y, qx, sx, M, N, K, ra, s);
 }
 int32_t launch_swiglu_linear_fused(const float *gate_up, float *h_out, const int8_t *qw, const float *sw, float *y, int8_t *q,
                                    float *scale, int64_t M, int64_t N, int64_t K, hipStream_t s)

@@ -268,3 +268,41 @@ def test_argument_errors(mi, dev):
     assert lib.mi_w8a8_gemm_i32(b.ptr, b.ptr, b.ptr, 0, 16, 128, None) == mi.OK
     assert lib.mi_w8a8_linear_f32(b.ptr, b.ptr, b.ptr, b.ptr, 4, 16, 128, 128, b.ptr, 16, None) == mi.ENOSPC
     dev.reset_to(mark)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (2, 16, 128), (2, 2064, 512), (2, 4096, 1024), (2, 6144, 4096), (2, 8208, 4096), (2, 16400, 2048), (2, 33040, 2176), (2, 41024, 3968),
+    (3, 20480, 2048), (3, 20496, 2048), (4, 20496, 2176), (3, 28672, 4096), (4, 33040, 3968),
+])
+@pytest.mark.parametrize("norm", [False, True])
+def test_few_tokens_in_one_launch_are_the_two_launches(mi, dev, M, N, K, norm):
+    """Rows a wave from none to many, whole chunks of K and not, both sides of the rule: y, codes, scales and the residual sum are
+    those of the row kernel and the contraction, bit for bit, and nothing is written past the last token's row."""
+    mark = dev.mark()
+    g = np.random.default_rng(M * N + K)
+    x, res = (dev.upload(g.standard_normal((M, K), dtype=np.float32)) for _ in range(2))
+    gain = dev.upload(1 + 0.1 * g.standard_normal(K, dtype=np.float32))
+    qw, sw = dev.upload(g.integers(-127, 128, (N, K), dtype=np.int8)), dev.upload(g.random(N, dtype=np.float32))
+    poison = np.full(M + 1, np.nan, np.float32)
+    y = dev.upload(np.repeat(poison[:, None], N, 1))
+    h = dev.upload(np.repeat(poison[:, None], K, 1))
+    xn = dev.upload(np.repeat(poison[:, None], K, 1))
+    ws = dev.empty(mi.lib.mi_w8a8_linear_workspace_bytes(M, N, K), np.uint8)
+    q, s, y2, h2, xn2 = dev.empty((M, K), np.int8), dev.empty(M, np.float32), dev.empty((M, N), np.float32), dev.empty((M, K), np.float32), dev.empty((M, K), np.float32)
+    if norm:
+        mi.check(mi.lib.mi_rmsnorm_linear_f32(x.ptr, res.ptr, gain.ptr, 1e-5, h.ptr, xn.ptr, qw.ptr, sw.ptr, y.ptr, M, N, K, 128, ws.ptr,
+                                              ws.nbytes, None))
+        mi.check(mi.lib.mi_rmsnorm_quant_f32_i8(x.ptr, res.ptr, gain.ptr, 1e-5, h2.ptr, xn2.ptr, q.ptr, s.ptr, M, K, 128, None))
+    else:
+        mi.check(mi.lib.mi_w8a8_linear_f32(x.ptr, qw.ptr, sw.ptr, y.ptr, M, N, K, 128, ws.ptr, ws.nbytes, None))
+        mi.fwht_quant(x, q, s, 128)
+    mi.gemm_dequant(q, s, qw, sw, y2)
+    al = (M * K + 255) // 256 * 256
+    assert np.array_equal(dev.download(ws.offset(0, (M, K), np.int8)), dev.download(q))
+    assert np.array_equal(dev.download(ws.offset(al, (M,), np.float32)), dev.download(s))
+    got = dev.download(y)
+    assert np.array_equal(got[:M], dev.download(y2)) and np.isnan(got[M]).all()
+    for a, b in ((h, h2), (xn, xn2)) if norm else ():
+        got = dev.download(a)
+        assert np.array_equal(got[:M], dev.download(b)) and np.isnan(got[M]).all()
+    dev.reset_to(mark)
