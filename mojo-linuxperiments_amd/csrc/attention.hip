@@ -36,18 +36,6 @@ namespace attn {
 
 constexpr int D = 128;
 
-template <int MASK>
-__device__ __forceinline__ float lane_xor(float v)
-{
-    const int i = __float_as_int(v);
-    int r;
-    if constexpr (MASK == 1) r = __builtin_amdgcn_update_dpp(i, i, 0xB1, 0xf, 0xf, false);
-    else if constexpr (MASK == 2) r = __builtin_amdgcn_update_dpp(i, i, 0x4E, 0xf, 0xf, false);
-    else if constexpr (MASK < 32) r = __builtin_amdgcn_ds_swizzle(i, 0x1F | (MASK << 10));
-    else r = __shfl_xor(i, 32, 64);
-    return __int_as_float(r);
-}
-
 __device__ __forceinline__ void fwht128(float (&v)[8], int j) { fwht_chunk<D>(v, j); }   // fwht_core.h
 
 struct Params {
@@ -70,17 +58,6 @@ struct Params {
     float score_scale;    // log2(e) / sqrt(D)
 };
 
-// value of lane (lane ^ OFF) for OFF in {8, 16, 32}
-template <int OFF>
-__device__ __forceinline__ float slot_xor(float v)
-{
-    const int i = __float_as_int(v);
-    int r;
-    if constexpr (OFF == 8) r = __builtin_amdgcn_update_dpp(0, i, 0x128, 0xf, 0xf, true);   // row_ror:8
-    else if constexpr (OFF == 16) r = __builtin_amdgcn_ds_swizzle(i, 0x401F);
-    else r = __shfl_xor(i, 32, 64);
-    return __int_as_float(r);
-}
 // one round of the transposed butterfly over token slots: keep the half of the values whose index bit
 // matches this lane's OFF bit, hand the other half to lane ^ OFF
 template <int V, int OFF>
@@ -89,9 +66,17 @@ __device__ __forceinline__ void fold_slots(float (&p)[64], int lane)
     const bool hi = (lane & OFF) != 0;
 #pragma unroll
     for (int i = 0; i < V / 2; ++i) {
-        const float keep = hi ? p[i + V / 2] : p[i];
-        const float send = hi ? p[i] : p[i + V / 2];
-        p[i] = keep + slot_xor<OFF>(send);
+        if constexpr (OFF == 32) {   // the exchange is one instruction
+            const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[i]), __float_as_uint(p[i + V / 2]), false, false);
+            p[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        } else if constexpr (OFF == 16) {
+            const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(p[i]), __float_as_uint(p[i + V / 2]), false, false);
+            p[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        } else {
+            const float keep = hi ? p[i + V / 2] : p[i];
+            const float send = hi ? p[i] : p[i + V / 2];
+            p[i] = keep + __int_as_float(xor_lane_i<OFF>(__float_as_int(send)));
+        }
     }
 }
 
@@ -266,10 +251,10 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
     // of this wave is taken against the wave's own maximum and rescaled when the waves meet
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
-        m4[h] = fmaxf(m4[h], lane_xor<1>(m4[h]));
-        m4[h] = fmaxf(m4[h], lane_xor<2>(m4[h]));
-        m4[h] = fmaxf(m4[h], lane_xor<4>(m4[h]));
-        m4[h] = fmaxf(m4[h], lane_xor<8>(m4[h]));
+        m4[h] = fmaxf(m4[h], __int_as_float(xor_lane_i<1>(__float_as_int(m4[h]))));
+        m4[h] = fmaxf(m4[h], __int_as_float(xor_lane_i<2>(__float_as_int(m4[h]))));
+        m4[h] = fmaxf(m4[h], __int_as_float(xor_lane_i<4>(__float_as_int(m4[h]))));
+        m4[h] = fmaxf(m4[h], __int_as_float(xor_lane_i<8>(__float_as_int(m4[h]))));
     }
     if (lane == 0) { s_m[wave][0] = m4[0]; s_m[wave][1] = m4[1]; s_m[wave][2] = m4[2]; s_m[wave][3] = m4[3]; }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -314,7 +299,7 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
     fold_slots<64, 32>(flat, lane);
     fold_slots<32, 16>(flat, lane);
     fold_slots<16, 8>(flat, lane);
-    lsum += slot_xor<8>(lsum); lsum += slot_xor<16>(lsum); lsum += slot_xor<32>(lsum);
+    lsum = add_lane<32>(add_lane<16>(add_lane<8>(lsum)));
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int fl = 8 * slot + j;   // = 4*e + head

@@ -409,8 +409,8 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
         });
     });
     // maximum per head over the wave's tokens: lanes r16, r16 + 16, r16 + 32, r16 + 48 hold the partial maxima
-    mrun = fmaxf(mrun, xor_lane<16>(mrun));
-    mrun = fmaxf(mrun, __shfl_xor(mrun, 32, 64));
+    const auto larger = [](float a, float b) { return fmaxf(a, b); };
+    mrun = with_far_lane<32>(with_far_lane<16>(mrun, larger), larger);
     if (lane < 4) s_m[wave][lane] = mrun;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -463,8 +463,7 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
     // the sum of the weights of head hh: over the quad, then over the four chunks c4
     lsum += xor_lane<1>(lsum);
     lsum += xor_lane<2>(lsum);
-    lsum += xor_lane<16>(lsum);
-    lsum += __shfl_xor(lsum, 32, 64);
+    lsum = add_lane<32>(add_lane<16>(lsum));
     if ((lane & 0x33) == 0) s_l[wave][hh] = lsum;   // lanes 0, 4, 8, 12
 
     // ---- digits -> fp32.  Lane (r16, c4) holds column d = 16*n + r16 of rows 4*c4 + i: digit i of head c4, worth

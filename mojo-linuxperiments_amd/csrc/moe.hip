@@ -32,7 +32,6 @@ static uint32_t topk_magic(int topk)
 }
 constexpr int64_t DISPATCH_MAX_WORDS = 36864;  // 144 KB of the 160 KB LDS
 
-__device__ __forceinline__ float shfl_xor_f(float v, int m) { return __shfl_xor(v, m, 64); }
 
 // ---------------------------------------------------------------- a9 router
 // Workgroup = E/16 waves, 4 tokens.  Wave eg owns experts 16*eg .. 16*eg+15 for
@@ -51,9 +50,17 @@ __device__ __forceinline__ void fold(float (&p)[NP], int lane)
     const bool hi = (lane & OFF) != 0;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-        const float keep = hi ? p[i + N] : p[i];
-        const float send = hi ? p[i] : p[i + N];
-        p[i] = keep + shfl_xor_f(send, OFF);
+        if constexpr (OFF == 32) {   // the exchange is one instruction
+            const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[i]), __float_as_uint(p[i + N]), false, false);
+            p[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        } else if constexpr (OFF == 16) {
+            const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(p[i]), __float_as_uint(p[i + N]), false, false);
+            p[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        } else {
+            const float keep = hi ? p[i + N] : p[i];
+            const float send = hi ? p[i] : p[i + N];
+            p[i] = keep + __int_as_float(xor_lane_i<OFF>(__float_as_int(send)));
+        }
     }
 }
 
@@ -240,14 +247,13 @@ __global__ __launch_bounds__(256) void k_moe_logits(const float *__restrict__ x,
     } else if constexpr (EW == 1) {
         fold<32, 2>(p, lane);
         fold<16, 1>(p, lane);
-#pragma unroll
-        for (int off = 8; off >= 1; off >>= 1) p[0] = p[0] + shfl_xor_f(p[0], off);
+        p[0] = add_lane<1>(add_lane<2>(add_lane<4>(add_lane<8>(p[0]))));
         const int t = t0 + (lane >> 4);   // the 16 lanes of a group hold the same token's sum
         if ((lane & 15) == 0 && t < T) logits[(int64_t)t * E + e0] = p[0];
     } else {
         static_assert(EW == 8, "experts per wave");
 #pragma unroll
-        for (int i = 0; i < 32; ++i) p[i] = p[i] + shfl_xor_f(p[i], 32);
+        for (int i = 0; i < 32; ++i) p[i] = add_lane<32>(p[i]);
         fold<16, 16>(p, lane);
         fold<8, 8>(p, lane);
         fold<4, 4>(p, lane);
