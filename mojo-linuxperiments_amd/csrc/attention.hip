@@ -56,6 +56,7 @@ struct Params {
     int max_pages, page_shift;    // P = 1 << page_shift tokens per page, P >= 16
     int tiles_per_split;  // 16-token tiles
     float score_scale;    // log2(e) / sqrt(D)
+    int out_rotated;      // DIRECT kernels: leave the rows in the rotated basis of V; they are the output [B, Hq, 128], at part_o
 };
 
 // one round of the transposed butterfly over token slots: keep the half of the values whose index bit
@@ -91,7 +92,8 @@ constexpr int RING = 8;           // loads a wave keeps in flight (1 KB each); t
 // loads; otherwise every address is base + constant.  Tokens past the end of the split are masked in the scores.
 // PAGED: the cache is a pool of pages [page][kv head][P tokens][128]; a 16-token tile lies in one page, so a wave
 // looks up one page per tile (uniform over the wave) and lanes are clamped inside their tile.
-template <bool DUMP, bool RAGGED, bool PAGED, int WAVE_TILES>
+// DIRECT: the workgroup sees the whole sequence and writes the output rows itself.
+template <bool DUMP, bool RAGGED, bool PAGED, int WAVE_TILES, bool DIRECT>
 __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int8_t (&s_q)[4][4][D], float (&s_sq)[4][4],
                                                float (&s_red)[4][4][D], float (&s_sc)[4][WAVE_TILES][16][4],
                                                float (&s_m)[4][4], float (&s_l)[4][4])
@@ -310,28 +312,54 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
 
     // the four waves meet: rescale each wave's sums from its own maximum to the common one
     const int64_t pbase = ((int64_t)bkv * gridDim.x + split);
-    for (int o = tid; o < 4 * D; o += 256) {
-        const int h = o >> 7, d = o & (D - 1);
-        const float m = fmaxf(fmaxf(s_m[0][h], s_m[1][h]), fmaxf(s_m[2][h], s_m[3][h]));
-        float sum = 0.0f;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const float f = (s_m[w][h] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(s_m[w][h] - m);
-            sum += s_red[w][h][d] * f;
-        }
-        p.part_o[(pbase * 4 + h) * D + d] = sum;
-    }
-    if (tid < 4) {
-        const float m = fmaxf(fmaxf(s_m[0][tid], s_m[1][tid]), fmaxf(s_m[2][tid], s_m[3][tid]));
+    auto common = [&](int h) { return fmaxf(fmaxf(s_m[0][h], s_m[1][h]), fmaxf(s_m[2][h], s_m[3][h])); };
+    auto rescale = [&](int w, int h, float m) { return (s_m[w][h] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(s_m[w][h] - m); };
+    auto weights = [&](int h, float m) {
         float l = 0.0f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) l += (s_m[w][tid] == -INFINITY) ? 0.0f : s_l[w][tid] * __builtin_amdgcn_exp2f(s_m[w][tid] - m);
+        for (int w = 0; w < 4; ++w) l += (s_m[w][h] == -INFINITY) ? 0.0f : s_l[w][h] * __builtin_amdgcn_exp2f(s_m[w][h] - m);
+        return l;
+    };
+    float total[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int o = tid + 256 * i, h = o >> 7, d = o & (D - 1);
+        const float m = common(h);
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) sum += s_red[w][h][d] * rescale(w, h, m);
+        if constexpr (DIRECT) {
+            const float l = weights(h, m);
+            total[i] = l > 0.0f ? sum * (1.0f / l) : 0.0f;
+        } else {
+            p.part_o[(pbase * 4 + h) * D + d] = sum;
+        }
+    }
+    if constexpr (DIRECT) {
+        __syncthreads();   // every sum has been read
+#pragma unroll
+        for (int i = 0; i < 2; ++i) s_red[0][(tid + 256 * i) >> 7][tid & (D - 1)] = total[i];
+        __syncthreads();
+        if (tid < 64 && hr < G) {   // 16 lanes per head row, as the merge kernel has them
+            float *const orow = p.part_o + ((int64_t)b * p.Hq + kvh * G + hr) * D;
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = s_red[0][hr][4 * jj + e];
+                v[4 + e] = s_red[0][hr][64 + 4 * jj + e];
+            }
+            if (!p.out_rotated) fwht128(v, jj);
+            *reinterpret_cast<float4 *>(orow + 4 * jj) = make_float4(v[0], v[1], v[2], v[3]);
+            *reinterpret_cast<float4 *>(orow + 64 + 4 * jj) = make_float4(v[4], v[5], v[6], v[7]);
+        }
+    } else if (tid < 4) {
+        const float m = common(tid);
         p.part_ml[pbase * 8 + tid] = m;
-        p.part_ml[pbase * 8 + 4 + tid] = l;
+        p.part_ml[pbase * 8 + 4 + tid] = weights(tid, m);
     }
 }
 
-template <bool DUMP, int WAVE_TILES>
+template <bool DUMP, int WAVE_TILES, bool DIRECT>
 __global__ __launch_bounds__(256) void k_gqa_split(Params p)
 {
     __shared__ __attribute__((aligned(16))) int8_t s_q[4][4][D];
@@ -346,6 +374,11 @@ __global__ __launch_bounds__(256) void k_gqa_split(Params p)
         const int b = blockIdx.y / p.Hkv;
         T = min(max(__builtin_amdgcn_readfirstlane(p.seq_len[b]), 0), p.T);
         if (tile_lo * 16 >= T) {
+            if constexpr (DIRECT) {   // a sequence of length 0: rows of zeros
+                const int64_t row0 = (int64_t)b * p.Hq + (blockIdx.y % p.Hkv) * p.G;
+                for (int o = threadIdx.x; o < p.G * D; o += 256) p.part_o[row0 * D + o] = 0.0f;
+                return;
+            }
             // this split lies past the end of the sequence: an empty partial (weight 0 in the merge)
             const int64_t pbase = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x);
             for (int o = threadIdx.x; o < 4 * D; o += 256) p.part_o[pbase * 4 * D + o] = 0.0f;
@@ -357,12 +390,12 @@ __global__ __launch_bounds__(256) void k_gqa_split(Params p)
         }
     }
     if (p.block_table) {
-        gqa_split_body<false, true, true, WAVE_TILES>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
+        gqa_split_body<false, true, true, WAVE_TILES, DIRECT>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
         return;
     }
     const bool full = (tile_lo + 4 * WAVE_TILES) * 16 <= T;
-    if (full) gqa_split_body<DUMP, false, false, WAVE_TILES>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
-    else gqa_split_body<DUMP, true, false, WAVE_TILES>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
+    if (full) gqa_split_body<DUMP, false, false, WAVE_TILES, DIRECT>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
+    else gqa_split_body<DUMP, true, false, WAVE_TILES, DIRECT>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
 }
 
 // Merge of the splits of one (b, h) row by the 16 lanes that own it (lane j: elements 4j..4j+3 and 64+4j..).
@@ -722,13 +755,22 @@ static int32_t run_attn(const float *q, const int8_t *kq, const float *ks, const
     p.tiles_per_split = (ntiles + splits - 1) / splits;
     p.score_scale = 1.4426950408889634f * 0.08838834764831845f;  // log2(e) / sqrt(128)
     const dim3 grid((unsigned)splits, (unsigned)(B * Hkv));
-    if (plan.wave_tiles == attn::TILES_LONG) {
-        if (ddots) launch_kernel((attn::k_gqa_split<true, attn::TILES_LONG>), grid, dim3(256), 0, s, p);
-        else launch_kernel((attn::k_gqa_split<false, attn::TILES_LONG>), grid, dim3(256), 0, s, p);
-    } else {
-        if (ddots) launch_kernel((attn::k_gqa_split<true, attn::TILES_SHORT>), grid, dim3(256), 0, s, p);
-        else launch_kernel((attn::k_gqa_split<false, attn::TILES_SHORT>), grid, dim3(256), 0, s, p);
-    }
+    // one span: its workgroup writes the output rows, with the bits that the merge of one split gives them, and no merge is launched.
+    // us, 8 heads: one sequence of 64 tokens 8.4 -> 6.6, 32 of 64 8.9 -> 7.0, 32 of 600 14.2 -> 12.2.  (Output on top of the queries: row
+    // by row, or with a merge.)
+    const bool direct = splits == 1 && o && !oq && !ddots && (o == q || !overlaps(o, B * Hq * D * 4, q, B * Hq * D * 4));
+    if (direct) p.part_o = o;
+    p.out_rotated = out_rotated;
+#define MI_SPLIT(TILES)                                                                                       \
+    do {                                                                                                      \
+        if (ddots) launch_kernel((attn::k_gqa_split<true, TILES, false>), grid, dim3(256), 0, s, p);          \
+        else if (direct) launch_kernel((attn::k_gqa_split<false, TILES, true>), grid, dim3(256), 0, s, p);    \
+        else launch_kernel((attn::k_gqa_split<false, TILES, false>), grid, dim3(256), 0, s, p);               \
+    } while (0)
+    if (plan.wave_tiles == attn::TILES_LONG) MI_SPLIT(attn::TILES_LONG);
+    else MI_SPLIT(attn::TILES_SHORT);
+#undef MI_SPLIT
+    if (direct) return launch_status();
     rc = launch_status();
     if (rc) return rc;
     if (!o && !oq) return rc;

@@ -780,7 +780,8 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
     if (workspace_bytes < mi_gqa_decode_workspace_bytes(B, Hq, Hkv, D, T_max)) return MI_ENOSPC;
     const avt::Plan plan = avt::pick(B, Hq, Hkv, T_max, oq != nullptr);
     // one workgroup sees the whole sequence: it writes the output rows (the gate takes the split form: it wants no o)
-    const bool direct = plan.splits == 1 && !oq && !dbg;
+    const int64_t obytes = B * Hq * D * 4;   // (on top of the queries: row by row, or with a merge)
+    const bool direct = plan.splits == 1 && !oq && !dbg && (o == q || !overlaps(o, obytes, q, obytes));
     avt::StepParams p = {};
     p.q = q; p.kq = kq; p.ks = ks; p.vt = vt; p.vs = vs;
     p.Hq = (int)Hq; p.Hkv = (int)Hkv; p.G = (int)(Hq / Hkv); p.T = (int)T_max;

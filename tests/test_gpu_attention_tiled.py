@@ -675,3 +675,29 @@ def test_few_rows_are_cut_into_whole_rounds(mi, dev, orc, B, Hkv, T):
         assert max(np.max(np.abs(a[i] - oo[0])), np.max(np.abs(b[i] - oo[0])), np.max(np.abs(c[i] - oor[0]))) <= 2e-5, i
         cq, cs = orc.quant_row(c[i].reshape(-1))
         assert np.array_equal(codes[i], cq) and scales[i] == cs, i
+
+
+@pytest.mark.parametrize("lens", [[0, 200, 1], [256, 0, 255]])
+def test_rows_kernel_writes_the_output_of_one_span(mi, dev, orc, lens):
+    """Row-major, at most 256 tokens: no merge, zeros for an empty sequence, and the output on top of the queries, in place or a row
+    further on."""
+    mark = dev.mark()
+    B, Hq, Hkv, T, D = 3, 6, 2, 256, 128
+    q, kq, ks, vq, vs, _, _ = make_cache(mi, dev, 77, B, Hq, Hkv, T, T)
+    dk, dks, dv, dvs, dl = dev.upload(kq), dev.upload(ks), dev.upload(vq), dev.upload(vs), dev.upload(np.array(lens, np.int32))
+    ws = dev.empty(mi.lib.mi_gqa_decode_workspace_bytes(B, Hq, Hkv, D, T), np.uint8)
+    for rotated in (0, 1):
+        for shift in (None, 0, D):
+            both = dev.upload(np.concatenate([q.reshape(-1), np.full(D, np.nan, np.float32)]))
+            o = dev.upload(np.full((B, Hq, D), np.nan, np.float32)) if shift is None else both.offset(4 * shift, (B, Hq, D), np.float32)
+            mi.check(mi.lib.mi_gqa_decode_attn_cache(both.ptr, dk.ptr, dks.ptr, dv.ptr, dvs.ptr, o.ptr, B, Hq, Hkv, D, T, dl.ptr, T,
+                                                     rotated, ws.ptr, ws.nbytes, None))
+            got = dev.download(o)
+            for b, m in enumerate(lens):
+                if m == 0:
+                    assert np.all(got[b] == 0)
+                    continue
+                want = orc.gqa_decode(q[b:b + 1], kq[b:b + 1, :, :m], ks[b:b + 1, :, :m], vq[b:b + 1, :, :m], vs[b:b + 1, :, :m],
+                                      out_rotated=bool(rotated))
+                assert np.max(np.abs(got[b] - want[0])) <= 2e-5, (rotated, shift, b)
+    dev.reset_to(mark)
