@@ -604,7 +604,8 @@ int max_splits(int64_t B, int64_t Hkv, int64_t T);
 // holds), else of 704: a wave goes through all of its tiles, those past the end of its span as well, so a span that is not filled
 // costs what a full one does.  us, 8 heads, before -> here (a sequence of up to 256 tokens ran in a span of 704, and few rows were cut
 // into halves and quarters of 256): one sequence of 16 to 256 tokens 12.3 -> 8.9 (6.6 now that a single span needs no
-// merge), of 1531 10.1 -> 9.6, 4 of 1500 13.8 -> 9.9, 32 of 256 13.3 -> 10.1, 16 of 1000 14.6 -> 14.0; three workgroups a unit, 32 of 700, 16.9 in spans of 256 and 15.3 in one of 704.
+// merge), of 1531 10.1 -> 9.6, 4 of 1500 13.8 -> 9.9, 32 of 256 13.3 -> 10.1, 16 of 1000 14.6 -> 14.0;
+// three workgroups a unit, 32 of 700, 16.9 in spans of 256 and 15.3 in one of 704.
 static SplitPlan pick_splits(int64_t B, int64_t Hkv, int64_t T)
 {
     const int ntiles = (int)((T + 15) / 16);
