@@ -742,14 +742,21 @@ static_assert(2 * RX_LDS <= 160 * 1024, "two workgroups a unit");
 // than 48: 180 us for the layer's FFN with passes of 48, 176 with 64.)
 constexpr int rx_most(int nsmax) { return nsmax > 6 ? 32 : nsmax > 4 ? 48 : 64; }
 
-// Where the down kernel makes the codes of its rows itself (OWN) and the quantizer's launch between the two expert kernels goes: with
-// so few tokens that every expert's are one pass, and few of them an expert, since every workgroup of an expert makes all of its
-// codes.  Layer, top-8, H = 2048, I = 768, 128 experts, us with the launch -> without: 1 token 31.4 -> 28.0, 4 50.6 -> 45.7,
-// 16 92.9 -> 88.0, 32 117.6 -> 116.3; 32 tokens of 64 experts, top-4, H = 1024, I = 512 40.2 -> 38.2; 16 of 16 experts, 8 rows an
-// expert, H = 1024, I = 256 28.0 -> 26.3.  Beyond: 128 of 128 experts 144.4 -> 144.6, 12 rows an expert (48 of 16 experts, top-4)
-// 43.4 -> 45.4, 64 of 16 experts, top-8, 30.3 -> 36.6, 512 of 128 174.8 -> 201.5.
-constexpr int OWN_PASS = 32;
+// Where the down kernel makes the codes of its rows itself (OWN) and the quantizer's launch between the two expert kernels goes.
+// Every workgroup of an expert makes all of its codes, at 0.8 us for each row of a wave (some 330 vector instructions, one wave a
+// SIMD), so what it costs is the rows of the fullest expert.  The host does not know them: at most T, and that many where all tokens
+// go to the same experts.  FFN, us with the launch -> without, top-8 of 128, H = 2048, I = 768: 16 tokens one to an expert 121.5 ->
+// 119.4, as a router sends them 94.2 -> 91.6, half of them to the same eight 68.1 -> 66.9, all of them 29.5 -> 30.8; 8 tokens to the
+// same eight 28.1 -> 27.6; top-4 of 64, H = 1024, I = 512, the four of 16 tokens 35.0 -> 32.9, 32.2 -> 29.7, 27.1 -> 26.4, 21.1 -> 20.9;
+// 1 token 26.1 -> 25.1 and 18.9 -> 17.1.  Beyond 16 tokens the rows of one expert can cost more than a launch: 24 tokens 104.0 -> 101.8 as
+// a router sends them, 32.2 -> 34.7 all to the same; 32 tokens 117.3 -> 114.5 and 33.2 -> 38.1.  And so with few experts: 16 of them, H =
+// 1024, I = 256, 8 rows an expert 28.0 -> 26.3, 12 rows an expert 43.4 -> 45.4.
+constexpr int OWN_PASS = 16;
 static bool own_codes(int64_t T, int64_t E, int topk) { return T <= OWN_PASS && T * topk <= 8 * E; }
+
+// (the compiler does not see that a pointer out of an asm statement is one to device memory)
+template <typename T>
+using global_ptr = __attribute__((address_space(1))) T *;
 
 // One pass: at most 16 * MTT of an expert's pairs (from pos0 on, n of them) against nch row chunks from chunk c0 on.
 // first: the workgroup's first pass over these chunks, which brings their weight scales.
@@ -820,7 +827,7 @@ __device__ __forceinline__ void rx_pass(char *smem, const int8_t *act, const flo
             else wsc_now[u] = ((o & 16) ? sc1 : sc0)[row0 + (o >> 5) * 16 + (o & 15)];
         }
     }
-    const int pos = pos0 + min(tid, n - 1), pair = perm[pos];
+    const int pos = pos0 + min(tid, n - 1), pair = *(global_ptr<const int32_t>)(perm + pos);
     // the weight stream starts first: its addresses do not depend on the tokens, whose lookups cost two dependent memory
     // round trips
     if (nsw > 0) {
@@ -834,68 +841,80 @@ __device__ __forceinline__ void rx_pass(char *smem, const int8_t *act, const flo
     int last_step = steps - 1 - s0;
     asm volatile("" : "+v"(last_step));   // (scalar registers are what this kernel has fewest of)
     if constexpr (OWN) {
-        // a wave a row, as the quantizer by itself; as many rows at a time as the sums' area holds, which this form does not use
-        static_assert(DOWN && NSMAX * 128 <= 1024, "rows of at most two chunks a lane");
-        constexpr int C = NSMAX * 128 > 512 ? 2 : 1;
+        // a wave a row, as the quantizer by itself, 8 or 16 rows at a time: the sums' area, which this form does not use, holds them.
+        // All rows are requested before the first is used: they were written all over the chip.  (Requested one by one, 16 tokens to
+        // the same eight experts took 32.9 us instead of 30.5, 92.8 -> 92.2 as a router sends them.)
+        static_assert(DOWN && MTT == 1 && NSMAX * 128 <= 1024, "one pass of rows of at most two chunks a lane");
+        constexpr int C = NSMAX * 128 > 512 ? 2 : 1, ROWS = 4;   // chunks a lane, rows a wave
+        constexpr int AT_ONCE = RX_RED_BYTES / (NSMAX * 128) < 16 ? 8 : 16;
+        static_assert(AT_ONCE * NSMAX * 128 <= RX_RED_BYTES, "");
         int8_t *const s_code = reinterpret_cast<int8_t *>(smem + RX_RING_BYTES);
-        constexpr int AT_ONCE = RX_RED_BYTES / (NSMAX * 128) < 16 ? RX_RED_BYTES / (NSMAX * 128) : 16;
         const int jq = lane & 31;
         int kd = Kdim, writes = c0;
         asm volatile("" : "+v"(kd), "+v"(writes));   // (as above)
-        static_for<MTT>([&](auto B) {
-            constexpr int b = decltype(B)::value;
-            const int end = min(n, 16 * b + 16);
-            for (int base = 16 * b; base < end; base += AT_ONCE) {
-                if (base) __syncthreads();   // the rows before have been read
-                for (int row = base + wave; row < min(end, base + AT_ONCE); row += 4) {
-                    const float *hr = h + (int64_t)(pos0 + row) * kd;
-                    float v[C][8];
-                    float amax = 0.0f;
+        float v[ROWS][C][8];
+        int there = n - wave;   // opaque, or the compiler keeps every comparison with it in scalar registers
 #pragma unroll
-                    for (int i = 0; i < C; ++i) {
-                        const int c = lane + 64 * i, of = (c >> 5) * 256 + 4 * jq;
-                        float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
-                        if ((C == 2 && i == 0) || c * 8 < kd) {   // (two chunks a lane: rows of more than 512)
-                            lo = *reinterpret_cast<const float4 *>(hr + of);
-                            hi = *reinterpret_cast<const float4 *>(hr + of + 128);
-                        }
-                        v[i][0] = lo.x; v[i][1] = lo.y; v[i][2] = lo.z; v[i][3] = lo.w;
-                        v[i][4] = hi.x; v[i][5] = hi.y; v[i][6] = hi.z; v[i][7] = hi.w;
-                    }
+        for (int k = 0; k < ROWS; ++k) {
+            asm volatile("" : "+s"(there));
+            const int row = 4 * k + wave;
+            if (4 * k >= there) continue;
+            const float *hr = h + (int64_t)(pos0 + row) * kd;
 #pragma unroll
-                    for (int i = 0; i < C; ++i) {
-                        fwht_codes<256>(v[i], jq);
-                        amax = fmaxf(amax, abs8(v[i]));
-                    }
-                    amax = max_lanes<64>(amax);
-                    const float sc = (amax == 0.0f) ? 1.0f : amax / 127.0f;
-                    const float inv = (amax == 0.0f) ? 0.0f : 127.0f / amax;
-                    if (lane == 0) s_tsc[row] = sc;
-                    if (lane == 0 && writes == 0) const_cast<float *>(act_scale)[pos0 + row] = sc;
-                    int8_t *const to = const_cast<int8_t *>(act) + (int64_t)(pos0 + row) * kd;
+            for (int i = 0; i < C; ++i) {
+                const int c = lane + 64 * i, of = (c >> 5) * 256 + 4 * jq;
+                v4f lo = (v4f){0.f, 0.f, 0.f, 0.f}, hi = lo;
+                if ((C == 2 && i == 0) || c * 8 < kd) {   // (two chunks a lane: rows of more than 512)
+                    lo = *(global_ptr<const v4f>)(hr + of);
+                    hi = *(global_ptr<const v4f>)(hr + of + 128);
+                }
 #pragma unroll
-                    for (int i = 0; i < C; ++i) {
-                        const int c = lane + 64 * i, of = (c >> 5) * 256 + 4 * jq;
-                        if (!(C == 2 && i == 0) && c * 8 >= kd) continue;
-                        const uint32_t q0 = quant4(v[i][0], v[i][1], v[i][2], v[i][3], inv), q1 = quant4(v[i][4], v[i][5], v[i][6], v[i][7], inv);
-                        *reinterpret_cast<uint32_t *>(s_code + (row - base) * kd + of) = q0;
-                        *reinterpret_cast<uint32_t *>(s_code + (row - base) * kd + of + 128) = q1;
-                        if (writes == 0) {
-                            *reinterpret_cast<uint32_t *>(to + of) = q0;
-                            *reinterpret_cast<uint32_t *>(to + of + 128) = q1;
-                        }
+                for (int e = 0; e < 4; ++e) v[k][i][e] = lo[e], v[k][i][4 + e] = hi[e];
+            }
+        }
+        static_for<16 / AT_ONCE>([&](auto Part) {
+            constexpr int base = decltype(Part)::value * AT_ONCE;
+            if (base >= n) return;
+            if (base) __syncthreads();   // the rows before have been read
+#pragma unroll
+            for (int k = base / 4; k < (base + AT_ONCE) / 4; ++k) {
+                asm volatile("" : "+s"(there));
+                const int row = 4 * k + wave;
+                if (4 * k >= there) continue;
+                float amax = 0.0f;
+#pragma unroll
+                for (int i = 0; i < C; ++i) {
+                    fwht_codes<256>(v[k][i], jq);
+                    amax = fmaxf(amax, abs8(v[k][i]));
+                }
+                amax = max_lanes<64>(amax);
+                const float sc = (amax == 0.0f) ? 1.0f : amax / 127.0f;
+                const float inv = (amax == 0.0f) ? 0.0f : 127.0f / amax;
+                if (lane == 0) s_tsc[row] = sc;
+                if (lane == 0 && writes == 0) *(global_ptr<float>)(const_cast<float *>(act_scale) + pos0 + row) = sc;
+                int8_t *const to = const_cast<int8_t *>(act) + (int64_t)(pos0 + row) * kd;
+#pragma unroll
+                for (int i = 0; i < C; ++i) {
+                    const int c = lane + 64 * i, of = (c >> 5) * 256 + 4 * jq;
+                    if (!(C == 2 && i == 0) && c * 8 >= kd) continue;
+                    const uint32_t q0 = quant4(v[k][i][0], v[k][i][1], v[k][i][2], v[k][i][3], inv), q1 = quant4(v[k][i][4], v[k][i][5], v[k][i][6], v[k][i][7], inv);
+                    *reinterpret_cast<uint32_t *>(s_code + (row - base) * kd + of) = q0;
+                    *reinterpret_cast<uint32_t *>(s_code + (row - base) * kd + of + 128) = q1;
+                    if (writes == 0) {
+                        *(global_ptr<uint32_t>)(to + of) = q0;
+                        *(global_ptr<uint32_t>)(to + of + 128) = q1;
                     }
                 }
-                __syncthreads();
-                const int mine = min(16 * b + r, n - 1);
-                if (mine >= base && mine < base + AT_ONCE) {
-                    const int8_t *xp = s_code + (mine - base) * kd + g_ * 16;
+            }
+            __syncthreads();
+            const int mine = min(r, n - 1);
+            if (mine >= base && mine < base + AT_ONCE) {
+                const int8_t *xp = s_code + (mine - base) * kd + g_ * 16;
 #pragma unroll
-                    for (int i = 0; i < NSMAX; ++i) {
-                        const int st = min(i, last_step) * 128;
-                        xr[b][i][0] = *reinterpret_cast<const v4i *>(xp + st);
-                        xr[b][i][1] = *reinterpret_cast<const v4i *>(xp + st + 64);
-                    }
+                for (int i = 0; i < NSMAX; ++i) {
+                    const int st = min(i, last_step) * 128;
+                    xr[0][i][0] = *reinterpret_cast<const v4i *>(xp + st);
+                    xr[0][i][1] = *reinterpret_cast<const v4i *>(xp + st + 64);
                 }
             }
         });
@@ -1089,9 +1108,9 @@ __global__ __launch_bounds__(256, 2) void k_moe_expert_rx(const int8_t *act, con
                 const int n = min(PASS, count - base);
 #define MI_RX_PASS(MT_) rx_pass<DOWN, NSMAX, MT_, OWN>(smem, act, act_scale, h, perm, w0, sc0, w1, sc1, out, Kdim, Nrows, topk, e, c0, \
                                                   nch, seg0 + base, n, base == 0)
-                if (n <= 16) MI_RX_PASS(1);
-                else if (n <= 32 || PASS == 32) MI_RX_PASS(2);
-                else if (n <= 48 || PASS == 48) MI_RX_PASS(PASS == 32 ? 2 : 3);
+                if (n <= 16 || PASS == 16) MI_RX_PASS(1);
+                else if (n <= 32 || PASS == 32) MI_RX_PASS(PASS == 16 ? 1 : 2);
+                else if (n <= 48 || PASS == 48) MI_RX_PASS(PASS <= 32 ? PASS / 16 : 3);
                 else MI_RX_PASS(PASS / 16);
 #undef MI_RX_PASS
             }

@@ -293,9 +293,12 @@ def test_layer_of_few_tokens_equals_route_and_ffn(mi, dev, orc, T, H, I, E, topk
     (1, 768, 16, 1), (8, 1024, 16, 8), (9, 1024, 16, 2), (10, 768, 16, 2), (11, 768, 16, 2), (16, 512, 16, 8),
     (17, 256, 32, 4), (27, 768, 32, 4), (32, 768, 64, 2), (32, 1024, 128, 8),
     (33, 768, 64, 2), (32, 768, 16, 8),     # the quantizer's own launch: a token more, more rows an expert
+    # every last row of a wave's four, on both sides of the rounds of eight rows (I > 512) and of the last token that takes this form
+    (4, 768, 16, 1), (5, 768, 16, 1), (12, 1024, 32, 2), (13, 1024, 32, 2), (15, 768, 32, 4), (16, 768, 128, 8), (16, 256, 16, 2),
+    (16, 1024, 64, 4), (17, 768, 128, 8), (13, 512, 32, 4), (3, 256, 16, 8),
 ])
 def test_codes_made_by_the_down_kernel(mi, dev, orc, T, I, E, topk):
-    """Every token picks expert 0, so that its rows fill the rounds of codes (8, 10 or 16 at a time) to their ends and past them."""
+    """Every token picks expert 0, so that its rows fill the rounds of codes (8 or 16 at a time) to their ends and past them."""
     H = 512
     rng = np.random.default_rng(T * I)
     idx = np.stack([np.concatenate([[0], 1 + rng.permutation(E - 1)[:topk - 1]]) for _ in range(T)]).astype(np.int32)
