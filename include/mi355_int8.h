@@ -504,7 +504,7 @@ MI_API int32_t mi_swiglu_quant_f32_i8(const float *gate_up, float *h_out, int8_t
 /* (residual +) RMSNorm + rotate + quantize + W8A8 contraction + dequant as one call: y = linear(rmsnorm(x (+ residual))).
  * For one token (block 128) it is ONE kernel (the GEMV normalizes and quantizes the row itself) where that is the faster
  * form: K up to 16384 with N up to 64 rows a compute unit, K from 1024 to 8192 with up to 160, and 2048, 3072 and 4096 with
- * any N.  So it is, of these K up to 4096, for two tokens, and from K = 2048 on for three and four with more than 80 rows a
+ * any N.  So it is, of these K up to 4096, for two tokens, and at K = 4096 for three and four with more than 80 rows a
  * compute unit.  Any other shape, and outputs or a workspace that overlap x, residual or g or each other, run
  * mi_rmsnorm_quant_f32_i8 and the contraction.  workspace as for mi_w8a8_linear_f32 (it receives the codes and the scale); h_out (the residual sum, required with a residual) and xn_out (the
  * normalized row, optional) as in mi_rmsnorm_quant_f32_i8. */

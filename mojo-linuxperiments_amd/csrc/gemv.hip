@@ -458,31 +458,34 @@ static int32_t launch_row(const float *x, const int8_t *qw, const float *sw, flo
 
 // The same for two tokens, and for three and four where the rows are many: every workgroup makes all the codes, which two launches
 // do once.  us of two launches -> one, weights from HBM, linear and with the norm, K = 512 to 4096, N = 16 to 40960: two tokens 0.69 to
-// 1.00 of the time and 0.75 to 1.02 (4096 x 4096 7.6 -> 5.7 and 8.5 -> 7.5, 28672 x 4096 25.3 -> 21.3 and 26.1 -> 21.9); three and four
-// from 80 rows a unit and K = 2048 on 0.83 to 1.00 and 0.87 to 1.01 (four, 28672 x 4096 25.7 -> 22.4 and 26.3 -> 23.6), fewer and
-// shorter rows 0.87 to 1.11 and up to 1.29.
-static bool rows_take(int64_t M, int64_t N, int64_t K)
+// 1.00 of the time and 0.77 to 0.97 (4096 x 4096 7.6 -> 5.7 and 7.7 -> 6.7, 28672 x 4096 25.3 -> 21.3 and 24.0 -> 20.8).  Three and four
+// from 80 rows a unit on: linear from K = 2048 on 0.85 to 1.00 (four, 28672 x 4096 25.7 -> 22.4), fewer and shorter rows 0.87 to 1.11;
+// with the norm, whose prologue is the longer, at K = 4096 0.87 to 1.02 (four, 28672 x 4096 23.8 -> 22.3, 22000 x 4096 21.2 -> 19.4,
+// at worst 20496 x 4096 and a residual 19.0 -> 19.4), 0.95 to 1.18 below it (20496 x 2048 11.6 -> 12.9, 24576 x 3072 17.4 -> 18.2,
+// 24576 x 3456 18.4 -> 20.0, 40960 x 2048 19.4 -> 18.6).
+static bool rows_take(int64_t M, int64_t N, int64_t K, bool norm)
 {
     if (M < 2 || M > 4 || K > 4096 || !row_takes(N, K)) return false;
-    return M == 2 || (K >= 2048 && N > 80 * compute_units());
+    return M == 2 || (K >= (norm ? 4096 : 2048) && N > 80 * compute_units());
 }
 
 template <RowOp OP>
 static int32_t launch_rows_of(const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx, int64_t M,
                               int64_t N, int64_t K, const RowArgs &ra, hipStream_t s)
 {
-    if (!rows_take(M, N, K) || !apart({{x, M * K * 4}, {ra.res, M * K * 4}, {ra.g, K * 4}},
+    if (!rows_take(M, N, K, OP == NORM) || !apart({{x, M * K * 4}, {ra.res, M * K * 4}, {ra.g, K * 4}},
                                       {{y, M * N * 4}, {qx, M * K}, {sx, M * 4}, {ra.h_out, M * K * 4}, {ra.xn_out, M * K * 4}}))
         return MI_EINVAL;
     const int cus = compute_units(), per_wave = (int)((N + 8 * cus - 1) / (8 * cus));
     switch ((K + 1023) >> 10) {
 #define MI_ROWS1(CW_, WHOLE_, MB_) start_row<CW_, WHOLE_, OP, MB_>(cus, per_wave, x, qw, sw, y, qx, sx, (int)N, (int)K, (int)M, ra, s)
+    // (three and four with the norm: four whole chunks)
 #define MI_ROWS(CW_)                                                          \
     case CW_:                                                                 \
         if (M == 2 && K % 1024) MI_ROWS1(CW_, false, 2);                      \
         else if (M == 2) MI_ROWS1(CW_, true, 2);                              \
-        else if constexpr (CW_ == 1) return MI_EINVAL;                        \
-        else if (K % 1024) MI_ROWS1(CW_, false, 4);                           \
+        else if constexpr (CW_ < (OP == NORM ? 4 : 2)) return MI_EINVAL;      \
+        else if (OP != NORM && K % 1024) MI_ROWS1(CW_, OP == NORM, 4);        \
         else MI_ROWS1(CW_, true, 4);                                          \
         break;
         MI_ROWS(1) MI_ROWS(2) MI_ROWS(3) MI_ROWS(4)

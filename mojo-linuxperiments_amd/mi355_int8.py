@@ -562,7 +562,8 @@ class DecoderLayer:
         residual add is left to the next layer (pass x=self.dn, residual=self.h1 to its step)."""
         B, H, Hq, Hkv, I, D, s = self.B, self.H, self.Hq, self.Hkv, self.I, 128, stream
         p = lambda b: b.ptr if b is not None else None
-        # norm + quantize + projection: one kernel for a token or two, two launches for more
+        # norm + quantize + projection: one kernel for a token or two (three and four where the rows are many and
+        # long enough), two launches for more
         check(lib.mi_rmsnorm_linear_f32(x.ptr, p(residual), self.g1.ptr, self.eps,
                                         self.h0.ptr if residual is not None else None, p(self.xn), self.wqkv[0].ptr,
                                         self.wqkv[1].ptr, self.qkv.ptr, B, self.NQKV, H, self.block, self.lin_ws.ptr,

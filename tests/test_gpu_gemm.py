@@ -273,6 +273,7 @@ def test_argument_errors(mi, dev):
 @pytest.mark.parametrize("M,N,K", [
     (2, 16, 128), (2, 2064, 512), (2, 4096, 1024), (2, 6144, 4096), (2, 8208, 4096), (2, 16400, 2048), (2, 33040, 2176), (2, 41024, 3968),
     (3, 20480, 2048), (3, 20496, 2048), (4, 20496, 2176), (3, 28672, 4096), (4, 33040, 3968),
+    (3, 20480, 4096), (3, 20496, 4096), (4, 20512, 4096),
 ])
 @pytest.mark.parametrize("norm", [False, True])
 def test_few_tokens_in_one_launch_are_the_two_launches(mi, dev, M, N, K, norm):
