@@ -404,15 +404,18 @@ static void start_row(int cus, int per_wave, const float *x, const int8_t *qw, c
                       y, qx, sx, N, K, M, ra);
     };
     using std::integral_constant;
-    if constexpr (MB == 4) return go(integral_constant<int, 1>{}, 2);   // (many rows, see rows_take)
-    if (per_wave <= 2) return go(integral_constant<int, 1>{}, 1);
-    if constexpr (CW <= 4) {
-        if (per_wave <= 4) return go(integral_constant<int, 2>{}, 1);
-        if constexpr (CW <= 2)
-            if (per_wave <= 8) return go(integral_constant<int, 4>{}, 1);
-        return go(integral_constant<int, 1>{}, MB == 1 && CW == 4 && per_wave > (OP == NORM ? 20 : 10) ? 3 : 2);
+    if constexpr (MB == 4) {   // many rows, see rows_take
+        go(integral_constant<int, 1>{}, 2);
+    } else {
+        if (per_wave <= 2) return go(integral_constant<int, 1>{}, 1);
+        if constexpr (CW <= 4) {
+            if (per_wave <= 4) return go(integral_constant<int, 2>{}, 1);
+            if constexpr (CW <= 2)
+                if (per_wave <= 8) return go(integral_constant<int, 4>{}, 1);
+            return go(integral_constant<int, 1>{}, MB == 1 && CW == 4 && per_wave > (OP == NORM ? 20 : 10) ? 3 : 2);
+        }
+        go(integral_constant<int, 1>{}, CW <= 8 && per_wave > 6 ? 2 : 1);
     }
-    go(integral_constant<int, 1>{}, CW <= 8 && per_wave > 6 ? 2 : 1);
 }
 
 // Where the one kernel is the faster form, against making the codes and contracting them one behind the other: linear, norm and
