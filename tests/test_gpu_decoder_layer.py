@@ -526,7 +526,8 @@ def test_rmsnorm_linear_one_call(mi, dev, orc, M, N, K):
     dev.reset_to(mark)
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 6144, 4096), (1, 272, 2048), (4, 512, 4096)])
+@pytest.mark.parametrize("M,N,K", [(1, 6144, 4096), (1, 272, 2048), (4, 512, 4096),
+                                   (2, 6144, 4096), (3, 20496, 4096), (4, 28672, 4096)])   # one launch for several tokens
 @pytest.mark.parametrize("target", ["residual", "x"])
 def test_rmsnorm_linear_residual_stream_updated_in_place(mi, dev, orc, M, N, K, target):
     """h_out written over the residual (or over x), the way a decoder updates its residual stream: the one-kernel

@@ -307,3 +307,39 @@ def test_few_tokens_in_one_launch_are_the_two_launches(mi, dev, M, N, K, norm):
         got = dev.download(a)
         assert np.array_equal(got[:M], dev.download(b)) and np.isnan(got[M]).all()
     dev.reset_to(mark)
+
+
+@pytest.mark.parametrize("M,N,K", [(2, 2064, 512), (2, 4096, 4096), (3, 20496, 4096), (4, 28672, 4096), (4, 20496, 2176)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_few_tokens_that_are_not_all_numbers(mi, dev, M, N, K, norm):
+    """One launch for several tokens: a row with an infinity, one with a NaN, one of zeros, without a residual.  Everything is as the
+    row kernel and the contraction have it, and a row spoils no other."""
+    mark = dev.mark()
+    g = np.random.default_rng(M + N + K)
+    rows = g.standard_normal((M, K), dtype=np.float32)
+    rows[0, 5] = np.inf
+    rows[M - 1, K - 3] = np.nan
+    if M > 2:
+        rows[1] = 0.0
+    x, gain = dev.upload(rows), dev.upload(1 + 0.1 * g.standard_normal(K, dtype=np.float32))
+    qw, sw = dev.upload(g.integers(-127, 128, (N, K), dtype=np.int8)), dev.upload(g.random(N, dtype=np.float32))
+    ws = dev.empty(mi.lib.mi_w8a8_linear_workspace_bytes(M, N, K), np.uint8)
+    y, y2, q, s = dev.empty((M, N), np.float32), dev.empty((M, N), np.float32), dev.empty((M, K), np.int8), dev.empty(M, np.float32)
+    xn, xn2 = dev.empty((M, K), np.float32), dev.empty((M, K), np.float32)
+    if norm:
+        mi.check(mi.lib.mi_rmsnorm_linear_f32(x.ptr, None, gain.ptr, 1e-5, None, xn.ptr, qw.ptr, sw.ptr, y.ptr, M, N, K, 128, ws.ptr,
+                                              ws.nbytes, None))
+        mi.check(mi.lib.mi_rmsnorm_quant_f32_i8(x.ptr, None, gain.ptr, 1e-5, None, xn2.ptr, q.ptr, s.ptr, M, K, 128, None))
+        assert np.array_equal(dev.download(xn), dev.download(xn2), equal_nan=True)
+    else:
+        mi.check(mi.lib.mi_w8a8_linear_f32(x.ptr, qw.ptr, sw.ptr, y.ptr, M, N, K, 128, ws.ptr, ws.nbytes, None))
+        mi.fwht_quant(x, q, s, 128)
+    mi.gemm_dequant(q, s, qw, sw, y2)
+    al = (M * K + 255) // 256 * 256
+    assert np.array_equal(dev.download(ws.offset(0, (M, K), np.int8)), dev.download(q))
+    assert np.array_equal(dev.download(ws.offset(al, (M,), np.float32)), dev.download(s), equal_nan=True)
+    got = dev.download(y)
+    assert np.array_equal(got, dev.download(y2), equal_nan=True)
+    if M > 2:
+        assert np.all(got[1] == 0)
+    dev.reset_to(mark)
