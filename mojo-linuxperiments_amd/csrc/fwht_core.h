@@ -227,8 +227,11 @@ __device__ __forceinline__ float tree_sum(const float *part)   // part[0 .. G-1]
     return t[0];
 }
 
-// g / (1 + e^-g), the bits of g / (1.0f + expf(-g)) for every g: e^x = 2^n 2^f with n + f = x log2(e), log2(e) in two parts.
-// Clamping x to where the sum no longer changes, or is infinite, does in one instruction what expf needs four for.
+// g / (1 + e^-g) with e^x = 2^n 2^f, n + f = x log2(e).  The steps and the two constants are those that the AMD compiler expands
+// expf into (the second is its own, not the float nearest to log2(e) - 0x1.715476p+0), so that results stay what they were when expf
+// was called here: compared over all floats with the expf of ROCm 7.2, the same bits.  What is relied upon is the error, at most
+// 3e-7 of the result: an ulp of the exponential, half of one each of the sum and the quotient.  In place of expf's selects at the
+// ends of its range, four instructions, x is clamped to where the sum no longer changes or is infinite, one.
 __device__ __forceinline__ float silu(float g)
 {
     const float x = -__builtin_amdgcn_fmed3f(g, -89.5f, 104.0f);

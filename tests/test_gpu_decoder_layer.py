@@ -110,6 +110,26 @@ def test_swiglu_at_the_ends_of_the_range(mi, dev):
     assert np.all(np.abs(got[f] - want[f]) <= 3e-7 * np.abs(want[f]) + 5e-37)
 
 
+def test_swiglu_over_all_gates(mi, dev):
+    """Every 1009th float, both signs, every exponent, and all floats around the two ends of the clamp: 3e-7, derived as above."""
+    def around(x, n):
+        return np.float32(x).view(np.uint32) + np.arange(-n, n, dtype=np.int64)
+    bits = np.concatenate([np.arange(0, 1 << 32, 1009), around(-89.5, 4096), around(-88.72284, 65536), around(104.0, 4096), around(16.6, 65536)])
+    bits = bits[:bits.size // 4096 * 4096].astype(np.uint32)
+    M, I = 8, bits.size // 8
+    g = bits.view(np.float32).reshape(M, I)
+    mark = dev.mark()
+    gu, h = dev.upload(np.concatenate([g, np.ones((M, I), np.float32)], axis=1)), dev.empty((M, I), np.float32)
+    mi.check(mi.lib.mi_swiglu_f32(gu.ptr, h.ptr, M, I, None))
+    got = dev.download(h)
+    dev.reset_to(mark)
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = g.astype(np.float64) / (1.0 + np.exp(-g.astype(np.float64)))
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    f = np.isfinite(want)
+    assert np.all(np.abs(got[f] - want[f]) <= 3e-7 * np.abs(want[f]) + 5e-37)
+
+
 def test_add(mi, dev):
     mark = dev.mark()
     a, b = workload.normal(1, (3, 1024), 0), workload.normal(1, (3, 1024), 1)
