@@ -76,7 +76,8 @@ def make_cache(mi, dev, seed, B, Hq, Hkv, T, T_cap):
 @pytest.mark.parametrize("B,Hq,Hkv,T,T_cap", [
     (2, 8, 2, 256, 256), (1, 4, 1, 16, 64), (1, 32, 8, 1000, 1024), (3, 6, 3, 77, 128), (2, 4, 4, 130, 192),
     (1, 8, 2, 1, 64), (1, 8, 2, 4096, 4096), (16, 32, 8, 700, 1024), (2, 8, 8, 64, 64),
-    (1, 32, 8, 2000, 2048), (2, 16, 4, 1500, 1536),     # 32 and 24 splits: the merge with 32 lanes per row
+    (1, 32, 8, 2000, 2048), (2, 16, 4, 1500, 1536),     # 8 and 6 splits
+    (1, 4, 1, 4300, 4352), (1, 8, 2, 7700, 7744),       # 17 and 31 splits: the merge with 32 lanes per row
 ])
 def test_vt_attention_matches_oracle(mi, dev, orc, B, Hq, Hkv, T, T_cap):
     mark = dev.mark()
@@ -641,6 +642,7 @@ def test_append_inside_the_attention_with_overlapping_buffers(mi, dev, T, q_at, 
     (1, 2, 65), (1, 2, 511), (1, 2, 512), (1, 2, 513), (3, 2, 512),       # one span of two to eight blocks, and the first cut
     (1, 1, 1700), (1, 1, 2304), (1, 1, 2800), (1, 1, 3500), (1, 1, 4096),  # 7, 9, 11, 14 and 16 spans
     (20, 8, 520), (20, 8, 1024), (33, 4, 900),                            # spans of 8 and 12 blocks, where 4 are too many workgroups
+    (1, 1, 4352), (1, 1, 8192), (1, 1, 8193), (2, 2, 5000),               # 17 and 32 spans, a token more, codes of two sequences
 ])
 def test_few_rows_are_cut_into_whole_rounds(mi, dev, orc, B, Hkv, T):
     """Both layouts at the ends of their spans and through every form of the merge, with codes and without."""
@@ -700,4 +702,31 @@ def test_rows_kernel_writes_the_output_of_one_span(mi, dev, orc, lens):
                 want = orc.gqa_decode(q[b:b + 1], kq[b:b + 1, :, :m], ks[b:b + 1, :, :m], vq[b:b + 1, :, :m], vs[b:b + 1, :, :m],
                                       out_rotated=bool(rotated))
                 assert np.max(np.abs(got[b] - want[0])) <= 2e-5, (rotated, shift, b)
+    dev.reset_to(mark)
+
+
+@pytest.mark.parametrize("rotated", [0, 1])
+def test_one_span_written_on_top_of_the_queries(mi, dev, orc, rotated):
+    """At most eight blocks: the kernel writes the output itself, in place of the queries or elsewhere; a row further on, where one
+    workgroup's output is another's query, the result is the same."""
+    mark = dev.mark()
+    B, Hq, Hkv, T, D = 3, 6, 2, 500, 128
+    lens = [500, 0, 65]
+    q, kq, ks, vq, vs, ks_c, vs_c = make_cache(mi, dev, 78, B, Hq, Hkv, T, 512)
+    dkt, dvt = convert(mi, dev, kq, vq, T, 512)
+    dks, dvs, dl = dev.upload(ks_c), dev.upload(vs_c), dev.upload(np.array(lens, np.int32))
+    ws = dev.empty(mi.lib.mi_gqa_decode_workspace_bytes(B, Hq, Hkv, D, T), np.uint8)
+    for shift in (None, 0, D):
+        both = dev.upload(np.concatenate([q.reshape(-1), np.full(D, np.nan, np.float32)]))
+        o = dev.upload(np.full((B, Hq, D), np.nan, np.float32)) if shift is None else both.offset(4 * shift, (B, Hq, D), np.float32)
+        mi.check(mi.lib.mi_gqa_decode_attn_tiled(both.ptr, dkt.ptr, dks.ptr, dvt.ptr, dvs.ptr, o.ptr, B, Hq, Hkv, D, 512, dl.ptr, T,
+                                                 rotated, ws.ptr, ws.nbytes, None))
+        got = dev.download(o)
+        for b, m in enumerate(lens):
+            if m == 0:
+                assert np.all(got[b] == 0)
+                continue
+            want = orc.gqa_decode(q[b:b + 1], kq[b:b + 1, :, :m], ks[b:b + 1, :, :m], vq[b:b + 1, :, :m], vs[b:b + 1, :, :m],
+                                  out_rotated=bool(rotated))
+            assert np.max(np.abs(got[b] - want[0])) <= 2e-5, (shift, b)
     dev.reset_to(mark)
