@@ -600,12 +600,15 @@ struct SplitPlan {
 
 int max_splits(int64_t B, int64_t Hkv, int64_t T);
 
-// Spans of 256 tokens where they are at most two workgroups a unit (and no more than the merge reads at once and the workspace
-// holds), else of 704: a wave goes through all of its tiles, those past the end of its span as well, so a span that is not filled
+// Spans of 256 tokens where they are at most two workgroups a unit (and no more than 32, which the merge without codes reads at
+// once, and the workspace holds), else of 704: a wave goes through all of its tiles, those past the end of its span as well, so a span that is not filled
 // costs what a full one does.  us, 8 heads, before -> here (a sequence of up to 256 tokens ran in a span of 704, and few rows were cut
 // into halves and quarters of 256): one sequence of 16 to 256 tokens 12.3 -> 8.9 (6.6 now that a single span needs no
 // merge), of 1531 10.1 -> 9.6, 4 of 1500 13.8 -> 9.9, 32 of 256 13.3 -> 10.1, 16 of 1000 14.6 -> 14.0;
-// three workgroups a unit, 32 of 700, 16.9 in spans of 256 and 15.3 in one of 704.
+// three workgroups a unit, 32 of 700, 16.9 in spans of 256 and 15.3 in one of 704.  Past 32 spans the merge costs more than the
+// units that long ones leave idle: one sequence of 8192, 8193 and 16384 tokens, 8 heads 11.1, 13.2 (21.3 in 33 spans of 256) and 15.3
+// (29.3), one head 10.0, 12.7 (17.7) and 13.9 (23.5).  The merge that makes codes reads 8 spans at once (12 and 16 too) and a token in
+// one workgroup: there long spans would be ahead before 32 (8192 tokens, 8 heads, 18.4, 8193 14.9; 19.3 and 25.4 before).
 static SplitPlan pick_splits(int64_t B, int64_t Hkv, int64_t T)
 {
     const int ntiles = (int)((T + 15) / 16);
@@ -633,8 +636,8 @@ int max_splits(int64_t B, int64_t Hkv, int64_t T)
 
 static bool merge_wide(int splits, int64_t rows) { return splits > 16 && splits <= 32 && rows <= 2 * compute_units(); }
 
-// How many dependent batches of loads the merge of `rows` rows makes: one up to 16 splits (8 where it quantizes) and in the kernel
-// for 17 to 32, one per eight splits otherwise.
+// How many dependent batches of loads the merge of `rows` rows makes: one up to 16 splits (where it quantizes up to 8, and for 12 and
+// 16) and in the kernel for 17 to 32, one per eight splits otherwise.
 int merge_batches(int splits, int64_t rows, bool quant)
 {
     if (splits <= (quant ? 8 : 16) || splits == 12 || splits == 16) return 1;

@@ -727,7 +727,9 @@ static Plan pick(int64_t B, int64_t Hq, int64_t Hkv, int64_t T, bool quant)
     return pl;
 }
 
-// the largest split count of the plans above for any length in [1, T], and of the row-major layout's where that is larger
+// At least the largest split count of the plans above for any length in [1, T]: what workspaces are sized for.  For few rows it is
+// the count of an earlier plan, which cut until every unit had a workgroup, up to four times what the present one uses, and stays so
+// that a workspace is the size it has always been.
 int max_splits(int64_t B, int64_t Hkv, int64_t T)
 {
     const int blocks = (int)((T + 63) / 64);
