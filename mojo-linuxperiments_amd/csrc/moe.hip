@@ -763,7 +763,7 @@ using global_ptr = __attribute__((address_space(1))) T *;
 // OWN (down, see own_codes): the pairs' codes are made here, from fp32 rows h; the workgroup with the expert's first
 // chunk leaves them in act and act_scale.
 template <bool DOWN, int NSMAX, int MTT, bool OWN>
-__device__ __forceinline__ void rx_pass(char *smem, const int8_t *act, const float *act_scale, const float *__restrict__ h,
+__device__ __forceinline__ void rx_pass(char *smem, int8_t *act, float *act_scale, const float *__restrict__ h,
                                         const int32_t *__restrict__ perm, const int8_t *__restrict__ w0,
                                         const float *__restrict__ sc0, const int8_t *__restrict__ w1,
                                         const float *__restrict__ sc1, float *__restrict__ out, int Kdim, int Nrows, int topk,
@@ -891,8 +891,8 @@ __device__ __forceinline__ void rx_pass(char *smem, const int8_t *act, const flo
                 const float sc = (amax == 0.0f) ? 1.0f : amax / 127.0f;
                 const float inv = (amax == 0.0f) ? 0.0f : 127.0f / amax;
                 if (lane == 0) s_tsc[row] = sc;
-                if (lane == 0 && writes == 0) *(global_ptr<float>)(const_cast<float *>(act_scale) + pos0 + row) = sc;
-                int8_t *const to = const_cast<int8_t *>(act) + (int64_t)(pos0 + row) * kd;
+                if (lane == 0 && writes == 0) *(global_ptr<float>)(act_scale + pos0 + row) = sc;
+                int8_t *const to = act + (int64_t)(pos0 + row) * kd;
 #pragma unroll
                 for (int i = 0; i < C; ++i) {
                     const int c = lane + 64 * i, of = (c >> 5) * 256 + 4 * jq;
@@ -1045,7 +1045,7 @@ __device__ __forceinline__ void rx_pass(char *smem, const int8_t *act, const flo
 // by_chunk: at most a chunk a workgroup, all of the same cost, with the compute units' own order as the balance.
 // OWN: see rx_pass.
 template <bool DOWN, int NSMAX, bool OWN>
-__global__ __launch_bounds__(256, 2) void k_moe_expert_rx(const int8_t *act, const float *act_scale, const float *__restrict__ h,
+__global__ __launch_bounds__(256, 2) void k_moe_expert_rx(int8_t *act, float *act_scale, const float *__restrict__ h,
                                                           const int32_t *__restrict__ perm,
                                                           const int32_t *__restrict__ seg_off,
                                                           const int8_t *__restrict__ w0, const float *__restrict__ sc0,
