@@ -490,7 +490,8 @@ struct DecoderLayer {
     int32_t step(const float *x, const float *residual, const int32_t *pos, const int32_t *seq_len, int64_t t_max,
                  float *out, void *stream) const
     {
-        // norm + quantize + projection: one kernel for a single token, two launches otherwise
+        // norm + quantize + projection: one kernel for a token or two (three and four where the rows are many and
+        // long enough), two launches for more
         int32_t rc = mi_rmsnorm_linear_f32(x, residual, g1, eps, residual ? h0 : nullptr, xn, qkv.qw, qkv.sw, qkv_out, B,
                                            qkv.N, H, 128, qkv.workspace, qkv.workspace_bytes, stream);
         const float *xin = residual ? h0 : x;
