@@ -1,25 +1,29 @@
 // W8A8 contraction for everything between the GEMV's few tokens and the sizes that fill the chip with 256-wide tiles:
 //   acc[m,n] = sum_k qx[m,k] * qw[n,k],   y = ((float)acc * sx[m]) * sw[n]
 //
-// One workgroup of four or eight waves per tile, the tile chosen from ten (16 x 16 to 128 x 128) so that every compute
+// One workgroup per tile, the tile chosen from ten (16 x 16 to 128 x 128) so that every compute
 // unit has one, and one load stream per workgroup: stages of 128 to 512 bytes of K go straight to LDS through a ring of D
 // buffers, D - 1 stages in flight, one barrier a stage.  All tiles but 128 x 128, 128 x 64 and 32 x 48 take at most half
 // of a unit's LDS: where there are tiles enough two workgroups share a unit and hide each other's first loads and last stores (16 rows,
-// 4096 -> 28672 inside a decode step: 24.3 instead of 27.2 us).  The barrier of stage s says that stage s + 1 has landed and
-// that everybody holds its fragments of stage s in registers; behind it a wave requests the fragments of stage s + 1,
-// the loads of stage s + D into the buffer just freed, and multiplies stage s.  Small tiles leave most
+// 4096 -> 28672 inside a decode step: 24.3 instead of 27.2 us).  Small tiles leave most
 // waves without rows of their own, so the waves split K inside a stage (WK slices of 64 bytes) and meet once, through
 // LDS, at the tile's end; every wave finishes an equal share of the matrix-instruction tiles.
 //
-// What bounds it.  The load path of a compute unit: at 128 x 128, K = 14336, one to 256 workgroups alike, a stage takes
-// 850 - 900 clocks of which the matrix instructions need 512 and, with the loads taken out, 705 (550 without the
-// fragment reads as well); no wait for memory is left in the stage.  32 direct-to-LDS loads of 1 KB at 28 clocks each are
-// those 900.  Measured and equal or slower: loads through registers and ds_write, 16 waves, the loads spread between the
-// matrix instructions, another K phase per workgroup, rows of 256 bytes.  So the tile decides: rows loaded per result.
+// Four or eight waves multiply and four more only load: they request a stage, wait until an older one has landed and say so
+// by the barrier.  A load holds its wave's issue until the path to the cache takes it, and with the loads dealt to the
+// multiplying waves the matrix instructions behind them waited for that path: a stage of a 128 x 128 tile alone on the
+// chip took 0.33 us, 0.29 with loading waves (512 clocks of matrix instructions, 32 loads at 16 clocks).  With the two
+// halves of the multiplying waves a phase apart: 0.33 without loading waves, 0.29 with them.  One or two loading waves measured
+// the same at large tiles and 0.1 to 0.2 us more at small ones, whose first loads they request one by one; eight mixed.
 //
-// Measured (us a call in a graph of them, weights from HBM, and with the LDS-tiled and ring kernels before):
-// 16 x 4096 -> 14336 12.0 (13.7), 32 x 4096 -> 4096 7.2 (9.0), 64 x 4096 -> 14336 15.1 (25.4), 200 x 4096 -> 14336
-// 24.2 (34.5), 256 x 14336 -> 4096 31.9 (91.3), 512 x 4096 -> 4096 17.7 (32.4).
+// What bounds it.  Few rows: HBM and launch to first byte.  128 x 128 tiles on a full chip: 0.39 us a stage, which falls to 0.34 with codes
+// that are all zero (the part's power limit), is the same with two, three or four stages in flight (not latency), and
+// of which the path to the cache takes 0.25 (130 GB/s a unit in a loop of nothing but loads).  So the tile decides: rows loaded per result.
+//
+// Measured (us a call in a graph of them, weights from HBM, and with the loads made by the waves that multiply):
+// 8 x 1408 -> 736 2.78 (3.00), 16 x 4096 -> 6144 7.14 (7.36), 32 x 4096 -> 4096 6.28 (6.51), 64 x 4096 -> 14336 15.2 (15.6),
+// 97 x 4096 -> 4096 8.12 (8.67), 168 x 2944 -> 2320 5.38 (6.18), 200 x 4096 -> 14336 23.6 (24.3), 256 x 14336 -> 4096 34.5 (34.5),
+// 397 x 3072 -> 7136 17.7 (18.4), 925 x 1664 -> 2784 10.7 (11.6), 1007 x 3456 -> 1296 10.8 (11.6); 16 x 4096 -> 28672 23.9 (23.9).
 //
 // LDS layout, swizzle and shape of the loads are those of gemm_tiled.hip: 1 KB blocks of 8 rows x 128 bytes, chunk position
 // XORed with sigma(row, block parity), free of bank conflicts for the fragment reads.  Operand A is the weights.
@@ -41,34 +45,30 @@ typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));   // four sca
 template <int TM_, int TN_, int WM_, int WN_, int WK_, int D_>
 struct Cfg {
     static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, WK = WK_, D = D_;
-    static constexpr int NW = WM * WN * WK, TPB = 64 * NW;
+    static constexpr int NW = WM * WN * WK, NL = 4, TPB = 64 * (NW + NL);   // waves that multiply, waves that load
     static constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
     static constexpr int SUB = WK / 2;                  // 128-byte K steps per stage
     static constexpr int BX = BM / 8, BW = BN / 8;      // 1 KB blocks (8 rows x 128 B) per step
     static constexpr int BLK = (BX + BW) * SUB;         // per stage
-    static constexpr int L = BLK / NW;                  // load instructions per wave and stage
+    static constexpr int L = BLK / NL;                  // load instructions per loading wave and stage
     static constexpr int STAGE = BLK * 1024;
     static constexpr int NF = TM * TN;                  // matrix-instruction tiles of a wave
     static constexpr int OWN = (NF + WK - 1) / WK;      // of which it finishes this many (the last waves fewer or none)
     static constexpr int PART = WM * WN * NF * (WK - 1) * 1024;
     static constexpr int LDS = D * STAGE > PART ? D * STAGE : PART;
     static constexpr bool PAIR = OWN % 2 == 0 && TN % 2 == 0 && NF % OWN == 0;
-    static constexpr int PRE = D > 3 ? 3 : D;           // stages requested before the first is waited for
-    static_assert(WK % 2 == 0 && BLK % NW == 0 && LDS <= 160 * 1024, "");
+    static_assert(WK % 2 == 0 && BLK % NL == 0 && LDS <= 160 * 1024, "");
     static_assert((D - 1) * L < 60 && D >= 2 && D <= 7, "vmcnt counts to 63");
 };
 
-template <typename C, bool DEQ>
-__device__ __forceinline__ void tile(const int8_t *__restrict__ qx, const int8_t *__restrict__ qw, const float *__restrict__ sx,
-                                     const float *__restrict__ sw, void *__restrict__ out, const int M, const int N, const int K,
-                                     const int m0, const int n0, char *smem)
+// A loading wave (`w` of NL): all stages of the tile, in step with the multiplying waves' barriers
+template <typename C>
+__device__ __forceinline__ void load_stages(const int8_t *__restrict__ qx, const int8_t *__restrict__ qw, const int M, const int N,
+                                            const int K, const int m0, const int n0, char *smem, const int w, const int lane)
 {
-    constexpr int TM = C::TM, TN = C::TN, WK = C::WK, D = C::D, SUB = C::SUB, L = C::L, OWN = C::OWN;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int D = C::D, SUB = C::SUB, L = C::L;
     const int nk = K >> 7, ns = (nk + SUB - 1) / SUB;
-
-    // load side: load i of wave w fills block b = w + NW * i of a stage; lane l = 8 * rho + c fetches chunk c ^ sigma of row rho
+    // load i fills block b = w + NL * i of a stage; lane l = 8 * rho + c fetches chunk c ^ sigma of row rho
     const int8_t *base[L];
     unsigned roff[L];
     int sub[L];
@@ -77,7 +77,7 @@ __device__ __forceinline__ void tile(const int8_t *__restrict__ qx, const int8_t
         const int8_t *const xt = qx + (int64_t)m0 * K, *const wt = qw + (int64_t)n0 * K;
 #pragma unroll
         for (int i = 0; i < L; ++i) {
-            const int b = wave + C::NW * i;
+            const int b = w + C::NL * i;
             sub[i] = SUB == 1 ? 0 : b / (C::BX + C::BW);
             const int rb = b - sub[i] * (C::BX + C::BW);
             const bool isx = rb < C::BX;
@@ -88,18 +88,58 @@ __device__ __forceinline__ void tile(const int8_t *__restrict__ qx, const int8_t
             roff[i] = (unsigned)row * (unsigned)K + (unsigned)((c ^ sigma) << 4);
         }
     }
-    const unsigned lds0 = (unsigned)(uintptr_t)(lptr_t)smem + wave * 1024;
+    const unsigned lds0 = (unsigned)(uintptr_t)(lptr_t)smem + w * 1024;
     auto issue = [&](int s, unsigned buf) {
 #pragma unroll
         for (int i = 0; i < L; ++i) {
             int k = s * SUB + sub[i];
             if (SUB > 1 && k > nk - 1) k = nk - 1;   // a last stage that is not whole: its steps past K are not used
-            dma16(base[i], roff[i] + (unsigned)(k << 7), lds0 + buf + i * C::NW * 1024);
+            dma16(base[i], roff[i] + (unsigned)(k << 7), lds0 + buf + i * C::NL * 1024);
         }
     };
+    // at most the loads of the `behind` stages issued after it may be in flight: a stage has landed (this wave's share)
+    auto landed = [&](int behind) {   // wave-uniform, below D - 1
+        if (D > 2 && behind == D - 2) wait_vm<(D > 2 ? D - 2 : 0) * L>();
+        else if (D > 3 && behind == D - 3) wait_vm<(D > 3 ? D - 3 : 0) * L>();
+        else if (D > 4 && behind == D - 4) wait_vm<(D > 4 ? D - 4 : 0) * L>();
+        else if (D > 5 && behind == D - 5) wait_vm<(D > 5 ? D - 5 : 0) * L>();
+        else wait_vm<0>();
+    };
 #pragma unroll
-    for (int s = 0; s < C::PRE; ++s)
+    for (int s = 0; s < D - 1; ++s)
         if (s < ns) issue(s, s * C::STAGE);
+    landed(min(ns, D - 1) - 1);
+    __builtin_amdgcn_s_barrier();   // the first stage has landed
+    unsigned buf = (D - 1) * C::STAGE;
+    int s = 0;
+    for (; s + D - 1 < ns; ++s) {   // the multiplying waves read stage s
+        issue(s + D - 1, buf);      // into the buffer of stage s - 1
+        buf = buf + C::STAGE == D * C::STAGE ? 0 : buf + C::STAGE;
+        wait_vm<(D - 2) * L>();
+        __builtin_amdgcn_s_barrier();   // stage s + 1 has landed and everybody holds stage s in registers
+    }
+    for (; s < ns; ++s) {
+        if (s + 1 < ns) landed(ns - 2 - s);
+        __builtin_amdgcn_s_barrier();
+    }
+}
+
+template <typename C, bool DEQ>
+__device__ __forceinline__ void tile(const int8_t *__restrict__ qx, const int8_t *__restrict__ qw, const float *__restrict__ sx,
+                                     const float *__restrict__ sw, void *__restrict__ out, const int M, const int N, const int K,
+                                     const int m0, const int n0, char *smem)
+{
+    constexpr int TM = C::TM, TN = C::TN, WK = C::WK, D = C::D, SUB = C::SUB, OWN = C::OWN;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nk = K >> 7, ns = (nk + SUB - 1) / SUB;
+
+    if (wave >= C::NW) {
+        load_stages<C>(qx, qw, M, N, K, m0, n0, smem, wave - C::NW, lane);
+        __syncthreads();   // the two at the tile's end
+        __syncthreads();
+        return;
+    }
 
     // read side: wave (wm, wn, wk) multiplies K half wk % 2 of step wk / 2 of every stage
     const int wk = wave % WK, wmn = wave / WK;
@@ -149,57 +189,23 @@ __device__ __forceinline__ void tile(const int8_t *__restrict__ qx, const int8_t
 #pragma unroll
     for (int f = 0; f < C::NF; ++f) acc[f] = (v4i){0, 0, 0, 0};
 
-    // at most the loads of the `behind` stages issued after it may be in flight: a stage has landed (this wave's share)
-    auto landed = [&](int behind) {   // wave-uniform
-        if (behind >= D - 1) wait_vm<(D - 1) * L>();
-        else if (D > 2 && behind == D - 2) wait_vm<(D > 2 ? D - 2 : 0) * L>();
-        else if (D > 3 && behind == D - 3) wait_vm<(D > 3 ? D - 3 : 0) * L>();
-        else if (D > 4 && behind == D - 4) wait_vm<(D > 4 ? D - 4 : 0) * L>();
-        else if (D > 5 && behind == D - 5) wait_vm<(D > 5 ? D - 5 : 0) * L>();
-        else wait_vm<0>();
-    };
-    landed(min(ns, C::PRE) - 1);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    Frags fa, fb;
-    fetch(fa, 0);
-#pragma unroll
-    for (int s = C::PRE; s < D; ++s)
-        if (s < ns) issue(s, s * C::STAGE);
-
+    Frags f;
     unsigned cur = 0;
-    auto body = [&](auto STEADY, int s, Frags &now, Frags &next) {
-        constexpr bool steady = decltype(STEADY)::value;   // stage s + D exists
-        const unsigned nxt = cur + C::STAGE == D * C::STAGE ? 0 : cur + C::STAGE;
-        // this stage's fragments are in registers, the next stage has landed; behind the barrier both hold for all waves
+    for (int s = 0; s < ns; ++s) {
+        fetch(f, cur);
         __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0), as an instruction that the compiler's own counting sees
-        if constexpr (steady) wait_vm<(D - 2) * L>();
-        else if (s + 1 < ns) landed(ns - 2 - s);
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        if (steady || s + 1 < ns) fetch(next, nxt);
-        if constexpr (steady) issue(s + D, cur);
-        if (steady || SUB == 1 || s * SUB + (wk >> 1) < nk) {
+        if (SUB == 1 || s * SUB + (wk >> 1) < nk) {
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
-                    acc[i * TN + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(now.w[j], now.x[i], acc[i * TN + j], 0, 0, 0);
+                    acc[i * TN + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f.w[j], f.x[i], acc[i * TN + j], 0, 0, 0);
         }
-        cur = nxt;
-    };
-    int s = 0;
-    for (; s + 1 + D < ns; s += 2) {
-        body(std::true_type{}, s, fa, fb);
-        body(std::true_type{}, s + 1, fb, fa);
-    }
-    if (s + D < ns) {
-        body(std::true_type{}, s++, fa, fb);
-        fa = fb;
-    }
-    for (; s < ns; s += 2) {
-        body(std::false_type{}, s, fa, fb);
-        if (s + 1 < ns) body(std::false_type{}, s + 1, fb, fa);
+        __builtin_amdgcn_s_barrier();   // as in load_stages
+        asm volatile("" ::: "memory");
+        cur = cur + C::STAGE == D * C::STAGE ? 0 : cur + C::STAGE;
     }
     __syncthreads();
 
