@@ -58,7 +58,12 @@ static int gemm_route(int M, int N, int K, int cus, int *which)
     if (gemv_takes(M, N, K, cus)) return 0;
     // by the two kernels' own estimates; at most 64 rows never fill the large tiles
     const float deep = deep_estimate(M, N, K, cus, which);
-    return (M <= 64 || deep < tiled_estimate(M, N, K, cus)) && deep_fits(*which, M, N) ? 1 : 2;
+    if (M > 64) {
+        const float tiled = tiled_estimate(M, N, K, cus);
+        *which = deep_fine(M, N, K, cus, deep < tiled ? *which : -1, tiled);
+        if (*which < 0) return 2;
+    }
+    return deep_fits(*which, M, N) ? 1 : 2;
 }
 
 int32_t gemm_dispatch(const int8_t *qx, const float *sx, const int8_t *qw, const float *sw, int32_t *acc, float *y,

@@ -17,6 +17,7 @@ struct DeepProblem {
 
 // microseconds that the launch would take; *which is the tile to pass on
 float deep_estimate(int M, int N, int K, int cus, int *which);
+int deep_fine(int M, int N, int K, int cus, int coarse, float tiled_us);   // the tile after all, or -1: not this kernel
 void deep_tile(int which, int32_t *rows, int32_t *cols);
 bool deep_fits(int which, int M, int N);   // no more tiles than the kernel's arithmetic covers
 float deep_batch_estimate(const int64_t *mnk, const int *idx, int n, int cus, int *which);   // problems idx[0 .. n-1], longest K first

@@ -1,7 +1,7 @@
 // W8A8 contraction for everything between the GEMV's few tokens and the sizes that fill the chip with 256-wide tiles:
 //   acc[m,n] = sum_k qx[m,k] * qw[n,k],   y = ((float)acc * sx[m]) * sw[n]
 //
-// One workgroup per tile, the tile chosen from ten (16 x 16 to 128 x 128) so that every compute
+// One workgroup per tile, the tile chosen from sixteen (16 x 16 to 192 x 128) so that every compute
 // unit has one, and one load stream per workgroup: stages of 128 to 512 bytes of K go straight to LDS through a ring of D
 // buffers, D - 1 stages in flight, one barrier a stage.  All tiles but 128 x 128, 128 x 64 and 32 x 48 take at most half
 // of a unit's LDS: where there are tiles enough two workgroups share a unit and hide each other's first loads and last stores (16 rows,
@@ -364,35 +364,45 @@ static int32_t launch(const int8_t *qx, const float *sx, const int8_t *qw, const
 struct Tile {
     int bm, bn, sub, per_cu;
 };
-constexpr Tile TILES[] = {{128, 128, 1, 1}, {128, 64, 1, 1}, {64, 64, 1, 2}, {64, 32, 1, 2}, {32, 48, 2, 1},
-                          {32, 32, 2, 2},   {32, 16, 2, 2},  {16, 48, 2, 2}, {16, 32, 2, 2}, {16, 16, 4, 2}};
+constexpr Tile TILES[] = {{128, 128, 1, 1}, {128, 64, 1, 1}, {64, 64, 1, 2},  {64, 32, 1, 2},  {32, 48, 2, 1},
+                          {32, 32, 2, 2},   {32, 16, 2, 2},  {16, 48, 2, 2},  {16, 32, 2, 2},  {16, 16, 4, 2},
+                          {160, 128, 1, 1}, {96, 128, 1, 1}, {128, 96, 1, 1}, {192, 128, 1, 1}, {96, 64, 1, 2}, {64, 96, 1, 2}};
+constexpr int COARSE = 10;   // tiles that pick() knows
 constexpr float PER_LAUNCH = 1.72f, PER_ROUND = 0.68f, PER_OUTPUT = 2.34e-4f, PER_ROW_STEP = 0.00169f, BESIDE = 0.82f,
                 LAST_ROUND = 1.04f, PER_MB = 0.202f;
 
-static float alone(const Tile &t, int64_t nk)   // a tile on a unit of its own, without PER_ROUND
+static inline float alone(const Tile &t, int64_t nk)   // a tile on a unit of its own, without PER_ROUND
 {
     return (float)(t.bm * t.bn) * PER_OUTPUT + (float)((nk + t.sub - 1) / t.sub * t.sub) * (float)(t.bm + t.bn) * PER_ROW_STEP;
 }
 
-// core time (without the memory's share) of the best tile
+// core time of a tile, without the memory's share (a template: the divisions by its sides are by constants)
+template <int I>
+static float core_time(int M, int N, int K, int cus)
+{
+    constexpr Tile t = TILES[I];
+    const uint64_t tiles = (uint64_t)(((unsigned)M + t.bm - 1) / t.bm) * (((unsigned)N + t.bn - 1) / t.bn);
+    const unsigned slots = (unsigned)(cus * t.per_cu);
+    const uint64_t full = tiles >> 32 ? tiles / slots : (unsigned)tiles / slots;
+    const unsigned rem = (unsigned)(tiles - full * slots);
+    const float one = alone(t, K >> 7), two = (1.0f + BESIDE) * one;
+    float c = (float)full * (PER_ROUND + (t.per_cu == 2 ? two : one));
+    if (rem) c += (full ? LAST_ROUND : 1.0f) * (PER_ROUND + (rem > (unsigned)cus ? two : one));
+    return c;
+}
+template <int... I>
+static void core_times(std::integer_sequence<int, I...>, float *t, int M, int N, int K, int cus)
+{
+    ((t[I] = core_time<I>(M, N, K, cus)), ...);
+}
+
+// core time of the best tile
 static float pick(int M, int N, int K, int cus, int *which)
 {
-    float best = 0.0f;
-    int at = -1;
-    for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
-        const Tile &t = TILES[i];
-        const uint64_t tiles = (uint64_t)(((unsigned)M + t.bm - 1) / t.bm) * (((unsigned)N + t.bn - 1) / t.bn);
-        const uint64_t slots = (uint64_t)(cus * t.per_cu), full = tiles / slots, rem = tiles - full * slots;
-        const float one = alone(t, K >> 7), two = (1.0f + BESIDE) * one;
-        float c = (float)full * (PER_ROUND + (t.per_cu == 2 ? two : one));
-        if (rem) c += (full ? LAST_ROUND : 1.0f) * (PER_ROUND + (rem > (uint64_t)cus ? two : one));
-        if (at < 0 || c < best) {
-            best = c;
-            at = i;
-        }
-    }
-    *which = at;
-    return best;
+    float t[COARSE];
+    core_times(std::make_integer_sequence<int, COARSE>{}, t, M, N, K, cus);
+    *which = (int)(std::min_element(t, t + COARSE) - t);
+    return t[*which];
 }
 
 static float with_memory(float core, double bytes)
@@ -427,6 +437,67 @@ float deep_estimate(int M, int N, int K, int cus, int *which)
     return 1.04f * (c0[w] + rounds * (per_round[w] + step * (float)(K >> 7)) + per_out_mb[w] * 4e-6f * (float)M * (float)N);
 }
 
+// A finer estimate for 129 to 1024 rows and K from 1024, where a ragged edge or a half-empty round costs most: six more tiles, and
+// a constant, a time per K step of a round, which grows with the share of the slots that have a tile, and the output for each tile
+// that is worth having there.  Least squares over the times of every tile of 1447 drawn shapes (N of 512 to 28672, K to 14336,
+// weights from HBM, behind the quantizer; standard deviation 7 to 8 %).  Below 129 rows the tiles above are within 1 % of the best
+// of all.  *us: microseconds of the tile that is returned.
+namespace deep {
+struct Fine {
+    int tile;
+    float c0, step, with_fill, out_mb;
+};
+constexpr Fine FINE[] = {{0, 3.32f, 0.445f, 0.141f, 0.318f},  {1, 2.51f, 0.312f, 0.133f, 0.344f},  {2, 2.27f, 0.225f, 0.194f, 0.138f},
+                         {3, 2.27f, 0.154f, 0.159f, 0.137f},  {5, 2.25f, 0.103f, 0.148f, 0.268f},  {10, 3.67f, 0.496f, 0.069f, 0.347f},
+                         {11, 3.07f, 0.407f, 0.159f, 0.259f}, {12, 2.69f, 0.395f, 0.076f, 0.339f}, {13, 3.65f, 0.569f, 0.037f, 0.330f},
+                         {14, 2.42f, 0.291f, 0.162f, 0.149f}, {15, 2.31f, 0.300f, 0.241f, 0.115f}};
+// (a template, as core_time: the divisions by a tile's sides are by constants.  The choice of a kernel takes the host 190 ns in this
+// range and 50 for few rows, 330 and 110 with loops over the tables; a small linear is bound by its host)
+template <int I>
+static float fine_time(unsigned M, unsigned N, unsigned nk, unsigned cus, float mem4)
+{
+    constexpr Fine f = FINE[I];
+    constexpr Tile t = TILES[f.tile];
+    static_assert(t.sub == 1 || t.sub == 2, "");
+    constexpr float two = 1.0f + BESIDE;
+    const unsigned tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    const unsigned slots = cus * t.per_cu, full = tiles / slots, rem = tiles - full * slots;
+    const float rounds = (float)full * (t.per_cu == 2 ? two : 1.0f) + (rem > cus ? two : rem ? 1.0f : 0.0f);
+    const float fill = (float)tiles / (float)(slots * (full + (rem != 0)));
+    const float steps = (float)(t.sub == 2 ? (nk + 1) & ~1u : nk);
+    const float core = rounds * f.step * steps * (1.0f + f.with_fill * fill * fill) + f.out_mb * 4e-6f * (float)M * (float)N, c2 = core * core;
+    return f.c0 + sqrtf(sqrtf(c2 * c2 + mem4));
+}
+constexpr int FINES = (int)(sizeof(FINE) / sizeof(FINE[0]));
+template <int... I>
+static void fine_times(std::integer_sequence<int, I...>, float *t, unsigned M, unsigned N, unsigned nk, unsigned cus, float mem4)
+{
+    ((t[I] = fine_time<I>(M, N, nk, cus, mem4)), ...);
+}
+}  // namespace deep
+
+// The tile to take in place of `coarse`, the choice of deep_estimate, or of the LDS-tiled kernel (coarse < 0) that would take
+// `tiled_us`; -1: stay with that kernel.  Another tile has to promise 8 %, as the estimates are good to that: over the 1447
+// shapes the contraction and its quantizer then take 0.98 of the time of the coarse choice with 129 to 256 rows, 0.94 with
+// 257 to 512 and 0.95 with 513 to 1024; 16 shapes lose more than 3 %, one 9 %.  290 x 4096 -> 14336 34.6 -> 27.9 us, 350 x 4096 -> 6144
+// 21.8 -> 17.4, 600 x 4096 -> 4096 21.1 -> 17.9, 1007 x 3456 -> 1296 10.7 -> 9.7.
+int deep_fine(int M, int N, int K, int cus, int coarse, float tiled_us)
+{
+    using namespace deep;
+    if (M <= 128 || M > 1024 || K < 1024 || N > 32768) return coarse;
+    const float mem = PER_MB * 1e-6f * ((float)N * (float)K + (float)M * (float)K + 4.0f * (float)M * (float)N), m2 = mem * mem;
+    int best = -1;
+    float us = 0.0f, now = -1.0f;
+    float t[FINES];
+    fine_times(std::make_integer_sequence<int, FINES>{}, t, (unsigned)M, (unsigned)N, (unsigned)K >> 7, (unsigned)cus, m2 * m2);
+    for (int i = 0; i < FINES; ++i) {
+        if (best < 0 || t[i] < us) best = FINE[i].tile, us = t[i];
+        if (FINE[i].tile == coarse) now = t[i];
+    }
+    if (coarse < 0) return 1.08f * us < tiled_us ? best : -1;
+    return us < 0.92f * now ? best : coarse;   // (now < 0: a tile for few rows, of few columns)
+}
+
 void deep_tile(int which, int32_t *rows, int32_t *cols)
 {
     *rows = deep::TILES[which].bm;
@@ -458,6 +529,12 @@ int32_t launch_deep(int which, const int8_t *qx, const float *sx, const int8_t *
     case 7: return launch<Cfg<1, 3, 1, 1, 4, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
     case 8: return launch<Cfg<1, 2, 1, 1, 4, 6>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
     case 9: return launch<Cfg<1, 1, 1, 1, 8, 4>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 10: return launch<Cfg<5, 4, 2, 2, 2, 4>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 11: return launch<Cfg<3, 4, 2, 2, 2, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 12: return launch<Cfg<4, 3, 2, 2, 2, 5>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 13: return launch<Cfg<6, 4, 2, 2, 2, 4>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 14: return launch<Cfg<3, 2, 2, 2, 2, 4>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
+    case 15: return launch<Cfg<2, 3, 2, 2, 2, 4>, DEQ>(qx, sx, qw, sw, out, M, N, K, s);
     default: return MI_EINVAL;
     }
 }

@@ -123,6 +123,19 @@ def test_small_tile_kernel_bit_exact(mi, dev, orc, M, N, K):
     assert np.array_equal(y, orc.dequant(want, sx, sw))
 
 
+@pytest.mark.parametrize("M,N,K,tile", [
+    # the tiles that 129 to 1024 rows with K from 1024 are given by the finer estimate, on a chip of 256 units: one row or 16
+    # columns in the last tile, whole tiles, the fewest stages, several rounds of tiles
+    (480, 9904, 1152, (160, 128)), (455, 10384, 1024, (160, 128)), (288, 7552, 2048, (96, 128)), (132, 12304, 1536, (96, 128)),
+    (129, 11072, 1280, (128, 96)), (133, 10960, 1280, (128, 96)), (384, 12576, 1152, (192, 128)), (330, 13840, 1024, (192, 128)),
+    (480, 3136, 1024, (96, 64)), (259, 5008, 1024, (96, 64)), (896, 1168, 1024, (64, 96)), (129, 5776, 1024, (64, 96)),
+])
+def test_small_tile_kernel_finer_tiles_bit_exact(mi, dev, orc, M, N, K, tile):
+    got = np.zeros(2, np.int32)
+    assert mi.lib.mi_w8a8_gemm_route_host(M, N, K, 256, got.ctypes.data) == 1 and tuple(got) == tile
+    test_small_tile_kernel_bit_exact(mi, dev, orc, M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K", [
     # two to four tokens in the GEMV: its smallest and largest N and K on a chip of 256 units, four to eight chunks of K, a
     # last chunk that is not whole, rows past N in the last workgroup, three tokens in the kernel for four
