@@ -637,7 +637,9 @@ using LC = Cfg;
 // Measured, weights from HBM, us before -> after: the four projections with 256 rows 150 -> 84, with 384 rows 157 -> 122,
 // with 509 rows 160 -> 131 (gate and up tiled, qkv and down in small tiles); 2048 -> 3072, 2048, 11008 and
 // 11008 -> 2048 with 512 rows 109 -> 59.  Of 124 drawn batches (256 to 2048 rows, one to five problems) 97 go over in whole or
-// in part and take 0.26 to 1.00 of the list's time, 0.55 in the mean.
+// in part and take 0.26 to 1.00 of the list's time, 0.55 in the mean.  With tiles of 160 and 192 rows among the small ones: the four
+// projections with 327 rows 114 -> 97, with 360 122 -> 100, with 526 166 -> 145; over 100 drawn batches 0.95 of the time in the mean
+// (loading waves included), at worst 1.07.
 struct Split {
     int n_tiled = 0, n_deep = 0;
     int tiled[MAX_PROBLEMS], deep[MAX_PROBLEMS];
@@ -668,13 +670,11 @@ static Load list_load(const int64_t *mnk, const int *idx, int n, int cus, int bn
     return {*std::max_element(load, load + nx), *std::max_element(blocks, blocks + nx)};
 }
 
-// The list in 256 x 128 tiles (gemm_stream.hip): 0.84 us a unit of tile cost and 4 us beside that at best, 0.88 to 0.95 with
-// weights from HBM; taken as 1.0, for what the other estimates are good to (at 0.95 five problems with 419 rows went over and
-// took 159 instead of 146 us).  Half as large, its tiles level out where the others do not: the four projections with 509 rows
-// 142 -> 118 us, 8608 and 6144 columns of 503 rows, K = 8704, 97 -> 80, 6192 columns of 1241 rows, K = 6272, 66 -> 56.  With many
-// rounds the large tiles are 1.2 times as fast (2048 rows 355 against 419 us).  Of 120 drawn batches nine go over, 0.83 to 0.96 of
-// the time before.  From STREAM_MIN_K on; batches with a shorter K stay where they were, also where this kernel would be faster
-// (nine such batches: 0.76 to 0.92 of their time).
+// The list in 256 x 128 tiles (gemm_stream.hip): 0.92 us a unit of tile cost and 4 us beside that, weights from HBM.  Half as
+// large, its tiles level out where the others do not: the four projections with 509 rows 142 -> 111 us, 8608 and 6144 columns of
+// 503 rows, K = 8704, 97 -> 80, 6192 columns of 1241 rows, K = 6272, 66 -> 56.  With many
+// rounds the large tiles are 1.1 times as fast (2048 rows 353 against 390 us).  From STREAM_MIN_K on; batches with a shorter K
+// stay where they were, also where this kernel would be faster (nine such batches: 0.76 to 0.92 of their time).
 
 // bytes of the lists of workgroups with at most this many tiles
 static int64_t list_bytes(int cus, int64_t tiles) { return cus * (tiles + 1) * (int64_t)sizeof(v4i); }
@@ -724,7 +724,7 @@ static Split split_batch(const int64_t *mnk, int n, int cus)
         }
         if (!s.n_tiled || mnk[3 * s.tiled[s.n_tiled - 1] + 2] < STREAM_MIN_K) continue;   // (the last has the shortest K)
         const Load narrow = list_load(mnk, s.tiled, s.n_tiled, cus, STREAM_BN);
-        const float t_stream = t + (s.n_deep ? 6.0f : 4.0f) + 1.0f * (float)narrow.cost;
+        const float t_stream = t + (s.n_deep ? 6.0f : 4.0f) + 0.92f * (float)narrow.cost;
         if (t_stream < t_best && stream_bytes(cus, narrow.tiles) <= list_bytes(cus, whole.tiles)) {
             t_best = t_stream;
             best = s;

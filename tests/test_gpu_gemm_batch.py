@@ -264,6 +264,17 @@ def test_batch_by_route(mi, dev, orc, shapes, small, tile):
     check_batch(mi, dev, orc, shapes, 501 + shapes[0][0])
 
 
+@pytest.mark.parametrize("shapes,small,tile", [
+    # small tiles of 160 and 192 rows (K up to 8192 and more, none under 1024): one problem and several, ragged, beside the list
+    ([(259, 5520, 8192), (613, 3648, 1152)], [1, 1], (160, 128)),
+    ([(580, 720, 1152), (265, 4704, 8192), (546, 4304, 1024)], [1, 1, 1], (160, 128)),
+    ([(515, 5216, 8192), (522, 4016, 1152)], [1, 1], (192, 128)),
+    ([(596, 6208, 8192), (376, 4480, 1280), (326, 2880, 8192)], [1, 0, 1], (192, 128)),
+])
+def test_batch_by_route_finer_tiles(mi, dev, orc, shapes, small, tile):
+    test_batch_by_route(mi, dev, orc, shapes, small, tile)
+
+
 @pytest.mark.parametrize("shapes", [
     [(783, 5008, 1664)],                                              # one tile a workgroup, moved inwards in rows and columns
     [(797, 2800, 1536), (257, 5808, 1536), (257, 2208, 1152)],
