@@ -19,8 +19,8 @@
 // digits of the four heads with the block, and the four int32 partial sums are recombined in fp32 when the wave is
 // done.  Inside a wave the sums are exact integers (any order), across waves and splits fp32 as before.
 //
-// A workgroup of four waves owns one span of 64-token blocks of one (batch, kv head) row; wave w takes blocks
-// w, w + 4, ... of it.  Pass 1 streams the wave's key blocks (8 loads of 1 KB each) and leaves the scores in LDS;
+// A workgroup of four waves (eight where it sees a whole sequence of 257 to 1024 tokens) owns one span of 64-token blocks of one
+// (batch, kv head) row; wave w takes blocks w, w + 4, ... of it.  Pass 1 streams the wave's key blocks (8 loads of 1 KB each) and leaves the scores in LDS;
 // pass 2 streams the value blocks.  All loads run through one ring of register slots that is refilled slot by slot,
 // keys first, values behind them, so that the same number of bytes stays in flight from the first instruction to
 // the last.  The per-token scales of the span are staged in LDS once, up front.
@@ -127,18 +127,20 @@ __device__ __forceinline__ void store_token(bool is_v, int j, int tp, int64_t bl
 // launches -> one: 16 sequences of 4096 tokens, four layers 402 -> 392; one of 1531, four layers 300 -> 287; 16 of 1024
 // with experts, two layers 286 -> 280.
 template <int NW, int NTM, int RING, bool DIRECT, bool APPEND>
-__global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_tiled_split(std::conditional_t<APPEND, StepParams, Params> p)
+__global__ __launch_bounds__(64 * NW, NW > 4 ? 2 : APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_tiled_split(std::conditional_t<APPEND, StepParams, Params> p)
 {
     constexpr int SPAN = NW * NTM * 64;                   // tokens a workgroup can cover
     constexpr int SC_BYTES = NW * NTM * 4 * SROW * 4;     // scores [wave][block][head][SROW]
     constexpr int SCALE_BYTES = 2 * SPAN * 4;             // ks, vs of the span
-    constexpr int RED_BYTES = NW * 4 * D * 4;             // [wave][head][d] fp32, reuses the space above
+    constexpr int RROW = D + 16;                          // so that the four heads of a store lie in different banks
+    constexpr int RED_BYTES = NW * 4 * RROW * 4;          // [wave][head][RROW] fp32, reuses the space above
     constexpr int UNION = (SC_BYTES + SCALE_BYTES > RED_BYTES) ? SC_BYTES + SCALE_BYTES : RED_BYTES;
     static_assert(SPAN <= 4 * 64 * NW, "one float4 of each scale array per thread");
     __shared__ __attribute__((aligned(16))) char s_mem[UNION];
     __shared__ __attribute__((aligned(16))) int8_t s_q[NW][4][D];
     __shared__ __attribute__((aligned(16))) float s_out[4][D];
-    __shared__ float s_sq[NW][4], s_m[NW][4], s_l[NW][4], s_vmax[NW];
+    __shared__ float s_sq[NW][4], s_vmax[NW];
+    __shared__ __attribute__((aligned(16))) float s_m[4][NW], s_l[4][NW];   // by head and wave
     float *s_sc = reinterpret_cast<float *>(s_mem);
     float *s_ks = reinterpret_cast<float *>(s_mem + SC_BYTES);
     float *s_vs = s_ks + SPAN;
@@ -411,7 +413,7 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
     // maximum per head over the wave's tokens: lanes r16, r16 + 16, r16 + 32, r16 + 48 hold the partial maxima
     const auto larger = [](float a, float b) { return fmaxf(a, b); };
     mrun = with_far_lane<32>(with_far_lane<16>(mrun, larger), larger);
-    if (lane < 4) s_m[wave][lane] = mrun;
+    if (lane < 4) s_m[lane][wave] = mrun;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -422,7 +424,7 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
     // (quad broadcasts).  The softmax is taken against the wave's own maximum (a wave whose tokens are all masked
     // has maximum -inf: its weights are 0, and 0 stands in for the maximum).
     const int hh = r16 >> 2, dg = r16 & 3;
-    const float m_raw = s_m[wave][hh];
+    const float m_raw = s_m[hh][wave];
     const float m_h = (m_raw == -INFINITY) ? 0.0f : m_raw;
     const unsigned sh = 21u - 7u * (unsigned)dg;
     v4i acc[8];
@@ -464,7 +466,6 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
     lsum += xor_lane<1>(lsum);
     lsum += xor_lane<2>(lsum);
     lsum = add_lane<32>(add_lane<16>(lsum));
-    if ((lane & 0x33) == 0) s_l[wave][hh] = lsum;   // lanes 0, 4, 8, 12
 
     // ---- digits -> fp32.  Lane (r16, c4) holds column d = 16*n + r16 of rows 4*c4 + i: digit i of head c4, worth
     // 2^(21 - 7*i) / fix: the four digits of a value are the four registers of one lane (low digits added first).
@@ -480,45 +481,45 @@ __global__ __launch_bounds__(64 * NW, APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_t
             val[n] = f;
         }
     }
-    // ---- the waves meet.  Every wave is done with the scores and scales before their space is reused.
+    // ---- the waves meet.  Behind the barrier every wave's maxima are known and the space of the scores and scales may be reused:
+    // a wave rescales its own sums (of head c4 in this lane) to the common maximum, and what is left is adding NW numbers
+    // (rescaled by the thread that adds them: NW exponentials a thread one behind the other.  One sequence of 200, 512 tokens and
+    // 4096 in six spans 4.7, 5.6, 8.0 us; so 4.5, 5.4, 7.8)
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    {
-        float *dst = s_red + (wave * 4 + c4) * D + r16;
+    auto common = [&](int head) {
+        float m = s_m[head][0];
 #pragma unroll
-        for (int n = 0; n < 8; ++n) dst[16 * n] = val[n];
+        for (int w = 1; w < NW; ++w) m = fmaxf(m, s_m[head][w]);
+        return m;
+    };
+    {
+        const float own = s_m[c4][wave];
+        const float f = own == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(own - common(c4));
+        float *dst = s_red + (wave * 4 + c4) * RROW + r16;
+#pragma unroll
+        for (int n = 0; n < 8; ++n) dst[16 * n] = val[n] * f;
+        if (r16 == 4 * c4) s_l[c4][wave] = lsum * f;   // (hh == c4 in that lane)
     }
     __syncthreads();
-    // rescale each wave's sums from its own maximum to the common one; thread -> (d, two heads)
-    if (tid < 256) {
-        const int d = tid & (D - 1), hp = (tid >> 7) * 2;
-        float m2[2] = {s_m[0][hp], s_m[0][hp + 1]};
+    constexpr int ADD = NW < 8 ? 256 : 512;   // threads that add
+    if (NW * 64 == ADD || tid < ADD) {
 #pragma unroll
-        for (int w = 1; w < NW; ++w) {
-            m2[0] = fmaxf(m2[0], s_m[w][hp]);
-            m2[1] = fmaxf(m2[1], s_m[w][hp + 1]);
-        }
-        float sum[2] = {0.0f, 0.0f}, l[2] = {0.0f, 0.0f};
+        for (int o = 0; o < 4 * D; o += ADD) {
+            const int d = tid & (D - 1), head = (tid + o) / D;
+            float sum = 0.0f, l = 0.0f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            const float2 v = make_float2(s_red[(w * 4 + hp) * D + d], s_red[(w * 4 + hp + 1) * D + d]);
-            const float f0 = (s_m[w][hp] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(s_m[w][hp] - m2[0]);
-            const float f1 = (s_m[w][hp + 1] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(s_m[w][hp + 1] - m2[1]);
-            sum[0] += v.x * f0;
-            sum[1] += v.y * f1;
-            l[0] += s_l[w][hp] * f0;
-            l[1] += s_l[w][hp + 1] * f1;
-        }
-        if constexpr (DIRECT) {
-            s_out[hp][d] = l[0] > 0.0f ? sum[0] * (1.0f / l[0]) : 0.0f;
-            s_out[hp + 1][d] = l[1] > 0.0f ? sum[1] * (1.0f / l[1]) : 0.0f;
-        } else {
-            p.part_o[(pbase * 4 + hp) * D + d] = sum[0];
-            p.part_o[(pbase * 4 + hp + 1) * D + d] = sum[1];
-            if (d == 0) {
-                p.part_ml[pbase * 8 + hp] = m2[0];
-                p.part_ml[pbase * 8 + hp + 1] = m2[1];
-                p.part_ml[pbase * 8 + 4 + hp] = l[0];
-                p.part_ml[pbase * 8 + 4 + hp + 1] = l[1];
+            for (int w = 0; w < NW; ++w) {
+                sum += s_red[(w * 4 + head) * RROW + d];
+                l += s_l[head][w];
+            }
+            if constexpr (DIRECT) {
+                s_out[head][d] = l > 0.0f ? sum * (1.0f / l) : 0.0f;
+            } else {
+                p.part_o[(pbase * 4 + head) * D + d] = sum;
+                if (d == 0) {
+                    p.part_ml[pbase * 8 + head] = common(head);
+                    p.part_ml[pbase * 8 + 4 + head] = l;
+                }
             }
         }
     }
@@ -666,6 +667,7 @@ constexpr int NT_MAX = 4;
 
 struct Plan {
     int splits, per;   // workgroups per cache row, 64-token blocks per workgroup
+    int waves;         // of a workgroup: 4, or 8 where it sees a whole sequence
 };
 
 int max_splits(int64_t B, int64_t Hkv, int64_t T);
@@ -685,13 +687,28 @@ int max_splits(int64_t B, int64_t Hkv, int64_t T);
 // us with spans of 16 blocks -> here: 24 sequences of 3001 tokens 35.2 -> 31.3, of 750 to 3001 in pages 29.0 -> 24.7, 12 of 2500
 // 21.4 -> 16.2, 25 of 600 to 2400 25.0 -> 19.7, 32 of 318 9.5 -> 7.1; 16 of 4096 are two workgroups a unit either way, 28.7.
 // Without BATCH three sequences of 32768 were cut into 64 spans instead of 32: 39.4 instead of 25.0, the merge alone 15 more.
-static Plan pick(int64_t B, int64_t Hq, int64_t Hkv, int64_t T, bool quant)
+//
+// A row of 5 to 16 blocks whose workgroup may write the output itself (`alone`) goes to one workgroup of eight waves: no merge and no
+// second launch.  Up to 8 blocks the waves take one block instead of two, which pays until the rows fill three quarters of the units; up
+// to 12 blocks the kernel takes what it took with the merge (16 sequences of 700 tokens, 8 heads 9.7 -> 8.7 us, 4 of 700 7.2 -> 7.3)
+// and the host issues one launch for two (4 of 700 one after the other 8.3 -> 7.1); from 13 blocks on the units have to be a quarter
+// full for that to hold (16 of 1024 10.4 -> 9.2; 4 of 1024 would take 7.6 for 7.1).  Sixteen waves took 2 us more than eight: what
+// every wave does for itself, the queries above all, and the waves' meeting.  (Not one sequence: it is cut alike with codes and
+// without, see below.)
+static Plan pick(int64_t B, int64_t Hq, int64_t Hkv, int64_t T, bool quant, bool alone)
 {
     constexpr int START = 3, MERGE = 5, BATCH = 4, DIRECT = 8;
     const int blocks = (int)((T + 63) / 64);
     const int64_t rows = B * Hkv, cus = compute_units();
     Plan pl;
+    pl.waves = 4;
     const int fewest = (blocks + 4 * NT_MAX - 1) / (4 * NT_MAX);
+    if (alone && B > 1 && rows < cus && blocks > 4 && blocks <= 16 && (blocks <= 12 ? 4 * rows < 3 * cus : 4 * rows >= cus)) {
+        pl.splits = 1;
+        pl.per = blocks;
+        pl.waves = 8;
+        return pl;
+    }
     if (rows * fewest < cus) {
         // (one sequence is cut alike with codes and without: the call with the projection makes its codes either way)
         const bool codes = quant && B > 1;
@@ -780,10 +797,11 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
         return MI_EINVAL;
     if (seq_len && !aligned4(seq_len)) return MI_EINVAL;
     if (workspace_bytes < mi_gqa_decode_workspace_bytes(B, Hq, Hkv, D, T_max)) return MI_ENOSPC;
-    const avt::Plan plan = avt::pick(B, Hq, Hkv, T_max, oq != nullptr);
-    // one workgroup sees the whole sequence: it writes the output rows (the gate takes the split form: it wants no o)
+    // where one workgroup sees the whole sequence it may write the output rows (the gate takes the split form: it wants no o)
     const int64_t obytes = B * Hq * D * 4;   // (on top of the queries: row by row, or with a merge)
-    const bool direct = plan.splits == 1 && !oq && !dbg && (o == q || !overlaps(o, obytes, q, obytes));
+    const bool alone = !oq && !dbg && (o == q || !overlaps(o, obytes, q, obytes));
+    const avt::Plan plan = avt::pick(B, Hq, Hkv, T_max, oq != nullptr, alone);
+    const bool direct = plan.splits == 1 && alone;
     avt::StepParams p = {};
     p.q = q; p.kq = kq; p.ks = ks; p.vt = vt; p.vs = vs;
     p.Hq = (int)Hq; p.Hkv = (int)Hkv; p.G = (int)(Hq / Hkv); p.T = (int)T_max;
@@ -804,8 +822,16 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
     }
     p.blocks_per_split = plan.per;
     const dim3 grid((unsigned)plan.splits, (unsigned)(B * Hkv));
-    const int nt = (plan.per + 3) / 4;
-#define MI_TILED(NT_, DIR_, APP_) launch_kernel((avt::k_gqa_tiled_split<4, NT_, 8, DIR_, APP_>), grid, dim3(256), 0, s, p)   // (p as its base without APPEND)
+    const int nt = (plan.per + plan.waves - 1) / plan.waves;
+    // (p as its base without APPEND)
+#define MI_WIDE(NT_, APP_) launch_kernel((avt::k_gqa_tiled_split<8, NT_, 8, true, APP_>), grid, dim3(512), 0, s, p)
+    if (plan.waves == 8) {
+        if (step) { if (nt <= 1) MI_WIDE(1, true); else MI_WIDE(2, true); }
+        else { if (nt <= 1) MI_WIDE(1, false); else MI_WIDE(2, false); }
+        return launch_status();
+    }
+#undef MI_WIDE
+#define MI_TILED(NT_, DIR_, APP_) launch_kernel((avt::k_gqa_tiled_split<4, NT_, 8, DIR_, APP_>), grid, dim3(256), 0, s, p)
 #define MI_TILED_NT(DIR_, APP_) do { if (nt <= 1) MI_TILED(1, DIR_, APP_); else if (nt <= 2) MI_TILED(2, DIR_, APP_); else if (nt <= 3) MI_TILED(3, DIR_, APP_); else MI_TILED(4, DIR_, APP_); } while (0)
     if (step) { if (direct) MI_TILED_NT(true, true); else MI_TILED_NT(false, true); }
     else { if (direct) MI_TILED_NT(true, false); else MI_TILED_NT(false, false); }

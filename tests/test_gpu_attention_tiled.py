@@ -679,6 +679,42 @@ def test_few_rows_are_cut_into_whole_rounds(mi, dev, orc, B, Hkv, T):
         assert np.array_equal(codes[i], cq) and scales[i] == cs, i
 
 
+@pytest.mark.parametrize("B,Hkv,T", [
+    (2, 1, 257), (3, 2, 512), (47, 4, 320),            # eight waves with a block each: 5 to 8 blocks, up to three quarters of 256 units
+    (2, 4, 513), (5, 3, 768), (23, 8, 700),            # with two blocks: 9 to 12
+    (16, 4, 769), (8, 8, 1024), (31, 8, 1000),         # 13 to 16, from a quarter of the units on
+])
+def test_one_workgroup_of_eight_waves_a_row(mi, dev, orc, B, Hkv, T):
+    """Dense and paged, mixed lengths from none to T: the output of the oracle, equal to each other bit for bit."""
+    mark = dev.mark()
+    G, D, T_cap = 2, 128, (T + 63) // 64 * 64
+    Hq, pages = G * Hkv, T_cap // 64
+    q, kq, ks, vq, vs, ks_c, vs_c = make_cache(mi, dev, 700 + T, B, Hq, Hkv, T, T_cap)
+    dkt, dvt = convert(mi, dev, kq, vq, T, T_cap)
+    lens = np.array([T - (i * T) // (B - 1) for i in range(B)], np.int32)
+    table = np.random.default_rng(T).permutation(B * pages).reshape(B, pages).astype(np.int32)
+    kt, vt = dev.download(dkt), dev.download(dvt)
+    pk, pv = (dev.upload(to_pages(a.reshape(B, Hkv, pages, 8192), table, Hkv, 1)) for a in (kt, vt))
+    pks, pvs = (dev.upload(to_pages(a.reshape(B, Hkv, pages, 64), table, Hkv, 1)) for a in (ks_c, vs_c))
+    dq, dks, dvs, dl, dt = dev.upload(q), dev.upload(ks_c), dev.upload(vs_c), dev.upload(lens), dev.upload(table)
+    ws = dev.empty(mi.lib.mi_gqa_decode_workspace_bytes(B, Hq, Hkv, D, T), np.uint8)
+    o1, o2 = dev.empty((B, Hq, D), np.float32), dev.empty((B, Hq, D), np.float32)
+    mi.check(mi.lib.mi_gqa_decode_attn_tiled(dq.ptr, dkt.ptr, dks.ptr, dvt.ptr, dvs.ptr, o1.ptr, B, Hq, Hkv, D, T_cap, dl.ptr, T, 0,
+                                             ws.ptr, ws.nbytes, None))
+    mi.check(mi.lib.mi_gqa_decode_attn_tiled_paged(dq.ptr, pk.ptr, pks.ptr, pv.ptr, pvs.ptr, o2.ptr, dt.ptr, pages, B, Hq, Hkv, D,
+                                                   dl.ptr, T, 0, ws.ptr, ws.nbytes, None))
+    a, b = dev.download(o1), dev.download(o2)
+    dev.reset_to(mark)
+    assert np.array_equal(a, b)
+    for i in sorted({0, 1, B // 2, B - 2, B - 1}):
+        n = int(lens[i])
+        if n == 0:
+            assert np.all(a[i] == 0)
+            continue
+        oo = orc.gqa_decode(q[i:i + 1], kq[i:i + 1, :, :n], ks[i:i + 1, :, :n], vq[i:i + 1, :, :n], vs[i:i + 1, :, :n])
+        assert np.max(np.abs(a[i] - oo[0])) <= 2e-5, i   # the bound of every form of this kernel, see the header
+
+
 @pytest.mark.parametrize("lens", [[0, 200, 1], [256, 0, 255]])
 def test_rows_kernel_writes_the_output_of_one_span(mi, dev, orc, lens):
     """Row-major, at most 256 tokens: no merge, zeros for an empty sequence, and the output on top of the queries, in place or a row
