@@ -507,13 +507,21 @@ __global__ __launch_bounds__(64 * NW, NW > 4 ? 2 : APPEND ? 1 : NTM > 1 ? 3 : 4)
         for (int o = 0; o < 4 * D; o += ADD) {
             const int d = tid & (D - 1), head = (tid + o) / D;
             float sum = 0.0f, l = 0.0f;
+            if constexpr (NW == 8) {   // in pairs, and divided: 0.97 of the error of four waves and a merge against 64-bit sums (12 shapes of 300 to 1024 tokens; one by one 1.02)
+                float a[8], b[8];
 #pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                sum += s_red[(w * 4 + head) * RROW + d];
-                l += s_l[head][w];
+                for (int w = 0; w < 8; ++w) a[w] = s_red[(w * 4 + head) * RROW + d], b[w] = s_l[head][w];
+                sum = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+                l = ((b[0] + b[1]) + (b[2] + b[3])) + ((b[4] + b[5]) + (b[6] + b[7]));
+            } else {
+#pragma unroll
+                for (int w = 0; w < NW; ++w) {
+                    sum += s_red[(w * 4 + head) * RROW + d];
+                    l += s_l[head][w];
+                }
             }
             if constexpr (DIRECT) {
-                s_out[head][d] = l > 0.0f ? sum * (1.0f / l) : 0.0f;
+                s_out[head][d] = l > 0.0f ? (NW == 8 ? sum / l : sum * (1.0f / l)) : 0.0f;
             } else {
                 p.part_o[(pbase * 4 + head) * D + d] = sum;
                 if (d == 0) {
