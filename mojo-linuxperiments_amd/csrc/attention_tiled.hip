@@ -33,6 +33,8 @@
 #include "fwht_core.h"
 
 namespace mi {
+bool row_takes(int64_t N, int64_t K);   // gemv.hip
+bool merged_takes(int splits, int64_t N, int64_t K);
 namespace attn {
 int max_splits(int64_t B, int64_t Hkv, int64_t T);   // the row-major layout's plan: the largest split count for any length up to T
 int merge_batches(int splits, int64_t rows, bool quant);
@@ -781,6 +783,13 @@ struct StepIn {
     const int32_t *pos;
 };
 
+// the partial results of a call whose caller merges them itself, where it may (splits 0: they have been merged, or never were)
+struct Unmerged {
+    int64_t N;   // columns of the projection behind it
+    const float *o, *ml;
+    int splits;
+};
+
 struct ScoreGate {
     int8_t *qq;
     float *sq;
@@ -791,7 +800,8 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
                       int8_t *oq, float *oscale, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t T_cap,
                       const int32_t *seq_len, int64_t T_max, int32_t out_rotated, void *workspace,
                       int64_t workspace_bytes, hipStream_t s, const int32_t *block_table = nullptr,
-                      int64_t max_pages = 0, const ScoreGate *dbg = nullptr, const StepIn *step = nullptr)
+                      int64_t max_pages = 0, const ScoreGate *dbg = nullptr, const StepIn *step = nullptr,
+                      Unmerged *unmerged = nullptr)
 {
     if (block_table) {   // paged: the capacity of a sequence is its share of the table
         if (max_pages <= 0 || max_pages > (1 << 18) || !seq_len || !aligned4(block_table)) return MI_EINVAL;
@@ -848,6 +858,12 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
     if (direct || dbg) return launch_status();
     int32_t rc = launch_status();
     if (rc) return rc;
+    if (unmerged && merged_takes(plan.splits, unmerged->N, Hq * D)) {
+        unmerged->o = p.part_o;
+        unmerged->ml = p.part_ml;
+        unmerged->splits = plan.splits;
+        return MI_OK;
+    }
     return attn::launch_merge(p.part_o, p.part_ml, o, oq, oscale, B, Hq, Hkv, plan.splits, out_rotated, s);
 }
 
@@ -887,7 +903,8 @@ extern "C" int32_t mi_gqa_decode_scores_tiled_i32(const float *q, const int8_t *
 }
 
 namespace mi {
-bool row_takes(int64_t N, int64_t K);
+int32_t launch_merged_linear(const float *, const float *, int, int, const int8_t *, const float *, float *, int8_t *, float *, int64_t,
+                             int64_t, hipStream_t);
 int32_t launch_linear_fused(const float *, const int8_t *, const float *, float *, int8_t *, float *, int64_t, int64_t,
                             int64_t, hipStream_t, bool);
 }
@@ -928,9 +945,14 @@ static int32_t attn_linear(const float *q, const int8_t *kq, const float *ks, co
         // (the same row quantizer on the same values: identical codes, scale and y).  Its workgroups read the row while
         // others write: an output on top of the row takes the other route.  So do rows of less than eight heads, whose merge has
         // the fewest workgroups (four heads, 4000 tokens, 4096 outputs 24.2 us there, 25.1 here; eight heads 27.1 and 26.1).
+        // Up to eight splits the GEMV merges them as well, where nobody asks for the merged row.
+        Unmerged parts = {N, nullptr, nullptr, 0};
+        const bool may = !o_rot && apart({{attn_ws, attn_bytes}}, {{y, N * 4}});
         int32_t rc = run_tiled(q, kq, ks, vt, vs, orow, nullptr, nullptr, B, Hq, Hkv, D, T_cap, seq_len, T_max, 1, attn_ws,
-                               attn_bytes, s, nullptr, 0, nullptr, step);
+                               attn_bytes, s, nullptr, 0, nullptr, step, may ? &parts : nullptr);
         if (rc) return rc;
+        if (parts.splits)
+            return launch_merged_linear(parts.o, parts.ml, parts.splits, (int)(Hq / Hkv), qw, sw, y, oq, oscale, N, K, s);
         return launch_linear_fused(orow, qw, sw, y, oq, oscale, 1, N, K, s, false);
     }
     int32_t rc = run_tiled(q, kq, ks, vt, vs, o_rot, oq, oscale, B, Hq, Hkv, D, T_cap, seq_len, T_max, 1, attn_ws,

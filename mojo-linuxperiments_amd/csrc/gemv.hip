@@ -9,6 +9,7 @@
 //  k_gemv_row makes the codes of its one token, or its two to four, itself (rotate + quantize, with RMSNorm or SwiGLU in front),
 //  for K up to 16384 (4096).
 #include <algorithm>
+#include "attn_merge.h"
 #include "common.h"
 #include "fwht_core.h"
 
@@ -149,12 +150,18 @@ __global__ __launch_bounds__(64 * WG) void k_gemv_reg(const int8_t *__restrict__
 //   NORM: v = ((x (+ res)) * r) * g with r = 1 / sqrt(mean((x + res)^2) + eps), then rotate + quantize; workgroup 0 also leaves
 //   the residual sum (h_out) and, on request, the normalized row (xn_out);
 //   SWIGLU: v = silu(gate) * up of a row [gate | up], then rotate + quantize; workgroup 0 leaves v in xn_out on request.
+//   MERGED: the row of one token's attention, merged here from the partial results of up to MERGED_MOST splits (x, and their maxima
+//   and sums in g), then quantized as it is.  A merge of its own is a launch of 2.4 us whose 16 KB every workgroup then reads; here
+//   each reads the splits' rows, 98 KB for six.  us of attention and projection of one sequence in a chain of them, 8 kv heads, 4096 ->
+//   4096: 1531 tokens (6 splits) 11.9 -> 10.3, 2048 (8) 12.2 -> 10.9; 4 kv heads, 2048 -> 2048, 2048 tokens 9.5 -> 8.9.
 // Workgroup 0 leaves codes and scale for the caller.
-enum RowOp { ROT, PLAIN, NORM, SWIGLU };
+enum RowOp { ROT, PLAIN, NORM, SWIGLU, MERGED };
+constexpr int MERGED_MOST = 8;
 struct RowArgs {
     const float *res, *g;
     float *h_out, *xn_out;
     float eps;
+    int splits, group;   // MERGED: splits, query heads a kv head
 };
 
 // CW: 1024-byte chunks of a weight row, the last one shorter unless WHOLE.  MB: tokens, M of which are there (the last one is made
@@ -201,11 +208,16 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
     float v[MB][CQ][8];
     int base[CQ];
     float4 gl[CQ], gh[CQ], rl[MB][CQ], rh[MB][CQ];
+    attn::Partials<OP == MERGED ? MERGED_MOST : 1, false> part;
+    static_assert(OP != MERGED || CQ == 1, "a head's chunk a thread");
 #pragma unroll
     for (int i = 0; i < CQ; ++i) {
         const int c = tid + i * 512;
         base[i] = (c / LPB) * BLOCK + 4 * j;
-        if (c < nchunk) {
+        if (OP == MERGED) {
+            const int head = min(c, nchunk - 1) / LPB, kv = head / ra.group, hl = head - kv * ra.group;
+            part.load(ra.g + kv * ra.splits * 8, x + ((int64_t)kv * ra.splits * 4 + hl) * BLOCK, ra.splits, hl, j);
+        } else if (c < nchunk) {
 #pragma unroll
             for (int m = 0; m < MB; ++m) {
                 const int64_t of = MB == 1 ? base[i] : (int64_t)min(m, M - 1) * K + base[i];
@@ -301,6 +313,16 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
             }
         }
     }
+    if constexpr (OP == MERGED) {
+        float l = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[0][0][e] = 0.0f;
+        part.add(ra.splits, v[0][0], l);
+        attn::normalize_row(l, v[0][0]);
+        if (tid >= nchunk)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[0][0][e] = 0.0f;
+    }
     if constexpr (OP == NORM || OP == SWIGLU) {
         if (keeper && ra.xn_out) leave(ra.xn_out);
     }
@@ -309,7 +331,7 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
         float amax = 0.0f;
 #pragma unroll
         for (int i = 0; i < CQ; ++i) {
-            if constexpr (OP != PLAIN) fwht_codes<BLOCK>(v[m][i], j);
+            if constexpr (OP != PLAIN && OP != MERGED) fwht_codes<BLOCK>(v[m][i], j);
             amax = fmaxf(amax, abs8(v[m][i]));
         }
         amax = max_lanes<64>(amax);
@@ -431,6 +453,12 @@ bool row_takes(int64_t N, int64_t K)
            (N <= 64 * cus || (K >= 1024 && K <= 8192 && N <= 160 * cus) || (K >= 2048 && K <= 4096 && K % 1024 == 0));
 }
 
+// Every workgroup reads every split: up to MERGED_MOST of them and 4096 values (128 KB).
+bool merged_takes(int splits, int64_t N, int64_t K)
+{
+    return splits > 1 && splits <= MERGED_MOST && K >= 1024 && K <= 4096 && row_takes(N, K);
+}
+
 template <RowOp OP>
 static int32_t launch_row(const float *x, const int8_t *qw, const float *sw, float *y, int8_t *qx, float *sx, int64_t N,
                           int64_t K, const RowArgs &ra, hipStream_t s)
@@ -505,6 +533,30 @@ int32_t launch_linear_fused(const float *x, const int8_t *qw, const float *sw, f
     const RowArgs none = {};
     if (M != 1) return rotate ? launch_rows_of<ROT>(x, qw, sw, y, qx, sx, M, N, K, none, s) : MI_EINVAL;
     return rotate ? launch_row<ROT>(x, qw, sw, y, qx, sx, N, K, none, s) : launch_row<PLAIN>(x, qw, sw, y, qx, sx, N, K, none, s);
+}
+
+// The projection of one token's attention row from its partial results (the layout of attn_merge.h): part_o and part_ml are not
+// touched by the outputs.  MI_EINVAL: not covered, merge first.
+int32_t launch_merged_linear(const float *part_o, const float *part_ml, int splits, int group, const int8_t *qw, const float *sw,
+                             float *y, int8_t *qx, float *sx, int64_t N, int64_t K, hipStream_t s)
+{
+    if (!merged_takes(splits, N, K)) return MI_EINVAL;
+    RowArgs ra = {};
+    ra.g = part_ml;
+    ra.splits = splits;
+    ra.group = group;
+    const int cus = compute_units(), per_wave = (int)((N + 8 * cus - 1) / (8 * cus));
+    switch ((K + 1023) >> 10) {
+#define MI_MERGED(CW_)                                                                                                              \
+    case CW_:                                                                                                                       \
+        if (K % 1024) start_row<CW_, false, MERGED, 1>(cus, per_wave, part_o, qw, sw, y, qx, sx, (int)N, (int)K, 1, ra, s);          \
+        else start_row<CW_, true, MERGED, 1>(cus, per_wave, part_o, qw, sw, y, qx, sx, (int)N, (int)K, 1, ra, s);                    \
+        break;
+        MI_MERGED(1) MI_MERGED(2) MI_MERGED(3) MI_MERGED(4)
+#undef MI_MERGED
+    default: return MI_EINVAL;
+    }
+    return launch_status();
 }
 
 // the same with the (residual +) RMSNorm, or SwiGLU of a row [gate | up], in front

@@ -339,6 +339,15 @@ def test_vt_attention_with_projection_is_the_two_calls(mi, dev, orc, B, Hq, Hkv,
     assert np.array_equal(a, b) and np.array_equal(a, c)
 
 
+@pytest.mark.parametrize("Hq,Hkv,T_cap,N", [
+    # the projection merges the row itself: three splits of rows of one and a half chunks, the most splits, and one more, which are
+    # merged first; a head a kv head and four, the longest row and one head more
+    (12, 4, 576, 1024), (32, 8, 2048, 4096), (32, 8, 2112, 4096), (8, 8, 576, 512), (9, 9, 1024, 1040), (33, 11, 768, 256),
+])
+def test_projection_of_one_token_merges_the_row(mi, dev, orc, Hq, Hkv, T_cap, N):
+    test_vt_attention_with_projection_is_the_two_calls(mi, dev, orc, 1, Hq, Hkv, T_cap, N)
+
+
 @pytest.mark.parametrize("Hq,Hkv,N", [(32, 8, 6000), (32, 8, 16400), (32, 8, 28672), (16, 4, 12304), (16, 4, 16400),
                                        (4, 1, 2048), (8, 2, 4112), (9, 3, 16400), (20, 5, 8208), (24, 8, 41008), (40, 10, 6144),
                                        (49, 49, 2048), (64, 16, 16400)])
