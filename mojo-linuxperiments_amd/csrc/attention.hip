@@ -86,19 +86,20 @@ __device__ __forceinline__ void fold_slots(float (&p)[64], int lane)
 // tiles (the ones past the end masked), so a workgroup wants a span it can fill: 11 tiles (704 tokens) when there
 // are (batch, kv head) rows enough to occupy the chip with such spans, 4 tiles (256 tokens) when there are few rows
 // and the cache has to be cut finer to give every compute unit work.
-constexpr int TILES_LONG = 11, TILES_SHORT = 4;
+constexpr int TILES_LONG = 11, TILES_SHORT = 4, TILES_WIDE = 8;   // (WIDE: of eight waves)
 constexpr int RING = 8;           // loads a wave keeps in flight (1 KB each); tiles per wave >= RING / 2
 
 // RAGGED: the span a workgroup can cover runs past the end of the cache and token indices are clamped for the
 // loads; otherwise every address is base + constant.  Tokens past the end of the split are masked in the scores.
 // PAGED: the cache is a pool of pages [page][kv head][P tokens][128]; a 16-token tile lies in one page, so a wave
 // looks up one page per tile (uniform over the wave) and lanes are clamped inside their tile.
-// DIRECT: the workgroup sees the whole sequence and writes the output rows itself.
-template <bool DUMP, bool RAGGED, bool PAGED, int WAVE_TILES, bool DIRECT>
-__device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int8_t (&s_q)[4][4][D], float (&s_sq)[4][4],
-                                               float (&s_red)[4][4][D], float (&s_sc)[4][WAVE_TILES][16][4],
-                                               float (&s_m)[4][4], float (&s_l)[4][4])
+// DIRECT: the workgroup sees the whole sequence and writes the output rows itself.  NW: its waves, four, or eight where it is DIRECT.
+template <bool DUMP, bool RAGGED, bool PAGED, int WAVE_TILES, bool DIRECT, int NW>
+__device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int8_t (&s_q)[NW][4][D], float (&s_sq)[NW][4],
+                                               float (&s_red)[NW][4][D], float (&s_sc)[NW][WAVE_TILES][16][4],
+                                               float (&s_m)[NW][4], float (&s_l)[NW][4])
 {
+    constexpr int APART = NW * 16;   // tokens from a wave's tile to its next
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int split = blockIdx.x, bkv = blockIdx.y;
@@ -113,7 +114,7 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
     // second half of the head dimension); pass 2 lane layout: token slot l/8 of an 8-token group, chunk l%8
     const int tk16 = lane & 15, ck = lane >> 4;
     const int hh = lane & 3, slot = lane >> 3, chunk = lane & 7;
-    const int t_wave = t_lo + wave * 16;      // first token of this wave's tile 0; tile j starts 64 tokens further
+    const int t_wave = t_lo + wave * 16;      // first token of this wave's tile 0; tile j starts j * APART tokens further
     const int8_t *kwave = p.kq + ((int64_t)bkv * p.Tstride + t_wave) * D;
     const int8_t *vwave = p.vq + ((int64_t)bkv * p.Tstride + t_wave) * D;
     const float *kswave = p.ks + (int64_t)bkv * p.Tstride + t_wave;
@@ -128,7 +129,7 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
         const int last_tile = (T - 1) & ~15;
 #pragma unroll
         for (int j = 0; j < WAVE_TILES; ++j) {
-            const int tt = min(t_wave + j * 64, last_tile);
+            const int tt = min(t_wave + j * APART, last_tile);
             const int page = __builtin_amdgcn_readfirstlane(p.block_table[(int64_t)b * p.max_pages + (tt >> p.page_shift)]);
             trow[j] = (((int64_t)page * p.Hkv + kvh) << p.page_shift) + (tt & ((1 << p.page_shift) - 1));
             tlast[j] = min(T - 1 - tt, 15);
@@ -154,14 +155,14 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
             ring[(2 * j + 1) % RING] = *reinterpret_cast<const v4i *>(p.kq + row * D + 64 + 16 * ck);
             ksr[j % (RING / 2)] = p.ks[row];
         } else if constexpr (RAGGED) {
-            const int tk = min(t_wave + j * 64 + tk16, T - 1) - t_wave;
+            const int tk = min(t_wave + j * APART + tk16, T - 1) - t_wave;
             ring[(2 * j) % RING] = *reinterpret_cast<const v4i *>(kwave + (int64_t)tk * D + 16 * ck);
             ring[(2 * j + 1) % RING] = *reinterpret_cast<const v4i *>(kwave + (int64_t)tk * D + 64 + 16 * ck);
             ksr[j % (RING / 2)] = kswave[tk];
         } else {
-            ring[(2 * j) % RING] = *reinterpret_cast<const v4i *>(kwave + (koff + (unsigned)(j * 64 * D)));
-            ring[(2 * j + 1) % RING] = *reinterpret_cast<const v4i *>(kwave + (koff + (unsigned)(j * 64 * D + 64)));
-            ksr[j % (RING / 2)] = kswave[(unsigned)(j * 64) + (unsigned)tk16];
+            ring[(2 * j) % RING] = *reinterpret_cast<const v4i *>(kwave + (koff + (unsigned)(j * APART * D)));
+            ring[(2 * j + 1) % RING] = *reinterpret_cast<const v4i *>(kwave + (koff + (unsigned)(j * APART * D + 64)));
+            ksr[j % (RING / 2)] = kswave[(unsigned)(j * APART) + (unsigned)tk16];
         }
     };
     auto load_v = [&](int u) {   // group u = 2*tile + half -> slot (2*WAVE_TILES + u) % RING
@@ -171,13 +172,13 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
             ring[(2 * WAVE_TILES + u) % RING] = *reinterpret_cast<const v4i *>(p.vq + row * D + 16 * chunk);
             vsr[u % RING] = p.vs[row];
         } else if constexpr (RAGGED) {
-            const int tk = min(t_wave + j * 64 + g * 8 + slot, T - 1) - t_wave;
+            const int tk = min(t_wave + j * APART + g * 8 + slot, T - 1) - t_wave;
             ring[(2 * WAVE_TILES + u) % RING] = *reinterpret_cast<const v4i *>(vwave + (int64_t)tk * D + 16 * chunk);
             vsr[u % RING] = vswave[tk];
         } else {
             ring[(2 * WAVE_TILES + u) % RING] =
-                *reinterpret_cast<const v4i *>(vwave + ((unsigned)(lane * 16) + (unsigned)(j * 64 * D + g * 8 * D)));
-            vsr[u % RING] = vswave[(unsigned)(j * 64 + g * 8) + (unsigned)slot];
+                *reinterpret_cast<const v4i *>(vwave + ((unsigned)(lane * 16) + (unsigned)(j * APART * D + g * 8 * D)));
+            vsr[u % RING] = vswave[(unsigned)(j * APART + g * 8) + (unsigned)slot];
         }
     };
     __builtin_amdgcn_sched_barrier(0);
@@ -230,7 +231,7 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
         if (j + RING / 2 < WAVE_TILES) load_k(j + RING / 2);
         else { load_v(2 * (j + RING / 2 - WAVE_TILES)); load_v(2 * (j + RING / 2 - WAVE_TILES) + 1); }
         __builtin_amdgcn_sched_barrier(0);
-        const int tt = t_wave + j * 64 + tk16;
+        const int tt = t_wave + j * APART + tk16;
         const bool live = tt < t_end;
         float4 sc;
         sc.x = live ? (float)dots[0] * (kscale * cq[0]) : -INFINITY;
@@ -311,24 +312,43 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
     if (lane < 4) s_l[wave][lane] = lsum;
     __syncthreads();
 
-    // the four waves meet: rescale each wave's sums from its own maximum to the common one
+    // the waves meet: rescale each wave's sums from its own maximum to the common one
     const int64_t pbase = ((int64_t)bkv * gridDim.x + split);
-    auto common = [&](int h) { return fmaxf(fmaxf(s_m[0][h], s_m[1][h]), fmaxf(s_m[2][h], s_m[3][h])); };
+    auto common = [&](int h) {
+        float m = s_m[0][h];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) m = fmaxf(m, s_m[w][h]);
+        return m;
+    };
     auto rescale = [&](int w, int h, float m) { return (s_m[w][h] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(s_m[w][h] - m); };
     auto weights = [&](int h, float m) {
         float l = 0.0f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) l += (s_m[w][h] == -INFINITY) ? 0.0f : s_l[w][h] * __builtin_amdgcn_exp2f(s_m[w][h] - m);
+        for (int w = 0; w < NW; ++w) l += (s_m[w][h] == -INFINITY) ? 0.0f : s_l[w][h] * __builtin_amdgcn_exp2f(s_m[w][h] - m);
         return l;
     };
-    float total[2];
+    constexpr int ADD = 64 * NW, EACH = 4 * D / ADD;   // outputs of a thread
+    float total[EACH];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int o = tid + 256 * i, h = o >> 7, d = o & (D - 1);
+    for (int i = 0; i < EACH; ++i) {
+        const int o = tid + ADD * i, h = o >> 7, d = o & (D - 1);
         const float m = common(h);
+        if constexpr (NW == 8) {   // in pairs, and divided: 0.98 of the error of four waves and a merge against 64-bit sums (9 shapes)
+            float a[8], c[8];
+#pragma unroll
+            for (int w = 0; w < 8; ++w) {
+                const float f = rescale(w, h, m);
+                a[w] = s_red[w][h][d] * f;
+                c[w] = s_l[w][h] * f;
+            }
+            const float sum = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+            const float l = ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
+            total[i] = l > 0.0f ? sum / l : 0.0f;
+            continue;
+        }
         float sum = 0.0f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) sum += s_red[w][h][d] * rescale(w, h, m);
+        for (int w = 0; w < NW; ++w) sum += s_red[w][h][d] * rescale(w, h, m);
         if constexpr (DIRECT) {
             const float l = weights(h, m);
             total[i] = l > 0.0f ? sum * (1.0f / l) : 0.0f;
@@ -339,7 +359,7 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
     if constexpr (DIRECT) {
         __syncthreads();   // every sum has been read
 #pragma unroll
-        for (int i = 0; i < 2; ++i) s_red[0][(tid + 256 * i) >> 7][tid & (D - 1)] = total[i];
+        for (int i = 0; i < EACH; ++i) s_red[0][(tid + ADD * i) >> 7][tid & (D - 1)] = total[i];
         __syncthreads();
         if (tid < 64 && hr < G) {   // 16 lanes per head row, as the merge kernel has them
             float *const orow = p.part_o + ((int64_t)b * p.Hq + kvh * G + hr) * D;
@@ -360,14 +380,15 @@ __device__ __forceinline__ void gqa_split_body(const Params &p, const int T, int
     }
 }
 
-template <bool DUMP, int WAVE_TILES, bool DIRECT>
-__global__ __launch_bounds__(256) void k_gqa_split(Params p)
+template <bool DUMP, int WAVE_TILES, bool DIRECT, int NW = 4>
+__global__ __launch_bounds__(64 * NW) void k_gqa_split(Params p)
 {
-    __shared__ __attribute__((aligned(16))) int8_t s_q[4][4][D];
-    __shared__ float s_sq[4][4];
-    __shared__ float s_red[4][4][D];
-    __shared__ __attribute__((aligned(16))) float s_sc[4][WAVE_TILES][16][4];
-    __shared__ float s_m[4][4], s_l[4][4];
+    static_assert(NW == 4 || (NW == 8 && DIRECT), "");
+    __shared__ __attribute__((aligned(16))) int8_t s_q[NW][4][D];
+    __shared__ float s_sq[NW][4];
+    __shared__ float s_red[NW][4][D];
+    __shared__ __attribute__((aligned(16))) float s_sc[NW][WAVE_TILES][16][4];
+    __shared__ float s_m[NW][4], s_l[NW][4];
     const int tile_lo = blockIdx.x * p.tiles_per_split;
     int T = p.T;
     if (p.seq_len) {
@@ -377,7 +398,7 @@ __global__ __launch_bounds__(256) void k_gqa_split(Params p)
         if (tile_lo * 16 >= T) {
             if constexpr (DIRECT) {   // a sequence of length 0: rows of zeros
                 const int64_t row0 = (int64_t)b * p.Hq + (blockIdx.y % p.Hkv) * p.G;
-                for (int o = threadIdx.x; o < p.G * D; o += 256) p.part_o[row0 * D + o] = 0.0f;
+                for (int o = threadIdx.x; o < p.G * D; o += 64 * NW) p.part_o[row0 * D + o] = 0.0f;
                 return;
             }
             // this split lies past the end of the sequence: an empty partial (weight 0 in the merge)
@@ -391,12 +412,12 @@ __global__ __launch_bounds__(256) void k_gqa_split(Params p)
         }
     }
     if (p.block_table) {
-        gqa_split_body<false, true, true, WAVE_TILES, DIRECT>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
+        gqa_split_body<false, true, true, WAVE_TILES, DIRECT, NW>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
         return;
     }
-    const bool full = (tile_lo + 4 * WAVE_TILES) * 16 <= T;
-    if (full) gqa_split_body<DUMP, false, false, WAVE_TILES, DIRECT>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
-    else gqa_split_body<DUMP, true, false, WAVE_TILES, DIRECT>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
+    const bool full = (tile_lo + NW * WAVE_TILES) * 16 <= T;
+    if (full) gqa_split_body<DUMP, false, false, WAVE_TILES, DIRECT, NW>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
+    else gqa_split_body<DUMP, true, false, WAVE_TILES, DIRECT, NW>(p, T, s_q, s_sq, s_red, s_sc, s_m, s_l);
 }
 
 // merge the splits of blockDim.x / 16 (b, h) rows per workgroup; 16 lanes per row.  Few rows with many splits (one
@@ -517,6 +538,7 @@ __global__ __launch_bounds__(1024) void k_gqa_merge_quant(const float *__restric
 
 struct SplitPlan {
     int splits, wave_tiles;
+    int waves;   // of a workgroup: 4, or 8 where it sees a whole sequence
 };
 
 int max_splits(int64_t B, int64_t Hkv, int64_t T);
@@ -530,14 +552,24 @@ int max_splits(int64_t B, int64_t Hkv, int64_t T);
 // units that long ones leave idle: one sequence of 8192, 8193 and 16384 tokens, 8 heads 11.1, 13.2 (21.3 in 33 spans of 256) and 15.3
 // (29.3), one head 10.0, 12.7 (17.7) and 13.9 (23.5).  The merge that makes codes reads 8 spans at once (12 and 16 too) and a token in
 // one workgroup: there long spans would be ahead before 32 (8192 tokens, 8 heads, 18.4, 8193 14.9; 19.3 and 25.4 before).
-static SplitPlan pick_splits(int64_t B, int64_t Hkv, int64_t T)
+//
+// A row of 257 to 512 tokens whose workgroup may write the output itself (`alone`) goes to one workgroup of eight waves, without a
+// merge: 2 sequences of 270 tokens, 8 heads 8.4 -> 7.7 us, 16 of 384 8.8 -> 8.3, 24 of 384 11.7 -> 8.4, and the host issues one launch for
+// two (9.5 -> 7.8 one after the other).  Beyond 384 tokens only from a quarter of the units on (2 of 512 would take 8.6 for 8.3).
+// Eight tiles a wave, up to 1024 tokens, pay where spans of 704 are two a row and the rows near the units: 24 of 900 19.3 -> 13.3, but 16 of
+// 900 12.9 -> 12.7 and 8 of 900 9.2 -> 12.4.  (Not one sequence: it is cut alike with codes and without.)
+static SplitPlan pick_splits(int64_t B, int64_t Hkv, int64_t T, bool alone)
 {
     const int ntiles = (int)((T + 15) / 16);
     const int64_t rows = B * Hkv, cus = compute_units();
     auto spans = [&](int tiles) { return (ntiles + 4 * tiles - 1) / (4 * tiles); };
+    if (alone && B > 1 && rows <= cus) {
+        if (ntiles > 16 && ntiles <= 32 && (ntiles <= 24 || 4 * rows >= cus)) return {1, TILES_SHORT, 8};
+        if (ntiles > 4 * TILES_LONG && ntiles <= 64 && 4 * rows >= 3 * cus) return {1, TILES_WIDE, 8};
+    }
     const int few = spans(TILES_SHORT);
-    if (few == 1 || (rows * few <= 2 * cus && few <= 32 && few <= max_splits(B, Hkv, T))) return {few, TILES_SHORT};
-    return {spans(TILES_LONG), TILES_LONG};
+    if (few == 1 || (rows * few <= 2 * cus && few <= 32 && few <= max_splits(B, Hkv, T))) return {few, TILES_SHORT, 4};
+    return {spans(TILES_LONG), TILES_LONG, 4};
 }
 
 // at least the largest split count pick_splits returns for any length in [1, T]: what workspaces are sized for
@@ -664,7 +696,9 @@ static int32_t run_attn(const float *q, const int8_t *kq, const float *ks, const
     if (!aligned16(q) || !aligned16(kq) || !aligned16(vq) || !aligned4(ks) || !aligned4(vs) || !aligned16(workspace))
         return MI_EINVAL;
     if (workspace_bytes < mi_gqa_decode_workspace_bytes(B, Hq, Hkv, D, T)) return MI_ENOSPC;
-    const attn::SplitPlan plan = attn::pick_splits(B, Hkv, T);
+    // (output on top of the queries: row by row, or with a merge)
+    const bool alone = o && !oq && !ddots && (o == q || !overlaps(o, B * Hq * D * 4, q, B * Hq * D * 4));
+    const attn::SplitPlan plan = attn::pick_splits(B, Hkv, T, alone);
     const int splits = plan.splits;
     const int ntiles = (int)((T + 15) / 16);
     attn::Params p;
@@ -681,9 +715,8 @@ static int32_t run_attn(const float *q, const int8_t *kq, const float *ks, const
     p.score_scale = 1.4426950408889634f * 0.08838834764831845f;  // log2(e) / sqrt(128)
     const dim3 grid((unsigned)splits, (unsigned)(B * Hkv));
     // one span: its workgroup writes the output rows, with the bits that the merge of one split gives them, and no merge is launched.
-    // us, 8 heads: one sequence of 64 tokens 8.4 -> 6.6, 32 of 64 8.9 -> 7.0, 32 of 600 14.2 -> 12.2.  (Output on top of the queries: row
-    // by row, or with a merge.)
-    const bool direct = splits == 1 && o && !oq && !ddots && (o == q || !overlaps(o, B * Hq * D * 4, q, B * Hq * D * 4));
+    // us, 8 heads: one sequence of 64 tokens 8.4 -> 6.6, 32 of 64 8.9 -> 7.0, 32 of 600 14.2 -> 12.2.
+    const bool direct = splits == 1 && alone;
     if (direct) p.part_o = o;
     p.out_rotated = out_rotated;
 #define MI_SPLIT(TILES)                                                                                       \
@@ -692,7 +725,10 @@ static int32_t run_attn(const float *q, const int8_t *kq, const float *ks, const
         else if (direct) launch_kernel((attn::k_gqa_split<false, TILES, true>), grid, dim3(256), 0, s, p);    \
         else launch_kernel((attn::k_gqa_split<false, TILES, false>), grid, dim3(256), 0, s, p);               \
     } while (0)
-    if (plan.wave_tiles == attn::TILES_LONG) MI_SPLIT(attn::TILES_LONG);
+    if (plan.waves == 8) {
+        if (plan.wave_tiles == attn::TILES_SHORT) launch_kernel((attn::k_gqa_split<false, attn::TILES_SHORT, true, 8>), grid, dim3(512), 0, s, p);
+        else launch_kernel((attn::k_gqa_split<false, attn::TILES_WIDE, true, 8>), grid, dim3(512), 0, s, p);
+    } else if (plan.wave_tiles == attn::TILES_LONG) MI_SPLIT(attn::TILES_LONG);
     else MI_SPLIT(attn::TILES_SHORT);
 #undef MI_SPLIT
     if (direct) return launch_status();

@@ -750,6 +750,41 @@ def test_rows_kernel_writes_the_output_of_one_span(mi, dev, orc, lens):
     dev.reset_to(mark)
 
 
+@pytest.mark.parametrize("B,Hkv,T", [
+    (2, 1, 257), (3, 2, 384), (16, 4, 385), (17, 4, 512), (64, 4, 400),   # four tiles a wave, up to a row for every one of 256 units
+    (24, 8, 705), (32, 8, 1024),                                          # eight tiles a wave
+])
+def test_rows_kernel_of_eight_waves(mi, dev, orc, B, Hkv, T):
+    """Row-major, dense and in 16-token pages, mixed lengths from none to T: the oracle's output, equal to each other bit for bit."""
+    mark = dev.mark()
+    G, D, T_cap, P = 2, 128, (T + 63) // 64 * 64, 16
+    Hq, pages = G * Hkv, T_cap // P
+    q, kq, ks, vq, vs, ks_c, vs_c = make_cache(mi, dev, 800 + T, B, Hq, Hkv, T, T_cap)
+    kr, vr = np.zeros((B, Hkv, T_cap, D), np.int8), np.zeros((B, Hkv, T_cap, D), np.int8)
+    kr[:, :, :T], vr[:, :, :T] = kq, vq
+    lens = np.array([T - (i * T) // (B - 1) for i in range(B)], np.int32)
+    table = np.random.default_rng(T).permutation(B * pages).reshape(B, pages).astype(np.int32)
+    pk, pv = (dev.upload(to_pages(a.reshape(B, Hkv, pages, P * D), table, Hkv, 1)) for a in (kr, vr))
+    pks, pvs = (dev.upload(to_pages(a.reshape(B, Hkv, pages, P), table, Hkv, 1)) for a in (ks_c, vs_c))
+    dk, dv, dq, dks, dvs, dl, dt = (dev.upload(a) for a in (kr, vr, q, ks_c, vs_c, lens, table))
+    ws = dev.empty(mi.lib.mi_gqa_decode_workspace_bytes(B, Hq, Hkv, D, T), np.uint8)
+    o1, o2 = dev.empty((B, Hq, D), np.float32), dev.empty((B, Hq, D), np.float32)
+    mi.check(mi.lib.mi_gqa_decode_attn_cache(dq.ptr, dk.ptr, dks.ptr, dv.ptr, dvs.ptr, o1.ptr, B, Hq, Hkv, D, T_cap, dl.ptr, T, 0,
+                                             ws.ptr, ws.nbytes, None))
+    mi.check(mi.lib.mi_gqa_decode_attn_paged(dq.ptr, pk.ptr, pks.ptr, pv.ptr, pvs.ptr, o2.ptr, dt.ptr, pages, P, B, Hq, Hkv, D, dl.ptr,
+                                             T, 0, ws.ptr, ws.nbytes, None))
+    a, b = dev.download(o1), dev.download(o2)
+    dev.reset_to(mark)
+    assert np.array_equal(a, b)
+    for i in sorted({0, 1, B // 2, B - 2, B - 1}):
+        n = int(lens[i])
+        if n == 0:
+            assert np.all(a[i] == 0)
+            continue
+        oo = orc.gqa_decode(q[i:i + 1], kq[i:i + 1, :, :n], ks[i:i + 1, :, :n], vq[i:i + 1, :, :n], vs[i:i + 1, :, :n])
+        assert np.max(np.abs(a[i] - oo[0])) <= 2e-5, i   # the bound of every form of this kernel, see the header
+
+
 @pytest.mark.parametrize("rotated", [0, 1])
 def test_one_span_written_on_top_of_the_queries(mi, dev, orc, rotated):
     """At most eight blocks: the kernel writes the output itself, in place of the queries or elsewhere; a row further on, where one
