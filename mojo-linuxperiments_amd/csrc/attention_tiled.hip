@@ -903,8 +903,8 @@ extern "C" int32_t mi_gqa_decode_scores_tiled_i32(const float *q, const int8_t *
 }
 
 namespace mi {
-int32_t launch_merged_linear(const float *, const float *, int, int, const int8_t *, const float *, float *, int8_t *, float *, int64_t,
-                             int64_t, hipStream_t);
+int32_t launch_merged_linear(const float *, const float *, int, int, const int8_t *, const float *, float *, float *, int8_t *, float *,
+                             int64_t, int64_t, hipStream_t);
 int32_t launch_linear_fused(const float *, const int8_t *, const float *, float *, int8_t *, float *, int64_t, int64_t,
                             int64_t, hipStream_t, bool);
 }
@@ -945,14 +945,15 @@ static int32_t attn_linear(const float *q, const int8_t *kq, const float *ks, co
         // (the same row quantizer on the same values: identical codes, scale and y).  Its workgroups read the row while
         // others write: an output on top of the row takes the other route.  So do rows of less than eight heads, whose merge has
         // the fewest workgroups (four heads, 4000 tokens, 4096 outputs 24.2 us there, 25.1 here; eight heads 27.1 and 26.1).
-        // Up to eight splits the GEMV merges them as well, where nobody asks for the merged row.
+        // Up to eight splits the GEMV merges them as well, and leaves the row in the workspace (a row of the caller's may lie
+        // on what the others still read).
         Unmerged parts = {N, nullptr, nullptr, 0};
         const bool may = !o_rot && apart({{attn_ws, attn_bytes}}, {{y, N * 4}});
         int32_t rc = run_tiled(q, kq, ks, vt, vs, orow, nullptr, nullptr, B, Hq, Hkv, D, T_cap, seq_len, T_max, 1, attn_ws,
                                attn_bytes, s, nullptr, 0, nullptr, step, may ? &parts : nullptr);
         if (rc) return rc;
         if (parts.splits)
-            return launch_merged_linear(parts.o, parts.ml, parts.splits, (int)(Hq / Hkv), qw, sw, y, oq, oscale, N, K, s);
+            return launch_merged_linear(parts.o, parts.ml, parts.splits, (int)(Hq / Hkv), qw, sw, y, row, oq, oscale, N, K, s);
         return launch_linear_fused(orow, qw, sw, y, oq, oscale, 1, N, K, s, false);
     }
     int32_t rc = run_tiled(q, kq, ks, vt, vs, o_rot, oq, oscale, B, Hq, Hkv, D, T_cap, seq_len, T_max, 1, attn_ws,

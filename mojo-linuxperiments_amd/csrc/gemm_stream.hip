@@ -31,7 +31,6 @@
 namespace mi {
 namespace stream {
 
-
 template <int TM_, int TN_, int WM_, int WN_, int D_, int NL_>
 struct Cfg {
     static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, D = D_, NL = NL_;   // a wave's tile in 16 x 16, waves, stage buffers, loading waves

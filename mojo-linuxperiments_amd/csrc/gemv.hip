@@ -152,8 +152,8 @@ __global__ __launch_bounds__(64 * WG) void k_gemv_reg(const int8_t *__restrict__
 //   SWIGLU: v = silu(gate) * up of a row [gate | up], then rotate + quantize; workgroup 0 leaves v in xn_out on request.
 //   MERGED: the row of one token's attention, merged here from the partial results of up to MERGED_MOST splits (x, and their maxima
 //   and sums in g), then quantized as it is.  A merge of its own is a launch of 2.4 us whose 16 KB every workgroup then reads; here
-//   each reads the splits' rows, 98 KB for six.  us of attention and projection of one sequence in a chain of them, 8 kv heads, 4096 ->
-//   4096: 1531 tokens (6 splits) 11.9 -> 10.3, 2048 (8) 12.2 -> 10.9; 4 kv heads, 2048 -> 2048, 2048 tokens 9.5 -> 8.9.
+//   each reads the splits' rows, 98 KB for six, and workgroup 0 leaves the merged row in xn_out.  us of attention and projection of one sequence in a chain of
+//   them, 8 kv heads, 4096 -> 4096: 1531 tokens (6 splits) 11.9 -> 10.3, 2048 (8) 12.2 -> 10.9; 4 kv heads, 2048 -> 2048, 2048 tokens 9.5 -> 8.9.
 // Workgroup 0 leaves codes and scale for the caller.
 enum RowOp { ROT, PLAIN, NORM, SWIGLU, MERGED };
 constexpr int MERGED_MOST = 8;
@@ -323,7 +323,7 @@ __global__ __launch_bounds__(512, 2) void k_gemv_row(const float *__restrict__ x
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[0][0][e] = 0.0f;
     }
-    if constexpr (OP == NORM || OP == SWIGLU) {
+    if constexpr (OP == NORM || OP == SWIGLU || OP == MERGED) {
         if (keeper && ra.xn_out) leave(ra.xn_out);
     }
 #pragma unroll
@@ -535,14 +535,15 @@ int32_t launch_linear_fused(const float *x, const int8_t *qw, const float *sw, f
     return rotate ? launch_row<ROT>(x, qw, sw, y, qx, sx, N, K, none, s) : launch_row<PLAIN>(x, qw, sw, y, qx, sx, N, K, none, s);
 }
 
-// The projection of one token's attention row from its partial results (the layout of attn_merge.h): part_o and part_ml are not
-// touched by the outputs.  MI_EINVAL: not covered, merge first.
+// The projection of one token's attention row from its partial results (the layout of attn_merge.h), row, codes and scale left for
+// the caller: part_o and part_ml are not touched by the outputs.  MI_EINVAL: not covered, merge first.
 int32_t launch_merged_linear(const float *part_o, const float *part_ml, int splits, int group, const int8_t *qw, const float *sw,
-                             float *y, int8_t *qx, float *sx, int64_t N, int64_t K, hipStream_t s)
+                             float *y, float *row, int8_t *qx, float *sx, int64_t N, int64_t K, hipStream_t s)
 {
     if (!merged_takes(splits, N, K)) return MI_EINVAL;
     RowArgs ra = {};
     ra.g = part_ml;
+    ra.xn_out = row;
     ra.splits = splits;
     ra.group = group;
     const int cus = compute_units(), per_wave = (int)((N + 8 * cus - 1) / (8 * cus));

@@ -348,6 +348,29 @@ def test_projection_of_one_token_merges_the_row(mi, dev, orc, Hq, Hkv, T_cap, N)
     test_vt_attention_with_projection_is_the_two_calls(mi, dev, orc, 1, Hq, Hkv, T_cap, N)
 
 
+@pytest.mark.parametrize("Hq,Hkv,T,N", [(12, 4, 576, 1024), (32, 8, 2048, 4096), (32, 8, 2112, 4096), (8, 8, 576, 512)])
+def test_projection_of_one_token_leaves_the_merged_row_in_its_workspace(mi, dev, orc, Hq, Hkv, T, N):
+    """The workspace starts with the merged row, whoever merges it: the row that comes back on request, bit for bit."""
+    lib = mi.lib
+    mark = dev.mark()
+    D, K = 128, Hq * 128
+    q, kq, _, vq, _, ks, vs = make_cache(mi, dev, 37, 1, Hq, Hkv, T, T)
+    dkt, dvt = convert(mi, dev, kq, vq, T, T)
+    g = np.random.default_rng(N)
+    dqw = dev.upload(g.integers(-127, 128, (N, K), dtype=np.int8))
+    dsw = dev.upload(g.uniform(0.001, 0.1, N).astype(np.float32))
+    args = tuple(dev.upload(a).ptr if isinstance(a, np.ndarray) else a.ptr for a in (q, dkt, ks, dvt, vs))
+    ws = dev.upload(np.full(lib.mi_gqa_decode_attn_linear_workspace_bytes(1, Hq, Hkv, D, T), 0xA5, np.uint8))
+    y, row = dev.empty((1, N), np.float32), dev.empty(K, np.float32)
+    tail = (dqw.ptr, dsw.ptr, y.ptr, 1, Hq, Hkv, D, T, None, T, N, ws.ptr, ws.nbytes, None)
+    mi.check(lib.mi_gqa_decode_attn_tiled_linear_f32(*args, None, *tail))
+    kept = dev.download(ws)[:4 * K].view(np.float32)
+    mi.check(lib.mi_gqa_decode_attn_tiled_linear_f32(*args, row.ptr, *tail))
+    asked = dev.download(row)
+    dev.reset_to(mark)
+    assert np.array_equal(kept, asked)
+
+
 @pytest.mark.parametrize("Hq,Hkv,N", [(32, 8, 6000), (32, 8, 16400), (32, 8, 28672), (16, 4, 12304), (16, 4, 16400),
                                        (4, 1, 2048), (8, 2, 4112), (9, 3, 16400), (20, 5, 8208), (24, 8, 41008), (40, 10, 6144),
                                        (49, 49, 2048), (64, 16, 16400)])
