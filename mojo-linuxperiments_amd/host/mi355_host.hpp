@@ -415,7 +415,8 @@ struct MoeFfn {
 };
 
 // One decoder layer of a decode step (one new token per sequence), chained on one stream, nine launches (six for a
-// single sequence; a row-major cache takes one more, for the append):
+// single sequence, five where its attention is cut into two to eight splits, which the output projection then merges itself; a
+// row-major cache takes one more, for the append):
 // (residual +) RMSNorm + quantize -> QKV GEMV -> rotary + cache append -> attention over the cache (split, merge +
 // quantize: the output projection takes the rows in the rotated basis of V) -> O GEMV -> residual + RMSNorm +
 // quantize -> gate|up GEMV -> SwiGLU + quantize -> down GEMV (-> residual).
