@@ -818,7 +818,7 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
     // where one workgroup sees the whole sequence it may write the output rows (the gate takes the split form: it wants no o)
     const int64_t obytes = B * Hq * D * 4;   // (on top of the queries: row by row, or with a merge)
     const bool alone = !oq && !dbg && (o == q || !overlaps(o, obytes, q, obytes));
-    const avt::Plan plan = avt::pick(B, Hq, Hkv, T_max, oq != nullptr, alone);
+    const avt::Plan plan = avt::pick(B, Hq, Hkv, T_max, oq != nullptr, alone && !step);   // (a step of several sequences asks for codes)
     const bool direct = plan.splits == 1 && alone;
     avt::StepParams p = {};
     p.q = q; p.kq = kq; p.ks = ks; p.vt = vt; p.vs = vs;
@@ -842,13 +842,11 @@ static int32_t run_tiled(const float *q, const int8_t *kq, const float *ks, cons
     const dim3 grid((unsigned)plan.splits, (unsigned)(B * Hkv));
     const int nt = (plan.per + plan.waves - 1) / plan.waves;
     // (p as its base without APPEND)
-#define MI_WIDE(NT_, APP_) launch_kernel((avt::k_gqa_tiled_split<8, NT_, 8, true, APP_>), grid, dim3(512), 0, s, p)
     if (plan.waves == 8) {
-        if (step) { if (nt <= 1) MI_WIDE(1, true); else MI_WIDE(2, true); }
-        else { if (nt <= 1) MI_WIDE(1, false); else MI_WIDE(2, false); }
+        if (nt <= 1) launch_kernel((avt::k_gqa_tiled_split<8, 1, 8, true, false>), grid, dim3(512), 0, s, p);
+        else launch_kernel((avt::k_gqa_tiled_split<8, 2, 8, true, false>), grid, dim3(512), 0, s, p);
         return launch_status();
     }
-#undef MI_WIDE
 #define MI_TILED(NT_, DIR_, APP_) launch_kernel((avt::k_gqa_tiled_split<4, NT_, 8, DIR_, APP_>), grid, dim3(256), 0, s, p)
 #define MI_TILED_NT(DIR_, APP_) do { if (nt <= 1) MI_TILED(1, DIR_, APP_); else if (nt <= 2) MI_TILED(2, DIR_, APP_); else if (nt <= 3) MI_TILED(3, DIR_, APP_); else MI_TILED(4, DIR_, APP_); } while (0)
     if (step) { if (direct) MI_TILED_NT(true, true); else MI_TILED_NT(false, true); }
