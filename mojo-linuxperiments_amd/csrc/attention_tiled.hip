@@ -13,11 +13,12 @@
 //   P.V      o[h, d]    = sum_t p[t, h] * vs[t] * vq[t, d]   A = 16 rows x 64 tokens, B = a vt piece (64 t x 16 d)
 //
 // For the second product the fp32 weights a[t, h] = exp2(s[t, h] - m[h]) * vs[t] are written as fixed-point
-// numbers of 28 bits relative to the largest V scale of the workgroup's span (rounded to nearest: a token whose V
+// numbers of 28 bits relative to the largest V scale of the workgroup's span, in workgroups of eight waves of the 64-token
+// block (rounded to nearest: a token whose V
 // scale is 1/r of that largest one keeps 28 - log2(r) bits of its weight, more than fp32's 24 while r < 16) and
 // cut into four 7-bit digits; digit k of head h is row 4*k + h of A, so that ONE instruction multiplies all four
 // digits of the four heads with the block, and the four int32 partial sums are recombined in fp32 when the wave is
-// done.  Inside a wave the sums are exact integers (any order), across waves and splits fp32 as before.
+// done (with eight waves: when the block is).  Inside a wave, or a block, the sums are exact integers (any order), across them fp32.
 //
 // A workgroup of four waves (eight where it sees a whole sequence of 257 to 1024 tokens) owns one span of 64-token blocks of one
 // (batch, kv head) row; wave w takes blocks w, w + 4, ... of it.  Pass 1 streams the wave's key blocks (8 loads of 1 KB each) and leaves the scores in LDS;
@@ -132,6 +133,13 @@ template <int NW, int NTM, int RING, bool DIRECT, bool APPEND>
 __global__ __launch_bounds__(64 * NW, NW > 4 ? 2 : APPEND ? 1 : NTM > 1 ? 3 : 4) void k_gqa_tiled_split(std::conditional_t<APPEND, StepParams, Params> p)
 {
     constexpr int SPAN = NW * NTM * 64;                   // tokens a workgroup can cover
+    // What the weights' fixed point is relative to: the largest V scale of the span, or, in the span of eight waves, that of each block,
+    // whose sums become fp32 by themselves.  That span is as long as the two to four of four waves that it stands for: relative to its
+    // largest scale a token keeps fewer bits than there.  Relative 2-norm error against 64-bit sums, 11 shapes of 270 to 1024 tokens, spans
+    // of four waves and a merge / one scale for eight waves / one a block: scales alike 2.68 / 2.66 / 2.66e-7, spread over a factor of
+    // 4096 2.69 / 2.68 / 2.68e-7, one token's 256 times the others' 12.0 / 15.0 / 5.4e-7.
+    constexpr bool BY_BLOCK = NW > 4;
+    static_assert(!(BY_BLOCK && APPEND), "a new token's scale counts for the span");
     constexpr int SC_BYTES = NW * NTM * 4 * SROW * 4;     // scores [wave][block][head][SROW]
     constexpr int SCALE_BYTES = 2 * SPAN * 4;             // ks, vs of the span
     constexpr int RROW = D + 16;                          // so that the four heads of a store lie in different banks
@@ -141,7 +149,7 @@ __global__ __launch_bounds__(64 * NW, NW > 4 ? 2 : APPEND ? 1 : NTM > 1 ? 3 : 4)
     __shared__ __attribute__((aligned(16))) char s_mem[UNION];
     __shared__ __attribute__((aligned(16))) int8_t s_q[NW][4][D];
     __shared__ __attribute__((aligned(16))) float s_out[4][D];
-    __shared__ float s_sq[NW][4], s_vmax[NW];
+    __shared__ float s_sq[NW][4], s_vmax[BY_BLOCK ? NW * NTM : NW];
     __shared__ __attribute__((aligned(16))) float s_m[4][NW], s_l[4][NW];   // by head and wave
     float *s_sc = reinterpret_cast<float *>(s_mem);
     float *s_ks = reinterpret_cast<float *>(s_mem + SC_BYTES);
@@ -320,13 +328,14 @@ __global__ __launch_bounds__(64 * NW, NW > 4 ? 2 : APPEND ? 1 : NTM > 1 ? 3 : 4)
         float vm = 0.0f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) vm = fmaxf(vm, (t_lo + sidx + e < t_end && (!APPEND || t_lo + sidx + e != tp)) ? v[e] : 0.0f);
-        vm = max_lanes<64>(vm);
+        vm = max_lanes<BY_BLOCK ? 16 : 64>(vm);   // (16 lanes hold a block's scales)
         if (APPEND && owner && tp < t_end) vm = fmaxf(vm, new_vs);
         if (sidx < SPAN) {
             *reinterpret_cast<float4 *>(s_ks + sidx) = ks4;
             *reinterpret_cast<float4 *>(s_vs + sidx) = vs4;
+            if (BY_BLOCK && (tid & 15) == 0) s_vmax[tid >> 4] = vm;
         }
-        if (lane == 0) s_vmax[wave] = vm;
+        if (!BY_BLOCK && lane == 0) s_vmax[wave] = vm;
     }
     // ---- query heads of this group: every wave rotates and quantizes them for itself
     {
@@ -362,10 +371,10 @@ __global__ __launch_bounds__(64 * NW, NW > 4 ? 2 : APPEND ? 1 : NTM > 1 ? 3 : 4)
         s_ks[tp - t_lo] = new_ks;
         s_vs[tp - t_lo] = new_vs;
     }
-    float vmax = s_vmax[0];
+    float vmax = s_vmax[BY_BLOCK ? wave : 0];
 #pragma unroll
-    for (int w = 1; w < NW; ++w) vmax = fmaxf(vmax, s_vmax[w]);
-    const float fix = vmax > 0.0f ? FIX_ONE / vmax : 0.0f;   // weight -> fixed point
+    for (int w = 1; w < (BY_BLOCK ? 1 : NW); ++w) vmax = fmaxf(vmax, s_vmax[w]);
+    float fix = vmax > 0.0f ? FIX_ONE / vmax : 0.0f;   // weight -> fixed point
     // MFMA operand B of the score product: column l%16 = query head (columns >= G are zero), 16-byte chunk l/16
     v4i qb0 = {0, 0, 0, 0}, qb1 = {0, 0, 0, 0};
     if (r16 < G) {
@@ -432,9 +441,29 @@ __global__ __launch_bounds__(64 * NW, NW > 4 ? 2 : APPEND ? 1 : NTM > 1 ? 3 : 4)
     v4i acc[8];
 #pragma unroll
     for (int n = 0; n < 8; ++n) acc[n] = (v4i){0, 0, 0, 0};
+    // digits -> fp32.  Lane (r16, c4) holds column d = 16*n + r16 of rows 4*c4 + i: digit i of head c4, worth
+    // 2^(21 - 7*i) / fix: the four digits of a value are the four registers of one lane (low digits added first).
+    float val[8];
+    auto value = [&](int n) {
+        const float unit = vmax > 0.0f ? vmax / FIX_ONE : 0.0f;
+        float f = (float)acc[n][3] * unit;
+        f += (float)acc[n][2] * (unit * 128.0f);
+        f += (float)acc[n][1] * (unit * 16384.0f);
+        f += (float)acc[n][0] * (unit * 2097152.0f);
+        return f;
+    };
     float lsum = 0.0f;
     static_for<NT>([&](auto J) {
         constexpr int j = decltype(J)::value;
+        if constexpr (BY_BLOCK && j > 0) {
+#pragma unroll
+            for (int n = 0; n < 8; ++n) {
+                val[n] = j > 1 ? val[n] + value(n) : value(n);
+                acc[n] = (v4i){0, 0, 0, 0};
+            }
+            vmax = s_vmax[NW * j + wave];
+            fix = vmax > 0.0f ? FIX_ONE / vmax : 0.0f;
+        }
         const float4 s4 = *reinterpret_cast<const float4 *>(sc_wave + (j * 4 + hh) * SROW + 16 * c4 + 4 * dg);
         const float4 v4 = *reinterpret_cast<const float4 *>(s_vs + (NW * j + wave) * 64 + 16 * c4 + 4 * dg);
         const float ss[4] = {s4.x, s4.y, s4.z, s4.w}, vv[4] = {v4.x, v4.y, v4.z, v4.w};
@@ -469,20 +498,8 @@ __global__ __launch_bounds__(64 * NW, NW > 4 ? 2 : APPEND ? 1 : NTM > 1 ? 3 : 4)
     lsum += xor_lane<2>(lsum);
     lsum = add_lane<32>(add_lane<16>(lsum));
 
-    // ---- digits -> fp32.  Lane (r16, c4) holds column d = 16*n + r16 of rows 4*c4 + i: digit i of head c4, worth
-    // 2^(21 - 7*i) / fix: the four digits of a value are the four registers of one lane (low digits added first).
-    float val[8];
-    {
-        const float unit = vmax > 0.0f ? vmax / FIX_ONE : 0.0f;
 #pragma unroll
-        for (int n = 0; n < 8; ++n) {
-            float f = (float)acc[n][3] * unit;
-            f += (float)acc[n][2] * (unit * 128.0f);
-            f += (float)acc[n][1] * (unit * 16384.0f);
-            f += (float)acc[n][0] * (unit * 2097152.0f);
-            val[n] = f;
-        }
-    }
+    for (int n = 0; n < 8; ++n) val[n] = BY_BLOCK && NT > 1 ? val[n] + value(n) : value(n);
     // ---- the waves meet.  Behind the barrier every wave's maxima are known and the space of the scores and scales may be reused:
     // a wave rescales its own sums (of head c4 in this lane) to the common maximum, and what is left is adding NW numbers
     // (rescaled by the thread that adds them: NW exponentials a thread one behind the other.  One sequence of 200, 512 tokens and
@@ -509,7 +526,7 @@ __global__ __launch_bounds__(64 * NW, NW > 4 ? 2 : APPEND ? 1 : NTM > 1 ? 3 : 4)
         for (int o = 0; o < 4 * D; o += ADD) {
             const int d = tid & (D - 1), head = (tid + o) / D;
             float sum = 0.0f, l = 0.0f;
-            if constexpr (NW == 8) {   // in pairs, and divided: 0.97 of the error of four waves and a merge against 64-bit sums (12 shapes of 300 to 1024 tokens; one by one 1.02)
+            if constexpr (NW == 8) {   // in pairs, and divided: with V scales alike no more error than four waves and a merge (above); one by one 1.02 of it
                 float a[8], b[8];
 #pragma unroll
                 for (int w = 0; w < 8; ++w) a[w] = s_red[(w * 4 + head) * RROW + d], b[w] = s_l[head][w];

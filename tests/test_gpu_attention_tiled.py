@@ -747,6 +747,34 @@ def test_one_workgroup_of_eight_waves_a_row(mi, dev, orc, B, Hkv, T):
         assert np.max(np.abs(a[i] - oo[0])) <= 2e-5, i   # the bound of every form of this kernel, see the header
 
 
+@pytest.mark.parametrize("T,loud", [
+    (704, 5), (704, 2),      # two blocks a wave: a block that is its wave's only one, and one beside block 10
+    (1000, 15), (500, 3),    # the last block; a block a wave
+])
+def test_eight_waves_beside_a_block_of_large_v_scales(mi, dev, orc, T, loud):
+    """The fixed point of a block's weights is relative to the V scales of that block alone: a block whose scales are 2^20 times those
+    of the others, and whose keys look away from every query (no weight at all), leaves the others their bits.  Relative to the whole
+    row they would keep 8 of 28."""
+    mark = dev.mark()
+    B, Hkv, D, T_cap = (8 if T > 768 else 3), 8, 128, (T + 63) // 64 * 64
+    q, kq, ks, vq, vs, ks_c, vs_c = make_cache(mi, dev, 900 + T, B, Hkv, Hkv, T, T_cap)
+    at = slice(64 * loud, min(64 * loud + 64, T))
+    kq[:, :, at] = -orc.rotate_quant_rows(q.reshape(-1, D), D)[0].reshape(B, Hkv, 1, D)
+    ks[:, :, at] = ks_c[:, :, at] = 1.0
+    vs[:, :, at] *= 2.0 ** 20
+    vs_c[:, :, at] = vs[:, :, at]
+    dkt, dvt = convert(mi, dev, kq, vq, T, T_cap)
+    ws = dev.empty(mi.lib.mi_gqa_decode_workspace_bytes(B, Hkv, Hkv, D, T), np.uint8)
+    do = dev.empty((B, Hkv, D), np.float32)
+    mi.check(mi.lib.mi_gqa_decode_attn_tiled(dev.upload(q).ptr, dkt.ptr, dev.upload(ks_c).ptr, dvt.ptr, dev.upload(vs_c).ptr, do.ptr,
+                                             B, Hkv, Hkv, D, T_cap, None, T, 0, ws.ptr, ws.nbytes, None))
+    o = dev.download(do)
+    dev.reset_to(mark)
+    oo = orc.gqa_decode(q, kq, ks, vq, vs)
+    assert float(np.max(np.abs(oo))) < 8.0               # no weight on the loud block
+    assert np.max(np.abs(o - oo)) <= 2e-5                # the bound of every form of this kernel, see the header
+
+
 @pytest.mark.parametrize("lens", [[0, 200, 1], [256, 0, 255]])
 def test_rows_kernel_writes_the_output_of_one_span(mi, dev, orc, lens):
     """Row-major, at most 256 tokens: no merge, zeros for an empty sequence, and the output on top of the queries, in place or a row
