@@ -268,6 +268,9 @@ __device__ __forceinline__ void tile(const int8_t *__restrict__ qx, const int8_t
     }
 }
 
+// A grid's threads in one direction stay below 2^32: more workgroups than 2^ROW_LOG2 lie in rows of that many, the last one not whole.
+constexpr int ROW_LOG2 = 22;
+
 // Tile of workgroup `id` of a problem (ids go round robin over the XCDs): an XCD takes an eighth of the tiles, column by
 // column, so that the row tiles of a weight column meet in its L2 and no XCD has a tile more than another.
 // magic = ceil(2^32 / tiles_m) divides exactly: tiles * tiles_m < 2^32.
@@ -287,7 +290,7 @@ __global__ __launch_bounds__(C::TPB) void k_w8a8_deep(const int8_t *__restrict__
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     int tm, tn;
-    if (!tile_of((int)blockIdx.x, tiles, tiles_m, magic, &tm, &tn)) return;
+    if (!tile_of((int)(blockIdx.x + (blockIdx.y << ROW_LOG2)), tiles, tiles_m, magic, &tm, &tn)) return;
     tile<C, DEQ>(qx, qw, sx, sw, out, M, N, K, tm * C::BM, tn * C::BN, smem);
 }
 
@@ -348,8 +351,11 @@ static int32_t launch(const int8_t *qx, const float *sx, const int8_t *qw, const
     int tiles, tiles_m;
     unsigned magic;
     if (!tile_grid(C::BM, C::BN, M, N, &tiles, &tiles_m, &magic)) return MI_ERANGE;
-    launch_kernel((k_w8a8_deep<C, DEQ>), dim3((unsigned)(tiles + 7) / 8 * 8), dim3(C::TPB), C::LDS, s, qx, qw, M, N, K,
-                  tiles, tiles_m, magic, sx, sw, out);
+    constexpr unsigned ROW = 1u << ROW_LOG2;
+    static_assert((uint64_t)ROW * C::TPB < (1ull << 32) && ROW % 8 == 0, "");
+    const unsigned wgs = (unsigned)(tiles + 7) / 8 * 8;
+    launch_kernel((k_w8a8_deep<C, DEQ>), wgs <= ROW ? dim3(wgs) : dim3(ROW, (wgs + ROW - 1) / ROW), dim3(C::TPB), C::LDS, s, qx, qw,
+                  M, N, K, tiles, tiles_m, magic, sx, sw, out);
     return launch_status();
 }
 

@@ -136,6 +136,35 @@ def test_small_tile_kernel_finer_tiles_bit_exact(mi, dev, orc, M, N, K, tile):
     test_small_tile_kernel_bit_exact(mi, dev, orc, M, N, K)
 
 
+def test_small_tile_kernel_more_workgroups_than_one_row_of_a_grid(mi, orc):
+    """2^23 tiles of 48 columns, the last with 16: 2^32 threads, more than a grid has in one direction.  The weights repeat after a
+    number of rows that shares nothing with a tile; columns around the ends of the grid's rows and others drawn are compared."""
+    M, N, K, period = 5, (48 << 23) - 32, 128, 999983
+    got = np.zeros(2, np.int32)
+    assert mi.lib.mi_w8a8_gemm_route_host(M, N, K, 256, got.ctypes.data) == 1 and tuple(got) == (16, 48)
+    big = mi.Device(arena_bytes=N * K + 4 * M * N + (1 << 20))
+    try:
+        qx, base = rand_codes(7, (M, K)), rand_codes(8, (period, K))
+        dqx, dqw, dacc = big.upload(qx), big.empty((N, K), np.int8), big.empty((M, N), np.int32)
+        mi.check(mi.lib.mi_memcpy_h2d(dqw.ptr, base.ctypes.data, base.nbytes, None))
+        done = period * K
+        while done < N * K:
+            n = min(done, N * K - done)
+            mi.check(mi.lib.mi_memcpy_d2d(dqw.ptr + done, dqw.ptr, n, None))
+            done += n
+        big.sync()
+        mi.gemm_i32(dqx, dqw, dacc)
+        want = orc.gemm_i8_i32(qx, base)
+        rng = np.random.default_rng(9)
+        rows = [48 * (k << 22) for k in (0, 1)] + [N]
+        for at in [max(0, min(n - 2048, N - 4096)) for n in rows] + [int(v) for v in rng.integers(0, N - 4096, 60)]:
+            for m in range(M):
+                acc = big.download(dacc.offset(4 * (m * N + at), (4096,), np.int32))
+                assert np.array_equal(acc, want[m, (at + np.arange(4096)) % period]), (m, at)
+    finally:
+        big.close()
+
+
 @pytest.mark.parametrize("M,N,K", [
     # two to four tokens in the GEMV: its smallest and largest N and K on a chip of 256 units, four to eight chunks of K, a
     # last chunk that is not whole, rows past N in the last workgroup, three tokens in the kernel for four
