@@ -716,12 +716,13 @@ int max_splits(int64_t B, int64_t Hkv, int64_t T);
 // Without BATCH three sequences of 32768 were cut into 64 spans instead of 32: 39.4 instead of 25.0, the merge alone 15 more.
 //
 // A row of 5 to 16 blocks whose workgroup may write the output itself (`alone`) goes to one workgroup of eight waves: no merge and no
-// second launch.  Up to 8 blocks the waves take one block instead of two, which pays until the rows fill three quarters of the units; up
-// to 12 blocks the kernel takes what it took with the merge (16 sequences of 700 tokens, 8 heads 9.7 -> 8.7 us, 4 of 700 7.2 -> 7.3)
-// and the host issues one launch for two (4 of 700 one after the other 8.3 -> 7.1); from 13 blocks on the units have to be a quarter
-// full for that to hold (16 of 1024 10.4 -> 9.2; 4 of 1024 would take 7.6 for 7.1).  Sixteen waves took 2 us more than eight: what
-// every wave does for itself, the queries above all, and the waves' meeting.  (Not one sequence: it is cut alike with codes and
-// without, see below.)
+// second launch.  Up to 8 blocks the waves take one block instead of two, which pays until the rows fill three quarters of the units
+// (0.90 to 0.98 of the time, recorded and replayed, 2 to 128 rows of 270 to 512 tokens).  From 9 blocks on it pays where the spans of
+// four blocks that it stands for are more than the units: 9 to 12 blocks 0.88 to 0.92 at 88 to 128 rows and 1.01 to 1.10 below
+// (2 sequences of 768, one head 6.7 -> 7.3 us; 21 of 704, 4 heads 8.1 -> 8.8), up to three quarters of the units (0.98 to 1.00
+// at 160 to 188); 13 to 16 blocks 0.88 to 0.97 from 66 rows on and 1.07 to 1.12 at 64 (16 of 1024, 4 heads 8.4 -> 9.4; one more 8.5 -> 8.2).
+// Sixteen waves took 2 us more than eight: what every wave does for itself, the queries above all, and the waves' meeting.
+// (Not one sequence: it is cut alike with codes and without, see below.)
 static Plan pick(int64_t B, int64_t Hq, int64_t Hkv, int64_t T, bool quant, bool alone)
 {
     constexpr int START = 3, MERGE = 5, BATCH = 4, DIRECT = 8;
@@ -730,7 +731,8 @@ static Plan pick(int64_t B, int64_t Hq, int64_t Hkv, int64_t T, bool quant, bool
     Plan pl;
     pl.waves = 4;
     const int fewest = (blocks + 4 * NT_MAX - 1) / (4 * NT_MAX);
-    if (alone && B > 1 && rows < cus && blocks > 4 && blocks <= 16 && (blocks <= 12 ? 4 * rows < 3 * cus : 4 * rows >= cus)) {
+    if (alone && B > 1 && blocks > 4 && blocks <= 16 && (blocks <= 8 || rows * ((blocks + 3) / 4) > cus) &&
+        (blocks <= 12 ? 4 * rows < 3 * cus : rows < cus)) {
         pl.splits = 1;
         pl.per = blocks;
         pl.waves = 8;

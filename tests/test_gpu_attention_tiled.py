@@ -715,6 +715,8 @@ def test_few_rows_are_cut_into_whole_rounds(mi, dev, orc, B, Hkv, T):
     (2, 1, 257), (3, 2, 512), (47, 4, 320),            # eight waves with a block each: 5 to 8 blocks, up to three quarters of 256 units
     (2, 4, 513), (5, 3, 768), (23, 8, 700),            # with two blocks: 9 to 12
     (16, 4, 769), (8, 8, 1024), (31, 8, 1000),         # 13 to 16, from a quarter of the units on
+    (29, 3, 513), (11, 8, 768), (47, 4, 640),          # 9 to 12 where three spans a row are more than 256 units: from 86 rows on
+    (13, 5, 769), (9, 8, 1024),                        # 13 to 16 where four are: from 65 rows on
 ])
 def test_one_workgroup_of_eight_waves_a_row(mi, dev, orc, B, Hkv, T):
     """Dense and paged, mixed lengths from none to T: the output of the oracle, equal to each other bit for bit."""
@@ -756,7 +758,7 @@ def test_eight_waves_beside_a_block_of_large_v_scales(mi, dev, orc, T, loud):
     of the others, and whose keys look away from every query (no weight at all), leaves the others their bits.  Relative to the whole
     row they would keep 8 of 28."""
     mark = dev.mark()
-    B, Hkv, D, T_cap = (8 if T > 768 else 3), 8, 128, (T + 63) // 64 * 64
+    B, Hkv, D, T_cap = (9 if T > 768 else 11 if T > 512 else 3), 8, 128, (T + 63) // 64 * 64
     q, kq, ks, vq, vs, ks_c, vs_c = make_cache(mi, dev, 900 + T, B, Hkv, Hkv, T, T_cap)
     at = slice(64 * loud, min(64 * loud + 64, T))
     kq[:, :, at] = -orc.rotate_quant_rows(q.reshape(-1, D), D)[0].reshape(B, Hkv, 1, D)
