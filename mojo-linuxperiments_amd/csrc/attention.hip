@@ -555,7 +555,9 @@ int max_splits(int64_t B, int64_t Hkv, int64_t T);
 //
 // A row of 257 to 512 tokens whose workgroup may write the output itself (`alone`) goes to one workgroup of eight waves, without a
 // merge: 2 sequences of 270 tokens, 8 heads 8.4 -> 7.7 us, 16 of 384 8.8 -> 8.3, 24 of 384 11.7 -> 8.4, and the host issues one launch for
-// two (9.5 -> 7.8 one after the other).  Beyond 384 tokens only from a quarter of the units on (2 of 512 would take 8.6 for 8.3).
+// two (9.5 -> 7.8 one after the other).  Beyond 384 tokens only from a quarter of the units on (2 of 512 would take 8.6 for 8.3;
+// 0.94 to 1.00 of the time at 64 to 128 rows of 390 to 480), and beyond 480 only where two short spans a row are more than the units (0.78
+// at 192 rows of 512, where the other plan's spans are long ones; 8 of 512, 8 heads 8.8 -> 9.0).
 // Eight tiles a wave, up to 1024 tokens, pay where spans of 704 are two a row and the rows near the units: 24 of 900 19.3 -> 13.3, but 16 of
 // 900 12.9 -> 12.7 and 8 of 900 9.2 -> 12.4.  (Not one sequence: it is cut alike with codes and without.)
 static SplitPlan pick_splits(int64_t B, int64_t Hkv, int64_t T, bool alone)
@@ -564,7 +566,7 @@ static SplitPlan pick_splits(int64_t B, int64_t Hkv, int64_t T, bool alone)
     const int64_t rows = B * Hkv, cus = compute_units();
     auto spans = [&](int tiles) { return (ntiles + 4 * tiles - 1) / (4 * tiles); };
     if (alone && B > 1 && rows <= cus) {
-        if (ntiles > 16 && ntiles <= 32 && (ntiles <= 24 || 4 * rows >= cus)) return {1, TILES_SHORT, 8};
+        if (ntiles > 16 && ntiles <= 32 && (ntiles <= 24 || (ntiles <= 30 && 4 * rows >= cus) || 2 * rows > cus)) return {1, TILES_SHORT, 8};
         if (ntiles > 4 * TILES_LONG && ntiles <= 64 && 4 * rows >= 3 * cus) return {1, TILES_WIDE, 8};
     }
     const int few = spans(TILES_SHORT);

@@ -805,6 +805,7 @@ def test_rows_kernel_writes_the_output_of_one_span(mi, dev, orc, lens):
 
 @pytest.mark.parametrize("B,Hkv,T", [
     (2, 1, 257), (3, 2, 384), (16, 4, 385), (17, 4, 512), (64, 4, 400),   # four tiles a wave, up to a row for every one of 256 units
+    (33, 4, 481), (32, 8, 512), (16, 4, 480),                             # 31 and 32 tiles where two spans a row are more than the units
     (24, 8, 705), (32, 8, 1024),                                          # eight tiles a wave
 ])
 def test_rows_kernel_of_eight_waves(mi, dev, orc, B, Hkv, T):
