@@ -342,8 +342,8 @@ MI_API int32_t mi_gqa_decode_attn_tiled_quant_i8(const float *q, const int8_t *k
  * mi_gqa_decode_attn_tiled_quant_i8 followed by mi_w8a8_gemm_dequant_f32, bit for bit; what differs is the division
  * of the work for ONE token (B == 1, Hq*D >= 1024, N as in mi_rmsnorm_linear_f32): the merge then runs over many workgroups and leaves the
  * fp32 row, and the projection's GEMV quantizes that row in its own prologue (three launches, none of which reads
- * every split's partials through one compute unit); with two to eight splits, Hq*D up to 4096 and no o_rot that
- * prologue makes the merge as well (two launches).  o_rot (optional, fp32 [B,Hq,D]) receives the merged row.
+ * every split's partials through one compute unit); with two to eight splits, Hq*D up to 2048 (4096), N up to 64 (32)
+ * times the compute units and no o_rot that prologue makes the merge as well (two launches).  o_rot (optional, fp32 [B,Hq,D]) receives the merged row.
  * Workspace: mi_gqa_decode_attn_linear_workspace_bytes(B, Hq, Hkv, D, T_max).  It starts with the merged rows
  * (fp32, B*Hq*D*4 bytes), their codes (int8 [B, Hq*D]) and their scales (fp32 [B]), each area rounded up to 256
  * bytes - a caller may read them there after the call - and the attention's own workspace follows.  No upstream

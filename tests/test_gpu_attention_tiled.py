@@ -348,6 +348,18 @@ def test_projection_of_one_token_merges_the_row(mi, dev, orc, Hq, Hkv, T_cap, N)
     test_vt_attention_with_projection_is_the_two_calls(mi, dev, orc, 1, Hq, Hkv, T_cap, N)
 
 
+@pytest.mark.parametrize("Hq,Hkv,T_cap,N", [
+    # every split of the rows that the merging projection has on 256 units, one to four chunks of a row, whole and not, three to eight
+    # splits: up to two rows a wave (above), four, and eight in up to two chunks; one row of 16 more, which is merged first
+    (8, 2, 576, 4112), (8, 2, 1280, 8208), (8, 2, 2048, 16384), (8, 2, 768, 16400), (12, 4, 1088, 4112), (15, 5, 768, 8208),
+    (16, 4, 1536, 16384), (16, 4, 2048, 16400), (20, 5, 768, 512), (20, 5, 1792, 4112), (20, 5, 2048, 8192), (24, 8, 1280, 1024),
+    (24, 8, 640, 8192), (24, 8, 2048, 8208), (31, 31, 2048, 1040), (31, 31, 1088, 4112), (30, 10, 1536, 8192), (32, 8, 1792, 8192),
+    (32, 8, 2048, 8208),
+])
+def test_projection_of_one_token_merges_the_row_for_many_columns(mi, dev, orc, Hq, Hkv, T_cap, N):
+    test_vt_attention_with_projection_is_the_two_calls(mi, dev, orc, 1, Hq, Hkv, T_cap, N)
+
+
 @pytest.mark.parametrize("Hq,Hkv,T,N", [(12, 4, 576, 1024), (32, 8, 2048, 4096), (32, 8, 2112, 4096), (8, 8, 576, 512)])
 def test_projection_of_one_token_leaves_the_merged_row_in_its_workspace(mi, dev, orc, Hq, Hkv, T, N):
     """The workspace starts with the merged row, whoever merges it: the row that comes back on request, bit for bit."""
