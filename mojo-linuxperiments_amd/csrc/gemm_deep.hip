@@ -483,10 +483,14 @@ static void fine_times(std::integer_sequence<int, I...>, float *t, unsigned M, u
 }  // namespace deep
 
 // The tile to take in place of `coarse`, the choice of deep_estimate, or of the LDS-tiled kernel (coarse < 0) that would take
-// `tiled_us`; -1: stay with that kernel.  Another tile has to promise 8 %, as the estimates are good to that: over the 1447
-// shapes the contraction and its quantizer then take 0.98 of the time of the coarse choice with 129 to 256 rows, 0.94 with
-// 257 to 512 and 0.95 with 513 to 1024; 16 shapes lose more than 3 %, one 9 %.  290 x 4096 -> 14336 34.6 -> 27.9 us, 350 x 4096 -> 6144
-// 21.8 -> 17.4, 600 x 4096 -> 4096 21.1 -> 17.9, 1007 x 3456 -> 1296 10.7 -> 9.7.
+// `tiled_us`; -1: stay with that kernel.  Another tile has to promise 8 %, as the estimates are good to that: over 1059 drawn
+// shapes, weights from HBM, the contraction then takes 0.96 of the time of the coarse choice with 129 to 256 rows, with 257 to 512 and with
+// 513 to 1024 (332 of them go over: 0.87); 15 shapes lose more than 3 %, most of them by two rounds of 160 rows in place of one of the
+// LDS-tiled kernel (291 x 3072 -> 21984 41.0 -> 46.9).  290 x 4096 -> 14336 34.6 -> 27.9 us, 350 x 4096 -> 6144
+// 21.8 -> 17.4, 600 x 4096 -> 4096 21.1 -> 17.9, 1007 x 3456 -> 1296 10.7 -> 9.7.  A lower tile of the same columns of which there are as
+// many does not keep that promise where the weights are long: rows past the edge cost the higher one little (they read one row), and its
+// ring is the longer.  Of 70 such shapes with K from 2688 the lower one took 1.02 of the time in the mean and up to 1.16 (270 x 6656 ->
+// 8288 28.5 -> 31.6, 273 x 5120 -> 5232 17.1 -> 18.6), 1.00 below K = 2560 (of 128 columns) and 5120 (of 64).
 int deep_fine(int M, int N, int K, int cus, int coarse, float tiled_us)
 {
     using namespace deep;
@@ -501,6 +505,9 @@ int deep_fine(int M, int N, int K, int cus, int coarse, float tiled_us)
         if (FINE[i].tile == coarse) now = t[i];
     }
     if (coarse < 0) return 1.08f * us < tiled_us ? best : -1;
+    if (K * TILES[best].bn >= 2560 * 128 && TILES[best].bn == TILES[coarse].bn && TILES[best].bm < TILES[coarse].bm &&
+        ((unsigned)M + TILES[best].bm - 1) / TILES[best].bm == ((unsigned)M + TILES[coarse].bm - 1) / TILES[coarse].bm)
+        return coarse;
     return us < 0.92f * now ? best : coarse;   // (now < 0: a tile for few rows, of few columns)
 }
 

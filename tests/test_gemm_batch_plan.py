@@ -126,6 +126,8 @@ def test_route_of_a_single_contraction(mi):
         kind, (bm, bn) = r(M, N, K)
         assert kind in (0, 1, 2, 3) and (kind == 0) == (bm == 0) and (kind != 0 or M <= 4) and (kind < 2 or M > 64)
         assert kind != 3 or (M % bm == 0 and N % bn == 0)
+    # three rows of tiles either way: of 96 rows they take up to 1.1 times as long where the weights are long
+    assert r(273, 5232, 5120) == (1, (128, 64)) and r(270, 8288, 6656) == (1, (128, 128)) and r(259, 5008, 1024) == (1, (96, 64))
     # more rows of tiles than the small-tile kernel counts
     assert r(1 << 30, 16, 128)[0] == 2
     for bad in [(0, 16, 128), (-1, 16, 128), (1, 8, 128), (1, 16, 64), (1, 0, 128), (1, 16, 128, 0)]:
