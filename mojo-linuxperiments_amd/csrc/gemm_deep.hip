@@ -558,7 +558,9 @@ template int32_t launch_deep<false>(int, const int8_t *, const float *, const in
 
 // ---- several contractions of at least 256 rows in one launch (a part of a batch, see gemm_list.hip)
 // Times as above; the tiles go to the units as these come free, longest K first.  A launch of several rounds takes 1.25
-// times the sum of its tiles (measured 147 us where the sum says 115 and 83 where it says 66; what the choice that rests on
+// times the sum of its tiles, one with at most a tile of 160 or 192 rows a unit 1.15 (1.11 and 1.13 in the mean of 53; without it 259 x
+// 10240 -> 560 and 4096 -> 13456 took 57 us in such tiles for 41, 259 x 8192 -> 5520 beside 613 x 1152 -> 3648 42 for 34)
+// (measured 147 us where the sum says 115 and 83 where it says 66; what the choice that rests on
 // it gives over 124 drawn batches stands in gemm_list.hip).
 float deep_batch_estimate(const int64_t *mnk, const int *idx, int n, int cus, int *which)
 {
@@ -602,6 +604,7 @@ float deep_batch_estimate(const int64_t *mnk, const int *idx, int n, int cus, in
             }
         }
         if (count > slots) end *= 1.25f;
+        else if (t >= COARSE) end *= 1.15f;
         if (best < 0.0f || end < best) {
             best = end;
             *which = t;

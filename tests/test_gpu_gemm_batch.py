@@ -266,10 +266,16 @@ def test_batch_by_route(mi, dev, orc, shapes, small, tile):
 
 @pytest.mark.parametrize("shapes,small,tile", [
     # small tiles of 160 and 192 rows (K up to 8192 and more, none under 1024): one problem and several, ragged, beside the list
-    ([(259, 5520, 8192), (613, 3648, 1152)], [1, 1], (160, 128)),
-    ([(580, 720, 1152), (265, 4704, 8192), (546, 4304, 1024)], [1, 1, 1], (160, 128)),
-    ([(515, 5216, 8192), (522, 4016, 1152)], [1, 1], (192, 128)),
-    ([(596, 6208, 8192), (376, 4480, 1280), (326, 2880, 8192)], [1, 0, 1], (192, 128)),
+    ([(513, 6640, 8192)], [1], (160, 128)),
+    ([(577, 5456, 1152), (388, 6544, 8192)], [1, 1], (160, 128)),
+    ([(502, 8720, 1024), (803, 5360, 8192)], [0, 1], (160, 128)),
+    ([(587, 4912, 1280), (675, 5152, 8192)], [1, 1], (192, 128)),
+    ([(596, 6208, 8192), (376, 4480, 1280), (326, 2880, 8192)], [1, 1, 1], (192, 128)),
+    ([(539, 3824, 8192), (821, 9408, 1152), (284, 8752, 8192)], [1, 0, 1], (192, 128)),
+    # less than a tile of 160 or 192 rows a unit, which would take 1.2 times as long
+    ([(259, 5520, 8192), (613, 3648, 1152)], [1, 1], (128, 128)),
+    ([(580, 720, 1152), (265, 4704, 8192), (546, 4304, 1024)], [1, 1, 1], (128, 64)),
+    ([(515, 5216, 8192), (522, 4016, 1152)], [1, 1], (128, 128)),
 ])
 def test_batch_by_route_finer_tiles(mi, dev, orc, shapes, small, tile):
     test_batch_by_route(mi, dev, orc, shapes, small, tile)
