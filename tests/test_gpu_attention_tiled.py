@@ -643,6 +643,47 @@ def test_append_in_spans_of_every_length(mi, dev, B, Hq, Hkv, T_cap, T_max):
     test_append_inside_the_attention_equals_the_two_calls(mi, dev, B, Hq, Hkv, T_cap, T_max)
 
 
+@pytest.mark.parametrize("Hq,Hkv,T_cap,T_max,N", [(32, 8, 1536, 1531, 4096), (32, 8, 2048, 2048, 1024), (12, 4, 576, 520, 4112)])
+def test_append_inside_the_attention_and_the_merge_inside_the_projection(mi, dev, Hq, Hkv, T_cap, T_max, N):
+    """One token, three to eight splits, no merged row asked for: what the append, the attention that makes codes and the contraction give
+    one behind the other, bit for bit, for sequences that end in the first splits (the others count nothing), for none at all, and
+    the merged row, codes and scale left in the workspace."""
+    mark = dev.mark()
+    lib, g, D, K = mi.lib, np.random.default_rng(T_cap), 128, Hq * 128
+    heads = Hq + 2 * Hkv
+    angle = np.arange(T_cap)[:, None] * (10000.0 ** (-np.arange(D // 2) * (2.0 / D)))[None]
+    cos, sin = dev.upload(np.cos(angle).astype(np.float32)), dev.upload(np.sin(angle).astype(np.float32))
+    kq0, vq0 = (g.integers(-127, 128, (1, Hkv, T_cap, D)).astype(np.int8) for _ in range(2))
+    ks0, vs0 = (((g.random((1, Hkv, T_cap)) + 0.5) * 0.03).astype(np.float32) for _ in range(2))
+    qw, sw = dev.upload(g.integers(-127, 128, (N, K)).astype(np.int8)), dev.upload(g.random(N, dtype=np.float32))
+    qkv, q0 = dev.upload(g.standard_normal((1, heads * D)).astype(np.float32)), g.standard_normal((1, Hq, D)).astype(np.float32)
+    al = lambda n: (n + 255) // 256 * 256
+    for pos_, len_ in [(T_max - 1, T_max), (0, 1), (76, 77), (T_max // 2 - 1, T_max // 2), (T_max - 1, 77), (5, 0), (-1, 0), (256, 257)]:
+        pos, lens = dev.upload(np.array([pos_], np.int32)), dev.upload(np.array([len_], np.int32))
+        inner = dev.mark()
+        q, cache = dev.upload(q0), [dev.upload(x) for x in (kq0, ks0, vq0, vs0)]
+        c = [b.ptr for b in cache]
+        row, oq, osc = dev.empty(K, np.float32), dev.empty((1, K), np.int8), dev.empty(1, np.float32)
+        y = dev.empty((1, N), np.float32)
+        ws = dev.empty(lib.mi_gqa_decode_workspace_bytes(1, Hq, Hkv, D, T_max), np.uint8)
+        mi.check(lib.mi_rope_kv_append_tiled_f32_i8(qkv.ptr, heads * D, cos.ptr, sin.ptr, q.ptr, *c, pos.ptr, 1, Hq, Hkv, D, T_cap, None))
+        mi.check(lib.mi_gqa_decode_attn_tiled_quant_i8(q.ptr, *c, row.ptr, oq.ptr, osc.ptr, 1, Hq, Hkv, D, T_cap, lens.ptr, T_max,
+                                                       ws.ptr, ws.nbytes, None))
+        mi.check(lib.mi_w8a8_gemm_dequant_f32(oq.ptr, osc.ptr, qw.ptr, sw.ptr, y.ptr, 1, N, K, None))
+        want = [dev.download(b) for b in [q, y, row, oq, osc] + cache]
+        q, cache = dev.upload(q0), [dev.upload(x) for x in (kq0, ks0, vq0, vs0)]
+        c = [b.ptr for b in cache]
+        ws = dev.upload(np.full(lib.mi_gqa_decode_attn_linear_workspace_bytes(1, Hq, Hkv, D, T_max), 0xA5, np.uint8))
+        mi.check(lib.mi_rope_append_attn_tiled_linear_f32(qkv.ptr, heads * D, cos.ptr, sin.ptr, q.ptr, *c, pos.ptr, None, qw.ptr, sw.ptr,
+                                                          y.ptr, 1, Hq, Hkv, D, T_cap, lens.ptr, T_max, N, ws.ptr, ws.nbytes, None))
+        left = (ws.offset(0, (K,), np.float32), ws.offset(al(4 * K), (1, K), np.int8), ws.offset(al(4 * K) + al(K), (1,), np.float32))
+        got = [dev.download(b) for b in [q, y, *left] + cache]
+        for name, a, b in zip(("q", "y", "row", "codes", "scale", "kq", "ks", "vq", "vs"), want, got):
+            assert np.array_equal(a, b), (name, pos_, len_)
+        dev.reset_to(inner)
+    dev.reset_to(mark)
+
+
 @pytest.mark.parametrize("T", [40, 3000])   # one split, which writes the output rows itself, and many
 @pytest.mark.parametrize("q_at,o_at", [("qkv", None), ("qkv", "qkv"), (None, "qkv"), ("both", "both")])
 def test_append_inside_the_attention_with_overlapping_buffers(mi, dev, T, q_at, o_at):
