@@ -124,6 +124,21 @@ def test_small_tile_kernel_bit_exact(mi, dev, orc, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K,tile", [
+    # the tiles of any number of rows on a chip of 256 units, with twice as many stages as their rings hold or more, so that every
+    # buffer is used again; ragged; a last stage that is whole and one that is not.  The last two: of a prompt and a chunk of it
+    (195, 12352, 1280, (128, 128)), (66, 8736, 1536, (128, 64)), (34, 8240, 1280, (64, 64)), (33, 6480, 1536, (64, 32)),
+    (33, 4384, 2944, (32, 48)), (33, 4528, 3072, (32, 48)), (17, 6608, 2560, (32, 32)), (17, 6576, 2432, (32, 32)),
+    (17, 2304, 3072, (32, 16)), (19, 2224, 3200, (32, 16)), (7, 8432, 2432, (16, 48)), (9, 8320, 2560, (16, 48)),
+    (7, 4176, 2944, (16, 32)), (9, 4112, 3072, (16, 32)), (17, 16, 3712, (16, 16)), (18, 16, 4096, (16, 16)),
+    (200, 14336, 4096, (128, 128)), (509, 4096, 14336, (128, 64)),
+])
+def test_small_tile_kernel_past_its_ring_bit_exact(mi, dev, orc, M, N, K, tile):
+    got = np.zeros(2, np.int32)
+    assert mi.lib.mi_w8a8_gemm_route_host(M, N, K, 256, got.ctypes.data) == 1 and tuple(got) == tile
+    test_small_tile_kernel_bit_exact(mi, dev, orc, M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
     # the tiles that 129 to 1024 rows with K from 1024 are given by the finer estimate, on a chip of 256 units: one row or 16
     # columns in the last tile, whole tiles, the fewest stages, several rounds of tiles
     (480, 9904, 1152, (160, 128)), (455, 10384, 1024, (160, 128)), (288, 7552, 2048, (96, 128)), (132, 12304, 1536, (96, 128)),
