@@ -21,7 +21,7 @@
 // done (with eight waves: when the block is).  Inside a wave, or a block, the sums are exact integers (any order), across them fp32.
 //
 // A workgroup of four waves (eight where it sees a whole sequence of 257 to 1024 tokens) owns one span of 64-token blocks of one
-// (batch, kv head) row; wave w takes blocks w, w + 4, ... of it.  Pass 1 streams the wave's key blocks (8 loads of 1 KB each) and leaves the scores in LDS;
+// (batch, kv head) row; wave w takes blocks w, w + 4 (w + 8), ... of it.  Pass 1 streams the wave's key blocks (8 loads of 1 KB each) and leaves the scores in LDS;
 // pass 2 streams the value blocks.  All loads run through one ring of register slots that is refilled slot by slot,
 // keys first, values behind them, so that the same number of bytes stays in flight from the first instruction to
 // the last.  The per-token scales of the span are staged in LDS once, up front.

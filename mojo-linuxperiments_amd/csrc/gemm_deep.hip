@@ -3,8 +3,8 @@
 //
 // One workgroup per tile, the tile chosen from sixteen (16 x 16 to 192 x 128) so that every compute
 // unit has one, and one load stream per workgroup: stages of 128 to 512 bytes of K go straight to LDS through a ring of D
-// buffers, D - 1 stages in flight, one barrier a stage.  All tiles but 128 x 128, 128 x 64 and 32 x 48 take at most half
-// of a unit's LDS: where there are tiles enough two workgroups share a unit and hide each other's first loads and last stores (16 rows,
+// buffers, D - 1 stages in flight, one barrier a stage.  The tiles of 128 columns, 128 x 96, 128 x 64 and 32 x 48 take more than half
+// of a unit's LDS, the others at most half: where there are tiles enough two workgroups share a unit and hide each other's first loads and last stores (16 rows,
 // 4096 -> 28672 inside a decode step: 24.3 instead of 27.2 us).  Small tiles leave most
 // waves without rows of their own, so the waves split K inside a stage (WK slices of 64 bytes) and meet once, through
 // LDS, at the tile's end; every wave finishes an equal share of the matrix-instruction tiles.
@@ -362,11 +362,12 @@ static int32_t launch(const int8_t *qx, const float *sx, const int8_t *qw, const
 // ---- which tile ----------------------------------------------------------------------------------------------------
 // Time of a launch in microseconds, fitted to 250 shapes (M of 2 to 1024, N of 784 to 28672, K of 1024 to 14336) times
 // every tile, each measured behind the quantizer that feeds it and with weights from HBM.  A unit moves (BM + BN) * 128
-// bytes per K step through its load path at 1.69 ns a row (76 GB/s: the direct-to-LDS loads of a workgroup take about
-// 28 clocks a KB, which is more than the matrix instructions of any of these tiles), 1.82 instead of 2 times as long
+// bytes per K step through its load path at 1.69 ns a row (76 GB/s, 28 clocks a KB: as it was when the waves that multiply made the
+// loads; with waves of their own a launch takes 2 to 6 % less, and the figures stay for the order of the tiles that they give), 1.82
+// instead of 2 times as long
 // for two workgroups side by side, and pays 0.7 us plus the tile's outputs per round of tiles.  The memory's share,
-// bytes at 5 TB/s, is joined as a 4-norm: it does not depend on the tile.  Picking by it costs 0.5 % on average over
-// picking the fastest tile of every shape, 15 % at worst.
+// bytes at 5 TB/s, is joined as a 4-norm: it does not depend on the tile.  Over 1059 drawn shapes of 129 to 1024 rows the choice that rests
+// on it takes 1.061 of the time of the best of all tiles and kernels, with the finer estimate below 1.016.
 struct Tile {
     int bm, bn, sub, per_cu;
 };
@@ -446,8 +447,8 @@ float deep_estimate(int M, int N, int K, int cus, int *which)
 // A finer estimate for 129 to 1024 rows and K from 1024, where a ragged edge or a half-empty round costs most: six more tiles, and
 // a constant, a time per K step of a round, which grows with the share of the slots that have a tile, and the output for each tile
 // that is worth having there.  Least squares over the times of every tile of 1447 drawn shapes (N of 512 to 28672, K to 14336,
-// weights from HBM, behind the quantizer; standard deviation 7 to 8 %).  Below 129 rows the tiles above are within 1 % of the best
-// of all.  *us: microseconds of the tile that is returned.
+// weights from HBM, behind the quantizer; standard deviation 7 to 8 %, of 1200 others 8 to 10).  Below 129 rows the tiles above are
+// within 1 % of the best of all; beyond 1024 no shape was timed.
 namespace deep {
 struct Fine {
     int tile;
@@ -558,17 +559,17 @@ template int32_t launch_deep<false>(int, const int8_t *, const float *, const in
 
 // ---- several contractions of at least 256 rows in one launch (a part of a batch, see gemm_list.hip)
 // Times as above; the tiles go to the units as these come free, longest K first.  A launch of several rounds takes 1.25
-// times the sum of its tiles, one with at most a tile of 160 or 192 rows a unit 1.15 (1.11 and 1.13 in the mean of 53; without it 259 x
-// 10240 -> 560 and 4096 -> 13456 took 57 us in such tiles for 41, 259 x 8192 -> 5520 beside 613 x 1152 -> 3648 42 for 34)
-// (measured 147 us where the sum says 115 and 83 where it says 66; what the choice that rests on
-// it gives over 124 drawn batches stands in gemm_list.hip).
+// times the sum of its tiles (measured 147 us where the sum says 115 and 83 where it says 66; what the choice that rests on
+// it gives over drawn batches stands in gemm_list.hip), one with at most a tile of 160 or 192 rows a unit 1.15 (1.11 and 1.13 in the mean
+// of 53; without it 259 x 10240 -> 560 and 4096 -> 13456 took 57 us in such tiles for 41, 259 x 8192 -> 5520 beside 613 x 1152 ->
+// 3648 42 for 34).
 float deep_batch_estimate(const int64_t *mnk, const int *idx, int n, int cus, int *which)
 {
     using namespace deep;
     // 128 x 128, 128 x 64, 64 x 64 and, where the longest K is from 8192 and the shortest from 1024, 160 x 128 and 192 x 128: the four
-    // projections with 300 rows 117 -> 101 us, with 384 134 -> 113, with 560 189 -> 167 (quantizer included).  Batches of shorter K
-    // mostly have a list that levels out: with these tiles there as well 60 drawn batches took 0.98 of the time in the mean, some
-    // 0.75 and some 1.05.
+    // projections with 300 rows 117 -> 101 us, with 384 134 -> 113, with 560 189 -> 167 (quantizer included).  The limits stand in for
+    // an estimate that tells batches of shorter K apart, which this one does not: with these tiles there as well 170 drawn batches took
+    // 0.93 of the time in the mean, 36 of them more than 1.03 and up to 1.24 of it.
     constexpr int TRY[] = {0, 1, 2, 10, 13};
     const bool finer = mnk[3 * idx[0] + 2] >= 8192 && mnk[3 * idx[n - 1] + 2] >= 1024;
     float best = -1.0f;

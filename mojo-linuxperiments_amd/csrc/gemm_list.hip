@@ -638,8 +638,8 @@ using LC = Cfg;
 // with 509 rows 160 -> 131 (gate and up tiled, qkv and down in small tiles); 2048 -> 3072, 2048, 11008 and
 // 11008 -> 2048 with 512 rows 109 -> 59.  Of 124 drawn batches (256 to 2048 rows, one to five problems) 97 go over in whole or
 // in part and take 0.26 to 1.00 of the list's time, 0.55 in the mean.  With tiles of 160 and 192 rows among the small ones: the four
-// projections with 327 rows 114 -> 97, with 360 122 -> 100, with 526 166 -> 145; over 100 drawn batches 0.95 of the time in the mean
-// (loading waves included), at worst 1.07.
+// projections with 327 rows 114 -> 97, with 360 122 -> 100, with 526 166 -> 145; 250 drawn batches that take them in whole or in part 0.91
+// of the time in the mean, 19 more than 1.03, at worst 1.19.  250 batches of all kinds, loading waves included, 0.95, two more than 1.03.
 struct Split {
     int n_tiled = 0, n_deep = 0;
     int tiled[MAX_PROBLEMS], deep[MAX_PROBLEMS];
@@ -673,7 +673,9 @@ static Load list_load(const int64_t *mnk, const int *idx, int n, int cus, int bn
 // The list in 256 x 128 tiles (gemm_stream.hip): 0.92 us a unit of tile cost and 4 us beside that, weights from HBM.  Half as
 // large, its tiles level out where the others do not: the four projections with 509 rows 142 -> 111 us, 8608 and 6144 columns of
 // 503 rows, K = 8704, 97 -> 80, 6192 columns of 1241 rows, K = 6272, 66 -> 56.  With many
-// rounds the large tiles are 1.1 times as fast (2048 rows 353 against 390 us).  From STREAM_MIN_K on; batches with a shorter K
+// rounds the large tiles are 1.1 times as fast (2048 rows 353 against 390 us).  60 drawn batches of five problems with 419 rows, which
+// an estimate of 0.95 once sent here at a loss, take 0.97 of the time without loading waves at an estimate of 1.0, at worst 1.10 (of which
+// none is in this list).  From STREAM_MIN_K on; batches with a shorter K
 // stay where they were, also where this kernel would be faster (nine such batches: 0.76 to 0.92 of their time).
 
 // bytes of the lists of workgroups with at most this many tiles

@@ -414,9 +414,10 @@ struct MoeFfn {
     }
 };
 
-// One decoder layer of a decode step (one new token per sequence), chained on one stream, nine launches (six for a
-// single sequence, five where its attention is cut into two to eight splits, which the output projection then merges itself; a
-// row-major cache takes one more, for the append):
+// One decoder layer of a decode step (one new token per sequence), chained on one stream, nine launches, six for a
+// single sequence; a row-major cache takes one more, for the append.  Five for a single sequence with a tiled cache whose attention is cut
+// into two to eight splits, which the output projection then merges itself (Hq * 128 from 1024 to 4096, H up to 64 times the
+// compute units, 32 beyond Hq * 128 = 2048, and no trace asked for):
 // (residual +) RMSNorm + quantize -> QKV GEMV -> rotary + cache append -> attention over the cache (split, merge +
 // quantize: the output projection takes the rows in the rotated basis of V) -> O GEMV -> residual + RMSNorm +
 // quantize -> gate|up GEMV -> SwiGLU + quantize -> down GEMV (-> residual).
